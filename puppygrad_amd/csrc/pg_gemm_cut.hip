@@ -1,0 +1,540 @@
+// Products of many rows on the bf16 matrix cores, with f32 inputs, f32 sums and W stored as f32, bf16 or
+// int8 rows (transposed_dense_projection_into, src/models/cpu.rs:58-75; QuantizedRows, cpu.rs:26-56).
+//
+// Every f32 operand is cut into three bf16 numbers whose sum is the value: hi = bf16(x), mid =
+// bf16(x - hi), lo = bf16(x - hi - mid), rounded to nearest, every difference exact; lo holds all that is
+// left of the 24 significant bits.  bf16 and int8 rows are bf16 numbers as they are (the scale of an int8 row
+// multiplies the row's sum), so x w = hi w + mid w + lo w: three v_mfma_f32_32x32x16_bf16 with every product
+// exact, sums in f32, where the f32 matrix cores take eight instructions of twice the duration.  For f32 rows
+// both operands are cut and the six products down to hi lo, mid mid and lo hi are formed.  The three left
+// out are below 2^-25 of x w together (|mid| <= 2^-9 |x|, |lo| <= 2^-17 |x|, the same of w), half of what
+// one rounding of the product to f32 is off; the sums see six roundings per 16 columns where all nine
+// products made nine.  Against an f64 product the error is that of the nine-product form and of the f32
+// cores or smaller (1000 x 4800 x 1600: 2.5e-7 of the result, f32 cores 2.7e-7).
+//
+// What bounds it: power.  With all matrix cores at work the clock goes down to 1.7 to 2.0 GHz (a plain bf16
+// product of the library reaches 1354 of 2500 TFLOP/s on this card), and what else the CU moves is paid
+// for in clock as well as in time.  So the inputs travel as stored: f32 rows of A go straight to LDS
+// (global_load_lds, no registers, no VALU), as do bf16 rows of W; a wavefront owns whole rows of the tile and
+// cuts its A operands itself, in registers, once for all columns it owns; W, which every wavefront needs,
+// is cut once on its way to LDS.  Against the form that cut A for the whole block and kept its planes in
+// LDS (128 x 128 tiles, 2 x 2 wavefronts) that is a quarter of the LDS reads and half the VALU
+// instructions per MFMA: 8192 x 4800 x 1600 bf16 488 -> 378 us, 8192 x 1600 x 6400 640 -> 470 us, int8
+// 643 -> 508 us; f32, nine products -> six, 4096 x 6400 x 1600 680 -> 503 us (one box, W from HBM).
+// The dot instruction that could take both subtractions of a cut (v_dot2_f32_bf16) runs on the matrix
+// cores' time: 6 % slower.
+#include "pg_gemm_dev.h"
+
+#include <type_traits>
+
+namespace pgk {
+
+namespace {
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) char* lds_ptr;
+
+// 16 bytes per lane from base + byte_off (per lane) to lds + 16 lane (LDS address, wavefront-uniform).
+// Inline assembly, so that the compiler's count of loads in flight does not know it: it would wait for all
+// of them at every LDS read.  vm_wait is the wait that belongs to it; a wait that the compiler places for a
+// load of its own is at worst too long (loads return in order).
+__device__ __forceinline__ void lds_dma16(const void* base, unsigned byte_off, unsigned lds) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2"
+      :
+      : "s"(lds), "v"(byte_off), "s"(base)
+      : "memory", "m0");
+}
+// At most N loads of the wavefront in flight.
+template <int N>
+__device__ __forceinline__ void vm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+__device__ __forceinline__ unsigned pk_bf16(float a, float b) {
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(f2{a, b}, bf16x2));
+}
+// Two values as three bf16 each, two to a register (a in the low half).
+__device__ __forceinline__ void cut2(float a, float b, unsigned& hi, unsigned& mid, unsigned& lo) {
+  hi = pk_bf16(a, b);
+  const float a1 = a - __uint_as_float(hi << 16), b1 = b - __uint_as_float(hi & 0xffff0000u);
+  mid = pk_bf16(a1, b1);
+  const float a2 = a1 - __uint_as_float(mid << 16), b2 = b1 - __uint_as_float(mid & 0xffff0000u);
+  lo = pk_bf16(a2, b2);
+}
+// Eight columns of a row as three MFMA operands.
+struct Cut {
+  u4v p[3];
+};
+__device__ __forceinline__ Cut cut8(f4 a, f4 b) {
+  Cut c;
+  unsigned h, m, l;
+  cut2(a.x, a.y, h, m, l);
+  c.p[0].x = h, c.p[1].x = m, c.p[2].x = l;
+  cut2(a.z, a.w, h, m, l);
+  c.p[0].y = h, c.p[1].y = m, c.p[2].y = l;
+  cut2(b.x, b.y, h, m, l);
+  c.p[0].z = h, c.p[1].z = m, c.p[2].z = l;
+  cut2(b.z, b.w, h, m, l);
+  c.p[0].w = h, c.p[1].w = m, c.p[2].w = l;
+  return c;
+}
+
+// WM x WN wavefronts, each on MB x NB blocks of 32 x 32 (MFMA operand: lane (l, half) holds columns
+// 8 half .. 8 half + 7 of row l; result: lane column l, value v row 8 (v / 4) + 4 half + v % 4).
+// K runs in stages of 32 columns (16 for f32 rows), a stage in steps of 16.  While the MFMAs of a step run, the
+// operands of the next one are read from LDS and cut, in the registers that the MFMAs have just freed; W of
+// the stage after it is cut and stored; A and W further ahead are on their way (A in NA buffers).  One
+// barrier per stage, in front of the step that reads the next stage: by then the wavefront has waited for
+// its own share of that stage, and has read the stage before it to the end, whose buffer is free for the
+// stage that is asked for next.  Every buffer has a fixed place in a turn of the loop, so that LDS
+// addresses are constants (no VALU).
+// SPLIT: the stages are cut into gridDim.y parts, raw partial tiles go to a.ws[part][M][N].
+// GROUPED: see launch_gemm_grouped.  WT: W holds f32 (0), bf16 (1) or int8 rows with a.w_scale (2).
+// OCC: wavefronts per SIMD that the registers are kept for.
+template <int WM, int WN, int MB, int NB, int WT, int EPI, int SPLIT, bool GROUPED, int OCC, int NA>
+__global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_cut(GemmArgs a) {
+  constexpr int NW = WM * WN, BM = 32 * MB * WM, BN = 32 * NB * WN;
+  constexpr int KT = WT == 0 ? 16 : 32, NS = KT / 16;
+  constexpr int AP = KT / 4;                          // 16-byte pieces of a row of A in LDS
+  constexpr int IA = BM * AP / 64 / NW;               // DMA instructions of A per wavefront and stage
+  constexpr int IB = WT == 1 ? BN * 4 / 64 / NW : 0;  // the same of W where it is multiplied as stored
+  constexpr int BLD = WT == 0 ? BN * 4 / (64 * NW) : WT == 2 ? BN * 2 / (64 * NW) : 0;  // else 16-byte loads per thread
+  constexpr int UN = WT == 1 ? NA : 4;  // stages per turn of the loop: every buffer has a fixed place in it
+  constexpr int RS = WT == 1 ? 1 : 4;   // sets of load registers
+  constexpr int NPB = WT == 0 ? 3 : 1;  // planes of W in LDS
+  constexpr int NBUF = WT == 1 ? NA : 2;
+  constexpr int BP = WT == 0 ? 2 : 4;   // 16-byte pieces of a row of a plane
+  static_assert(UN % 2 == 0 && UN % NA == 0 && UN <= 4);
+  static_assert(IA >= 1 && BM * AP % (64 * NW) == 0);
+  static_assert(WT == 1 ? IB >= 1 : BLD >= 1);
+  __shared__ u4v As[NA][BM * AP];
+  __shared__ u4v Bs[NBUF][NPB][BN * BP];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
+  int tile;
+  {
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int per_xcd = ((int)gridDim.x + 7) >> 3;
+    tile = xcd * per_xcd + slot;
+  }
+  if (tile >= tiles_m * tiles_n) return;
+  int tm, tn;
+  tile_coords(tile, tiles_m, tiles_n, a.band_rows, &tm, &tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int group = GROUPED ? a.group_tile[tm] : 0;
+  if (GROUPED && group < 0) return;
+
+  const int T_all = a.K / KT;
+  const int kt0 = SPLIT ? (int)(((long)blockIdx.y * T_all) / gridDim.y) : 0;
+  const int kt1 = SPLIT ? (int)(((long)(blockIdx.y + 1) * T_all) / gridDim.y) : T_all;
+  const int T = kt1 - kt0;
+  const int half = lane >> 5, l32 = lane & 31;
+
+  // DMA: the lane's piece of each instruction.  A row's pieces lie permuted (`turn`), so that the 16
+  // lanes that an LDS read serves in one go, 16 rows at the same piece, are on different banks; the
+  // permutation is in the address that a lane loads from, as the instruction stores lane after lane.
+  unsigned aoff[IA], boff[IB ? IB : 1];
+#pragma unroll
+  for (int i = 0; i < IA; ++i) {
+    const int at = (wave * IA + i) * 64 + lane, row = at / AP, slot = at % AP;
+    const int turn = KT == 32 ? (row >> 1) & 7 : (row >> 2) & 3;
+    const int src = GROUPED ? group_row(a, m0 + row) : min(m0 + row, a.M - 1) - m0;
+    aoff[i] = (unsigned)src * (unsigned)a.lda * 4u + (unsigned)(slot ^ turn) * 16u;
+  }
+  constexpr int WBYTES = WT == 0 ? 4 : WT == 1 ? 2 : 1;
+#pragma unroll
+  for (int i = 0; i < IB; ++i) {
+    const int at = (wave * IB + i) * 64 + lane, row = at / 4, slot = at % 4;
+    const int piece = slot ^ ((row >> 2) & 3);
+    boff[i] = (unsigned)(min(n0 + row, a.N - 1) - n0) * (unsigned)a.K * WBYTES + (unsigned)piece * 16u;
+  }
+  const char* Ab = reinterpret_cast<const char*>(a.A + (GROUPED ? (size_t)0 : (size_t)m0 * a.lda) + (size_t)kt0 * KT);
+  const char* Wb = reinterpret_cast<const char*>(a.W) +
+                   (((size_t)n0 + (GROUPED ? (size_t)group * a.N : 0)) * a.K + (size_t)kt0 * KT) * WBYTES;
+  const unsigned as_lds = (unsigned)(size_t)(lds_ptr)(void*)&As[0][0], bs_lds = (unsigned)(size_t)(lds_ptr)(void*)&Bs[0][0][0];
+  auto dma = [&](int t, int buf) __attribute__((always_inline)) {
+    const size_t k = (size_t)min(t, T - 1) * KT;
+#pragma unroll
+    for (int i = 0; i < IA; ++i)
+      lds_dma16(Ab + k * 4, aoff[i], as_lds + (unsigned)(buf * BM * AP * 16 + (wave * IA + i) * 1024));
+#pragma unroll
+    for (int i = 0; i < IB; ++i)
+      lds_dma16(Wb + k * WBYTES, boff[i], bs_lds + (unsigned)(buf * BN * BP * 16 + (wave * IB + i) * 1024));
+  };
+  // W through registers (f32 to be cut, int8 to be widened), asked for RS stages ahead
+  struct Regs { u4v r[BLD ? BLD : 1]; };
+  constexpr int LPR = WT == 0 ? 4 : 2;  // lanes per row
+  const int lr = tid / LPR, lp = tid % LPR;
+  unsigned roff[BLD ? BLD : 1];
+#pragma unroll
+  for (int i = 0; i < BLD; ++i)
+    roff[i] = (unsigned)(min(n0 + lr + i * (64 * NW / LPR), a.N - 1) - n0) * (unsigned)a.K * WBYTES + (unsigned)lp * 16u;
+  auto load_b = [&](int t, Regs& g) __attribute__((always_inline)) {
+    const char* w = Wb + (size_t)min(t, T - 1) * (KT * WBYTES);
+#pragma unroll
+    for (int i = 0; i < BLD; ++i) g.r[i] = *reinterpret_cast<const u4v*>(w + roff[i]);
+  };
+  auto store_b = [&](int buf, const Regs& g) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < BLD; ++i) {
+      const int row = lr + i * (64 * NW / LPR);
+      if constexpr (WT == 0) {
+        const f4 x = __builtin_bit_cast(f4, g.r[i]);
+        unsigned h0, d0, l0, h1, d1, l1;
+        cut2(x.x, x.y, h0, d0, l0);
+        cut2(x.z, x.w, h1, d1, l1);
+        const int piece = (lp >> 1) ^ (((row >> 2) ^ (row >> 3)) & 1);
+        reinterpret_cast<u2v*>(&Bs[buf][0][row * BP + piece])[lp & 1] = u2v{h0, h1};
+        reinterpret_cast<u2v*>(&Bs[buf][1 % NPB][row * BP + piece])[lp & 1] = u2v{d0, d1};
+        reinterpret_cast<u2v*>(&Bs[buf][2 % NPB][row * BP + piece])[lp & 1] = u2v{l0, l1};
+      } else if constexpr (WT == 2) {
+        unsigned w[8];
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+            w[2 * d + b] = pk_bf16((float)((int)(g.r[i][d] << (24 - 16 * b)) >> 24), (float)((int)(g.r[i][d] << (16 - 16 * b)) >> 24));
+        const int turn = (row >> 2) & 3;
+        Bs[buf][0][row * BP + ((2 * lp) ^ turn)] = u4v{w[0], w[1], w[2], w[3]};
+        Bs[buf][0][row * BP + ((2 * lp + 1) ^ turn)] = u4v{w[4], w[5], w[6], w[7]};
+      }
+    }
+  };
+
+  f16v acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+
+  struct Raw { f4 x[MB][2]; };
+  struct Planes { Cut c[MB]; };
+  u4v bb[NPB][NB];
+  auto read_a = [&](int buf, int s, Raw& r) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      const int row = (wm * MB + i) * 32 + l32;
+      const int turn = KT == 32 ? (row >> 1) & 7 : (row >> 2) & 3;
+      const int p = 4 * s + 2 * half;
+      r.x[i][0] = __builtin_bit_cast(f4, As[buf][row * AP + (p ^ turn)]);
+      r.x[i][1] = __builtin_bit_cast(f4, As[buf][row * AP + ((p + 1) ^ turn)]);
+    }
+  };
+  auto read_b = [&](int buf, int s, int j) __attribute__((always_inline)) {
+    const int row = (wn * NB + j) * 32 + l32;
+    const int piece = WT == 0 ? half ^ (((row >> 2) ^ (row >> 3)) & 1) : (2 * s + half) ^ ((row >> 2) & 3);
+#pragma unroll
+    for (int pl = 0; pl < NPB; ++pl) bb[pl][j] = Bs[buf][pl][row * BP + piece];
+  };
+  constexpr int JG = MB == 1 ? 2 : 1;  // column blocks whose sums are taken in turn (a sum waits for its last MFMA)
+  static_assert(NB % JG == 0);
+  constexpr int NP = WT == 0 ? 6 : 3;
+  // one 16-column step: MFMAs of the operands at hand; the next step's operands come in as the
+  // registers get free
+  auto step = [&](const Planes& cur, Planes& nxt, int abuf, int bbuf, int s) __attribute__((always_inline)) {
+    Raw raw;
+    read_a(abuf, s, raw);
+#pragma unroll
+    for (int jg = 0; jg < NB; jg += JG) {
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        constexpr int kPA[6] = {2, 1, 0, 1, 0, 0}, kPB[6] = {0, 1, 2, 0, 1, 0};  // small terms first
+        const int pa = WT == 0 ? kPA[p] : 2 - p, pb = WT == 0 ? kPB[p] : 0;
+#pragma unroll
+        for (int j = jg; j < jg + JG; ++j)
+#pragma unroll
+          for (int i = 0; i < MB; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, cur.c[i].p[pa]),
+                                                               __builtin_bit_cast(bf16x8, bb[pb % NPB][j]), acc[i][j], 0, 0, 0);
+      }
+#pragma unroll
+      for (int j = jg; j < jg + JG; ++j) read_b(bbuf, s, j);
+    }
+#pragma unroll
+    for (int i = 0; i < MB; ++i) nxt.c[i] = cut8(raw.x[i][0], raw.x[i][1]);
+  };
+  // the order of what a step does: an MFMA, and in its shadow a share of the other work
+  auto interleave = [&](auto with_b) __attribute__((always_inline)) {
+    constexpr bool wb = decltype(with_b)::value;
+    constexpr int NM = NP * MB * NB;
+    constexpr int NV = (MB * 46 + (wb ? BLD * (WT == 0 ? 26 : 32) : 0) + NM - 1) / NM + 1;
+    constexpr int NR = (2 * MB + NPB * NB + NM - 1) / NM;
+    __builtin_amdgcn_sched_group_barrier(0x100, 2 * MB, 0);
+#pragma unroll
+    for (int g = 0; g < NM; ++g) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, NR, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, NV, 0);
+      if constexpr (wb) {
+        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  if (T > 0) {
+    Planes pa, pb;
+    Regs r[RS];
+#pragma unroll
+    for (int t = 0; t < NA; ++t) dma(t, t);
+    if constexpr (WT != 1) {
+#pragma unroll
+      for (int t = 0; t < RS; ++t) load_b(t, r[t]);
+      store_b(0, r[0]);
+      load_b(RS, r[0]);
+      store_b(1, r[1]);
+      load_b(RS + 1, r[1]);
+    }
+    vm_wait<(WT == 1 ? (NA - 2) * (IA + IB) : RS * BLD)>();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    {
+      Raw raw;
+      read_a(0, 0, raw);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) read_b(0, 0, j);
+#pragma unroll
+      for (int i = 0; i < MB; ++i) pa.c[i] = cut8(raw.x[i][0], raw.x[i][1]);
+    }
+    const std::true_type yes;
+    const std::false_type no;
+    // stage t, t % UN == U
+    auto stage = [&](auto u, int t, Planes& p0, Planes& p1) __attribute__((always_inline)) {
+      constexpr int U = decltype(u)::value, ab = U % NA, nb = (U + 1) % NA, odd = U & 1;
+      if constexpr (NS == 2) {
+        step(p0, p1, ab, WT == 1 ? ab : odd, 1);
+        interleave(no);
+      }
+      // stage t + 1 has landed once nothing but what was asked for after it is in flight
+      vm_wait<(NA - 2) * (IA + IB) + (NA - 1) * BLD>();
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      dma(t + NA, ab);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (WT != 1) {
+        store_b(odd, r[(U + 2) % RS]);
+        load_b(t + 2 + RS, r[(U + 2) % RS]);
+      }
+      if constexpr (NS == 2) step(p1, p0, nb, WT == 1 ? nb : odd ^ 1, 0);
+      else step(p0, p1, nb, odd ^ 1, 0);
+      interleave(yes);
+    };
+    for (int t = 0; t < T; t += UN) {
+      auto at = [&](auto u) __attribute__((always_inline)) {
+        constexpr int U = decltype(u)::value;
+        if (t + U < T) {
+          if constexpr (NS == 2 || U % 2 == 0) stage(u, t + U, pa, pb);
+          else stage(u, t + U, pb, pa);
+        }
+      };
+      at(std::integral_constant<int, 0>());
+      if (UN > 1) at(std::integral_constant<int, 1 % UN>());
+      if constexpr (UN > 2) {
+        at(std::integral_constant<int, 2 % UN>());
+        at(std::integral_constant<int, 3 % UN>());
+      }
+    }
+    vm_wait<0>();  // (nothing may land in LDS once the block has left it)
+  }
+
+  // an operand that is infinite, or becomes so when it is rounded to bf16, makes the sums it meets
+  // NaN (inf - inf): the wavefront's tile once more in plain f32 arithmetic
+  float bad = 0.0f;
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) bad = fmaf(acc[i][j][v], 0.0f, bad);
+  if (__any(bad != 0.0f)) {
+    redo_tile<MB, NB, WT, EPI, SPLIT, GROUPED>(a, m0 + wm * 32 * MB, n0 + wn * 32 * NB, kt0 * KT, kt1 * KT,
+                                               (int)blockIdx.y, (size_t)group * a.N);
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int n = n0 + (wn * NB + j) * 32 + l32;
+      if (n >= a.N) continue;
+      const float wscale = WT == 2 ? a.w_scale[n] : 1.0f;
+      const float bias = !SPLIT && a.bias ? a.bias[n] : 0.0f;
+      float* part = SPLIT ? a.ws + (size_t)blockIdx.y * a.M * a.N : nullptr;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int m = m0 + (wm * MB + i) * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
+        if (m >= a.M) continue;
+        float c = WT == 2 ? wscale * acc[i][j][v] : acc[i][j][v];
+        if constexpr (SPLIT != 0) {
+          part[(size_t)m * a.N + n] = c;
+          continue;
+        }
+        c = bias + c;
+        if constexpr (EPI == GEMM_SILU_PAIR) {
+          store_silu_pair(a, m, n, c);
+          continue;
+        }
+        if (EPI == GEMM_GELU) c = gelu_tanh(c);
+        if (EPI == GEMM_SQRELU) c = sq_relu(c);
+        if (kAddsResid<EPI>) c = a.resid[(size_t)m * a.ldc + n] + col_scaled<EPI>(a, n, c);
+        a.C[(size_t)m * a.ldc + n] = c;
+      }
+    }
+}
+
+// ---- launchers ---------------------------------------------------------------------------------
+template <int WM, int WN, int MB, int NB, int WT, int OCC, int NA>
+struct Shape {
+  static constexpr int bm = 32 * MB * WM, bn = 32 * NB * WN, threads = 64 * WM * WN;
+  static GemmArgs numbered(const GemmArgs& a0, int* grid) {
+    GemmArgs a = a0;
+    const int tiles_m = (a.M + bm - 1) / bm, tiles_n = (a.N + bn - 1) / bn, tiles = tiles_m * tiles_n;
+    a.band_rows = a.plan_band ? std::min(a.plan_band, tiles_m) : choose_band(tiles_m, std::max(1, (tiles + 7) / 8), bm, bn);
+    *grid = (tiles + 7) / 8 * 8;  // whole rounds over the 8 XCDs
+    return a;
+  }
+  template <int EPI, int SPLIT>
+  static hipError_t start(const GemmArgs& a0, int parts, hipStream_t s) {
+    int grid;
+    const GemmArgs a = numbered(a0, &grid);
+    hipLaunchKernelGGL((k_gemm_cut<WM, WN, MB, NB, WT, EPI, SPLIT, false, OCC, NA>), dim3(grid, parts), dim3(threads), 0, s, a);
+    return hipGetLastError();
+  }
+  static hipError_t launch(const GemmArgs& a, int epi, int parts, hipStream_t s) {
+    if (parts > 1) return start<GEMM_BIAS, 1>(a, parts, s);
+    switch (epi) {
+      case GEMM_BIAS: return start<GEMM_BIAS, 0>(a, 1, s);
+      case GEMM_GELU: return start<GEMM_GELU, 0>(a, 1, s);
+      case GEMM_RESID: return start<GEMM_RESID, 0>(a, 1, s);
+      case GEMM_RESID_SCALED: return start<GEMM_RESID_SCALED, 0>(a, 1, s);
+      case GEMM_SQRELU: return start<GEMM_SQRELU, 0>(a, 1, s);
+      default: return hipErrorInvalidValue;
+    }
+  }
+  static hipError_t launch_grouped(const GemmArgs& a0, int epi, hipStream_t s) {
+    int grid;
+    const GemmArgs a = numbered(a0, &grid);
+    if (epi == GEMM_BIAS)
+      hipLaunchKernelGGL((k_gemm_cut<WM, WN, MB, NB, WT, GEMM_BIAS, 0, true, OCC, NA>), dim3(grid), dim3(threads), 0, s, a);
+    else
+      hipLaunchKernelGGL((k_gemm_cut<WM, WN, MB, NB, WT, GEMM_SILU_PAIR, 0, true, OCC, NA>), dim3(grid), dim3(threads), 0, s, a);
+    return hipGetLastError();
+  }
+};
+// f32 rows: the cut of W costs as much as that of A, so that two wavefronts share an A row block and two
+// wavefronts per SIMD overlap; bf16 and int8 rows: a wavefront owns whole rows of the tile.
+template <int WT>
+using Tile64x128 = Shape<2, 2, 1, 2, WT, 3, WT == 0 ? 4 : 2>;
+template <int WT>
+using Tile128x128 = std::conditional_t<WT == 0, Shape<4, 2, 1, 2, 0, 4, 4>, Shape<4, 1, 1, 4, WT, 3, 2>>;
+using Tile256x128 = Shape<8, 1, 1, 4, 0, 2, 2>;  // (f32 rows)
+template <int WT>
+using Tile128x256 = Shape<4, 1, 1, 8, WT, 2, 2>;  // (bf16 and int8 rows)
+
+template <int WT>
+hipError_t launch_tile(const GemmArgs& a, int epi, CutPlan p, hipStream_t s) {
+  if (p.tile == CUT_64x128) return Tile64x128<WT>::launch(a, epi, p.parts, s);
+  if (p.tile == CUT_128x128) return Tile128x128<WT>::launch(a, epi, p.parts, s);
+  if constexpr (WT == 0) {
+    if (p.tile == CUT_256x128) return Tile256x128::launch(a, epi, p.parts, s);
+  } else {
+    if (p.tile == CUT_128x256) return Tile128x256<WT>::launch(a, epi, p.parts, s);
+  }
+  return hipErrorInvalidValue;
+}
+
+bool takes(const GemmArgs& a) {
+  const int kt = !a.w_bf16 && !a.w_scale ? 16 : 32;
+  // (offsets within a tile's rows are 32 bits)
+  return !(a.w_bf16 && a.w_scale) && a.K % kt == 0 && a.K >= kt && !a.a_packed && !a.c_packed &&
+         (size_t)a.lda * 256 * 4 < ((size_t)1 << 31) && (size_t)a.K * 256 * 4 < ((size_t)1 << 31);
+}
+
+// Time of a product in microseconds: a start, the stages of K at the pace of the CU with the most items,
+// and for a cut K the partial tiles' way through memory.  The constants are least squares over 144 shapes
+// (the four GPT-2 widths' projections at 96 to 2048 rows, W from HBM) with 1 to 8 parts each; they meet the
+// measured times within 6 %, and the plan of least predicted time is 2 % slower than the best measured
+// one in the mean.
+struct Pace {
+  float start, stage, more, part;  // start; a stage alone; each further item on the CU; a partly filled round
+};
+struct Reduce {
+  float start, part, rest;  // a reduction's launch; a part and what is left per 10^6 outputs
+};
+// [storage][64 x 128, 128 x 128, 256 x 128]
+constexpr Pace kPace[3][3] = {
+    {{6.6f, 0.458f, 0.197f, 0.155f}, {6.6f, 0.553f, 0.440f, 0.144f}, {8.6f, 0.880f, 1.008f, 0.097f}},
+    {{7.3f, 0.385f, 0.246f, 0.074f}, {9.1f, 0.521f, 0.415f, 0.087f}, {}},
+    {{7.0f, 0.589f, 0.268f, 0.010f}, {8.5f, 0.742f, 0.368f, 0.000f}, {}}};
+constexpr Reduce kReduce[3] = {{2.8f, 1.30f, 0.5f}, {2.0f, 1.20f, 0.2f}, {5.0f, 1.55f, 0.4f}};
+
+}  // namespace
+
+bool gemm_cut_plan(const GemmArgs& a, int num_cus, CutPlan* plan) {
+  if (!takes(a) || a.M <= 64) return false;  // (37 x 5120 x 1280, int8: a tile of 64 rows is half padding)
+  const int wt = a.w_scale ? 2 : a.w_bf16 ? 1 : 0;
+  const long tiles64 = (long)((a.M + 63) / 64) * ((a.N + 127) / 128);
+  if (wt == 0) {
+    // Few tiles: the f32 cores' 64 x 64 tiles are as fast or faster (96 x 768 x 768: 9.4 against 12.0 us, 128 x
+    // 1024 x 4096: 20.3 against 24.8; from 20 tiles on the other way round, 256 x 768 x 768: 13.6 against
+    // 13.2, 192 x 4800 x 1600: 38.5 against 31.2).
+    if (a.b9_min_rows ? a.M < a.b9_min_rows : tiles64 < 20) return false;
+  } else if (tiles64 < (wt == 1 ? 13 : 24)) {
+    return false;  // (96 x 768 x 768, bf16: 9.9 against 11.3 us; 100 x 1280 x 1280, int8: 14.2 against 15.5)
+  }
+  // Many tiles of 128 x 256 (bf16 and int8 rows; at least two to a CU): half the cuts of A per MFMA
+  // (8192 x 4800 x 1600 bf16: 378 against 388 us, int8 8192 x 1600 x 6400: 508 against 535).
+  if (wt != 0 && (long)((a.M + 127) / 128) * ((a.N + 255) / 256) * 4 >= 7L * num_cus) {
+    *plan = {CUT_128x256, 1};
+    return true;
+  }
+  const float mn = (float)a.M * (float)a.N * 1e-6f;
+  const int stages = a.K / (wt == 0 ? 16 : 32);
+  const bool norm = a.ln_out || a.post_x;  // rides on the reduction of a cut K, else a launch of its own
+  const int most = a.ws && a.N % 4 == 0 ? (int)std::min<size_t>(std::min(8, a.K / 128), a.ws_floats / ((size_t)a.M * a.N)) : 1;
+  const Reduce& red = kReduce[wt];
+  float best = 0.0f;
+  for (int t = 0; t < (wt == 0 && a.M >= 512 ? 3 : 2); ++t) {
+    const int bm = 64 << t;
+    const long tiles = (long)((a.M + bm - 1) / bm) * ((a.N + 127) / 128);
+    for (int parts = 1; parts <= std::max(1, most); ++parts) {
+      const long items = tiles * parts;
+      const float on_cu = (float)((items + num_cus - 1) / num_cus), round = std::max(0.0f, (float)items / (float)num_cus - 1.0f);
+      const Pace& p = kPace[wt][t];
+      const float us = p.start + (float)((stages + parts - 1) / parts) * (p.stage + (on_cu - 1.0f) * p.more + round * p.part) +
+                       (parts > 1 ? red.start + (red.part * (float)parts + red.rest) * mn : norm ? 4.0f + 2.0f * mn : 0.0f);
+      if (best == 0.0f || us < best) {
+        best = us;
+        *plan = {(CutTile)t, parts};
+      }
+    }
+  }
+  return true;
+}
+
+hipError_t launch_gemm_cut(const GemmArgs& a, int epi, CutPlan plan, hipStream_t s) {
+  if (!takes(a) || plan.parts < 1 || plan.parts > 8) return hipErrorInvalidValue;
+  if (plan.parts > 1 && (!a.ws || a.N % 4 != 0 || (size_t)plan.parts * a.M * a.N > a.ws_floats)) return hipErrorInvalidValue;
+  if (a.w_scale) return launch_tile<2>(a, epi, plan, s);
+  return a.w_bf16 ? launch_tile<1>(a, epi, plan, s) : launch_tile<0>(a, epi, plan, s);
+}
+
+hipError_t launch_gemm_cut_grouped(const GemmArgs& a, int epi, int tile_rows, hipStream_t s) {
+  // (a row of A lies anywhere among at most M: 32-bit offsets from A)
+  if (!takes(a) || !a.w_bf16 || (size_t)a.M * a.lda * 4 >= ((size_t)1 << 32)) return hipErrorInvalidValue;
+  if (tile_rows == 64) return Tile64x128<1>::launch_grouped(a, epi, s);
+  if (tile_rows == 128) return Tile128x128<1>::launch_grouped(a, epi, s);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace pgk

@@ -1,0 +1,152 @@
+// What the product kernels of pg_prefill.hip and pg_gemm_cut.hip share.
+#pragma once
+#include <math.h>
+
+#include <algorithm>
+
+#include "pg_kernels.h"
+
+namespace pgk {
+
+// A product on the bf16 matrix cores (pg_gemm_cut.hip): the tile and the number of parts that K is
+// cut into (1: whole tiles; otherwise raw partial tiles to GemmArgs::ws, for a reduce kernel).
+enum CutTile : int { CUT_64x128 = 0, CUT_128x128 = 1, CUT_256x128 = 2, CUT_128x256 = 3 };
+struct CutPlan {
+  CutTile tile;
+  int parts;
+};
+// False where these kernels do not take the product, or are not the faster ones for it.
+bool gemm_cut_plan(const GemmArgs& a, int num_cus, CutPlan* plan);
+hipError_t launch_gemm_cut(const GemmArgs& a, int epi, CutPlan plan, hipStream_t s);
+// (bf16 rows; tiles of tile_rows = 64 or 128 rows)
+hipError_t launch_gemm_cut_grouped(const GemmArgs& a, int epi, int tile_rows, hipStream_t s);
+
+namespace {
+
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f16v __attribute__((ext_vector_type(16)));
+typedef unsigned u2v __attribute__((ext_vector_type(2)));
+typedef unsigned u4v __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ float gelu_tanh(float x) {
+  return 0.5f * x * (1.0f + tanhf(0.7978846f * (x + 0.044715f * x * x * x)));
+}
+// Epilogues that add to the residual, and what column n of the product adds
+// (GEMM_RESID_SCALED: GemmArgs::col_scale).
+template <int EPI>
+constexpr bool kAddsResid = EPI == GEMM_RESID || EPI == GEMM_RESID_SCALED;
+template <int EPI>
+__device__ __forceinline__ float col_scaled(const GemmArgs& a, int n, float c) {
+  if constexpr (EPI == GEMM_RESID_SCALED) return a.col_scale[n] * c;
+  return c;
+}
+
+__device__ __forceinline__ float sq_relu(float x) {
+  const float p = fmaxf(x, 0.0f);
+  return p * p;
+}
+// Grouped products: the row of A that row m takes.
+__device__ __forceinline__ int group_row(const GemmArgs& a, int m) {
+  return a.group_rows ? max(a.group_rows[m], 0) : m;
+}
+// GEMM_SILU_PAIR: column n of the product with its partner column in the neighbouring lane; even
+// columns write.
+__device__ __forceinline__ void store_silu_pair(const GemmArgs& a, int m, int n, float c) {
+  const float up = __shfl_xor(c, 1, 64);
+  if ((n & 1) == 0) a.C[(size_t)m * a.ldc + (n >> 1)] = c / (1.0f + expf(-c)) * up;
+}
+
+// Tile number -> tile coordinates.  Tiles are numbered band by band (a band is `band` tile
+// rows high), down the columns of a band, so that a run of consecutive numbers, which is
+// what one XCD computes, is a compact block of C: its tiles share few rows of A and of W,
+// which that XCD's L2 then fetches once.  (Row-major numbering makes every XCD read all of
+// W.)
+__device__ __forceinline__ void tile_coords(int tile, int tiles_m, int tiles_n, int band, int* tm, int* tn) {
+  const int per_band = band * tiles_n;
+  const int b = tile / per_band, rem = tile - b * per_band;
+  const int bh = min(band, tiles_m - b * band);
+  const int col = rem / bh;
+  *tn = col;
+  *tm = b * band + (rem - col * bh);
+}
+
+// A wavefront's tile once more in plain f32 arithmetic, sums over columns [k0, k1), finished and
+// written out as the kernel's own epilogue would (SPLIT: the raw partial tile of part `part`):
+// where an operand is infinite, or so large that its first part is, the cut values give NaN (inf - inf)
+// and f32 arithmetic gives the reference's result.  The tile is MB x NB blocks of 32 x 32 at (mbase,
+// nbase), a lane's values those of its accumulators.  WT: W holds f32 (0), bf16 (1) or int8 (2) rows;
+// `wrow` is the row of W that column 0 meets, `rows` (may be null) the rows of A as group_row gives
+// them.  It keeps no more than a dozen sums at a time, so that its registers stay below what the
+// kernel's own loop needs; slow, and next to never run.
+template <int MB, int NB, int WT, int EPI, int SPLIT, bool GROUPED>
+__device__ __forceinline__ void redo_tile(const GemmArgs& a, int mbase, int nbase, int k0, int k1, int part, size_t wrow) {
+  const int lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
+  auto w_at = [&](int n, int k) -> float {
+    const size_t at = (wrow + n) * a.K + k;
+    if (WT == 1) return __uint_as_float((unsigned)reinterpret_cast<const unsigned short*>(a.W)[at] << 16);
+    if (WT == 2) return (float)reinterpret_cast<const signed char*>(a.W)[at];
+    return a.W[at];
+  };
+  for (int i = 0; i < MB; ++i)
+    for (int g = 0; g < 4; ++g) {  // four consecutive rows at a time
+      const int mrow = mbase + 32 * i + 8 * g + 4 * half;
+      float sum[4][NB];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) sum[r][j] = 0.0f;
+      for (int k = k0; k < k1; ++k) {
+        float wv[NB], av[4];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) wv[j] = w_at(min(nbase + 32 * j + l32, a.N - 1), k);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) av[r] = a.A[(size_t)(GROUPED ? group_row(a, mrow + r) : min(mrow + r, a.M - 1)) * a.lda + k];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int j = 0; j < NB; ++j) sum[r][j] = fmaf(av[r], wv[j], sum[r][j]);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          const int m = mrow + r, n = nbase + 32 * j + l32;
+          if (m >= a.M || n >= a.N) continue;
+          float c = WT == 2 ? a.w_scale[n] * sum[r][j] : sum[r][j];
+          if (SPLIT) {
+            a.ws[((size_t)part * a.M + m) * a.N + n] = c;
+            continue;
+          }
+          c = (a.bias ? a.bias[n] : 0.0f) + c;
+          if constexpr (EPI == GEMM_SILU_PAIR) {
+            store_silu_pair(a, m, n, c);
+            continue;
+          }
+          if (EPI == GEMM_GELU) c = gelu_tanh(c);
+          if (EPI == GEMM_SQRELU) c = sq_relu(c);
+          if (kAddsResid<EPI>) c = a.resid[(size_t)m * a.ldc + n] + col_scaled<EPI>(a, n, c);
+          a.C[(size_t)m * a.ldc + n] = c;
+        }
+    }
+}
+
+// Band height for tile_coords: a run of `run` consecutive tiles (one XCD's share) should
+// touch as few rows of A and W as it can: hb tile rows and run / hb tile columns.
+inline int choose_band(int tiles_m, int run, int bm, int bn) {
+  int best = 1;
+  long best_cost = -1;
+  for (int hb = 1; hb <= tiles_m; ++hb) {
+    const int bands = (tiles_m + hb - 1) / hb;
+    const int last = tiles_m - (bands - 1) * hb;  // a short last band makes short, wide runs
+    const long cost = (long)hb * bm + (long)((run + hb - 1) / hb) * bn + (last < hb ? (long)(hb - last) * bm / 2 : 0);
+    if (best_cost < 0 || cost < best_cost) {
+      best_cost = cost;
+      best = hb;
+    }
+  }
+  return best;
+}
+
+}  // namespace
+}  // namespace pgk

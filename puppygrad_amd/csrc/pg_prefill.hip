@@ -1,55 +1,19 @@
 // Full-sequence (prefill) kernels for gfx950: fp32 MFMA GEMM with LDS staging and
-// causal attention with LDS-staged K/V tiles; the GEMM also on the bf16 matrix cores with the
-// f32 operands cut into three bf16 parts whose products are exact (k_gemm_b3 for bf16 rows,
-// k_gemm_b9 for f32 rows, the bf16 rows of k_gemm_rows32).
+// causal attention with LDS-staged K/V tiles; the products of many rows that run on the bf16
+// matrix cores are in pg_gemm_cut.hip.
 //
 // They cover Gpt2Model::forward / block_forward / causal_self_attention
 // (src/models/gpt2/rust.rs:831-882, 1053-1134, 1580-1659): the same arithmetic as
 // the reference's token-by-token prefill (rust.rs:910-927), which the reference
 // itself checks against forward() at 1e-5 (rust.rs:1900-1913).
-#include "pg_kernels.h"
+#include "pg_gemm_dev.h"
 #include "pg_mixers.h"
-
-#include <math.h>
-
-#include <algorithm>
 
 #include <type_traits>
 
 namespace pgk {
 
 namespace {
-
-typedef float f4 __attribute__((ext_vector_type(4)));
-typedef float f16v __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ float gelu_tanh(float x) {
-  return 0.5f * x * (1.0f + tanhf(0.7978846f * (x + 0.044715f * x * x * x)));
-}
-// Epilogues that add to the residual, and what column n of the product adds
-// (GEMM_RESID_SCALED: GemmArgs::col_scale).
-template <int EPI>
-constexpr bool kAddsResid = EPI == GEMM_RESID || EPI == GEMM_RESID_SCALED;
-template <int EPI>
-__device__ __forceinline__ float col_scaled(const GemmArgs& a, int n, float c) {
-  if constexpr (EPI == GEMM_RESID_SCALED) return a.col_scale[n] * c;
-  return c;
-}
-
-__device__ __forceinline__ float sq_relu(float x) {
-  const float p = fmaxf(x, 0.0f);
-  return p * p;
-}
-// Grouped products: the row of A that row m takes.
-__device__ __forceinline__ int group_row(const GemmArgs& a, int m) {
-  return a.group_rows ? max(a.group_rows[m], 0) : m;
-}
-// GEMM_SILU_PAIR: column n of the product with its partner column in the neighbouring lane; even
-// columns write.
-__device__ __forceinline__ void store_silu_pair(const GemmArgs& a, int m, int n, float c) {
-  const float up = __shfl_xor(c, 1, 64);
-  if ((n & 1) == 0) a.C[(size_t)m * a.ldc + (n >> 1)] = c / (1.0f + expf(-c)) * up;
-}
 
 // ---------------------------------------------------------------------------
 // C[M,N] = epilogue(A[M,K] . W[N,K]^T + bias)   (transposed_dense_projection_into,
@@ -98,7 +62,6 @@ __device__ __forceinline__ f4 load_w4(const float* W, size_t idx) {
 
 // The same in two steps, so that a tile's widening happens when it is stored to LDS and
 // not where it would wait for the load: the raw 16, 8 or 4 bytes, and their four floats.
-typedef unsigned u2v __attribute__((ext_vector_type(2)));
 template <int WT>
 __device__ __forceinline__ auto load_w_raw(const float* W, size_t idx) {
   if constexpr (WT == 2) {
@@ -128,20 +91,6 @@ __device__ __forceinline__ f4 widen_w(R w) {
   } else {
     return w;
   }
-}
-
-// Tile number -> tile coordinates.  Tiles are numbered band by band (a band is `band` tile
-// rows high), down the columns of a band, so that a run of consecutive numbers, which is
-// what one XCD computes, is a compact block of C: its tiles share few rows of A and of W,
-// which that XCD's L2 then fetches once.  (Row-major numbering makes every XCD read all of
-// W.)
-__device__ __forceinline__ void tile_coords(int tile, int tiles_m, int tiles_n, int band, int* tm, int* tn) {
-  const int per_band = band * tiles_n;
-  const int b = tile / per_band, rem = tile - b * per_band;
-  const int bh = min(band, tiles_m - b * band);
-  const int col = rem / bh;
-  *tn = col;
-  *tm = b * band + (rem - col * bh);
 }
 
 // SPLIT = 1: the K range is cut into gridDim.y parts: part blockIdx.y multiplies its
@@ -368,578 +317,6 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs a) {
           store_silu_pair(a, m, n, c);
           continue;
         }
-        if (EPI == GEMM_GELU) c = gelu_tanh(c);
-        if (EPI == GEMM_SQRELU) c = sq_relu(c);
-        if (kAddsResid<EPI>) c = a.resid[(size_t)m * a.ldc + n] + col_scaled<EPI>(a, n, c);
-        a.C[(size_t)m * a.ldc + n] = c;
-      }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// The same product for W stored as bf16, on the bf16 matrix cores, without giving up f32
-// inputs: every input value is cut into three bf16 numbers whose sum is the value exactly
-// (its 24 significant bits in three groups of 8, by truncation), W's values are bf16 as they
-// are, so x . w = hi . w + mid . w + lo . w with every product exact in f32 and the sums
-// accumulated in f32 as before.  Three v_mfma_f32_32x32x16_bf16 do per 16 columns what eight
-// v_mfma_f32_32x32x2_f32 of four times the duration did.  An infinity in the input stays whole
-// in the first part and a NaN is NaN in all three, so both meet the weights as they would in
-// f32.  One case differs from the f32 product: an infinite bf16 WEIGHT meets the zero second and
-// third parts of a value that fits the first (0 * inf), and the sum is NaN where f32 arithmetic
-// gives an infinity.  (Where W is f32 and cut as well, k_gemm_b9, any infinity would meet zero
-// parts of the other operand: a block that has cut one computes its tile again in plain f32
-// arithmetic, redo_tile, so the result is the f32 product's for infinite inputs and weights.)
-// 256 threads = 4 wavefronts (2 x 2) on a BM x BN tile; k-tiles of 32 columns, staged in LDS
-// row-major ([row][32 bf16] = 64 bytes, the three input planes and W): the operand of a lane
-// is 16 consecutive bytes of its row (8 columns; lanes 32..63 take the second 8 of a 16-column
-// step), and the 16-byte pieces of a row are permuted (lds_piece_turn) so that the lanes of
-// one read hit different banks.  Two LDS buffers; the next tile's global loads are in flight
-// while the current one is multiplied.  K must be a multiple of 32.
-// ---------------------------------------------------------------------------
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef unsigned u4v __attribute__((ext_vector_type(4)));
-
-// The 16-byte pieces of LDS row `row` are stored permuted by this value (xor): the rows that a
-// group of 8 or of 16 lanes reads in one cycle then lie on different banks, whether the LDS
-// serves 32 or 64 banks a cycle.
-__device__ __forceinline__ int lds_piece_turn(int row) { return ((row >> 1) ^ (row >> 3)) & 3; }
-
-struct Split3 {
-  u2v hi, mid, lo;  // four bf16 each, lowest column in the low half of .x
-};
-// GUARD: an infinity stays whole in the first part (inf - inf would make the other two NaN), so
-// its products and sums behave as in f32 arithmetic; a NaN is NaN in all three parts and in
-// every sum it meets, as in f32 arithmetic, with or without the guard.  k_gemm_b9, which cuts
-// both operands, does so without the guard (two instructions a value in its busiest loop: 13 %
-// of an XL prefill) and instead repeats a tile in plain f32 arithmetic when one of its values
-// was infinite (tile_has_infinity, redo_tile).
-template <bool GUARD = true>
-__device__ __forceinline__ Split3 split3_bf16(f4 x) {
-  unsigned h[4], m[4], l[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    h[j] = __float_as_uint(x[j]) & 0xffff0000u;
-    // exact: the 16 low bits of the significand
-    // (v_cmp_class: bits 2 and 9 of the mask are -inf and +inf)
-    const bool whole = GUARD && __builtin_amdgcn_class(x[j], 0x204);
-    const float r1 = whole ? 0.0f : x[j] - __uint_as_float(h[j]);
-    m[j] = __float_as_uint(r1) & 0xffff0000u;
-    const float r2 = r1 - __uint_as_float(m[j]);    // exact: at most 8 significant bits left
-    l[j] = __float_as_uint(r2);
-  }
-  Split3 r;
-  r.hi.x = (h[0] >> 16) | h[1];
-  r.hi.y = (h[2] >> 16) | h[3];
-  r.mid.x = (m[0] >> 16) | m[1];
-  r.mid.y = (m[2] >> 16) | m[3];
-  r.lo.x = (l[0] >> 16) | (l[1] & 0xffff0000u);
-  r.lo.y = (l[2] >> 16) | (l[3] & 0xffff0000u);
-  return r;
-}
-
-// Largest magnitude seen so far (a NaN does not count: it becomes NaN in all three parts and
-// in every sum it meets, as in f32 arithmetic).
-__device__ __forceinline__ float abs_max4(float mx, const f4& v) {
-  return fmaxf(fmaxf(mx, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
-}
-// True for every thread of the block when any thread saw an infinity (mx from abs_max4).
-__device__ __forceinline__ bool tile_has_infinity(float mx, int* flag) {
-  if (mx == INFINITY) *flag = 1;  // (*flag was cleared before the block's first barrier)
-  __syncthreads();
-  return *flag != 0;
-}
-// The block's tile once more in plain f32 arithmetic, sums over columns [k0, k1), finished and
-// written out as the kernel's own epilogue would (SPLIT: the raw partial tile of part `part`):
-// where an operand is infinite the cut values give NaN (a zero part times the infinity) and f32
-// arithmetic gives the reference's result.  The thread's outputs are those of the accumulator
-// layout of the 2 x 2 wavefronts of k_gemm_b3 / k_gemm_b9 (wavefront tile at mbase, nbase).
-// WT: W holds f32 (0), bf16 (1) or int8 (2) rows.  It keeps no more than a dozen sums at a time,
-// so that its registers stay below what the kernel's own loop needs; slow, and next to never run.
-template <int MB, int NB, int WT, int EPI, int SPLIT>
-__device__ __forceinline__ void redo_tile(const GemmArgs& a, int mbase, int nbase, int k0, int k1, int part) {
-  const int lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
-  auto w_at = [&](int n, int k) -> float {
-    const size_t at = (size_t)n * a.K + k;
-    if (WT == 1) return __uint_as_float((unsigned)reinterpret_cast<const unsigned short*>(a.W)[at] << 16);
-    if (WT == 2) return (float)reinterpret_cast<const signed char*>(a.W)[at];
-    return a.W[at];
-  };
-  for (int i = 0; i < MB; ++i)
-    for (int g = 0; g < 4; ++g) {  // four consecutive rows at a time
-      const int mrow = mbase + 32 * i + 8 * g + 4 * half;
-      float sum[4][NB];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int j = 0; j < NB; ++j) sum[r][j] = 0.0f;
-      for (int k = k0; k < k1; ++k) {
-        float wv[NB], av[4];
-#pragma unroll
-        for (int j = 0; j < NB; ++j) wv[j] = w_at(min(nbase + 32 * j + l32, a.N - 1), k);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) av[r] = a.A[(size_t)min(mrow + r, a.M - 1) * a.lda + k];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int j = 0; j < NB; ++j) sum[r][j] = fmaf(av[r], wv[j], sum[r][j]);
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-          const int m = mrow + r, n = nbase + 32 * j + l32;
-          if (m >= a.M || n >= a.N) continue;
-          float c = WT == 2 ? a.w_scale[n] * sum[r][j] : sum[r][j];
-          if (SPLIT) {
-            a.ws[((size_t)part * a.M + m) * a.N + n] = c;
-            continue;
-          }
-          c = (a.bias ? a.bias[n] : 0.0f) + c;
-          if (EPI == GEMM_GELU) c = gelu_tanh(c);
-          if (EPI == GEMM_SQRELU) c = sq_relu(c);
-          if (kAddsResid<EPI>) c = a.resid[(size_t)m * a.ldc + n] + col_scaled<EPI>(a, n, c);
-          a.C[(size_t)m * a.ldc + n] = c;
-        }
-    }
-}
-
-// SPLIT = 1: the k-tiles are cut into gridDim.y parts, the raw partial tiles go to
-// a.ws[part][M][N] and k_splitk_reduce(_ln) finishes them, as for k_gemm.
-// WT = 2: W holds int8 rows with a.w_scale[n] per row (QuantizedRows, cpu.rs:26-56).  The int8
-// values are bf16 numbers as they are, so the same three products per value are exact; the
-// row's scale multiplies the row's sum at the end (the reference scales every weight,
-// cpu.rs:173-184: the two differ by rounding only).
-template <int BM, int BN, int EPI, int SPLIT = 0, int WT = 1, bool GROUPED = false>
-__global__ __launch_bounds__(256) void k_gemm_b3(GemmArgs a) {
-  constexpr int KT = 32;                     // columns per k-tile
-  constexpr int WM = BM / 2, WN = BN / 2;    // per-wavefront tile
-  constexpr int MB = WM / 32, NB = WN / 32;  // 32x32 blocks per wavefront
-  constexpr int ALD = BM / 32;               // float4 loads of A per thread and tile (8 lanes per row)
-  // 16-byte loads of W per thread and tile: bf16 rows 4 lanes per row, int8 rows 2
-  constexpr int BLD = WT == 2 ? BN / 128 : BN / 64;
-  static_assert(BLD >= 1, "tile width");
-  // [buffer][plane][row][piece]: a row is four 16-byte pieces
-  __shared__ u4v As[2][3][BM][4];
-  __shared__ u4v Bs[2][BN][4];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int tiles_n = (a.N + BN - 1) / BN;
-  const int tiles_all = ((a.M + BM - 1) / BM) * tiles_n;
-  int tile;
-  {
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int per_xcd = ((int)gridDim.x + 7) >> 3;
-    tile = xcd * per_xcd + slot;
-  }
-  if (tile >= tiles_all) return;
-  int tm, tn;
-  tile_coords(tile, (a.M + BM - 1) / BM, tiles_n, a.band_rows, &tm, &tn);
-  const int m0 = tm * BM, n0 = tn * BN;
-  const int group = GROUPED ? a.group_tile[tm] : 0;
-  if (GROUPED && group < 0) return;
-
-  // global loads: A eight lanes to a row (a float4 each), W four lanes to a row (8 bf16 each)
-  const int ar = tid >> 3, ak = (tid & 7) * 4;
-  const int br = WT == 2 ? tid >> 1 : tid >> 2;   // W row of the lane's load (of a pass)
-  const int bp = WT == 2 ? 2 * (tid & 1) : tid & 3;  // its first 16-byte piece of the row in LDS
-  const float* Ag[ALD];
-  const char* Wg[BLD];
-#pragma unroll
-  for (int i = 0; i < ALD; ++i)
-    Ag[i] = a.A + (size_t)(GROUPED ? group_row(a, m0 + ar + 32 * i) : min(m0 + ar + 32 * i, a.M - 1)) * a.lda + ak;
-#pragma unroll
-  for (int i = 0; i < BLD; ++i) {
-    constexpr int RP = WT == 2 ? 128 : 64;  // rows per pass
-    const size_t row = (size_t)min(n0 + br + RP * i, a.N - 1) + (GROUPED ? (size_t)group * a.N : 0);
-    Wg[i] = reinterpret_cast<const char*>(a.W) + (WT == 2 ? row * a.K + (tid & 1) * 16 : (row * a.K + bp * 8) * 2);
-  }
-
-  f16v acc[MB][NB];
-#pragma unroll
-  for (int i = 0; i < MB; ++i)
-#pragma unroll
-    for (int j = 0; j < NB; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-  const int T_all = a.K / KT;
-  const int kt0 = SPLIT ? (int)(((long)blockIdx.y * T_all) / gridDim.y) : 0;
-  const int kt1 = SPLIT ? (int)(((long)(blockIdx.y + 1) * T_all) / gridDim.y) : T_all;
-  const int T = kt1 - kt0;  // this block's k-tiles [kt0, kt1)
-  const int half = lane >> 5, l32 = lane & 31;
-  // two sets of load registers: a tile is requested two tiles' arithmetic before it is stored
-  f4 ra0[ALD], ra1[ALD];
-  u4v rb0[BLD], rb1[BLD];
-  auto load_tile = [&](int t, f4 (&ra)[ALD], u4v (&rb)[BLD]) __attribute__((always_inline)) {
-    const size_t k = (size_t)(kt0 + t) * KT;
-#pragma unroll
-    for (int i = 0; i < ALD; ++i) ra[i] = *reinterpret_cast<const f4*>(Ag[i] + k);
-#pragma unroll
-    for (int i = 0; i < BLD; ++i) rb[i] = *reinterpret_cast<const u4v*>(Wg[i] + k * (WT == 2 ? 1 : 2));
-  };
-  auto store_tile = [&](int buf, f4 (&ra)[ALD], u4v (&rb)[BLD]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < ALD; ++i) {
-      const int row = ar + 32 * i;
-      const int piece = (ak >> 3) ^ lds_piece_turn(row);
-      const Split3 sp = split3_bf16(ra[i]);
-      const int h8 = (ak >> 2) & 1;  // which half of the piece
-      reinterpret_cast<u2v*>(&As[buf][0][row][piece])[h8] = sp.hi;
-      reinterpret_cast<u2v*>(&As[buf][1][row][piece])[h8] = sp.mid;
-      reinterpret_cast<u2v*>(&As[buf][2][row][piece])[h8] = sp.lo;
-    }
-#pragma unroll
-    for (int i = 0; i < BLD; ++i) {
-      if constexpr (WT == 2) {
-        // sixteen int8 -> sixteen bf16 (exact), two pieces
-        const int row = br + 128 * i;
-        unsigned hb[16];
-#pragma unroll
-        for (int d = 0; d < 4; ++d)
-#pragma unroll
-          for (int b = 0; b < 4; ++b)
-            hb[4 * d + b] = __float_as_uint((float)((int)(rb[i][d] << (24 - 8 * b)) >> 24));
-        u4v lo8, hi8;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          lo8[e] = (hb[2 * e] >> 16) | (hb[2 * e + 1] & 0xffff0000u);
-          hi8[e] = (hb[8 + 2 * e] >> 16) | (hb[8 + 2 * e + 1] & 0xffff0000u);
-        }
-        Bs[buf][row][bp ^ lds_piece_turn(row)] = lo8;
-        Bs[buf][row][(bp + 1) ^ lds_piece_turn(row)] = hi8;
-      } else {
-        const int row = br + 64 * i;
-        Bs[buf][row][bp ^ lds_piece_turn(row)] = rb[i];
-      }
-    }
-  };
-  // the operands of one 16-column step of a tile: three planes of MB row blocks, NB column blocks
-  struct Ops {
-    u4v a[3][MB], b[NB];
-  };
-  auto read_ops = [&](int buf, int kc, Ops& o) __attribute__((always_inline)) {
-    const int piece = 2 * kc + half;
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      const int row = wn * WN + 32 * j + l32;
-      o.b[j] = Bs[buf][row][piece ^ lds_piece_turn(row)];
-    }
-#pragma unroll
-    for (int i = 0; i < MB; ++i) {
-      const int row = wm * WM + 32 * i + l32;
-#pragma unroll
-      for (int pl = 0; pl < 3; ++pl) o.a[pl][i] = As[buf][pl][row][piece ^ lds_piece_turn(row)];
-    }
-  };
-  auto mfma_ops = [&](const Ops& o) __attribute__((always_inline)) {
-#pragma unroll
-    for (int pl = 2; pl >= 0; --pl)  // the small terms first
-#pragma unroll
-      for (int i = 0; i < MB; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, o.a[pl][i]),
-                                                             __builtin_bit_cast(bf16x8, o.b[j]),
-                                                             acc[i][j], 0, 0, 0);
-  };
-  constexpr int NM = 3 * MB * NB;  // MFMAs per 16-column step
-  // A tile in two halves, each a run of NM MFMAs with the other work of the wavefront placed
-  // between them (an MFMA keeps the matrix core busy for 32 clocks, during which the
-  // wavefront can issue a handful of other instructions):
-  //   first 16 columns of tile t   + LDS reads of its second 16 columns
-  //                                + tile t+1 from its load registers, cut in three, to the other LDS buffer
-  //   barrier
-  //   second 16 columns of tile t  + LDS reads of tile t+1's first 16 columns
-  //                                + request of tile t+3 into the load registers just emptied
-  // (r, rb) hold tile t+1.
-  Ops o0, o1;
-  auto tile_step = [&](auto more_c, int t, f4 (&r)[ALD], u4v (&rb)[BLD]) __attribute__((always_inline)) {
-    constexpr bool more = decltype(more_c)::value;  // a tile t+1 exists
-    mfma_ops(o0);
-    read_ops(t & 1, 1, o1);
-    if (more) store_tile((t + 1) & 1, r, rb);
-#pragma unroll
-    for (int g = 0; g < NM; ++g) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
-      __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // a few VALU
-      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // one LDS write
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
-    __builtin_amdgcn_sched_barrier(0);
-    mfma_ops(o1);
-    if (more) {
-      read_ops((t + 1) & 1, 0, o0);
-      load_tile(min(t + 3, T - 1), r, rb);  // past the end: the last tile again, never used
-    }
-#pragma unroll
-    for (int g = 0; g < NM; ++g) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // one global load
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-
-  if (T > 0) {
-    load_tile(0, ra0, rb0);
-    load_tile(min(1, T - 1), ra1, rb1);
-    store_tile(0, ra0, rb0);
-    __syncthreads();
-    read_ops(0, 0, o0);
-    load_tile(min(2, T - 1), ra0, rb0);
-    const std::true_type yes;
-    const std::false_type no;
-    int t = 0;
-    for (; t + 2 < T; t += 2) {
-      tile_step(yes, t, ra1, rb1);
-      tile_step(yes, t + 1, ra0, rb0);
-    }
-    if (T - t == 2) {
-      tile_step(yes, t, ra1, rb1);
-      tile_step(no, t + 1, ra0, rb0);
-    } else {
-      tile_step(no, t, ra1, rb1);
-    }
-  }
-
-#pragma unroll
-  for (int i = 0; i < MB; ++i)
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      const int n = n0 + wn * WN + 32 * j + l32;
-      if (n >= a.N) continue;
-      const float wscale = WT == 2 ? a.w_scale[n] : 1.0f;
-      if (SPLIT) {
-        float* part = a.ws + (size_t)blockIdx.y * a.M * a.N;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int m = m0 + wm * WM + 32 * i + 8 * (v >> 2) + 4 * half + (v & 3);
-          if (m < a.M) part[(size_t)m * a.N + n] = WT == 2 ? wscale * acc[i][j][v] : acc[i][j][v];
-        }
-        continue;
-      }
-      const float bias = a.bias ? a.bias[n] : 0.0f;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int m = m0 + wm * WM + 32 * i + 8 * (v >> 2) + 4 * half + (v & 3);
-        if (m >= a.M) continue;
-        float c = bias + (WT == 2 ? wscale * acc[i][j][v] : acc[i][j][v]);
-        if constexpr (EPI == GEMM_SILU_PAIR) {
-          store_silu_pair(a, m, n, c);
-          continue;
-        }
-        if (EPI == GEMM_GELU) c = gelu_tanh(c);
-        if (EPI == GEMM_SQRELU) c = sq_relu(c);
-        if (kAddsResid<EPI>) c = a.resid[(size_t)m * a.ldc + n] + col_scaled<EPI>(a, n, c);
-        a.C[(size_t)m * a.ldc + n] = c;
-      }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// The same for W stored as f32: both the input and W are cut into three bf16 parts when their
-// tile is staged and all nine products of the parts are formed, whose sum is x . w exactly —
-// nothing is given up against the f32 matrix instruction, which takes 512 clocks for the 16
-// columns that nine bf16 ones cover in 288.  k-tiles of 16 columns (a row of a plane is 32
-// bytes, two 16-byte pieces, swapped in every second group of four rows against bank
-// conflicts), so that two LDS buffers of six planes are 48 KB and two workgroups share a CU.
-// A tile's 9 MB NB MFMAs run in two halves: the first with the cut + LDS stores of tile t+1
-// between them, then the barrier, the second with the operand reads of tile t+1 and the
-// request of tile t+3.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ int lds_piece_turn2(int row) { return ((row >> 2) ^ (row >> 3)) & 1; }
-
-template <int BM, int BN, int EPI, int SPLIT = 0>
-__global__ __launch_bounds__(256) void k_gemm_b9(GemmArgs a) {
-  constexpr int KT = 16;
-  constexpr int WM = BM / 2, WN = BN / 2;
-  constexpr int MB = WM / 32, NB = WN / 32;
-  constexpr int ALD = BM / 64, BLD = BN / 64;  // float4 loads per thread and tile (4 lanes per row)
-  __shared__ u4v As[2][3][BM][2];
-  __shared__ u4v Bs[2][3][BN][2];
-  __shared__ int s_infinity;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (tid == 0) s_infinity = 0;
-  float in_max = 0.0f;  // largest |input| and |weight| this thread has cut
-  const int wm = wave >> 1, wn = wave & 1;
-  const int tiles_n = (a.N + BN - 1) / BN;
-  const int tiles_all = ((a.M + BM - 1) / BM) * tiles_n;
-  int tile;
-  {
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int per_xcd = ((int)gridDim.x + 7) >> 3;
-    tile = xcd * per_xcd + slot;
-  }
-  if (tile >= tiles_all) return;
-  int tm, tn;
-  tile_coords(tile, (a.M + BM - 1) / BM, tiles_n, a.band_rows, &tm, &tn);
-  const int m0 = tm * BM, n0 = tn * BN;
-
-  const int lr = tid >> 2, lk = (tid & 3) * 4;  // four lanes to a row, a float4 each
-  const float* Ag[ALD];
-  const float* Wg[BLD];
-#pragma unroll
-  for (int i = 0; i < ALD; ++i) Ag[i] = a.A + (size_t)min(m0 + lr + 64 * i, a.M - 1) * a.lda + lk;
-#pragma unroll
-  for (int i = 0; i < BLD; ++i) Wg[i] = a.W + (size_t)min(n0 + lr + 64 * i, a.N - 1) * a.K + lk;
-
-  f16v acc[MB][NB];
-#pragma unroll
-  for (int i = 0; i < MB; ++i)
-#pragma unroll
-    for (int j = 0; j < NB; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-  const int T_all = a.K / KT;
-  const int kt0 = SPLIT ? (int)(((long)blockIdx.y * T_all) / gridDim.y) : 0;
-  const int kt1 = SPLIT ? (int)(((long)(blockIdx.y + 1) * T_all) / gridDim.y) : T_all;
-  const int T = kt1 - kt0;
-  const int half = lane >> 5, l32 = lane & 31;
-  struct Regs {
-    f4 a[ALD], b[BLD];
-  };
-  Regs r0, r1;
-  auto load_tile = [&](int t, Regs& r) __attribute__((always_inline)) {
-    const size_t k = (size_t)(kt0 + t) * KT;
-#pragma unroll
-    for (int i = 0; i < ALD; ++i) r.a[i] = *reinterpret_cast<const f4*>(Ag[i] + k);
-#pragma unroll
-    for (int i = 0; i < BLD; ++i) r.b[i] = *reinterpret_cast<const f4*>(Wg[i] + k);
-  };
-  auto store_tile = [&](int buf, const Regs& r) __attribute__((always_inline)) {
-    const int h8 = (lk >> 2) & 1;
-#pragma unroll
-    for (int i = 0; i < ALD + BLD; ++i) {
-      const int row = lr + 64 * (i < ALD ? i : i - ALD);
-      const int piece = (lk >> 3) ^ lds_piece_turn2(row);
-      in_max = abs_max4(in_max, i < ALD ? r.a[i] : r.b[i - ALD]);
-      const Split3 sp = split3_bf16<false>(i < ALD ? r.a[i] : r.b[i - ALD]);
-      if (i < ALD) {
-        reinterpret_cast<u2v*>(&As[buf][0][row][piece])[h8] = sp.hi;
-        reinterpret_cast<u2v*>(&As[buf][1][row][piece])[h8] = sp.mid;
-        reinterpret_cast<u2v*>(&As[buf][2][row][piece])[h8] = sp.lo;
-      } else {
-        reinterpret_cast<u2v*>(&Bs[buf][0][row][piece])[h8] = sp.hi;
-        reinterpret_cast<u2v*>(&Bs[buf][1][row][piece])[h8] = sp.mid;
-        reinterpret_cast<u2v*>(&Bs[buf][2][row][piece])[h8] = sp.lo;
-      }
-    }
-  };
-  struct Ops {
-    u4v a[3][MB], b[3][NB];
-  };
-  auto read_ops = [&](int buf, Ops& o) __attribute__((always_inline)) {
-#pragma unroll
-    for (int pl = 0; pl < 3; ++pl) {
-#pragma unroll
-      for (int j = 0; j < NB; ++j) {
-        const int row = wn * WN + 32 * j + l32;
-        o.b[pl][j] = Bs[buf][pl][row][half ^ lds_piece_turn2(row)];
-      }
-#pragma unroll
-      for (int i = 0; i < MB; ++i) {
-        const int row = wm * WM + 32 * i + l32;
-        o.a[pl][i] = As[buf][pl][row][half ^ lds_piece_turn2(row)];
-      }
-    }
-  };
-  // MFMAs [g0, g1) of a tile's nine plane pairs (the small terms first), MB NB each
-  auto mfma_ops = [&](const Ops& o, int g0, int g1) __attribute__((always_inline)) {
-#pragma unroll
-    for (int g = g0; g < g1; ++g) {
-      const int pa = 2 - g / 3, pw = 2 - g % 3;
-#pragma unroll
-      for (int i = 0; i < MB; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, o.a[pa][i]),
-                                                             __builtin_bit_cast(bf16x8, o.b[pw][j]),
-                                                             acc[i][j], 0, 0, 0);
-    }
-  };
-  constexpr int G1 = 5;  // plane pairs before the barrier
-  // tile t's operands are in `cur`; `r` holds tile t+1; `nxt` receives tile t+1's operands
-  auto tile_step = [&](auto more_c, int t, const Ops& cur, Ops& nxt, Regs& r) __attribute__((always_inline)) {
-    constexpr bool more = decltype(more_c)::value;
-    mfma_ops(cur, 0, G1);
-    if (more) store_tile((t + 1) & 1, r);
-#pragma unroll
-    for (int g = 0; g < G1 * MB * NB; ++g) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-      __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // a few VALU
-      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // one LDS write
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
-    __builtin_amdgcn_sched_barrier(0);
-    mfma_ops(cur, G1, 9);
-    if (more) {
-      read_ops((t + 1) & 1, nxt);
-      load_tile(min(t + 3, T - 1), r);  // past the end: the last tile again, never used
-    }
-#pragma unroll
-    for (int g = 0; g < (9 - G1) * MB * NB; ++g) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // one global load
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-
-  if (T > 0) {
-    Ops o0, o1;
-    load_tile(0, r0);
-    load_tile(min(1, T - 1), r1);
-    store_tile(0, r0);
-    __syncthreads();
-    read_ops(0, o0);
-    load_tile(min(2, T - 1), r0);
-    const std::true_type yes;
-    const std::false_type no;
-    int t = 0;
-    for (; t + 2 < T; t += 2) {
-      tile_step(yes, t, o0, o1, r1);
-      tile_step(yes, t + 1, o1, o0, r0);
-    }
-    if (T - t == 2) {
-      tile_step(yes, t, o0, o1, r1);
-      tile_step(no, t + 1, o1, o0, r0);
-    } else {
-      tile_step(no, t, o0, o1, r1);
-    }
-  }
-  __syncthreads();  // (also orders the clearing of s_infinity when the block had no k-tile)
-  if (tile_has_infinity(in_max, &s_infinity)) {
-    redo_tile<MB, NB, 0, EPI, SPLIT>(a, m0 + wm * WM, n0 + wn * WN, kt0 * KT, kt1 * KT, (int)blockIdx.y);
-    return;
-  }
-
-#pragma unroll
-  for (int i = 0; i < MB; ++i)
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      const int n = n0 + wn * WN + 32 * j + l32;
-      if (n >= a.N) continue;
-      if (SPLIT) {
-        float* part = a.ws + (size_t)blockIdx.y * a.M * a.N;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int m = m0 + wm * WM + 32 * i + 8 * (v >> 2) + 4 * half + (v & 3);
-          if (m < a.M) part[(size_t)m * a.N + n] = acc[i][j][v];
-        }
-        continue;
-      }
-      const float bias = a.bias ? a.bias[n] : 0.0f;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int m = m0 + wm * WM + 32 * i + 8 * (v >> 2) + 4 * half + (v & 3);
-        if (m >= a.M) continue;
-        float c = bias + acc[i][j][v];
         if (EPI == GEMM_GELU) c = gelu_tanh(c);
         if (EPI == GEMM_SQRELU) c = sq_relu(c);
         if (kAddsResid<EPI>) c = a.resid[(size_t)m * a.ldc + n] + col_scaled<EPI>(a, n, c);
@@ -1226,6 +603,35 @@ __global__ __launch_bounds__(256) void k_gemv_rows(GemmArgs a) {
   if (EPI == GEMM_SQRELU) c = sq_relu(c);
   if (kAddsResid<EPI>) c = a.resid[(size_t)b * a.ldc + n] + col_scaled<EPI>(a, n, c);
   a.C[(size_t)b * a.ldc + n] = c;
+}
+
+// Four values as three bf16 each whose sum is the value exactly (its 24 significant bits in three
+// groups of 8, by truncation).  An infinity stays whole in the first part (inf - inf would make the
+// other two NaN), so its products and sums behave as in f32 arithmetic; a NaN is NaN in all three.
+struct Split3 {
+  u2v hi, mid, lo;  // four bf16 each, lowest column in the low half of .x
+};
+__device__ __forceinline__ Split3 split3_bf16(f4 x) {
+  unsigned h[4], m[4], l[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    h[j] = __float_as_uint(x[j]) & 0xffff0000u;
+    // exact: the 16 low bits of the significand
+    // (v_cmp_class: bits 2 and 9 of the mask are -inf and +inf)
+    const bool whole = __builtin_amdgcn_class(x[j], 0x204);
+    const float r1 = whole ? 0.0f : x[j] - __uint_as_float(h[j]);
+    m[j] = __float_as_uint(r1) & 0xffff0000u;
+    const float r2 = r1 - __uint_as_float(m[j]);    // exact: at most 8 significant bits left
+    l[j] = __float_as_uint(r2);
+  }
+  Split3 r;
+  r.hi.x = (h[0] >> 16) | h[1];
+  r.hi.y = (h[2] >> 16) | h[3];
+  r.mid.x = (m[0] >> 16) | m[1];
+  r.mid.y = (m[2] >> 16) | m[3];
+  r.lo.x = (l[0] >> 16) | (l[1] & 0xffff0000u);
+  r.lo.y = (l[2] >> 16) | (l[3] & 0xffff0000u);
+  return r;
 }
 
 // ---------------------------------------------------------------------------
@@ -1904,8 +1310,6 @@ __global__ __launch_bounds__(256) void k_layer_norm_rows(const float* src, float
   for (int i = threadIdx.x; i < cols; i += 256) out_at(i) = (row[i] - mean) * inv * g[i] + b[i];
 }
 
-int choose_band_fwd(int tiles_m, int run, int bm, int bn);
-hipError_t launch_splitk_reduce_fwd(const GemmArgs& a, int epi, int parts, hipStream_t s, bool* ln_done);
 
 template <int BM, int BN, int WBF, int BKT = BK>
 hipError_t launch_gemm_tile(const GemmArgs& a, int epi, hipStream_t s) {
@@ -1924,100 +1328,6 @@ hipError_t launch_gemm_tile(const GemmArgs& a, int epi, hipStream_t s) {
   else
     return hipErrorInvalidValue;
   return hipGetLastError();
-}
-
-// The bf16 matrix-core form (k_gemm_b3): W stored as bf16 or as int8 rows.
-bool gemm_b3_ok(const GemmArgs& a) {
-  return (a.w_bf16 != 0) != (a.w_scale != nullptr) && a.K % 32 == 0 && a.K >= 32 && !a.a_packed && !a.c_packed;
-}
-template <int BM, int BN, int WT>
-hipError_t launch_gemm_b3_shape(const GemmArgs& a0, int epi, hipStream_t s) {
-  GemmArgs a = a0;
-  const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
-  const int tiles = tiles_m * tiles_n;
-  a.band_rows = a.plan_band ? std::min(a.plan_band, tiles_m) : choose_band_fwd(tiles_m, std::max(1, (tiles + 7) / 8), BM, BN);
-  const int grid = (tiles + 7) / 8 * 8;
-  if (epi == GEMM_BIAS)
-    hipLaunchKernelGGL((k_gemm_b3<BM, BN, GEMM_BIAS, 0, WT>), dim3(grid), dim3(256), 0, s, a);
-  else if (epi == GEMM_GELU)
-    hipLaunchKernelGGL((k_gemm_b3<BM, BN, GEMM_GELU, 0, WT>), dim3(grid), dim3(256), 0, s, a);
-  else if (epi == GEMM_SQRELU)
-    hipLaunchKernelGGL((k_gemm_b3<BM, BN, GEMM_SQRELU, 0, WT>), dim3(grid), dim3(256), 0, s, a);
-  else if (epi == GEMM_RESID)
-    hipLaunchKernelGGL((k_gemm_b3<BM, BN, GEMM_RESID, 0, WT>), dim3(grid), dim3(256), 0, s, a);
-  else if (epi == GEMM_RESID_SCALED)
-    hipLaunchKernelGGL((k_gemm_b3<BM, BN, GEMM_RESID_SCALED, 0, WT>), dim3(grid), dim3(256), 0, s, a);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
-}
-// 128 x 128 tiles (two workgroups to a CU); for bf16 rows 128 x 256 for a long K where those
-// still fill the chip twice over (measured: 4096 x 1600 x 6400, 275 against 302 us);
-// a.plan_bn forces one.
-hipError_t launch_gemm_b3(const GemmArgs& a, int epi, int num_cus, hipStream_t s) {
-  if (!gemm_b3_ok(a)) return hipErrorInvalidValue;
-  if (a.w_scale) return launch_gemm_b3_shape<128, 128, 2>(a, epi, s);
-  const long tiles_wide = (long)((a.M + 127) / 128) * ((a.N + 255) / 256);
-  const bool wide = a.plan_bn ? a.plan_bn == 256 : a.K >= 4096 && tiles_wide >= 2L * num_cus;
-  return wide ? launch_gemm_b3_shape<128, 256, 1>(a, epi, s) : launch_gemm_b3_shape<128, 128, 1>(a, epi, s);
-}
-// f32 rows on the bf16 matrix cores (k_gemm_b9), whole tiles or cut along K into `parts`.
-hipError_t launch_gemm_b9(const GemmArgs& a0, int epi, int parts, hipStream_t s, bool* ln_done) {
-  if (a0.w_bf16 || a0.w_scale || a0.a_packed || a0.c_packed || a0.K % 16 != 0) return hipErrorInvalidValue;
-  GemmArgs a = a0;
-  const int tiles_m = (a.M + 127) / 128, tiles_n = (a.N + 127) / 128;
-  const int tiles = tiles_m * tiles_n;
-  a.band_rows = a.plan_band ? std::min(a.plan_band, tiles_m) : choose_band_fwd(tiles_m, std::max(1, (tiles + 7) / 8), 128, 128);
-  const int grid = (tiles + 7) / 8 * 8;
-  if (parts > 1) {
-    if (!a.ws || (size_t)parts * a.M * a.N > a.ws_floats || a.N % 4 != 0 || parts > 8) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_gemm_b9<128, 128, GEMM_BIAS, 1>), dim3(grid, parts), dim3(256), 0, s, a);
-    return launch_splitk_reduce_fwd(a, epi, parts, s, ln_done);
-  }
-  if (epi == GEMM_BIAS)
-    hipLaunchKernelGGL((k_gemm_b9<128, 128, GEMM_BIAS>), dim3(grid), dim3(256), 0, s, a);
-  else if (epi == GEMM_GELU)
-    hipLaunchKernelGGL((k_gemm_b9<128, 128, GEMM_GELU>), dim3(grid), dim3(256), 0, s, a);
-  else if (epi == GEMM_SQRELU)
-    hipLaunchKernelGGL((k_gemm_b9<128, 128, GEMM_SQRELU>), dim3(grid), dim3(256), 0, s, a);
-  else if (epi == GEMM_RESID)
-    hipLaunchKernelGGL((k_gemm_b9<128, 128, GEMM_RESID>), dim3(grid), dim3(256), 0, s, a);
-  else if (epi == GEMM_RESID_SCALED)
-    hipLaunchKernelGGL((k_gemm_b9<128, 128, GEMM_RESID_SCALED>), dim3(grid), dim3(256), 0, s, a);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
-}
-// Whether the planner sends a product there whole: from a quarter of a tile per CU on (below
-// that a tile's own k loop, one workgroup deep, is too long).
-bool gemm_b3_pays(const GemmArgs& a, int num_cus, int min_share = 4) {
-  return gemm_b3_ok(a) && (long)((a.M + 127) / 128) * ((a.N + 127) / 128) * min_share >= num_cus;
-}
-// Fewer tiles than that (prompts of 65 to a few hundred tokens): the k-tiles cut into up to 8
-// parts so that about two items per CU exist, each at least four k-tiles long; 0 where that
-// does not apply (no workspace, N no multiple of 4, K too short, hardly any tiles).
-int gemm_b3_split_parts(const GemmArgs& a, int num_cus) {
-  // (int8 rows of 33..64 inputs were measured too: XL, 48 tokens, 4.7 ms on the f32-core tiles,
-  // 6.0 ms here)
-  if (!gemm_b3_ok(a) || !a.ws || a.N % 4 != 0 || a.M <= 64) return 0;
-  const long tiles = (long)((a.M + 127) / 128) * ((a.N + 127) / 128);
-  if (!a.plan_parts && tiles < 12) return 0;  // (a dozen short items: the f32 forms' 64 x 64 tiles do better)
-  int parts = a.plan_parts ? a.plan_parts : (int)((2L * num_cus + tiles - 1) / tiles);
-  parts = std::min(parts, a.K / 32 / 4);
-  parts = std::min(parts, 8);  // what the reduce kernels take
-  while (parts > 1 && (size_t)parts * a.M * a.N > a.ws_floats) --parts;
-  return parts >= 2 ? parts : 0;
-}
-hipError_t launch_gemm_b3_split(const GemmArgs& a0, int epi, int parts, hipStream_t s, bool* ln_done) {
-  GemmArgs a = a0;
-  const int tiles_m = (a.M + 127) / 128, tiles_n = (a.N + 127) / 128;
-  const int tiles = tiles_m * tiles_n;
-  a.band_rows = a.plan_band ? std::min(a.plan_band, tiles_m) : choose_band_fwd(tiles_m, std::max(1, (tiles + 7) / 8), 128, 128);
-  if (a.w_scale)
-    hipLaunchKernelGGL((k_gemm_b3<128, 128, GEMM_BIAS, 1, 2>), dim3((tiles + 7) / 8 * 8, parts), dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL((k_gemm_b3<128, 128, GEMM_BIAS, 1, 1>), dim3((tiles + 7) / 8 * 8, parts), dim3(256), 0, s, a);
-  return launch_splitk_reduce_fwd(a, epi, parts, s, ln_done);
 }
 
 }  // namespace
@@ -2295,27 +1605,6 @@ hipError_t launch_tiles_shape(const GemmArgs& a, int epi, int form, int parts, h
   if (a.K % 32 == 0 && !a.plan_bk16) return launch_tiles_depth<BM, BN, WBF, 32>(a, epi, form, parts, s, ln_done);
   return launch_tiles_depth<BM, BN, WBF, 16>(a, epi, form, parts, s, ln_done);
 }
-// Band height for tile_coords: a run of `run` consecutive tiles (one XCD's share) should
-// touch as few rows of A and W as it can: hb tile rows and run / hb tile columns.
-int choose_band(int tiles_m, int run, int bm, int bn) {
-  int best = 1;
-  long best_cost = -1;
-  for (int hb = 1; hb <= tiles_m; ++hb) {
-    const int bands = (tiles_m + hb - 1) / hb;
-    const int last = tiles_m - (bands - 1) * hb;  // a short last band makes short, wide runs
-    const long cost = (long)hb * bm + (long)((run + hb - 1) / hb) * bn + (last < hb ? (long)(hb - last) * bm / 2 : 0);
-    if (best_cost < 0 || cost < best_cost) {
-      best_cost = cost;
-      best = hb;
-    }
-  }
-  return best;
-}
-
-int choose_band_fwd(int tiles_m, int run, int bm, int bn) { return choose_band(tiles_m, run, bm, bn); }
-hipError_t launch_splitk_reduce_fwd(const GemmArgs& a, int epi, int parts, hipStream_t s, bool* ln_done) {
-  return launch_splitk_reduce(a, epi, parts, s, ln_done);
-}
 
 // WBF: 0 f32, 1 bf16, 2 int8 rows (k_gemm's WT)
 template <int WBF>
@@ -2416,25 +1705,15 @@ hipError_t launch_gemm_grouped(const GemmArgs& a0, int epi, int tile_rows, const
 #undef PG_ROWS
     return hipGetLastError();
   }
-  const int bn = a.w_bf16 ? 128 : 64;
-  const int tiles_m = a.M / tile_rows, tiles_n = (a.N + bn - 1) / bn, tiles = tiles_m * tiles_n;
-  a.band_rows = choose_band(tiles_m, std::max(1, (tiles + 7) / 8), tile_rows, bn);
+  if (a.w_bf16) return launch_gemm_cut_grouped(a, epi, tile_rows, s);
+  if (tile_rows != 64) return hipErrorInvalidValue;
+  const int tiles_m = a.M / tile_rows, tiles_n = (a.N + 63) / 64, tiles = tiles_m * tiles_n;
+  a.band_rows = choose_band(tiles_m, std::max(1, (tiles + 7) / 8), tile_rows, 64);
   const dim3 grid((tiles + 7) / 8 * 8);
-#define PG_GROUPED(KERNEL, BM, ...)                                                                          \
-  if (epi == GEMM_BIAS) hipLaunchKernelGGL((KERNEL<BM, GEMM_BIAS, __VA_ARGS__>), grid, dim3(256), 0, s, a);   \
-  else hipLaunchKernelGGL((KERNEL<BM, GEMM_SILU_PAIR, __VA_ARGS__>), grid, dim3(256), 0, s, a);
-#define PG_TILE(M, N) M, N
-  if (a.w_bf16 && tile_rows == 128) {
-    PG_GROUPED(k_gemm_b3, PG_TILE(128, 128), 0, 1, true)
-  } else if (a.w_bf16 && tile_rows == 64) {
-    PG_GROUPED(k_gemm_b3, PG_TILE(64, 128), 0, 1, true)
-  } else if (!a.w_bf16 && tile_rows == 64) {
-    PG_GROUPED(k_gemm, PG_TILE(64, 64), 0, 0, 32, true)
-  } else {
-    return hipErrorInvalidValue;
-  }
-#undef PG_TILE
-#undef PG_GROUPED
+  if (epi == GEMM_BIAS)
+    hipLaunchKernelGGL((k_gemm<64, 64, GEMM_BIAS, 0, 0, 32, true>), grid, dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((k_gemm<64, 64, GEMM_SILU_PAIR, 0, 0, 32, true>), grid, dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
@@ -2447,78 +1726,38 @@ bool gemm_takes_rows32(int M, int K, int lda, int w_bf16) {
 namespace {
 hipError_t launch_gemm_form(const GemmArgs& a, int epi, int num_cus, hipStream_t s, bool* ln_done) {
   if (!gemm_supported(a)) return hipErrorInvalidValue;
+  const bool packed = a.a_packed || a.c_packed || a.ln_packed;
+  if (a.w_scale && (packed || a.w_bf16)) return hipErrorInvalidValue;
   // A small decode batch over a short K: whole rows of W per wavefront, no MFMA tiles.
   // (Every block stages all input vectors; beyond 16 x 1024 values that costs more than it
   // saves.)
-  const bool packed = a.a_packed || a.c_packed || a.ln_packed;
-  if (a.w_scale) {  // int8 rows: up to 32 input rows on the 32-row kernel, else the 64x64 tile form
-    if (packed || a.w_bf16) return hipErrorInvalidValue;
-    if (const int rp = a.plan_form ? 0 : gemm_rows32_parts(a, num_cus))
-      return launch_gemm_rows32<2>(a, epi, rp, num_cus, s, ln_done);
-    int bm = a.plan_bm, bn = a.plan_bn, form = a.plan_form, parts = a.plan_parts;
-    if (form == 4) {  // forced: the 32-row kernel
-      const int rp = gemm_rows32_parts(a, num_cus);
-      return rp ? launch_gemm_rows32<2>(a, epi, rp, num_cus, s, ln_done) : hipErrorInvalidValue;
-    }
-    if (form == 5) return launch_gemm_b3(a, epi, num_cus, s);
-    if (form == 6) {
-      const int bp = gemm_b3_split_parts(a, num_cus);
-      return bp ? launch_gemm_b3_split(a, epi, bp, s, ln_done) : hipErrorInvalidValue;
-    }
-    // on the bf16 matrix cores (int8 values are bf16 numbers), in the order of the bf16 rows
-    if (!form && gemm_b3_pays(a, num_cus, 2)) return launch_gemm_b3(a, epi, num_cus, s);
-    if (!form)
-      if (const int bp = gemm_b3_split_parts(a, num_cus)) return launch_gemm_b3_split(a, epi, bp, s, ln_done);
-    if (!form && gemm_b3_pays(a, num_cus, 4)) return launch_gemm_b3(a, epi, num_cus, s);
-    GemmArgs t = a;
-    if (!form) plan_tiles(t, num_cus, &bm, &bn, &form, &parts);
-    else if (form == 3 && !gemm_tail_plan(t, num_cus, bm, bn)) return hipErrorInvalidValue;
-    return launch_tiles<2>(t, epi, bm, bn, form, parts, s, ln_done);
-  }
-  if (a.plan_form == 5) return launch_gemm_b3(a, epi, num_cus, s);  // forced: the bf16 matrix-core form
-  if (a.plan_form == 7) return launch_gemm_b9(a, epi, std::max(1, a.plan_parts), s, ln_done);  // forced: f32 rows there
-  if (a.plan_form == 6) {                                           // forced: the same, cut along K
-    const int bp = gemm_b3_split_parts(a, num_cus);
-    return bp ? launch_gemm_b3_split(a, epi, bp, s, ln_done) : hipErrorInvalidValue;
-  }
-  if (a.plan_form == 4) {  // forced: the 32-row kernel
-    const int rp = gemm_rows32_parts(a, num_cus);
-    if (!rp) return hipErrorInvalidValue;
-    return a.w_bf16 ? launch_gemm_rows32<1>(a, epi, rp, num_cus, s, ln_done) : launch_gemm_rows32<0>(a, epi, rp, num_cus, s, ln_done);
-  }
-  if (!a.plan_form && gemm_prefers_gemv_rows(a)) {
+  if (!a.w_scale && !a.plan_form && gemm_prefers_gemv_rows(a)) {
     if (packed) return hipErrorInvalidValue;
     return a.w_bf16 ? launch_gemv_rows<true>(a, epi, num_cus, s) : launch_gemv_rows<false>(a, epi, num_cus, s);
   }
-  // other decode batches of up to 32 rows: 32 rows of W per block on the matrix cores
-  if (const int rp = a.plan_form ? 0 : gemm_rows32_parts(a, num_cus))
-    return a.w_bf16 ? launch_gemm_rows32<1>(a, epi, rp, num_cus, s, ln_done)
-                    : launch_gemm_rows32<0>(a, epi, rp, num_cus, s, ln_done);
+  // other batches of up to 32 rows (64, f32 and bf16 rows): 32 rows of W per block on the matrix cores
+  if (a.plan_form == 0 || a.plan_form == 4) {
+    if (const int rp = gemm_rows32_parts(a, num_cus))
+      return a.w_scale  ? launch_gemm_rows32<2>(a, epi, rp, num_cus, s, ln_done)
+             : a.w_bf16 ? launch_gemm_rows32<1>(a, epi, rp, num_cus, s, ln_done)
+                        : launch_gemm_rows32<0>(a, epi, rp, num_cus, s, ln_done);
+    if (a.plan_form == 4) return hipErrorInvalidValue;
+  }
   if (packed) return hipErrorInvalidValue;  // only the 32-row kernel knows the packed form
-  // Tile forms.  A forced plan (benchmarks, tests) or the planner's choice.
+  // more rows: on the bf16 matrix cores where the planner finds enough tiles
+  if (a.plan_form == 0) {
+    CutPlan plan;
+    if (gemm_cut_plan(a, num_cus, &plan)) {
+      const hipError_t e = launch_gemm_cut(a, epi, plan, s);
+      return e != hipSuccess || plan.parts == 1 ? e : launch_splitk_reduce(a, epi, plan.parts, s, ln_done);
+    }
+  }
+  // f32 matrix cores: a forced plan (benchmarks, tests) or the planner's choice
   int bm = a.plan_bm, bn = a.plan_bn, form = a.plan_form, parts = a.plan_parts;
   GemmArgs t = a;
-  // bf16 rows and enough tiles: on the bf16 matrix cores
-  // f32 rows of long inputs (1024 rows and more): on the bf16 matrix cores as nine exact
-  // products per value pair (k_gemm_b9) where that was measured faster than the f32-core
-  // forms: whole 128 x 128 tiles from 0.75 of a tile per CU on (XL c_fc at 1024 rows 199 ->
-  // 176 us, at 4096 rows 818 -> 590 us), tiles cut in four along K between a quarter and
-  // 0.56 of a tile per CU (XL second MLP projection at 1024 rows 213 -> 177 us)
-  if (!form && !a.w_bf16 && !a.w_scale && a.M >= a.b9_min_rows && a.M >= 128 && a.K % 16 == 0) {
-    const long tiles = (long)((a.M + 127) / 128) * ((a.N + 127) / 128);
-    if (tiles * 4 > 3L * num_cus) return launch_gemm_b9(a, epi, 1, s, ln_done);
-    if (tiles * 4 >= num_cus && tiles * 16 < 9L * num_cus && a.K >= 1024 && a.ws && a.N % 4 == 0 &&
-        (size_t)4 * a.M * a.N <= a.ws_floats)
-      return launch_gemm_b9(a, epi, 4, s, ln_done);
-  }
-  // bf16 rows: on the bf16 matrix cores; whole tiles from half a tile per CU on, else cut
-  // along K (measured crossover, XL c_attn / c_fc: 128 to 150 tiles), else whole again
-  if (!form && gemm_b3_pays(a, num_cus, 2)) return launch_gemm_b3(a, epi, num_cus, s);
-  if (!form)
-    if (const int bp = gemm_b3_split_parts(a, num_cus)) return launch_gemm_b3_split(a, epi, bp, s, ln_done);
-  if (!form && gemm_b3_pays(a, num_cus, 4)) return launch_gemm_b3(a, epi, num_cus, s);
   if (!form) plan_tiles(t, num_cus, &bm, &bn, &form, &parts);
   else if (form == 3 && !gemm_tail_plan(t, num_cus, bm, bn)) return hipErrorInvalidValue;
+  if (a.w_scale) return launch_tiles<2>(t, epi, bm, bn, form, parts, s, ln_done);
   return a.w_bf16 ? launch_tiles<1>(t, epi, bm, bn, form, parts, s, ln_done)
                   : launch_tiles<0>(t, epi, bm, bn, form, parts, s, ln_done);
 }
