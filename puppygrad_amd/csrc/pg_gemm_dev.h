@@ -5,6 +5,7 @@
 #include <algorithm>
 
 #include "pg_kernels.h"
+#include "pg_math.h"
 
 namespace pgk {
 
@@ -29,9 +30,6 @@ typedef unsigned u2v __attribute__((ext_vector_type(2)));
 typedef unsigned u4v __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-__device__ __forceinline__ float gelu_tanh(float x) {
-  return 0.5f * x * (1.0f + tanhf(0.7978846f * (x + 0.044715f * x * x * x)));
-}
 // Epilogues that add to the residual, and what column n of the product adds
 // (GEMM_RESID_SCALED: GemmArgs::col_scale).
 template <int EPI>

@@ -7,6 +7,7 @@
 // Shapes the launchers assume are checked on the host before any launch
 // (pg_host.cpp); kernels themselves guard only the ragged tails.
 #include "pg_kernels.h"
+#include "pg_math.h"
 
 #include <math.h>
 
@@ -52,10 +53,6 @@ __device__ __forceinline__ float block_max(float v, float* red) {
 }
 
 // gelu_in_place (cpu.rs:145-150).
-__device__ __forceinline__ float gelu_tanh(float x) {
-  return 0.5f * x * (1.0f + tanhf(0.7978846f * (x + 0.044715f * x * x * x)));
-}
-
 // layer_norm_in_place (cpu.rs:119-143) on a vector already staged in LDS:
 // two-pass mean / biased variance, eps inside the sqrt.
 __device__ __forceinline__ void ln_in_lds(float* sx, int K, const float* g, const float* b,

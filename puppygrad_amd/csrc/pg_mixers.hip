@@ -4,6 +4,7 @@
 //
 // Shapes are checked on the host before any launch (pg_stack.cpp); kernels guard ragged tails.
 #include "pg_mixers.h"
+#include "pg_math.h"
 
 #include <math.h>
 
@@ -17,9 +18,6 @@ namespace {
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 
-__device__ __forceinline__ float gelu_tanh(float x) {
-  return 0.5f * x * (1.0f + tanhf(0.7978846f * (x + 0.044715f * x * x * x)));
-}
 __device__ __forceinline__ float sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 __device__ __forceinline__ float silu(float x) { return x / (1.0f + expf(-x)); }
 __device__ __forceinline__ float softplus(float x) { return fmaxf(x, 0.0f) + log1pf(expf(-fabsf(x))); }
