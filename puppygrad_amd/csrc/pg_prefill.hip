@@ -658,12 +658,12 @@ __device__ __forceinline__ Split3 split3_bf16(f4 x) {
 // MT: tiles of 32 input rows (2: up to 64 rows, row-major input only; the W operands of a step
 // are used twice).
 // WT: W holds f32 (0), bf16 (1) or int8 rows with a.w_scale (2; a weight is (float)q * scale,
-// formed when its piece is read back; row-major input of up to 32 rows only).
+// formed when its piece is read back; row-major input only).
 // GROUPED: see launch_gemm_grouped; blockIdx.z is the tile of 32 rows.
 template <int EPI, int WT, bool XP, bool M16, int NR, int MT, bool GROUPED = false>
 __global__ __launch_bounds__(512) void k_gemm_rows32(GemmArgs a) {
   static_assert(NR == 32 || (NR == 16 && M16), "rows per block");
-  static_assert(MT == 1 || (MT == 2 && !M16 && !XP && WT != 2), "input rows");
+  static_assert(MT == 1 || (MT == 2 && !M16 && !XP), "input rows");
   static_assert(WT != 2 || !XP, "int8 rows: row-major input");
   static_assert(!GROUPED || (!XP && !M16 && MT == 1 && WT != 2), "grouped rows");
   constexpr int CPP = WT == 2 ? 16 : WT == 1 ? 8 : 4;  // columns in a 16-byte piece of a W row
@@ -675,7 +675,9 @@ __global__ __launch_bounds__(512) void k_gemm_rows32(GemmArgs a) {
   constexpr int XSTR = KS + 4;           // row stride of the input tile
   // per wavefront: W tile, input tile; the reduce tile [32 MT][33] lies over them
   constexpr int SLAB = 32 * WSTR + 32 * MT * XSTR > 32 * MT * 33 ? 32 * WSTR + 32 * MT * XSTR : 32 * MT * 33;
-  constexpr int PD = 2;                  // steps requested ahead (3, 4, 6 measured slower)
+  // steps requested ahead (3, 4, 6 measured slower; 64 rows against int8 rows: a second step's 64 input
+  // registers spill, large prompt of 37 tokens 2.85 against 2.28 ms)
+  constexpr int PD = WT == 2 && MT == 2 ? 1 : 2;
   __shared__ __attribute__((aligned(16))) float slab[8][SLAB];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int row0 = GROUPED ? 32 * (int)blockIdx.z : 0, M = GROUPED ? 32 : a.M;
@@ -1444,8 +1446,7 @@ bool gemm_prefers_gemv_rows(const GemmArgs& a) {
 }
 int gemm_rows32_parts(const GemmArgs& a, int num_cus) {
   const int U = a.w_scale ? 64 : a.w_bf16 ? 32 : 16;  // columns per step of the kernel
-  if (a.M > (a.a_packed || a.c_packed || a.ln_packed || a.w_scale ? 32 : 64) || a.K % U != 0 || a.lda % 4 != 0)
-    return 0;
+  if (a.M > (a.a_packed || a.c_packed || a.ln_packed ? 32 : 64) || a.K % U != 0 || a.lda % 4 != 0) return 0;
   const long tiles = (a.N + 31) / 32;
   // (a cut in two plus its reduce launch costs more than it saves: 355M c_attn and c_fc)
   long parts = tiles * 4 > num_cus ? 1 : std::max<long>(1, num_cus / tiles);
@@ -1487,8 +1488,8 @@ template <int WT, bool XP>
 hipError_t launch_gemm_rows32_x(const GemmArgs& a, int epi, int parts, int num_cus, hipStream_t s) {
   const int rows = rows32_block_rows(a, parts, num_cus);
   if (a.M > 32) {
-    // (the packed form holds 32 rows; the int8 form's input tile is sized for 32)
-    if constexpr (XP || WT == 2) return hipErrorInvalidValue;
+    // (the packed form holds 32 rows)
+    if constexpr (XP) return hipErrorInvalidValue;
     else return launch_gemm_rows32_m<WT, false, false, 32, 2>(a, epi, parts, rows, s);
   }
   if (a.M > 16) return launch_gemm_rows32_m<WT, XP, false, 32>(a, epi, parts, rows, s);

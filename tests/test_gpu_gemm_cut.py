@@ -40,8 +40,9 @@ def test_f32_rows(rows, k, n):
     within_f32_sums(got, x, w, b)
 
 
-# one to three stages of 32 columns upward; the last shape has 512 tiles of 128 x 256
-@pytest.mark.parametrize("rows,k,n", [(65, 64, 1600), (129, 128, 1537), (191, 192, 800), (600, 320, 1031), (2000, 64, 8000)])
+# 33 to 64 rows: the small-batch kernel with two tiles of rows, one step of 64 columns for eight wavefronts and
+# more, K cut over blocks; then one to three stages of 32 columns upward; the last shape has 512 tiles of 128 x 256
+@pytest.mark.parametrize("rows,k,n", [(33, 64, 100), (37, 1280, 3840), (64, 576, 5120), (50, 5120, 1280), (65, 64, 1600), (129, 128, 1537), (191, 192, 800), (600, 320, 1031), (2000, 64, 8000)])
 def test_int8_rows(rows, k, n):
     x, w, b = operands(rows, k, n)
     q = np.random.default_rng(n).integers(-127, 128, (n, k)).astype(np.int8)
