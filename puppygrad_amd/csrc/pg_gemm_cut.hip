@@ -31,8 +31,6 @@ namespace pgk {
 
 namespace {
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) char* lds_ptr;
 
 // 16 bytes per lane from base + byte_off (per lane) to lds + 16 lane (LDS address, wavefront-uniform).
@@ -52,35 +50,6 @@ __device__ __forceinline__ void lds_dma16(const void* base, unsigned byte_off, u
 template <int N>
 __device__ __forceinline__ void vm_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-__device__ __forceinline__ unsigned pk_bf16(float a, float b) {
-  return __builtin_bit_cast(unsigned, __builtin_convertvector(f2{a, b}, bf16x2));
-}
-// Two values as three bf16 each, two to a register (a in the low half).
-__device__ __forceinline__ void cut2(float a, float b, unsigned& hi, unsigned& mid, unsigned& lo) {
-  hi = pk_bf16(a, b);
-  const float a1 = a - __uint_as_float(hi << 16), b1 = b - __uint_as_float(hi & 0xffff0000u);
-  mid = pk_bf16(a1, b1);
-  const float a2 = a1 - __uint_as_float(mid << 16), b2 = b1 - __uint_as_float(mid & 0xffff0000u);
-  lo = pk_bf16(a2, b2);
-}
-// Eight columns of a row as three MFMA operands.
-struct Cut {
-  u4v p[3];
-};
-__device__ __forceinline__ Cut cut8(f4 a, f4 b) {
-  Cut c;
-  unsigned h, m, l;
-  cut2(a.x, a.y, h, m, l);
-  c.p[0].x = h, c.p[1].x = m, c.p[2].x = l;
-  cut2(a.z, a.w, h, m, l);
-  c.p[0].y = h, c.p[1].y = m, c.p[2].y = l;
-  cut2(b.x, b.y, h, m, l);
-  c.p[0].z = h, c.p[1].z = m, c.p[2].z = l;
-  cut2(b.z, b.w, h, m, l);
-  c.p[0].w = h, c.p[1].w = m, c.p[2].w = l;
-  return c;
 }
 
 // WM x WN wavefronts, each on MB x NB blocks of 32 x 32 (MFMA operand: lane (l, half) holds columns

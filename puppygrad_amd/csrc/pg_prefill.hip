@@ -605,35 +605,6 @@ __global__ __launch_bounds__(256) void k_gemv_rows(GemmArgs a) {
   a.C[(size_t)b * a.ldc + n] = c;
 }
 
-// Four values as three bf16 each whose sum is the value exactly (its 24 significant bits in three
-// groups of 8, by truncation).  An infinity stays whole in the first part (inf - inf would make the
-// other two NaN), so its products and sums behave as in f32 arithmetic; a NaN is NaN in all three.
-struct Split3 {
-  u2v hi, mid, lo;  // four bf16 each, lowest column in the low half of .x
-};
-__device__ __forceinline__ Split3 split3_bf16(f4 x) {
-  unsigned h[4], m[4], l[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    h[j] = __float_as_uint(x[j]) & 0xffff0000u;
-    // exact: the 16 low bits of the significand
-    // (v_cmp_class: bits 2 and 9 of the mask are -inf and +inf)
-    const bool whole = __builtin_amdgcn_class(x[j], 0x204);
-    const float r1 = whole ? 0.0f : x[j] - __uint_as_float(h[j]);
-    m[j] = __float_as_uint(r1) & 0xffff0000u;
-    const float r2 = r1 - __uint_as_float(m[j]);    // exact: at most 8 significant bits left
-    l[j] = __float_as_uint(r2);
-  }
-  Split3 r;
-  r.hi.x = (h[0] >> 16) | h[1];
-  r.hi.y = (h[2] >> 16) | h[3];
-  r.mid.x = (m[0] >> 16) | m[1];
-  r.mid.y = (m[2] >> 16) | m[3];
-  r.lo.x = (l[0] >> 16) | (l[1] & 0xffff0000u);
-  r.lo.y = (l[2] >> 16) | (l[3] & 0xffff0000u);
-  return r;
-}
-
 // ---------------------------------------------------------------------------
 // A batch of at most 32 rows (64 with MT = 2) against W on the matrix cores.  A block owns 32 rows of W;
 // its eight wavefronts take the steps of the block's K range in turn.  MFMA 32x32x2 wants lane
@@ -794,15 +765,9 @@ __global__ __launch_bounds__(512) void k_gemm_rows32(GemmArgs a) {
       // bf16 and int8 rows: on the bf16 matrix cores.  A piece of a bf16 W row is the operand
       // as it is (8 consecutive columns); a piece of an int8 row is 16 columns, converted to
       // two operands (an int8 value is a bf16 number).  The 8 input values that meet an
-      // operand are cut into three bf16 parts whose sum is the value exactly (split3_bf16), so
-      // the three products are exact and the sums f32 as in the other forms; an int8 row's
-      // scale multiplies its sum at the end.
-      auto cut8 = [](const f4& lo4, const f4& hi4, u4v (&part)[3]) {
-        const Split3 s0 = split3_bf16(lo4), s1 = split3_bf16(hi4);
-        part[0] = u4v{s0.hi.x, s0.hi.y, s1.hi.x, s1.hi.y};
-        part[1] = u4v{s0.mid.x, s0.mid.y, s1.mid.x, s1.mid.y};
-        part[2] = u4v{s0.lo.x, s0.lo.y, s1.lo.x, s1.lo.y};
-      };
+      // operand are cut into three bf16 parts whose sum is the value exactly (cut8), so the three
+      // products are exact and the sums f32 as in the other forms; an int8 row's scale
+      // multiplies its sum at the end.
       // operand h (8 columns) of a piece of W
       auto w_operand = [](const f4& piece, int h) -> u4v {
         const u4v raw = __builtin_bit_cast(u4v, piece);
@@ -822,14 +787,13 @@ __global__ __launch_bounds__(512) void k_gemm_rows32(GemmArgs a) {
       if (M16) {
 #pragma unroll
         for (int h = 0; h < OPS; ++h) {
-          u4v xp3[3];
-          cut8(xo[2 * h], xo[2 * h + 1], xp3);
+          const Cut x3 = cut8(xo[2 * h], xo[2 * h + 1]);
 #pragma unroll
           for (int g = 0; g < NR / 16; ++g) {
             const u4v wop = w_operand(wo[g], h);
 #pragma unroll
             for (int pl = 2; pl >= 0; --pl)
-              acc16[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xp3[pl]),
+              acc16[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x3.p[pl]),
                                                                 __builtin_bit_cast(bf16x8, wop), acc16[g], 0, 0, 0);
           }
         }
@@ -841,11 +805,10 @@ __global__ __launch_bounds__(512) void k_gemm_rows32(GemmArgs a) {
             const u4v wop = w_operand(wo[u], h);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
-              u4v xp3[3];
-              cut8(xo[mt * XT + u * XF + 2 * h], xo[mt * XT + u * XF + 2 * h + 1], xp3);
+              const Cut x3 = cut8(xo[mt * XT + u * XF + 2 * h], xo[mt * XT + u * XF + 2 * h + 1]);
 #pragma unroll
               for (int pl = 2; pl >= 0; --pl)
-                acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xp3[pl]),
+                acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, x3.p[pl]),
                                                                   __builtin_bit_cast(bf16x8, wop), acc[mt], 0, 0, 0);
             }
           }
@@ -919,6 +882,20 @@ __global__ __launch_bounds__(512) void k_gemm_rows32(GemmArgs a) {
     float sum = red_at(0, b, nl);
 #pragma unroll
     for (int w = 1; w < 8; ++w) sum += red_at(w, b, nl);
+    if (WT != 0 && sum != sum) {
+      // (an input that is infinite as bf16 makes its parts NaN: the block's columns in f32 arithmetic)
+      sum = 0.0f;
+      const char* wr = wg + (size_t)n * rowbytes;
+      for (int k = 0; k < a.K; ++k) {
+        const int in_turn = k / KS % pieces - 8 * (int)blockIdx.y;
+        if (in_turn < 0 || in_turn >= 8) continue;
+        const float x = XP ? a.A[packed32_index((size_t)b, (size_t)k)]
+                           : a.A[(size_t)(GROUPED ? group_row(a, row0 + b) : b) * a.lda + k];
+        const float w = WT == 2 ? (float)reinterpret_cast<const signed char*>(wr)[k]
+                                : __uint_as_float((unsigned)reinterpret_cast<const unsigned short*>(wr)[k] << 16);
+        sum = fmaf(x, w, sum);
+      }
+    }
     if (WT == 2) sum *= escale[q];
     if (gridDim.y > 1) {
       a.ws[((size_t)blockIdx.y * a.M + b) * a.N + n] = sum;
