@@ -454,10 +454,11 @@ bool gemm_cut_plan(const GemmArgs& a, int num_cus, CutPlan* plan) {
   const int wt = a.w_scale ? 2 : a.w_bf16 ? 1 : 0;
   const long tiles64 = (long)((a.M + 63) / 64) * ((a.N + 127) / 128);
   if (wt == 0) {
-    // Few tiles: the f32 cores' 64 x 64 tiles are as fast or faster (96 x 768 x 768: 9.4 against 12.0 us, 128 x
-    // 1024 x 4096: 20.3 against 24.8; from 20 tiles on the other way round, 256 x 768 x 768: 13.6 against
-    // 13.2, 192 x 4800 x 1600: 38.5 against 31.2).
-    if (a.b9_min_rows ? a.M < a.b9_min_rows : tiles64 < 20) return false;
+    // Little work: the f32 cores' 64 x 64 tiles are as fast or faster (192 x 2304 x 768: 17.0 against 18.4 us, 128 x
+    // 1280 x 5120: 30.9 against 32.5), unless K is deep enough and the tiles are many (66 x 4800 x 1600: 28
+    // against 23 us); from there on the other way round (256 x 4096 x 1024: 30.7 against 24.1).
+    const double mnk = (double)a.M * a.N * a.K;
+    if (a.b9_min_rows ? a.M < a.b9_min_rows : !(tiles64 >= 20 && mnk >= 0.85e9) && !(tiles64 >= 60 && a.K >= 1280)) return false;
   } else if (tiles64 < (wt == 1 ? 13 : 24)) {
     return false;  // (96 x 768 x 768, bf16: 9.9 against 11.3 us; 100 x 1280 x 1280, int8: 14.2 against 15.5)
   }

@@ -86,6 +86,7 @@ struct GemvPair {
   // part_splits > 0: x1[part_col + i], i < part_n, is instead the sum over part[split][part_n][i]
   const float* part = nullptr;
   int part_splits = 0, part_n = 0, part_col = 0;
+  int num_cus = 256;
 };
 constexpr int kPairMaxSplits = 8;
 constexpr int kPairMaxK = 16320;

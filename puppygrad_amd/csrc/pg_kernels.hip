@@ -9,6 +9,8 @@
 #include "pg_kernels.h"
 #include "pg_math.h"
 
+#include <algorithm>
+
 #include <math.h>
 
 namespace pgk {
@@ -159,11 +161,14 @@ __global__ __launch_bounds__(kBlock) void k_gemv(GemvArgs a) {
   constexpr int kPre = 4;
   const int KV = WM == WM_F32X4 ? K >> 2 : WM == WM_BF16X8 ? K >> 3 : K >> 4;  // chunks per row
   const gv_u4* Wv = reinterpret_cast<const gv_u4*>(a.W);
-  // PRO_STACK: inputs of up to 4096 values and what they are normed with, in registers (asked for before
-  // the weights: loads return in order)
+  // Inputs of up to 4096 values (PRO_STACK: and what they are normed with) in registers, asked for before the
+  // weights: loads return in order, and behind the weights the input was the launch's last wait.
   constexpr int kIn = 4;
-  const bool in_regs = PRO == PRO_STACK && K <= 4 * kIn * kBlock;
-  float4 vx[PRO == PRO_STACK ? kIn : 1], va[PRO == PRO_STACK ? kIn : 1], vg[PRO == PRO_STACK ? kIn : 1],
+  constexpr bool kPlain = kVec && (PRO == PRO_NONE || PRO == PRO_RMS);
+  const bool in_regs = PRO == PRO_STACK ? K <= 4 * kIn * kBlock
+                                        : kPlain && K <= 4 * kIn * kBlock && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0;
+  float ss_x = 0.0f;  // PRO_RMS: sum of the squares of the thread's inputs
+  float4 vx[PRO == PRO_STACK || kPlain ? kIn : 1], va[PRO == PRO_STACK ? kIn : 1], vg[PRO == PRO_STACK ? kIn : 1],
       vn[PRO == PRO_STACK ? kIn : 1];
   if constexpr (PRO == PRO_STACK) {
     if (in_regs) {
@@ -179,6 +184,16 @@ __global__ __launch_bounds__(kBlock) void k_gemv(GemvArgs a) {
           }
           if (a.gain) vn[p] = reinterpret_cast<const float4*>(a.gain)[i];
         }
+      }
+    }
+  }
+  if constexpr (kPlain) {
+    if (in_regs) {
+#pragma unroll
+      for (int p = 0; p < kIn; ++p) {
+        const int i = tid + kBlock * p;
+        vx[p] = float4{0.f, 0.f, 0.f, 0.f};
+        if (4 * i < K) vx[p] = reinterpret_cast<const float4*>(a.x)[i];
       }
     }
   }
@@ -265,6 +280,16 @@ __global__ __launch_bounds__(kBlock) void k_gemv(GemvArgs a) {
       }
     }
   }
+  if constexpr (kPlain) {
+    if (in_regs) {
+#pragma unroll
+      for (int p = 0; p < kIn; ++p) {
+        const int i = tid + kBlock * p;
+        if (4 * i < K) reinterpret_cast<float4*>(sx)[i] = vx[p];
+        if (PRO == PRO_RMS) ss_x += (vx[p].x * vx[p].x + vx[p].y * vx[p].y) + (vx[p].z * vx[p].z + vx[p].w * vx[p].w);
+      }
+    }
+  }
   if (in_regs) {
   } else if (PRO == PRO_ATTN_COMBINE) {
     for (int i = tid; i < K; i += kBlock)
@@ -310,8 +335,9 @@ __global__ __launch_bounds__(kBlock) void k_gemv(GemvArgs a) {
   // RMS norm with one gain: a factor of the finished sums
   float row_mul = 1.0f;
   if (PRO == PRO_RMS) {
-    float ss = 0.0f;
-    for (int i = tid; i < K; i += kBlock) ss += sx[i] * sx[i];
+    float ss = ss_x;
+    if (!in_regs)
+      for (int i = tid; i < K; i += kBlock) ss += sx[i] * sx[i];
     row_mul = a.ln_g[0] / sqrtf(block_sum(ss, red) / (float)a.norm_n + a.eps);
     if (a.out_mul != 0.0f) row_mul *= a.out_mul;
   }
@@ -410,14 +436,19 @@ __global__ __launch_bounds__(kBlock) void k_gemv(GemvArgs a) {
   }
 }
 
-// launch_gemv_pair: one wavefront per row of both matrices, both inputs in LDS.
+constexpr int kPairMaxThreads = 512;
+// launch_gemv_pair: one wavefront per row of both matrices, both inputs in LDS.  The inputs are asked for before
+// the rows (loads return in order), and blocks have as many wavefronts (up to 8) as leave one block to a CU:
+// with partial sums in front of it a block's inputs are half as many bytes as its rows.  1600 rows of 3648 bf16
+// values at a batch of one: 9.7 us with blocks of four wavefronts and the rows first.
 template <int RPW, int WM>
-__global__ __launch_bounds__(kBlock) void k_gemv_pair(GemvPair a) {
+__global__ __launch_bounds__(kPairMaxThreads) void k_gemv_pair(GemvPair a) {
   extern __shared__ __attribute__((aligned(16))) float sx[];  // K1 + K2 floats
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int row0 = (blockIdx.x * kWaves + wave) * RPW;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, threads = blockDim.x;
+  const int row0 = ((int)blockIdx.x * (threads >> 6) + wave) * RPW;
   constexpr int PER = WM == WM_F32X4 ? 4 : 8;  // weights per 16-byte chunk
   constexpr int kPre = 12;
+  constexpr int kIn = 4, kPart = 4;  // of a thread: float4 of inputs, columns of partial sums asked for at once
   const int KV1 = a.K1 / PER, KV2 = a.K2 / PER, KV = KV1 + KV2;
   const gv_u4* W1 = reinterpret_cast<const gv_u4*>(a.W1);
   const gv_u4* W2 = reinterpret_cast<const gv_u4*>(a.W2);
@@ -425,6 +456,25 @@ __global__ __launch_bounds__(kBlock) void k_gemv_pair(GemvPair a) {
   auto chunk = [&](int row, int j) {
     return __builtin_nontemporal_load(j < KV1 ? &W1[(size_t)row * KV1 + j] : &W2[(size_t)row * KV2 + (j - KV1)]);
   };
+  const float4* x1 = reinterpret_cast<const float4*>(a.x1);
+  const float4* x2 = reinterpret_cast<const float4*>(a.x2);
+  const int n1 = a.K1 >> 2, n2 = a.K2 >> 2;
+  // columns that are still partial sums, then the others (whole float4 of the range are left out)
+  const int p0 = a.part_splits > 0 ? a.part_col : 0, p1 = a.part_splits > 0 ? p0 + a.part_n : 0;
+  auto input = [&](int i) { return i < n1 ? x1[i] : x2[i - n1]; };
+  auto whole_input = [&](int i) { return i < n1 + n2 && (4 * i >= p1 || 4 * i + 4 <= p0); };
+  auto part_at = [&](int k, int i) { return a.part[(size_t)min(k, a.part_splits - 1) * a.part_n + i]; };
+  float vp[kPart][kPairMaxSplits];
+  float4 vx[kIn];
+#pragma unroll
+  for (int q = 0; q < kPart; ++q)
+    if (tid + threads * q < p1 - p0) {
+#pragma unroll
+      for (int k = 0; k < kPairMaxSplits; ++k) vp[q][k] = part_at(k, tid + threads * q);
+    }
+#pragma unroll
+  for (int q = 0; q < kIn; ++q)
+    if (whole_input(tid + threads * q)) vx[q] = input(tid + threads * q);
   gv_u4 pre[RPW][kPre];
 #pragma unroll
   for (int r = 0; r < RPW; ++r)
@@ -435,25 +485,29 @@ __global__ __launch_bounds__(kBlock) void k_gemv_pair(GemvPair a) {
       if (row0 + r < a.nout && j < KV) pre[r][i] = chunk(row0 + r, j);
     }
   {
-    const float4* x1 = reinterpret_cast<const float4*>(a.x1);
-    const float4* x2 = reinterpret_cast<const float4*>(a.x2);
     float4* d = reinterpret_cast<float4*>(sx);
-    const int n1 = a.K1 >> 2, n2 = a.K2 >> 2;
-    // columns that are still partial sums, then the others (whole float4 of the range are left out)
-    const int p0 = a.part_splits > 0 ? a.part_col : 0, p1 = a.part_splits > 0 ? p0 + a.part_n : 0;
-    for (int i = tid; i < p1 - p0; i += kBlock) {
-      float v[kPairMaxSplits];
-#pragma unroll
-      for (int k = 0; k < kPairMaxSplits; ++k) v[k] = a.part[(size_t)min(k, a.part_splits - 1) * a.part_n + i];
+    auto sum = [&](const float (&v)[kPairMaxSplits]) {
       float s = 0.0f;
 #pragma unroll
       for (int k = 0; k < kPairMaxSplits; ++k) s += k < a.part_splits ? v[k] : 0.0f;
-      sx[p0 + i] = s;
+      return s;
+    };
+#pragma unroll
+    for (int q = 0; q < kPart; ++q)
+      if (tid + threads * q < p1 - p0) sx[p0 + tid + threads * q] = sum(vp[q]);
+    for (int i = tid + threads * kPart; i < p1 - p0; i += threads) {
+      float v[kPairMaxSplits];
+#pragma unroll
+      for (int k = 0; k < kPairMaxSplits; ++k) v[k] = part_at(k, i);
+      sx[p0 + i] = sum(v);
     }
-    for (int i = tid; i < n1 + n2; i += kBlock) {
+#pragma unroll
+    for (int q = 0; q < kIn; ++q)
+      if (whole_input(tid + threads * q)) d[tid + threads * q] = vx[q];
+    for (int i = tid; i < n1 + n2; i += threads) {
       const int e = 4 * i;
-      if (e >= p1 || e + 4 <= p0) {
-        d[i] = i < n1 ? x1[i] : x2[i - n1];
+      if (whole_input(i)) {
+        if (i >= threads * kIn) d[i] = input(i);
       } else if (e < p0 || e + 4 > p1) {
         for (int k = e; k < e + 4; ++k)
           if (k < p0 || k >= p1) sx[k] = a.x1[k];
@@ -1370,11 +1424,12 @@ hipError_t launch_gemv_pair(const GemvPair& a, hipStream_t s) {
   if (a.K1 % 32 != 0 || a.K2 % 32 != 0 || a.K1 + a.K2 > kPairMaxK || (a.W2 == nullptr) != (a.K2 == 0))
     return hipErrorInvalidValue;
   const size_t lds = (size_t)(a.K1 + a.K2) * sizeof(float);
-  const dim3 grid((a.nout + kWaves - 1) / kWaves);
+  const int waves = std::min(kPairMaxThreads / 64, std::max(kWaves, (a.nout + a.num_cus - 1) / a.num_cus));
+  const dim3 grid((a.nout + waves - 1) / waves);
   if (a.w_bf16)
-    hipLaunchKernelGGL((k_gemv_pair<1, WM_BF16X8>), grid, dim3(kBlock), lds, s, a);
+    hipLaunchKernelGGL((k_gemv_pair<1, WM_BF16X8>), grid, dim3(64 * waves), lds, s, a);
   else
-    hipLaunchKernelGGL((k_gemv_pair<1, WM_F32X4>), grid, dim3(kBlock), lds, s, a);
+    hipLaunchKernelGGL((k_gemv_pair<1, WM_F32X4>), grid, dim3(64 * waves), lds, s, a);
   return hipGetLastError();
 }
 

@@ -1200,6 +1200,7 @@ pg_status step_launches(const pg_model* model, pg_kv_cache* c, ProfileMarks* mar
     if (B == 1) {
       pgk::GemvPair p{};
       p.w_bf16 = model->w_bf16;
+      p.num_cus = model->num_cus;
       p.W1 = l.out_w; p.x1 = st.mix; p.s1 = l.ls1; p.K1 = l.mix_pad;
       p.resid = st.x; p.y = st.x; p.nout = Cp;
       if (sum_in_pair) {
