@@ -146,13 +146,15 @@ __device__ __forceinline__ float chunk_dot(gv_u4 w, const float4* sx4, int j, fl
          (i8_at(ww, 3) * s) * x3.w;
 }
 
-template <int PRO, int EPI, int RPW, int WM>
+// TURNS: the grid holds fewer rows than there are and takes them in turns.
+template <int PRO, int EPI, int RPW, int WM, bool TURNS = false>
 __global__ __launch_bounds__(kBlock) void k_gemv(GemvArgs a) {
   extern __shared__ __attribute__((aligned(16))) float sx[];  // K floats
   __shared__ float red[kWaves];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int K = a.K;
-  const int row0 = (blockIdx.x * kWaves + wave) * RPW;
+  int row0 = (blockIdx.x * kWaves + wave) * RPW;
+  const int row_step = (int)gridDim.x * kWaves * RPW;
 
   // Vector modes: the first chunks of this wavefront's rows are requested before the input
   // vector is staged and normalised, so that the two latencies overlap (a short row is
@@ -164,7 +166,7 @@ __global__ __launch_bounds__(kBlock) void k_gemv(GemvArgs a) {
   // Inputs of up to 4096 values (PRO_STACK: and what they are normed with) in registers, asked for before the
   // weights: loads return in order, and behind the weights the input was the launch's last wait.
   constexpr int kIn = 4;
-  constexpr bool kPlain = kVec && (PRO == PRO_NONE || PRO == PRO_RMS);
+  constexpr bool kPlain = kVec && (PRO == PRO_NONE || PRO == PRO_RMS || PRO == PRO_LN);
   const bool in_regs = PRO == PRO_STACK ? K <= 4 * kIn * kBlock
                                         : kPlain && K <= 4 * kIn * kBlock && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0;
   float ss_x = 0.0f;  // PRO_RMS: sum of the squares of the thread's inputs
@@ -198,17 +200,17 @@ __global__ __launch_bounds__(kBlock) void k_gemv(GemvArgs a) {
     }
   }
   gv_u4 pre[RPW][kPre];
-  if (kVec) {
+  auto request = [&](gv_u4 (&w)[RPW][kPre], int first) {
 #pragma unroll
     for (int r = 0; r < RPW; ++r)
 #pragma unroll
       for (int i = 0; i < kPre; ++i) {
         const int j = lane + 64 * i;
-        pre[r][i] = gv_u4{0u, 0u, 0u, 0u};
-        if (row0 + r < a.nout && j < KV)
-          pre[r][i] = __builtin_nontemporal_load(&Wv[(size_t)(row0 + r) * KV + j]);
+        w[r][i] = gv_u4{0u, 0u, 0u, 0u};
+        if (first + r < a.nout && j < KV) w[r][i] = __builtin_nontemporal_load(&Wv[(size_t)(first + r) * KV + j]);
       }
-  }
+  };
+  if (kVec) request(pre, row0);
 
   if constexpr (PRO == PRO_STACK) {
     if (in_regs) {
@@ -342,96 +344,111 @@ __global__ __launch_bounds__(kBlock) void k_gemv(GemvArgs a) {
     if (a.out_mul != 0.0f) row_mul *= a.out_mul;
   }
 
-  if (row0 >= a.nout) return;
-  float acc[RPW];
-#pragma unroll
-  for (int r = 0; r < RPW; ++r) acc[r] = 0.0f;
-
-  if (kVec) {
-    const float4* sx4 = reinterpret_cast<const float4*>(sx);
-    float sc[RPW];
-#pragma unroll
-    for (int r = 0; r < RPW; ++r)
-      sc[r] = WM == WM_I8X16 ? a.w_scale[min(row0 + r, a.nout - 1)] : 1.0f;
-#pragma unroll
-    for (int i = 0; i < kPre; ++i) {
-      const int j = lane + 64 * i;
-      if (j < KV) {
-#pragma unroll
-        for (int r = 0; r < RPW; ++r)
-          if (row0 + r < a.nout) acc[r] += chunk_dot<WM>(pre[r][i], sx4, j, sc[r]);
-      }
+  // the wavefront's rows; the next turn's are asked for before this turn's are used
+  for (;; row0 += row_step) {
+    if (row0 >= a.nout) return;
+    gv_u4 nxt[TURNS ? RPW : 1][TURNS ? kPre : 1];
+    const bool again = TURNS && row0 + row_step < a.nout;
+    if constexpr (TURNS) {
+      if (again) request(nxt, row0 + row_step);
     }
+    float acc[RPW];
+#pragma unroll
+    for (int r = 0; r < RPW; ++r) acc[r] = 0.0f;
+
+    if (kVec) {
+      const float4* sx4 = reinterpret_cast<const float4*>(sx);
+      float sc[RPW];
+#pragma unroll
+      for (int r = 0; r < RPW; ++r)
+        sc[r] = WM == WM_I8X16 ? a.w_scale[min(row0 + r, a.nout - 1)] : 1.0f;
+#pragma unroll
+      for (int i = 0; i < kPre; ++i) {
+        const int j = lane + 64 * i;
+        if (j < KV) {
+#pragma unroll
+          for (int r = 0; r < RPW; ++r)
+            if (row0 + r < a.nout) acc[r] += chunk_dot<WM>(pre[r][i], sx4, j, sc[r]);
+        }
+      }
 #pragma unroll 2
-    for (int j = lane + 64 * kPre; j < KV; j += 64) {
+      for (int j = lane + 64 * kPre; j < KV; j += 64) {
 #pragma unroll
-      for (int r = 0; r < RPW; ++r) {
-        const int row = row0 + r;
-        if (row < a.nout) {
-          const gv_u4 w = __builtin_nontemporal_load(&Wv[(size_t)row * KV + j]);
-          acc[r] += chunk_dot<WM>(w, sx4, j, sc[r]);
+        for (int r = 0; r < RPW; ++r) {
+          const int row = row0 + r;
+          if (row < a.nout) {
+            const gv_u4 w = __builtin_nontemporal_load(&Wv[(size_t)row * KV + j]);
+            acc[r] += chunk_dot<WM>(w, sx4, j, sc[r]);
+          }
+        }
+      }
+    } else if (WM == WM_I8) {
+      const signed char* Wq = reinterpret_cast<const signed char*>(a.W);
+      for (int j = lane; j < K; j += 64) {
+        float xv = sx[j];
+#pragma unroll
+        for (int r = 0; r < RPW; ++r) {
+          int row = row0 + r;
+          if (row < a.nout) acc[r] += ((float)Wq[(size_t)row * K + j] * a.w_scale[row]) * xv;
+        }
+      }
+    } else if (WM == WM_BF16) {
+      const unsigned short* Wh = reinterpret_cast<const unsigned short*>(a.W);
+      for (int j = lane; j < K; j += 64) {
+        float xv = sx[j];
+#pragma unroll
+        for (int r = 0; r < RPW; ++r) {
+          int row = row0 + r;
+          if (row < a.nout) acc[r] += bf16_lo(Wh[(size_t)row * K + j]) * xv;
+        }
+      }
+    } else {
+      for (int j = lane; j < K; j += 64) {
+        float xv = sx[j];
+#pragma unroll
+        for (int r = 0; r < RPW; ++r) {
+          int row = row0 + r;
+          if (row < a.nout) acc[r] += a.W[(size_t)row * K + j] * xv;
         }
       }
     }
-  } else if (WM == WM_I8) {
-    const signed char* Wq = reinterpret_cast<const signed char*>(a.W);
-    for (int j = lane; j < K; j += 64) {
-      float xv = sx[j];
 #pragma unroll
-      for (int r = 0; r < RPW; ++r) {
-        int row = row0 + r;
-        if (row < a.nout) acc[r] += ((float)Wq[(size_t)row * K + j] * a.w_scale[row]) * xv;
-      }
-    }
-  } else if (WM == WM_BF16) {
-    const unsigned short* Wh = reinterpret_cast<const unsigned short*>(a.W);
-    for (int j = lane; j < K; j += 64) {
-      float xv = sx[j];
-#pragma unroll
-      for (int r = 0; r < RPW; ++r) {
-        int row = row0 + r;
-        if (row < a.nout) acc[r] += bf16_lo(Wh[(size_t)row * K + j]) * xv;
-      }
-    }
-  } else {
-    for (int j = lane; j < K; j += 64) {
-      float xv = sx[j];
-#pragma unroll
-      for (int r = 0; r < RPW; ++r) {
-        int row = row0 + r;
-        if (row < a.nout) acc[r] += a.W[(size_t)row * K + j] * xv;
-      }
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < RPW; ++r) acc[r] = wave_sum(acc[r]);
+    for (int r = 0; r < RPW; ++r) acc[r] = wave_sum(acc[r]);
 
-  if (lane == 0) {
+    if (lane == 0) {
 #pragma unroll
-    for (int r = 0; r < RPW; ++r) {
-      int o = row0 + r;
-      if (o >= a.nout) break;
-      float v = (a.bias ? a.bias[o] : 0.0f) + (PRO == PRO_RMS ? row_mul * acc[r] : acc[r]);
-      if (EPI == EPI_BIAS) {
-        a.y[o] = v;
-      } else if (EPI == EPI_GELU) {
-        a.y[o] = gelu_tanh(v);
-      } else if (EPI == EPI_SQRELU) {
-        const float p = fmaxf(v, 0.0f);
-        a.y[o] = p * p;
-      } else if (EPI == EPI_RESID) {
-        a.y[o] = a.resid[o] + v;  // add_in_place (cpu.rs:167-171)
-      } else {  // EPI_QKV: K/V append of cached_self_attention_into (rust.rs:1677-1683)
-        if (o < a.C) {
+      for (int r = 0; r < RPW; ++r) {
+        int o = row0 + r;
+        if (o >= a.nout) break;
+        float v = (a.bias ? a.bias[o] : 0.0f) + (PRO == PRO_RMS ? row_mul * acc[r] : acc[r]);
+        if (EPI == EPI_BIAS) {
           a.y[o] = v;
-        } else {
-          int which = o >= 2 * a.C;
-          int c = o - (which ? 2 * a.C : a.C);
-          int h = c / a.head_dim, d = c - h * a.head_dim;
-          float* dst = which ? a.vcache : a.kcache;
-          dst[((size_t)h * a.P + a.pos) * a.head_dim + d] = v;
+        } else if (EPI == EPI_GELU) {
+          a.y[o] = gelu_tanh(v);
+        } else if (EPI == EPI_SQRELU) {
+          const float p = fmaxf(v, 0.0f);
+          a.y[o] = p * p;
+        } else if (EPI == EPI_RESID) {
+          a.y[o] = a.resid[o] + v;  // add_in_place (cpu.rs:167-171)
+        } else {  // EPI_QKV: K/V append of cached_self_attention_into (rust.rs:1677-1683)
+          if (o < a.C) {
+            a.y[o] = v;
+          } else {
+            int which = o >= 2 * a.C;
+            int c = o - (which ? 2 * a.C : a.C);
+            int h = c / a.head_dim, d = c - h * a.head_dim;
+            float* dst = which ? a.vcache : a.kcache;
+            dst[((size_t)h * a.P + a.pos) * a.head_dim + d] = v;
+          }
         }
       }
+    }
+    if (!again) return;
+    if constexpr (TURNS) {
+#pragma unroll
+      for (int r = 0; r < RPW; ++r)
+#pragma unroll
+        for (int i = 0; i < kPre; ++i) pre[r][i] = nxt[r][i];
     }
   }
 }
@@ -1372,6 +1389,21 @@ hipError_t launch_gemv_pe(const GemvArgs& a, hipStream_t s) {
   const int rpw = two ? 2 : 1;
   const int blocks = (a.nout + kWaves * rpw - 1) / (kWaves * rpw);
   const int blocks1 = (a.nout + kWaves - 1) / kWaves;
+  // Many rows (the logits) behind a prologue that reads and sums several vectors: four blocks to a CU that
+  // take the rows in turns, so that the prologue runs 1024 times instead of 6283 (161 MB of bf16 rows behind
+  // PRO_STACK 35.8 -> 27.8 us; behind PRO_RMS, a sum of one vector, whole blocks are faster: 25.3 us).
+  constexpr int kTurnBlocks = 1024;
+  if constexpr ((PRO == PRO_STACK || PRO == PRO_LN) && EPI == EPI_BIAS) {
+    if (blocks >= 2 * kTurnBlocks && aligned && a.K % (a.w_scale ? 16 : a.w_bf16 ? 8 : 4) == 0) {
+      if (a.w_scale)
+        hipLaunchKernelGGL((k_gemv<PRO, EPI, 2, WM_I8X16, true>), dim3(kTurnBlocks), dim3(kBlock), lds, s, a);
+      else if (a.w_bf16)
+        hipLaunchKernelGGL((k_gemv<PRO, EPI, 2, WM_BF16X8, true>), dim3(kTurnBlocks), dim3(kBlock), lds, s, a);
+      else
+        hipLaunchKernelGGL((k_gemv<PRO, EPI, 2, WM_F32X4, true>), dim3(kTurnBlocks), dim3(kBlock), lds, s, a);
+      return hipGetLastError();
+    }
+  }
   if (a.w_scale) {
     if (aligned && a.K % 16 == 0) {
       if (two)
