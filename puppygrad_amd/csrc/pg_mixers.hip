@@ -1567,16 +1567,27 @@ __global__ __launch_bounds__(256) void k_add_norm_rows(float* dst, const float* 
     return s;
   };
   float keep[PER], old[PER], g[PER], ss = 0.0f;
+  // (All columns of an expert's row at once: column by column, each behind a branch of its own, a row of 1600 and two
+  // experts took 7.3 us instead of 5.)
+  auto add = [&](float w, const float* from) {
+    float v[PER];
+#pragma unroll
+    for (int p = 0; p < PER; ++p) v[p] = from[min((int)threadIdx.x + 256 * p, cols - 1)];
+#pragma unroll
+    for (int p = 0; p < PER; ++p) keep[p] += w * v[p];
+  };
 #pragma unroll
   for (int p = 0; p < PER; ++p) {
-    const int i = threadIdx.x + 256 * p;
-    const bool in = i < cols;
-    old[p] = in ? x[i] : 0.0f;
-    g[p] = in ? gain[i] : 0.0f;
-    keep[p] = in ? value(i) : 0.0f;
+    const int i = min((int)threadIdx.x + 256 * p, cols - 1);
+    old[p] = x[i];
+    g[p] = gain[i];
+    keep[p] = top == 0 ? src[row * ld + i] : 0.0f;
   }
+#pragma unroll 2
+  for (int k = 0; k < top; ++k) add(weight[row * top + k], src + (size_t)slot[row * top + k] * ld);
 #pragma unroll
-  for (int p = 0; p < PER; ++p) ss += keep[p] * keep[p];
+  for (int p = 0; p < PER; ++p)
+    if ((int)threadIdx.x + 256 * p < cols) ss += keep[p] * keep[p];
   for (int i = threadIdx.x + 256 * PER; i < cols; i += 256) {
     const float v = value(i);
     ss += v * v;
