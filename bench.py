@@ -436,7 +436,7 @@ def bf16_prefill_roofline(flops, gemm_flops, sec, traffic=None, traffic_source=N
     r = {"bound": "mfma", "achieved": round(achieved, 2), "peak": BF16_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
          "frac": round(achieved / BF16_MFMA_PEAK_TFLOPS, 4), "traffic": traffic, "passes": 3,
          "executed": round((2 * gemm_flops + flops) / sec / 1e12, 2),
-         "kernel": "whole prefill (k_gemm_b3 on the bf16 matrix cores, k_attn_prefill64 and lm_head in f32)",
+         "kernel": "whole prefill (k_gemm_cut on the bf16 matrix cores, k_attn_prefill64 and lm_head in f32)",
          "algorithmic_flops_per_step": int(flops), "gemm_flops_per_step": int(gemm_flops)}
     if traffic_source:
         r["traffic_source"] = traffic_source
@@ -507,7 +507,7 @@ def bench_prefill(args, cfg, model, ids, n_prefill) -> int:
                    "backend": model.describe()},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 2), "peak": FP32_MFMA_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(achieved / FP32_MFMA_PEAK_TFLOPS, 4), "traffic": None,
-                     "kernel": "whole prefill (k_gemm, or k_gemm_b9 from 1024 rows on where it is faster; "
+                     "kernel": "whole prefill (k_gemm, or k_gemm_cut where it is faster; "
                                "k_attn_prefill64, LayerNorm, split-K reduces, lm_head)",
                      "algorithmic_flops_per_step": int(flops), "gemm_flops_per_step": int(gemm_flops)},
     }
@@ -704,8 +704,8 @@ TRAFFIC_SOURCE_355M_B16 = "profiles/batched_decode_355m_b16_xl_bf16_b32.txt"
 # Bytes through the L2s to and from the fabric per XL bf16 prefill of 32 x 512 tokens (FETCH_SIZE
 # scaled by 1.9994 + WRITE_SIZE over all launches of a step; most of the reads are operand
 # re-reads that the Infinity Cache serves).
-TRAFFIC_XL_BF16_PREFILL_B32_512 = 573030000000
-TRAFFIC_SOURCE_XL_BF16_PREFILL = "profiles/k_gemm_b3_xl_bf16_prefill_b32_512.txt"
+TRAFFIC_XL_BF16_PREFILL_B32_512 = 372400000000
+TRAFFIC_SOURCE_XL_BF16_PREFILL = "profiles/k_gemm_cut_xl_bf16_prefill_b32_512.txt"
 
 
 def measured_traffic(args, n_prefill, persistent, bytes_per_launch):
