@@ -6,11 +6,21 @@
 // left of the 24 significant bits.  bf16 and int8 rows are bf16 numbers as they are (the scale of an int8 row
 // multiplies the row's sum), so x w = hi w + mid w + lo w: three v_mfma_f32_32x32x16_bf16 with every product
 // exact, sums in f32, where the f32 matrix cores take eight instructions of twice the duration.  For f32 rows
-// both operands are cut and the six products down to hi lo, mid mid and lo hi are formed.  The three left
-// out are below 2^-25 of x w together (|mid| <= 2^-9 |x|, |lo| <= 2^-17 |x|, the same of w), half of what
-// one rounding of the product to f32 is off; the sums see six roundings per 16 columns where all nine
-// products made nine.  Against an f64 product the error is that of the nine-product form and of the f32
-// cores or smaller (1000 x 4800 x 1600: 2.5e-7 of the result, f32 cores 2.7e-7).
+// both operands are cut and the six products down to hi lo, mid mid and lo hi are formed.  |mid| <= 2^-8 |x|
+// and |lo| <= 2^-17 |x|, the same of w, so the three left out are at most 2^-24 of x w together, one
+// rounding of the product to f32; over ordinary values they are of either sign.
+//
+// How the sums round: the instruction adds two groups of eight products to the accumulator one after the other
+// and rounds to f32 each time; before that it cuts off products below 2^-24 of the group's largest, and downward
+// the accumulator below the same and the group's sum below 2^-31 of the accumulator.  With all products of K in one
+// register the small ones (mid, lo) cost as many roundings at the whole sum's size as hi hi does, the
+// error has a mean (-8e-8 of the result at K = 1600), and rows that are alike get the same error from hi lo,
+// which is a few units of the sum's last place: keys and values of a whole cache are off the same way,
+// which attention does not average out (XL, logits behind 896 tokens: 5.8e-7 with f32-core products, 9.2e-7
+// so).  Tiles that have the registers therefore keep two sums, hi hi (bf16 and int8 rows: hi w) and all that
+// is smaller, added at the end (TWO): the same logits 4.1e-7; 895 x 4800 x 1600 against f64 2.4e-7 of the
+// result for f32 rows (one sum 6.2e-7, f32 cores 7.1e-7) and 2.4e-7 for bf16 rows (one sum 4.3e-7).  The
+// 128 x 256 tile has no room for a second sum: as precise as one sum, 4.3e-7.
 //
 // What bounds it: power.  With all matrix cores at work the clock goes down to 1.7 to 2.0 GHz (a plain bf16
 // product of the library reaches 1354 of 2500 TFLOP/s on this card), and what else the CU moves is paid
@@ -63,8 +73,8 @@ __device__ __forceinline__ void vm_wait() {
 // addresses are constants (no VALU).
 // SPLIT: the stages are cut into gridDim.y parts, raw partial tiles go to a.ws[part][M][N].
 // GROUPED: see launch_gemm_grouped.  WT: W holds f32 (0), bf16 (1) or int8 rows with a.w_scale (2).
-// OCC: wavefronts per SIMD that the registers are kept for.
-template <int WM, int WN, int MB, int NB, int WT, int EPI, int SPLIT, bool GROUPED, int OCC, int NA>
+// OCC: wavefronts per SIMD that the registers are kept for.  TWO: small products have a sum of their own.
+template <int WM, int WN, int MB, int NB, int WT, int EPI, int SPLIT, bool GROUPED, int OCC, int NA, bool TWO>
 __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_cut(GemmArgs a) {
   constexpr int NW = WM * WN, BM = 32 * MB * WM, BN = 32 * NB * WN;
   constexpr int KT = WT == 0 ? 16 : 32, NS = KT / 16;
@@ -177,13 +187,16 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_cut(GemmArgs a) {
     }
   };
 
-  f16v acc[MB][NB];
+  f16v acc[MB][NB], low[TWO ? MB : 1][TWO ? NB : 1];
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+      for (int v = 0; v < 16; ++v) {
+        acc[i][j][v] = 0.0f;
+        if constexpr (TWO) low[i][j][v] = 0.0f;
+      }
 
   struct Raw { f4 x[MB][2]; };
   struct Planes { Cut c[MB]; };
@@ -221,9 +234,11 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_cut(GemmArgs a) {
 #pragma unroll
         for (int j = jg; j < jg + JG; ++j)
 #pragma unroll
-          for (int i = 0; i < MB; ++i)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, cur.c[i].p[pa]),
-                                                               __builtin_bit_cast(bf16x8, bb[pb % NPB][j]), acc[i][j], 0, 0, 0);
+          for (int i = 0; i < MB; ++i) {
+            f16v& sum = TWO && pa + pb > 0 ? low[TWO ? i : 0][TWO ? j : 0] : acc[i][j];
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, cur.c[i].p[pa]),
+                                                         __builtin_bit_cast(bf16x8, bb[pb % NPB][j]), sum, 0, 0, 0);
+          }
       }
 #pragma unroll
       for (int j = jg; j < jg + JG; ++j) read_b(bbuf, s, j);
@@ -324,7 +339,10 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_cut(GemmArgs a) {
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) bad = fmaf(acc[i][j][v], 0.0f, bad);
+      for (int v = 0; v < 16; ++v) {
+        if constexpr (TWO) acc[i][j][v] += low[i][j][v];
+        bad = fmaf(acc[i][j][v], 0.0f, bad);
+      }
   if (__any(bad != 0.0f)) {
     redo_tile<MB, NB, WT, EPI, SPLIT, GROUPED>(a, m0 + wm * 32 * MB, n0 + wn * 32 * NB, kt0 * KT, kt1 * KT,
                                                (int)blockIdx.y, (size_t)group * a.N);
@@ -362,7 +380,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_cut(GemmArgs a) {
 }
 
 // ---- launchers ---------------------------------------------------------------------------------
-template <int WM, int WN, int MB, int NB, int WT, int OCC, int NA>
+template <int WM, int WN, int MB, int NB, int WT, int OCC, int NA, bool TWO>
 struct Shape {
   static constexpr int bm = 32 * MB * WM, bn = 32 * NB * WN, threads = 64 * WM * WN;
   static GemmArgs numbered(const GemmArgs& a0, int* grid) {
@@ -376,7 +394,7 @@ struct Shape {
   static hipError_t start(const GemmArgs& a0, int parts, hipStream_t s) {
     int grid;
     const GemmArgs a = numbered(a0, &grid);
-    hipLaunchKernelGGL((k_gemm_cut<WM, WN, MB, NB, WT, EPI, SPLIT, false, OCC, NA>), dim3(grid, parts), dim3(threads), 0, s, a);
+    hipLaunchKernelGGL((k_gemm_cut<WM, WN, MB, NB, WT, EPI, SPLIT, false, OCC, NA, TWO>), dim3(grid, parts), dim3(threads), 0, s, a);
     return hipGetLastError();
   }
   static hipError_t launch(const GemmArgs& a, int epi, int parts, hipStream_t s) {
@@ -394,27 +412,31 @@ struct Shape {
     int grid;
     const GemmArgs a = numbered(a0, &grid);
     if (epi == GEMM_BIAS)
-      hipLaunchKernelGGL((k_gemm_cut<WM, WN, MB, NB, WT, GEMM_BIAS, 0, true, OCC, NA>), dim3(grid), dim3(threads), 0, s, a);
+      hipLaunchKernelGGL((k_gemm_cut<WM, WN, MB, NB, WT, GEMM_BIAS, 0, true, OCC, NA, TWO>), dim3(grid), dim3(threads), 0, s, a);
     else
-      hipLaunchKernelGGL((k_gemm_cut<WM, WN, MB, NB, WT, GEMM_SILU_PAIR, 0, true, OCC, NA>), dim3(grid), dim3(threads), 0, s, a);
+      hipLaunchKernelGGL((k_gemm_cut<WM, WN, MB, NB, WT, GEMM_SILU_PAIR, 0, true, OCC, NA, TWO>), dim3(grid), dim3(threads), 0, s, a);
     return hipGetLastError();
   }
 };
-// f32 rows: the cut of W costs as much as that of A, so that two wavefronts share an A row block and two
-// wavefronts per SIMD overlap; bf16 and int8 rows: a wavefront owns whole rows of the tile.
+// Two wavefronts share an A row block in the smallest tile; in the others a wavefront owns whole rows.  With two
+// sums two wavefronts per SIMD fit (128 x 128, f32 rows, one sum, eight wavefronts and four per SIMD:
+// 4096 x 6400 x 1600 467 us, here 457; bf16 rows, one sum, three per SIMD: 236 us, here 246).  f32 rows and no more
+// than one tile to a CU: eight wavefronts on it, two to a row block (1024 x 2304 x 768 37 us, four wavefronts 42).
 template <int WT>
-using Tile64x128 = Shape<2, 2, 1, 2, WT, 3, WT == 0 ? 4 : 2>;
+using Tile64x128 = Shape<2, 2, 1, 2, WT, 3, WT == 0 ? 4 : 2, true>;
 template <int WT>
-using Tile128x128 = std::conditional_t<WT == 0, Shape<4, 2, 1, 2, 0, 4, 4>, Shape<4, 1, 1, 4, WT, 3, 2>>;
-using Tile256x128 = Shape<8, 1, 1, 4, 0, 2, 2>;  // (f32 rows)
+using Tile128x128 = Shape<4, 1, 1, 4, WT, 2, 2, true>;
+using Tile128x128by8 = Shape<4, 2, 1, 2, 0, 2, 4, true>;  // (f32 rows)
+using Tile256x128 = Shape<8, 1, 1, 4, 0, 2, 2, true>;  // (f32 rows)
 template <int WT>
-using Tile128x256 = Shape<4, 1, 1, 8, WT, 2, 2>;  // (bf16 and int8 rows)
+using Tile128x256 = Shape<4, 1, 1, 8, WT, 2, 2, false>;  // (bf16 and int8 rows)
 
 template <int WT>
 hipError_t launch_tile(const GemmArgs& a, int epi, CutPlan p, hipStream_t s) {
   if (p.tile == CUT_64x128) return Tile64x128<WT>::launch(a, epi, p.parts, s);
   if (p.tile == CUT_128x128) return Tile128x128<WT>::launch(a, epi, p.parts, s);
   if constexpr (WT == 0) {
+    if (p.tile == CUT_128x128_8) return Tile128x128by8::launch(a, epi, p.parts, s);
     if (p.tile == CUT_256x128) return Tile256x128::launch(a, epi, p.parts, s);
   } else {
     if (p.tile == CUT_128x256) return Tile128x256<WT>::launch(a, epi, p.parts, s);
@@ -430,21 +452,21 @@ bool takes(const GemmArgs& a) {
 }
 
 // Time of a product in microseconds: a start, the stages of K at the pace of the CU with the most items,
-// and for a cut K the partial tiles' way through memory.  The constants are least squares over 144 shapes
-// (the four GPT-2 widths' projections at 96 to 2048 rows, W from HBM) with 1 to 8 parts each; they meet the
-// measured times within 6 %, and the plan of least predicted time is 2 % slower than the best measured
-// one in the mean.
+// and for a cut K the partial tiles' way through memory.  The constants are those of the
+// least regret over 416 shapes (the four GPT-2 widths' projections at 66 to 6000 rows, W from HBM) with 1 to 8
+// parts each: the plan of least predicted time is 1 % slower than the best measured one in the mean (2 %
+// for bf16 rows), 2 % over the shapes that were held out.
 struct Pace {
   float start, stage, more, part;  // start; a stage alone; each further item on the CU; a partly filled round
 };
 struct Reduce {
   float start, part, rest;  // a reduction's launch; a part and what is left per 10^6 outputs
 };
-// [storage][64 x 128, 128 x 128, 256 x 128]
-constexpr Pace kPace[3][3] = {
-    {{6.6f, 0.458f, 0.197f, 0.155f}, {6.6f, 0.553f, 0.440f, 0.144f}, {8.6f, 0.880f, 1.008f, 0.097f}},
-    {{7.3f, 0.385f, 0.246f, 0.074f}, {9.1f, 0.521f, 0.415f, 0.087f}, {}},
-    {{7.0f, 0.589f, 0.268f, 0.010f}, {8.5f, 0.742f, 0.368f, 0.000f}, {}}};
+// [storage][CutTile]
+constexpr Pace kPace[3][4] = {
+    {{5.2f, 0.468f, 0.160f, 0.197f}, {6.2f, 0.710f, 0.323f, 0.273f}, {9.3f, 1.027f, 1.661f, 0.249f}, {7.0f, 0.581f, 0.0f, 0.0f}},
+    {{3.4f, 0.461f, 0.204f, 0.131f}, {9.1f, 0.661f, 0.316f, 0.302f}, {}, {}},
+    {{7.9f, 0.518f, 0.234f, 0.139f}, {12.0f, 0.807f, 0.285f, 0.383f}, {}, {}}};
 constexpr Reduce kReduce[3] = {{2.8f, 1.30f, 0.5f}, {2.0f, 1.20f, 0.2f}, {5.0f, 1.55f, 0.4f}};
 
 }  // namespace
@@ -462,7 +484,7 @@ bool gemm_cut_plan(const GemmArgs& a, int num_cus, CutPlan* plan) {
   } else if (tiles64 < (wt == 1 ? 13 : 24)) {
     return false;  // (96 x 768 x 768, bf16: 9.9 against 11.3 us; 100 x 1280 x 1280, int8: 14.2 against 15.5)
   }
-  // Many tiles of 128 x 256 (bf16 and int8 rows; at least two to a CU): half the cuts of A per MFMA
+  // Many tiles of 128 x 256 (bf16 and int8 rows; 1.75 to a CU): half the cuts of A per MFMA
   // (8192 x 4800 x 1600 bf16: 378 against 388 us, int8 8192 x 1600 x 6400: 508 against 535).
   if (wt != 0 && (long)((a.M + 127) / 128) * ((a.N + 255) / 256) * 4 >= 7L * num_cus) {
     *plan = {CUT_128x256, 1};
@@ -474,11 +496,13 @@ bool gemm_cut_plan(const GemmArgs& a, int num_cus, CutPlan* plan) {
   const int most = a.ws && a.N % 4 == 0 ? (int)std::min<size_t>(std::min(8, a.K / 128), a.ws_floats / ((size_t)a.M * a.N)) : 1;
   const Reduce& red = kReduce[wt];
   float best = 0.0f;
-  for (int t = 0; t < (wt == 0 && a.M >= 512 ? 3 : 2); ++t) {
-    const int bm = 64 << t;
+  for (int t = CUT_64x128; t <= (wt == 0 ? CUT_128x128_8 : CUT_128x128); ++t) {
+    if (t == CUT_256x128 && a.M < 512) continue;
+    const int bm = t == CUT_64x128 ? 64 : t == CUT_256x128 ? 256 : 128;
     const long tiles = (long)((a.M + bm - 1) / bm) * ((a.N + 127) / 128);
     for (int parts = 1; parts <= std::max(1, most); ++parts) {
-      const long items = tiles * parts;
+      const long items = (tiles + 7) / 8 * 8 * parts;  // (as many to each XCD as the fullest one has)
+      if (t == CUT_128x128_8 && items > num_cus) continue;
       const float on_cu = (float)((items + num_cus - 1) / num_cus), round = std::max(0.0f, (float)items / (float)num_cus - 1.0f);
       const Pace& p = kPace[wt][t];
       const float us = p.start + (float)((stages + parts - 1) / parts) * (p.stage + (on_cu - 1.0f) * p.more + round * p.part) +
@@ -490,6 +514,16 @@ bool gemm_cut_plan(const GemmArgs& a, int num_cus, CutPlan* plan) {
     }
   }
   return true;
+}
+
+bool gemm_cut_forced(const GemmArgs& a, CutPlan* plan) {
+  const bool f32_rows = !a.w_bf16 && !a.w_scale;
+  const int bm = a.plan_bm, bn = a.plan_bn;
+  plan->parts = std::max(1, a.plan_parts);
+  plan->tile = bn == 256 ? CUT_128x256 : bm == 256 ? CUT_256x128 : a.plan_waves ? CUT_128x128_8 : bm == 64 ? CUT_64x128 : CUT_128x128;
+  if (plan->parts > std::max(1, a.K / 32)) return false;
+  if (a.plan_waves && (a.plan_waves != 8 || bm != 128 || bn != 128 || !f32_rows)) return false;
+  return (bn == 128 && (bm == 64 || bm == 128 || (bm == 256 && f32_rows))) || (bn == 256 && bm == 128 && !f32_rows);
 }
 
 hipError_t launch_gemm_cut(const GemmArgs& a, int epi, CutPlan plan, hipStream_t s) {

@@ -11,13 +11,16 @@ namespace pgk {
 
 // A product on the bf16 matrix cores (pg_gemm_cut.hip): the tile and the number of parts that K is
 // cut into (1: whole tiles; otherwise raw partial tiles to GemmArgs::ws, for a reduce kernel).
-enum CutTile : int { CUT_64x128 = 0, CUT_128x128 = 1, CUT_256x128 = 2, CUT_128x256 = 3 };
+// (CUT_128x128_8: by eight wavefronts)
+enum CutTile : int { CUT_64x128 = 0, CUT_128x128 = 1, CUT_256x128 = 2, CUT_128x128_8 = 3, CUT_128x256 = 4 };
 struct CutPlan {
   CutTile tile;
   int parts;
 };
 // False where these kernels do not take the product, or are not the faster ones for it.
 bool gemm_cut_plan(const GemmArgs& a, int num_cus, CutPlan* plan);
+// The plan that GemmArgs::plan_bm, plan_bn and plan_parts ask for; false where there is none such.
+bool gemm_cut_forced(const GemmArgs& a, CutPlan* plan);
 hipError_t launch_gemm_cut(const GemmArgs& a, int epi, CutPlan plan, hipStream_t s);
 // (bf16 rows; tiles of tile_rows = 64 or 128 rows)
 hipError_t launch_gemm_cut_grouped(const GemmArgs& a, int epi, int tile_rows, hipStream_t s);

@@ -1723,9 +1723,10 @@ hipError_t launch_gemm_form(const GemmArgs& a, int epi, int num_cus, hipStream_t
   }
   if (packed) return hipErrorInvalidValue;  // only the 32-row kernel knows the packed form
   // more rows: on the bf16 matrix cores where the planner finds enough tiles
-  if (a.plan_form == 0) {
+  if (a.plan_form == 0 || a.plan_form == 5) {
     CutPlan plan;
-    if (gemm_cut_plan(a, num_cus, &plan)) {
+    if (a.plan_form == 5 && !gemm_cut_forced(a, &plan)) return hipErrorInvalidValue;
+    if (a.plan_form == 5 || gemm_cut_plan(a, num_cus, &plan)) {
       const hipError_t e = launch_gemm_cut(a, epi, plan, s);
       return e != hipSuccess || plan.parts == 1 ? e : launch_splitk_reduce(a, epi, plan.parts, s, ln_done);
     }

@@ -99,3 +99,40 @@ class DeviceArray:
 
     def free(self):
         assert self.lib.pg_device_free(0, self.ptr) == 0
+
+
+def product_dev(x, w, bias=None, scales=None, tile=None, parts=1, ws_floats=0, packed=False):
+    """x [rows][k] times w [n][k] (f32, bf16 as uint16 or int8 with scales) through the library's testing entry:
+    a given tile (rows, columns and, where it is not the usual one, the number of wavefronts) and number of parts of
+    the bf16 matrix-core kernels, or (tile None) the planner's choice."""
+    import ctypes as C
+    from puppygrad_amd import _lib
+    lib = _lib.load()
+    f = lib.pg_testing_product_dev
+    u, v, i = C.c_uint64, C.c_void_p, C.c_int32
+    f.argtypes, f.restype = [i, v, v, u, u, u, v, i, v, v, v, i, i, i, i, i, v, u], C.c_int
+    (rows, k), n = x.shape, w.shape[0]
+    storage = {np.dtype(np.float32): _lib.PG_STORE_F32, np.dtype(np.uint16): _lib.PG_STORE_BF16,
+               np.dtype(np.int8): _lib.PG_STORE_INT8}[w.dtype]
+    stored = x
+    if packed:  # float4 of four columns of all 32 rows side by side
+        stored = np.zeros((k // 4, 32, 4), np.float32)
+        stored[:, :rows] = x.reshape(rows, k // 4, 4).transpose(1, 0, 2)
+    held = [DeviceArray(stored), DeviceArray(w, dtype=w.dtype), DeviceArray(np.full((rows, n), np.nan))]
+    scale = DeviceArray(scales) if scales is not None else None
+    b = DeviceArray(bias) if bias is not None else None
+    ws = DeviceArray(np.full(ws_floats, np.nan)) if ws_floats else None
+    held += [d for d in (scale, b, ws) if d is not None]
+    ptr = lambda d: d.ptr if d is not None else None
+    status = f(0, None, held[0].ptr, rows, k, n, held[1].ptr, storage, ptr(scale), ptr(b), held[2].ptr, int(packed),
+               *(tuple(tile or ()) + (0, 0, 0))[:3], parts, ptr(ws), ws_floats)
+    got = held[2].download()
+    for d in held:
+        d.free()
+    assert status == 0, lib.pg_last_error_message().decode()
+    return got
+
+
+def as_bf16(a):
+    """uint16 of a value that is a bf16 number already."""
+    return (np.ascontiguousarray(a, np.float32).view(np.uint32) >> 16).astype(np.uint16)

@@ -1,9 +1,10 @@
-"""Products of more than 64 rows on the bf16 matrix cores with f32 operands cut into three bf16 parts: every
-tile shape at its edges, one to a few stages of K, whole tiles and cut K, each storage of the weights."""
+"""Products of more than 64 rows, most of them on the bf16 matrix cores with f32 operands cut into three bf16
+parts: the planner's choice through the public entry points, and every tile of those kernels by name at its edges,
+with one to a few stages of K, whole and cut, against each storage of the weights."""
 import numpy as np
 import pytest
 
-from helpers import DeviceArray
+from helpers import DeviceArray, as_bf16, product_dev
 from puppygrad_amd import Gpt2Config, Gpt2HipConfig, Gpt2Model, _lib, synth
 
 pytestmark = pytest.mark.gpu
@@ -14,8 +15,8 @@ def ok(status):
 
 
 def within_f32_sums(got, x, w, b):
-    """|error| <= (K + 8) 2^-24 sum |x w| + 2^-23 |result|: f32 sums of K exact products in any order, products
-    right to 2^-25, the bias and (int8) the row scale each rounded once."""
+    """|error| <= (K + 8) 2^-24 sum |x w| + 2^-23 |result|: f32 sums of K products in any order, products
+    right to 2^-24, the bias and (int8) the row scale each rounded once."""
     x, w = x.astype(np.float64), w.astype(np.float64)
     want = x @ w.T + b
     bound = (x.shape[1] + 8) * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T) + 2.0 ** -23 * np.abs(want)
@@ -85,5 +86,113 @@ def test_values_past_bf16_meet_the_weights_as_in_f32(value):
     want = x[17].astype(np.float64) @ w.astype(np.float64).T
     np.testing.assert_array_equal(np.isnan(got[17]), np.isnan(want))
     np.testing.assert_array_equal(np.isposinf(got[17]), np.isposinf(want))
+    if np.isfinite(value):
+        np.testing.assert_allclose(got[17], want, rtol=1e-6)
+
+
+# ---- the tiles by name -------------------------------------------------------------------------
+F32_TILES, BYTE_TILES = [(64, 128), (128, 128), (128, 128, 8), (256, 128)], [(64, 128), (128, 128), (128, 256)]
+STORED = {"f32": F32_TILES, "bf16": BYTE_TILES, "int8": BYTE_TILES}
+TILES = [(s, t) for s, tiles in STORED.items() for t in tiles]
+
+
+def stored_rows(w, storage):
+    """(matrix as it is handed over, scales, the values it stands for)"""
+    if storage == "f32":
+        return w, None, w.astype(np.float64)
+    if storage == "bf16":
+        w = synth.round_bf16(w.reshape(-1)).reshape(w.shape)
+        return as_bf16(w), None, w.astype(np.float64)
+    q = np.random.default_rng(w.shape).integers(-127, 128, w.shape).astype(np.int8)
+    scales = np.abs(w[:, 0]) + np.float32(1e-3)
+    return q, scales, q * scales[:, None].astype(np.float64)
+
+
+# one stage of K and the first few (32 columns; f32 rows 16), ragged rows and columns
+@pytest.mark.parametrize("rows,k,n", [(65, 32, 129), (1, 64, 31), (127, 96, 257), (300, 160, 385), (257, 224, 640)])
+@pytest.mark.parametrize("storage,tile", TILES)
+def test_tiles_at_their_edges(storage, tile, rows, k, n):
+    for k in ((k, k - 16) if storage == "f32" else (k,)):
+        x, w, b = operands(rows, k, n)
+        stored, scales, values = stored_rows(w, storage)
+        within_f32_sums(product_dev(x, stored, b, scales, tile=tile), x, values, b)
+
+
+@pytest.mark.parametrize("parts", [2, 5, 8])
+@pytest.mark.parametrize("storage,tile", TILES)
+def test_tiles_with_k_cut(storage, tile, parts):
+    for rows, k, n in ((65, 256, 132), (200, 1088, 388)):
+        x, w, b = operands(rows, k, n)
+        stored, scales, values = stored_rows(w, storage)
+        within_f32_sums(product_dev(x, stored, b, scales, tile=tile, parts=parts, ws_floats=parts * rows * n), x, values, b)
+
+
+def one_sided(shape, seed, top):
+    """Values whose three bf16 parts are all of the value's sign and nearly as large as they can be: 2^e (1 + a 2^-7
+    + b 2^-8 + c 2^-17), so that every one of the products of parts adds to the same side."""
+    r = np.random.default_rng(seed)
+    m = 1.0 + r.integers(0, 32, shape) * 2.0 ** -7 + r.uniform(0.8, 0.99, shape) * 2.0 ** -8
+    x = (m * 2.0 ** r.integers(-top, top + 1, shape)).astype(np.float32)
+    return ((x.view(np.uint32) & ~np.uint32(0x7f)) | r.integers(0x30, 0x40, shape).astype(np.uint32)).view(np.float32)
+
+
+@pytest.mark.parametrize("storage,tile", TILES)
+def test_every_product_of_parts_counts(storage, tile):
+    """With one sign throughout, leaving out lo or mid mid would show as at least 2^-18 of the result; what the
+    six products leave out is 2^-24 of it, and each of the 2 K / 16 groups of hi hi products rounds the sum by at
+    most 2^-24, the sum of the small products the same of a 2^-7th, two last additions once each."""
+    for k in (32, 64):
+        x, w = one_sided((160, k), 1, 1), one_sided((200, k), 2, 1)
+        stored, scales, values = stored_rows(w, storage)
+        if storage == "int8":
+            stored = (64 + np.abs(stored) // 2).astype(np.int8)
+            values = stored * scales[:, None].astype(np.float64)
+        got = product_dev(x, stored, None, scales, tile=tile).astype(np.float64)
+        want = x.astype(np.float64) @ values.T
+        groups = k / 8 * (3 if tile == (128, 256) else 1)
+        assert (np.abs(got - want) <= (1 + groups * 1.05 + 3) * 2.0 ** -24 * want).all()
+
+
+@pytest.mark.parametrize("storage,tile", [c for c in TILES if c[1] != (128, 256)])
+def test_small_products_have_a_sum_of_their_own(storage, tile):
+    """The 2-norm of the error over the result's: K / 8 roundings of the running sum s, whose mean square is k / K
+    of the result's; a rounding is uniform in a unit of the last place, 2^-23 |s| times a square mean of 0.541.
+    With the small products in the same sum (twelve or six roundings per 16 columns instead of two) it is 2.4 or 1.7 times this."""
+    rows, k, n = 700, 1600, 520
+    r = np.random.default_rng(8)
+    x, w = r.standard_normal((rows, k)).astype(np.float32), r.standard_normal((n, k)).astype(np.float32)
+    stored, scales, values = stored_rows(w, storage)
+    want = x.astype(np.float64) @ values.T
+    err = product_dev(x, stored, None, scales, tile=tile) - want
+    expected = np.sqrt(k / 8 / 2 * 0.541 / 12) * 2.0 ** -23
+    assert np.linalg.norm(err) <= 1.25 * expected * np.linalg.norm(want)
+    # rows that are nearly alike: what their errors have in common is what the mean of independent ones is (three
+    # times that), and what the roundings downward leave
+    common = r.standard_normal(k)
+    x = (common + 0.05 * r.standard_normal((rows, k))).astype(np.float32)
+    want = x.astype(np.float64) @ values.T
+    err = product_dev(x, stored, None, scales, tile=tile) - want
+    size = np.sqrt((want ** 2).mean())
+    assert np.sqrt((err.mean(0) ** 2).mean()) <= (3 * expected / np.sqrt(rows) + 3e-8) * size
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, np.float32(3.4e38)])
+@pytest.mark.parametrize("storage,tile,parts", [(s, t, p) for s, t in TILES for p in (1, 3)])
+def test_tiles_with_values_past_bf16(storage, tile, parts, value):
+    x, w, b = operands(150, 192, 260)
+    x = np.clip(x, -10, 10)
+    w[:] = np.sign(w) * 0.25
+    stored, scales, values = stored_rows(w, storage)
+    if storage == "int8":
+        stored, scales = np.sign(stored) + (stored == 0).astype(np.int8), np.full(260, 0.25, np.float32)
+        values = stored * 0.25
+    x[17, 3] = value
+    got = product_dev(x, stored, b, scales, tile=tile, parts=parts, ws_floats=parts * 150 * 260 if parts > 1 else 0)
+    others = np.arange(150) != 17
+    within_f32_sums(got[others], x[others], values, b)
+    want = x[17].astype(np.float64) @ values.T
+    np.testing.assert_array_equal(np.isnan(got[17]), np.isnan(want))
+    np.testing.assert_array_equal(np.isposinf(got[17]), np.isposinf(want))
+    np.testing.assert_array_equal(np.isneginf(got[17]), np.isneginf(want))
     if np.isfinite(value):
         np.testing.assert_allclose(got[17], want, rtol=1e-6)
