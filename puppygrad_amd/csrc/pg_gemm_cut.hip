@@ -56,6 +56,16 @@ __device__ __forceinline__ void lds_dma16(const void* base, unsigned byte_off, u
       : "s"(lds), "v"(byte_off), "s"(base)
       : "memory", "m0");
 }
+// The same from an address per lane.
+__device__ __forceinline__ void lds_dma16_at(const void* from, unsigned lds) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off"
+      :
+      : "s"(lds), "v"(from)
+      : "memory", "m0");
+}
 // At most N loads of the wavefront in flight.
 template <int N>
 __device__ __forceinline__ void vm_wait() {
@@ -119,13 +129,15 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_cut(GemmArgs a) {
   // DMA: the lane's piece of each instruction.  A row's pieces lie permuted (`turn`), so that the 16
   // lanes that an LDS read serves in one go, 16 rows at the same piece, are on different banks; the
   // permutation is in the address that a lane loads from, as the instruction stores lane after lane.
-  unsigned aoff[IA], boff[IB ? IB : 1];
+  unsigned aoff[GROUPED ? 1 : IA], boff[IB ? IB : 1];
+  const char* arow[GROUPED ? IA : 1];  // (a grouped row lies anywhere in A, further than 32 bits reach)
 #pragma unroll
   for (int i = 0; i < IA; ++i) {
     const int at = (wave * IA + i) * 64 + lane, row = at / AP, slot = at % AP;
     const int turn = KT == 32 ? (row >> 1) & 7 : (row >> 2) & 3;
-    const int src = GROUPED ? group_row(a, m0 + row) : min(m0 + row, a.M - 1) - m0;
-    aoff[i] = (unsigned)src * (unsigned)a.lda * 4u + (unsigned)(slot ^ turn) * 16u;
+    const unsigned piece = (unsigned)(slot ^ turn) * 16u;
+    if constexpr (GROUPED) arow[i] = reinterpret_cast<const char*>(a.A + (size_t)group_row(a, m0 + row) * a.lda) + piece;
+    else aoff[i] = (unsigned)(min(m0 + row, a.M - 1) - m0) * (unsigned)a.lda * 4u + piece;
   }
   constexpr int WBYTES = WT == 0 ? 4 : WT == 1 ? 2 : 1;
 #pragma unroll
@@ -134,15 +146,18 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_cut(GemmArgs a) {
     const int piece = slot ^ ((row >> 2) & 3);
     boff[i] = (unsigned)(min(n0 + row, a.N - 1) - n0) * (unsigned)a.K * WBYTES + (unsigned)piece * 16u;
   }
-  const char* Ab = reinterpret_cast<const char*>(a.A + (GROUPED ? (size_t)0 : (size_t)m0 * a.lda) + (size_t)kt0 * KT);
+  const char* Ab = reinterpret_cast<const char*>(a.A + (size_t)m0 * a.lda + (size_t)kt0 * KT);
   const char* Wb = reinterpret_cast<const char*>(a.W) +
                    (((size_t)n0 + (GROUPED ? (size_t)group * a.N : 0)) * a.K + (size_t)kt0 * KT) * WBYTES;
   const unsigned as_lds = (unsigned)(size_t)(lds_ptr)(void*)&As[0][0], bs_lds = (unsigned)(size_t)(lds_ptr)(void*)&Bs[0][0][0];
   auto dma = [&](int t, int buf) __attribute__((always_inline)) {
     const size_t k = (size_t)min(t, T - 1) * KT;
 #pragma unroll
-    for (int i = 0; i < IA; ++i)
-      lds_dma16(Ab + k * 4, aoff[i], as_lds + (unsigned)(buf * BM * AP * 16 + (wave * IA + i) * 1024));
+    for (int i = 0; i < IA; ++i) {
+      const unsigned to = as_lds + (unsigned)(buf * BM * AP * 16 + (wave * IA + i) * 1024);
+      if constexpr (GROUPED) lds_dma16_at(arow[i] + k * 4, to);
+      else lds_dma16(Ab + k * 4, aoff[i], to);
+    }
 #pragma unroll
     for (int i = 0; i < IB; ++i)
       lds_dma16(Wb + k * WBYTES, boff[i], bs_lds + (unsigned)(buf * BN * BP * 16 + (wave * IB + i) * 1024));
@@ -534,8 +549,7 @@ hipError_t launch_gemm_cut(const GemmArgs& a, int epi, CutPlan plan, hipStream_t
 }
 
 hipError_t launch_gemm_cut_grouped(const GemmArgs& a, int epi, int tile_rows, hipStream_t s) {
-  // (a row of A lies anywhere among at most M: 32-bit offsets from A)
-  if (!takes(a) || !a.w_bf16 || (size_t)a.M * a.lda * 4 >= ((size_t)1 << 32)) return hipErrorInvalidValue;
+  if (!takes(a) || !a.w_bf16) return hipErrorInvalidValue;
   if (tile_rows == 64) return Tile64x128<1>::launch_grouped(a, epi, s);
   if (tile_rows == 128) return Tile128x128<1>::launch_grouped(a, epi, s);
   return hipErrorInvalidValue;

@@ -136,3 +136,25 @@ def product_dev(x, w, bias=None, scales=None, tile=None, parts=1, ws_floats=0, p
 def as_bf16(a):
     """uint16 of a value that is a bf16 number already."""
     return (np.ascontiguousarray(a, np.float32).view(np.uint32) >> 16).astype(np.uint16)
+
+
+def grouped_dev(x, rows, w, group_tile, group_rows, tile_rows, silu_pair=False):
+    """launch_gemm_grouped through the library's testing entry: x a device pointer to rows of w.shape[2] values, w
+    [groups][n][k] (f32 or bf16 as uint16), `rows` slots with their padding."""
+    import ctypes as C
+    from puppygrad_amd import _lib
+    lib = _lib.load()
+    f = lib.pg_testing_grouped_dev
+    u, v, i = C.c_uint64, C.c_void_p, C.c_int32
+    f.argtypes, f.restype = [i, v, v, u, u, u, v, i, i, v, i, v, v], C.c_int
+    _, n, k = w.shape
+    dw, tiles = DeviceArray(w, dtype=w.dtype), DeviceArray(group_tile, dtype=np.int32)
+    slots = DeviceArray(group_rows, dtype=np.int32) if group_rows is not None else None
+    out = DeviceArray(np.full((rows, n // 2 if silu_pair else n), np.nan))
+    status = f(0, None, x, rows, k, n, dw.ptr, _lib.PG_STORE_BF16 if w.dtype == np.uint16 else _lib.PG_STORE_F32,
+               int(silu_pair), out.ptr, tile_rows, tiles.ptr, slots.ptr if slots else None)
+    got = out.download()
+    for d in (dw, tiles, out) + ((slots,) if slots else ()):
+        d.free()
+    assert status == 0, lib.pg_last_error_message().decode()
+    return got

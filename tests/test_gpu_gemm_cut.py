@@ -1,10 +1,12 @@
 """Products of more than 64 rows, most of them on the bf16 matrix cores with f32 operands cut into three bf16
 parts: the planner's choice through the public entry points, and every tile of those kernels by name at its edges,
 with one to a few stages of K, whole and cut, against each storage of the weights."""
+import ctypes
+
 import numpy as np
 import pytest
 
-from helpers import DeviceArray, as_bf16, product_dev
+from helpers import DeviceArray, as_bf16, grouped_dev, product_dev
 from puppygrad_amd import Gpt2Config, Gpt2HipConfig, Gpt2Model, _lib, synth
 
 pytestmark = pytest.mark.gpu
@@ -196,3 +198,30 @@ def test_tiles_with_values_past_bf16(storage, tile, parts, value):
     np.testing.assert_array_equal(np.isneginf(got[17]), np.isneginf(want))
     if np.isfinite(value):
         np.testing.assert_allclose(got[17], want, rtol=1e-6)
+
+
+@pytest.mark.parametrize("storage,tile_rows", [("bf16", 32), ("bf16", 64), ("bf16", 128), ("f32", 32), ("f32", 64)])
+def test_grouped_rows_past_four_gigabytes(storage, tile_rows):
+    """Experts' slots (and the rows they take) whose offsets need more than 32 bits: only the last two tiles hold any."""
+    lib, k, n = _lib.load(), 16000, 96
+    slots = (1 << 32) // (4 * k) // 128 * 128 + 384
+    first = slots - 2 * tile_rows
+    assert first * k * 4 >= 1 << 32
+    x, w, _ = operands(2 * tile_rows, k, 2 * n)
+    stored, _, values = stored_rows(w, storage)
+    a = ctypes.c_void_p()
+    ok(lib.pg_device_alloc(0, slots * k * 4, ctypes.byref(a)))
+    try:
+        ok(lib.pg_device_upload(0, ctypes.c_void_p(a.value + first * k * 4), x.ctypes.data_as(ctypes.c_void_p), x.nbytes))
+        tiles = np.full(slots // tile_rows, -1, np.int32)
+        tiles[-2:] = (1, 0)
+        got = grouped_dev(a, slots, stored.reshape(2, n, k), tiles, None, tile_rows)[first:]
+        within_f32_sums(got[:tile_rows], x[:tile_rows], values[n:], 0.0)
+        within_f32_sums(got[tile_rows:], x[tile_rows:], values[:n], 0.0)
+        # few slots that take those rows, in another order
+        order = np.random.default_rng(3).permutation(2 * tile_rows)
+        got = grouped_dev(a, 2 * tile_rows, stored.reshape(2, n, k), [0, 1], first + order, tile_rows)
+        within_f32_sums(got[:tile_rows], x[order[:tile_rows]], values[:n], 0.0)
+        within_f32_sums(got[tile_rows:], x[order[tile_rows:]], values[n:], 0.0)
+    finally:
+        ok(lib.pg_device_free(0, a))
