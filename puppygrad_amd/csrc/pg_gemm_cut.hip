@@ -20,7 +20,8 @@
 // so).  Tiles that have the registers therefore keep two sums, hi hi (bf16 and int8 rows: hi w) and all that
 // is smaller, added at the end (TWO): the same logits 4.1e-7; 895 x 4800 x 1600 against f64 2.4e-7 of the
 // result for f32 rows (one sum 6.2e-7, f32 cores 7.1e-7) and 2.4e-7 for bf16 rows (one sum 4.3e-7).  The
-// 128 x 256 tile has no room for a second sum: as precise as one sum, 4.3e-7.
+// 128 x 256 tile has no room for a second sum, and where there are more than two 128 x 128 tiles to a CU the third
+// one there is worth more: 4.3e-7, as such products always had.
 //
 // What bounds it: power.  With all matrix cores at work the clock goes down to 1.7 to 2.0 GHz (a plain bf16
 // product of the library reaches 1354 of 2500 TFLOP/s on this card), and what else the CU moves is paid
@@ -437,12 +438,16 @@ struct Shape {
 // sums two wavefronts per SIMD fit (128 x 128, f32 rows, one sum, eight wavefronts and four per SIMD:
 // 4096 x 6400 x 1600 467 us, here 457; bf16 rows, one sum, three per SIMD: 236 us, here 246).  f32 rows and no more
 // than one tile to a CU: eight wavefronts on it, two to a row block (1024 x 2304 x 768 37 us, four wavefronts 42).
+// bf16 and int8 rows and more than two 128 x 128 tiles to a CU: one sum, so that three of them are there (3200 x 3840 x
+// 1280 85 us, two sums 100; int8 92, 113); so many tiles have always been whole and had one sum.
 template <int WT>
 using Tile64x128 = Shape<2, 2, 1, 2, WT, 3, WT == 0 ? 4 : 2, true>;
 template <int WT>
 using Tile128x128 = Shape<4, 1, 1, 4, WT, 2, 2, true>;
 using Tile128x128by8 = Shape<4, 2, 1, 2, 0, 2, 4, true>;  // (f32 rows)
 using Tile256x128 = Shape<8, 1, 1, 4, 0, 2, 2, true>;  // (f32 rows)
+template <int WT>
+using Tile128x128by3 = Shape<4, 1, 1, 4, WT, 3, 2, false>;  // (bf16 and int8 rows)
 template <int WT>
 using Tile128x256 = Shape<4, 1, 1, 8, WT, 2, 2, false>;  // (bf16 and int8 rows)
 
@@ -454,6 +459,7 @@ hipError_t launch_tile(const GemmArgs& a, int epi, CutPlan p, hipStream_t s) {
     if (p.tile == CUT_128x128_8) return Tile128x128by8::launch(a, epi, p.parts, s);
     if (p.tile == CUT_256x128) return Tile256x128::launch(a, epi, p.parts, s);
   } else {
+    if (p.tile == CUT_128x128_3) return Tile128x128by3<WT>::launch(a, epi, p.parts, s);
     if (p.tile == CUT_128x256) return Tile128x256<WT>::launch(a, epi, p.parts, s);
   }
   return hipErrorInvalidValue;
@@ -478,10 +484,10 @@ struct Reduce {
   float start, part, rest;  // a reduction's launch; a part and what is left per 10^6 outputs
 };
 // [storage][CutTile]
-constexpr Pace kPace[3][4] = {
-    {{5.2f, 0.468f, 0.160f, 0.197f}, {6.2f, 0.710f, 0.323f, 0.273f}, {9.3f, 1.027f, 1.661f, 0.249f}, {7.0f, 0.581f, 0.0f, 0.0f}},
-    {{3.4f, 0.461f, 0.204f, 0.131f}, {9.1f, 0.661f, 0.316f, 0.302f}, {}, {}},
-    {{7.9f, 0.518f, 0.234f, 0.139f}, {12.0f, 0.807f, 0.285f, 0.383f}, {}, {}}};
+constexpr Pace kPace[3][5] = {
+    {{5.2f, 0.468f, 0.160f, 0.197f}, {6.2f, 0.710f, 0.323f, 0.273f}, {9.3f, 1.027f, 1.661f, 0.249f}, {7.0f, 0.581f, 0.0f, 0.0f}, {}},
+    {{3.4f, 0.461f, 0.204f, 0.131f}, {9.1f, 0.661f, 0.316f, 0.302f}, {}, {}, {12.3f, 0.403f, 0.404f, 0.311f}},
+    {{7.9f, 0.518f, 0.234f, 0.139f}, {12.0f, 0.807f, 0.285f, 0.383f}, {}, {}, {14.0f, 0.101f, 0.630f, 0.288f}}};
 constexpr Reduce kReduce[3] = {{2.8f, 1.30f, 0.5f}, {2.0f, 1.20f, 0.2f}, {5.0f, 1.55f, 0.4f}};
 
 }  // namespace
@@ -511,13 +517,14 @@ bool gemm_cut_plan(const GemmArgs& a, int num_cus, CutPlan* plan) {
   const int most = a.ws && a.N % 4 == 0 ? (int)std::min<size_t>(std::min(8, a.K / 128), a.ws_floats / ((size_t)a.M * a.N)) : 1;
   const Reduce& red = kReduce[wt];
   float best = 0.0f;
-  for (int t = CUT_64x128; t <= (wt == 0 ? CUT_128x128_8 : CUT_128x128); ++t) {
-    if (t == CUT_256x128 && a.M < 512) continue;
+  for (int t = CUT_64x128; t <= CUT_128x128_3; ++t) {
+    if (wt == 0 ? t == CUT_128x128_3 || (t == CUT_256x128 && a.M < 512) : t == CUT_256x128 || t == CUT_128x128_8) continue;
     const int bm = t == CUT_64x128 ? 64 : t == CUT_256x128 ? 256 : 128;
     const long tiles = (long)((a.M + bm - 1) / bm) * ((a.N + 127) / 128);
     for (int parts = 1; parts <= std::max(1, most); ++parts) {
       const long items = (tiles + 7) / 8 * 8 * parts;  // (as many to each XCD as the fullest one has)
       if (t == CUT_128x128_8 && items > num_cus) continue;
+      if (wt != 0 && t != CUT_64x128 && (t == CUT_128x128_3) != (parts == 1 && items > 2 * num_cus)) continue;
       const float on_cu = (float)((items + num_cus - 1) / num_cus), round = std::max(0.0f, (float)items / (float)num_cus - 1.0f);
       const Pace& p = kPace[wt][t];
       const float us = p.start + (float)((stages + parts - 1) / parts) * (p.stage + (on_cu - 1.0f) * p.more + round * p.part) +
@@ -535,9 +542,13 @@ bool gemm_cut_forced(const GemmArgs& a, CutPlan* plan) {
   const bool f32_rows = !a.w_bf16 && !a.w_scale;
   const int bm = a.plan_bm, bn = a.plan_bn;
   plan->parts = std::max(1, a.plan_parts);
-  plan->tile = bn == 256 ? CUT_128x256 : bm == 256 ? CUT_256x128 : a.plan_waves ? CUT_128x128_8 : bm == 64 ? CUT_64x128 : CUT_128x128;
+  plan->tile = bn == 256    ? CUT_128x256
+               : bm == 256  ? CUT_256x128
+               : bm == 64   ? CUT_64x128
+               : a.plan_alt ? (f32_rows ? CUT_128x128_8 : CUT_128x128_3)
+                            : CUT_128x128;
   if (plan->parts > std::max(1, a.K / 32)) return false;
-  if (a.plan_waves && (a.plan_waves != 8 || bm != 128 || bn != 128 || !f32_rows)) return false;
+  if (a.plan_alt && (bm != 128 || bn != 128)) return false;
   return (bn == 128 && (bm == 64 || bm == 128 || (bm == 256 && f32_rows))) || (bn == 256 && bm == 128 && !f32_rows);
 }
 
@@ -551,7 +562,7 @@ hipError_t launch_gemm_cut(const GemmArgs& a, int epi, CutPlan plan, hipStream_t
 hipError_t launch_gemm_cut_grouped(const GemmArgs& a, int epi, int tile_rows, hipStream_t s) {
   if (!takes(a) || !a.w_bf16) return hipErrorInvalidValue;
   if (tile_rows == 64) return Tile64x128<1>::launch_grouped(a, epi, s);
-  if (tile_rows == 128) return Tile128x128<1>::launch_grouped(a, epi, s);
+  if (tile_rows == 128) return Tile128x128by3<1>::launch_grouped(a, epi, s);  // (many rows: many tiles)
   return hipErrorInvalidValue;
 }
 

@@ -11,8 +11,8 @@ namespace pgk {
 
 // A product on the bf16 matrix cores (pg_gemm_cut.hip): the tile and the number of parts that K is
 // cut into (1: whole tiles; otherwise raw partial tiles to GemmArgs::ws, for a reduce kernel).
-// (CUT_128x128_8: by eight wavefronts)
-enum CutTile : int { CUT_64x128 = 0, CUT_128x128 = 1, CUT_256x128 = 2, CUT_128x128_8 = 3, CUT_128x256 = 4 };
+// (CUT_128x128_8: by eight wavefronts; CUT_128x128_3: three of them on a CU)
+enum CutTile : int { CUT_64x128 = 0, CUT_128x128 = 1, CUT_256x128 = 2, CUT_128x128_8 = 3, CUT_128x128_3 = 4, CUT_128x256 = 5 };
 struct CutPlan {
   CutTile tile;
   int parts;

@@ -265,7 +265,7 @@ struct GemmArgs {
   // shape, form (1 whole tiles, 2 every tile cut along K into plan_parts, 3 only the last
   // partial round of tiles cut, 4 the 32-row kernel, 5 the bf16 matrix cores of pg_gemm_cut.hip).
   int plan_bm = 0, plan_bn = 0, plan_form = 0, plan_parts = 0;
-  int plan_waves = 0;  // form 5: wavefronts of the tile (0: as many as it has where more than one fits a CU)
+  int plan_alt = 0;  // form 5, 128 x 128: 1 by eight wavefronts (f32 rows) or with one sum, three to a CU (the others)
   int plan_band = 0;  // band height of the tile numbering (0: chosen by the launcher)
   int plan_bk16 = 0;  // 1: k-tiles of 16 columns also where K would allow 32
   const int *group_tile = nullptr, *group_rows = nullptr;  // launch_gemm_grouped

@@ -347,12 +347,13 @@ pg_status pg_op_quantized_dense_dev(int32_t device, void* stream, const float* x
 
 // ---- for the tests of the product kernels, no part of the C interface: a product in a given form ------------
 
-// tile_rows x tile_cols of pg_gemm_cut.hip (by tile_waves wavefronts, 0: the usual) with K in `parts` parts, or (tile_rows 0) as the planner has it; ws as
-// GemmArgs::ws.  storage: pg_weight_storage's values.  packed: x is in the packed form of 32 rows.
+// tile_rows x tile_cols of pg_gemm_cut.hip (tile_alt: GemmArgs::plan_alt) with K in `parts` parts, or (tile_rows 0)
+// as the planner has it; ws as GemmArgs::ws.  storage: pg_weight_storage's values.  packed: x is in the packed
+// form of 32 rows.
 pg_status pg_testing_product_dev(int32_t device, void* stream, const float* x, uint64_t rows, uint64_t in_f,
                                  uint64_t out_f, const void* weight, int32_t storage, const float* scales,
                                  const float* bias, float* out, int32_t packed, int32_t tile_rows,
-                                 int32_t tile_cols, int32_t tile_waves, int32_t parts, float* ws, uint64_t ws_floats) {
+                                 int32_t tile_cols, int32_t tile_alt, int32_t parts, float* ws, uint64_t ws_floats) {
   if (!x || !weight || !out || (storage == PG_STORE_INT8) != (scales != nullptr))
     return pgh::fail(PG_INVALID_INPUT, "null argument");
   if (rows == 0 || rows > (1u << 20) || in_f == 0 || in_f > pgh::kMaxStagedFloats || out_f == 0 || out_f > (1u << 24))
@@ -363,7 +364,7 @@ pg_status pg_testing_product_dev(int32_t device, void* stream, const float* x, u
   a.A = x; a.W = static_cast<const float*>(weight); a.w_bf16 = storage == PG_STORE_BF16; a.w_scale = scales;
   a.bias = bias; a.C = out; a.M = (int)rows; a.N = (int)out_f; a.K = (int)in_f; a.lda = (int)in_f; a.ldc = (int)out_f;
   a.ws = ws; a.ws_floats = ws_floats; a.a_packed = packed;
-  if (tile_rows) a.plan_form = 5, a.plan_bm = tile_rows, a.plan_bn = tile_cols, a.plan_waves = tile_waves, a.plan_parts = parts;
+  if (tile_rows) a.plan_form = 5, a.plan_bm = tile_rows, a.plan_bn = tile_cols, a.plan_alt = tile_alt, a.plan_parts = parts;
   int cus = 0;
   PG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   PG_HIP(pgk::launch_gemm(a, pgk::GEMM_BIAS, cus, static_cast<hipStream_t>(stream)));

@@ -103,8 +103,8 @@ class DeviceArray:
 
 def product_dev(x, w, bias=None, scales=None, tile=None, parts=1, ws_floats=0, packed=False):
     """x [rows][k] times w [n][k] (f32, bf16 as uint16 or int8 with scales) through the library's testing entry:
-    a given tile (rows, columns and, where it is not the usual one, the number of wavefronts) and number of parts of
-    the bf16 matrix-core kernels, or (tile None) the planner's choice."""
+    a given tile (rows, columns and 1 for the other form of that size) and number of parts of the bf16
+    matrix-core kernels, or (tile None) the planner's choice."""
     import ctypes as C
     from puppygrad_amd import _lib
     lib = _lib.load()

@@ -93,9 +93,10 @@ def test_values_past_bf16_meet_the_weights_as_in_f32(value):
 
 
 # ---- the tiles by name -------------------------------------------------------------------------
-F32_TILES, BYTE_TILES = [(64, 128), (128, 128), (128, 128, 8), (256, 128)], [(64, 128), (128, 128), (128, 256)]
+F32_TILES, BYTE_TILES = [(64, 128), (128, 128), (128, 128, 1), (256, 128)], [(64, 128), (128, 128), (128, 128, 1), (128, 256)]
 STORED = {"f32": F32_TILES, "bf16": BYTE_TILES, "int8": BYTE_TILES}
 TILES = [(s, t) for s, tiles in STORED.items() for t in tiles]
+ONE_SUM = [(s, t) for s in ("bf16", "int8") for t in ((128, 128, 1), (128, 256))]
 
 
 def stored_rows(w, storage):
@@ -151,11 +152,11 @@ def test_every_product_of_parts_counts(storage, tile):
             values = stored * scales[:, None].astype(np.float64)
         got = product_dev(x, stored, None, scales, tile=tile).astype(np.float64)
         want = x.astype(np.float64) @ values.T
-        groups = k / 8 * (3 if tile == (128, 256) else 1)
+        groups = k / 8 * (3 if (storage, tile) in ONE_SUM else 1)
         assert (np.abs(got - want) <= (1 + groups * 1.05 + 3) * 2.0 ** -24 * want).all()
 
 
-@pytest.mark.parametrize("storage,tile", [c for c in TILES if c[1] != (128, 256)])
+@pytest.mark.parametrize("storage,tile", [c for c in TILES if c not in ONE_SUM])
 def test_small_products_have_a_sum_of_their_own(storage, tile):
     """The 2-norm of the error over the result's: K / 8 roundings of the running sum s, whose mean square is k / K
     of the result's; a rounding is uniform in a unit of the last place, 2^-23 |s| times a square mean of 0.541.
