@@ -882,8 +882,9 @@ __global__ __launch_bounds__(512) void k_gemm_rows32(GemmArgs a) {
     float sum = red_at(0, b, nl);
 #pragma unroll
     for (int w = 1; w < 8; ++w) sum += red_at(w, b, nl);
-    if (WT != 0 && sum != sum) {
-      // (an input that is infinite as bf16 makes its parts NaN: the block's columns in f32 arithmetic)
+    if (WT != 0 && !(fabsf(sum) < INFINITY)) {
+      // An input that is infinite as bf16 makes its parts NaN, and a first part rounded up may give an infinite
+      // product where the value's own is finite: the block's columns in f32 arithmetic.
       sum = 0.0f;
       const char* wr = wg + (size_t)n * rowbytes;
       for (int k = 0; k < a.K; ++k) {
