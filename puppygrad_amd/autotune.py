@@ -272,7 +272,7 @@ def main(argv: Optional[Sequence[str]] = None) -> int:
     ap.add_argument("--attn-item-keys", default="128,256")
     ap.add_argument("--attn-blocks-per-cu", default="4")
     ap.add_argument("--gemm-split-items-per-cu", default="3")
-    ap.add_argument("--gemm-b9-min-rows", default="0", help="0: the planner's rule")
+    ap.add_argument("--gemm-b9-min-rows", default="0", help="0: the built-in 65")
     ap.add_argument("--seq-gemm-min-tokens", default="0", help="0: the built-in 4")
     ap.add_argument("--score", choices=sorted(SCORES), default="decode",
                     help="what ranks the candidates (the reference: decode)")

@@ -493,7 +493,7 @@ constexpr Reduce kReduce[3] = {{2.8f, 1.30f, 0.5f}, {2.0f, 1.20f, 0.2f}, {5.0f, 
 }  // namespace
 
 bool gemm_cut_plan(const GemmArgs& a, int num_cus, CutPlan* plan) {
-  if (!takes(a) || a.M <= 64) return false;  // (37 x 5120 x 1280, int8: a tile of 64 rows is half padding)
+  if (!takes(a) || a.M < kCutMinRows) return false;  // (37 x 5120 x 1280, int8: a tile of 64 rows is half padding)
   const int wt = a.w_scale ? 2 : a.w_bf16 ? 1 : 0;
   const long tiles64 = (long)((a.M + 63) / 64) * ((a.N + 127) / 128);
   if (wt == 0) {
@@ -501,7 +501,7 @@ bool gemm_cut_plan(const GemmArgs& a, int num_cus, CutPlan* plan) {
     // 1280 x 5120: 30.9 against 32.5), unless K is deep enough and the tiles are many (66 x 4800 x 1600: 28
     // against 23 us); from there on the other way round (256 x 4096 x 1024: 30.7 against 24.1).
     const double mnk = (double)a.M * a.N * a.K;
-    if (a.b9_min_rows ? a.M < a.b9_min_rows : !(tiles64 >= 20 && mnk >= 0.85e9) && !(tiles64 >= 60 && a.K >= 1280)) return false;
+    if (a.M < a.b9_min_rows || (!(tiles64 >= 20 && mnk >= 0.85e9) && !(tiles64 >= 60 && a.K >= 1280))) return false;
   } else if (tiles64 < (wt == 1 ? 13 : 24)) {
     return false;  // (96 x 768 x 768, bf16: 9.9 against 11.3 us; 100 x 1280 x 1280, int8: 14.2 against 15.5)
   }

@@ -978,7 +978,7 @@ pg_status pg_gpt2_create(const pg_gpt2_config* config, const pg_gpt2_weights_vie
   m->item_keys_auto = opts.attn_item_keys == 0;
   m->attn_blocks_per_cu = opts.attn_blocks_per_cu ? (int)opts.attn_blocks_per_cu : 4;
   m->gemm_split_items = opts.gemm_split_items_per_cu ? (int)opts.gemm_split_items_per_cu : 3;
-  m->gemm_b9_min_rows = (int)std::min(opts.gemm_b9_min_rows, 0x7fffffffu);
+  m->gemm_b9_min_rows = opts.gemm_b9_min_rows ? (int)std::min(opts.gemm_b9_min_rows, 0x7fffffffu) : pgk::kCutMinRows;
   m->seq_gemm_min_tokens = opts.seq_gemm_min_tokens ? opts.seq_gemm_min_tokens : 4;
   hipDeviceProp_t prop;
   PG_HIP(hipGetDeviceProperties(&prop, opts.device));
@@ -1185,7 +1185,7 @@ pg_status pg_model_describe(const pg_model* m, char* dst, size_t cap) {
                   "gemm_split_items_per_cu=%d, gemm_b9_min_rows=%d)",
                   m->device, m->num_cus, m->w_bf16 ? "bf16" : "f32", pgh::architecture_of(m),
                   m->opts.decode_path == PG_DECODE_KERNELS ? "kernels" : "graph", m->gemm_split_items,
-                  m->gemm_b9_min_rows ? m->gemm_b9_min_rows : 1024);
+                  m->gemm_b9_min_rows);
     return PG_OK;
   }
   std::snprintf(dst, cap,
@@ -1194,7 +1194,7 @@ pg_status pg_model_describe(const pg_model* m, char* dst, size_t cap) {
                 "seq_gemm_min_tokens=%zu)",
                 m->device, m->num_cus, m->w_bf16 ? "bf16" : m->w_i8 ? "int8" : "f32",
                 m->persistent ? "persistent" : "kernels", m->item_keys, m->attn_blocks_per_cu,
-                m->gemm_split_items, m->gemm_b9_min_rows ? m->gemm_b9_min_rows : 1024, m->seq_gemm_min_tokens);
+                m->gemm_split_items, m->gemm_b9_min_rows, m->seq_gemm_min_tokens);
   return PG_OK;
 }
 

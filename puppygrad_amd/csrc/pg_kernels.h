@@ -216,6 +216,7 @@ enum GemmEpilogue : int {
 };
 // C[M,N] = epilogue(A[M,K] . W[N,K]^T + bias): A rows lda floats apart, C (and resid)
 // rows ldc apart, W dense [N][K]; bias may be nullptr.
+constexpr int kCutMinRows = 65;  // (fewer: the 32-row kernel)
 struct GemmArgs {
   int w_bf16 = 0;  // W holds bf16 values
   const float* w_scale = nullptr;  // != nullptr: W holds int8 values, w_scale[n] scales row n
@@ -258,9 +259,9 @@ struct GemmArgs {
   // Tunable: a GEMM whose M x N leaves CUs idle is cut along K into about this many work items
   // per CU (gemm_split_parts).
   int split_items_per_cu = 3;
-  // Tunable: f32 rows go to the bf16 matrix cores (pg_gemm_cut.hip) from this many input rows on (0: the
-  // planner's rule).
-  int b9_min_rows = 0;
+  // Tunable: f32 rows go to the bf16 matrix cores (pg_gemm_cut.hip) from this many input rows on, where the
+  // planner finds enough tiles (kCutMinRows: wherever it does).
+  int b9_min_rows = kCutMinRows;
   // A forced plan for the tile forms (benchmarks and tests; 0 = the planner chooses): tile
   // shape, form (1 whole tiles, 2 every tile cut along K into plan_parts, 3 only the last
   // partial round of tiles cut, 4 the 32-row kernel, 5 the bf16 matrix cores of pg_gemm_cut.hip).

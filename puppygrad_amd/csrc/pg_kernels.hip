@@ -54,7 +54,6 @@ __device__ __forceinline__ float block_max(float v, float* red) {
   return t;
 }
 
-// gelu_in_place (cpu.rs:145-150).
 // layer_norm_in_place (cpu.rs:119-143) on a vector already staged in LDS:
 // two-pass mean / biased variance, eps inside the sqrt.
 __device__ __forceinline__ void ln_in_lds(float* sx, int K, const float* g, const float* b,

@@ -1714,7 +1714,7 @@ hipError_t launch_gemm_form(const GemmArgs& a, int epi, int num_cus, hipStream_t
     if (packed) return hipErrorInvalidValue;
     return a.w_bf16 ? launch_gemv_rows<true>(a, epi, num_cus, s) : launch_gemv_rows<false>(a, epi, num_cus, s);
   }
-  // other batches of up to 32 rows (64, f32 and bf16 rows): 32 rows of W per block on the matrix cores
+  // other batches of up to 64 rows (packed: 32): 32 rows of W per block on the matrix cores
   if (a.plan_form == 0 || a.plan_form == 4) {
     if (const int rp = gemm_rows32_parts(a, num_cus))
       return a.w_scale  ? launch_gemm_rows32<2>(a, epi, rp, num_cus, s, ln_done)

@@ -796,7 +796,7 @@ pg_status stack_create(const std::string& config_path, const Json& config, const
   model->opts = opts;
   model->w_bf16 = opts.weight_storage == PG_STORE_BF16 ? 1 : 0;
   model->gemm_split_items = opts.gemm_split_items_per_cu ? (int)opts.gemm_split_items_per_cu : 3;
-  model->gemm_b9_min_rows = (int)std::min(opts.gemm_b9_min_rows, 0x7fffffffu);
+  model->gemm_b9_min_rows = opts.gemm_b9_min_rows ? (int)std::min(opts.gemm_b9_min_rows, 0x7fffffffu) : pgk::kCutMinRows;
   hipDeviceProp_t prop;
   PG_HIP(hipGetDeviceProperties(&prop, opts.device));
   model->num_cus = prop.multiProcessorCount;

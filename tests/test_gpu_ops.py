@@ -50,16 +50,13 @@ def test_dense_matches_oracle(rows, k, n):
                                       (1024, 1024, 4096), (1024, 4096, 1024), (1100, 1600, 1600)])
 def test_dense_many_rows_uses_mfma_gemm(rows, k, n):
     # rows >= 16 and K % 16 == 0 take the MFMA GEMM; tails in M and N are exercised.
-    # (64, 6400, 1600), (16, 1024, 3072) and (32, 1600, 6400) cut the whole K range into
-    # parts; (512, 768, 2304), (1024, 768, 2304) and (512, 768, 3072) have 288 / 576 / 384
-    # tiles of 64x64 on 256 CUs and cut only the tiles of the last partial round.
+    # (64, 6400, 1600), (16, 1024, 3072) and (32, 1600, 6400) cut the whole K range into parts.
+    # From 65 rows on, products of enough tiles and work run on the bf16 matrix cores with input and
+    # weights cut into three bf16 parts each: (128, 1600, 4800), (1000, 1024, 4096), (512 and 1024, 768, 2304),
+    # (512, 768, 3072), (1024, 3072, 768), (1024, 1600, 4800) and the last three, whole or cut along K as the
+    # planner has it.  The other products of more than 64 rows run on the f32 matrix cores, some with K cut.
     # K = 48 and 112 are not multiples of 32 and take k-tiles of 16 columns; K = 16 and 32 are a
-    # single k-tile (the pipelined loop's shortest cases); (1024, 3072, 768) has a deep K on 192
-    # tiles and is cut in four.  From 1024 rows on, products with enough 128x128 tiles run on the
-    # bf16 matrix cores with input and weights cut into three bf16 parts each and all nine
-    # products formed (exact): whole tiles for (1024, 1600, 4800) and (1024, 1024, 4096), tiles
-    # cut in four along K for (1024, 4096, 1024) and (1100, 1600, 1600), whose last tile row is
-    # ragged.
+    # single k-tile (the pipelined loop's shortest cases).
     # Up to 32 rows take the MFMA kernel of the decode batch: 16 rows its 16x16x4 form, with 16
     # rows of W per block where 32 would leave CUs idle ((16, 768, 2304), (16, 1024, 3072),
     # (16, 768, 1000) with a ragged last block) and 32 otherwise ((16, 1600, 4800); (16, 4096,
@@ -81,8 +78,7 @@ def test_dense_many_rows_uses_mfma_gemm(rows, k, n):
 def test_dense_with_selection_weights_returns_the_inputs_bit_for_bit(rows, k, n):
     """W[o, :] is a unit vector, so out[r, o] must be exactly x[r, o % k] whatever the
     summation order: every other product is 0.  For the first two shapes the product runs on
-    the bf16 matrix cores with x and W cut into three bf16 parts each (whole tiles; tiles cut
-    in four along K): the parts of a value must add up to the value in all its 24 bits, at any
+    the bf16 matrix cores with x and W cut into three bf16 parts each: the parts of a value must add up to the value in all its 24 bits, at any
     exponent.  (96 rows: the f32 matrix cores, for comparison.)"""
     rng = np.random.default_rng(rows + n)
     x = (rng.standard_normal(rows * k) * 10.0 ** rng.uniform(-6, 6, rows * k)).astype(np.float32)
@@ -101,8 +97,7 @@ def test_dense_keeps_infinities_and_nans_of_the_input(rows, k, n):
     arithmetic does: +inf times a positive weight is +inf, opposite infinities in one row give
     NaN, inf times a zero weight gives NaN, a NaN stays a NaN, and rows without such a value are
     untouched.  48 rows run on the f32 matrix cores.  The first two shapes run on the bf16 matrix
-    cores with x AND W cut into three bf16 parts each (whole tiles; tiles cut in four along K),
-    where a zero part times an infinity would be NaN: a tile that has met an infinity is computed
+    cores with x AND W cut into three bf16 parts each, where a zero part times an infinity would be NaN: a tile that has met an infinity is computed
     again in f32 arithmetic, so the result is the reference's there as well."""
     rng = np.random.default_rng(rows + k)
     x = rng.standard_normal((rows, k)).astype(np.float32)

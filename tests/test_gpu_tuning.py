@@ -102,7 +102,7 @@ def test_per_operation_and_batched_paths_with_other_split_plans(blocks, items):
 def test_planner_tunables_move_the_prompt_to_other_kernels_with_the_same_logits():
     """seq_gemm_min_tokens decides from which prompt length the GEMM prefill runs,
     gemm_b9_min_rows from which row count f32 products take the bf16 matrix cores: every
-    setting gives the oracle's logits (the nine-product form is exact in its products)."""
+    setting gives the oracle's logits (there the products are right to 2^-24)."""
     cfg = Gpt2Config(vocab_size=97, n_positions=512, n_embd=768, n_layer=1, n_head=12)
     w = synth.random_weights(cfg, 0x5EED0650, perturb=True)
     ref = oracle.Model(cfg, w, oracle.rust_config(8))
@@ -113,11 +113,31 @@ def test_planner_tunables_move_the_prompt_to_other_kernels_with_the_same_logits(
         model = Gpt2Model.new(cfg, w, Gpt2HipConfig(**kw))
         text = model.describe()
         assert f"seq_gemm_min_tokens={kw.get('seq_gemm_min_tokens', 4)}" in text
-        assert f"gemm_b9_min_rows={min(kw.get('gemm_b9_min_rows', 1024), 0x7fffffff)}" in text
+        assert f"gemm_b9_min_rows={min(kw.get('gemm_b9_min_rows', 65), 0x7fffffff)}" in text
         for n, logits in want.items():
             cache = model.new_kv_cache()
             assert_logits_close(model.prefill(ids[:n], cache).to_host(), logits)
             assert cache.seq_len == n
+
+
+def test_min_rows_of_the_bf16_cores_is_a_bound_beside_the_planners_rule():
+    """The default is its smallest value, and products of more rows but too few tiles stay on the f32 cores."""
+    cfg = Gpt2Config(vocab_size=97, n_positions=1100, n_embd=128, n_layer=1, n_head=2)
+    w = synth.random_weights(cfg, 0x5EED0651, perturb=True)
+    ids = [int(t) for t in synth.token_ids(1100, 0x70C00651, 97)]
+
+    def logits(weights, config, prompt, rows):
+        model = Gpt2Model.new(config, weights, Gpt2HipConfig(gemm_b9_min_rows=rows))
+        return model.prefill(prompt, model.new_kv_cache()).to_host()
+
+    few_tiles = logits(w, cfg, ids, 0xffffffff)
+    for rows in (0, 65, 128, 1024):
+        np.testing.assert_array_equal(logits(w, cfg, ids, rows), few_tiles)
+    cfg = Gpt2Config(vocab_size=97, n_positions=512, n_embd=768, n_layer=1, n_head=12)
+    w, ids = synth.random_weights(cfg, 0x5EED0650, perturb=True), ids[:512]
+    np.testing.assert_array_equal(logits(w, cfg, ids, 0), logits(w, cfg, ids, 65))
+    np.testing.assert_array_equal(logits(w, cfg, ids, 513), logits(w, cfg, ids, 0xffffffff))
+    assert (logits(w, cfg, ids, 0) != logits(w, cfg, ids, 513)).any()
 
 
 def test_model_directory_tuning_file_is_read(tmp_path):
