@@ -49,6 +49,7 @@
 // the abort word (global) and the halt word (LDS); every other wait observes one of
 // them and all wavefronts leave the kernel.
 #include "pg_kernels.h"
+#include "pg_math.h"
 
 #include <math.h>
 
@@ -139,10 +140,6 @@ __device__ __forceinline__ float wmax(float v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
   return v;
-}
-
-__device__ __forceinline__ float gelu_tanh(float x) {
-  return 0.5f * x * (1.0f + tanhf(0.7978846f * (x + 0.044715f * x * x * x)));
 }
 
 // Control block in LDS.

@@ -347,3 +347,29 @@ def test_config3_gpt2_medium_batch16_to_the_end():
                 assert_logits_close(host[b], want[b], what=f"step {step} seq {b}")
         nxt = logits.argmax()
     assert cache.seq_len == n + steps == 383
+
+
+@pytest.mark.parametrize("x", [-6.5, -3.3, -2.1, -1.37, -0.83, -0.29, -0.013, 0.007, 0.41, 0.77, 1.19, 1.73, 2.45, 3.6])
+def test_both_decode_paths_have_the_same_gelu(x):
+    """Two hidden units whose input is the bias x alone add gelu(x) and -gelu(x) to two columns; the mean is 0, the
+    epsilon a power of 4 that absorbs the variance, so that the logit is gelu(x) in every order of sums."""
+    cfg = Gpt2Config(vocab_size=1031, n_positions=64, n_embd=768, n_layer=1, n_head=12,
+                     layer_norm_epsilon=2.0 ** 26)
+    w = synth.random_weights(cfg, 0, std=0.0)
+    wide = max(cfg.n_embd, cfg.n_inner)
+    block, wte = w.blocks[0], w.wte.reshape(cfg.vocab_size, cfg.n_embd)
+    block.c_fc_b[:2] = x
+    block.c_proj_mlp_w[0] = 1.0
+    for row in (cfg.n_embd, wide):  # (column 1 of unit 1, whichever way the matrix lies; the other entry meets 0)
+        block.c_proj_mlp_w[row + 1] = -1.0
+    w.ln_f_g[:] = 2.0 ** 13
+    wte[1:3, 0], wte[3:5, 1] = 1.0, 1.0
+    got = []
+    for path in (0, 1):
+        model = Gpt2Model.new(cfg, w, Gpt2HipConfig(decode_path=path))
+        assert ("decode=persistent", "decode=kernels")[path] in model.describe()
+        got.append(model.forward_one(0, model.new_kv_cache()).to_host().reshape(-1))
+    want = oracle.gelu(np.full(1, x, np.float32))[0]
+    for logits in got:
+        np.testing.assert_allclose(logits[1:5], [want, want, -want, -want], rtol=1e-5, atol=1e-7)
+    np.testing.assert_array_equal(got[0], got[1])
