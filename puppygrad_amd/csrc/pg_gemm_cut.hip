@@ -474,9 +474,11 @@ bool takes(const GemmArgs& a) {
 
 // Time of a product in microseconds: a start, the stages of K at the pace of the CU with the most items,
 // and for a cut K the partial tiles' way through memory.  The constants are those of the
-// least regret over 416 shapes (the four GPT-2 widths' projections at 66 to 6000 rows, W from HBM) with 1 to 8
-// parts each: the plan of least predicted time is 1 % slower than the best measured one in the mean (2 %
-// for bf16 rows), 2 % over the shapes that were held out.
+// least regret over the four GPT-2 widths' projections at 66 to 8192 rows (464 shapes a storage, W from HBM) with 1 to 8
+// parts each.  f32 rows: timed with the epilogue and norm that each has in the model, the plan of least predicted time
+// is 0.3 % slower than the best measured one in the mean, 6 % at most (fitted to bare products 1.0 and 14 %: whole
+// 64 x 128 tiles where two parts of 128 x 128 were faster, 420 x 3072 x 768 with GELU 31.4 us against 27.5).  bf16 and int8
+// rows: fitted to bare products, 1.7 and 1.8 % with the epilogues.
 struct Pace {
   float start, stage, more, part;  // start; a stage alone; each further item on the CU; a partly filled round
 };
@@ -485,10 +487,10 @@ struct Reduce {
 };
 // [storage][CutTile]
 constexpr Pace kPace[3][5] = {
-    {{5.2f, 0.468f, 0.160f, 0.197f}, {6.2f, 0.710f, 0.323f, 0.273f}, {9.3f, 1.027f, 1.661f, 0.249f}, {7.0f, 0.581f, 0.0f, 0.0f}, {}},
+    {{7.79f, 0.496f, 0.171f, 0.167f}, {8.78f, 0.647f, 0.497f, 0.080f}, {9.31f, 1.018f, 0.988f, 0.207f}, {8.69f, 0.612f, 0.0f, 0.0f}, {}},
     {{3.4f, 0.461f, 0.204f, 0.131f}, {9.1f, 0.661f, 0.316f, 0.302f}, {}, {}, {12.3f, 0.403f, 0.404f, 0.311f}},
     {{7.9f, 0.518f, 0.234f, 0.139f}, {12.0f, 0.807f, 0.285f, 0.383f}, {}, {}, {14.0f, 0.101f, 0.630f, 0.288f}}};
-constexpr Reduce kReduce[3] = {{2.8f, 1.30f, 0.5f}, {2.0f, 1.20f, 0.2f}, {5.0f, 1.55f, 0.4f}};
+constexpr Reduce kReduce[3] = {{0.06f, 1.33f, 0.126f}, {2.0f, 1.20f, 0.2f}, {5.0f, 1.55f, 0.4f}};
 
 }  // namespace
 
@@ -497,11 +499,13 @@ bool gemm_cut_plan(const GemmArgs& a, int num_cus, CutPlan* plan) {
   const int wt = a.w_scale ? 2 : a.w_bf16 ? 1 : 0;
   const long tiles64 = (long)((a.M + 63) / 64) * ((a.N + 127) / 128);
   if (wt == 0) {
-    // Little work: the f32 cores' 64 x 64 tiles are as fast or faster (192 x 2304 x 768: 17.0 against 18.4 us, 128 x
-    // 1280 x 5120: 30.9 against 32.5), unless K is deep enough and the tiles are many (66 x 4800 x 1600: 28
-    // against 23 us); from there on the other way round (256 x 4096 x 1024: 30.7 against 24.1).
+    // Little work: the f32 cores' 64 x 64 tiles are as fast or faster (192 x 2304 x 768: 17.0 against 18.4 us), and so
+    // they are where two rows of tiles leave most CUs with one (100 x 3840 x 1280: 23.2 against 28.2 us, 128 x 4800 x
+    // 1600 33.9 against 35.0, 128 x 6400 x 1600 35.0 against 35.8); from there on the other way round (134 x 6400 x
+    // 1600: 50.3 against 41.1 us, 134 x 4800 x 1600 35.8 against 34.9, 256 x 4096 x 1024 28.8 against 27.7).
     const double mnk = (double)a.M * a.N * a.K;
-    if (a.M < a.b9_min_rows || (!(tiles64 >= 20 && mnk >= 0.85e9) && !(tiles64 >= 60 && a.K >= 1280))) return false;
+    if (a.M < a.b9_min_rows || (a.M <= 128 && 2 * tiles64 <= num_cus)) return false;
+    if (!(tiles64 >= 20 && mnk >= 0.85e9) && !(tiles64 >= 60 && a.K >= 1280)) return false;
   } else if (tiles64 < (wt == 1 ? 13 : 24)) {
     return false;  // (96 x 768 x 768, bf16: 9.9 against 11.3 us; 100 x 1280 x 1280, int8: 14.2 against 15.5)
   }

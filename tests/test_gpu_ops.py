@@ -52,7 +52,7 @@ def test_dense_many_rows_uses_mfma_gemm(rows, k, n):
     # rows >= 16 and K % 16 == 0 take the MFMA GEMM; tails in M and N are exercised.
     # (64, 6400, 1600), (16, 1024, 3072) and (32, 1600, 6400) cut the whole K range into parts.
     # From 65 rows on, products of enough tiles and work run on the bf16 matrix cores with input and
-    # weights cut into three bf16 parts each: (128, 1600, 4800), (1000, 1024, 4096), (512 and 1024, 768, 2304),
+    # weights cut into three bf16 parts each: (1000, 1024, 4096), (512 and 1024, 768, 2304),
     # (512, 768, 3072), (1024, 3072, 768), (1024, 1600, 4800) and the last three, whole or cut along K as the
     # planner has it.  The other products of more than 64 rows run on the f32 matrix cores, some with K cut.
     # K = 48 and 112 are not multiples of 32 and take k-tiles of 16 columns; K = 16 and 32 are a

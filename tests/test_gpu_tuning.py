@@ -138,6 +138,12 @@ def test_min_rows_of_the_bf16_cores_is_a_bound_beside_the_planners_rule():
     np.testing.assert_array_equal(logits(w, cfg, ids, 0), logits(w, cfg, ids, 65))
     np.testing.assert_array_equal(logits(w, cfg, ids, 513), logits(w, cfg, ids, 0xffffffff))
     assert (logits(w, cfg, ids, 0) != logits(w, cfg, ids, 513)).any()
+    # two rows of tiles that leave half of the CUs without one stay on the f32 cores, three do not
+    cfg = Gpt2Config(vocab_size=97, n_positions=256, n_embd=1280, n_layer=1, n_head=20)
+    w = synth.random_weights(cfg, 0x5EED0652, perturb=True)
+    for rows in (66, 128):
+        np.testing.assert_array_equal(logits(w, cfg, ids[:rows], 0), logits(w, cfg, ids[:rows], 0xffffffff))
+    assert (logits(w, cfg, ids[:134], 0) != logits(w, cfg, ids[:134], 0xffffffff)).any()
 
 
 def test_model_directory_tuning_file_is_read(tmp_path):
