@@ -380,7 +380,7 @@ def measure_prefill(model, cfg, ids, T, steps, warmup):
                          "unit": "TFLOP/s", "frac": round(whole / FP32_MFMA_PEAK_TFLOPS, 4),
                          "traffic": TRAFFIC_124M_PREFILL_1024 if T == 1024 else None,
                          "traffic_source": TRAFFIC_SOURCE_124M_PREFILL if T == 1024 else None,
-                         "kernel": "whole prefill (k_gemm, k_attn_prefill64, LayerNorm, split-K reduces, lm_head)",
+                         "kernel": "whole prefill (k_gemm_cut, k_gemm, k_attn_prefill64, LayerNorm, split-K reduces, lm_head)",
                          "algorithmic_flops_per_step": int(flops)},
             "gemm_part": {"ms": round(gemm_s * 1e3, 4), "achieved": round(gemm, 2), "unit": "TFLOP/s",
                           "frac": round(gemm / FP32_MFMA_PEAK_TFLOPS, 4), "flops": int(gemm_flops),
@@ -695,8 +695,8 @@ TRAFFIC_SOURCE = "profiles/k_decode_persistent_1600_xl_decode_traffic.txt"
 TRAFFIC_RATIO_124M = 0.983
 TRAFFIC_SOURCE_124M = "profiles/k_decode_persistent_768_124m_decode.txt"
 # HBM bytes of one 124M prefill (FETCH_SIZE + WRITE_SIZE of all its launches, scaled)
-TRAFFIC_124M_PREFILL_1024 = 3208200000
-TRAFFIC_124M_PREFILL_32 = 631400000
+TRAFFIC_124M_PREFILL_1024 = 3175900000
+TRAFFIC_124M_PREFILL_32 = 630900000
 TRAFFIC_SOURCE_124M_PREFILL = "profiles/prefill_124m_traffic.txt"
 TRAFFIC_RATIO_355M_B16 = 1.093
 TRAFFIC_RATIO_XL_BF16_B32 = 1.073  # same file, section (c)
@@ -704,7 +704,7 @@ TRAFFIC_SOURCE_355M_B16 = "profiles/batched_decode_355m_b16_xl_bf16_b32.txt"
 # Bytes through the L2s to and from the fabric per XL bf16 prefill of 32 x 512 tokens (FETCH_SIZE
 # scaled by 1.9994 + WRITE_SIZE over all launches of a step; most of the reads are operand
 # re-reads that the Infinity Cache serves).
-TRAFFIC_XL_BF16_PREFILL_B32_512 = 372400000000
+TRAFFIC_XL_BF16_PREFILL_B32_512 = 372600000000
 TRAFFIC_SOURCE_XL_BF16_PREFILL = "profiles/k_gemm_cut_xl_bf16_prefill_b32_512.txt"
 
 

@@ -23,15 +23,17 @@
 // 128 x 256 tile has no room for a second sum, and where there are more than two 128 x 128 tiles to a CU the third
 // one there is worth more: 4.3e-7, as such products always had.
 //
-// What bounds it: power.  With all matrix cores at work the clock goes down to 1.7 to 2.0 GHz (a plain bf16
+// What bounds it: in large products the clock goes down to 1.9 to 2.1 GHz with the matrix cores at work (a plain bf16
 // product of the library reaches 1354 of 2500 TFLOP/s on this card), and what else the CU moves is paid
-// for in clock as well as in time.  So the inputs travel as stored: f32 rows of A go straight to LDS
+// for in clock as well as in time; the matrix cores are busy for 0.64 to 0.71 of the clocks in which a CU is, the rest is
+// waits and VALU work that no MFMA covers.  In small ones (one tile on 144 to 240 of 256 CUs, 0.44 to 0.49) the clock stays
+// and a tile's start and end count.  So the inputs travel as stored: f32 rows of A go straight to LDS
 // (global_load_lds, no registers, no VALU), as do bf16 rows of W; a wavefront owns whole rows of the tile and
 // cuts its A operands itself, in registers, once for all columns it owns; W, which every wavefront needs,
 // is cut once on its way to LDS.  Against the form that cut A for the whole block and kept its planes in
 // LDS (128 x 128 tiles, 2 x 2 wavefronts) that is a quarter of the LDS reads and half the VALU
 // instructions per MFMA: 8192 x 4800 x 1600 bf16 488 -> 378 us, 8192 x 1600 x 6400 640 -> 470 us, int8
-// 643 -> 508 us; f32, nine products -> six, 4096 x 6400 x 1600 680 -> 503 us (one box, W from HBM).
+// 643 -> 508 us; f32, nine products -> six, 4096 x 6400 x 1600 680 -> 457 us (one box, W from HBM).
 // The dot instruction that could take both subtractions of a cut (v_dot2_f32_bf16) runs on the matrix
 // cores' time: 6 % slower.
 #include "pg_gemm_dev.h"

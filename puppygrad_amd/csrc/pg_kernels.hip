@@ -1389,8 +1389,8 @@ hipError_t launch_gemv_pe(const GemvArgs& a, hipStream_t s) {
   const int blocks = (a.nout + kWaves * rpw - 1) / (kWaves * rpw);
   const int blocks1 = (a.nout + kWaves - 1) / kWaves;
   // Many rows (the logits) behind a prologue that reads and sums several vectors: four blocks to a CU that
-  // take the rows in turns, so that the prologue runs 1024 times instead of 6283 (161 MB of bf16 rows behind
-  // PRO_STACK 35.8 -> 27.8 us; behind PRO_RMS, a sum of one vector, whole blocks are faster: 25.3 us).
+  // take the rows in turns (256 CUs), so that the prologue runs 1024 times instead of 6283 (161 MB of bf16 rows behind
+  // PRO_STACK 35.8 -> 27.8 us, the seventh turn nearly empty; behind PRO_RMS, a sum of one vector, whole blocks are faster: 25.3 us).
   constexpr int kTurnBlocks = 1024;
   if constexpr ((PRO == PRO_STACK || PRO == PRO_LN) && EPI == EPI_BIAS) {
     if (blocks >= 2 * kTurnBlocks && aligned && a.K % (a.w_scale ? 16 : a.w_bf16 ? 8 : 4) == 0) {
