@@ -105,7 +105,8 @@ typedef struct pg_hip_options {
   uint32_t gemm_b9_min_rows;        /* f32 weights: products over at least this many input rows
                                        run on the bf16 matrix cores with both operands cut into
                                        three bf16 parts where the planner finds enough tiles
-                                       (default 65; 0xffffffff: never) */
+                                       (default 65: from 33 rows on where they are better kept
+                                       cut, too; 0xffffffff: never) */
   uint32_t seq_gemm_min_tokens;     /* prompts of at least this many tokens take the GEMM
                                        prefill, shorter ones run token by token through the
                                        decode path (default 4; at most 65536) */

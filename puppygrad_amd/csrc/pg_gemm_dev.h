@@ -4,6 +4,7 @@
 
 #include <algorithm>
 
+#include "pg_cut.h"
 #include "pg_kernels.h"
 #include "pg_math.h"
 
@@ -22,31 +23,22 @@ bool gemm_cut_plan(const GemmArgs& a, int num_cus, CutPlan* plan);
 // The plan that GemmArgs::plan_bm, plan_bn and plan_parts ask for; false where there is none such.
 bool gemm_cut_forced(const GemmArgs& a, CutPlan* plan);
 hipError_t launch_gemm_cut(const GemmArgs& a, int epi, CutPlan plan, hipStream_t s);
+// A product of an activation matrix in cut form (pg_gemm_rows.hip): input rows per block (16 mt), rows of W per block
+// (at most 16 ng, a multiple of eight) and parts of K.
+struct CutRowsPlan {
+  int mt, ng, rows, parts;
+};
+bool gemm_cut_rows_plan(const GemmArgs& a, int num_cus, CutRowsPlan* plan);
+hipError_t launch_gemm_cut_rows(const GemmArgs& a, int epi, const CutRowsPlan& p, hipStream_t s);
+// x[M][K] into cut form (K a multiple of 8)
+hipError_t launch_to_cut(const float* x, void* to, int M, int K, hipStream_t s);
 // (bf16 rows; tiles of tile_rows = 64 or 128 rows)
 hipError_t launch_gemm_cut_grouped(const GemmArgs& a, int epi, int tile_rows, hipStream_t s);
 
 namespace {
 
-typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f16v __attribute__((ext_vector_type(16)));
-typedef unsigned u2v __attribute__((ext_vector_type(2)));
 typedef unsigned u4v __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ unsigned pk_bf16(float a, float b) {
-  return __builtin_bit_cast(unsigned, __builtin_convertvector(f2{a, b}, bf16x2));
-}
-// Two values as three bf16 each whose sum is the value, two to a register (a in the low half): rounded to
-// nearest, every difference exact.  A value that is infinite as bf16 gives NaN in the second and third part.
-__device__ __forceinline__ void cut2(float a, float b, unsigned& hi, unsigned& mid, unsigned& lo) {
-  hi = pk_bf16(a, b);
-  const float a1 = a - __uint_as_float(hi << 16), b1 = b - __uint_as_float(hi & 0xffff0000u);
-  mid = pk_bf16(a1, b1);
-  const float a2 = a1 - __uint_as_float(mid << 16), b2 = b1 - __uint_as_float(mid & 0xffff0000u);
-  lo = pk_bf16(a2, b2);
-}
 // Eight columns of a row as three MFMA operands.
 struct Cut {
   u4v p[3];

@@ -512,10 +512,13 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
   DevBuf SCR, LOG;
   // split-K partial tiles of the projections back to n_embd columns (up to 8 parts)
   const size_t ws_floats = 8 * n * g.C;
+  // the projections' inputs (XN, ATT, HB) in cut form
+  const bool cut = hd == pgk::kHeadDim && pgk::gemm_takes_cut(T, C, I, m->w_bf16, m->w_i8, m->gemm_b9_min_rows);
   {
+    auto form = [&](size_t cols) { return cut ? std::max(n * cols, pgk::cut_floats(n, cols)) : n * cols; };
     auto up = [](size_t v) { return (v + 63) / 64 * 64; };  // 256-byte boundaries
-    const size_t sizes[7] = {up(n * g.C), up(n * g.C), up(n * 3 * g.C), up(n * g.C),
-                             up(n * g.I), up(n),       up(ws_floats)};
+    const size_t sizes[7] = {up(n * g.C),   up(form(g.C)), up(n * 3 * g.C), up(form(g.C)),
+                             up(form(g.I)), up(n),         up(ws_floats)};
     size_t total = 0;
     for (size_t v : sizes) total += v;
     if (c->seq_scratch_floats < total) {
@@ -559,9 +562,10 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
   // same call: fused into the projection's reduce where it has one)
   auto gemm = [&](const float* A, int lda, const float* W, const float* bias, float* Cout,
                   int ldc, int N, int K, int epi, const float* ln_g = nullptr,
-                  const float* ln_b = nullptr) -> hipError_t {
+                  const float* ln_b = nullptr, int a_cut = 0, int c_cut = 0) -> hipError_t {
     pgk::GemmArgs a{};
     a.A = A; a.w_bf16 = m->w_bf16; a.W = W; a.bias = bias; a.resid = Cout; a.C = Cout;
+    a.a_cut = a.ln_cut = a_cut; a.c_cut = c_cut;
     a.M = T; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc;
     if (m->w_i8) a.w_scale = i8_scales_of(W, (size_t)N, (size_t)K);
     a.ws = WS.p; a.ws_floats = ws_floats;
@@ -570,23 +574,25 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
     a.b9_min_rows = m->gemm_b9_min_rows;
     return pgk::launch_gemm(a, epi, m->num_cus, s);
   };
-  PG_HIP(pgk::launch_layer_norm_rows(X.p, XN.p, T, C, m->layers[0].ln_1_g, m->layers[0].ln_1_b, g.eps, s));
+  PG_HIP(pgk::launch_layer_norm_rows(X.p, XN.p, T, C, m->layers[0].ln_1_g, m->layers[0].ln_1_b, g.eps, s,
+                                     cut ? pgk::FORM_CUT : pgk::FORM_ROWS));
   PG_MARK(kLayerNorm);
   for (size_t l = 0; l < g.L; ++l) {
     const pgk::LayerW& w = m->layers[l];
     // the LayerNorm after this layer: the next layer's ln_1; ln_f is applied where it is needed
     const float* next_g = l + 1 < g.L ? m->layers[l + 1].ln_1_g : nullptr;
     const float* next_b = l + 1 < g.L ? m->layers[l + 1].ln_1_b : nullptr;
-    PG_HIP(gemm(XN.p, C, w.c_attn_w, w.c_attn_b, QKV.p, 3 * C, 3 * C, C, pgk::GEMM_BIAS));
+    PG_HIP(gemm(XN.p, C, w.c_attn_w, w.c_attn_b, QKV.p, 3 * C, 3 * C, C, pgk::GEMM_BIAS, nullptr, nullptr, cut));
     PG_MARK(kQkv);
     PG_HIP(pgk::launch_attn_prefill(QKV.p, Ts, C, H, hd, P, c->k_panel(l, b), c->v_panel(l, b),
-                                    ATT.p, SCR.p, s, (int)nb, g.H * g.P * g.hd()));
+                                    ATT.p, SCR.p, s, (int)nb, g.H * g.P * g.hd(),
+                                    cut ? pgk::FORM_CUT : pgk::FORM_ROWS));
     PG_MARK(kAttention);
-    PG_HIP(gemm(ATT.p, C, w.c_proj_w, w.c_proj_b, X.p, C, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b));
+    PG_HIP(gemm(ATT.p, C, w.c_proj_w, w.c_proj_b, X.p, C, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b, cut));
     PG_MARK(kAttnProj);
-    PG_HIP(gemm(XN.p, C, w.c_fc_w, w.c_fc_b, HB.p, I, I, C, pgk::GEMM_GELU));
+    PG_HIP(gemm(XN.p, C, w.c_fc_w, w.c_fc_b, HB.p, I, I, C, pgk::GEMM_GELU, nullptr, nullptr, cut, cut));
     PG_MARK(kMlpFc);
-    PG_HIP(gemm(HB.p, I, w.c_proj_mlp_w, w.c_proj_mlp_b, X.p, C, C, I, pgk::GEMM_RESID, next_g, next_b));
+    PG_HIP(gemm(HB.p, I, w.c_proj_mlp_w, w.c_proj_mlp_b, X.p, C, C, I, pgk::GEMM_RESID, next_g, next_b, cut));
     PG_MARK(kMlpProj);
   }
   if (all_logits_dst) {
@@ -653,16 +659,19 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
   // same call: fused into the projection's reduce where it has one)
   // c->pack32: the inputs of the projections (xn_b, att_b, hbuf) are held in the packed form
   // that the 32-row kernel reads with contiguous loads; their producers write them that way.
-  const int pk = c->pack32 ? 1 : 0;
+  // c->cut_form: the same in cut form, except for the logits' input.
+  const int pk = c->pack32 ? 1 : 0, cut = c->cut_form ? 1 : 0;
+  const int form = cut ? pgk::FORM_CUT : pk ? pgk::FORM_PACKED32 : pgk::FORM_ROWS;
   auto gemm = [&](const float* A, int lda, const float* W, const float* bias, float* Cout,
                   int ldc, int N, int K, int epi, const float* ln_g = nullptr,
-                  const float* ln_b = nullptr, int c_packed = 0) -> hipError_t {
+                  const float* ln_b = nullptr, int a_cut = 0, int ln_cut = 0) -> hipError_t {
     pgk::GemmArgs a{};
     a.A = A; a.w_bf16 = m->w_bf16; a.W = W; a.bias = bias; a.resid = Cout; a.C = Cout;
     a.M = B; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc;
     if (m->w_i8) a.w_scale = i8_scales_of(W, (size_t)N, (size_t)K);
     a.ws = c->gemm_ws; a.ws_floats = c->gemm_ws_floats;
-    a.a_packed = pk; a.c_packed = c_packed;
+    a.a_packed = pk; a.c_packed = epi == pgk::GEMM_GELU ? pk : 0;
+    a.a_cut = a_cut; a.c_cut = epi == pgk::GEMM_GELU ? cut : 0; a.ln_cut = ln_cut;
     if (ln_g) { a.ln_out = c->xn_b; a.ln_g = ln_g; a.ln_b = ln_b; a.ln_eps = g.eps; a.ln_packed = pk; }
     a.split_items_per_cu = m->gemm_split_items;
     a.b9_min_rows = m->gemm_b9_min_rows;
@@ -670,13 +679,13 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
   };
   PG_HIP(pgk::launch_embed_batch(c->x, m->wte, m->wpe, d_ids, B, (int)pos, C, s, m->w_bf16));
   PG_HIP(pgk::launch_layer_norm_rows(c->x, c->xn_b, B, C, m->layers[0].ln_1_g, m->layers[0].ln_1_b,
-                                     g.eps, s, pk));
+                                     g.eps, s, form));
   for (size_t l = 0; l < g.L; ++l) {
     const pgk::LayerW& w = m->layers[l];
     // the LayerNorm after this layer: the next layer's ln_1, or ln_f
     const float* next_g = l + 1 < g.L ? m->layers[l + 1].ln_1_g : m->ln_f_g;
     const float* next_b = l + 1 < g.L ? m->layers[l + 1].ln_1_b : m->ln_f_b;
-    PG_HIP(gemm(c->xn_b, C, w.c_attn_w, w.c_attn_b, c->qkv_b, 3 * C, 3 * C, C, pgk::GEMM_BIAS));
+    PG_HIP(gemm(c->xn_b, C, w.c_attn_w, w.c_attn_b, c->qkv_b, 3 * C, 3 * C, C, pgk::GEMM_BIAS, nullptr, nullptr, cut));
     // K/V append (rust.rs:1677-1683): by the attention launch itself for head_dim 64
     const bool fused_append = hd == pgk::kHeadDim;
     if (!fused_append)
@@ -684,13 +693,14 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
                                    c->v_panel(l, 0), bs.kv, s));
     PG_HIP(pgk::launch_attn_decode(c->qkv_b, c->k_panel(l, 0), c->v_panel(l, 0), (int)pos, P, H,
                                    hd, nsplit, c->part_acc, c->part_m, c->part_l, s, B, bs,
-                                   fused_append ? C : 0, one_split ? c->att_b : nullptr, pk));
+                                   fused_append ? C : 0, one_split ? c->att_b : nullptr, form));
     if (!one_split)
       PG_HIP(pgk::launch_attn_finish(c->part_acc, c->part_m, c->part_l, H, hd, nsplit, c->att_b, s,
-                                     B, bs, pk));
-    PG_HIP(gemm(c->att_b, C, w.c_proj_w, w.c_proj_b, c->x, C, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b));
-    PG_HIP(gemm(c->xn_b, C, w.c_fc_w, w.c_fc_b, c->hbuf, I, I, C, pgk::GEMM_GELU, nullptr, nullptr, pk));
-    PG_HIP(gemm(c->hbuf, I, w.c_proj_mlp_w, w.c_proj_mlp_b, c->x, C, C, I, pgk::GEMM_RESID, next_g, next_b));
+                                     B, bs, form));
+    PG_HIP(gemm(c->att_b, C, w.c_proj_w, w.c_proj_b, c->x, C, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b, cut, cut));
+    PG_HIP(gemm(c->xn_b, C, w.c_fc_w, w.c_fc_b, c->hbuf, I, I, C, pgk::GEMM_GELU, nullptr, nullptr, cut));
+    PG_HIP(gemm(c->hbuf, I, w.c_proj_mlp_w, w.c_proj_mlp_b, c->x, C, C, I, pgk::GEMM_RESID, next_g, next_b, cut,
+                cut && l + 1 < g.L));
   }
   PG_HIP(gemm(c->xn_b, C, m->lm_w, nullptr, c->logits_buf, (int)g.V, (int)g.V, C, pgk::GEMM_BIAS));
   return PG_OK;
@@ -1236,11 +1246,16 @@ pg_status pg_kv_cache_create(const pg_model* m, uint32_t batch, pg_kv_cache** ou
   PG_HIP(hipMalloc(&raw->q, B * g.C * sizeof(float)));
   // Batches whose projections all run on the 32-row kernel keep that kernel's inputs packed
   // (32 row slots whatever B is).
-  raw->pack32 = B > 1 && B <= 32 && g.C % 16 == 0 && g.I % 16 == 0 && !m->w_i8 &&
+  raw->cut_form = B > 1 && hd == pgk::kHeadDim &&
+                  pgk::gemm_takes_cut((int)B, (int)g.C, (int)g.I, m->w_bf16, m->w_i8, m->gemm_b9_min_rows);
+  raw->pack32 = !raw->cut_form && B > 1 && B <= 32 && g.C % 16 == 0 && g.I % 16 == 0 && !m->w_i8 &&
                 pgk::gemm_takes_rows32((int)B, (int)g.C, (int)g.C, m->w_bf16) &&
                 pgk::gemm_takes_rows32((int)B, (int)g.I, (int)g.I, m->w_bf16);
   const size_t act_rows = raw->pack32 ? 32 : B;
-  PG_HIP(hipMalloc(&raw->hbuf, act_rows * g.I * sizeof(float)));
+  auto act_floats = [&](size_t cols) {
+    return raw->cut_form ? std::max(act_rows * cols, pgk::cut_floats(B, cols)) : act_rows * cols;
+  };
+  PG_HIP(hipMalloc(&raw->hbuf, act_floats(g.I) * sizeof(float)));
   if (B > 1) {
     raw->gemm_ws_floats = 8 * B * std::max<size_t>(3 * g.C, g.I);
     PG_HIP(hipMalloc(&raw->gemm_ws, raw->gemm_ws_floats * sizeof(float)));
@@ -1250,8 +1265,8 @@ pg_status pg_kv_cache_create(const pg_model* m, uint32_t batch, pg_kv_cache** ou
   PG_HIP(hipMalloc(&raw->part_l, parts * sizeof(float)));
   PG_HIP(hipMalloc(&raw->logits_buf, B * g.V * sizeof(float)));
   PG_HIP(hipMalloc(&raw->qkv_b, B * 3 * g.C * sizeof(float)));
-  PG_HIP(hipMalloc(&raw->xn_b, act_rows * g.C * sizeof(float)));
-  PG_HIP(hipMalloc(&raw->att_b, act_rows * g.C * sizeof(float)));
+  PG_HIP(hipMalloc(&raw->xn_b, act_floats(g.C) * sizeof(float)));
+  PG_HIP(hipMalloc(&raw->att_b, act_floats(g.C) * sizeof(float)));
   PG_HIP(hipMalloc(&raw->d_tok, B * sizeof(uint32_t)));
   PG_HIP(hipMalloc(&raw->d_out_ids, g.P * B * sizeof(uint32_t)));
   PG_HIP(hipHostMalloc(&raw->h_ids, g.P * B * sizeof(uint32_t), hipHostMallocDefault));

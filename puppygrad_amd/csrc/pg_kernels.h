@@ -111,7 +111,7 @@ hipError_t launch_attn_decode(const float* q, const float* kcache, const float* 
                               int P, int H, int head_dim, int nsplit, float* part_acc,
                               float* part_m, float* part_l, hipStream_t s, int batch = 1,
                               BatchStrides bs = BatchStrides{}, int append_C = 0,
-                              float* direct_out = nullptr, int out_packed = 0);
+                              float* direct_out = nullptr, int out_form = 0);
 // blocks_per_cu: (head, split) blocks per CU to aim for (tunable, 4 by default).
 int choose_nsplit(int n_keys, int H, int num_cus, int blocks_per_cu = 4);
 
@@ -194,7 +194,7 @@ hipError_t launch_transpose(const float* src, float* dst, int in_f, int out_f, h
 // Attention output from a single split's (acc, m, l): out = acc / l per head.
 hipError_t launch_attn_finish(const float* part_acc, const float* part_m, const float* part_l,
                               int H, int head_dim, int nsplit, float* out, hipStream_t s,
-                              int batch = 1, BatchStrides bs = BatchStrides{}, int out_packed = 0);
+                              int batch = 1, BatchStrides bs = BatchStrides{}, int out_form = 0);
 hipError_t launch_fill_zero(float* p, size_t n, hipStream_t s);
 // out[2 o] = sum_i W[o,i] g[i], out[2 o + 1] = (bias ? bias[o] : 0) + sum_i W[o,i] b[i] for the
 // rows of W[rows][cols] as stored (w_bytes 4: f32, 2: bf16, 1: int8 with scales[o]); sums in f64.
@@ -256,6 +256,9 @@ struct GemmArgs {
   // A, C and ln_out are held that way.  Only the 32-row decode kernel reads a packed A, so
   // launch_gemm refuses the flags for any other form (gemm_takes_rows32 tells beforehand).
   int a_packed = 0, c_packed = 0, ln_packed = 0;
+  // Which of A, C and ln_out are in cut form (FORM_CUT).  launch_gemm refuses what gemm_takes_cut does not
+  // name; a_cut decides the kernel, the other two may go with it only.
+  int a_cut = 0, c_cut = 0, ln_cut = 0;
   // Tunable: a GEMM whose M x N leaves CUs idle is cut along K into about this many work items
   // per CU (gemm_split_parts).
   int split_items_per_cu = 3;
@@ -278,6 +281,15 @@ struct GemmArgs {
 __host__ __device__ inline size_t packed32_index(size_t b, size_t k) {
   return (((k >> 2) * 32 + b) << 2) + (k & 3);
 }
+// How an activation matrix lies in memory: its rows one after the other; packed32_index; or in cut form, as three
+// bf16 numbers per value (store_cut4 in pg_cut.h).
+enum ActForm : int { FORM_ROWS = 0, FORM_PACKED32 = 1, FORM_CUT = 2 };
+// Rows that an activation matrix of M rows in cut form has room for; it takes 6 * K * cut_rows(M) bytes.
+__host__ __device__ inline int cut_rows(int M) { return (M + 15) / 16 * 16; }
+inline size_t cut_floats(size_t M, size_t K) { return (M + 15) / 16 * 16 * K * 3 / 2; }
+// Whether M rows of activations K and N columns wide (each a multiple of 32) are best kept in cut form where they meet
+// rows of W stored so.
+bool gemm_takes_cut(int M, int K, int N, int w_bf16, int w_int8, int b9_min_rows);
 // Whether launch_gemm multiplies an M x K input with the 32-row decode kernel.
 bool gemm_takes_rows32(int M, int K, int lda, int w_bf16);
 bool gemm_supported(const GemmArgs& a);
@@ -297,13 +309,13 @@ hipError_t launch_gemm_grouped(const GemmArgs& a, int epilogue, int tile_rows, c
 // lie kv_stride floats after sequence i - 1's.
 hipError_t launch_attn_prefill(const float* qkv, int T, int C, int H, int head_dim, int P,
                                float* kcache, float* vcache, float* out, float* scratch,
-                               hipStream_t s, int nseq = 1, size_t kv_stride = 0);
+                               hipStream_t s, int nseq = 1, size_t kv_stride = 0, int out_form = 0);
 // rows rows; row t is position t % period of its sequence (wpe may be null)
 hipError_t launch_embed_rows(float* x, const float* wte, const float* wpe, const uint32_t* ids,
                              int rows, int C, hipStream_t s, int w_bf16 = 0, int period = 0);
-// (dst_packed: dst is a packed activation matrix, rows <= 32)
+// (dst_form: an ActForm; packed: rows <= 32; cut: cols a multiple of 8)
 hipError_t launch_layer_norm_rows(const float* src, float* dst, int rows, int cols, const float* g,
-                                  const float* b, float eps, hipStream_t s, int dst_packed = 0);
+                                  const float* b, float eps, hipStream_t s, int dst_form = 0);
 
 // ---- persistent batch-1 decode (pg_decode.hip) --------------------------------
 struct DecodeParams {

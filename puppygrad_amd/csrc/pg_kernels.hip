@@ -6,6 +6,7 @@
 //
 // Shapes the launchers assume are checked on the host before any launch
 // (pg_host.cpp); kernels themselves guard only the ragged tails.
+#include "pg_cut.h"
 #include "pg_kernels.h"
 #include "pg_math.h"
 
@@ -16,8 +17,6 @@
 namespace pgk {
 
 namespace {
-
-typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int kBlock = 256;  // 4 wavefronts of 64 lanes
 constexpr int kWaves = kBlock / 64;
@@ -602,16 +601,17 @@ __device__ __forceinline__ float4 nt_load4(const float4* p) {
 // softmax_in_place, cpu.rs:152-165, rescaled when the max moves); the four are merged
 // through LDS at the end, and the per-split (acc, m, l) by the consumer.
 // The launcher picks IT so that one chunk covers the split where the split count allows.
-template <int IT>
+// CUT: direct_out is in cut form.
+template <int IT, bool CUT>
 __global__ __launch_bounds__(kBlock) void k_attn_decode64(const float* __restrict__ q,
                                                           const float* kcache, const float* vcache,
                                                           int pos, int P, int nsplit,
                                                           float* part_acc, float* part_m,
                                                           float* part_l, BatchStrides bs,
                                                           int append_C, float* direct_out,
-                                                          int out_packed) {
+                                                          int out_form) {
   // direct_out (only with nsplit == 1): the block's result is the head's attention output
-  // and is written there (row blockIdx.z, packed or row-major), with no partials and no
+  // and is written there (row blockIdx.z, in whichever ActForm), with no partials and no
   // merge launch.
   // append_C > 0: the rows of position pos are not in the cache yet.  They are the k and v
   // parts of this step's interleaved qkv row (q + append_C, q + 2 append_C); the block whose
@@ -735,7 +735,8 @@ __global__ __launch_bounds__(kBlock) void k_attn_decode64(const float* __restric
     }
     if (direct_out) {
       const size_t b = blockIdx.z, i = (size_t)h * 64 + tid;
-      direct_out[out_packed ? packed32_index(b, i) : b * bs.out + i] = t / l;
+      if constexpr (CUT) store_cut1(direct_out, cut_rows((int)gridDim.z), b, i, t / l);
+      else direct_out[out_form == FORM_PACKED32 ? packed32_index(b, i) : b * bs.out + i] = t / l;
       return;
     }
     part_acc[pidx * 64 + tid] = t;
@@ -794,17 +795,19 @@ __global__ __launch_bounds__(kBlock) void k_attn_decode_any(const float* q, cons
   }
 }
 
+template <bool CUT>
 __global__ void k_attn_finish(const float* part_acc, const float* part_m, const float* part_l,
                               int C, int hd, int nsplit, float* out, BatchStrides bs,
-                              int out_packed) {
+                              int out_form) {
   const size_t b = blockIdx.y;
   part_acc += b * bs.part * hd;
   part_m += b * bs.part;
   part_l += b * bs.part;
   int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < C)
-    out[out_packed ? packed32_index(b, (size_t)i) : b * bs.out + i] =
-        attn_combine_elem(part_acc, part_m, part_l, nsplit, hd, i);
+  if (i >= C) return;
+  const float v = attn_combine_elem(part_acc, part_m, part_l, nsplit, hd, i);
+  if constexpr (CUT) store_cut1(out, cut_rows((int)gridDim.y), b, (size_t)i, v);
+  else out[out_form == FORM_PACKED32 ? packed32_index(b, (size_t)i) : b * bs.out + i] = v;
 }
 
 // argmax_logits (generation.rs:269-279): strict '>' from -inf, first maximum
@@ -1489,22 +1492,24 @@ int choose_nsplit(int n_keys, int H, int num_cus, int blocks_per_cu) {
 hipError_t launch_attn_decode(const float* q, const float* kcache, const float* vcache, int pos,
                               int P, int H, int head_dim, int nsplit, float* part_acc,
                               float* part_m, float* part_l, hipStream_t s, int batch,
-                              BatchStrides bs, int append_C, float* direct_out, int out_packed) {
-  if (direct_out && (head_dim != kHeadDim || nsplit != 1 || (out_packed && batch > 32)))
+                              BatchStrides bs, int append_C, float* direct_out, int out_form) {
+  if (direct_out && (head_dim != kHeadDim || nsplit != 1 || (out_form == FORM_PACKED32 && batch > 32)))
     return hipErrorInvalidValue;
   if (head_dim == kHeadDim) {
     const int per = (pos + 1 + nsplit - 1) / nsplit;
     const dim3 grid(nsplit, H, batch);
     // steps of 16 keys a block needs for its split: the chunk is sized to it
-    if (per <= 32)
-      hipLaunchKernelGGL(k_attn_decode64<2>, grid, dim3(kBlock), 0, s, q, kcache, vcache, pos, P,
-                         nsplit, part_acc, part_m, part_l, bs, append_C, direct_out, out_packed);
-    else if (per <= 64)
-      hipLaunchKernelGGL(k_attn_decode64<4>, grid, dim3(kBlock), 0, s, q, kcache, vcache, pos, P,
-                         nsplit, part_acc, part_m, part_l, bs, append_C, direct_out, out_packed);
-    else
-      hipLaunchKernelGGL(k_attn_decode64<8>, grid, dim3(kBlock), 0, s, q, kcache, vcache, pos, P,
-                         nsplit, part_acc, part_m, part_l, bs, append_C, direct_out, out_packed);
+#define PG_ATTN(IT, CUT)                                                                                          \
+  hipLaunchKernelGGL((k_attn_decode64<IT, CUT>), grid, dim3(kBlock), 0, s, q, kcache, vcache, pos, P, nsplit, part_acc, \
+                     part_m, part_l, bs, append_C, direct_out, out_form)
+    const bool cut = direct_out && out_form == FORM_CUT;
+    if (per <= 32 && cut) PG_ATTN(2, true);
+    else if (per <= 32) PG_ATTN(2, false);
+    else if (per <= 64 && cut) PG_ATTN(4, true);
+    else if (per <= 64) PG_ATTN(4, false);
+    else if (cut) PG_ATTN(8, true);
+    else PG_ATTN(8, false);
+#undef PG_ATTN
   } else {
     hipLaunchKernelGGL(k_attn_decode_any, dim3(1, H, batch), dim3(kBlock),
                        (pos + 1) * sizeof(float), s, q, kcache, vcache, pos, P, head_dim, part_acc,
@@ -1515,11 +1520,14 @@ hipError_t launch_attn_decode(const float* q, const float* kcache, const float* 
 
 hipError_t launch_attn_finish(const float* part_acc, const float* part_m, const float* part_l,
                               int H, int head_dim, int nsplit, float* out, hipStream_t s,
-                              int batch, BatchStrides bs, int out_packed) {
+                              int batch, BatchStrides bs, int out_form) {
   int C = H * head_dim;
-  if (out_packed && batch > 32) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_attn_finish, dim3((C + 255) / 256, batch), dim3(256), 0, s, part_acc,
-                     part_m, part_l, C, head_dim, nsplit, out, bs, out_packed);
+  if (out_form == FORM_PACKED32 && batch > 32) return hipErrorInvalidValue;
+  const dim3 grid((C + 255) / 256, batch);
+  if (out_form == FORM_CUT)
+    hipLaunchKernelGGL(k_attn_finish<true>, grid, dim3(256), 0, s, part_acc, part_m, part_l, C, head_dim, nsplit, out, bs, out_form);
+  else
+    hipLaunchKernelGGL(k_attn_finish<false>, grid, dim3(256), 0, s, part_acc, part_m, part_l, C, head_dim, nsplit, out, bs, out_form);
   return hipGetLastError();
 }
 

@@ -152,6 +152,7 @@ struct pg_kv_cache {
   float *x = nullptr, *q = nullptr, *hbuf = nullptr, *part_acc = nullptr, *part_m = nullptr,
         *part_l = nullptr, *logits_buf = nullptr;
   float *qkv_b = nullptr, *xn_b = nullptr, *att_b = nullptr;  // batched step: [B][3C], [B][C], [B][C]
+  bool cut_form = false;  // batched step: xn_b, att_b and hbuf are in cut form (pgk::FORM_CUT)
   bool pack32 = false;  // batched step: xn_b, att_b and hbuf are packed (pgk::packed32_index)
   // device-side candidate selection for sampling, allocated at first use: kept candidates
   // (ids, then values, then [count]) and the recent ids of the repeat penalty, with pinned

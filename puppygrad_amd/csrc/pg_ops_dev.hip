@@ -12,6 +12,7 @@
 #include <mutex>
 #include <string>
 
+#include "pg_gemm_dev.h"
 #include "pg_internal.h"
 #include "pg_kernels.h"
 
@@ -368,6 +369,29 @@ pg_status pg_testing_product_dev(int32_t device, void* stream, const float* x, u
   int cus = 0;
   PG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   PG_HIP(pgk::launch_gemm(a, pgk::GEMM_BIAS, cus, static_cast<hipStream_t>(stream)));
+  return PG_OK;
+}
+
+// x in cut form through pg_gemm_rows.hip, in blocks of 16 mt input rows and `block_rows` rows of W (at most 16 ng), K in
+// `parts` parts (more than one: the raw parts [parts][rows][out_f] to out, without bias).  cut: 6 * in_f * (rows rounded
+// up to 16) bytes.
+pg_status pg_testing_cut_product_dev(int32_t device, void* stream, const float* x, uint64_t rows, uint64_t in_f,
+                                     uint64_t out_f, const void* weight, int32_t storage, const float* scales,
+                                     const float* bias, float* out, int32_t mt, int32_t ng, int32_t block_rows,
+                                     int32_t parts, void* cut) {
+  if (!x || !weight || !out || !cut || (storage == PG_STORE_INT8) != (scales != nullptr))
+    return pgh::fail(PG_INVALID_INPUT, "null argument");
+  if (rows == 0 || rows > 4096 || in_f < 32 || in_f % 32 != 0 || in_f > pgh::kMaxStagedFloats || out_f < 8 || out_f % 8 != 0 ||
+      out_f > (1u << 20) || parts < 1 || parts > 8)
+    return pgh::fail(PG_INVALID_INPUT, "product: sizes");
+  pg_status s;
+  if ((s = select_device(device))) return s;
+  pgk::GemmArgs a{};
+  a.A = static_cast<const float*>(cut); a.W = static_cast<const float*>(weight); a.w_bf16 = storage == PG_STORE_BF16;
+  a.w_scale = scales; a.bias = bias; a.C = out; a.M = (int)rows; a.N = (int)out_f; a.K = (int)in_f; a.lda = (int)in_f;
+  a.ldc = (int)out_f; a.a_cut = 1; a.ws = out; a.ws_floats = (size_t)parts * rows * out_f;
+  PG_HIP(pgk::launch_to_cut(x, cut, (int)rows, (int)in_f, static_cast<hipStream_t>(stream)));
+  PG_HIP(pgk::launch_gemm_cut_rows(a, pgk::GEMM_BIAS, {mt, ng, block_rows, parts}, static_cast<hipStream_t>(stream)));
   return PG_OK;
 }
 

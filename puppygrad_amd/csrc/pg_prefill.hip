@@ -362,10 +362,14 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(GemmArgs a, int parts) {
 // EARLY: everything a thread reads is requested before the first use (a few rows: the launch
 // is a chain of memory round trips and this takes two out of it); otherwise column block by
 // column block, with few registers, for the many rows of a long prompt.
-template <int EPI, bool EARLY>
+// CUT: a.ln_out is in cut form.
+template <int EPI, bool EARLY, bool CUT = false>
 __global__ __launch_bounds__(256) void k_splitk_reduce_ln(GemmArgs a, int parts) {
   __shared__ float red[4];
-  const size_t m = blockIdx.x;
+  // Eight rows of a matrix in cut form share cache lines: their blocks are on one XCD (block % 8), whose L2 then writes
+  // whole lines back.
+  const size_t m = CUT ? blockIdx.x / 64 * 64 + blockIdx.x % 8 * 8 + blockIdx.x % 64 / 8 : blockIdx.x;
+  if (CUT && m >= (size_t)a.M) return;
   const int n4 = a.N / 4;
   const size_t stride = (size_t)a.M * a.N;
   auto bsum = [&](float v) {
@@ -454,7 +458,8 @@ __global__ __launch_bounds__(256) void k_splitk_reduce_ln(GemmArgs a, int parts)
       o.y = (c[q].y - mean) * inv * g.y + b.y;
       o.z = (c[q].z - mean) * inv * g.z + b.z;
       o.w = (c[q].w - mean) * inv * g.w + b.w;
-      *reinterpret_cast<f4*>(a.ln_out + (a.ln_packed ? packed32_index(m, n) : m * a.N + n)) = o;
+      if constexpr (CUT) store_cut4(a.ln_out, cut_rows(a.M), m, n, o);
+      else *reinterpret_cast<f4*>(a.ln_out + (a.ln_packed ? packed32_index(m, n) : m * a.N + n)) = o;
     }
   }
 }
@@ -970,14 +975,14 @@ __device__ __forceinline__ float other_half(float x) {
   return (threadIdx.x & 32) ? __uint_as_float(r.x) : __uint_as_float(r.y);
 }
 
-template <int NWV>  // wavefronts per block
+// NWV: wavefronts per block.  CUT: out is in cut form.
+template <int NWV, bool CUT>
 __global__ __launch_bounds__(64 * NWV) void k_attn_prefill64(const float* __restrict__ qkv, int T,
                                                         int C, int P, float* __restrict__ kcache,
                                                         float* __restrict__ vcache,
                                                         float* __restrict__ out, size_t kv_stride) {
   // blockIdx.z: the sequence (T rows of qkv and out each, panels kv_stride apart)
   qkv += (size_t)blockIdx.z * T * 3 * C;
-  out += (size_t)blockIdx.z * T * C;
   kcache += (size_t)blockIdx.z * kv_stride;
   vcache += (size_t)blockIdx.z * kv_stride;
   constexpr int KT = 32;   // keys per tile
@@ -1172,14 +1177,20 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_prefill64(const float* __rest
   // wavefront w writes d in [8 w, 8 w + 8): lane -> (query l32, 4 d values by half)
   if (qi < T) {
     const float inv = 1.0f / L;
-    float* dst = out + (size_t)qi * C + h * 64;
+    const size_t row = (size_t)blockIdx.z * T + qi;
 #pragma unroll
-    for (int j = 0; j < 64 / NWV / 2; ++j) {
+    for (int j = 0; j < 64 / NWV / 2; j += 4) {
       const int d = (64 / NWV) * wave + (64 / NWV / 2) * half + j;
-      float sum = 0.0f;
+      f4 r;
 #pragma unroll
-      for (int w = 0; w < NWV; ++w) sum += reinterpret_cast<float (*)[KT + 1]>(Vs[w])[d][l32];
-      dst[d] = sum * inv;
+      for (int e = 0; e < 4; ++e) {
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NWV; ++w) sum += reinterpret_cast<float (*)[KT + 1]>(Vs[w])[d + e][l32];
+        r[e] = sum * inv;
+      }
+      if constexpr (CUT) store_cut4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r);
+      else *reinterpret_cast<f4*>(out + row * C + h * 64 + d) = r;
     }
   }
 }
@@ -1234,13 +1245,15 @@ __global__ void k_embed_rows(float* x, const float* wte, const float* wpe, const
 
 // dst[r] = LayerNorm(src[r])  (layer_norm_in_place, cpu.rs:119-143), one block per row
 // (dst_packed: dst is a packed activation matrix, see packed32_index)
+template <bool CUT>
 __global__ __launch_bounds__(256) void k_layer_norm_rows(const float* src, float* dst, int cols,
                                                          const float* g, const float* b,
-                                                         float eps, int dst_packed) {
+                                                         float eps, int dst_form) {
   __shared__ float red[4];
   const float* row = src + (size_t)blockIdx.x * cols;
-  auto out_at = [&](int i) -> float& {
-    return dst[dst_packed ? packed32_index(blockIdx.x, (size_t)i) : (size_t)blockIdx.x * cols + i];
+  auto put = [&](int i, float v) {
+    if (CUT) store_cut1(dst, cut_rows((int)gridDim.x), blockIdx.x, (size_t)i, v);
+    else dst[dst_form == FORM_PACKED32 ? packed32_index(blockIdx.x, (size_t)i) : (size_t)blockIdx.x * cols + i] = v;
   };
   auto bsum = [&](float v) {
 #pragma unroll
@@ -1273,7 +1286,7 @@ __global__ __launch_bounds__(256) void k_layer_norm_rows(const float* src, float
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int i = (int)threadIdx.x + 256 * j;
-      if (i < cols) out_at(i) = (x[j] - mean) * inv * g[i] + b[i];
+      if (i < cols) put(i, (x[j] - mean) * inv * g[i] + b[i]);
     }
     return;
   }
@@ -1287,7 +1300,7 @@ __global__ __launch_bounds__(256) void k_layer_norm_rows(const float* src, float
   }
   const float var = bsum(v) / (float)cols;
   const float inv = 1.0f / sqrtf(var + eps);
-  for (int i = threadIdx.x; i < cols; i += 256) out_at(i) = (row[i] - mean) * inv * g[i] + b[i];
+  for (int i = threadIdx.x; i < cols; i += 256) put(i, (row[i] - mean) * inv * g[i] + b[i]);
 }
 
 
@@ -1329,26 +1342,35 @@ hipError_t launch_splitk_reduce(const GemmArgs& a, int epi, int parts, hipStream
   }
   if (a.ln_out && a.N % 4 == 0 && a.N <= 4096 && a.ldc == a.N) {
     const bool early = a.M <= 64;
+    if (a.ln_cut) {
+      const dim3 rows((a.M + 63) / 64 * 64);
+      if (epi != GEMM_RESID) return hipErrorInvalidValue;
+      if (early) hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_RESID, true, true>), rows, dim3(256), 0, s, a, parts);
+      else hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_RESID, false, true>), rows, dim3(256), 0, s, a, parts);
+      *ln_done = true;
+      return hipGetLastError();
+    }
+    const dim3 rows(a.M);
     if (epi == GEMM_BIAS && early)
-      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_BIAS, true>), dim3(a.M), dim3(256), 0, s, a, parts);
+      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_BIAS, true>), rows, dim3(256), 0, s, a, parts);
     else if (epi == GEMM_BIAS)
-      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_BIAS, false>), dim3(a.M), dim3(256), 0, s, a, parts);
+      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_BIAS, false>), rows, dim3(256), 0, s, a, parts);
     else if (epi == GEMM_GELU && early)
-      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_GELU, true>), dim3(a.M), dim3(256), 0, s, a, parts);
+      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_GELU, true>), rows, dim3(256), 0, s, a, parts);
     else if (epi == GEMM_GELU)
-      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_GELU, false>), dim3(a.M), dim3(256), 0, s, a, parts);
+      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_GELU, false>), rows, dim3(256), 0, s, a, parts);
     else if (epi == GEMM_SQRELU && early)
-      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_SQRELU, true>), dim3(a.M), dim3(256), 0, s, a, parts);
+      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_SQRELU, true>), rows, dim3(256), 0, s, a, parts);
     else if (epi == GEMM_SQRELU)
-      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_SQRELU, false>), dim3(a.M), dim3(256), 0, s, a, parts);
+      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_SQRELU, false>), rows, dim3(256), 0, s, a, parts);
     else if (epi == GEMM_RESID && early)
-      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_RESID, true>), dim3(a.M), dim3(256), 0, s, a, parts);
+      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_RESID, true>), rows, dim3(256), 0, s, a, parts);
     else if (epi == GEMM_RESID_SCALED && early)
-      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_RESID_SCALED, true>), dim3(a.M), dim3(256), 0, s, a, parts);
+      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_RESID_SCALED, true>), rows, dim3(256), 0, s, a, parts);
     else if (epi == GEMM_RESID)
-      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_RESID, false>), dim3(a.M), dim3(256), 0, s, a, parts);
+      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_RESID, false>), rows, dim3(256), 0, s, a, parts);
     else if (epi == GEMM_RESID_SCALED)
-      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_RESID_SCALED, false>), dim3(a.M), dim3(256), 0, s, a, parts);
+      hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_RESID_SCALED, false>), rows, dim3(256), 0, s, a, parts);
     else
       return hipErrorInvalidValue;
     *ln_done = true;
@@ -1659,7 +1681,8 @@ hipError_t launch_gemm(const GemmArgs& a, int epi, int num_cus, hipStream_t s) {
     return a.ln_packed ? hipErrorInvalidValue
                        : launch_rms_rows(a.C, a.ln_out, a.M, a.rms_cols, a.N, a.ln_g, a.ln_eps, 1.0f, nullptr, s);
   if (e == hipSuccess && a.ln_out && !ln_done)
-    e = launch_layer_norm_rows(a.C, a.ln_out, a.M, a.N, a.ln_g, a.ln_b, a.ln_eps, s, a.ln_packed);
+    e = launch_layer_norm_rows(a.C, a.ln_out, a.M, a.N, a.ln_g, a.ln_b, a.ln_eps, s,
+                               a.ln_cut ? FORM_CUT : a.ln_packed ? FORM_PACKED32 : FORM_ROWS);
   return e;
 }
 
@@ -1704,7 +1727,13 @@ bool gemm_takes_rows32(int M, int K, int lda, int w_bf16) {
 
 namespace {
 hipError_t launch_gemm_form(const GemmArgs& a, int epi, int num_cus, hipStream_t s, bool* ln_done) {
-  if (!gemm_supported(a)) return hipErrorInvalidValue;
+  if (a.a_cut) {
+    CutRowsPlan plan;
+    if (!gemm_cut_rows_plan(a, num_cus, &plan)) return hipErrorInvalidValue;
+    const hipError_t e = launch_gemm_cut_rows(a, epi, plan, s);
+    return e != hipSuccess || plan.parts == 1 ? e : launch_splitk_reduce(a, epi, plan.parts, s, ln_done);
+  }
+  if (!gemm_supported(a) || a.c_cut || a.ln_cut) return hipErrorInvalidValue;
   const bool packed = a.a_packed || a.c_packed || a.ln_packed;
   if (a.w_scale && (packed || a.w_bf16)) return hipErrorInvalidValue;
   // A small decode batch over a short K: whole rows of W per wavefront, no MFMA tiles.
@@ -1745,20 +1774,23 @@ hipError_t launch_gemm_form(const GemmArgs& a, int epi, int num_cus, hipStream_t
 
 hipError_t launch_attn_prefill(const float* qkv, int T, int C, int H, int head_dim, int P,
                                float* kcache, float* vcache, float* out, float* scratch,
-                               hipStream_t s, int nseq, size_t kv_stride) {
-  if (nseq < 1 || nseq > 65535) return hipErrorInvalidValue;
+                               hipStream_t s, int nseq, size_t kv_stride, int out_form) {
+  if (nseq < 1 || nseq > 65535 || out_form == FORM_PACKED32 || (out_form && head_dim != 64)) return hipErrorInvalidValue;
   if (head_dim == 64) {
     const int qblocks = (T + 31) / 32;
     // Eight wavefronts share a query block's key tiles.  Several sequences of up to 512 tokens
     // are many blocks of at most 16 tiles each: four wavefronts (half the LDS, two blocks to a
     // CU) measured 2 to 4 % shorter prefills there (XL bf16, 32 x 512 tokens: 187 -> 179 ms);
     // single prompts are equal up to 512 tokens and 3 % slower at 1024.
-    if (nseq >= 2 && T <= 512)
-      hipLaunchKernelGGL(k_attn_prefill64<4>, dim3(H, qblocks, nseq), dim3(256), 0, s, qkv, T, C, P, kcache,
-                         vcache, out, kv_stride);
-    else
-      hipLaunchKernelGGL(k_attn_prefill64<8>, dim3(H, qblocks, nseq), dim3(512), 0, s, qkv, T, C, P, kcache,
-                         vcache, out, kv_stride);
+    const dim3 grid(H, qblocks, nseq);
+    const bool four = nseq >= 2 && T <= 512;
+#define PG_ATTN(NWV, CUT) \
+  hipLaunchKernelGGL((k_attn_prefill64<NWV, CUT>), grid, dim3(64 * NWV), 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride)
+    if (four && out_form == FORM_CUT) PG_ATTN(4, true);
+    else if (four) PG_ATTN(4, false);
+    else if (out_form == FORM_CUT) PG_ATTN(8, true);
+    else PG_ATTN(8, false);
+#undef PG_ATTN
   } else {
     // (test-sized models: one launch per sequence, all using the same scratch in turn)
     const int n = T * H;
@@ -1778,10 +1810,12 @@ hipError_t launch_embed_rows(float* x, const float* wte, const float* wpe, const
 }
 
 hipError_t launch_layer_norm_rows(const float* src, float* dst, int rows, int cols, const float* g,
-                                  const float* b, float eps, hipStream_t s, int dst_packed) {
-  if (dst_packed && rows > 32) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_layer_norm_rows, dim3(rows), dim3(256), 0, s, src, dst, cols, g, b, eps,
-                     dst_packed);
+                                  const float* b, float eps, hipStream_t s, int dst_form) {
+  if ((dst_form == FORM_PACKED32 && rows > 32) || (dst_form == FORM_CUT && cols % 8 != 0)) return hipErrorInvalidValue;
+  if (dst_form == FORM_CUT)
+    hipLaunchKernelGGL(k_layer_norm_rows<true>, dim3(rows), dim3(256), 0, s, src, dst, cols, g, b, eps, dst_form);
+  else
+    hipLaunchKernelGGL(k_layer_norm_rows<false>, dim3(rows), dim3(256), 0, s, src, dst, cols, g, b, eps, dst_form);
   return hipGetLastError();
 }
 
