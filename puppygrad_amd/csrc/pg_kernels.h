@@ -310,6 +310,11 @@ hipError_t launch_gemm_grouped(const GemmArgs& a, int epilogue, int tile_rows, c
 hipError_t launch_attn_prefill(const float* qkv, int T, int C, int H, int head_dim, int P,
                                float* kcache, float* vcache, float* out, float* scratch,
                                hipStream_t s, int nseq = 1, size_t kv_stride = 0, int out_form = 0);
+// The same with both products on the bf16 matrix cores (pg_attn_cut.hip), head_dim 64, in blocks of one of these shapes:
+// 41, 22, 42, 24 (groups of 32 queries, groups of keys).  attn_cut_shape: the one to take, 0: none.
+int attn_cut_shape(int T, int H, int nseq);
+hipError_t launch_attn_prefill_cut(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, float* out,
+                                   hipStream_t s, int nseq, size_t kv_stride, int out_form, int shape);
 // rows rows; row t is position t % period of its sequence (wpe may be null)
 hipError_t launch_embed_rows(float* x, const float* wte, const float* wpe, const uint32_t* ids,
                              int rows, int C, hipStream_t s, int w_bf16 = 0, int period = 0);

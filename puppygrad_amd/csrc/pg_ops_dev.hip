@@ -395,6 +395,25 @@ pg_status pg_testing_cut_product_dev(int32_t device, void* stream, const float* 
   return PG_OK;
 }
 
+// Attention of `sequences` prompts of `rows` tokens each, head size 64, keys and values to panels [sequences][heads][rows][64]:
+// in blocks of the given shape of pg_attn_cut.hip (0: as the planner has it).
+pg_status pg_testing_attention_rows_dev(int32_t device, void* stream, const float* qkv, uint64_t rows, uint64_t heads,
+                                        uint64_t sequences, int32_t shape, float* keys, float* values, float* out) {
+  if (!qkv || !keys || !values || !out) return pgh::fail(PG_INVALID_INPUT, "null argument");
+  if (rows == 0 || rows > 4096 || heads == 0 || heads > 64 || sequences == 0 || sequences > 1024)
+    return pgh::fail(PG_INVALID_INPUT, "attention: sizes");
+  pg_status s;
+  if ((s = select_device(device))) return s;
+  const int T = (int)rows, H = (int)heads, C = 64 * H;
+  const size_t stride = (size_t)H * T * 64;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (shape > 0)
+    PG_HIP(pgk::launch_attn_prefill_cut(qkv, T, C, H, T, keys, values, out, st, (int)sequences, stride, pgk::FORM_ROWS, shape));
+  else
+    PG_HIP(pgk::launch_attn_prefill(qkv, T, C, H, 64, T, keys, values, out, nullptr, st, (int)sequences, stride));
+  return PG_OK;
+}
+
 // launch_gemm_grouped: `rows` with their padding; out has out_f columns, or half as many (silu_pair).
 pg_status pg_testing_grouped_dev(int32_t device, void* stream, const float* x, uint64_t rows, uint64_t in_f,
                                  uint64_t out_f, const void* weight, int32_t storage, int32_t silu_pair,

@@ -1777,11 +1777,13 @@ hipError_t launch_attn_prefill(const float* qkv, int T, int C, int H, int head_d
                                hipStream_t s, int nseq, size_t kv_stride, int out_form) {
   if (nseq < 1 || nseq > 65535 || out_form == FORM_PACKED32 || (out_form && head_dim != 64)) return hipErrorInvalidValue;
   if (head_dim == 64) {
+    if (const int shape = attn_cut_shape(T, H, nseq))
+      return launch_attn_prefill_cut(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, out_form, shape);
     const int qblocks = (T + 31) / 32;
     // Eight wavefronts share a query block's key tiles.  Several sequences of up to 512 tokens
-    // are many blocks of at most 16 tiles each: four wavefronts (half the LDS, two blocks to a
-    // CU) measured 2 to 4 % shorter prefills there (XL bf16, 32 x 512 tokens: 187 -> 179 ms);
-    // single prompts are equal up to 512 tokens and 3 % slower at 1024.
+    // are more blocks of at most 16 tiles each: four wavefronts (half the LDS, two blocks to a
+    // CU) measured 2 to 4 % shorter prefills there (before the many-block ones went to
+    // pg_attn_cut.hip).
     const dim3 grid(H, qblocks, nseq);
     const bool four = nseq >= 2 && T <= 512;
 #define PG_ATTN(NWV, CUT) \
