@@ -635,13 +635,13 @@ __global__ __launch_bounds__(256) void k_gemv_rows(GemmArgs a) {
 // are used twice).
 // WT: W holds f32 (0), bf16 (1) or int8 rows with a.w_scale (2; a weight is (float)q * scale,
 // formed when its piece is read back; row-major input only).
-// GROUPED: see launch_gemm_grouped; blockIdx.z is the tile of 32 rows.
+// GROUPED: see launch_gemm_grouped; blockIdx.z is the tile of 32 rows (M16: 16).
 template <int EPI, int WT, bool XP, bool M16, int NR, int MT, bool GROUPED = false>
 __global__ __launch_bounds__(512) void k_gemm_rows32(GemmArgs a) {
   static_assert(NR == 32 || (NR == 16 && M16), "rows per block");
   static_assert(MT == 1 || (MT == 2 && !M16 && !XP), "input rows");
   static_assert(WT != 2 || !XP, "int8 rows: row-major input");
-  static_assert(!GROUPED || (!XP && !M16 && MT == 1 && WT != 2), "grouped rows");
+  static_assert(!GROUPED || (!XP && MT == 1 && WT != 2), "grouped rows");
   constexpr int CPP = WT == 2 ? 16 : WT == 1 ? 8 : 4;  // columns in a 16-byte piece of a W row
   constexpr int XF = CPP / 4;            // float4 of input that meet one piece
   constexpr int KS = 4 * CPP;            // columns per step: 64 bytes of a row of W
@@ -650,13 +650,14 @@ __global__ __launch_bounds__(512) void k_gemm_rows32(GemmArgs a) {
   constexpr int WSTR = 20;               // row stride of the W tile (floats; 64 bytes + pad)
   constexpr int XSTR = KS + 4;           // row stride of the input tile
   // per wavefront: W tile, input tile; the reduce tile [32 MT][33] lies over them
-  constexpr int SLAB = 32 * WSTR + 32 * MT * XSTR > 32 * MT * 33 ? 32 * WSTR + 32 * MT * XSTR : 32 * MT * 33;
+  constexpr int TR = M16 ? 16 : 32 * MT;  // input rows
+  constexpr int SLAB = 32 * WSTR + TR * XSTR > TR * 33 ? 32 * WSTR + TR * XSTR : TR * 33;
   // steps requested ahead (3, 4, 6 measured slower; 64 rows against int8 rows: a second step's 64 input
   // registers spill, large prompt of 37 tokens 2.85 against 2.28 ms)
   constexpr int PD = WT == 2 && MT == 2 ? 1 : 2;
   __shared__ __attribute__((aligned(16))) float slab[8][SLAB];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int row0 = GROUPED ? 32 * (int)blockIdx.z : 0, M = GROUPED ? 32 : a.M;
+  const int row0 = GROUPED ? TR * (int)blockIdx.z : 0, M = GROUPED ? TR : a.M;
   const int group = GROUPED ? a.group_tile[blockIdx.z] : 0;
   if (GROUPED && group < 0) return;
   // operand position of the lane: row orow, 16-byte piece opc of the row's 64 bytes
@@ -1694,16 +1695,23 @@ hipError_t launch_gemm_grouped(const GemmArgs& a0, int epi, int tile_rows, const
   if (!gemm_supported(a) || a.K % 32 != 0 || a.w_scale || a.bias || a.N % 2 != 0 || !group_tile || a.M % tile_rows != 0)
     return hipErrorInvalidValue;
   if (epi != GEMM_BIAS && epi != GEMM_SILU_PAIR) return hipErrorInvalidValue;
-  if (tile_rows == 32) {  // few rows: blocks own rows of W, as many as leave two blocks to a CU
-    const int tiles = a.M / 32;
+  if (tile_rows == 32 || tile_rows == 16) {  // few rows: blocks own rows of W, as many as leave two blocks to a CU
+    const int tiles = a.M / tile_rows;
     a.rows_per_block = std::max(8, std::min(32, (int)((long)a.N * std::min(tiles, 16) / 512) / 2 * 2));
     const dim3 grid((a.N + a.rows_per_block - 1) / a.rows_per_block, 1, tiles);
     if (tiles > 65535) return hipErrorInvalidValue;
-#define PG_ROWS(EPI, WT) hipLaunchKernelGGL((k_gemm_rows32<EPI, WT, false, false, 32, 1, true>), grid, dim3(512), 0, s, a)
-    if (epi == GEMM_BIAS && a.w_bf16) PG_ROWS(GEMM_BIAS, 1);
-    else if (epi == GEMM_BIAS) PG_ROWS(GEMM_BIAS, 0);
-    else if (a.w_bf16) PG_ROWS(GEMM_SILU_PAIR, 1);
-    else PG_ROWS(GEMM_SILU_PAIR, 0);
+#define PG_ROWS(EPI, WT)                                                                                             \
+  if (tile_rows == 16) hipLaunchKernelGGL((k_gemm_rows32<EPI, WT, false, true, 32, 1, true>), grid, dim3(512), 0, s, a); \
+  else hipLaunchKernelGGL((k_gemm_rows32<EPI, WT, false, false, 32, 1, true>), grid, dim3(512), 0, s, a)
+    if (epi == GEMM_BIAS && a.w_bf16) {
+      PG_ROWS(GEMM_BIAS, 1);
+    } else if (epi == GEMM_BIAS) {
+      PG_ROWS(GEMM_BIAS, 0);
+    } else if (a.w_bf16) {
+      PG_ROWS(GEMM_SILU_PAIR, 1);
+    } else {
+      PG_ROWS(GEMM_SILU_PAIR, 0);
+    }
 #undef PG_ROWS
     return hipGetLastError();
   }

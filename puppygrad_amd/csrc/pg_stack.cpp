@@ -832,6 +832,7 @@ namespace {
 // Slots to a tile of the sorted pairs: few rows stream the experts' weights, many fill tiles.
 int moe_tile_rows(const pgk::Moe& m, int rows) {
   const long pairs = (long)rows * m.top;
+  if (pairs <= 12L * m.experts) return 16;
   if (pairs <= 32L * m.experts) return 32;
   return m.w_bf16 && pairs >= 512L * m.experts ? 128 : 64;
 }
