@@ -232,6 +232,9 @@ struct GemmArgs {
   int lda, ldc;
   float* ws = nullptr;    // optional workspace for the split-K form (may be nullptr)
   size_t ws_floats = 0;   // its size
+  // (GEMM_BIAS without bias or norm) Optional: where the chosen form is the 32-row kernel with K cut, the parts are left in
+  // ws [parts][M][N] and their number goes here; otherwise it stays what it is.
+  int* raw_parts = nullptr;
   int rows_per_block = 0;  // 32-row kernel: rows of W a block owns (filled by its launcher)
   int tail_first = 0;     // filled by gemm_tail_plan: first tile of the tail that is cut along K,
   int tail_parts = 1;     // and the number of parts

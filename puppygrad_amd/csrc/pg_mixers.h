@@ -279,7 +279,10 @@ struct MoeRoute {
   int* tile;       // [max_slots / tile_rows]: expert of a tile, -1 past the end
 };
 int moe_max_slots(const Moe& m, int rows, int tile_rows);
-hipError_t launch_moe_route(const Moe& m, const MoeRoute& r, const float* logits, int rows, hipStream_t s);
+// logits: [rows][experts_pad], or the raw parts of a product with a cut K, [parts][rows][experts_pad], where
+// moe_route_adds_parts.
+bool moe_route_adds_parts(const Moe& m, int rows);
+hipError_t launch_moe_route(const Moe& m, const MoeRoute& r, const float* logits, int rows, hipStream_t s, int parts = 1);
 
 // What a one-token step keeps on the device: the position of the step that is running, that of the
 // next one, and, for generations that run ahead of the host, where the next ids are listed

@@ -28,17 +28,17 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
-// One wavefront: the `top` largest logits of z[experts] in descending order (equal ones: the lower
+// One wavefront: the `top` largest of the logits z(e), e < experts, in descending order (equal ones: the lower
 // index first), each with its softmax over all experts; each(k, expert, weight) in every lane.
 // NP: logits per lane, experts <= 64 NP.
-template <int NP, typename F>
-__device__ __forceinline__ void choose_experts(const float* z, int experts, int top, F each) {
+template <int NP, typename Z, typename F>
+__device__ __forceinline__ void choose_experts(Z z, int experts, int top, F each) {
   const int lane = threadIdx.x & 63;
   float v[NP], mx = -INFINITY;
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     const int e = lane + 64 * p;
-    v[p] = e < experts ? z[e] : -INFINITY;
+    v[p] = e < experts ? z(e) : -INFINITY;
     mx = fmaxf(mx, v[p]);
   }
   mx = wave_max(mx);
@@ -72,8 +72,8 @@ __device__ __forceinline__ void choose_experts(const float* z, int experts, int 
     each(k, at, expf(best - mx) / sum);
   }
 }
-template <typename F>
-__device__ __forceinline__ void choose_any(const float* z, int experts, int top, F each) {
+template <typename Z, typename F>
+__device__ __forceinline__ void choose_any(Z z, int experts, int top, F each) {
   if (experts <= 64) choose_experts<1>(z, experts, top, each);
   else if (experts <= 256) choose_experts<4>(z, experts, top, each);
   else choose_experts<kPerLane>(z, experts, top, each);
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) void k_moe_act(Moe m, MoeRow r) {
     z = zs;
   }
   if (wave == 0)
-    choose_any(z, m.experts, k + 1, [&](int i, int e, float w) {
+    choose_any([&](int e) { return z[e]; }, m.experts, k + 1, [&](int i, int e, float w) {
       if (i == k && tid == 0) {
         expert = e;
         if (blockIdx.x == 0) {
@@ -289,7 +289,8 @@ __global__ __launch_bounds__(256) void k_moe_choose(Moe m, MoeRoute r, const flo
   __syncthreads();
   for (int i = wave; i < kRouteRows && row0 + i < rows; i += 4) {
     const int row = row0 + i;
-    choose_any(logits + (size_t)row * m.experts_pad, m.experts, m.top, [&](int k, int e, float w) {
+    const float* z = logits + (size_t)row * m.experts_pad;
+    choose_any([&](int e) { return z[e]; }, m.experts, m.top, [&](int k, int e, float w) {
       if ((tid & 63) == 0) {
         const size_t p = (size_t)row * m.top + k;
         r.expert[p] = e;
@@ -345,7 +346,8 @@ __global__ __launch_bounds__(256) void k_moe_place(Moe m, MoeRoute r, int pairs)
 
 // All of it in one block, for a few rows.
 constexpr int kRouteSmallRows = 128, kRouteSmallPairs = 4096;
-__global__ __launch_bounds__(1024) void k_moe_route_small(Moe m, MoeRoute r, const float* logits, int rows) {
+// logits: [parts][rows][experts_pad], the parts of a cut K to be added here (a reduction of its own was 4.5 us a layer).
+__global__ __launch_bounds__(1024) void k_moe_route_small(Moe m, MoeRoute r, const float* logits, int rows, int parts) {
   __shared__ int count[kMoeMaxExperts], first[kMoeMaxExperts + 1];
   __shared__ int pair[kRouteSmallPairs];  // expert and number within it
   const int tid = threadIdx.x, wave = tid >> 6;
@@ -353,14 +355,37 @@ __global__ __launch_bounds__(1024) void k_moe_route_small(Moe m, MoeRoute r, con
   for (int i = tid; i < r.max_slots; i += 1024) r.slot_row[i] = -1;
   for (int i = tid; i < r.max_slots / r.tile_rows; i += 1024) r.tile[i] = -1;
   __syncthreads();
-  for (int row = wave; row < rows; row += 16)
-    choose_any(logits + (size_t)row * m.experts_pad, m.experts, m.top, [&](int k, int e, float w) {
+  auto logit = [&](int row, int e) {
+    const float* z = logits + (size_t)row * m.experts_pad + e;
+    const size_t stride = (size_t)rows * m.experts_pad;
+    float v[8];
+#pragma unroll
+    for (int p = 0; p < 8; ++p) v[p] = z[min(p, parts - 1) * stride];
+    float sum = v[0];
+#pragma unroll
+    for (int p = 1; p < 8; ++p)
+      if (p < parts) sum += v[p];
+    return sum;
+  };
+  auto choose = [&](int row, auto z) {
+    choose_any(z, m.experts, m.top, [&](int k, int e, float w) {
       if ((tid & 63) == 0) {
         const size_t p = (size_t)row * m.top + k;
         r.weight[p] = w;
         pair[p] = e << 16 | atomicAdd(&count[e], 1);
       }
     });
+  };
+  if (m.experts <= 64) {  // a logit a lane: those of two rows are asked for together
+    const int e = min(tid & 63, m.experts - 1);
+    for (int row = wave; row < rows; row += 32) {
+      const float z0 = logit(row, e), z1 = logit(min(row + 16, rows - 1), e);
+      choose(row, [&](int) { return z0; });
+      if (row + 16 < rows) choose(row + 16, [&](int) { return z1; });
+    }
+  } else {
+    for (int row = wave; row < rows; row += 16) choose(row, [&](int e) { return logit(row, e); });
+  }
   __syncthreads();
   if (tid < 64) first_slots(m, r.tile_rows, count, first);
   __syncthreads();
@@ -417,12 +442,15 @@ int moe_max_slots(const Moe& m, int rows, int tile_rows) {
   return (int)((pairs + used * (tile_rows - 1)) / tile_rows * tile_rows);
 }
 
-hipError_t launch_moe_route(const Moe& m, const MoeRoute& r, const float* logits, int rows, hipStream_t s) {
-  if (m.experts > kMoeMaxExperts || m.top > kMoeMaxTop || m.top > m.experts || r.max_slots != moe_max_slots(m, rows, r.tile_rows))
+bool moe_route_adds_parts(const Moe& m, int rows) { return rows <= kRouteSmallRows && rows * m.top <= kRouteSmallPairs; }
+
+hipError_t launch_moe_route(const Moe& m, const MoeRoute& r, const float* logits, int rows, hipStream_t s, int parts) {
+  if (m.experts > kMoeMaxExperts || m.top > kMoeMaxTop || m.top > m.experts || r.max_slots != moe_max_slots(m, rows, r.tile_rows) ||
+      parts < 1 || parts > 8 || (parts > 1 && !moe_route_adds_parts(m, rows)))
     return hipErrorInvalidValue;
   const int pairs = rows * m.top;
-  if (rows <= kRouteSmallRows && pairs <= kRouteSmallPairs) {
-    hipLaunchKernelGGL(k_moe_route_small, dim3(1), dim3(1024), 0, s, m, r, logits, rows);
+  if (moe_route_adds_parts(m, rows)) {
+    hipLaunchKernelGGL(k_moe_route_small, dim3(1), dim3(1024), 0, s, m, r, logits, rows, parts);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(k_moe_clear, dim3((std::max(m.experts, r.max_slots) + 255) / 256), dim3(256), 0, s, r, m.experts,

@@ -1508,6 +1508,10 @@ hipError_t launch_gemm_rows32(const GemmArgs& a, int epi, int parts, int num_cus
                    : launch_gemm_rows32_x<WT, false>(a, epi, parts, num_cus, s);
   }
   if (e != hipSuccess) return e;
+  if (parts > 1 && a.raw_parts) {
+    *a.raw_parts = parts;
+    return hipGetLastError();
+  }
   if (parts > 1) return launch_splitk_reduce(a, epi, parts, s, ln_done);
   return hipGetLastError();
 }
@@ -1674,6 +1678,7 @@ hipError_t launch_gemm(const GemmArgs& a, int epi, int num_cus, hipStream_t s) {
   if ((epi == GEMM_RESID_SCALED) != (a.col_scale != nullptr) || (a.rms_cols && epi != GEMM_RESID_SCALED))
     return hipErrorInvalidValue;
   if (a.post_x && (epi != GEMM_BIAS || a.ln_out || a.ldc != a.N)) return hipErrorInvalidValue;
+  if (a.raw_parts && (epi != GEMM_BIAS || a.bias || a.ln_out || a.post_x)) return hipErrorInvalidValue;
   bool ln_done = false;
   hipError_t e = launch_gemm_form(a, epi, num_cus, s, &ln_done);
   if (e == hipSuccess && a.post_x && !ln_done)

@@ -855,39 +855,6 @@ struct MoeSizes {
   }
 };
 
-// x += norm2 of the experts' output, rows of x whose router logits are in b.logits.  sub: as many rows
-// of working memory.
-pg_status moe_rows(const pg_model* model, const StackLayer& l, const StackCache::MoeBuffers& b, float* x, float* sub, int rows,
-                   hipStream_t s, ProfileMarks* marks) {
-  const StackModel& m = *model->stack;
-  const pgk::Moe& e = l.ffn.moe;
-  const int Cp = m.width_pad;
-  if (rows == 1) {
-    pgk::MoeRow r{};
-    r.x = x; r.logits = b.logits; r.width = m.width; r.width_pad = Cp; r.eps = m.eps;
-    r.act = b.act; r.out = sub; r.expert = b.route.expert; r.weight = b.route.weight;
-    PG_HIP(pgk::launch_moe_row(e, r, s));
-    PG_MARK(kMlpFc);
-    PG_HIP(pgk::launch_add_norm_rows(x, sub, rows, m.width, Cp, l.norm2, m.eps, nullptr, nullptr, 0, s));
-    return PG_OK;
-  }
-  pgk::MoeRoute t = b.route;
-  t.tile_rows = moe_tile_rows(e, rows);
-  t.max_slots = pgk::moe_max_slots(e, rows, t.tile_rows);
-  PG_HIP(pgk::launch_moe_route(e, t, b.logits, rows, s));
-  pgk::GemmArgs g{};
-  g.w_bf16 = e.w_bf16; g.M = t.max_slots;
-  g.A = x; g.lda = Cp; g.W = static_cast<const float*>(e.gate_up); g.N = 2 * e.ff_pad; g.K = Cp;
-  g.C = b.act; g.ldc = e.ff_pad;
-  PG_HIP(pgk::launch_gemm_grouped(g, pgk::GEMM_SILU_PAIR, t.tile_rows, t.tile, t.slot_row, s));
-  PG_MARK(kMlpFc);
-  g.A = b.act; g.lda = e.ff_pad; g.W = static_cast<const float*>(e.down); g.N = Cp; g.K = e.ff_pad;
-  g.C = b.slot_out; g.ldc = Cp;
-  PG_HIP(pgk::launch_gemm_grouped(g, pgk::GEMM_BIAS, t.tile_rows, t.tile, nullptr, s));
-  PG_HIP(pgk::launch_add_norm_rows(x, b.slot_out, rows, m.width, Cp, l.norm2, m.eps, t.slot, t.weight, e.top, s));
-  return PG_OK;
-}
-
 }  // namespace
 
 pg_status stack_cache_create(const pg_model* model, pg_kv_cache* c) {
@@ -1002,8 +969,10 @@ struct Gemm {
   // C[n_rows][N] = epilogue(A[n_rows][lda] . W[N][K]^T + bias)
   // (post_x: the rows' norm is added to it instead, C is working memory)
   hipError_t product(int n_rows, const float* A, int lda, const void* W, float* C, int N, int K, const float* bias = nullptr,
-                     int epilogue = pgk::GEMM_BIAS, float* post_x = nullptr, const float* post_gain = nullptr) const {
+                     int epilogue = pgk::GEMM_BIAS, float* post_x = nullptr, const float* post_gain = nullptr,
+                     int* raw_parts = nullptr) const {
     pgk::GemmArgs a{};
+    a.raw_parts = raw_parts;
     a.A = A; a.w_bf16 = m->w_bf16; a.W = static_cast<const float*>(W); a.bias = bias; a.C = C;
     a.M = n_rows; a.N = N; a.K = K; a.lda = lda; a.ldc = N;
     a.ws = ws; a.ws_floats = ws_floats;
@@ -1013,6 +982,41 @@ struct Gemm {
     return pgk::launch_gemm(a, epilogue, m->num_cus, s);
   }
 };
+
+// x += norm2 of the experts' output for rows of x.  sub: as many rows of working memory.
+pg_status moe_rows(const pg_model* model, const StackLayer& l, const StackCache::MoeBuffers& b, const Gemm& gemm, float* x,
+                   float* sub, int rows, hipStream_t s, ProfileMarks* marks) {
+  const StackModel& m = *model->stack;
+  const pgk::Moe& e = l.ffn.moe;
+  const int Cp = m.width_pad;
+  int parts = 1;  // of the router's product that launch_moe_route adds up
+  PG_HIP(gemm.product(rows, x, Cp, l.ffn.router_w, b.logits, e.experts_pad, Cp, nullptr, pgk::GEMM_BIAS, nullptr, nullptr,
+                      rows > 1 && pgk::moe_route_adds_parts(e, rows) ? &parts : nullptr));
+  if (rows == 1) {
+    pgk::MoeRow r{};
+    r.x = x; r.logits = b.logits; r.width = m.width; r.width_pad = Cp; r.eps = m.eps;
+    r.act = b.act; r.out = sub; r.expert = b.route.expert; r.weight = b.route.weight;
+    PG_HIP(pgk::launch_moe_row(e, r, s));
+    PG_MARK(kMlpFc);
+    PG_HIP(pgk::launch_add_norm_rows(x, sub, rows, m.width, Cp, l.norm2, m.eps, nullptr, nullptr, 0, s));
+    return PG_OK;
+  }
+  pgk::MoeRoute t = b.route;
+  t.tile_rows = moe_tile_rows(e, rows);
+  t.max_slots = pgk::moe_max_slots(e, rows, t.tile_rows);
+  PG_HIP(pgk::launch_moe_route(e, t, parts > 1 ? gemm.ws : b.logits, rows, s, parts));
+  pgk::GemmArgs g{};
+  g.w_bf16 = e.w_bf16; g.M = t.max_slots;
+  g.A = x; g.lda = Cp; g.W = static_cast<const float*>(e.gate_up); g.N = 2 * e.ff_pad; g.K = Cp;
+  g.C = b.act; g.ldc = e.ff_pad;
+  PG_HIP(pgk::launch_gemm_grouped(g, pgk::GEMM_SILU_PAIR, t.tile_rows, t.tile, t.slot_row, s));
+  PG_MARK(kMlpFc);
+  g.A = b.act; g.lda = e.ff_pad; g.W = static_cast<const float*>(e.down); g.N = Cp; g.K = e.ff_pad;
+  g.C = b.slot_out; g.ldc = Cp;
+  PG_HIP(pgk::launch_gemm_grouped(g, pgk::GEMM_BIAS, t.tile_rows, t.tile, nullptr, s));
+  PG_HIP(pgk::launch_add_norm_rows(x, b.slot_out, rows, m.width, Cp, l.norm2, m.eps, t.slot, t.weight, e.top, s));
+  return PG_OK;
+}
 
 // Logits of rows of x (rows_at: device list, null for rows 0 .. n - 1) into dst.
 pg_status head_rows(const pg_model* model, const Gemm& gemm, const float* x, float* h, const int* rows_at,
@@ -1132,10 +1136,10 @@ pg_status post_norm_step(const pg_model* model, pg_kv_cache* c, ProfileMarks* ma
       PG_HIP(leave(st.act, f.down_w, f.down_b, f.ff_pad, nullptr, 0, 0, l.norm2));
     } else if (f.kind == PostFeedForward::kMoe) {
       const bool fused = B == 1 && pgk::moe_router_fits(f.moe, Cp);
-      if (!fused) PG_HIP(enter(f.router_w, nullptr, st.moe.logits, f.moe.experts_pad, false));
       if (B > 1) {
-        if (pg_status e = moe_rows(model, l, st.moe, x, st.sub, B, s, marks)) return e;
+        if (pg_status e = moe_rows(model, l, st.moe, gemm, x, st.sub, B, s, marks)) return e;
       } else {
+        if (!fused) PG_HIP(enter(f.router_w, nullptr, st.moe.logits, f.moe.experts_pad, false));
         pgk::MoeRow r{};
         r.x = x; r.width = m.width; r.width_pad = Cp; r.eps = m.eps;
         r.act = st.moe.act; r.out = st.sub; r.expert = st.moe.route.expert; r.weight = st.moe.route.weight;
@@ -1397,8 +1401,7 @@ pg_status post_norm_rows(const pg_model* model, pg_kv_cache* c, const uint32_t* 
       PG_MARK(kMlpFc);
       PG_HIP(gemm.product(R, act, f.ff_pad, f.down_w, sub, (int)Cp, f.ff_pad, f.down_b, pgk::GEMM_BIAS, x, l.norm2));
     } else if (f.kind == PostFeedForward::kMoe) {
-      PG_HIP(gemm.product(R, x, (int)Cp, f.router_w, moe.logits, f.moe.experts_pad, (int)Cp));
-      if (pg_status e = moe_rows(model, l, moe, x, sub, R, s, marks)) return e;
+      if (pg_status e = moe_rows(model, l, moe, gemm, x, sub, R, s, marks)) return e;
     }
     PG_MARK(kMlpProj);
   }
