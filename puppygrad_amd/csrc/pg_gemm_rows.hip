@@ -247,18 +247,21 @@ constexpr float kReduceLaunch = 4.5f, kNormLaunch = 4.0f, kNormValues = 2.0f;
 // first).  They end where a CU has more than one block and the tiles of pg_gemm_cut.hip, which read an input row once
 // for 128 columns instead of 64, have one each:
 //  - f32 rows: width 1600, 150 rows 7.42 / 6.68, 200 rows 7.93 / 8.40; 1280, 256 rows 4.87 / 4.66, 300 rows 5.65 / 5.87;
-//    1024, 300 rows 2.95 / 2.65, 350 rows 3.08 / 3.17; 768, 400 rows 1.40 / 1.26.  33 rows, 1280: 2.62 / 2.26.
+//    1024, 300 rows 2.95 / 2.65, 350 rows 3.08 / 3.17.  33 rows, 1280: 2.62 / 2.26.  At width 768 the tiles leave a third of
+//    the CUs without one at 1024 rows yet: 500 rows 1.45 / 1.30, 700 rows 1.77 / 1.76, 1024 rows 2.07 / 1.99.
 //  - bf16 rows: 1600, 100 rows 4.57 / 4.06, 150 rows 5.09 / 5.15; 1280, 200 rows 3.83 / 3.49, 300 rows 4.34 / 4.41; 1024, 300
-//    rows 2.45 / 2.18, 350 rows 2.60 / 2.69.  33 rows, 1280: 2.12 / 1.98; at 32 and fewer the 32-row kernel is as fast.
+//    rows 2.45 / 2.18, 350 rows 2.60 / 2.69; 768, 500 rows 1.14 / 1.08, 600 rows 1.21 / 1.25.  33 rows, 1280: 2.12 / 1.98; at 32 and fewer the 32-row kernel is as fast.
 //  - int8 rows: 1600, 400 rows 9.15 / 8.23, 500 rows 9.98 / 10.53; 1280, 500 rows 5.81 / 5.11, 600 rows 6.64 / 6.83; 768, 850 rows
 //    1.65 / 1.52.  Up to 32 rows, a step of 20 at 1280 1.89 / 1.85, of 32 2.13 / 2.15, of 32 at 768 0.60 / 0.57.
 bool gemm_takes_cut(int M, int K, int N, int w_bf16, int w_int8, int b9_min_rows) {
   if (K % 32 != 0 || N % 32 != 0) return false;
   const double mn = (double)M * N, mnk = mn * K;
   if (w_int8) return M >= 17 && mn <= 2.7e6 && (M > 32 || mnk <= 0.17e9);
-  if (M < 33 || mn > 1.4e6) return false;
-  if (w_bf16) return mnk <= 1.35e9;
-  return mnk <= 1.7e9 && (M >= b9_min_rows || b9_min_rows <= kCutMinRows);
+  if (M < 33) return false;
+  const bool narrow = K <= 768;
+  if (w_bf16) return mn <= (narrow ? 1.6e6 : 1.4e6) && mnk <= 1.35e9;
+  if (!(narrow ? mn <= 3.2e6 : mn <= 1.4e6 && mnk <= 1.7e9)) return false;
+  return M >= b9_min_rows || b9_min_rows <= kCutMinRows;
 }
 
 bool gemm_cut_rows_plan(const GemmArgs& a, int num_cus, CutRowsPlan* plan) {
