@@ -521,12 +521,14 @@ __global__ __launch_bounds__(kTopkStepThreads) void k_topk_step(SampleStep a) {
   unsigned* pen_bits = reinterpret_cast<unsigned*>(smem_raw + sizeof(Smem));
   unsigned long long* const sorted = reinterpret_cast<unsigned long long*>(sm.hist);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (!step_begin<TB>(a)) return;
-  unsigned long long state = 0;
-  const double u = next_unit(a.rng[0], &state);
+  // (the row is asked for before the words that may call the step off: a round trip less in front of it)
   float v[NR];
 #pragma unroll
-  for (int r = 0; r < NR; ++r) v[r] = a.logits[min(r * TB + tid, a.V - 1)];  // (ids >= V: dropped below)
+  for (int r = 0; r < NR; ++r) v[r] = a.logits[min(r * TB + tid, a.V - 1)];  // (ids >= V: the last one once more)
+  const unsigned long long state_in = a.rng[0];
+  if (!step_begin<TB>(a)) return;
+  unsigned long long state = 0;
+  const double u = next_unit(state_in, &state);
   if (a.recent > 0) {
     mark_recent<TB>(pen_bits, a.V, a.hist + (a.n_hist - a.recent), a.recent);
     const RowCandidates row{a.logits, a.V, pen_bits, a.recent, a.penalty};
@@ -537,17 +539,13 @@ __global__ __launch_bounds__(kTopkStepThreads) void k_topk_step(SampleStep a) {
     }
   }
   float lm = -INFINITY;  // this thread's largest candidate
-  unsigned n = 0;
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
     bool cand = is_finite(v[r]);
     if (r * TB + TB > a.V) cand = cand && r * TB + tid < a.V;  // (block-uniform: the last ids)
     v[r] = cand ? v[r] : NAN;  // NaN: not a candidate
     lm = fmaxf(lm, v[r]);      // (the maximum of a number and a NaN is the number)
-    n += cand ? 1u : 0u;
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
   // the m-th largest of the wavefront's lane maxima, equal ones counted each (-inf when fewer
   // than m lanes hold a candidate): bit by bit from the top of the order key, a bit stays set
   // when at least m maxima reach the key built so far with that bit set (32 ballots on the
@@ -568,19 +566,25 @@ __global__ __launch_bounds__(kTopkStepThreads) void k_topk_step(SampleStep a) {
       bound = __uint_as_float(bits);
     }
   }
-  if (lane == 0) {
-    sm.wave_f[0][wave] = bound;
-    sm.wave_u[wave] = n;
-  }
+  if (lane == 0) sm.wave_f[0][wave] = bound;
   if (tid == 0) sm.n_items = 0u;
   __syncthreads();
   float L = sm.wave_f[0][0];
-  unsigned total = sm.wave_u[0];
-  for (int w = 1; w < NW; ++w) {
-    L = fminf(L, sm.wave_f[0][w]);
-    total += sm.wave_u[w];
+  for (int w = 1; w < NW; ++w) L = fminf(L, sm.wave_f[0][w]);
+  // a bound that is a number has 8 m >= k candidates at or above it; their number is needed only without one
+  unsigned kk = (unsigned)a.top_k;
+  if (L == -INFINITY) {  // (block-uniform)
+    unsigned n = 0;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) n += v[r] == v[r] ? 1u : 0u;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+    if (lane == 0) sm.wave_u[wave] = n;
+    __syncthreads();
+    n = sm.wave_u[0];
+    for (int w = 1; w < NW; ++w) n += sm.wave_u[w];
+    kk = min(n, kk);
   }
-  const unsigned kk = min(total, (unsigned)a.top_k);
   int st = 0;
   unsigned token = 0;
   if (kk == 0) {
@@ -615,11 +619,23 @@ __global__ __launch_bounds__(kTopkStepThreads) void k_topk_step(SampleStep a) {
         return __uint_as_float(bits);
       };
       const double max_logit = (double)value_at(0) / a.temperature;  // generation.rs:318
-      for (unsigned i = tid; i < (unsigned)kBinCap; i += TB)
-        sm.weight[i] = i < kk ? exp((double)value_at(i) / a.temperature - max_logit) : 0.0;
+      // running weights of at most kTopkStepMaxK candidates: two wavefronts, one candidate a lane
+      static_assert(kTopkStepMaxK <= 128, "two wavefronts");
+      if (tid < 128) {
+        double w = (unsigned)tid < kk ? exp((double)value_at(tid) / a.temperature - max_logit) : 0.0;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const double up = shfl_up_d(w, off);
+          if (lane >= off) w += up;
+        }
+        sm.weight[tid] = w;
+      }
       __syncthreads();
-      block_scan_2048<TB>(sm.weight, sm.wave_d);
-      const double full = sm.weight[kBinCap - 1];
+      const double first_half = sm.weight[63];
+      __syncthreads();
+      if (tid >= 64 && tid < 128) sm.weight[tid] += first_half;
+      __syncthreads();
+      const double full = sm.weight[127];
       if (!(full > 0.0) || !isfinite(full)) {
         st = 2;  // (generation.rs:344-346 takes the first candidate: left to the host)
       } else {
