@@ -9,6 +9,7 @@
 #include "pg_cut.h"
 #include "pg_kernels.h"
 #include "pg_math.h"
+#include "pg_wave.h"
 
 #include <algorithm>
 
@@ -21,16 +22,6 @@ namespace {
 constexpr int kBlock = 256;  // 4 wavefronts of 64 lanes
 constexpr int kWaves = kBlock / 64;
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-  return v;
-}
 // Sum over the block; every thread receives the result.  red holds kWaves floats.
 __device__ __forceinline__ float block_sum(float v, float* red) {
   v = wave_sum(v);
@@ -677,15 +668,11 @@ __global__ __launch_bounds__(kBlock) void k_attn_decode64(const float* __restric
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
       float t = qv.x * kr[i].x + qv.y * kr[i].y + qv.z * kr[i].z + qv.w * kr[i].w;
-      t += __shfl_xor(t, 1, 64);
-      t += __shfl_xor(t, 2, 64);
-      t += __shfl_xor(t, 4, 64);
-      t += __shfl_xor(t, 8, 64);
+      t = lanes16(t, AddLanes{});
       sc[i] = kfirst + kGroups * i < k1 ? t * scale : -INFINITY;
       cm = fmaxf(cm, sc[i]);
     }
-    cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
-    cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
+    cm = with_lane32(with_lane16(cm, MaxLanes{}), MaxLanes{});
     const float m_new = fmaxf(m_run, cm);
     if (m_new == -INFINITY) continue;  // (wavefront-uniform) no key of this wavefront so far
     const float corr = expf(m_run - m_new);
@@ -704,18 +691,11 @@ __global__ __launch_bounds__(kBlock) void k_attn_decode64(const float* __restric
       acc.z += pk * vr[i].z;
       acc.w += pk * vr[i].w;
     }
-    ls += __shfl_xor(ls, 16, 64);  // (the sixteen lanes of a key hold the same value)
-    ls += __shfl_xor(ls, 32, 64);
-    l_run += ls;
+    l_run += with_lane32(with_lane16(ls, AddLanes{}), AddLanes{});  // (the sixteen lanes of a key hold the same value)
     m_run = m_new;
   }
-#pragma unroll
-  for (int off = 16; off <= 32; off <<= 1) {
-    acc.x += __shfl_xor(acc.x, off, 64);
-    acc.y += __shfl_xor(acc.y, off, 64);
-    acc.z += __shfl_xor(acc.z, off, 64);
-    acc.w += __shfl_xor(acc.w, off, 64);
-  }
+  auto all_keys = [](float v) { return with_lane32(with_lane16(v, AddLanes{}), AddLanes{}); };
+  acc = make_float4(all_keys(acc.x), all_keys(acc.y), all_keys(acc.z), all_keys(acc.w));
   if (sub == 0) reinterpret_cast<float4*>(accs[wave])[d4] = acc;
   if (lane == 0) {
     wm[wave] = m_run;

@@ -8,6 +8,7 @@
 //
 // Shapes are checked on the host before any launch (pg_stack.cpp); kernels guard ragged tails.
 #include "pg_mixers.h"
+#include "pg_wave.h"
 
 #include <math.h>
 
@@ -23,11 +24,6 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 constexpr float kLog2e = 1.44269504088896341f;
 constexpr float kNone = -1e30f;  // a running maximum before the first key
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
 __device__ __forceinline__ float block_sum(float v, float* red) {  // 256 threads
   v = wave_sum(v);
   __syncthreads();
@@ -244,13 +240,11 @@ __global__ __launch_bounds__(256, NT <= 8 && ROT <= 64 ? 2 : 1) void k_latent_at
       const float2 p1 = *reinterpret_cast<const float2*>(&ps[1][h][key]);
       const float z0 = k0 + key < j1 ? p0.x + p1.x : -INFINITY, z1 = k0 + key + 1 < j1 ? p0.y + p1.y : -INFINITY;
       float mx = fmaxf(z0, z1);
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+      mx = lanes16(mx, MaxLanes{});
       const float old = ms[h], now = fmaxf(old, mx);
       const float w0 = __builtin_amdgcn_exp2f(z0 - now), w1 = __builtin_amdgcn_exp2f(z1 - now);
       float sum = w0 + w1;
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+      sum = lanes16(sum, AddLanes{});
       *reinterpret_cast<float2*>(&ps[0][h][key]) = float2{w0, w1};
       if (l16 == 0) {
         const float f = __builtin_amdgcn_exp2f(old - now);
@@ -328,9 +322,7 @@ __global__ __launch_bounds__(256) void k_latent_out(LatentDecode m, LatentAttn a
       w[r][c] = load_w4<BF16>(a.up_w, row * a.kv_pad + min(4 * lane + 256 * c, a.kv_pad - 4));
     }
   if (wave == 0) {
-    float top = fmaxf(mx, sink);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) top = fmaxf(top, __shfl_xor(top, off, 64));
+    const float top = wave_max(fmaxf(mx, sink));
     const float f = l > 0.0f ? exp2f(mx - top) : 0.0f;
     const float sum = wave_sum(l * f) + exp2f(sink - top);
     ws[lane] = f / sum;

@@ -5,6 +5,7 @@
 // Shapes are checked on the host before any launch (pg_stack.cpp); kernels guard ragged tails.
 #include "pg_mixers.h"
 #include "pg_math.h"
+#include "pg_wave.h"
 
 #include <math.h>
 
@@ -28,11 +29,6 @@ __device__ __forceinline__ f4 bf16x4(const unsigned short* p) {
             __uint_as_float(u.y & 0xffff0000u)};
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
 // Sum over a block of 256 threads; every thread receives the result.  red holds 4 floats.
 __device__ __forceinline__ float block_sum(float v, float* red) {
   v = wave_sum(v);
@@ -317,8 +313,7 @@ struct LowRankRows {
     const int i0 = threadIdx.x >> 3, sub = threadIdx.x & 7;
     auto dot = [](const f4& a, const f4& b) { return (a.x * b.x + a.y * b.y) + (a.z * b.z + a.w * b.w); };
     auto finish = [&](int i, float s) __attribute__((always_inline)) {
-#pragma unroll
-      for (int off = 4; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+      s = lanes8(s, AddLanes{});
       if (sub == 0 && i < n) dst[i] = s;
     };
     auto rest = [&](int i, int k0, float s) __attribute__((always_inline)) {
@@ -930,11 +925,8 @@ __global__ __launch_bounds__(256) void k_delta_chunk(MixRows r, Recurrence c, Ch
       qq += q * q;
       kk += k * k;
     }
-#pragma unroll
-    for (int off = 4; off > 0; off >>= 1) {
-      qq += __shfl_xor(qq, off, 64);
-      kk += __shfl_xor(kk, off, 64);
-    }
+    qq = lanes8(qq, AddLanes{});
+    kk = lanes8(kk, AddLanes{});
     const float qm = c.q_scale / sqrtf(qq + 1e-6f), km = 1.0f / sqrtf(kk + 1e-6f);
     for (int i = sub; i < dp; i += 8) {
       Qs[t * LD + i] *= qm;
@@ -1184,11 +1176,8 @@ __global__ __launch_bounds__(256) void k_channel_delta_chunk(MixRows r, Recurren
       qq += q * q;
       kk += k * k;
     }
-#pragma unroll
-    for (int off = 4; off > 0; off >>= 1) {
-      qq += __shfl_xor(qq, off, 64);
-      kk += __shfl_xor(kk, off, 64);
-    }
+    qq = lanes8(qq, AddLanes{});
+    kk = lanes8(kk, AddLanes{});
     const float qm = c.q_scale / sqrtf(qq + 1e-6f), km = 1.0f / sqrtf(kk + 1e-6f);
     for (int i = sub; i < dp; i += 8) {
       Qs[t * LD + i] *= qm;
@@ -1243,8 +1232,7 @@ __global__ __launch_bounds__(256) void k_channel_delta_chunk(MixRows r, Recurren
     const int t = tid >> 3, sub = tid & 7;
     float s = 0.0f;
     for (int d = sub; d < dim; d += 8) s += Qs[t * LD + d] * Ks[t * LD + d];
-#pragma unroll
-    for (int off = 4; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    s = lanes8(s, AddLanes{});
     if (sub == 0) {
       w.P[tile * 1024 + t * 33] = s;
       As[t][t] = 0.0f;
@@ -1472,8 +1460,7 @@ __global__ __launch_bounds__(256) void k_chunk_out(MixRows r, Recurrence c, Chun
 #pragma unroll
   for (int v = 0; v < 16; ++v) {
     float x = o[0][v] * o[0][v] + o[1][v] * o[1][v];
-#pragma unroll
-    for (int off = 16; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+    x = with_lane16(lanes16(x, AddLanes{}), AddLanes{});
     if (l32 == 0) ss[wave][8 * (v >> 2) + 4 * half + (v & 3)] = x;
   }
   __syncthreads();

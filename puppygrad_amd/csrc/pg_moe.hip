@@ -3,6 +3,7 @@
 //
 // Shapes are checked on the host before any launch (pg_stack.cpp).
 #include "pg_mixers.h"
+#include "pg_wave.h"
 
 #include <math.h>
 
@@ -17,16 +18,6 @@ typedef unsigned u4v __attribute__((ext_vector_type(4)));
 
 constexpr int kPerLane = kMoeMaxExperts / 64;  // logits a lane holds
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-  return v;
-}
 
 // One wavefront: the `top` largest of the logits z(e), e < experts, in descending order (equal ones: the lower
 // index first), each with its softmax over all experts; each(k, expert, weight) in every lane.

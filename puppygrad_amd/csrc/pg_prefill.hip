@@ -8,6 +8,7 @@
 // itself checks against forward() at 1e-5 (rust.rs:1900-1913).
 #include "pg_gemm_dev.h"
 #include "pg_mixers.h"
+#include "pg_wave.h"
 
 #include <type_traits>
 
@@ -373,8 +374,7 @@ __global__ __launch_bounds__(256) void k_splitk_reduce_ln(GemmArgs a, int parts)
   const int n4 = a.N / 4;
   const size_t stride = (size_t)a.M * a.N;
   auto bsum = [&](float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    v = wave_sum(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
@@ -500,8 +500,7 @@ __global__ __launch_bounds__(256) void k_splitk_reduce_post(GemmArgs a, int part
     }
     ss += (c[q].x * c[q].x + c[q].y * c[q].y) + (c[q].z * c[q].z + c[q].w * c[q].w);
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+  ss = wave_sum(ss);
   if ((tid & 63) == 0) red[tid >> 6] = ss;
   __syncthreads();
   const float k = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)a.post_n + a.ln_eps);
@@ -1257,8 +1256,7 @@ __global__ __launch_bounds__(256) void k_layer_norm_rows(const float* src, float
     else dst[dst_form == FORM_PACKED32 ? packed32_index(blockIdx.x, (size_t)i) : (size_t)blockIdx.x * cols + i] = v;
   };
   auto bsum = [&](float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    v = wave_sum(v);
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();

@@ -1,0 +1,54 @@
+// Sums and maxima over the lanes of a wavefront without a trip through LDS: __shfl_xor is one (about 100 clocks before
+// the next step can start, 0.25 us for the six of a wavefront, which a launch of 4 to 8 us waits for once to three
+// times); moves within a row of 16 lanes ride on the addition itself, and rows are brought together by a swap.  All lanes
+// have to be active, and all get the result.
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace pgk {
+namespace {
+
+// The value of a lane of the same row: 0xB1 lane ^ 1, 0x4E lane ^ 2, 0x141 lane ^ 7 and 0x140 lane ^ 15 (mirrors, which
+// serve as lane ^ 4 and lane ^ 8 where the lanes in between hold the same).
+template <int CTRL>
+__device__ __forceinline__ float row_lane(float x) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+struct AddLanes {
+  __device__ __forceinline__ float operator()(float a, float b) const { return a + b; }
+};
+struct MaxLanes {
+  __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); }
+};
+// over each 8 (16) neighbouring lanes
+template <typename Op>
+__device__ __forceinline__ float lanes8(float v, Op op) {
+  v = op(v, row_lane<0xB1>(v));
+  v = op(v, row_lane<0x4E>(v));
+  return op(v, row_lane<0x141>(v));
+}
+template <typename Op>
+__device__ __forceinline__ float lanes16(float v, Op op) {
+  v = lanes8(v, op);
+  return op(v, row_lane<0x140>(v));
+}
+// with the lane 16 (32) away
+template <typename Op>
+__device__ __forceinline__ float with_lane16(float v, Op op) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+template <typename Op>
+__device__ __forceinline__ float with_lane32(float v, Op op) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float wave_sum(float v) {
+  return with_lane32(with_lane16(lanes16(v, AddLanes{}), AddLanes{}), AddLanes{});
+}
+__device__ __forceinline__ float wave_max(float v) {
+  return with_lane32(with_lane16(lanes16(v, MaxLanes{}), MaxLanes{}), MaxLanes{});
+}
+
+}  // namespace
+}  // namespace pgk
