@@ -823,11 +823,7 @@ __global__ __launch_bounds__(1024) void k_argmax(const float* v, int n, uint32_t
         b.i = (uint32_t)min(i0 + 1024 * u, n - 1);
       }
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    Best o{__shfl_xor(b.v, off, 64), (uint32_t)__shfl_xor((int)b.i, off, 64)};
-    b = better(b, o);
-  }
+  wave_best(b.v, b.i, [](float v, unsigned i, float ov, unsigned oi) { return ov > v || (ov == v && oi < i); });
   int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) {
     sv[wave] = b.v;

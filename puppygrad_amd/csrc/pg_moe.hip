@@ -40,27 +40,21 @@ __device__ __forceinline__ void choose_experts(Z z, int experts, int top, F each
   unsigned taken = 0;  // bit p: logit p of this lane
   for (int k = 0; k < top; ++k) {
     float best = -INFINITY;
-    int at = kMoeMaxExperts;
+    unsigned at = kMoeMaxExperts;
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
       const int e = lane + 64 * p;
       if (e < experts && !(taken >> p & 1) && (at == kMoeMaxExperts || v[p] > best)) {
         best = v[p];
-        at = e;
+        at = (unsigned)e;
       }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ob = __shfl_xor(best, off, 64);
-      const int oa = __shfl_xor(at, off, 64);
-      if (oa != kMoeMaxExperts && (at == kMoeMaxExperts || ob > best || (ob == best && oa < at))) {
-        best = ob;
-        at = oa;
-      }
-    }
-    at = min(at, experts - 1);  // (logits that are not numbers)
-    if ((at & 63) == lane) taken |= 1u << (at >> 6);
-    each(k, at, expf(best - mx) / sum);
+    wave_best(best, at, [](float v, unsigned i, float ov, unsigned oi) {
+      return oi != kMoeMaxExperts && (i == kMoeMaxExperts || ov > v || (ov == v && oi < i));
+    });
+    const int chosen = min((int)at, experts - 1);  // (logits that are not numbers)
+    if ((chosen & 63) == lane) taken |= 1u << (chosen >> 6);
+    each(k, chosen, expf(best - mx) / sum);
   }
 }
 template <typename Z, typename F>

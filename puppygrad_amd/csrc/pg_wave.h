@@ -5,6 +5,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace pgk {
 namespace {
 
@@ -48,6 +50,36 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 __device__ __forceinline__ float wave_max(float v) {
   return with_lane32(with_lane16(lanes16(v, MaxLanes{}), MaxLanes{}), MaxLanes{});
+}
+// The better of all lanes' (value, index) pairs; take(v, i, ov, oi): whether (ov, oi) is better than (v, i).
+template <typename Take>
+__device__ __forceinline__ void wave_best(float& v, unsigned& i, Take take) {
+  auto with = [&](float ov, unsigned oi) {
+    if (take(v, i, ov, oi)) v = ov, i = oi;
+  };
+  auto in_row = [](unsigned x, auto ctrl) {
+    return (unsigned)__builtin_amdgcn_mov_dpp((int)x, decltype(ctrl)::value, 0xf, 0xf, true);
+  };
+  auto step = [&](auto ctrl) {
+    const float ov = __uint_as_float(in_row(__float_as_uint(v), ctrl));
+    with(ov, in_row(i, ctrl));
+  };
+  step(std::integral_constant<int, 0xB1>{});
+  step(std::integral_constant<int, 0x4E>{});
+  step(std::integral_constant<int, 0x141>{});
+  step(std::integral_constant<int, 0x140>{});
+  {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(i, i, false, false);
+    v = __uint_as_float(a[0]), i = b[0];
+    with(__uint_as_float(a[1]), b[1]);
+  }
+  {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(i, i, false, false);
+    v = __uint_as_float(a[0]), i = b[0];
+    with(__uint_as_float(a[1]), b[1]);
+  }
 }
 
 }  // namespace
