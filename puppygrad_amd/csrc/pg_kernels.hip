@@ -200,6 +200,7 @@ __global__ __launch_bounds__(kBlock) void k_gemv(GemvArgs a) {
       }
   };
   if (kVec) request(pre, row0);
+  const float rms_gain = PRO == PRO_RMS ? a.ln_g[0] : 0.0f;  // (asked for where it is used, it was waited for there)
 
   if constexpr (PRO == PRO_STACK) {
     if (in_regs) {
@@ -251,9 +252,17 @@ __global__ __launch_bounds__(kBlock) void k_gemv(GemvArgs a) {
 #pragma unroll
               for (int g = 0; g < 4; ++g) ss[g] += at >= g * n && at < (g + 1) * n ? v * v : 0.0f;
             }
+          // (all groups' sums behind one meeting of the wavefronts)
+          __shared__ float red4[4][kWaves];
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const float s = wave_sum(ss[g]);
+            if (lane == 0) red4[g][wave] = s;
+          }
+          __syncthreads();
 #pragma unroll
           for (int g = 0; g < 4; ++g)
-            if (g < a.groups) inv[g] = 1.0f / sqrtf(block_sum(ss[g], red) / (float)n + a.eps);
+            inv[g] = 1.0f / sqrtf(((red4[g][0] + red4[g][1]) + (red4[g][2] + red4[g][3])) / (float)n + a.eps);
 #pragma unroll
           for (int p = 0; p < kIn; ++p)
 #pragma unroll
@@ -329,7 +338,7 @@ __global__ __launch_bounds__(kBlock) void k_gemv(GemvArgs a) {
     float ss = ss_x;
     if (!in_regs)
       for (int i = tid; i < K; i += kBlock) ss += sx[i] * sx[i];
-    row_mul = a.ln_g[0] / sqrtf(block_sum(ss, red) / (float)a.norm_n + a.eps);
+    row_mul = rms_gain / sqrtf(block_sum(ss, red) / (float)a.norm_n + a.eps);
     if (a.out_mul != 0.0f) row_mul *= a.out_mul;
   }
 
@@ -490,6 +499,15 @@ __global__ __launch_bounds__(kPairMaxThreads) void k_gemv_pair(GemvPair a) {
       pre[r][i] = gv_u4{0u, 0u, 0u, 0u};
       if (row0 + r < a.nout && j < KV) pre[r][i] = chunk(row0 + r, j);
     }
+  // what the sums meet at the end (asked for there it was a round trip to memory of its own)
+  float er[RPW], e1[RPW], e2[RPW];
+#pragma unroll
+  for (int r = 0; r < RPW; ++r) {
+    const int o = min(row0 + r, a.nout - 1);
+    er[r] = a.resid[o];
+    e1[r] = a.s1[o];
+    e2[r] = a.W2 ? a.s2[o] : 0.0f;
+  }
   {
     float4* d = reinterpret_cast<float4*>(sx);
     auto sum = [&](const float (&v)[kPairMaxSplits]) {
@@ -557,8 +575,8 @@ __global__ __launch_bounds__(kPairMaxThreads) void k_gemv_pair(GemvPair a) {
     for (int r = 0; r < RPW; ++r) {
       const int o = row0 + r;
       if (o >= a.nout) break;
-      float v = a.resid[o] + a.s1[o] * acc1[r];
-      if (a.W2) v += a.s2[o] * acc2[r];
+      float v = er[r] + e1[r] * acc1[r];
+      if (a.W2) v += e2[r] * acc2[r];
       a.y[o] = v;
     }
   }
