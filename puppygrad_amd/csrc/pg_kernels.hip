@@ -819,7 +819,7 @@ __device__ __forceinline__ Best better(Best a, Best b) {
   return a;
 }
 // U: loads in flight per thread.  One block pulls a row in at the pace of its round trips to memory: 50257 logits, 8 at a
-// time 7.1 us, all 50 at once 4.6 us (a launch by itself is 2).  out may be pinned host memory.
+// time 7.1 us, all 50 at once 4.9 us (a launch by itself is 2).  out may be pinned host memory.
 template <int U>
 __global__ __launch_bounds__(1024) void k_argmax(const float* v, int n, uint32_t* out) {
   v += (size_t)blockIdx.x * n;  // one block per row
