@@ -262,7 +262,7 @@ __global__ __launch_bounds__(kBlock) void k_gemv(GemvArgs a) {
           __syncthreads();
 #pragma unroll
           for (int g = 0; g < 4; ++g)
-            inv[g] = 1.0f / sqrtf(((red4[g][0] + red4[g][1]) + (red4[g][2] + red4[g][3])) / (float)n + a.eps);
+            inv[g] = 1.0f / sqrtf((((red4[g][0] + red4[g][1]) + red4[g][2]) + red4[g][3]) / (float)n + a.eps);
 #pragma unroll
           for (int p = 0; p < kIn; ++p)
 #pragma unroll
@@ -686,7 +686,7 @@ __global__ __launch_bounds__(kBlock) void k_attn_decode64(const float* __restric
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
       float t = qv.x * kr[i].x + qv.y * kr[i].y + qv.z * kr[i].z + qv.w * kr[i].w;
-      t = lanes16(t, AddLanes{});
+      t = lanes16_up(t, AddLanes{});
       sc[i] = kfirst + kGroups * i < k1 ? t * scale : -INFINITY;
       cm = fmaxf(cm, sc[i]);
     }

@@ -324,7 +324,7 @@ __global__ __launch_bounds__(256) void k_latent_out(LatentDecode m, LatentAttn a
   if (wave == 0) {
     const float top = wave_max(fmaxf(mx, sink));
     const float f = l > 0.0f ? exp2f(mx - top) : 0.0f;
-    const float sum = wave_sum(l * f) + exp2f(sink - top);
+    const float sum = wave_sum_of_products(l, f) + exp2f(sink - top);
     ws[lane] = f / sum;
   }
   __syncthreads();

@@ -404,7 +404,7 @@ __device__ void recurrence_role(const MixDecode& m, int b, int h, float* lds) {
         ks[tid] = kv;
       }
     } else {
-    float qn = wave_sum(qv * qv), kn = wave_sum(kv * kv);
+    float qn = wave_sum_of_products(qv, qv), kn = wave_sum_of_products(kv, kv);
     if ((tid & 63) == 0 && tid < 256) {  // (nothing past kMixMaxDim = 256)
       redw[tid >> 6] = qn;
       redw[4 + (tid >> 6)] = kn;
@@ -502,7 +502,7 @@ __device__ void recurrence_role(const MixDecode& m, int b, int h, float* lds) {
     if (tid < vdim) m.out[(size_t)b * m.ld_out + c.out_col + h * vdim + tid] = (out + skip) * silu(gate);
     return;
   }
-  float ss = wave_sum(out * out);
+  float ss = wave_sum_of_products(out, out);
   if ((tid & 63) == 0 && tid < 256) redw[tid >> 6] = ss;
   __syncthreads();
   ss = (redw[0] + redw[1]) + (redw[2] + redw[3]);
@@ -1460,7 +1460,7 @@ __global__ __launch_bounds__(256) void k_chunk_out(MixRows r, Recurrence c, Chun
 #pragma unroll
   for (int v = 0; v < 16; ++v) {
     float x = o[0][v] * o[0][v] + o[1][v] * o[1][v];
-    x = with_lane16(lanes16(x, AddLanes{}), AddLanes{});
+    x = lanes16(with_lane16(x, AddLanes{}), AddLanes{});
     if (l32 == 0) ss[wave][8 * (v >> 2) + 4 * half + (v & 3)] = x;
   }
   __syncthreads();

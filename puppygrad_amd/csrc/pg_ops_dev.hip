@@ -15,6 +15,7 @@
 #include "pg_gemm_dev.h"
 #include "pg_internal.h"
 #include "pg_kernels.h"
+#include "pg_wave.h"
 
 namespace {
 
@@ -171,6 +172,17 @@ __global__ __launch_bounds__(kBlk) void k_attention_rows(const float* __restrict
     for (int gg = 0; gg < groups; ++gg) t += part[gg * hd + tid];
     out[(size_t)query * state + (size_t)head * hd + tid] = t;
   }
+}
+
+// (for the tests: the sums of pg_wave.h, a wavefront a block)
+__global__ __launch_bounds__(64) void k_lane_sums(const float* x, const float* y, float* out) {
+  const size_t i = (size_t)blockIdx.x * 64 + threadIdx.x, n = (size_t)gridDim.x * 64;
+  const float a = x[i], b = y[i];
+  out[i] = pgk::wave_sum(a);
+  out[n + i] = pgk::wave_sum_of_products(a, b);
+  out[2 * n + i] = pgk::lanes8(a, pgk::AddLanes{});
+  out[3 * n + i] = pgk::lanes16(a, pgk::AddLanes{});
+  out[4 * n + i] = pgk::lanes16_up(a, pgk::AddLanes{});
 }
 
 }  // namespace
@@ -369,6 +381,18 @@ pg_status pg_testing_product_dev(int32_t device, void* stream, const float* x, u
   int cus = 0;
   PG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   PG_HIP(pgk::launch_gemm(a, pgk::GEMM_BIAS, cus, static_cast<hipStream_t>(stream)));
+  return PG_OK;
+}
+
+// The sums of pg_wave.h over `rows` wavefronts: x, y [rows][64], out [5][rows][64]: wave_sum of x, wave_sum_of_products of x
+// and y, lanes8, lanes16 and lanes16_up of x.
+pg_status pg_testing_lane_sums_dev(int32_t device, void* stream, const float* x, const float* y, uint64_t rows, float* out) {
+  if (!x || !y || !out) return pgh::fail(PG_INVALID_INPUT, "null argument");
+  if (rows == 0 || rows > 4096) return pgh::fail(PG_INVALID_INPUT, "lane sums: sizes");
+  pg_status s;
+  if ((s = select_device(device))) return s;
+  hipLaunchKernelGGL(k_lane_sums, dim3((unsigned)rows), dim3(64), 0, static_cast<hipStream_t>(stream), x, y, out);
+  PG_HIP(hipGetLastError());
   return PG_OK;
 }
 

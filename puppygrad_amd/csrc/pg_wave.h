@@ -2,6 +2,9 @@
 // the next step can start, 0.25 us for the six of a wavefront, which a launch of 4 to 8 us waits for once to three
 // times); moves within a row of 16 lanes ride on the addition itself, and rows are brought together by a swap.  All lanes
 // have to be active, and all get the result.
+// The order of the additions is that of __shfl_xor by 32, 16, 8, 4, 2 and 1, to the last bit: a stream that is drawn
+// over a whole row walks 50257 ids by value, and a logit that moves by its last bit makes it take another id, and other
+// ids from there on, about once in five streams of 80.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -10,8 +13,8 @@
 namespace pgk {
 namespace {
 
-// The value of a lane of the same row: 0xB1 lane ^ 1, 0x4E lane ^ 2, 0x141 lane ^ 7 and 0x140 lane ^ 15 (mirrors, which
-// serve as lane ^ 4 and lane ^ 8 where the lanes in between hold the same).
+// The value of a lane of the same row of 16: 0xB1 lane ^ 1, 0x4E lane ^ 2, 0x1B lane ^ 3, 0x141 lane ^ 7, 0x140 lane ^ 15,
+// 0x128 lane ^ 8, and 0x124 lane - 4, which serves as lane ^ 4 where lanes 8 apart hold the same.
 template <int CTRL>
 __device__ __forceinline__ float row_lane(float x) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xf, 0xf, true));
@@ -22,16 +25,27 @@ struct AddLanes {
 struct MaxLanes {
   __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); }
 };
-// over each 8 (16) neighbouring lanes
+// over each 8 neighbouring lanes: lane ^ 4, ^ 2, ^ 1
 template <typename Op>
 __device__ __forceinline__ float lanes8(float v, Op op) {
-  v = op(v, row_lane<0xB1>(v));
+  v = op(v, row_lane<0x1B>(row_lane<0x141>(v)));
   v = op(v, row_lane<0x4E>(v));
-  return op(v, row_lane<0x141>(v));
+  return op(v, row_lane<0xB1>(v));
 }
+// over each 16: lane ^ 8, ^ 4, ^ 2, ^ 1
 template <typename Op>
 __device__ __forceinline__ float lanes16(float v, Op op) {
-  v = lanes8(v, op);
+  v = op(v, row_lane<0x128>(v));
+  v = op(v, row_lane<0x124>(v));
+  v = op(v, row_lane<0x4E>(v));
+  return op(v, row_lane<0xB1>(v));
+}
+// over each 16 the other way round: lane ^ 1, ^ 2, ^ 4, ^ 8 (mirrors: the lanes in between hold the same)
+template <typename Op>
+__device__ __forceinline__ float lanes16_up(float v, Op op) {
+  v = op(v, row_lane<0xB1>(v));
+  v = op(v, row_lane<0x4E>(v));
+  v = op(v, row_lane<0x141>(v));
   return op(v, row_lane<0x140>(v));
 }
 // with the lane 16 (32) away
@@ -46,10 +60,17 @@ __device__ __forceinline__ float with_lane32(float v, Op op) {
   return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 __device__ __forceinline__ float wave_sum(float v) {
-  return with_lane32(with_lane16(lanes16(v, AddLanes{}), AddLanes{}), AddLanes{});
+  return lanes16(with_lane16(with_lane32(v, AddLanes{}), AddLanes{}), AddLanes{});
+}
+// of a * b: the first addition takes this lane's product unrounded (what a product met by __shfl_xor is compiled to)
+__device__ __forceinline__ float wave_sum_of_products(float a, float b) {
+  const unsigned p = __float_as_uint(a * b);
+  const auto r = __builtin_amdgcn_permlane32_swap(p, p, false, false);
+  const float other = __uint_as_float((threadIdx.x & 32) ? r[0] : r[1]);
+  return lanes16(with_lane16(fmaf(a, b, other), AddLanes{}), AddLanes{});
 }
 __device__ __forceinline__ float wave_max(float v) {
-  return with_lane32(with_lane16(lanes16(v, MaxLanes{}), MaxLanes{}), MaxLanes{});
+  return lanes16(with_lane16(with_lane32(v, MaxLanes{}), MaxLanes{}), MaxLanes{});
 }
 // The better of all lanes' (value, index) pairs; take(v, i, ov, oi): whether (ov, oi) is better than (v, i).
 template <typename Take>
