@@ -513,7 +513,7 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
   // split-K partial tiles of the projections back to n_embd columns (up to 8 parts)
   const size_t ws_floats = 8 * n * g.C;
   // the projections' inputs (XN, ATT, HB) in cut form
-  const bool cut = hd == pgk::kHeadDim && pgk::gemm_takes_cut(T, C, I, m->w_bf16, m->w_i8, m->gemm_b9_min_rows);
+  const bool cut = !c->drawn && hd == pgk::kHeadDim && pgk::gemm_takes_cut(T, C, I, m->w_bf16, m->w_i8, m->gemm_b9_min_rows);
   {
     auto form = [&](size_t cols) { return cut ? std::max(n * cols, pgk::cut_floats(n, cols)) : n * cols; };
     auto up = [](size_t v) { return (v + 63) / 64 * 64; };  // 256-byte boundaries
@@ -586,7 +586,7 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
     PG_MARK(kQkv);
     PG_HIP(pgk::launch_attn_prefill(QKV.p, Ts, C, H, hd, P, c->k_panel(l, b), c->v_panel(l, b),
                                     ATT.p, SCR.p, s, (int)nb, g.H * g.P * g.hd(),
-                                    cut ? pgk::FORM_CUT : pgk::FORM_ROWS));
+                                    cut ? pgk::FORM_CUT : pgk::FORM_ROWS, c->drawn));
     PG_MARK(kAttention);
     PG_HIP(gemm(ATT.p, C, w.c_proj_w, w.c_proj_b, X.p, C, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b, cut));
     PG_MARK(kAttnProj);
@@ -2024,6 +2024,7 @@ static pg_status stream_core(const pg_model* m, const uint32_t* ids, size_t n,
   pg_kv_cache* c = nullptr;
   if ((s = pg_kv_cache_create(m, 1, &c))) return s;
   std::unique_ptr<pg_kv_cache, void (*)(pg_kv_cache*)> holder(c, pg_kv_cache_destroy);
+  c->drawn = sampling->temperature > 0.0f;
   auto first_start = Clock::now();
   auto prefill_start = Clock::now();
   pg_logits* logits = nullptr;

@@ -152,6 +152,11 @@ struct pg_kv_cache {
   float *x = nullptr, *q = nullptr, *hbuf = nullptr, *part_acc = nullptr, *part_m = nullptr,
         *part_l = nullptr, *logits_buf = nullptr;
   float *qkv_b = nullptr, *xn_b = nullptr, *att_b = nullptr;  // batched step: [B][3C], [B][C], [B][C]
+  // A stream's ids are drawn from what this cache holds: a prompt's products, attention and experts stay with the kernels
+  // whose sums a seed's ids were drawn from so far.  Over a whole row the draw walks 50257 ids by value, neighbours 10^-5
+  // apart, and logits moved by their last bits (another kernel's order of additions: 5 10^-7) change two streams of 80 in
+  // five from some id on.  Decode steps have one kernel either way.
+  bool drawn = false;
   bool cut_form = false;  // batched step: xn_b, att_b and hbuf are in cut form (pgk::FORM_CUT)
   bool pack32 = false;  // batched step: xn_b, att_b and hbuf are packed (pgk::packed32_index)
   // device-side candidate selection for sampling, allocated at first use: kept candidates

@@ -829,10 +829,10 @@ namespace {
     if (marks) PG_HIP(marks->mark(s, ProfileMarks::b)); \
   } while (0)
 
-// Slots to a tile of the sorted pairs: few rows stream the experts' weights, many fill tiles.
-int moe_tile_rows(const pgk::Moe& m, int rows) {
+// Slots to a tile of the sorted pairs: few rows stream the experts' weights, many fill tiles.  drawn: pg_kv_cache's.
+int moe_tile_rows(const pgk::Moe& m, int rows, bool drawn) {
   const long pairs = (long)rows * m.top;
-  if (pairs <= 12L * m.experts) return 16;
+  if (pairs <= 12L * m.experts && !drawn) return 16;
   if (pairs <= 32L * m.experts) return 32;
   return m.w_bf16 && pairs >= 512L * m.experts ? 128 : 64;
 }
@@ -840,12 +840,12 @@ int moe_tile_rows(const pgk::Moe& m, int rows) {
 // Working memory of a mixture of experts over `rows` rows, large enough for each layer added.
 struct MoeSizes {
   size_t logits = 0, act = 0, slot_out = 0, experts = 0, pairs = 0, slots = 0, tiles = 0;
-  void add(const pgk::Moe& m, int rows, int width_pad) {
+  void add(const pgk::Moe& m, int rows, int width_pad, bool drawn) {
     logits = std::max(logits, (size_t)rows * m.experts_pad);
     pairs = std::max(pairs, (size_t)rows * m.top);
     act = std::max(act, (size_t)rows * m.top * m.ff_pad);
     if (rows == 1) return;
-    const int tile = moe_tile_rows(m, rows);
+    const int tile = moe_tile_rows(m, rows, drawn);
     const size_t n = (size_t)pgk::moe_max_slots(m, rows, tile);
     experts = std::max(experts, (size_t)m.experts);
     slots = std::max(slots, n);
@@ -898,7 +898,7 @@ pg_status stack_cache_create(const pg_model* model, pg_kv_cache* c) {
     return s;
   MoeSizes ms;
   for (const StackLayer& l : m.layers)
-    if (l.ffn.kind == PostFeedForward::kMoe) ms.add(l.ffn.moe, (int)B, m.width_pad);
+    if (l.ffn.kind == PostFeedForward::kMoe) ms.add(l.ffn.moe, (int)B, m.width_pad, c->drawn);
   if (ms.logits) {
     float* ints[6];
     const size_t n[6] = {ms.experts, ms.pairs, ms.pairs, ms.pairs, ms.slots, ms.tiles};
@@ -985,7 +985,7 @@ struct Gemm {
 
 // x += norm2 of the experts' output for rows of x.  sub: as many rows of working memory.
 pg_status moe_rows(const pg_model* model, const StackLayer& l, const StackCache::MoeBuffers& b, const Gemm& gemm, float* x,
-                   float* sub, int rows, hipStream_t s, ProfileMarks* marks) {
+                   float* sub, int rows, bool drawn, hipStream_t s, ProfileMarks* marks) {
   const StackModel& m = *model->stack;
   const pgk::Moe& e = l.ffn.moe;
   const int Cp = m.width_pad;
@@ -1002,7 +1002,7 @@ pg_status moe_rows(const pg_model* model, const StackLayer& l, const StackCache:
     return PG_OK;
   }
   pgk::MoeRoute t = b.route;
-  t.tile_rows = moe_tile_rows(e, rows);
+  t.tile_rows = moe_tile_rows(e, rows, drawn);
   t.max_slots = pgk::moe_max_slots(e, rows, t.tile_rows);
   PG_HIP(pgk::launch_moe_route(e, t, parts > 1 ? gemm.ws : b.logits, rows, s, parts));
   pgk::GemmArgs g{};
@@ -1137,7 +1137,7 @@ pg_status post_norm_step(const pg_model* model, pg_kv_cache* c, ProfileMarks* ma
     } else if (f.kind == PostFeedForward::kMoe) {
       const bool fused = B == 1 && pgk::moe_router_fits(f.moe, Cp);
       if (B > 1) {
-        if (pg_status e = moe_rows(model, l, st.moe, gemm, x, st.sub, B, s, marks)) return e;
+        if (pg_status e = moe_rows(model, l, st.moe, gemm, x, st.sub, B, c->drawn, s, marks)) return e;
       } else {
         if (!fused) PG_HIP(enter(f.router_w, nullptr, st.moe.logits, f.moe.experts_pad, false));
         pgk::MoeRow r{};
@@ -1337,7 +1337,7 @@ pg_status post_norm_rows(const pg_model* model, pg_kv_cache* c, const uint32_t* 
       kv_floats = std::max(kv_floats, all * up(l.latent.v_row + l.latent.heads * l.latent.vdim, 4));
     }
     if (l.ffn.kind == PostFeedForward::kDense) act_floats = std::max(act_floats, rows * l.ffn.ff_pad);
-    if (l.ffn.kind == PostFeedForward::kMoe) ms.add(l.ffn.moe, (int)rows, m.width_pad);
+    if (l.ffn.kind == PostFeedForward::kMoe) ms.add(l.ffn.moe, (int)rows, m.width_pad, c->drawn);
   }
   act_floats = std::max(act_floats, ms.act);
   const size_t ws_floats = 8 * rows * Cp;
@@ -1401,7 +1401,7 @@ pg_status post_norm_rows(const pg_model* model, pg_kv_cache* c, const uint32_t* 
       PG_MARK(kMlpFc);
       PG_HIP(gemm.product(R, act, f.ff_pad, f.down_w, sub, (int)Cp, f.ff_pad, f.down_b, pgk::GEMM_BIAS, x, l.norm2));
     } else if (f.kind == PostFeedForward::kMoe) {
-      if (pg_status e = moe_rows(model, l, moe, gemm, x, sub, R, s, marks)) return e;
+      if (pg_status e = moe_rows(model, l, moe, gemm, x, sub, R, c->drawn, s, marks)) return e;
     }
     PG_MARK(kMlpProj);
   }
