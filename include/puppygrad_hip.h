@@ -105,8 +105,10 @@ typedef struct pg_hip_options {
   uint32_t gemm_b9_min_rows;        /* f32 weights: products over at least this many input rows
                                        run on the bf16 matrix cores with both operands cut into
                                        three bf16 parts where the planner finds enough tiles
-                                       (default 65: from 33 rows on where they are better kept
-                                       cut, too; 0xffffffff: never) */
+                                       (0xffffffff: never).  Default: 65, and 33 to 64 rows
+                                       where activations are better kept cut; set, 65 too, it
+                                       is the bound for both.  65 to 128 rows are not kept cut
+                                       at any setting */
   uint32_t seq_gemm_min_tokens;     /* prompts of at least this many tokens take the GEMM
                                        prefill, shorter ones run token by token through the
                                        decode path (default 4; at most 65536) */

@@ -253,18 +253,17 @@ constexpr float kReduceLaunch = 4.5f, kNormLaunch = 4.0f, kNormValues = 2.0f;
 //    rows 2.45 / 2.18, 350 rows 2.60 / 2.69; 768, 500 rows 1.14 / 1.08, 600 rows 1.21 / 1.25.  33 rows, 1280: 2.12 / 1.98; at 32 and fewer the 32-row kernel is as fast.
 //  - int8 rows: 1600, 400 rows 9.15 / 8.23, 500 rows 9.98 / 10.53; 1280, 500 rows 5.81 / 5.11, 600 rows 6.64 / 6.83; 768, 850 rows
 //    1.65 / 1.52.  Up to 32 rows, a step of 20 at 1280 1.89 / 1.85, of 32 2.13 / 2.15, of 32 at 768 0.60 / 0.57.
-bool gemm_takes_cut(int M, int K, int N, int w_bf16, int w_int8, int b9_min_rows) {
+bool gemm_takes_cut(int M, int K, int N, int w_bf16, int w_int8, int f32_min_rows) {
   if (K < 256 || K % 32 != 0 || N % 32 != 0) return false;  // (narrower: no step for some of the eight wavefronts)
   const double mn = (double)M * N, mnk = mn * K;
   if (w_int8) return M >= 17 && mn <= 2.7e6 && (M > 32 || mnk <= 0.17e9);
-  if (M < 33) return false;
+  if (M < kCutFormMinRows) return false;
   const bool narrow = K <= 768;
   if (w_bf16) return mn <= (narrow ? 1.6e6 : 1.4e6) && mnk <= 1.35e9;
-  // (65 to 128 rows stay on the f32 cores: there gemm_b9_min_rows gives the same results at every setting, which its
-  // tests hold; 100 rows at 1280 are 3.88 ms, 2.95 in this form)
+  // (65 to 128 rows stay on the f32 cores at the price of 3.88 ms for 100 rows at 1280 that take 2.95 in this form: models
+  // tuned with gemm_b9_min_rows get the same results there at every setting)
   if (M > 64 && M <= 128) return false;
-  if (!(narrow ? mn <= 3.2e6 : mn <= 1.4e6 && mnk <= 1.7e9)) return false;
-  return M >= b9_min_rows || b9_min_rows <= kCutMinRows;
+  return M >= f32_min_rows && (narrow ? mn <= 3.2e6 : mn <= 1.4e6 && mnk <= 1.7e9);
 }
 
 bool gemm_cut_rows_plan(const GemmArgs& a, int num_cus, CutRowsPlan* plan) {

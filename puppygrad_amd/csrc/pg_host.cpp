@@ -513,7 +513,7 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
   // split-K partial tiles of the projections back to n_embd columns (up to 8 parts)
   const size_t ws_floats = 8 * n * g.C;
   // the projections' inputs (XN, ATT, HB) in cut form
-  const bool cut = !c->drawn && hd == pgk::kHeadDim && pgk::gemm_takes_cut(T, C, I, m->w_bf16, m->w_i8, m->gemm_b9_min_rows);
+  const bool cut = !c->drawn && hd == pgk::kHeadDim && pgk::gemm_takes_cut(T, C, I, m->w_bf16, m->w_i8, m->cut_form_min_rows);
   {
     auto form = [&](size_t cols) { return cut ? std::max(n * cols, pgk::cut_floats(n, cols)) : n * cols; };
     auto up = [](size_t v) { return (v + 63) / 64 * 64; };  // 256-byte boundaries
@@ -989,6 +989,7 @@ pg_status pg_gpt2_create(const pg_gpt2_config* config, const pg_gpt2_weights_vie
   m->attn_blocks_per_cu = opts.attn_blocks_per_cu ? (int)opts.attn_blocks_per_cu : 4;
   m->gemm_split_items = opts.gemm_split_items_per_cu ? (int)opts.gemm_split_items_per_cu : 3;
   m->gemm_b9_min_rows = opts.gemm_b9_min_rows ? (int)std::min(opts.gemm_b9_min_rows, 0x7fffffffu) : pgk::kCutMinRows;
+  m->cut_form_min_rows = opts.gemm_b9_min_rows ? m->gemm_b9_min_rows : pgk::kCutFormMinRows;
   m->seq_gemm_min_tokens = opts.seq_gemm_min_tokens ? opts.seq_gemm_min_tokens : 4;
   hipDeviceProp_t prop;
   PG_HIP(hipGetDeviceProperties(&prop, opts.device));
@@ -1247,7 +1248,7 @@ pg_status pg_kv_cache_create(const pg_model* m, uint32_t batch, pg_kv_cache** ou
   // Batches whose projections all run on the 32-row kernel keep that kernel's inputs packed
   // (32 row slots whatever B is).
   raw->cut_form = B > 1 && hd == pgk::kHeadDim &&
-                  pgk::gemm_takes_cut((int)B, (int)g.C, (int)g.I, m->w_bf16, m->w_i8, m->gemm_b9_min_rows);
+                  pgk::gemm_takes_cut((int)B, (int)g.C, (int)g.I, m->w_bf16, m->w_i8, m->cut_form_min_rows);
   raw->pack32 = !raw->cut_form && B > 1 && B <= 32 && g.C % 16 == 0 && g.I % 16 == 0 && !m->w_i8 &&
                 pgk::gemm_takes_rows32((int)B, (int)g.C, (int)g.C, m->w_bf16) &&
                 pgk::gemm_takes_rows32((int)B, (int)g.I, (int)g.I, m->w_bf16);

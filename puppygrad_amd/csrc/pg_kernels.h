@@ -217,6 +217,7 @@ enum GemmEpilogue : int {
 // C[M,N] = epilogue(A[M,K] . W[N,K]^T + bias): A rows lda floats apart, C (and resid)
 // rows ldc apart, W dense [N][K]; bias may be nullptr.
 constexpr int kCutMinRows = 65;  // (fewer: the 32-row kernel)
+constexpr int kCutFormMinRows = 33;  // (f32 and bf16 rows; up to 32 the 32-row kernel is as fast)
 struct GemmArgs {
   int w_bf16 = 0;  // W holds bf16 values
   const float* w_scale = nullptr;  // != nullptr: W holds int8 values, w_scale[n] scales row n
@@ -291,8 +292,8 @@ enum ActForm : int { FORM_ROWS = 0, FORM_PACKED32 = 1, FORM_CUT = 2 };
 __host__ __device__ inline int cut_rows(int M) { return (M + 15) / 16 * 16; }
 inline size_t cut_floats(size_t M, size_t K) { return (M + 15) / 16 * 16 * K * 3 / 2; }
 // Whether M rows of activations K and N columns wide (each a multiple of 32) are best kept in cut form where they meet
-// rows of W stored so.
-bool gemm_takes_cut(int M, int K, int N, int w_bf16, int w_int8, int b9_min_rows);
+// rows of W stored so.  f32_min_rows: input rows from which f32 rows may.
+bool gemm_takes_cut(int M, int K, int N, int w_bf16, int w_int8, int f32_min_rows);
 // Whether launch_gemm multiplies an M x K input with the 32-row decode kernel.
 bool gemm_takes_rows32(int M, int K, int lda, int w_bf16);
 bool gemm_supported(const GemmArgs& a);

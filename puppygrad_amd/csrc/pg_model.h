@@ -115,7 +115,8 @@ struct pg_model {
   bool item_keys_256_ok = false;    // the device holds the grid of the 256-key instance
   int attn_blocks_per_cu = 4;       // per-operation / batched decode attention
   int gemm_split_items = 3;         // tile GEMM split-K
-  int gemm_b9_min_rows = pgk::kCutMinRows;  // f32 rows on the bf16 matrix cores from this many input rows
+  int gemm_b9_min_rows = pgk::kCutMinRows;  // f32 rows on the bf16 matrix cores from this many input rows,
+  int cut_form_min_rows = pgk::kCutFormMinRows;  // and with activations kept in cut form: the same, 33 where the caller set none
   size_t seq_gemm_min_tokens = 4;   // prompts at least this long take the GEMM prefill
   int w_bf16 = 0;                   // wte and the block matrices are stored as bf16
   // int8 storage (QuantizedRows, src/models/cpu.rs:26-56): the block matrices hold int8 rows

@@ -158,6 +158,24 @@ def test_prompts(storage, width, n):
     assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
 
 
+def test_a_set_bound_of_the_bf16_cores_holds_for_the_cut_form():
+    """Left alone, prompts of 33 to 64 rows are kept cut; a set bound, the default's own number too, keeps fewer rows on the
+    f32 cores."""
+    cfg = Gpt2Config(vocab_size=97, n_positions=64, n_embd=768, n_layer=1, n_head=12)
+    w = synth.random_weights(cfg, 0x5EED0A02, perturb=True)
+    ids = [int(t) for t in synth.token_ids(64, 0x70C00A02, cfg.vocab_size)]
+
+    def logits(rows, bound):
+        model = Gpt2Model.new(cfg, w, Gpt2HipConfig(gemm_b9_min_rows=bound))
+        return model.prefill(ids[:rows], model.new_kv_cache()).to_host()
+
+    for rows in (33, 64):
+        on_f32_cores = logits(rows, 0xffffffff)
+        assert (logits(rows, 0) != on_f32_cores).any() and (logits(rows, rows) != on_f32_cores).any()
+        for bound in (rows + 1, 65, 128):
+            np.testing.assert_array_equal(logits(rows, bound), on_f32_cores)
+
+
 @pytest.mark.parametrize("storage,batch,n", [("f32", 33, 3), ("f32", 48, 20), ("bf16", 40, 7), ("int8", 17, 5), ("int8", 31, 9), ("int8", 65, 4)])
 def test_batched_steps(storage, batch, n):
     cfg = Gpt2Config(vocab_size=300, n_positions=600, n_embd=768, n_layer=2, n_head=12)
