@@ -490,6 +490,13 @@ bool gemm_path_ok(const pg_model* m, size_t n) {
          (g.hd() == 64 || n * g.H * n * sizeof(float) <= (256u << 20));
 }
 
+// Whether the inputs of the model's projections are best kept in cut form when they have so many rows.
+bool takes_cut_form(const pg_model* m, size_t rows) {
+  const Cfg& g = m->cfg;
+  return g.hd() == pgk::kHeadDim &&
+         pgk::gemm_takes_cut((int)rows, (int)g.C, (int)g.I, m->w_bf16, m->w_i8, m->cut_form_min_rows);
+}
+
 // Full-sequence forward of the nb sequences b .. b + nb - 1 over ids[nb][n] (each one
 // Gpt2Model::forward, src/models/gpt2/rust.rs:831-882, block_forward at 1053-1134) with MFMA
 // GEMMs over all nb * n rows at once and tiled causal attention per sequence; K and V of every
@@ -513,7 +520,7 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
   // split-K partial tiles of the projections back to n_embd columns (up to 8 parts)
   const size_t ws_floats = 8 * n * g.C;
   // the projections' inputs (XN, ATT, HB) in cut form
-  const bool cut = !c->drawn && hd == pgk::kHeadDim && pgk::gemm_takes_cut(T, C, I, m->w_bf16, m->w_i8, m->cut_form_min_rows);
+  const bool cut = !c->drawn && takes_cut_form(m, n);
   {
     auto form = [&](size_t cols) { return cut ? std::max(n * cols, pgk::cut_floats(n, cols)) : n * cols; };
     auto up = [](size_t v) { return (v + 63) / 64 * 64; };  // 256-byte boundaries
@@ -659,8 +666,9 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
   // same call: fused into the projection's reduce where it has one)
   // c->pack32: the inputs of the projections (xn_b, att_b, hbuf) are held in the packed form
   // that the 32-row kernel reads with contiguous loads; their producers write them that way.
-  // c->cut_form: the same in cut form, except for the logits' input.
-  const int pk = c->pack32 ? 1 : 0, cut = c->cut_form ? 1 : 0;
+  // c->cut_form: there is room for them in cut form, which this model's rows take (the cache may have been made for
+  // another model of these sizes); not the logits' input.
+  const int pk = c->pack32 ? 1 : 0, cut = c->cut_form && takes_cut_form(m, c->B) ? 1 : 0;
   const int form = cut ? pgk::FORM_CUT : pk ? pgk::FORM_PACKED32 : pgk::FORM_ROWS;
   auto gemm = [&](const float* A, int lda, const float* W, const float* bias, float* Cout,
                   int ldc, int N, int K, int epi, const float* ln_g = nullptr,
@@ -1247,8 +1255,7 @@ pg_status pg_kv_cache_create(const pg_model* m, uint32_t batch, pg_kv_cache** ou
   PG_HIP(hipMalloc(&raw->q, B * g.C * sizeof(float)));
   // Batches whose projections all run on the 32-row kernel keep that kernel's inputs packed
   // (32 row slots whatever B is).
-  raw->cut_form = B > 1 && hd == pgk::kHeadDim &&
-                  pgk::gemm_takes_cut((int)B, (int)g.C, (int)g.I, m->w_bf16, m->w_i8, m->cut_form_min_rows);
+  raw->cut_form = B > 1 && takes_cut_form(m, B);
   raw->pack32 = !raw->cut_form && B > 1 && B <= 32 && g.C % 16 == 0 && g.I % 16 == 0 && !m->w_i8 &&
                 pgk::gemm_takes_rows32((int)B, (int)g.C, (int)g.C, m->w_bf16) &&
                 pgk::gemm_takes_rows32((int)B, (int)g.I, (int)g.I, m->w_bf16);

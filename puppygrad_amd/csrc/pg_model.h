@@ -158,7 +158,7 @@ struct pg_kv_cache {
   // apart, and logits moved by their last bits (another kernel's order of additions: 5 10^-7) change two streams of 80 in
   // five from some id on.  Decode steps have one kernel either way.
   bool drawn = false;
-  bool cut_form = false;  // batched step: xn_b, att_b and hbuf are in cut form (pgk::FORM_CUT)
+  bool cut_form = false;  // batched step: xn_b, att_b and hbuf have room for the cut form (pgk::FORM_CUT)
   bool pack32 = false;  // batched step: xn_b, att_b and hbuf are packed (pgk::packed32_index)
   // device-side candidate selection for sampling, allocated at first use: kept candidates
   // (ids, then values, then [count]) and the recent ids of the repeat penalty, with pinned

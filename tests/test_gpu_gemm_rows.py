@@ -192,3 +192,26 @@ def test_batched_steps(storage, batch, n):
         model.forward_one(int(ids[b, n]), single)
         want = model.forward_one(int(ids[b, n + 1]), single).to_host()
         assert np.linalg.norm(got[b] - want) <= 1e-5 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("maker,user,batch", [("f32", "f32 never", 40), ("int8", "f32", 17), ("int8", "bf16", 31)])
+def test_a_cache_of_another_model_leaves_the_step_to_its_own(maker, user, batch):
+    """The form of a batched step's activations is the stepping model's, whichever model of these sizes made the cache."""
+    cfg = Gpt2Config(vocab_size=300, n_positions=32, n_embd=768, n_layer=2, n_head=12)
+    w = synth.random_weights(cfg, 0x5EED0A03, perturb=True)
+    store = {"f32": _lib.PG_STORE_F32, "bf16": _lib.PG_STORE_BF16, "int8": _lib.PG_STORE_INT8}
+
+    def model(name):
+        bound = 0xffffffff if name.endswith("never") else 0
+        return Gpt2Model.new(cfg, w, Gpt2HipConfig(weight_storage=store[name.split()[0]], gemm_b9_min_rows=bound))
+
+    ids = synth.token_ids(batch * 6, 0x70C00A03, cfg.vocab_size).reshape(batch, 6)
+    m, other = model(user), model(maker)
+    steps = []
+    for cache in (m.new_kv_cache(batch), other.new_kv_cache(batch)):
+        m.prefill_batch(np.ascontiguousarray(ids[:, :5]), cache)
+        steps.append(m.forward_one_batch(ids[:, 5], cache).to_host())
+    if batch > 32:
+        np.testing.assert_array_equal(steps[1], steps[0])
+    else:  # (a cache of the model's own is packed: the same kernel, sums of at most 3072 terms in other orders)
+        assert np.linalg.norm(steps[1] - steps[0]) <= 1e-5 * np.linalg.norm(steps[0])
