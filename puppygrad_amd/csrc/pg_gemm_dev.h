@@ -30,8 +30,6 @@ struct CutRowsPlan {
 };
 bool gemm_cut_rows_plan(const GemmArgs& a, int num_cus, CutRowsPlan* plan);
 hipError_t launch_gemm_cut_rows(const GemmArgs& a, int epi, const CutRowsPlan& p, hipStream_t s);
-// x[M][K] into cut form (K a multiple of 8)
-hipError_t launch_to_cut(const float* x, void* to, int M, int K, hipStream_t s);
 // (bf16 rows; tiles of tile_rows = 64 or 128 rows)
 hipError_t launch_gemm_cut_grouped(const GemmArgs& a, int epi, int tile_rows, hipStream_t s);
 

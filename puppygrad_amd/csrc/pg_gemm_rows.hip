@@ -199,21 +199,15 @@ __global__ __launch_bounds__(512) void k_gemm_cut_rows(GemmArgs a) {
   }
 }
 
-// x[M][K] in cut form
-__global__ __launch_bounds__(256) void k_to_cut(const float* x, void* to, int M, int K) {
-  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
-  if (i >= (size_t)M * K) return;
-  store_cut4(to, cut_rows(M), i / K, i % K, f4{x[i], x[i + 1], x[i + 2], x[i + 3]});
-}
-
 template <int EPI, int WT>
 hipError_t launch_form(const GemmArgs& a, const CutRowsPlan& p, hipStream_t s) {
   const dim3 grid((unsigned)((a.N + a.rows_per_block - 1) / a.rows_per_block), (unsigned)p.parts,
                   (unsigned)((a.M + 16 * p.mt - 1) / (16 * p.mt)));
 #define PG_CASE(MT, NG) \
   if (p.mt == MT && p.ng == NG) { hipLaunchKernelGGL((k_gemm_cut_rows<EPI, WT, MT, NG>), grid, dim3(512), 0, s, a); return hipGetLastError(); }
-  PG_CASE(2, 1) PG_CASE(3, 1) PG_CASE(4, 1)
-  PG_CASE(2, 2) PG_CASE(3, 2) PG_CASE(4, 2)
+  if constexpr (WT == 2) { PG_CASE(2, 1) PG_CASE(2, 2) }  // (17 to 32 rows, which the other storages leave to the 32-row kernel)
+  PG_CASE(3, 1) PG_CASE(4, 1)
+  PG_CASE(3, 2) PG_CASE(4, 2)
   PG_CASE(3, 3) PG_CASE(4, 3)
   if constexpr (WT != 0) { PG_CASE(3, 4) PG_CASE(4, 4) }
 #undef PG_CASE
@@ -271,7 +265,7 @@ bool gemm_cut_rows_plan(const GemmArgs& a, int num_cus, CutRowsPlan* plan) {
       a.c_packed || a.ln_packed || a.ldc % 4 != 0 || a.rms_cols || a.post_x || (a.c_cut && a.ldc != a.N))
     return false;
   const int wt = a.w_scale ? 2 : a.w_bf16 ? 1 : 0;
-  const int groups = (a.M + 63) / 64, mt = std::max(2, ((a.M + groups - 1) / groups + 15) / 16);
+  const int groups = (a.M + 63) / 64, mt = std::max(wt == 2 ? 2 : 3, ((a.M + groups - 1) / groups + 15) / 16);
   const int m_blocks = (a.M + 16 * mt - 1) / (16 * mt), steps = a.K / 32;
   const float mn = (float)a.M * (float)a.N * 1e-6f;
   const RowsPace& p = kRowsPace[wt];
@@ -306,12 +300,6 @@ hipError_t launch_gemm_cut_rows(const GemmArgs& a0, int epi, const CutRowsPlan& 
   a.rows_per_block = p.rows;
   if (a.w_scale) return launch_wt<2>(a, epi, p, s);
   return a.w_bf16 ? launch_wt<1>(a, epi, p, s) : launch_wt<0>(a, epi, p, s);
-}
-
-hipError_t launch_to_cut(const float* x, void* to, int M, int K, hipStream_t s) {
-  if (M < 1 || K < 8 || K % 8 != 0 || (size_t)M * K > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_to_cut, dim3((unsigned)(((size_t)M * K / 4 + 255) / 256)), dim3(256), 0, s, x, to, M, K);
-  return hipGetLastError();
 }
 
 }  // namespace pgk

@@ -174,6 +174,13 @@ __global__ __launch_bounds__(kBlk) void k_attention_rows(const float* __restrict
   }
 }
 
+// (for the tests: x[M][K] in cut form, K a multiple of 8)
+__global__ __launch_bounds__(256) void k_to_cut(const float* x, void* to, int M, int K) {
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= (size_t)M * K) return;
+  pgk::store_cut4(to, pgk::cut_rows(M), i / K, i % K, pgk::f4{x[i], x[i + 1], x[i + 2], x[i + 3]});
+}
+
 // (for the tests: the sums of pg_wave.h, a wavefront a block)
 __global__ __launch_bounds__(64) void k_lane_sums(const float* x, const float* y, float* out) {
   const size_t i = (size_t)blockIdx.x * 64 + threadIdx.x, n = (size_t)gridDim.x * 64;
@@ -414,7 +421,9 @@ pg_status pg_testing_cut_product_dev(int32_t device, void* stream, const float* 
   a.A = static_cast<const float*>(cut); a.W = static_cast<const float*>(weight); a.w_bf16 = storage == PG_STORE_BF16;
   a.w_scale = scales; a.bias = bias; a.C = out; a.M = (int)rows; a.N = (int)out_f; a.K = (int)in_f; a.lda = (int)in_f;
   a.ldc = (int)out_f; a.a_cut = 1; a.ws = out; a.ws_floats = (size_t)parts * rows * out_f;
-  PG_HIP(pgk::launch_to_cut(x, cut, (int)rows, (int)in_f, static_cast<hipStream_t>(stream)));
+  hipLaunchKernelGGL(k_to_cut, dim3((unsigned)((rows * in_f / 4 + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream), x,
+                     cut, (int)rows, (int)in_f);
+  PG_HIP(hipGetLastError());
   PG_HIP(pgk::launch_gemm_cut_rows(a, pgk::GEMM_BIAS, {mt, ng, block_rows, parts}, static_cast<hipStream_t>(stream)));
   return PG_OK;
 }
