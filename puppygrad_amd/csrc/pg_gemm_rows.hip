@@ -223,41 +223,48 @@ hipError_t launch_wt(const GemmArgs& a, int epi, const CutRowsPlan& p, hipStream
     default: return hipErrorInvalidValue;
   }
 }
-// Time of a product in microseconds, fitted over 1820 plans of the four GPT-2 widths' projections at 24 to 320 rows (W
-// from HBM): the plan of least predicted time is 1 % slower than the best measured one in the mean (f32 rows 1.1, bf16
-// 1.3, int8 0.9 %; 27 % at most).  `most`: a block of 64 x 64, whose registers spill.
+// Time of a product in microseconds, fitted over 24860 plans of the four GPT-2 widths' projections, W from HBM, at rows on
+// both sides of where the form ends (f32 rows to 1100, bf16 to 700, int8 to 1200; plans near the best weigh most): the
+// plan of least predicted time is 1.9 % slower than the best measured one in the mean for f32 rows, 1.6 bf16, 1.1 int8 (20 %
+// at most; constants from 24 to 320 rows alone: 2.8, 2.7 and 2.0 %, 47 % at most).  `most`: a block of 64 x 64, whose
+// registers spill.  `reduce`: the launch that adds the parts; `norm`, `norm_values`: that of a norm by itself, and per
+// 10^6 values.
 struct RowsPace {
-  float start, round, step, mt, ng, both, most, fill, part;
+  float start, round, step, mt, ng, both, most, fill, part, reduce, norm, norm_values;
 };
-constexpr RowsPace kRowsPace[3] = {{2.93f, 0.252f, -0.151f, 0.144f, 0.522f, 0.013f, 0.0f, 0.145f, 1.393f},
-                                   {2.763f, -0.129f, -0.004f, 0.167f, 0.329f, -0.010f, 0.55f, 0.087f, 1.735f},
-                                   {2.838f, 0.314f, 0.034f, 0.163f, 0.170f, 0.016f, 0.10f, 0.056f, 1.08f}};
-// A reduction's launch, with or without a norm; a norm by itself, and what it takes per 10^6 values.
-constexpr float kReduceLaunch = 4.5f, kNormLaunch = 4.0f, kNormValues = 2.0f;
+constexpr RowsPace kRowsPace[3] = {
+    {3.025f, 1.212f, -0.950f, 0.258f, 0.848f, -0.080f, 0.0f, 0.164f, 2.563f, 2.957f, 2.585f, 4.907f},
+    {2.364f, 1.014f, -0.375f, 0.131f, 0.328f, 0.003f, 0.443f, 0.106f, 2.572f, 3.491f, 3.242f, 5.680f},
+    {2.593f, 1.357f, -0.184f, 0.082f, 0.073f, 0.063f, 0.113f, 0.074f, 2.538f, 3.331f, 2.816f, 7.044f}};
 
 }  // namespace
 
 // The rows up to which a model's four projections take this form, from whole prompts timed both ways (ms, other kernels
-// first).  They end where a CU has more than one block and the tiles of pg_gemm_cut.hip, which read an input row once
-// for 128 columns instead of 64, have one each:
-//  - f32 rows: width 1600, 150 rows 7.42 / 6.68, 200 rows 7.93 / 8.40; 1280, 256 rows 4.87 / 4.66, 300 rows 5.65 / 5.87;
-//    1024, 300 rows 2.95 / 2.65, 350 rows 3.08 / 3.17.  33 rows, 1280: 2.62 / 2.26.  At width 768 the tiles leave a third of
-//    the CUs without one at 1024 rows yet: 500 rows 1.45 / 1.30, 700 rows 1.77 / 1.76, 1024 rows 2.07 / 1.99.
-//  - bf16 rows: 1600, 100 rows 4.57 / 4.06, 150 rows 5.09 / 5.15; 1280, 200 rows 3.83 / 3.49, 300 rows 4.34 / 4.41; 1024, 300
-//    rows 2.45 / 2.18, 350 rows 2.60 / 2.69; 768, 500 rows 1.14 / 1.08, 600 rows 1.21 / 1.25.  33 rows, 1280: 2.12 / 1.98; at 32 and fewer the 32-row kernel is as fast.
-//  - int8 rows: 1600, 400 rows 9.15 / 8.23, 500 rows 9.98 / 10.53; 1280, 500 rows 5.81 / 5.11, 600 rows 6.64 / 6.83; 768, 850 rows
-//    1.65 / 1.52.  Up to 32 rows, a step of 20 at 1280 1.89 / 1.85, of 32 2.13 / 2.15, of 32 at 768 0.60 / 0.57.
-bool gemm_takes_cut(int M, int K, int N, int w_bf16, int w_int8, int f32_min_rows) {
+// first).  A step in this form's time is a round of blocks (64 rows by 48 rows of W, 64 for int8 rows) over the CUs, so the
+// line is a number of rounds of the widest product, past which the tiles of pg_gemm_cut.hip, which read an input row once
+// for 128 columns, are the faster ones:
+//  - f32 and bf16 rows, two rounds.  f32 at width 1600: 192 rows 7.54 / 6.76, 193 rows 7.80 / 8.31; 1280: 256 rows 4.82 /
+//    4.54, 257 rows 5.38 / 5.59; 1024: 320 rows 2.99 / 2.64, 400 rows 3.37 / 3.31, 600 rows 4.05 / 4.20; 33 rows, 1600: 4.02 / 3.43.
+//    bf16 at 1600: 131 rows 4.96 / 4.51, 192 rows 5.23 / 5.23, 193 rows 5.74 / 6.37; 1280: 256 rows 3.89 / 3.60, 257 rows
+//    3.99 / 4.23; 1024: 320 rows 2.41 / 2.15, 400 rows 2.62 / 2.60; 768: 512 rows 1.09 / 1.03, 560 rows 1.19 / 1.17, 800 rows
+//    1.18 / 1.36.
+//  - f32 rows up to width 768, where the tiles leave a third of the CUs without one: four rounds and 1024 rows.  768: 512 rows
+//    1.46 / 1.29, 700 rows 1.76 / 1.70, 1024 rows 2.11 / 2.03 (8 x 128 1.90 / 1.80), 1026 rows 2.09 / 2.36; 512: 600 rows 1.12 /
+//    1.04, 1000 rows 1.41 / 1.39, 1200 rows 1.47 / 1.57.
+//  - int8 rows, three rounds.  1600: 448 rows 9.24 / 8.40, 449 rows 9.69 / 9.88; 1280: 576 rows 6.37 / 5.65, 577 rows 6.54 /
+//    6.53; 1024: 768 rows 3.89 / 3.74, 769 rows 4.08 / 4.00; 768: 1024 rows 1.73 / 1.61, 1026 rows 1.69 / 1.72.  Up to 32 rows,
+//    a step of 20 at 1280 1.89 / 1.85, of 32 2.13 / 2.15, of 32 at 768 0.60 / 0.57.
+bool gemm_takes_cut(int M, int K, int N, int w_bf16, int w_int8, int f32_min_rows, int num_cus) {
   if (K < 256 || K % 32 != 0 || N % 32 != 0) return false;  // (narrower: no step for some of the eight wavefronts)
-  const double mn = (double)M * N, mnk = mn * K;
-  if (w_int8) return M >= 17 && mn <= 2.7e6 && (M > 32 || mnk <= 0.17e9);
+  const int cols = w_int8 ? 64 : 48;  // of a full block, 64 rows
+  const long blocks = (long)((std::max(N, 3 * K) + cols - 1) / cols) * ((M + 63) / 64);
+  if (w_int8) return M >= 17 && blocks <= 3L * num_cus && (M > 32 || (double)M * N * K <= 0.17e9);
   if (M < kCutFormMinRows) return false;
-  const bool narrow = K <= 768;
-  if (w_bf16) return mn <= (narrow ? 1.6e6 : 1.4e6) && mnk <= 1.35e9;
+  if (w_bf16) return blocks <= 2L * num_cus;
   // (65 to 128 rows stay on the f32 cores at the price of 3.88 ms for 100 rows at 1280 that take 2.95 in this form: models
   // tuned with gemm_b9_min_rows get the same results there at every setting)
   if (M > 64 && M <= 128) return false;
-  return M >= f32_min_rows && (narrow ? mn <= 3.2e6 : mn <= 1.4e6 && mnk <= 1.7e9);
+  return M >= f32_min_rows && (K <= 768 ? blocks <= 4L * num_cus && M <= 4 * num_cus : blocks <= 2L * num_cus);
 }
 
 bool gemm_cut_rows_plan(const GemmArgs& a, int num_cus, CutRowsPlan* plan) {
@@ -281,7 +288,7 @@ bool gemm_cut_rows_plan(const GemmArgs& a, int num_cus, CutRowsPlan* plan) {
       const float rounds = (float)(((steps + parts - 1) / parts + 7) / 8);
       const float us = p.start + turns * (p.round + rounds * (p.step + p.mt * mt + p.ng * ng + p.both * mt * ng + (mt * ng == 16 ? p.most : 0.0f))) +
                        p.fill * (float)blocks / (float)num_cus * rounds * mt +
-                       (parts > 1 ? kReduceLaunch + p.part * parts * mn : a.ln_out ? kNormLaunch + kNormValues * mn : 0.0f);
+                       (parts > 1 ? p.reduce + p.part * parts * mn : a.ln_out ? p.norm + p.norm_values * mn : 0.0f);
       if (best == 0.0f || us < best) {
         best = us;
         *plan = {mt, ng, rows, parts};

@@ -494,7 +494,7 @@ bool gemm_path_ok(const pg_model* m, size_t n) {
 bool takes_cut_form(const pg_model* m, size_t rows) {
   const Cfg& g = m->cfg;
   return g.hd() == pgk::kHeadDim &&
-         pgk::gemm_takes_cut((int)rows, (int)g.C, (int)g.I, m->w_bf16, m->w_i8, m->cut_form_min_rows);
+         pgk::gemm_takes_cut((int)rows, (int)g.C, (int)g.I, m->w_bf16, m->w_i8, m->cut_form_min_rows, m->num_cus);
 }
 
 // Full-sequence forward of the nb sequences b .. b + nb - 1 over ids[nb][n] (each one

@@ -293,7 +293,7 @@ __host__ __device__ inline int cut_rows(int M) { return (M + 15) / 16 * 16; }
 inline size_t cut_floats(size_t M, size_t K) { return (M + 15) / 16 * 16 * K * 3 / 2; }
 // Whether M rows of activations K and N columns wide (each a multiple of 32) are best kept in cut form where they meet
 // rows of W stored so.  f32_min_rows: input rows from which f32 rows may.
-bool gemm_takes_cut(int M, int K, int N, int w_bf16, int w_int8, int f32_min_rows);
+bool gemm_takes_cut(int M, int K, int N, int w_bf16, int w_int8, int f32_min_rows, int num_cus);
 // Whether launch_gemm multiplies an M x K input with the 32-row decode kernel.
 bool gemm_takes_rows32(int M, int K, int lda, int w_bf16);
 bool gemm_supported(const GemmArgs& a);

@@ -428,6 +428,11 @@ pg_status pg_testing_cut_product_dev(int32_t device, void* stream, const float* 
   return PG_OK;
 }
 
+// gemm_takes_cut
+int32_t pg_testing_takes_cut(int32_t rows, int32_t width, int32_t inner, int32_t storage, int32_t f32_min_rows, int32_t num_cus) {
+  return pgk::gemm_takes_cut(rows, width, inner, storage == PG_STORE_BF16, storage == PG_STORE_INT8, f32_min_rows, num_cus);
+}
+
 // Attention of `sequences` prompts of `rows` tokens each, head size 64, keys and values to panels [sequences][heads][rows][64]:
 // in blocks of the given shape of pg_attn_cut.hip (0: as the planner has it).
 pg_status pg_testing_attention_rows_dev(int32_t device, void* stream, const float* qkv, uint64_t rows, uint64_t heads,

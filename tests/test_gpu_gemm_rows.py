@@ -131,13 +131,16 @@ def test_infinite_weights_and_weights_past_bf16():
     np.testing.assert_allclose(got[:, [9, 11]], x.astype(np.float64) @ w[[9, 11]].astype(np.float64).T, rtol=1e-5)
 
 
-# the first and the last sizes that take the form, ragged blocks between them; logits of a prompt against those of its
-# last token alone behind the others, which the one-sequence kernels form
+# sizes that take the form: the first and the last of a width, ragged blocks between them; and the first past them (test_cut_form.py
+# has all of them).  Logits of a prompt against those of its last token alone behind the others, which the one-sequence
+# kernels form
 @pytest.mark.parametrize("storage,width,n", [("f32", 768, 33), ("f32", 768, 64), ("f32", 1024, 130), ("f32", 1600, 166), ("bf16", 768, 49),
                                              ("bf16", 1600, 131), ("int8", 768, 17), ("int8", 768, 97), ("int8", 1600, 420),
-                                             ("int8", 1280, 300), ("f32", 768, 455), ("f32", 768, 456)])
+                                             ("int8", 1280, 300), ("f32", 768, 455), ("f32", 768, 456), ("f32", 768, 1024), ("f32", 768, 1025),
+                                             ("f32", 1280, 256), ("f32", 1600, 192), ("bf16", 768, 512), ("bf16", 768, 513), ("bf16", 1600, 192),
+                                             ("int8", 768, 1024), ("int8", 768, 1025), ("int8", 1600, 448)])
 def test_prompts(storage, width, n):
-    cfg = Gpt2Config(vocab_size=300, n_positions=512, n_embd=width, n_layer=2, n_head=width // 64)
+    cfg = Gpt2Config(vocab_size=300, n_positions=1100 if n > 512 else 512, n_embd=width, n_layer=2, n_head=width // 64)
     store = {"f32": _lib.PG_STORE_F32, "bf16": _lib.PG_STORE_BF16, "int8": _lib.PG_STORE_INT8}[storage]
     model = Gpt2Model.new(cfg, synth.random_weights(cfg, 0x5EED0A00, perturb=True), Gpt2HipConfig(weight_storage=store))
     ids = [int(t) for t in synth.token_ids(n, 0x70C00A00 + n, cfg.vocab_size)]
@@ -174,7 +177,8 @@ def test_a_set_bound_of_the_bf16_cores_holds_for_the_cut_form():
             np.testing.assert_array_equal(logits(rows, bound), on_f32_cores)
 
 
-@pytest.mark.parametrize("storage,batch,n", [("f32", 33, 3), ("f32", 48, 20), ("bf16", 40, 7), ("int8", 17, 5), ("int8", 31, 9), ("int8", 65, 4)])
+@pytest.mark.parametrize("storage,batch,n", [("f32", 33, 3), ("f32", 48, 20), ("bf16", 40, 7), ("int8", 17, 5), ("int8", 31, 9), ("int8", 65, 4),
+                                             ("f32", 128, 3), ("f32", 129, 3), ("f32", 130, 2)])
 def test_batched_steps(storage, batch, n):
     cfg = Gpt2Config(vocab_size=300, n_positions=600, n_embd=768, n_layer=2, n_head=12)
     store = {"f32": _lib.PG_STORE_F32, "bf16": _lib.PG_STORE_BF16, "int8": _lib.PG_STORE_INT8}[storage]
