@@ -5,6 +5,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
+import attn_parts
 from helpers import DeviceArray
 from puppygrad_amd import _lib
 
@@ -66,6 +67,16 @@ def check(qkv, heads, shape):
 def test_shapes_at_their_edges(shape, rows, heads, n):
     rng = np.random.default_rng([rows, heads, n])
     check(rng.standard_normal((n, rows, 192 * heads)).astype(np.float32), heads, shape)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("which", ["scores", "weights"])
+def test_every_product_of_the_parts_counts(shape, which):
+    """A product of the parts left out is twice the bound and more (test_attn_parts.py)."""
+    qkv = attn_parts.operands(which)
+    got, size = attention_rows_dev(qkv, 1, shape)[2][0, attn_parts.FIRST:], attn_parts.attention(qkv)[1]
+    err = np.abs(got - attn_parts.exact(qkv)) / (attn_parts.BOUND[which] * size)
+    assert (err <= 1.0).all(), f"{err.max():.2f} of the bound"
 
 
 @pytest.mark.parametrize("shape", SHAPES)
