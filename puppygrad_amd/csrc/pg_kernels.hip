@@ -818,8 +818,10 @@ __device__ __forceinline__ Best better(Best a, Best b) {
   if (b.v > a.v || (b.v == a.v && b.i < a.i)) return b;
   return a;
 }
-// U: loads in flight per thread.  One block pulls a row in at the pace of its round trips to memory: 50257 logits, 8 at a
-// time 7.1 us, all 50 at once 4.9 us (a launch by itself is 2).  out may be pinned host memory.
+// U: loads in flight per thread.  One block pulls a row in at the pace of its round trips to memory (50257 values, 8 loads at
+// a time 7.1 us, all at once 4.7; a launch by itself is 2), so a row of up to 65536 is asked for at once (16385 3.2 us, 65536
+// 5.3), a longer one in as few turns of equal length (120000 7.9); the instance is the one of fewer than four loads past the
+// row's end.  out may be pinned host memory.
 template <int U>
 __global__ __launch_bounds__(1024) void k_argmax(const float* v, int n, uint32_t* out) {
   v += (size_t)blockIdx.x * n;  // one block per row
@@ -1553,10 +1555,17 @@ hipError_t launch_topk_select(const float* logits, int V, const uint32_t* pen_id
   return hipGetLastError();
 }
 
-hipError_t launch_argmax(const float* v, int n, uint32_t* out, hipStream_t s, int rows) {
-  if (n > 16384) hipLaunchKernelGGL(k_argmax<50>, dim3(rows), dim3(1024), 0, s, v, n, out);
-  else hipLaunchKernelGGL(k_argmax<8>, dim3(rows), dim3(1024), 0, s, v, n, out);
+// each: loads per thread and turn
+template <int U>
+static hipError_t launch_argmax_of(long each, const float* v, int n, uint32_t* out, hipStream_t s, int rows) {
+  if constexpr (U < 64)
+    if (each > U) return launch_argmax_of<U + 4>(each, v, n, out, s, rows);
+  hipLaunchKernelGGL(k_argmax<U>, dim3(rows), dim3(1024), 0, s, v, n, out);
   return hipGetLastError();
+}
+hipError_t launch_argmax(const float* v, int n, uint32_t* out, hipStream_t s, int rows) {
+  const int turns = (int)std::max(1L, ((long)n + 65535) / 65536);
+  return launch_argmax_of<4>(((long)n + 1024L * turns - 1) / (1024L * turns), v, n, out, s, rows);
 }
 
 hipError_t launch_layer_norm(float* x, int rows, int cols, const float* g, const float* b,
