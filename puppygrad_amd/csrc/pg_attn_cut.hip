@@ -289,8 +289,8 @@ void start(const float* qkv, int T, int C, int H, int P, float* kcache, float* v
 }
 }  // namespace
 
-// Which block shape is the fastest, or 0 where k_attn_prefill64 is: by the blocks that there are, us of k_attn_prefill64
-// and of the shape that is taken.
+// Which block shape is the fastest, or 0 where k_attn_prefill64 is: by the blocks that there are to a CU, us of k_attn_prefill64
+// and of the shape that is taken, on 256 CUs (whose blocks the lines below count; a part of the chip has its share).
 //  - up to 32 positions it is one tile a sequence: equal or slower here (32 x 20, 25 heads 13.5 / 15.3);
 //  - 128 queries a block where that fills the chip: 32 x 200, 25 heads 131 / 80; 32 x 512, 25 heads 490 / 265.  64 for sequences
 //    that short (32 x 60, 25 heads 30.7 / 22.4), and where the longer blocks of fewer queries even out the CUs (4 x 700, 20
@@ -298,9 +298,10 @@ void start(const float* qkv, int T, int C, int H, int P, float* kcache, float* v
 //  - eight wavefronts a block, the keys in two or four shares, with fewer blocks: 16 x 100, 12 heads 19.9 / 14.6; 1000, 25
 //    heads 62 / 43; 1024, 20 heads 49 / 39; 4 x 200, 12 heads 17.3 / 12.7;
 //  - fewer still: k_attn_prefill64's blocks of 32 queries (1024, 12 heads 31 / 35; 200, 20 heads 10.4 / 11.6).
-int attn_cut_shape(int T, int H, int nseq) {
+int attn_cut_shape(int T, int H, int nseq, int num_cus) {
   if (T <= 32) return 0;
-  const long nb128 = (long)H * nseq * ((T + 127) / 128), nb64 = (long)H * nseq * ((T + 63) / 64);
+  auto blocks = [&](int queries) { return (double)H * nseq * ((T + queries - 1) / queries) * 256.0 / num_cus; };
+  const double nb128 = blocks(128), nb64 = blocks(64);
   if (T <= 64) return nb64 >= 192 ? 22 : 0;
   if (nb128 >= 320) return T > 256 && nb64 <= (T <= 512 ? 2800 : 1024) ? 22 : 41;
   if (nb128 >= 192) return T <= 400 ? 42 : 24;

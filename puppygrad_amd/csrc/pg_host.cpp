@@ -592,7 +592,7 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
     PG_HIP(gemm(XN.p, C, w.c_attn_w, w.c_attn_b, QKV.p, 3 * C, 3 * C, C, pgk::GEMM_BIAS, nullptr, nullptr, cut));
     PG_MARK(kQkv);
     PG_HIP(pgk::launch_attn_prefill(QKV.p, Ts, C, H, hd, P, c->k_panel(l, b), c->v_panel(l, b),
-                                    ATT.p, SCR.p, s, (int)nb, g.H * g.P * g.hd(),
+                                    ATT.p, SCR.p, m->num_cus, s, (int)nb, g.H * g.P * g.hd(),
                                     cut ? pgk::FORM_CUT : pgk::FORM_ROWS, c->drawn));
     PG_MARK(kAttention);
     PG_HIP(gemm(ATT.p, C, w.c_proj_w, w.c_proj_b, X.p, C, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b, cut));

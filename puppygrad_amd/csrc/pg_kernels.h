@@ -312,12 +312,12 @@ hipError_t launch_gemm_grouped(const GemmArgs& a, int epilogue, int tile_rows, c
 // nseq sequences of T positions each, one after the other in qkv / out; sequence i's panels
 // lie kv_stride floats after sequence i - 1's.  f32_cores: on the f32 matrix cores, however many blocks there are.
 hipError_t launch_attn_prefill(const float* qkv, int T, int C, int H, int head_dim, int P,
-                               float* kcache, float* vcache, float* out, float* scratch,
+                               float* kcache, float* vcache, float* out, float* scratch, int num_cus,
                                hipStream_t s, int nseq = 1, size_t kv_stride = 0, int out_form = 0,
                                bool f32_cores = false);
 // The same with both products on the bf16 matrix cores (pg_attn_cut.hip), head_dim 64, in blocks of one of these shapes:
 // 41, 22, 42, 24 (groups of 32 queries, groups of keys).  attn_cut_shape: the one to take, 0: none.
-int attn_cut_shape(int T, int H, int nseq);
+int attn_cut_shape(int T, int H, int nseq, int num_cus);
 hipError_t launch_attn_prefill_cut(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, float* out,
                                    hipStream_t s, int nseq, size_t kv_stride, int out_form, int shape);
 // rows rows; row t is position t % period of its sequence (wpe may be null)

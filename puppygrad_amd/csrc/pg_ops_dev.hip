@@ -433,6 +433,11 @@ int32_t pg_testing_takes_cut(int32_t rows, int32_t width, int32_t inner, int32_t
   return pgk::gemm_takes_cut(rows, width, inner, storage == PG_STORE_BF16, storage == PG_STORE_INT8, f32_min_rows, num_cus);
 }
 
+// attn_cut_shape
+int32_t pg_testing_attn_shape(int32_t rows, int32_t heads, int32_t sequences, int32_t num_cus) {
+  return pgk::attn_cut_shape(rows, heads, sequences, num_cus);
+}
+
 // Attention of `sequences` prompts of `rows` tokens each, head size 64, keys and values to panels [sequences][heads][rows][64]:
 // in blocks of the given shape of pg_attn_cut.hip (0: as the planner has it).
 pg_status pg_testing_attention_rows_dev(int32_t device, void* stream, const float* qkv, uint64_t rows, uint64_t heads,
@@ -445,10 +450,12 @@ pg_status pg_testing_attention_rows_dev(int32_t device, void* stream, const floa
   const int T = (int)rows, H = (int)heads, C = 64 * H;
   const size_t stride = (size_t)H * T * 64;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  int cus = 0;
+  PG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   if (shape > 0)
     PG_HIP(pgk::launch_attn_prefill_cut(qkv, T, C, H, T, keys, values, out, st, (int)sequences, stride, pgk::FORM_ROWS, shape));
   else
-    PG_HIP(pgk::launch_attn_prefill(qkv, T, C, H, 64, T, keys, values, out, nullptr, st, (int)sequences, stride));
+    PG_HIP(pgk::launch_attn_prefill(qkv, T, C, H, 64, T, keys, values, out, nullptr, cus, st, (int)sequences, stride));
   return PG_OK;
 }
 

@@ -1784,11 +1784,11 @@ hipError_t launch_gemm_form(const GemmArgs& a, int epi, int num_cus, hipStream_t
 }  // namespace
 
 hipError_t launch_attn_prefill(const float* qkv, int T, int C, int H, int head_dim, int P,
-                               float* kcache, float* vcache, float* out, float* scratch,
+                               float* kcache, float* vcache, float* out, float* scratch, int num_cus,
                                hipStream_t s, int nseq, size_t kv_stride, int out_form, bool f32_cores) {
   if (nseq < 1 || nseq > 65535 || out_form == FORM_PACKED32 || (out_form && head_dim != 64)) return hipErrorInvalidValue;
   if (head_dim == 64) {
-    if (const int shape = f32_cores ? 0 : attn_cut_shape(T, H, nseq))
+    if (const int shape = f32_cores ? 0 : attn_cut_shape(T, H, nseq, num_cus))
       return launch_attn_prefill_cut(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, out_form, shape);
     const int qblocks = (T + 31) / 32;
     // Eight wavefronts share a query block's key tiles.  Several sequences of up to 512 tokens
