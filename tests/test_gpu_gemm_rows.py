@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from helpers import DeviceArray, as_bf16
+from test_cut_form import LAST, takes
 from puppygrad_amd import Gpt2Config, Gpt2HipConfig, Gpt2Model, _lib, synth
 
 pytestmark = pytest.mark.gpu
@@ -142,6 +143,7 @@ def test_infinite_weights_and_weights_past_bf16():
 def test_prompts(storage, width, n):
     cfg = Gpt2Config(vocab_size=300, n_positions=1100 if n > 512 else 512, n_embd=width, n_layer=2, n_head=width // 64)
     store = {"f32": _lib.PG_STORE_F32, "bf16": _lib.PG_STORE_BF16, "int8": _lib.PG_STORE_INT8}[storage]
+    assert takes(n, width, store) == (n <= LAST[store][width])
     model = Gpt2Model.new(cfg, synth.random_weights(cfg, 0x5EED0A00, perturb=True), Gpt2HipConfig(weight_storage=store))
     ids = [int(t) for t in synth.token_ids(n, 0x70C00A00 + n, cfg.vocab_size)]
     cache, other = model.new_kv_cache(), model.new_kv_cache()
