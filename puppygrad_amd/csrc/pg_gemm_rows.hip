@@ -223,19 +223,18 @@ hipError_t launch_wt(const GemmArgs& a, int epi, const CutRowsPlan& p, hipStream
     default: return hipErrorInvalidValue;
   }
 }
-// Time of a product in microseconds, fitted over 24860 plans of the four GPT-2 widths' projections, W from HBM, at rows on
-// both sides of where the form ends (f32 rows to 1100, bf16 to 700, int8 to 1200; plans near the best weigh most): the
-// plan of least predicted time is 1.9 % slower than the best measured one in the mean for f32 rows, 1.6 bf16, 1.1 int8 (20 %
-// at most; constants from 24 to 320 rows alone: 2.8, 2.7 and 2.0 %, 47 % at most).  `most`: a block of 64 x 64, whose
-// registers spill.  `reduce`: the launch that adds the parts; `norm`, `norm_values`: that of a norm by itself, and per
-// 10^6 values.
+// What a plan of a product costs, in microseconds but for a constant, chosen so that the plan of least cost is close to the
+// best measured one, over 24860 plans of the four GPT-2 widths' projections, W from HBM, at rows on both sides of where
+// the form ends.  At other rows, and at widths 384, 512 and 2048 too (35054 plans, which the int8 constants have seen), a
+// layer's four products are 1.0 % slower than the best plans in the mean for f32 rows, 1.3 bf16, 0.6 int8 (9 % at most;
+// constants from times at 24 to 320 rows: 1.9, 2.7 and 2.5 %, 12 % at most).  `most`: a block of 64 x 64, whose registers spill.  `reduce`: the launch that adds the parts; `norm`,
+// `norm_values`: that of a norm by itself, and per 10^6 values.
 struct RowsPace {
-  float start, round, step, mt, ng, both, most, fill, part, reduce, norm, norm_values;
+  float round, step, mt, ng, both, most, fill, part, reduce, norm, norm_values;
 };
-constexpr RowsPace kRowsPace[3] = {
-    {3.025f, 1.212f, -0.950f, 0.258f, 0.848f, -0.080f, 0.0f, 0.164f, 2.563f, 2.957f, 2.585f, 4.907f},
-    {2.364f, 1.014f, -0.375f, 0.131f, 0.328f, 0.003f, 0.443f, 0.106f, 2.572f, 3.491f, 3.242f, 5.680f},
-    {2.593f, 1.357f, -0.184f, 0.082f, 0.073f, 0.063f, 0.113f, 0.074f, 2.538f, 3.331f, 2.816f, 7.044f}};
+constexpr RowsPace kRowsPace[3] = {{11.237f, -0.786f, 0.179f, 0.891f, -0.013f, 0.0f, 0.203f, 3.578f, 2.545f, 3.175f, 0.731f},
+                                   {0.357f, -0.208f, 0.129f, 0.086f, 0.039f, 0.307f, 0.117f, 4.787f, 2.433f, 2.971f, 3.534f},
+                                   {0.039f, -0.064f, 0.170f, -0.025f, 0.054f, -0.033f, 0.022f, 4.668f, 3.294f, 2.652f, 7.051f}};
 
 }  // namespace
 
@@ -243,17 +242,17 @@ constexpr RowsPace kRowsPace[3] = {
 // first).  A step in this form's time is a round of blocks (64 rows by 48 rows of W, 64 for int8 rows) over the CUs, so the
 // line is a number of rounds of the widest product, past which the tiles of pg_gemm_cut.hip, which read an input row once
 // for 128 columns, are the faster ones:
-//  - f32 and bf16 rows, two rounds.  f32 at width 1600: 192 rows 7.54 / 6.76, 193 rows 7.80 / 8.31; 1280: 256 rows 4.82 /
-//    4.54, 257 rows 5.38 / 5.59; 1024: 320 rows 2.99 / 2.64, 400 rows 3.37 / 3.31, 600 rows 4.05 / 4.20; 33 rows, 1600: 4.02 / 3.43.
-//    bf16 at 1600: 131 rows 4.96 / 4.51, 192 rows 5.23 / 5.23, 193 rows 5.74 / 6.37; 1280: 256 rows 3.89 / 3.60, 257 rows
-//    3.99 / 4.23; 1024: 320 rows 2.41 / 2.15, 400 rows 2.62 / 2.60; 768: 512 rows 1.09 / 1.03, 560 rows 1.19 / 1.17, 800 rows
-//    1.18 / 1.36.
+//  - f32 and bf16 rows, two rounds.  f32 at width 1600: 192 rows 7.52 / 6.58, 193 rows 7.79 / 8.15; 1280: 256 rows 4.83 /
+//    4.59, 300 rows 5.41 / 5.53; 1024: 320 rows 2.98 / 2.60, 400 rows 3.29 / 3.22, 600 rows 3.93 / 4.09; 33 rows, 1600: 4.03 / 3.43.
+//    bf16 at 1600: 131 rows 5.00 / 4.49, 192 rows 5.28 / 5.22, 193 rows 5.76 / 6.36; 1280: 256 rows 3.90 / 3.65, 257 rows
+//    3.99 / 4.02; 1024: 320 rows 2.44 / 2.15, 400 rows 2.57 / 2.54; 768: 512 rows 1.08 / 1.01, 560 rows 1.17 / 1.17, 800 rows
+//    1.16 / 1.34.
 //  - f32 rows up to width 768, where the tiles leave a third of the CUs without one: four rounds and 1024 rows.  768: 512 rows
-//    1.46 / 1.29, 700 rows 1.76 / 1.70, 1024 rows 2.11 / 2.03 (8 x 128 1.90 / 1.80), 1026 rows 2.09 / 2.36; 512: 600 rows 1.12 /
-//    1.04, 1000 rows 1.41 / 1.39, 1200 rows 1.47 / 1.57.
-//  - int8 rows, three rounds.  1600: 448 rows 9.24 / 8.40, 449 rows 9.69 / 9.88; 1280: 576 rows 6.37 / 5.65, 577 rows 6.54 /
-//    6.53; 1024: 768 rows 3.89 / 3.74, 769 rows 4.08 / 4.00; 768: 1024 rows 1.73 / 1.61, 1026 rows 1.69 / 1.72.  Up to 32 rows,
-//    a step of 20 at 1280 1.89 / 1.85, of 32 2.13 / 2.15, of 32 at 768 0.60 / 0.57.
+//    1.41 / 1.26, 700 rows 1.71 / 1.65, 1024 rows 2.01 / 1.93 (8 x 128 1.82 / 1.73), 1026 rows 2.03 / 2.27; 512: 600 rows 1.12 /
+//    1.06, 1000 rows 1.39 / 1.38, 1200 rows 1.47 / 1.57.
+//  - int8 rows, three rounds.  1600: 448 rows 9.28 / 8.34, 449 rows 9.71 / 9.63, 500 rows 9.96 / 10.2; 1280: 576 rows 6.41 / 5.61,
+//    577 rows 6.58 / 6.36; 1024: 768 rows 3.86 / 3.63, 769 rows 4.02 / 3.92; 768: 1024 rows 1.72 / 1.61, 1026 rows 1.68 / 1.71.  Up to
+//    32 rows, a step of 20 at 1280 1.89 / 1.85, of 32 2.13 / 2.15, of 32 at 768 0.60 / 0.57.
 bool gemm_takes_cut(int M, int K, int N, int w_bf16, int w_int8, int f32_min_rows, int num_cus) {
   if (K < 256 || K % 32 != 0 || N % 32 != 0) return false;  // (narrower: no step for some of the eight wavefronts)
   const int cols = w_int8 ? 64 : 48;  // of a full block, 64 rows
@@ -278,7 +277,7 @@ bool gemm_cut_rows_plan(const GemmArgs& a, int num_cus, CutRowsPlan* plan) {
   const RowsPace& p = kRowsPace[wt];
   // (a part: a step at least for each wavefront)
   const int most = a.ws && !a.c_cut ? (int)std::min<size_t>(std::min(8, steps / 8), a.ws_floats / ((size_t)a.M * a.N)) : 1;
-  float best = 0.0f;
+  float best = -1.0f;
   for (int parts = 1; parts <= std::max(1, most); ++parts)
     for (int rows = 8; rows <= 64; rows += 8) {
       const int ng = (rows + 15) / 16;
@@ -286,10 +285,10 @@ bool gemm_cut_rows_plan(const GemmArgs& a, int num_cus, CutRowsPlan* plan) {
       const long blocks = (long)((a.N + rows - 1) / rows) * m_blocks * parts;
       const float turns = (float)((blocks + num_cus - 1) / num_cus);
       const float rounds = (float)(((steps + parts - 1) / parts + 7) / 8);
-      const float us = p.start + turns * (p.round + rounds * (p.step + p.mt * mt + p.ng * ng + p.both * mt * ng + (mt * ng == 16 ? p.most : 0.0f))) +
+      const float us = turns * (p.round + rounds * (p.step + p.mt * mt + p.ng * ng + p.both * mt * ng + (mt * ng == 16 ? p.most : 0.0f))) +
                        p.fill * (float)blocks / (float)num_cus * rounds * mt +
                        (parts > 1 ? p.reduce + p.part * parts * mn : a.ln_out ? p.norm + p.norm_values * mn : 0.0f);
-      if (best == 0.0f || us < best) {
+      if (best < 0.0f || us < best) {
         best = us;
         *plan = {mt, ng, rows, parts};
       }
