@@ -436,7 +436,7 @@ def bf16_prefill_roofline(flops, gemm_flops, sec, traffic=None, traffic_source=N
     r = {"bound": "mfma", "achieved": round(achieved, 2), "peak": BF16_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
          "frac": round(achieved / BF16_MFMA_PEAK_TFLOPS, 4), "traffic": traffic, "passes": 3,
          "executed": round((2 * gemm_flops + flops) / sec / 1e12, 2),
-         "kernel": "whole prefill (k_gemm_cut on the bf16 matrix cores, k_attn_prefill64 and lm_head in f32)",
+         "kernel": "whole prefill (k_gemm_cut and k_attn_prefill_cut on the bf16 matrix cores, lm_head in f32)",
          "algorithmic_flops_per_step": int(flops), "gemm_flops_per_step": int(gemm_flops)}
     if traffic_source:
         r["traffic_source"] = traffic_source
