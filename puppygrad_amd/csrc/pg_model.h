@@ -155,8 +155,8 @@ struct pg_kv_cache {
   float *qkv_b = nullptr, *xn_b = nullptr, *att_b = nullptr;  // batched step: [B][3C], [B][C], [B][C]
   // A stream's ids are drawn from what this cache holds: a prompt's products, attention and experts stay with the kernels
   // whose sums a seed's ids were drawn from so far.  Over a whole row the draw walks 50257 ids by value, neighbours 10^-5
-  // apart, and logits moved by their last bits (another kernel's order of additions: 5 10^-7) change two streams of 80 in
-  // five from some id on.  Decode steps have one kernel either way.
+  // apart, and logits moved by their last bits (another kernel's order of additions: 5 10^-7) changed two in five streams
+  // of 80 ids from some id on.  Decode steps have one kernel either way.
   bool drawn = false;
   bool cut_form = false;  // batched step: xn_b, att_b and hbuf have room for the cut form (pgk::FORM_CUT)
   bool pack32 = false;  // batched step: xn_b, att_b and hbuf are packed (pgk::packed32_index)

@@ -3,8 +3,8 @@
 // times); moves within a row of 16 lanes ride on the addition itself, and rows are brought together by a swap.  All lanes
 // have to be active, and all get the result.
 // The order of the additions is that of __shfl_xor by 32, 16, 8, 4, 2 and 1, to the last bit: a stream that is drawn
-// over a whole row walks 50257 ids by value, and a logit that moves by its last bit makes it take another id, and other
-// ids from there on, about once in five streams of 80.
+// over a whole row walks 50257 ids by value, neighbours 10^-5 apart, and where a logit's last bit swaps two of them it
+// takes another id, and other ids from there on.
 #pragma once
 #include <hip/hip_runtime.h>
 
