@@ -104,7 +104,8 @@ typedef struct pg_hip_options {
                                        into about this many work items per CU (default 3) */
   uint32_t gemm_b9_min_rows;        /* f32 weights: products over at least this many input rows
                                        run on the bf16 matrix cores with both operands cut into
-                                       three bf16 parts where the planner finds enough tiles
+                                       three bf16 parts, or on the f16 ones in two f16 parts,
+                                       where the planner finds enough tiles
                                        (0xffffffff: never).  Default: 65, and 33 to 64 rows
                                        where activations are better kept cut; set, 65 too, it
                                        is the bound for both.  65 to 128 rows are not kept cut

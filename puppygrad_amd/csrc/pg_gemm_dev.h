@@ -33,6 +33,22 @@ hipError_t launch_gemm_cut_rows(const GemmArgs& a, int epi, const CutRowsPlan& p
 // (bf16 rows; tiles of tile_rows = 64 or 128 rows)
 hipError_t launch_gemm_cut_grouped(const GemmArgs& a, int epi, int tile_rows, hipStream_t s);
 
+// A product with activations and W in half form (pg_gemm_half.hip): the tile, or blocks of 16 mt input rows and `rows` rows of W
+// (HALF_ROWS), and parts of K (1: whole tiles; otherwise raw partial tiles to GemmArgs::ws).
+// (HALF_128x128_8: by eight wavefronts)
+enum HalfTile : int { HALF_64x128 = 0, HALF_128x128 = 1, HALF_128x128_8 = 2, HALF_128x256 = 3, HALF_ROWS = 4 };
+struct HalfPlan {
+  int tile, parts, mt, rows;
+};
+bool gemm_half_takes(const GemmArgs& a, int epi);
+HalfPlan gemm_half_plan(const GemmArgs& a, int epi, int num_cus);
+hipError_t launch_gemm_half_plan(const GemmArgs& a, int epi, const HalfPlan& p, hipStream_t s);
+// Reduction and norm behind it, and all of it.
+hipError_t finish_gemm_half(const GemmArgs& a, int epi, const HalfPlan& p, hipStream_t s);
+hipError_t launch_gemm_half(const GemmArgs& a, int epi, int num_cus, hipStream_t s);
+// Adds the parts of a cut K (GemmArgs::ws) with bias and epilogue; *ln_done: and the norm.
+hipError_t launch_splitk_reduce(const GemmArgs& a, int epi, int parts, hipStream_t s, bool* ln_done);
+
 namespace {
 
 typedef float f16v __attribute__((ext_vector_type(16)));

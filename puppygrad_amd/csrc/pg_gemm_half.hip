@@ -1,0 +1,789 @@
+// Products of some tens to many thousands of rows with activations in half form (FORM_HALF; pg_half.h) and W in half
+// form beside its stored rows (transposed_dense_projection_into, src/models/cpu.rs:58-75).
+//
+// f32 inputs and sums on the f16 matrix cores.  An input value times a power of two is two f16 numbers, hi and lo, an
+// f32 weight too (its row times a power of two of its own); a bf16 or int8 weight is one f16 number as it is.  So
+// x w = hi w + lo w, two v_mfma_f32_32x32x16_f16 with exact products, where three bf16 parts take three instructions
+// (pg_gemm_cut.hip); for f32 rows three, hi hi + hi lo + lo hi, where they take six.
+//
+// What is lost: two f16 hold 23 of a value's 24 significant bits, all 24 of three values in four, so that a product is off by
+// 6 10^-8 in the mean, of either sign, and lo lo is 2^-24 and less.  Over a sum of K products that is 7 10^-8 of the result
+// (bf16 and int8 rows 4 10^-8), below what its roundings cost: with one f32 sum over K = 1600 2.7 10^-7.  Those are made
+// fewer for it: a chain of matrix instructions ends after CH stages, 64 to 128 columns, and is added to a total, and wherever
+// there are registers for it the small products are a chain of their own (in one with the others they are cut downward, and
+// the error has a mean: a model's logits were off by up to 1.4 times as much).  Error against f64 (values N(0, 1) by N(0, 0.02), of
+// the result's norm, 512 rows), one part of K, before -> now: 1280 x 1280 f32 rows 2.1 10^-7 -> 1.3, K = 5120 4.5 -> 1.6 (64 x
+// 64 a wavefront: 1.4, 2.1); bf16 rows 2.1 -> 1.1, 4.5 -> 1.5; 128 x 256 tiles, one chain, 16384 x 1600 x 1600 4.3 -> 3.6.
+// Logits of prompts of 450 to 1000 tokens, all sizes: 0.65 to 0.85 of what they were off by.
+//
+// The range of f16: values are scaled so that they cannot be past 2^15 whatever the inputs are (half_bounds: what a
+// LayerNorm, a projection of one, an average of such or a GELU of such can reach at most), and below 2^-2 a value is right
+// to 2^-25, 2^-40 of that bound.  f16 subnormals count in these instructions.
+//
+// How operands travel: a producer cuts a value once, in its epilogue; here all are operands as they lie, whole KB by
+// global_load_lds without registers, LDS reads free of conflicts without a permutation, no vector instruction in the loop
+// but a chain's end.  1000 x 4800 x 1600 f32 rows 102 us and a reduction of 11 -> 52, 1000 x 6400 x 1600 113 -> 58, 8192 x
+// 4800 x 1600 606 -> 337; bf16 16384 x 4800 x 1600 610 -> 436, 16384 x 1600 x 6400 880 -> 606 (1125 TFLOP/s of matrix
+// instructions; a plain library product reaches 1354).
+#include "pg_gemm_dev.h"
+#include "pg_half.h"
+#include "pg_wave.h"
+
+#include <type_traits>
+
+namespace pgk {
+
+namespace {
+
+typedef __attribute__((address_space(3))) char* lds_ptr;
+
+// 16 bytes per lane from base + byte_off (per lane) to lds + 16 lane (LDS address, wavefront-uniform); vm_wait is the
+// wait that belongs to it (inline assembly, which the compiler's own count of loads does not know).
+__device__ __forceinline__ void lds_dma16(const void* base, unsigned byte_off, unsigned lds) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2"
+      :
+      : "s"(lds), "v"(byte_off), "s"(base)
+      : "memory", "m0");
+}
+// At most N loads of the wavefront in flight.
+template <int N>
+__device__ __forceinline__ void vm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// WM x WN wavefronts, each on MB x NB blocks of 32 x 32.  The operands are turned round: lane (l, half) of the first holds
+// columns 8 half .. 8 half + 7 of row l of W, of the second those of input row l, so that the result's lane is a row
+// of C and its values four by four neighbouring columns.  PW: parts of a weight (2: f32 rows).  K runs in stages of KT
+// columns in NA buffers, a stage in steps of 16 whose operands are read during the step before.  One barrier per stage, in front of the step that reads the next stage: by then the wavefront has
+// waited for its own share of that stage, and has read the stage before it to the end, whose buffer is free for the stage that
+// is asked for next.  CH: stages in a chain of matrix instructions (0: one chain).  TWO: the small products of a chain have a
+// sum of their own.  SPLIT: the stages are cut into gridDim.y parts, raw partial tiles go to a.ws[part][M][N].  OCC:
+// wavefronts per SIMD that the registers are kept for.
+template <int WM, int WN, int MB, int NB, int PW, int EPI, int SPLIT, int OCC, int NA, int KT, int CH, bool TWO>
+__global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
+  constexpr int NW = WM * WN, BM = 32 * MB * WM, BN = 32 * NB * WN, NO = KT / 8, NS = KT / 16;
+  constexpr int IA = NO * 2 * BM / 64 / NW, IB = NO * PW * BN / 64 / NW;
+  constexpr int UN = CH ? CH : NA;
+  static_assert(UN % NA == 0 && (NS == 2 || UN % 2 == 0) && UN <= 8 && (CH != 0 || !TWO));
+  static_assert(NO * 2 * BM % (64 * NW) == 0 && NO * PW * BN % (64 * NW) == 0 && BM % 64 == 0 && BN % 64 == 0);
+  __shared__ u4v As[NA][NO * 2 * BM];
+  __shared__ u4v Bs[NA][NO * PW * BN];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int half = lane >> 5, l32 = lane & 31;
+  const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
+  int tile;
+  {
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int per_xcd = ((int)gridDim.x + 7) >> 3;
+    tile = xcd * per_xcd + slot;
+  }
+  if (tile >= tiles_m * tiles_n) return;
+  int tm, tn;
+  tile_coords(tile, tiles_m, tiles_n, a.band_rows, &tm, &tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int mp = cut_rows(a.M);
+
+  const int T_all = a.K / KT;
+  const int kt0 = SPLIT ? (int)(((long)blockIdx.y * T_all) / gridDim.y) : 0;
+  const int kt1 = SPLIT ? (int)(((long)(blockIdx.y + 1) * T_all) / gridDim.y) : T_all;
+  const int T = kt1 - kt0;
+
+  unsigned aoff[IA], boff[IB];
+#pragma unroll
+  for (int i = 0; i < IA; ++i) {
+    const int at = (wave * IA + i) * 64, plane = at / BM, row = at % BM + lane;
+    aoff[i] = ((unsigned)plane * (unsigned)mp + (unsigned)min(m0 + row, a.M - 1)) * 16u;
+  }
+#pragma unroll
+  for (int i = 0; i < IB; ++i) {
+    const int at = (wave * IB + i) * 64, plane = at / BN, row = at % BN + lane;
+    boff[i] = ((unsigned)plane * (unsigned)a.N + (unsigned)min(n0 + row, a.N - 1)) * 16u;
+  }
+  const size_t astage = (size_t)NO * 2 * mp * 16, bstage = (size_t)NO * PW * a.N * 16;
+  const char* Ab = reinterpret_cast<const char*>(a.A) + kt0 * astage;
+  const char* Wb = static_cast<const char*>(a.w_half) + kt0 * bstage;
+  const unsigned as_lds = (unsigned)(size_t)(lds_ptr)(void*)&As[0][0], bs_lds = (unsigned)(size_t)(lds_ptr)(void*)&Bs[0][0];
+  auto dma = [&](int t, int buf) __attribute__((always_inline)) {
+    const size_t k = (size_t)min(t, T - 1);
+#pragma unroll
+    for (int i = 0; i < IA; ++i) lds_dma16(Ab + k * astage, aoff[i], as_lds + (unsigned)(buf * NO * 2 * BM * 16 + (wave * IA + i) * 1024));
+#pragma unroll
+    for (int i = 0; i < IB; ++i) lds_dma16(Wb + k * bstage, boff[i], bs_lds + (unsigned)(buf * NO * PW * BN * 16 + (wave * IB + i) * 1024));
+  };
+
+  f16v acc[MB][NB], tot[CH ? MB : 1][CH ? NB : 1], low[TWO ? MB : 1][TWO ? NB : 1];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        acc[i][j][v] = 0.0f;
+        if constexpr (CH != 0) tot[i][j][v] = 0.0f;
+      }
+  struct Ops { u4v x[MB][2], w[NB][PW]; };
+  auto read = [&](int buf, int s, Ops& o) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 1; p >= 0; --p) {  // in the order in which the products need them
+#pragma unroll
+      for (int i = 0; i < MB; ++i) o.x[i][p] = As[buf][((2 * s + half) * 2 + p) * BM + (wm * MB + i) * 32 + l32];
+      const int q = 1 - p;
+      if (q < PW) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) o.w[j][q] = Bs[buf][((2 * s + half) * PW + q) * BN + (wn * NB + j) * 32 + l32];
+      }
+    }
+  };
+  // products of parts (input, weight), small ones first
+  constexpr int NP = PW + 1;
+  auto step = [&](auto first, const Ops& cur, Ops& nxt, int buf, int s) __attribute__((always_inline)) {
+    constexpr bool fresh = CH != 0 && decltype(first)::value;
+    read(buf, s, nxt);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+          const int px = p == 0 ? 1 : 0, pw = p == 1 && PW == 2 ? 1 : 0;
+          f16v& sum = TWO && p < NP - 1 ? low[TWO ? i : 0][TWO ? j : 0] : acc[i][j];
+          if (fresh && (p == 0 || (TWO && p == NP - 1))) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) sum[v] = 0.0f;
+          }
+          sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, cur.w[j][pw]), __builtin_bit_cast(h8v, cur.x[i][px]), sum, 0, 0, 0);
+        }
+    }
+  };
+  auto interleave = [&] __attribute__((always_inline)) {
+    constexpr int NM = NP * MB * NB, NR = 2 * MB + PW * NB, PER = (NR + NM - 1) / NM;
+#pragma unroll
+    for (int g = 0; g < NM; ++g) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if (g * PER < NR) __builtin_amdgcn_sched_group_barrier(0x100, PER, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  if (T > 0) {
+    Ops pa, pb;
+#pragma unroll
+    for (int t = 0; t < NA; ++t) dma(t, t);
+    vm_wait<(NA - 1) * (IA + IB)>();
+    asm volatile("s_barrier" ::: "memory");
+    read(0, 0, pa);
+    auto stage = [&](auto u, int t, Ops& p0, Ops& p1) __attribute__((always_inline)) {
+      constexpr int U = decltype(u)::value, ab = U % NA, nb = (U + 1) % NA;
+      const std::integral_constant<bool, U == 0> head;
+      const std::false_type rest;
+      if constexpr (NS == 2) {
+        step(head, p0, p1, ab, 1);
+        interleave();
+      }
+      vm_wait<(NA - 2) * (IA + IB)>();
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      dma(t + NA, ab);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (NS == 2) {
+        step(rest, p1, p0, nb, 0);
+        interleave();
+      } else {
+        step(head, p0, p1, nb, 0);
+        interleave();
+      }
+    };
+    for (int t = 0; t < T; t += UN) {
+      auto at = [&](auto u) __attribute__((always_inline)) {
+        constexpr int U = decltype(u)::value;
+        if (t + U < T) {
+          if constexpr (NS == 2 || U % 2 == 0) stage(u, t + U, pa, pb);
+          else stage(u, t + U, pb, pa);
+        }
+      };
+      at(std::integral_constant<int, 0>());
+      if constexpr (UN > 1) at(std::integral_constant<int, 1 % UN>());
+      if constexpr (UN > 2) at(std::integral_constant<int, 2 % UN>());
+      if constexpr (UN > 3) at(std::integral_constant<int, 3 % UN>());
+      if constexpr (UN > 4) at(std::integral_constant<int, 4 % UN>());
+      if constexpr (UN > 5) at(std::integral_constant<int, 5 % UN>());
+      if constexpr (UN > 6) at(std::integral_constant<int, 6 % UN>());
+      if constexpr (UN > 7) at(std::integral_constant<int, 7 % UN>());
+      if constexpr (CH != 0) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int i = 0; i < MB; ++i) {
+            if constexpr (TWO) acc[i][j] += low[TWO ? i : 0][TWO ? j : 0];
+            tot[CH ? i : 0][CH ? j : 0] += acc[i][j];
+          }
+      }
+    }
+    vm_wait<0>();
+  }
+  // lane: row m of C; value v: column 8 (v / 4) + 4 half + v % 4
+#pragma unroll
+  for (int j = 0; j < NB; ++j)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int n = n0 + (wn * NB + j) * 32 + 8 * g + 4 * half;
+      if (n >= a.N) continue;
+      const f4 mul = *reinterpret_cast<const f4*>(a.w_half_mul + n) * a.a_unscale;
+      f4 bias = f4{0.f, 0.f, 0.f, 0.f};
+      if (!SPLIT && a.bias) bias = *reinterpret_cast<const f4*>(a.bias + n);
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        const int m = m0 + (wm * MB + i) * 32 + l32;
+        if (m >= a.M) continue;
+        f4 c;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c[e] = CH ? tot[CH ? i : 0][CH ? j : 0][4 * g + e] : acc[i][j][4 * g + e];
+        c *= mul;
+        if constexpr (SPLIT != 0) {
+          *reinterpret_cast<f4*>(a.ws + ((size_t)blockIdx.y * a.M + m) * a.N + n) = c;
+          continue;
+        }
+        c += bias;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (EPI == GEMM_GELU) c[e] = gelu_tanh(c[e]);
+        if (EPI == GEMM_RESID) c += *reinterpret_cast<const f4*>(a.resid + (size_t)m * a.ldc + n);
+        if constexpr (EPI == GEMM_GELU) store_half4(a.C, mp, (size_t)m, (size_t)n, c, a.c_scale);
+        else *reinterpret_cast<f4*>(a.C + (size_t)m * a.ldc + n) = c;
+      }
+    }
+}
+
+// ---- some tens to some hundreds of rows --------------------------------------------------------
+// A block owns 16 MT input rows (blockIdx.z) and up to 16 NG rows of W (a.rows_per_block of them, a multiple of eight); its
+// eight wavefronts take the steps of 32 columns in turn, operands from L2 straight to registers, and the eight partial tiles
+// are added through LDS.  gridDim.y > 1: K is cut over blocks as well, raw tiles go to a.ws[part][M][N].  As k_gemm_cut_rows
+// (pg_gemm_rows.hip), with 4 bytes per input value for 6, and rows of W that need no turn through LDS and no cut.
+template <int EPI, int PW, int MT, int NG>
+__global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
+  constexpr int CSTR = 16 * NG + 4;  // row stride of the partial tile, floats
+  constexpr int PD = MT * NG * 8 + 8 * (NG * PW + MT * 2) <= 184 ? 2 : 1;  // steps requested ahead
+  __shared__ __attribute__((aligned(16))) float slab[8][16 * MT * CSTR];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int i16 = lane & 15, kq = lane >> 4;
+  const int n0 = (int)blockIdx.x * a.rows_per_block, n1 = min(n0 + a.rows_per_block, a.N);
+  const int m0 = (int)blockIdx.z * 16 * MT;
+  const int mp = cut_rows(a.M);
+  const int piece = (int)blockIdx.y * 8 + wave, pieces = (int)gridDim.y * 8;
+  const int steps_all = a.K / 32;
+  const int steps = piece < steps_all ? (steps_all - piece + pieces - 1) / pieces : 0;
+
+  const char* wp[NG];
+#pragma unroll
+  for (int g = 0; g < NG; ++g)
+    wp[g] = static_cast<const char*>(a.w_half) + ((size_t)kq * PW * a.N + min(n0 + 16 * g + i16, n1 - 1)) * 16;
+  const char* xp[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+    xp[mt] = reinterpret_cast<const char*>(a.A) + ((size_t)kq * 2 * mp + min(m0 + 16 * mt + i16, a.M - 1)) * 16;
+  const size_t wpart = (size_t)a.N * 16, wstep = wpart * 4 * PW, xpart = (size_t)mp * 16, xstep = xpart * 8;
+
+  // The write-out takes four columns of a row at a time, neighbouring lanes neighbouring columns, or, into a matrix
+  // in half form, neighbouring rows, which lie next to each other there.  What it adds is requested first.
+  constexpr int ITEMS = 16 * MT * 4 * NG;
+  constexpr int IPT = (ITEMS + 511) / 512;
+  const bool c_half = EPI == GEMM_GELU;
+  auto row_of = [&](int idx) { return c_half ? idx % (16 * MT) : idx / (4 * NG); };
+  auto col_of = [&](int idx) { return 4 * (c_half ? idx / (16 * MT) : idx % (4 * NG)); };
+  f4 ebias[IPT], eres[IPT], emul[IPT];
+#pragma unroll
+  for (int q = 0; q < IPT; ++q) {
+    const int idx = tid + 512 * q, m = m0 + row_of(idx), n = n0 + col_of(idx);
+    const bool live = idx < ITEMS && m < a.M && n < n1;
+    ebias[q] = eres[q] = emul[q] = f4{0.f, 0.f, 0.f, 0.f};
+    if (live) emul[q] = *reinterpret_cast<const f4*>(a.w_half_mul + n) * a.a_unscale;
+    if (gridDim.y > 1) continue;
+    if (live && a.bias) ebias[q] = *reinterpret_cast<const f4*>(a.bias + n);
+    if (live && EPI == GEMM_RESID) eres[q] = *reinterpret_cast<const f4*>(a.resid + (size_t)m * a.ldc + n);
+  }
+
+  f4 tot[MT][NG];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int g = 0; g < NG; ++g) tot[mt][g] = f4{0.f, 0.f, 0.f, 0.f};
+
+  u4v rw[PD][NG][PW], rx[PD][MT][2];
+  auto load_step = [&](int s, u4v (&w)[NG][PW], u4v (&x)[MT][2]) {
+    const size_t col = (size_t)piece + (size_t)pieces * min(s, steps - 1);
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int p = 0; p < PW; ++p) w[g][p] = *reinterpret_cast<const u4v*>(wp[g] + col * wstep + p * wpart);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) x[mt][p] = *reinterpret_cast<const u4v*>(xp[mt] + col * xstep + p * xpart);
+  };
+  auto mul_step = [&](const u4v (&w)[NG][PW], const u4v (&x)[MT][2]) {
+    // a chain of matrix instructions is a step, the small products one of their own; each product over a row of tiles before
+    // the next
+    auto one = [](const u4v& x, const u4v& w, const f4& c) {
+      return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8v, x), __builtin_bit_cast(h8v, w), c, 0, 0, 0);
+    };
+    const f4 zero{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+      f4 c[NG], big[NG];
+#pragma unroll
+      for (int g = 0; g < NG; ++g) c[g] = one(x[mt][1], w[g][0], zero);
+      if constexpr (PW == 2) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) c[g] = one(x[mt][0], w[g][PW - 1], c[g]);
+      }
+#pragma unroll
+      for (int g = 0; g < NG; ++g) big[g] = one(x[mt][0], w[g][0], zero);
+#pragma unroll
+      for (int g = 0; g < NG; ++g) tot[mt][g] += big[g] + c[g];
+    }
+  };
+  if (steps > 0) {
+#pragma unroll
+    for (int i = 0; i < PD; ++i) load_step(i, rw[i], rx[i]);
+    int s = 0;
+    for (; s + 2 * PD <= steps; s += PD) {
+#pragma unroll
+      for (int i = 0; i < PD; ++i) {
+        mul_step(rw[i], rx[i]);
+        load_step(s + i + PD, rw[i], rx[i]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < PD; ++i) {
+      if (s + i < steps) mul_step(rw[i], rx[i]);
+      if (s + i + PD < steps) load_step(s + i + PD, rw[i], rx[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < PD; ++i)
+      if (s + PD + i < steps) mul_step(rw[i], rx[i]);
+  }
+  // tot[mt][g][r] is row 16 mt + 4 kq + r, column 16 g + i16
+  float* mine = slab[wave];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        mine[(16 * mt + 4 * kq + r) * CSTR + 16 * g + i16] = tot[mt][g][r];
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < IPT; ++q) {
+    const int idx = tid + 512 * q, mr = row_of(idx), nl = col_of(idx);
+    const int m = m0 + mr, n = n0 + nl;
+    if (idx >= ITEMS || m >= a.M || n >= n1) continue;
+    f4 part[8];
+#pragma unroll
+    for (int w = 0; w < 8; ++w) part[w] = *reinterpret_cast<const f4*>(slab[w] + mr * CSTR + nl);
+    const f4 sum = (((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]))) * emul[q];
+    if (gridDim.y > 1) {
+      *reinterpret_cast<f4*>(a.ws + ((size_t)blockIdx.y * a.M + m) * a.N + n) = sum;
+      continue;
+    }
+    f4 c = ebias[q] + sum;
+    if (EPI == GEMM_GELU) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) c[e] = gelu_tanh(c[e]);
+      store_half4(a.C, mp, (size_t)m, (size_t)n, c, a.c_scale);
+      continue;
+    }
+    if (EPI == GEMM_RESID) c += eres[q];
+    *reinterpret_cast<f4*>(a.C + (size_t)m * a.ldc + n) = c;
+  }
+}
+
+// ---- norms -------------------------------------------------------------------------------------
+// Rows of N values to LayerNorm in half form (layer_norm_in_place, cpu.rs:119-143: mean, biased variance in a second pass,
+// eps inside the root), a wavefront a row, four rows a block: the 16-byte pieces of four rows lie next to each other in half
+// form, and the block writes them so, through LDS.  PARTS: the row is first put together from the parts of a cut K, bias and
+// residual, and written to a.C; otherwise it is read from there.  NQ: 256 NQ >= N.
+// Pairs of blocks whose rows share cache lines are on one XCD (block % 8).
+template <int NQ, bool PARTS>
+__global__ __launch_bounds__(256) void k_norm_rows_half(GemmArgs a, int parts) {
+  extern __shared__ __attribute__((aligned(16))) char staged[];
+  constexpr int OSTR = 2 * 4 * 16 + 16;  // an octet of columns: two parts, four rows; padded
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int b = (int)blockIdx.x / 16 * 16 + (int)blockIdx.x % 8 * 2 + (int)blockIdx.x % 16 / 8;
+  const int m0 = 4 * b, m = min(m0 + wave, a.M - 1), n4 = a.N / 4;
+  if (m0 >= a.M) return;
+  f4 c[NQ], g[NQ], sh[NQ];
+  auto col = [&](int q) { return 4 * (size_t)min(lane + 64 * q, n4 - 1); };
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) c[q] = *reinterpret_cast<const f4*>((PARTS ? a.resid : a.C) + (size_t)m * a.ldc + col(q));
+  if constexpr (PARTS) {
+    f4 s[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) s[q] = *reinterpret_cast<const f4*>(a.ws + (size_t)m * a.N + col(q));
+    for (int p = 1; p < parts; ++p)
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) s[q] += *reinterpret_cast<const f4*>(a.ws + ((size_t)p * a.M + m) * a.N + col(q));
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      if (a.bias) s[q] = *reinterpret_cast<const f4*>(a.bias + col(q)) + s[q];
+      c[q] = c[q] + s[q];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    g[q] = *reinterpret_cast<const f4*>(a.ln_g + col(q));
+    sh[q] = *reinterpret_cast<const f4*>(a.ln_b + col(q));
+  }
+  float sum = 0.0f;
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const bool live = lane + 64 * q < n4;
+    if (PARTS && live && m0 + wave < a.M) *reinterpret_cast<f4*>(a.C + (size_t)m * a.ldc + col(q)) = c[q];
+    if (live) sum += (c[q].x + c[q].y) + (c[q].z + c[q].w);
+  }
+  const float mean = wave_sum(sum) / (float)a.N;
+  float var = 0.0f;
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const f4 d = c[q] - mean;
+    if (lane + 64 * q < n4) var += (d.x * d.x + d.y * d.y) + (d.z * d.z + d.w * d.w);
+  }
+  const float inv = 1.0f / sqrtf(wave_sum(var) / (float)a.N + a.ln_eps);
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const int i = lane + 64 * q;
+    if (i >= n4) continue;
+    const f4 o = (c[q] - mean) * inv * g[q] + sh[q];
+    unsigned h0, l0, h1, l1;
+    halves2(o.x, o.y, a.ln_scale, h0, l0);
+    halves2(o.z, o.w, a.ln_scale, h1, l1);
+    char* at = staged + (i >> 1) * OSTR + wave * 16 + (i & 1) * 8;
+    *reinterpret_cast<u2v*>(at) = u2v{h0, h1};
+    *reinterpret_cast<u2v*>(at + 64) = u2v{l0, l1};
+  }
+  __syncthreads();
+  const int mp = cut_rows(a.M);
+  for (int i = threadIdx.x; i < a.N; i += 256) {  // (octet, part, row)
+    const int row = i & 3;
+    if (m0 + row >= a.M) continue;
+    *reinterpret_cast<u4v*>(reinterpret_cast<char*>(a.ln_out) + ((size_t)(i >> 2) * mp + m0 + row) * 16) =
+        *reinterpret_cast<const u4v*>(staged + (i >> 3) * OSTR + (i & 7) * 16);
+  }
+}
+
+template <bool PARTS>
+hipError_t launch_norm_rows(const GemmArgs& a, int parts, hipStream_t s) {
+  if (a.N % 8 != 0 || a.N > 4096 || a.ldc != a.N || a.ln_scale == 0.0f) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)((a.M + 63) / 64 * 16));
+  const size_t lds = (size_t)a.N / 8 * (2 * 4 * 16 + 16);
+  if (a.N <= 768) hipLaunchKernelGGL((k_norm_rows_half<3, PARTS>), grid, dim3(256), lds, s, a, parts);
+  else if (a.N <= 1280) hipLaunchKernelGGL((k_norm_rows_half<5, PARTS>), grid, dim3(256), lds, s, a, parts);
+  else if (a.N <= 1792) hipLaunchKernelGGL((k_norm_rows_half<7, PARTS>), grid, dim3(256), lds, s, a, parts);
+  else hipLaunchKernelGGL((k_norm_rows_half<16, PARTS>), grid, dim3(256), lds, s, a, parts);
+  return hipGetLastError();
+}
+// ---- weights -----------------------------------------------------------------------------------
+// Rows of W as stored (WT as elsewhere: f32, bf16, int8 with their scales) to half form: part p of element (n, k) is the
+// (k % 8)-th f16 of the 16 bytes at ((k / 8 * PW + p) * N + n) * 16, times mul[n]^-1; a f32 or bf16 row is scaled by the power of
+// two that puts its largest value between 2^14 and 2^15.  *refused is set where a bf16 weight is not a f16 number so (a row
+// that spans more than 2^32), a value is not finite, or a row is so small or large that its power of two would matter.
+template <int WT>
+__global__ __launch_bounds__(256) void k_half_rows(const void* W, const float* scales, void* to, float* mul, unsigned* refused,
+                                                   int N, int K) {
+  constexpr int PW = WT == 0 ? 2 : 1;
+  __shared__ float biggest[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n = (int)blockIdx.x * 64 + lane, row = min(n, N - 1);
+  auto get = [&](int k, float (&x)[8]) {  // columns k .. k + 7
+    if constexpr (WT == 0) {
+      const f4* w = reinterpret_cast<const f4*>(static_cast<const float*>(W) + (size_t)row * K + k);
+      const f4 u = w[0], v = w[1];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = u[e], x[4 + e] = v[e];
+    } else if constexpr (WT == 1) {
+      const u4v w = *reinterpret_cast<const u4v*>(static_cast<const unsigned short*>(W) + (size_t)row * K + k);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = __uint_as_float(e & 1 ? w[e / 2] & 0xffff0000u : w[e / 2] << 16);
+    } else {
+      const u2v w = *reinterpret_cast<const u2v*>(static_cast<const signed char*>(W) + (size_t)row * K + k);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = (float)((int)(w[e / 4] << (24 - 8 * (e % 4))) >> 24);
+    }
+  };
+  float x[8], scale = 1.0f;
+  bool bad = false;
+  if constexpr (WT != 2) {
+    float most = 0.0f;
+    for (int k = 8 * wave; k < K; k += 32) {
+      get(k, x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        bad |= !(fabsf(x[e]) < INFINITY);
+        most = fmaxf(most, fabsf(x[e]));
+      }
+    }
+    biggest[wave][lane] = most;
+    __syncthreads();
+    most = fmaxf(fmaxf(biggest[0][lane], biggest[1][lane]), fmaxf(biggest[2][lane], biggest[3][lane]));
+    int e = 15;
+    if (most > 0.0f && most < INFINITY) frexpf(most, &e);
+    bad |= most > 0.0f && abs(15 - e) > kHalfMostExp;
+    scale = bad ? 1.0f : ldexpf(1.0f, 15 - e);
+  } else {
+    bad = !(fabsf(scales[row]) < INFINITY);
+  }
+  if (wave == 0 && n < N) mul[n] = WT == 2 ? scales[row] : 1.0f / scale;
+  for (int k = 8 * wave; k < K; k += 32) {
+    get(k, x);
+    u4v h, l;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      unsigned hi, lo;
+      halves2(x[2 * e], x[2 * e + 1], scale, hi, lo);
+      h[e] = hi, l[e] = lo;
+      const h2v f = __builtin_bit_cast(h2v, hi);
+      if (PW == 1) bad |= (float)f.x != x[2 * e] * scale || (float)f.y != x[2 * e + 1] * scale;
+    }
+    if (n < N) {
+      u4v* at = static_cast<u4v*>(to) + (size_t)(k / 8) * PW * N + n;
+      at[0] = h;
+      if (PW == 2) at[N] = l;
+    }
+  }
+  if (bad) atomicOr(refused, 1u);
+}
+
+// The largest that an output of a projection behind a LayerNorm can be: the norm's values before scale and shift are at most
+// sqrt(C) long together, so |W_o . (g z + b) + bias_o| <= sqrt(C) |W_o g| + |W_o . b + bias_o|, the second as fold has it
+// (launch_ln_fold).  The maximum over the rows goes to *most, bits of a float that is not negative.
+template <int WT>
+__global__ __launch_bounds__(256) void k_half_bound(const void* W, const float* scales, const float* g, const float* fold,
+                                                    unsigned* most, int N, int K) {
+  const int lane = threadIdx.x & 63, row = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= N) return;
+  float ss = 0.0f;
+  for (int k = lane; k < K; k += 64) {
+    const size_t at = (size_t)row * K + k;
+    const float w = WT == 0   ? static_cast<const float*>(W)[at]
+                    : WT == 1 ? __uint_as_float((unsigned)static_cast<const unsigned short*>(W)[at] << 16)
+                              : (float)static_cast<const signed char*>(W)[at] * scales[row];
+    ss = fmaf(w * g[k], w * g[k], ss);
+  }
+  ss = wave_sum(ss);
+  if (lane == 0) {
+    const float b = sqrtf(ss * (float)K) + fabsf(fold[2 * row + 1]);
+    atomicMax(most, b < INFINITY ? __float_as_uint(b) : 0x7f800000u);  // (NaN too)
+  }
+}
+// The same of the norm's own values: sqrt(C) |g_c| + |b_c|.
+__global__ __launch_bounds__(256) void k_half_bound_norm(const float* g, const float* b, unsigned* most, int C) {
+  const int i = (int)blockIdx.x * 256 + threadIdx.x;
+  if (i >= C) return;
+  const float v = fabsf(g[i]) * sqrtf((float)C) + fabsf(b[i]);
+  atomicMax(most, v < INFINITY ? __float_as_uint(v) : 0x7f800000u);
+}
+
+// ---- launchers ---------------------------------------------------------------------------------
+template <int WM, int WN, int MB, int NB, int PW, int OCC, int NA, int KT, int CH, bool TWO>
+struct Shape {
+  static constexpr int bm = 32 * MB * WM, bn = 32 * NB * WN;
+  template <int EPI, int SPLIT>
+  static hipError_t start(const GemmArgs& a0, int parts, hipStream_t s) {
+    GemmArgs a = a0;
+    const int tiles_m = (a.M + bm - 1) / bm, tiles_n = (a.N + bn - 1) / bn, tiles = tiles_m * tiles_n;
+    a.band_rows = choose_band(tiles_m, std::max(1, (tiles + 7) / 8), bm, bn);
+    const dim3 grid((unsigned)((tiles + 7) / 8 * 8), (unsigned)parts);  // whole rounds over the 8 XCDs
+    hipLaunchKernelGGL((k_gemm_half<WM, WN, MB, NB, PW, EPI, SPLIT, OCC, NA, KT, CH, TWO>), grid, dim3(64 * WM * WN), 0, s, a);
+    return hipGetLastError();
+  }
+  static hipError_t launch(const GemmArgs& a, int epi, int parts, hipStream_t s) {
+    if (parts > 1) return start<GEMM_BIAS, 1>(a, parts, s);
+    switch (epi) {
+      case GEMM_BIAS: return start<GEMM_BIAS, 0>(a, 1, s);
+      case GEMM_GELU: return start<GEMM_GELU, 0>(a, 1, s);
+      case GEMM_RESID: return start<GEMM_RESID, 0>(a, 1, s);
+      default: return hipErrorInvalidValue;
+    }
+  }
+};
+hipError_t launch_tile(const GemmArgs& a, int epi, const HalfPlan& p, hipStream_t s) {
+  if (a.w_half_parts == 2) {
+    switch (p.tile) {
+      case HALF_64x128: return Shape<2, 2, 1, 2, 2, 3, 2, 32, 4, true>::launch(a, epi, p.parts, s);
+      case HALF_128x128: return Shape<2, 2, 2, 2, 2, 2, 4, 16, 4, false>::launch(a, epi, p.parts, s);
+      case HALF_128x128_8: return Shape<4, 2, 1, 2, 2, 2, 4, 32, 4, true>::launch(a, epi, p.parts, s);
+      default: return hipErrorInvalidValue;
+    }
+  }
+  switch (p.tile) {
+    case HALF_64x128: return Shape<2, 2, 1, 2, 1, 3, 2, 32, 4, true>::launch(a, epi, p.parts, s);
+    case HALF_128x128: return Shape<2, 2, 2, 2, 1, 2, 4, 16, 4, false>::launch(a, epi, p.parts, s);
+    case HALF_128x128_8: return Shape<4, 2, 1, 2, 1, 2, 4, 32, 4, true>::launch(a, epi, p.parts, s);
+    case HALF_128x256: return Shape<2, 2, 2, 4, 1, 2, 4, 16, 0, false>::launch(a, epi, p.parts, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+template <int EPI, int PW>
+hipError_t launch_rows_form(const GemmArgs& a, const HalfPlan& p, hipStream_t s) {
+  const dim3 grid((unsigned)((a.N + a.rows_per_block - 1) / a.rows_per_block), (unsigned)p.parts,
+                  (unsigned)((a.M + 16 * p.mt - 1) / (16 * p.mt)));
+  const int ng = (p.rows + 15) / 16;
+#define PG_CASE(MT, NG) \
+  if (p.mt == MT && ng == NG) { hipLaunchKernelGGL((k_gemm_half_rows<EPI, PW, MT, NG>), grid, dim3(512), 0, s, a); return hipGetLastError(); }
+  PG_CASE(2, 1) PG_CASE(3, 1) PG_CASE(4, 1)
+  PG_CASE(2, 2) PG_CASE(3, 2) PG_CASE(4, 2)
+  PG_CASE(3, 3) PG_CASE(4, 3)
+  PG_CASE(3, 4) PG_CASE(4, 4)
+#undef PG_CASE
+  return hipErrorInvalidValue;
+}
+template <int PW>
+hipError_t launch_rows(const GemmArgs& a, int epi, const HalfPlan& p, hipStream_t s) {
+  if (p.parts > 1) return launch_rows_form<GEMM_BIAS, PW>(a, p, s);
+  switch (epi) {
+    case GEMM_BIAS: return launch_rows_form<GEMM_BIAS, PW>(a, p, s);
+    case GEMM_GELU: return launch_rows_form<GEMM_GELU, PW>(a, p, s);
+    case GEMM_RESID: return launch_rows_form<GEMM_RESID, PW>(a, p, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+// Time of a product in microseconds.  Tiles: a start, the stages of 32 columns at the pace of the CU with the most items (a stage
+// alone, each further item, a partly filled round).  Blocks of rows: rounds of the blocks over the CUs, of a block's steps over
+// its wavefronts.  And what is left to do behind it: the launch that adds the parts, with or without a norm, per part and
+// value, or a norm by itself.  Constants of the least regret over the four projections of widths 512 to 1600 at 17 to 8192 rows,
+// W from HBM (29000 plans): the plan of least predicted time is 1.2 % slower than the best measured one in the mean.
+struct TilePace {
+  float start, stage, more, part;
+};
+struct Finish {
+  float reduce_norm, part, values_norm, reduce, values, norm, norm_values;
+};
+struct RowsPace {
+  float start, turn, step, mt, ng, both, fill_mt, fill_ng;
+};
+// [one f16 number a weight][HalfTile]
+constexpr TilePace kTilePace[2][4] = {
+    {{3.796f, 0.532f, 0.032f, 0.251f}, {5.756f, 0.612f, 0.372f, 0.096f}, {5.263f, 0.48f, 0.654f, 1.153f}, {}},
+    {{5.567f, 0.356f, 0.007f, 0.175f}, {7.833f, 0.372f, 0.202f, 0.157f}, {6.345f, 0.331f, 0.72f, -0.094f}, {8.862f, 0.706f, 0.349f, 0.166f}}};
+constexpr Finish kFinish[2] = {{2.922f, 1.748f, -0.459f, 3.138f, -0.459f, 1.276f, 1.735f},
+                               {5.609f, 1.263f, 0.344f, 3.75f, -0.147f, 5.585f, 1.314f}};
+constexpr RowsPace kRowsPace[2] = {{1.161f, 0.813f, -0.651f, 0.288f, 0.59f, -0.099f, -0.01f, 0.189f},
+                                   {1.271f, 1.95f, -0.585f, 0.182f, 0.245f, -0.007f, -0.006f, 0.098f}};
+
+}  // namespace
+
+bool gemm_half_takes(const GemmArgs& a, int epi) {
+  const uintptr_t at = reinterpret_cast<uintptr_t>(a.A) | reinterpret_cast<uintptr_t>(a.w_half) | reinterpret_cast<uintptr_t>(a.C) |
+                       reinterpret_cast<uintptr_t>(a.w_half_mul) | reinterpret_cast<uintptr_t>(a.bias) |
+                       reinterpret_cast<uintptr_t>(a.resid) | reinterpret_cast<uintptr_t>(a.ws) | reinterpret_cast<uintptr_t>(a.ln_out) |
+                       reinterpret_cast<uintptr_t>(a.ln_g) | reinterpret_cast<uintptr_t>(a.ln_b);
+  return a.w_half && a.w_half_mul && (a.w_half_parts == 1 || a.w_half_parts == 2) && !(at & 15) && a.M >= 1 && a.M < (1 << 23) &&
+         a.K >= 64 && a.K % 32 == 0 && a.N >= 64 && a.N % 8 == 0 && a.N < (1 << 24) && a.ldc % 4 == 0 && a.a_unscale > 0.0f &&
+         (epi == GEMM_GELU) == (a.c_scale > 0.0f) && (!a.ln_out || a.ln_scale > 0.0f) &&
+         (epi == GEMM_BIAS || epi == GEMM_GELU || epi == GEMM_RESID) && (epi != GEMM_GELU || a.ldc == a.N);
+}
+
+HalfPlan gemm_half_plan(const GemmArgs& a, int epi, int num_cus) {
+  const bool one = a.w_half_parts == 1;
+  const int steps = a.K / 32, cus = num_cus;
+  const float mn = (float)a.M * (float)a.N * 1e-6f;
+  const int most = epi != GEMM_GELU && a.ws ? (int)std::min<size_t>(std::min(8, a.K / 256), a.ws_floats / ((size_t)a.M * a.N)) : 1;
+  const Finish& f = kFinish[one];
+  auto finish = [&](int parts) {
+    if (parts == 1) return a.ln_out ? f.norm + f.norm_values * mn : 0.0f;
+    return (a.ln_out ? f.reduce_norm : f.reduce) + (f.part * (float)parts + (a.ln_out ? f.values_norm : f.values)) * mn;
+  };
+  HalfPlan best{HALF_128x128, 1, 0, 0};
+  float best_us = INFINITY;
+  auto take = [&](const HalfPlan& p, float us) {
+    if (us < best_us) best = p, best_us = us;
+  };
+  for (int t : {HALF_64x128, HALF_128x128, HALF_128x128_8, HALF_128x256}) {
+    if (t == HALF_128x256 && !one) continue;
+    const int bm = t == HALF_64x128 ? 64 : 128, bn = t == HALF_128x256 ? 256 : 128;
+    const long tiles = (long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
+    for (int parts = 1; parts <= std::max(1, most); ++parts) {
+      const long items = (tiles + 7) / 8 * 8 * parts;  // (as many to each XCD as the fullest one has)
+      const float on_cu = (float)((items + cus - 1) / cus), round = std::max(0.0f, (float)items / (float)cus - 1.0f);
+      const TilePace& p = kTilePace[one][t];
+      take({t, parts, 0, 0}, p.start + (float)((steps + parts - 1) / parts) * (p.stage + (on_cu - 1.0f) * p.more + round * p.part) + finish(parts));
+    }
+  }
+  const int groups = (a.M + 63) / 64, mt = std::max(2, ((a.M + groups - 1) / groups + 15) / 16);
+  const int m_blocks = (a.M + 16 * mt - 1) / (16 * mt);
+  const RowsPace& p = kRowsPace[one];
+  for (int parts = 1; m_blocks <= 65535 && parts <= std::max(1, most); ++parts)
+    for (int rows = 8; rows <= (mt == 2 ? 32 : 64); rows += 8) {
+      const int ng = (rows + 15) / 16;
+      const long blocks = (long)((a.N + rows - 1) / rows) * m_blocks * parts;
+      const float turns = (float)((blocks + cus - 1) / cus), fill = (float)blocks / (float)cus;
+      const float rounds = (float)(((steps + parts - 1) / parts + 7) / 8);
+      take({HALF_ROWS, parts, mt, rows},
+           p.start + turns * (p.turn + rounds * (p.step + p.mt * mt + p.ng * ng + p.both * mt * ng)) +
+               fill * rounds * (p.fill_mt * mt + p.fill_ng * ng) + finish(parts));
+    }
+  return best;
+}
+
+hipError_t launch_gemm_half_plan(const GemmArgs& a0, int epi, const HalfPlan& p, hipStream_t s) {
+  GemmArgs a = a0;
+  if (!gemm_half_takes(a, epi) || p.parts < 1 || p.parts > 8) return hipErrorInvalidValue;
+  if (p.parts > 1 && (epi == GEMM_GELU || !a.ws || a.K / 32 < p.parts || (size_t)p.parts * a.M * a.N > a.ws_floats)) return hipErrorInvalidValue;
+  if (p.tile != HALF_ROWS) return launch_tile(a, epi, p, s);
+  if (p.rows < 8 || p.rows % 8 != 0 || (a.M + 16 * p.mt - 1) / (16 * p.mt) > 65535) return hipErrorInvalidValue;
+  a.rows_per_block = p.rows;
+  return a.w_half_parts == 2 ? launch_rows<2>(a, epi, p, s) : launch_rows<1>(a, epi, p, s);
+}
+
+hipError_t launch_gemm_half(const GemmArgs& a, int epi, int num_cus, hipStream_t s) {
+  if (!gemm_half_takes(a, epi)) return hipErrorInvalidValue;
+  const HalfPlan p = gemm_half_plan(a, epi, num_cus);
+  const hipError_t e = launch_gemm_half_plan(a, epi, p, s);
+  return e != hipSuccess ? e : finish_gemm_half(a, epi, p, s);
+}
+hipError_t finish_gemm_half(const GemmArgs& a, int epi, const HalfPlan& p, hipStream_t s) {
+  if (p.parts == 1) return a.ln_out ? launch_norm_rows<false>(a, 0, s) : hipSuccess;
+  if (a.ln_out && epi == GEMM_RESID) return launch_norm_rows<true>(a, p.parts, s);
+  bool ln_done = false;
+  return a.ln_out ? hipErrorInvalidValue : launch_splitk_reduce(a, epi, p.parts, s, &ln_done);
+}
+
+hipError_t launch_norm_rows_half(const float* src, void* dst, int rows, int cols, const float* g, const float* b, float eps,
+                                 float scale, hipStream_t s) {
+  GemmArgs a{};
+  a.C = const_cast<float*>(src); a.ln_out = static_cast<float*>(dst); a.M = rows; a.N = a.ldc = cols;
+  a.ln_g = g; a.ln_b = b; a.ln_eps = eps; a.ln_scale = scale;
+  return launch_norm_rows<false>(a, 0, s);
+}
+
+hipError_t launch_half_rows(const void* W, int w_bytes, const float* scales, size_t rows, int cols, void* to, float* mul,
+                            unsigned* refused, hipStream_t s) {
+  const dim3 grid((unsigned)((rows + 63) / 64));
+  if (cols % 32 != 0 || rows > (1u << 24)) return hipErrorInvalidValue;
+  if (w_bytes == 4) hipLaunchKernelGGL(k_half_rows<0>, grid, dim3(256), 0, s, W, scales, to, mul, refused, (int)rows, cols);
+  else if (w_bytes == 2) hipLaunchKernelGGL(k_half_rows<1>, grid, dim3(256), 0, s, W, scales, to, mul, refused, (int)rows, cols);
+  else hipLaunchKernelGGL(k_half_rows<2>, grid, dim3(256), 0, s, W, scales, to, mul, refused, (int)rows, cols);
+  return hipGetLastError();
+}
+hipError_t launch_half_bound(const void* W, int w_bytes, const float* scales, const float* g, const float* fold, size_t rows, int cols,
+                             unsigned* most, hipStream_t s) {
+  const dim3 grid((unsigned)((rows + 3) / 4));
+  if (w_bytes == 4) hipLaunchKernelGGL(k_half_bound<0>, grid, dim3(256), 0, s, W, scales, g, fold, most, (int)rows, cols);
+  else if (w_bytes == 2) hipLaunchKernelGGL(k_half_bound<1>, grid, dim3(256), 0, s, W, scales, g, fold, most, (int)rows, cols);
+  else hipLaunchKernelGGL(k_half_bound<2>, grid, dim3(256), 0, s, W, scales, g, fold, most, (int)rows, cols);
+  return hipGetLastError();
+}
+hipError_t launch_half_bound_norm(const float* g, const float* b, int cols, unsigned* most, hipStream_t s) {
+  hipLaunchKernelGGL(k_half_bound_norm, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, s, g, b, most, cols);
+  return hipGetLastError();
+}
+
+}  // namespace pgk

@@ -497,6 +497,82 @@ bool takes_cut_form(const pg_model* m, size_t rows) {
          pgk::gemm_takes_cut((int)rows, (int)g.C, (int)g.I, m->w_bf16, m->w_i8, m->cut_form_min_rows, m->num_cus);
 }
 
+// Whether so many rows of activations are kept in half form: from the rows on that the cut form starts at.  f32 rows: 65 to 128
+// stay on the f32 cores as they do there, and a set bound (gemm_b9_min_rows) holds for this form too.
+bool takes_half_form(const pg_model* m, size_t rows) {
+  if (m->half.empty()) return false;
+  if (m->w_bf16 || m->w_i8) return rows >= (size_t)pgk::kCutFormMinRows;
+  return rows >= (size_t)m->cut_form_min_rows && (rows <= 64 || rows > 128);
+}
+
+// The block matrices in half form.  Nothing of it is needed to serve a call: where it cannot be had the model goes without.
+pg_status make_half_form(pg_model* m) {
+  const Cfg& g = m->cfg;
+  if (g.hd() != pgk::kHeadDim || g.C < 256 || g.C % 32 != 0 || g.C > 4096 || g.I < 256 || g.I % 32 != 0) return PG_OK;
+  const int wb = m->w_i8 ? 1 : m->w_bf16 ? 2 : 4, pw = wb == 4 ? 2 : 1;
+  auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+  const size_t C = g.C, I = g.I;
+  const size_t rows[4] = {3 * C, C, I, C}, cols[4] = {C, C, C, I};
+  size_t layer = 0;
+  for (int i = 0; i < 4; ++i) layer += up(rows[i] * cols[i] * 2 * pw) + up(rows[i] * 4);
+  constexpr int kBounds = 4;  // of a layer: both norms, values, hidden
+  const size_t words = up((g.L * kBounds + 1) * 4);
+  if (hipMalloc(&m->half_arena, g.L * layer + words) != hipSuccess) {
+    (void)hipGetLastError();
+    m->half_arena = nullptr;
+    return PG_OK;
+  }
+  unsigned* bounds = reinterpret_cast<unsigned*>(m->half_arena);
+  unsigned* refused = bounds + g.L * kBounds;
+  PG_HIP(pgk::launch_fill_zero(reinterpret_cast<float*>(bounds), g.L * kBounds + 1, nullptr));
+  m->half.resize(g.L);
+  char* at = m->half_arena + words;
+  for (size_t l = 0; l < g.L; ++l) {
+    const pgk::LayerW& w = m->layers[l];
+    const float* mats[4] = {w.c_attn_w, w.c_proj_w, w.c_fc_w, w.c_proj_mlp_w};
+    const float* scales[4] = {w.c_attn_s, w.c_proj_s, w.c_fc_s, w.c_proj_mlp_s};
+    void* to[4];
+    float* mul[4];
+    for (int i = 0; i < 4; ++i) {
+      to[i] = at;
+      at += up(rows[i] * cols[i] * 2 * pw);
+      mul[i] = reinterpret_cast<float*>(at);
+      at += up(rows[i] * 4);
+      PG_HIP(pgk::launch_half_rows(mats[i], wb, scales[i], rows[i], (int)cols[i], to[i], mul[i], refused, nullptr));
+    }
+    m->half[l] = pg_model::HalfLayer{to[0], to[1], to[2], to[3], mul[0], mul[1], mul[2], mul[3], 0, 0, 0, 0};
+    unsigned* b = bounds + l * kBounds;
+    PG_HIP(pgk::launch_half_bound_norm(w.ln_1_g, w.ln_1_b, (int)C, b, nullptr));
+    PG_HIP(pgk::launch_half_bound_norm(w.ln_2_g, w.ln_2_b, (int)C, b + 1, nullptr));
+    const char* values = reinterpret_cast<const char*>(w.c_attn_w) + 2 * C * C * wb;  // (an average of values is no larger than they are)
+    PG_HIP(pgk::launch_half_bound(values, wb, w.c_attn_s ? w.c_attn_s + 2 * C : nullptr, w.ln_1_g, w.c_attn_f + 4 * C, C, (int)C, b + 2, nullptr));
+    PG_HIP(pgk::launch_half_bound(w.c_fc_w, wb, w.c_fc_s, w.ln_2_g, w.c_fc_f, I, (int)C, b + 3, nullptr));  // (|gelu(x)| <= |x|)
+  }
+  std::vector<unsigned> got(g.L * kBounds + 1);
+  PG_HIP(hipMemcpy(got.data(), bounds, got.size() * 4, hipMemcpyDeviceToHost));
+  bool ok = got.back() == 0;
+  auto scale = [&](unsigned bits) {
+    float bound;
+    memcpy(&bound, &bits, 4);
+    int e = 0;
+    if (!std::isfinite(bound)) ok = false;
+    else if (bound > 0.0f) frexpf(bound, &e);
+    if (std::abs(15 - e) > pgk::kHalfMostExp) ok = false;
+    return ldexpf(1.0f, ok ? 15 - e : 0);
+  };
+  for (size_t l = 0; l < g.L; ++l) {
+    pg_model::HalfLayer& w = m->half[l];
+    w.norm_1 = scale(got[l * kBounds]), w.norm_2 = scale(got[l * kBounds + 1]);
+    w.attn = scale(got[l * kBounds + 2]), w.hidden = scale(got[l * kBounds + 3]);
+  }
+  if (!ok) {
+    m->half.clear();
+    (void)hipFree(m->half_arena);
+    m->half_arena = nullptr;
+  }
+  return PG_OK;
+}
+
 // Full-sequence forward of the nb sequences b .. b + nb - 1 over ids[nb][n] (each one
 // Gpt2Model::forward, src/models/gpt2/rust.rs:831-882, block_forward at 1053-1134) with MFMA
 // GEMMs over all nb * n rows at once and tiled causal attention per sequence; K and V of every
@@ -519,10 +595,12 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
   DevBuf SCR, LOG;
   // split-K partial tiles of the projections back to n_embd columns (up to 8 parts)
   const size_t ws_floats = 8 * n * g.C;
-  // the projections' inputs (XN, ATT, HB) in cut form
+  // the projections' inputs (XN, ATT, HB) in half form or in cut form
   const bool cut = !c->drawn && takes_cut_form(m, n);
+  const bool half = !cut && !c->drawn && takes_half_form(m, n);
+  const int form_of = half ? pgk::FORM_HALF : cut ? pgk::FORM_CUT : pgk::FORM_ROWS;
   {
-    auto form = [&](size_t cols) { return cut ? std::max(n * cols, pgk::cut_floats(n, cols)) : n * cols; };
+    auto form = [&](size_t cols) { return cut ? std::max(n * cols, pgk::cut_floats(n, cols)) : half ? pgk::half_floats(n, cols) : n * cols; };
     auto up = [](size_t v) { return (v + 63) / 64 * 64; };  // 256-byte boundaries
     const size_t sizes[7] = {up(n * g.C),   up(form(g.C)), up(n * 3 * g.C), up(form(g.C)),
                              up(form(g.I)), up(n),         up(ws_floats)};
@@ -569,10 +647,15 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
   // same call: fused into the projection's reduce where it has one)
   auto gemm = [&](const float* A, int lda, const float* W, const float* bias, float* Cout,
                   int ldc, int N, int K, int epi, const float* ln_g = nullptr,
-                  const float* ln_b = nullptr, int a_cut = 0, int c_cut = 0) -> hipError_t {
+                  const float* ln_b = nullptr, int a_cut = 0, int c_cut = 0, const void* w_half = nullptr,
+                  const float* w_half_mul = nullptr, float a_scale = 0.0f, float c_scale = 0.0f, float ln_scale = 0.0f) -> hipError_t {
     pgk::GemmArgs a{};
     a.A = A; a.w_bf16 = m->w_bf16; a.W = W; a.bias = bias; a.resid = Cout; a.C = Cout;
     a.a_cut = a.ln_cut = a_cut; a.c_cut = c_cut;
+    if (w_half) {
+      a.w_half = w_half; a.w_half_mul = w_half_mul; a.w_half_parts = m->w_bf16 || m->w_i8 ? 1 : 2;
+      a.a_unscale = 1.0f / a_scale; a.c_scale = c_scale; a.ln_scale = ln_g ? ln_scale : 0.0f;
+    }
     a.M = T; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc;
     if (m->w_i8) a.w_scale = i8_scales_of(W, (size_t)N, (size_t)K);
     a.ws = WS.p; a.ws_floats = ws_floats;
@@ -581,25 +664,33 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
     a.b9_min_rows = m->gemm_b9_min_rows;
     return pgk::launch_gemm(a, epi, m->num_cus, s);
   };
-  PG_HIP(pgk::launch_layer_norm_rows(X.p, XN.p, T, C, m->layers[0].ln_1_g, m->layers[0].ln_1_b, g.eps, s,
-                                     cut ? pgk::FORM_CUT : pgk::FORM_ROWS));
+  if (half)
+    PG_HIP(pgk::launch_norm_rows_half(X.p, XN.p, T, C, m->layers[0].ln_1_g, m->layers[0].ln_1_b, g.eps, m->half[0].norm_1, s));
+  else
+    PG_HIP(pgk::launch_layer_norm_rows(X.p, XN.p, T, C, m->layers[0].ln_1_g, m->layers[0].ln_1_b, g.eps, s, form_of));
   PG_MARK(kLayerNorm);
   for (size_t l = 0; l < g.L; ++l) {
     const pgk::LayerW& w = m->layers[l];
+    const pg_model::HalfLayer hw = half ? m->half[l] : pg_model::HalfLayer{};
     // the LayerNorm after this layer: the next layer's ln_1; ln_f is applied where it is needed
     const float* next_g = l + 1 < g.L ? m->layers[l + 1].ln_1_g : nullptr;
     const float* next_b = l + 1 < g.L ? m->layers[l + 1].ln_1_b : nullptr;
-    PG_HIP(gemm(XN.p, C, w.c_attn_w, w.c_attn_b, QKV.p, 3 * C, 3 * C, C, pgk::GEMM_BIAS, nullptr, nullptr, cut));
+    const float next_norm = half && l + 1 < g.L ? m->half[l + 1].norm_1 : 0.0f;
+    PG_HIP(gemm(XN.p, C, w.c_attn_w, w.c_attn_b, QKV.p, 3 * C, 3 * C, C, pgk::GEMM_BIAS, nullptr, nullptr, cut, 0,
+                hw.c_attn, hw.c_attn_mul, hw.norm_1));
     PG_MARK(kQkv);
     PG_HIP(pgk::launch_attn_prefill(QKV.p, Ts, C, H, hd, P, c->k_panel(l, b), c->v_panel(l, b),
                                     ATT.p, SCR.p, m->num_cus, s, (int)nb, g.H * g.P * g.hd(),
-                                    cut ? pgk::FORM_CUT : pgk::FORM_ROWS, c->drawn));
+                                    form_of, c->drawn, hw.attn));
     PG_MARK(kAttention);
-    PG_HIP(gemm(ATT.p, C, w.c_proj_w, w.c_proj_b, X.p, C, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b, cut));
+    PG_HIP(gemm(ATT.p, C, w.c_proj_w, w.c_proj_b, X.p, C, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b, cut, 0,
+                hw.c_proj, hw.c_proj_mul, hw.attn, 0.0f, hw.norm_2));
     PG_MARK(kAttnProj);
-    PG_HIP(gemm(XN.p, C, w.c_fc_w, w.c_fc_b, HB.p, I, I, C, pgk::GEMM_GELU, nullptr, nullptr, cut, cut));
+    PG_HIP(gemm(XN.p, C, w.c_fc_w, w.c_fc_b, HB.p, I, I, C, pgk::GEMM_GELU, nullptr, nullptr, cut, cut,
+                hw.c_fc, hw.c_fc_mul, hw.norm_2, hw.hidden));
     PG_MARK(kMlpFc);
-    PG_HIP(gemm(HB.p, I, w.c_proj_mlp_w, w.c_proj_mlp_b, X.p, C, C, I, pgk::GEMM_RESID, next_g, next_b, cut));
+    PG_HIP(gemm(HB.p, I, w.c_proj_mlp_w, w.c_proj_mlp_b, X.p, C, C, I, pgk::GEMM_RESID, next_g, next_b, cut, 0,
+                hw.c_proj_mlp, hw.c_proj_mlp_mul, hw.hidden, 0.0f, next_norm));
     PG_MARK(kMlpProj);
   }
   if (all_logits_dst) {
@@ -1030,6 +1121,7 @@ pg_status pg_gpt2_create(const pg_gpt2_config* config, const pg_gpt2_weights_vie
     bool ok = false;
     ~Guard() {
       if (!ok && m->arena) (void)hipFree(m->arena);
+      if (!ok && m->half_arena) (void)hipFree(m->half_arena);
     }
   } guard{m.get()};
 
@@ -1174,6 +1266,7 @@ pg_status pg_gpt2_create(const pg_gpt2_config* config, const pg_gpt2_weights_vie
     m->persistent = shape_ok && opts.decode_path != PG_DECODE_KERNELS;
     m->persistent_grid = grid;
   }
+  if ((s = make_half_form(m.get()))) return s;
   guard.ok = true;
   guard2.ok = true;
   *out = m.release();
@@ -1184,6 +1277,7 @@ void pg_model_destroy(pg_model* m) {
   if (!m) return;
   if (hipSetDevice(m->device) == hipSuccess) {
     if (m->arena) (void)hipFree(m->arena);
+    if (m->half_arena) (void)hipFree(m->half_arena);
     if (m->d_layers) (void)hipFree(m->d_layers);
     m->stack.reset();
   }

@@ -263,6 +263,13 @@ struct GemmArgs {
   // Which of A, C and ln_out are in cut form (FORM_CUT).  launch_gemm refuses what gemm_takes_cut does not
   // name; a_cut decides the kernel, the other two may go with it only.
   int a_cut = 0, c_cut = 0, ln_cut = 0;
+  // a_unscale > 0: A is in half form (FORM_HALF), its values 1 / a_unscale times what they stand for, and W's half form is
+  // w_half (launch_half_rows), of w_half_parts f16 numbers a weight.  GEMM_GELU then writes C in half form, times c_scale,
+  // and ln_out is in half form, times ln_scale; no other form goes with it.  Powers of two.
+  const void* w_half = nullptr;
+  const float* w_half_mul = nullptr;
+  int w_half_parts = 0;
+  float a_unscale = 0.0f, c_scale = 0.0f, ln_scale = 0.0f;
   // Tunable: a GEMM whose M x N leaves CUs idle is cut along K into about this many work items
   // per CU (gemm_split_parts).
   int split_items_per_cu = 3;
@@ -286,8 +293,24 @@ __host__ __device__ inline size_t packed32_index(size_t b, size_t k) {
   return (((k >> 2) * 32 + b) << 2) + (k & 3);
 }
 // How an activation matrix lies in memory: its rows one after the other; packed32_index; or in cut form, as three
-// bf16 numbers per value (store_cut4 in pg_cut.h).
-enum ActForm : int { FORM_ROWS = 0, FORM_PACKED32 = 1, FORM_CUT = 2 };
+// bf16 numbers per value (store_cut4 in pg_cut.h); or in half form, as two f16 numbers per value and a power of two
+// (store_half4 in pg_half.h; 4 * K * cut_rows(M) bytes).
+enum ActForm : int { FORM_ROWS = 0, FORM_PACKED32 = 1, FORM_CUT = 2, FORM_HALF = 3 };
+inline size_t half_floats(size_t M, size_t K) { return (M + 15) / 16 * 16 * K; }
+// LayerNorm of rows to half form, times scale; cols a multiple of 8 up to 4096.
+hipError_t launch_norm_rows_half(const float* src, void* dst, int rows, int cols, const float* g, const float* b, float eps,
+                                 float scale, hipStream_t s);
+// W[rows][cols] as stored (w_bytes 4: f32, 2: bf16, 1: int8 with scales[row]) in half form: two f16 numbers a weight (f32
+// rows) or one, cols a multiple of 32, and what a sum over them is to be multiplied with, mul[rows].  *refused is set (never
+// cleared) where the rows do not allow it (k_half_rows).
+constexpr int kHalfMostExp = 60;
+hipError_t launch_half_rows(const void* W, int w_bytes, const float* scales, size_t rows, int cols, void* to, float* mul,
+                            unsigned* refused, hipStream_t s);
+// *most = max(*most, the largest magnitude that an output of these rows behind a LayerNorm with scale g can have; fold as
+// launch_ln_fold leaves it), and that of the norm's own values.  Bits of floats; infinite where there is no bound.
+hipError_t launch_half_bound(const void* W, int w_bytes, const float* scales, const float* g, const float* fold, size_t rows, int cols,
+                             unsigned* most, hipStream_t s);
+hipError_t launch_half_bound_norm(const float* g, const float* b, int cols, unsigned* most, hipStream_t s);
 // Rows that an activation matrix of M rows in cut form has room for; it takes 6 * K * cut_rows(M) bytes.
 __host__ __device__ inline int cut_rows(int M) { return (M + 15) / 16 * 16; }
 inline size_t cut_floats(size_t M, size_t K) { return (M + 15) / 16 * 16 * K * 3 / 2; }
@@ -314,12 +337,12 @@ hipError_t launch_gemm_grouped(const GemmArgs& a, int epilogue, int tile_rows, c
 hipError_t launch_attn_prefill(const float* qkv, int T, int C, int H, int head_dim, int P,
                                float* kcache, float* vcache, float* out, float* scratch, int num_cus,
                                hipStream_t s, int nseq = 1, size_t kv_stride = 0, int out_form = 0,
-                               bool f32_cores = false);
+                               bool f32_cores = false, float out_scale = 1.0f);
 // The same with both products on the bf16 matrix cores (pg_attn_cut.hip), head_dim 64, in blocks of one of these shapes:
 // 41, 22, 42, 24 (groups of 32 queries, groups of keys).  attn_cut_shape: the one to take, 0: none.
 int attn_cut_shape(int T, int H, int nseq, int num_cus);
 hipError_t launch_attn_prefill_cut(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, float* out,
-                                   hipStream_t s, int nseq, size_t kv_stride, int out_form, int shape);
+                                   hipStream_t s, int nseq, size_t kv_stride, int out_form, int shape, float out_scale = 1.0f);
 // rows rows; row t is position t % period of its sequence (wpe may be null)
 hipError_t launch_embed_rows(float* x, const float* wte, const float* wpe, const uint32_t* ids,
                              int rows, int C, hipStream_t s, int w_bf16 = 0, int period = 0);

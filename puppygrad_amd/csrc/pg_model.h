@@ -127,6 +127,16 @@ struct pg_model {
   float* lm_w = nullptr;
   float* lm_s = nullptr;
   float* lm_f = nullptr;  // [2 V]: LN_f folded into the lm_head rows (pgk::launch_ln_fold)
+  // The block matrices in half form beside their rows (pgk::launch_half_rows), and what a layer's activations are multiplied
+  // with where they are kept so: powers of two that put the largest value that each can have (pgk::launch_half_bound) at
+  // 2^15 at most.  Empty where the weights do not allow it or there was no memory for them.
+  struct HalfLayer {
+    const void *c_attn, *c_proj, *c_fc, *c_proj_mlp;
+    const float *c_attn_mul, *c_proj_mul, *c_fc_mul, *c_proj_mlp_mul;
+    float norm_1, attn, norm_2, hidden;
+  };
+  char* half_arena = nullptr;
+  std::vector<HalfLayer> half;
   // Set for stack models (pg_stack.h); the GPT-2 fields above are then unused.
   std::shared_ptr<pgh::StackModel> stack;
 };

@@ -13,6 +13,7 @@
 #include <string>
 
 #include "pg_gemm_dev.h"
+#include "pg_half.h"
 #include "pg_internal.h"
 #include "pg_kernels.h"
 #include "pg_wave.h"
@@ -179,6 +180,13 @@ __global__ __launch_bounds__(256) void k_to_cut(const float* x, void* to, int M,
   const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= (size_t)M * K) return;
   pgk::store_cut4(to, pgk::cut_rows(M), i / K, i % K, pgk::f4{x[i], x[i + 1], x[i + 2], x[i + 3]});
+}
+
+// (for the tests: x[M][K] in half form, times scale, K a multiple of 8)
+__global__ __launch_bounds__(256) void k_to_half(const float* x, void* to, int M, int K, float scale) {
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= (size_t)M * K) return;
+  pgk::store_half4(to, pgk::cut_rows(M), i / K, i % K, pgk::f4{x[i], x[i + 1], x[i + 2], x[i + 3]}, scale);
 }
 
 // (for the tests: the sums of pg_wave.h, a wavefront a block)
@@ -425,6 +433,41 @@ pg_status pg_testing_cut_product_dev(int32_t device, void* stream, const float* 
                      cut, (int)rows, (int)in_f);
   PG_HIP(hipGetLastError());
   PG_HIP(pgk::launch_gemm_cut_rows(a, pgk::GEMM_BIAS, {mt, ng, block_rows, parts}, static_cast<hipStream_t>(stream)));
+  return PG_OK;
+}
+
+// x, times scale, in half form through pg_gemm_half.hip: the given tile (pgk::HalfTile), or blocks of 16 mt input rows and `block_rows`
+// rows of W, K in `parts` parts (more than one: the raw parts [parts][rows][out_f] to out, without bias); gelu: with GELU, out
+// in half form times 1.  work: 4 * in_f * (rows rounded up to 16) bytes, as many as W's half form takes, 4 * out_f and 4, each
+// rounded up to 256; its last word says whether W was refused.
+pg_status pg_testing_half_product_dev(int32_t device, void* stream, const float* x, uint64_t rows, uint64_t in_f,
+                                      uint64_t out_f, const void* weight, int32_t storage, const float* scales,
+                                      const float* bias, float* out, float scale, int32_t tile, int32_t parts, int32_t mt,
+                                      int32_t block_rows, int32_t gelu, char* work) {
+  if (!x || !weight || !out || !work || (storage == PG_STORE_INT8) != (scales != nullptr))
+    return pgh::fail(PG_INVALID_INPUT, "null argument");
+  if (rows == 0 || rows > (1u << 20) || in_f < 64 || in_f % 32 != 0 || in_f > pgh::kMaxStagedFloats || out_f < 64 || out_f % 8 != 0 ||
+      out_f > (1u << 20) || parts < 1 || parts > 8)
+    return pgh::fail(PG_INVALID_INPUT, "product: sizes");
+  pg_status s;
+  if ((s = select_device(device))) return s;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+  const int pw = storage == PG_STORE_F32 ? 2 : 1;
+  char* w_half = work + up(in_f * pgk::cut_rows((int)rows) * 4);
+  float* mul = reinterpret_cast<float*>(w_half + up(in_f * out_f * 2 * pw));
+  unsigned* refused = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(mul) + up(out_f * 4));
+  PG_HIP(pgk::launch_fill_zero(reinterpret_cast<float*>(refused), 1, st));
+  PG_HIP(pgk::launch_half_rows(weight, storage == PG_STORE_F32 ? 4 : storage == PG_STORE_BF16 ? 2 : 1, scales, out_f, (int)in_f,
+                               w_half, mul, refused, st));
+  hipLaunchKernelGGL(k_to_half, dim3((unsigned)((rows * in_f / 4 + 255) / 256)), dim3(256), 0, st, x, work, (int)rows, (int)in_f, scale);
+  PG_HIP(hipGetLastError());
+  pgk::GemmArgs a{};
+  a.A = reinterpret_cast<const float*>(work); a.w_half = w_half; a.w_half_mul = mul; a.w_half_parts = pw; a.a_unscale = 1.0f / scale;
+  a.bias = bias; a.C = out; a.M = (int)rows; a.N = (int)out_f; a.K = (int)in_f; a.ldc = (int)out_f;
+  a.ws = out; a.ws_floats = (size_t)parts * rows * out_f;
+  if (gelu) a.c_scale = 1.0f;
+  PG_HIP(pgk::launch_gemm_half_plan(a, gelu ? pgk::GEMM_GELU : pgk::GEMM_BIAS, {tile, parts, mt, block_rows}, st));
   return PG_OK;
 }
 

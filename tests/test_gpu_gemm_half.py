@@ -1,0 +1,183 @@
+"""Products in half form (pg_gemm_half.hip): every tile and block shape by name at its edges, inputs over the range that half form
+holds, weights that it refuses, and the models that take it."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from helpers import DeviceArray, as_bf16
+from puppygrad_amd import Gpt2Config, Gpt2HipConfig, Gpt2Model, _lib, synth
+
+pytestmark = pytest.mark.gpu
+
+STORE = {"f32": _lib.PG_STORE_F32, "bf16": _lib.PG_STORE_BF16, "int8": _lib.PG_STORE_INT8}
+TILE_64x128, TILE_128x128, TILE_128x128_8, TILE_128x256, ROWS = range(5)
+FORMS = [(s, t, 0, 0) for s in STORE for t in (TILE_64x128, TILE_128x128, TILE_128x128_8, TILE_128x256) if s != "f32" or t != TILE_128x256]
+FORMS += [(s, ROWS, mt, rows) for s in STORE for mt in (2, 3, 4) for rows in (8, 16, 24, 32, 40, 48, 56, 64) if mt > 2 or rows <= 32]
+
+
+def up(n):
+    return (n + 255) // 256 * 256
+
+
+def half_product_dev(x, w, bias, scales, scale, tile, parts, mt, rows, gelu=False):
+    """The product, and whether its weights were refused."""
+    f = _lib.load().pg_testing_half_product_dev
+    u, v, i = C.c_uint64, C.c_void_p, C.c_int32
+    f.argtypes, f.restype = [i, v, v, u, u, u, v, i, v, v, v, C.c_float, i, i, i, i, i, v], C.c_int
+    (m, k), n = x.shape, w.shape[0]
+    storage = {np.dtype(np.float32): "f32", np.dtype(np.uint16): "bf16", np.dtype(np.int8): "int8"}[w.dtype]
+    mp = (m + 15) // 16 * 16
+    size = up(4 * k * mp) + up(k * n * (4 if storage == "f32" else 2)) + up(4 * n) + 256
+    # (room for padded rows: NaN, which no result may show)
+    held = [DeviceArray(x), DeviceArray(w, dtype=w.dtype), DeviceArray(np.full(parts * max(m, mp) * n, np.nan, np.float32)), DeviceArray(bias),
+            DeviceArray(np.full(size // 4, np.nan, np.float32))]
+    if scales is not None:
+        held.append(DeviceArray(scales))
+    status = f(0, None, held[0].ptr, m, k, n, held[1].ptr, STORE[storage], held[5].ptr if scales is not None else None, held[3].ptr,
+               held[2].ptr, scale, tile, parts, mt, rows, gelu, held[4].ptr)
+    got, work = held[2].download(), held[4].download()
+    for d in held:
+        d.free()
+    assert status == 0, _lib.load().pg_last_error_message().decode()
+    refused = work.view(np.uint32)[(size - 256) // 4] != 0
+    if gelu:  # back from half form
+        parts_of = got.view(np.float16).reshape(-1)[:2 * n * mp].reshape(n // 8, 2, mp, 8)[:, :, :m].astype(np.float64)
+        return parts_of.sum(1).transpose(1, 0, 2).reshape(m, n), refused
+    got = got[:parts * m * n].reshape(parts, m, n)
+    return (got[0] if parts == 1 else got.sum(0, dtype=np.float64) + bias), refused
+
+
+def operands(m, k, n, storage):
+    rng = np.random.default_rng([m, k, n])
+    x = (rng.standard_normal((m, k)) * 10.0 ** rng.uniform(-3, 1, (m, k))).astype(np.float32)
+    w = (rng.standard_normal((n, k)) * 10.0 ** rng.uniform(-3, 1, (n, 1))).astype(np.float32)
+    b = rng.standard_normal(n).astype(np.float32)
+    if storage == "f32":
+        return x, w, None, w.astype(np.float64), b
+    if storage == "bf16":
+        w = synth.round_bf16(w.reshape(-1)).reshape(w.shape)
+        return x, as_bf16(w), None, w.astype(np.float64), b
+    q, scales = rng.integers(-127, 128, (n, k)).astype(np.int8), np.abs(w[:, 0]) + np.float32(1e-3)
+    return x, q, scales, q * scales[:, None].astype(np.float64), b
+
+
+def bound_of(x, w, b, scale):
+    """f32 sums of K products in any order, their operands off by 2^-23 (of x besides 2^-25 of the scaled unit) and lo lo left
+    out, 2^-22; the bias and an int8 row's scale each rounded once."""
+    want = x @ w.T + b
+    return want, (x.shape[1] + 20) * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T) + 2.0 ** -25 / scale * np.abs(w).sum(1) + 2.0 ** -23 * np.abs(want)
+
+
+# a row, an octet of columns more than a tile, two stages of K; a tile's rows and one more or less on both sides; chains of uneven
+# length, and parts of one stage
+@pytest.mark.parametrize("m,k,n,parts", [(1, 64, 64, 1), (63, 96, 136, 1), (65, 288, 128, 1), (128, 256, 264, 2), (129, 1056, 72, 1),
+                                         (200, 416, 256, 5), (257, 544, 384, 1), (37, 2080, 520, 8)])
+@pytest.mark.parametrize("storage,tile,mt,rows", FORMS)
+def test_forms_at_their_edges(storage, tile, mt, rows, m, k, n, parts):
+    x, w, scales, values, b = operands(m, k, n, storage)
+    got, refused = half_product_dev(x, w, b, scales, 256.0, tile, parts, mt, rows)
+    want, bound = bound_of(x.astype(np.float64), values, b, 256.0)
+    assert not refused and (np.abs(got - want) <= bound).all(), f"{(np.abs(got - want) / bound).max():.2f} of the bound"
+
+
+@pytest.mark.parametrize("storage,tile,mt,rows", [(s, t, 3, 24) for s in STORE for t in (TILE_64x128, TILE_128x128, TILE_128x128_8, TILE_128x256, ROWS)
+                                                  if s != "f32" or t != TILE_128x256])
+def test_every_product_of_the_parts_counts(storage, tile, mt, rows):
+    """Operands of one sign whose second parts are large: left out, one product of them is 2^-12 of the sum."""
+    rng = np.random.default_rng(5)
+    x = (1.0 + 2.0 ** -12 + rng.integers(0, 4, (70, 256)) * 2.0 ** -22).astype(np.float32)
+    w = (1.0 + 2.0 ** -12 + rng.integers(0, 4, (136, 256)) * 2.0 ** -22).astype(np.float32)
+    scales = None
+    if storage == "bf16":
+        w = synth.round_bf16(w.reshape(-1)).reshape(w.shape)
+    stored, values = (as_bf16(w) if storage == "bf16" else w), w.astype(np.float64)
+    if storage == "int8":
+        stored, scales = rng.integers(100, 128, w.shape).astype(np.int8), np.full(len(w), 0.5, np.float32)
+        values = stored * 0.5
+    want = x.astype(np.float64) @ values.T
+    got, _ = half_product_dev(x, stored, np.zeros(len(w), np.float32), scales, 1.0, tile, 1, mt, rows)
+    # (chains of at most 512 products, 2^-24 each; lo lo, 2^-24 here)
+    assert (np.abs(got - want) <= 64 * 2.0 ** -24 * want).all(), (np.abs(got - want) / want).max() * 2.0 ** 24
+
+
+@pytest.mark.parametrize("tile,mt,rows", [(TILE_64x128, 0, 0), (TILE_128x256, 0, 0), (ROWS, 4, 40)])
+def test_gelu_in_half_form(tile, mt, rows):
+    x, w, scales, values, b = operands(77, 96, 136, "bf16")
+    got, _ = half_product_dev(x, w, b, scales, 64.0, tile, 1, mt, rows, gelu=True)
+    want, bound = bound_of(x.astype(np.float64), values, b, 64.0)
+    gelu = 0.5 * want * (1.0 + np.tanh(np.sqrt(2.0 / np.pi) * (want + 0.044715 * want ** 3)))
+    # (its slope is at most 1.13; f32 arithmetic of a few steps; 2^-25 of half form's unit)
+    assert (np.abs(got - gelu) <= 1.13 * bound + 2.0 ** -20 * np.abs(want) + 2.0 ** -24).all()
+
+
+@pytest.mark.parametrize("storage", ["f32", "bf16"])
+def test_weights_that_half_form_refuses(storage):
+    """Values that are not finite; a row too small or too large to be scaled; bf16: a row that spans more than f16 numbers do."""
+    x, _, _, _, b = operands(40, 64, 64, "f32")
+    rng = np.random.default_rng(3)
+    for value, least, refused in ((1.0, 2.0 ** -20, False), (np.inf, 1.0, True), (np.nan, 1.0, True), (2.0 ** 80, 1.0, True),
+                                  (2.0 ** -80, None, True), (1.0, 2.0 ** -45, storage == "bf16"), (0.0, 0.0, False)):
+        w = synth.round_bf16(rng.standard_normal(64 * 64).astype(np.float32)).reshape(64, 64)
+        if least is None or value == 0.0:
+            w[5] = 0.0
+        else:
+            w[5, 9] = np.float32(1.0078125 * least)
+        w[5, 7] = value
+        _, got = half_product_dev(x, as_bf16(w) if storage == "bf16" else w, b, None, 256.0, TILE_64x128, 1, 0, 0)
+        assert got == refused, (value, least)
+
+
+def logits(model, ids):
+    return model.prefill(ids, model.new_kv_cache()).to_host()
+
+
+# the first rows that take the form, tiles that end in the middle, one prompt and several
+@pytest.mark.parametrize("storage,width,batch,n", [("f32", 768, 1, 1026), ("f32", 1280, 1, 257), ("bf16", 1024, 1, 330), ("int8", 1600, 1, 460),
+                                                   ("f32", 1600, 3, 131), ("bf16", 768, 5, 207), ("int8", 768, 2, 700), ("f32", 512, 9, 130)])
+def test_prompts(storage, width, batch, n):
+    cfg = Gpt2Config(vocab_size=300, n_positions=1100, n_embd=width, n_layer=2, n_head=width // 64)
+    w = synth.random_weights(cfg, 0x5EED0B00, perturb=True)
+    model = Gpt2Model.new(cfg, w, Gpt2HipConfig(weight_storage=STORE[storage]))
+    ids = synth.token_ids(batch * n, 0x70C00B00 + n, 300).reshape(batch, n)
+    cache = model.new_kv_cache(batch)
+    got = (model.prefill_batch(ids, cache) if batch > 1 else model.prefill(ids[0], cache)).to_host().reshape(batch, -1)
+    for b in (0, batch - 1):  # the one-sequence kernels form the last token behind a prompt of other products' rows
+        other = model.new_kv_cache()
+        at = min(n - 1, 32)
+        model.prefill([int(t) for t in ids[b, :at]], other)
+        for t in ids[b, at:n - 1]:
+            model.forward_one(int(t), other)
+        want = model.forward_one(int(ids[b, n - 1]), other).to_host()
+        # (the same values, sums of at most 6400 terms in other orders)
+        assert np.linalg.norm(got[b] - want) <= 1e-5 * np.linalg.norm(want)
+
+
+def test_scales_hold_for_models_of_any_size_of_values():
+    """Gains, weights and shifts far from the usual: the bounds move with them."""
+    cfg = Gpt2Config(vocab_size=97, n_positions=400, n_embd=512, n_layer=1, n_head=8)
+    ids = [int(t) for t in synth.token_ids(400, 0x70C00B02, 97)]
+    for gain, weight in ((1e3, 1.0), (1e-4, 1.0), (1.0, 1e-4), (3.0, 30.0)):
+        w = synth.random_weights(cfg, 0x5EED0B02, perturb=True)
+        for blk in w.blocks:
+            blk.ln_1_g, blk.ln_2_g = blk.ln_1_g * np.float32(gain), blk.ln_2_g * np.float32(gain)
+            blk.c_fc_w, blk.c_attn_w = blk.c_fc_w * np.float32(weight), blk.c_attn_w * np.float32(weight / gain)
+        here = Gpt2Model.new(cfg, w, Gpt2HipConfig(weight_storage=STORE["bf16"]))
+        # (the f32 cores' products of the same bf16 values)
+        for blk in w.blocks:
+            for name in ("c_attn_w", "c_proj_w", "c_fc_w", "c_proj_mlp_w"):
+                a = getattr(blk, name)
+                setattr(blk, name, synth.round_bf16(a.reshape(-1)).reshape(a.shape))
+        w.wte = synth.round_bf16(w.wte.reshape(-1)).reshape(w.wte.shape)
+        there = Gpt2Model.new(cfg, w, Gpt2HipConfig(gemm_b9_min_rows=0xffffffff))
+        got, want = logits(here, ids), logits(there, ids)
+        assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want), (gain, weight)
+
+
+def test_weights_without_half_form_are_served_as_before():
+    cfg = Gpt2Config(vocab_size=97, n_positions=400, n_embd=512, n_layer=1, n_head=8)
+    ids = [int(t) for t in synth.token_ids(400, 0x70C00B03, 97)]
+    w = synth.random_weights(cfg, 0x5EED0B03, perturb=True)
+    w.blocks[0].c_fc_b[3] = np.inf
+    got = logits(Gpt2Model.new(cfg, w, Gpt2HipConfig(weight_storage=STORE["bf16"])), ids)
+    assert got.shape == (97,)
