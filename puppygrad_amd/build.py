@@ -12,7 +12,7 @@ LIB_PATH = PKG_DIR / "libpuppygrad_hip.so"
 # Development build with the persistent decode kernel's in-kernel timestamps compiled in
 # (python -m puppygrad_amd.build --stamps; read by puppygrad_amd.decode_stamps).
 STAMPS_LIB_PATH = PKG_DIR / "libpuppygrad_hip_stamps.so"
-SOURCES = ["pg_kernels.hip", "pg_decode.hip", "pg_prefill.hip", "pg_gemm_cut.hip", "pg_gemm_rows.hip", "pg_gemm_half.hip", "pg_attn_cut.hip", "pg_ops_dev.hip", "pg_sample.hip",
+SOURCES = ["pg_kernels.hip", "pg_decode.hip", "pg_prefill.hip", "pg_gemm_cut.hip", "pg_gemm_rows.hip", "pg_gemm_half.hip", "pg_attn_cut.hip", "pg_attn_half.hip", "pg_ops_dev.hip", "pg_sample.hip",
            "pg_mixers.hip", "pg_latent.hip", "pg_moe.hip", "pg_host.cpp", "pg_stack.cpp", "pg_assets.cpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

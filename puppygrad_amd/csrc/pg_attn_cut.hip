@@ -1,6 +1,5 @@
 // Causal attention of prompts on the bf16 matrix cores.
 #include "pg_gemm_dev.h"
-#include "pg_half.h"
 
 namespace pgk {
 namespace {
@@ -27,11 +26,11 @@ __device__ __forceinline__ f16v mfma16(const u4v& a, const u4v& b, const f16v& c
 // It appends K and V to the cache panels.  Grid: x = head, y = block of queries, longest rows first, z = sequence.
 // 512 tokens x 32, 25 heads: 490 us by k_attn_prefill64, here 265; error against f64 3.9 and 3.6 10^-7.  What is left: per tile
 // and wavefront 1536 clocks of matrix and about 1500 of vector instructions (128 queries a block), and two barriers.
-template <int QG, int KG, int FORM>
+template <int QG, int KG, bool CUT>
 __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_cut(const float* __restrict__ qkv, int T, int C, int P,
                                                                       float* __restrict__ kcache,
                                                                       float* __restrict__ vcache,
-                                                                      float* __restrict__ out, size_t kv_stride, float out_scale) {
+                                                                      float* __restrict__ out, size_t kv_stride) {
   constexpr int NW = QG * KG;
   constexpr int KSTR = 32 * 16 + 16;            // bytes of an octet of dims of 32 keys, padded
   constexpr int KPART = 8 * KSTR, VPART = 4 * 64 * 16;
@@ -274,22 +273,19 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_cut(const floa
       }
       r = t / l;
     }
-    if constexpr (FORM == FORM_CUT) store_cut4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r);
-    else if constexpr (FORM == FORM_HALF) store_half4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r, out_scale);
+    if constexpr (CUT) store_cut4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r);
     else *reinterpret_cast<f4*>(out + row * C + h * 64 + d) = r;
   }
 }
 
 template <int QG, int KG>
 void start(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, float* out, hipStream_t s, int nseq,
-           size_t kv_stride, int out_form, float out_scale) {
+           size_t kv_stride, int out_form) {
   const dim3 grid(H, (T + 32 * QG - 1) / (32 * QG), nseq), block(64 * QG * KG);
-#define PG_START(FORM) \
-  hipLaunchKernelGGL((k_attn_prefill_cut<QG, KG, FORM>), grid, block, 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, out_scale)
-  if (out_form == FORM_CUT) PG_START(FORM_CUT);
-  else if (out_form == FORM_HALF) PG_START(FORM_HALF);
-  else PG_START(FORM_ROWS);
-#undef PG_START
+  if (out_form == FORM_CUT)
+    hipLaunchKernelGGL((k_attn_prefill_cut<QG, KG, true>), grid, block, 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride);
+  else
+    hipLaunchKernelGGL((k_attn_prefill_cut<QG, KG, false>), grid, block, 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride);
 }
 }  // namespace
 
@@ -313,11 +309,11 @@ int attn_cut_shape(int T, int H, int nseq, int num_cus) {
 }
 
 hipError_t launch_attn_prefill_cut(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, float* out,
-                                   hipStream_t s, int nseq, size_t kv_stride, int out_form, int shape, float out_scale) {
-  if (shape == 41) start<4, 1>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, out_form, out_scale);
-  else if (shape == 22) start<2, 2>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, out_form, out_scale);
-  else if (shape == 42) start<4, 2>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, out_form, out_scale);
-  else if (shape == 24) start<2, 4>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, out_form, out_scale);
+                                   hipStream_t s, int nseq, size_t kv_stride, int out_form, int shape) {
+  if (shape == 41) start<4, 1>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, out_form);
+  else if (shape == 22) start<2, 2>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, out_form);
+  else if (shape == 42) start<4, 2>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, out_form);
+  else if (shape == 24) start<2, 4>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, out_form);
   else return hipErrorInvalidValue;
   return hipGetLastError();
 }

@@ -515,7 +515,7 @@ pg_status make_half_form(pg_model* m) {
   const size_t rows[4] = {3 * C, C, I, C}, cols[4] = {C, C, C, I};
   size_t layer = 0;
   for (int i = 0; i < 4; ++i) layer += up(rows[i] * cols[i] * 2 * pw) + up(rows[i] * 4);
-  constexpr int kBounds = 4;  // of a layer: both norms, values, hidden
+  constexpr int kBounds = 6;  // of a layer: both norms, hidden, queries, keys, values
   const size_t words = up((g.L * kBounds + 1) * 4);
   if (hipMalloc(&m->half_arena, g.L * layer + words) != hipSuccess) {
     (void)hipGetLastError();
@@ -540,13 +540,14 @@ pg_status make_half_form(pg_model* m) {
       at += up(rows[i] * 4);
       PG_HIP(pgk::launch_half_rows(mats[i], wb, scales[i], rows[i], (int)cols[i], to[i], mul[i], refused, nullptr));
     }
-    m->half[l] = pg_model::HalfLayer{to[0], to[1], to[2], to[3], mul[0], mul[1], mul[2], mul[3], 0, 0, 0, 0};
+    m->half[l] = pg_model::HalfLayer{to[0], to[1], to[2], to[3], mul[0], mul[1], mul[2], mul[3], 0, 0, 0, {}};
     unsigned* b = bounds + l * kBounds;
     PG_HIP(pgk::launch_half_bound_norm(w.ln_1_g, w.ln_1_b, (int)C, b, nullptr));
     PG_HIP(pgk::launch_half_bound_norm(w.ln_2_g, w.ln_2_b, (int)C, b + 1, nullptr));
-    const char* values = reinterpret_cast<const char*>(w.c_attn_w) + 2 * C * C * wb;  // (an average of values is no larger than they are)
-    PG_HIP(pgk::launch_half_bound(values, wb, w.c_attn_s ? w.c_attn_s + 2 * C : nullptr, w.ln_1_g, w.c_attn_f + 4 * C, C, (int)C, b + 2, nullptr));
-    PG_HIP(pgk::launch_half_bound(w.c_fc_w, wb, w.c_fc_s, w.ln_2_g, w.c_fc_f, I, (int)C, b + 3, nullptr));  // (|gelu(x)| <= |x|)
+    PG_HIP(pgk::launch_half_bound(w.c_fc_w, wb, w.c_fc_s, w.ln_2_g, w.c_fc_f, I, (int)C, b + 2, nullptr));  // (|gelu(x)| <= |x|)
+    for (size_t part = 0; part < 3; ++part)  // (an average of values is no larger than they are)
+      PG_HIP(pgk::launch_half_bound(reinterpret_cast<const char*>(w.c_attn_w) + part * C * C * wb, wb, w.c_attn_s ? w.c_attn_s + part * C : nullptr,
+                                    w.ln_1_g, w.c_attn_f + 2 * part * C, C, (int)C, b + 3 + part, nullptr));
   }
   std::vector<unsigned> got(g.L * kBounds + 1);
   PG_HIP(hipMemcpy(got.data(), bounds, got.size() * 4, hipMemcpyDeviceToHost));
@@ -562,8 +563,9 @@ pg_status make_half_form(pg_model* m) {
   };
   for (size_t l = 0; l < g.L; ++l) {
     pg_model::HalfLayer& w = m->half[l];
-    w.norm_1 = scale(got[l * kBounds]), w.norm_2 = scale(got[l * kBounds + 1]);
-    w.attn = scale(got[l * kBounds + 2]), w.hidden = scale(got[l * kBounds + 3]);
+    const unsigned* b = got.data() + l * kBounds;
+    w.norm_1 = scale(b[0]), w.norm_2 = scale(b[1]), w.hidden = scale(b[2]);
+    w.attn = {scale(b[3]), scale(b[4]), scale(b[5])};
   }
   if (!ok) {
     m->half.clear();
@@ -598,7 +600,7 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
   // the projections' inputs (XN, ATT, HB) in half form or in cut form
   const bool cut = !c->drawn && takes_cut_form(m, n);
   const bool half = !cut && !c->drawn && takes_half_form(m, n);
-  const int form_of = half ? pgk::FORM_HALF : cut ? pgk::FORM_CUT : pgk::FORM_ROWS;
+  const int form_of = cut ? pgk::FORM_CUT : pgk::FORM_ROWS;
   {
     auto form = [&](size_t cols) { return cut ? std::max(n * cols, pgk::cut_floats(n, cols)) : half ? pgk::half_floats(n, cols) : n * cols; };
     auto up = [](size_t v) { return (v + 63) / 64 * 64; };  // 256-byte boundaries
@@ -679,12 +681,15 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
     PG_HIP(gemm(XN.p, C, w.c_attn_w, w.c_attn_b, QKV.p, 3 * C, 3 * C, C, pgk::GEMM_BIAS, nullptr, nullptr, cut, 0,
                 hw.c_attn, hw.c_attn_mul, hw.norm_1));
     PG_MARK(kQkv);
-    PG_HIP(pgk::launch_attn_prefill(QKV.p, Ts, C, H, hd, P, c->k_panel(l, b), c->v_panel(l, b),
-                                    ATT.p, SCR.p, m->num_cus, s, (int)nb, g.H * g.P * g.hd(),
-                                    form_of, c->drawn, hw.attn));
+    if (half)
+      PG_HIP(pgk::launch_attn_prefill_half(QKV.p, Ts, C, H, P, c->k_panel(l, b), c->v_panel(l, b), ATT.p, s, (int)nb,
+                                           g.H * g.P * g.hd(), hw.attn, pgk::attn_half_shape(Ts, H, (int)nb, m->num_cus)));
+    else
+      PG_HIP(pgk::launch_attn_prefill(QKV.p, Ts, C, H, hd, P, c->k_panel(l, b), c->v_panel(l, b),
+                                      ATT.p, SCR.p, m->num_cus, s, (int)nb, g.H * g.P * g.hd(), form_of, c->drawn));
     PG_MARK(kAttention);
     PG_HIP(gemm(ATT.p, C, w.c_proj_w, w.c_proj_b, X.p, C, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b, cut, 0,
-                hw.c_proj, hw.c_proj_mul, hw.attn, 0.0f, hw.norm_2));
+                hw.c_proj, hw.c_proj_mul, hw.attn.v, 0.0f, hw.norm_2));
     PG_MARK(kAttnProj);
     PG_HIP(gemm(XN.p, C, w.c_fc_w, w.c_fc_b, HB.p, I, I, C, pgk::GEMM_GELU, nullptr, nullptr, cut, cut,
                 hw.c_fc, hw.c_fc_mul, hw.norm_2, hw.hidden));

@@ -337,12 +337,21 @@ hipError_t launch_gemm_grouped(const GemmArgs& a, int epilogue, int tile_rows, c
 hipError_t launch_attn_prefill(const float* qkv, int T, int C, int H, int head_dim, int P,
                                float* kcache, float* vcache, float* out, float* scratch, int num_cus,
                                hipStream_t s, int nseq = 1, size_t kv_stride = 0, int out_form = 0,
-                               bool f32_cores = false, float out_scale = 1.0f);
+                               bool f32_cores = false);
 // The same with both products on the bf16 matrix cores (pg_attn_cut.hip), head_dim 64, in blocks of one of these shapes:
 // 41, 22, 42, 24 (groups of 32 queries, groups of keys).  attn_cut_shape: the one to take, 0: none.
 int attn_cut_shape(int T, int H, int nseq, int num_cus);
 hipError_t launch_attn_prefill_cut(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, float* out,
-                                   hipStream_t s, int nseq, size_t kv_stride, int out_form, int shape, float out_scale = 1.0f);
+                                   hipStream_t s, int nseq, size_t kv_stride, int out_form, int shape);
+// The same on the f16 matrix cores (pg_attn_half.hip): out in half form times scales.v; the scales are powers of two with which no
+// query, key or value is past 2^15.  Shapes (groups of 32 queries, groups of
+// keys) 41, 22, 24, 18, 14; attn_half_shape: the one to take.
+struct HalfScales {
+  float q, k, v;
+};
+int attn_half_shape(int T, int H, int nseq, int num_cus);
+hipError_t launch_attn_prefill_half(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, void* out,
+                                    hipStream_t s, int nseq, size_t kv_stride, const HalfScales& scales, int shape);
 // rows rows; row t is position t % period of its sequence (wpe may be null)
 hipError_t launch_embed_rows(float* x, const float* wte, const float* wpe, const uint32_t* ids,
                              int rows, int C, hipStream_t s, int w_bf16 = 0, int period = 0);

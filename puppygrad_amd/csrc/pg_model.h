@@ -133,7 +133,8 @@ struct pg_model {
   struct HalfLayer {
     const void *c_attn, *c_proj, *c_fc, *c_proj_mlp;
     const float *c_attn_mul, *c_proj_mul, *c_fc_mul, *c_proj_mlp_mul;
-    float norm_1, attn, norm_2, hidden;
+    float norm_1, norm_2, hidden;
+    pgk::HalfScales attn;  // queries, keys, values (and what attention makes of them)
   };
   char* half_arena = nullptr;
   std::vector<HalfLayer> half;

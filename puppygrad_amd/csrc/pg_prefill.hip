@@ -7,7 +7,6 @@
 // the reference's token-by-token prefill (rust.rs:910-927), which the reference
 // itself checks against forward() at 1e-5 (rust.rs:1900-1913).
 #include "pg_gemm_dev.h"
-#include "pg_half.h"
 #include "pg_mixers.h"
 #include "pg_wave.h"
 
@@ -976,12 +975,12 @@ __device__ __forceinline__ float other_half(float x) {
   return (threadIdx.x & 32) ? __uint_as_float(r.x) : __uint_as_float(r.y);
 }
 
-// NWV: wavefronts per block.  FORM: how out lies (ActForm; FORM_HALF: times out_scale).
-template <int NWV, int FORM>
+// NWV: wavefronts per block.  CUT: out is in cut form.
+template <int NWV, bool CUT>
 __global__ __launch_bounds__(64 * NWV) void k_attn_prefill64(const float* __restrict__ qkv, int T,
                                                         int C, int P, float* __restrict__ kcache,
                                                         float* __restrict__ vcache,
-                                                        float* __restrict__ out, size_t kv_stride, float out_scale) {
+                                                        float* __restrict__ out, size_t kv_stride) {
   // blockIdx.z: the sequence (T rows of qkv and out each, panels kv_stride apart)
   qkv += (size_t)blockIdx.z * T * 3 * C;
   kcache += (size_t)blockIdx.z * kv_stride;
@@ -1190,8 +1189,7 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_prefill64(const float* __rest
         for (int w = 0; w < NWV; ++w) sum += reinterpret_cast<float (*)[KT + 1]>(Vs[w])[d + e][l32];
         r[e] = sum * inv;
       }
-      if constexpr (FORM == FORM_CUT) store_cut4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r);
-      else if constexpr (FORM == FORM_HALF) store_half4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r, out_scale);
+      if constexpr (CUT) store_cut4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r);
       else *reinterpret_cast<f4*>(out + row * C + h * 64 + d) = r;
     }
   }
@@ -1792,11 +1790,11 @@ hipError_t launch_gemm_form(const GemmArgs& a, int epi, int num_cus, hipStream_t
 
 hipError_t launch_attn_prefill(const float* qkv, int T, int C, int H, int head_dim, int P,
                                float* kcache, float* vcache, float* out, float* scratch, int num_cus,
-                               hipStream_t s, int nseq, size_t kv_stride, int out_form, bool f32_cores, float out_scale) {
+                               hipStream_t s, int nseq, size_t kv_stride, int out_form, bool f32_cores) {
   if (nseq < 1 || nseq > 65535 || out_form == FORM_PACKED32 || (out_form && head_dim != 64)) return hipErrorInvalidValue;
   if (head_dim == 64) {
     if (const int shape = f32_cores ? 0 : attn_cut_shape(T, H, nseq, num_cus))
-      return launch_attn_prefill_cut(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, out_form, shape, out_scale);
+      return launch_attn_prefill_cut(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, out_form, shape);
     const int qblocks = (T + 31) / 32;
     // Eight wavefronts share a query block's key tiles.  Several sequences of up to 512 tokens
     // are more blocks of at most 16 tiles each: four wavefronts (half the LDS, two blocks to a
@@ -1804,18 +1802,12 @@ hipError_t launch_attn_prefill(const float* qkv, int T, int C, int H, int head_d
     // pg_attn_cut.hip).
     const dim3 grid(H, qblocks, nseq);
     const bool four = nseq >= 2 && T <= 512;
-#define PG_ATTN(NWV)                                                                                                        \
-  if (out_form == FORM_CUT)                                                                                                 \
-    hipLaunchKernelGGL((k_attn_prefill64<NWV, FORM_CUT>), grid, dim3(64 * NWV), 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, out_scale); \
-  else if (out_form == FORM_HALF)                                                                                           \
-    hipLaunchKernelGGL((k_attn_prefill64<NWV, FORM_HALF>), grid, dim3(64 * NWV), 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, out_scale); \
-  else                                                                                                                      \
-    hipLaunchKernelGGL((k_attn_prefill64<NWV, FORM_ROWS>), grid, dim3(64 * NWV), 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, out_scale)
-    if (four) {
-      PG_ATTN(4);
-    } else {
-      PG_ATTN(8);
-    }
+#define PG_ATTN(NWV, CUT) \
+  hipLaunchKernelGGL((k_attn_prefill64<NWV, CUT>), grid, dim3(64 * NWV), 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride)
+    if (four && out_form == FORM_CUT) PG_ATTN(4, true);
+    else if (four) PG_ATTN(4, false);
+    else if (out_form == FORM_CUT) PG_ATTN(8, true);
+    else PG_ATTN(8, false);
 #undef PG_ATTN
   } else {
     // (test-sized models: one launch per sequence, all using the same scratch in turn)
