@@ -106,9 +106,9 @@ typedef struct pg_hip_options {
                                        run on the bf16 matrix cores with both operands cut into
                                        three bf16 parts, or on the f16 ones in two f16 parts,
                                        where the planner finds enough tiles
-                                       (0xffffffff: never).  Default: 65, and 33 to 64 rows
-                                       where activations are better kept cut; set, 65 too, it
-                                       is the bound for both.  65 to 128 rows are not kept cut
+                                       (0xffffffff: never).  Default: 65, and up to 64 rows
+                                       where activations are better kept in parts; set, 65 too,
+                                       it is the bound for all.  65 to 128 rows are not kept so
                                        at any setting */
   uint32_t seq_gemm_min_tokens;     /* prompts of at least this many tokens take the GEMM
                                        prefill, shorter ones run token by token through the

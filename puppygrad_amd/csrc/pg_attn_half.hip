@@ -26,7 +26,7 @@ __device__ __forceinline__ void halves8(f4 a, f4 b, float mul, u4v (&part)[2]) {
 // causal_self_attention (src/models/gpt2/rust.rs:1580-1659) for head_dim 64 over qkv[T][3C], as k_attn_prefill_cut
 // (pg_attn_cut.hip) with two f16 numbers a value for three bf16 numbers: three products of the parts for six, half of the
 // cutting.  Q, K and V are scaled by powers of two, sq, sk and sv, with which none can be past 2^15 (half_bounds); the weights,
-// whose largest is 1, by 2^7, and out is in half form times sv, as the projection behind it wants it.  Scores, maxima, weights
+// whose largest is 1, by 2^7.  FORM: out is in half form times sv, or in cut form, as the projection behind it wants it.  Scores, maxima, weights
 // and sums are f32.  A tile's products are chains of their own that are added to the output: over 1000 keys one chain of f32
 // roundings is off by more than all else in here.
 // A block holds QG x 32 queries: the QG wavefronts of a key group share a tile of 32 keys that they have cut once, in operand
@@ -38,7 +38,7 @@ __device__ __forceinline__ void halves8(f4 a, f4 b, float mul, u4v (&part)[2]) {
 // It appends K and V to the cache panels.  512 tokens x 32, 25 heads 231 us (k_attn_prefill_cut) -> 177; 1000 tokens 42 -> 32; 1024
 // tokens, 12 heads 29.5 (k_attn_prefill64) -> 23.6.  Error against f64 1.4 to 1.8 10^-7, as on the f32 cores (1.2 to 1.9).
 // What bounds it: per tile and wavefront 768 clocks of matrix instructions and about 1100 of vector ones.  Grid: x = head, y = block of queries, longest rows first, z = sequence.
-template <int QG, int KG>
+template <int QG, int KG, int FORM>
 __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const float* __restrict__ qkv, int T, int C, int P,
                                                                       float* __restrict__ kcache,
                                                                       float* __restrict__ vcache,
@@ -245,29 +245,35 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const flo
   __syncthreads();
   if (qi >= T) return;
   // the wavefronts of a query group share its 64 dims; lane: query l32, half of the wavefront's share
-  const float inv = 1.0f / L;
+  const float inv = 1.0f / L, inv_rest = fmaf(-L, inv, 1.0f);
   const size_t row = (size_t)blockIdx.z * T + qi;
   constexpr int ND = 64 / KG / 2;
 #pragma unroll
   for (int j = 0; j < ND; j += 4) {
     const int d = 2 * ND * kg + ND * half + j;
-    f4 r;
+    f4 r, rest;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       float sum = 0.0f;
 #pragma unroll
       for (int g = 0; g < KG; ++g) sum += reinterpret_cast<float (*)[33]>(lds + (g * QG + qg) * MERGE)[d + e][l32];
       r[e] = sum * inv;
+      rest[e] = fmaf(sum, inv, -r[e]) + r[e] * inv_rest;  // (what f32 rounds away: half form keeps some of it)
     }
-    store_half4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r, 1.0f);  // (times sv, as the values were)
+    // (times sv, as the values were)
+    if constexpr (FORM == FORM_HALF) store_half4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r, rest, 1.0f);
+    else store_cut4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r * (1.0f / sv));
   }
 }
 
 template <int QG, int KG>
 hipError_t start(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, void* out, hipStream_t s, int nseq,
-                 size_t kv_stride, const HalfScales& f) {
+                 size_t kv_stride, const HalfScales& f, int out_form) {
   const dim3 grid(H, (T + 32 * QG - 1) / (32 * QG), nseq), block(64 * QG * KG);
-  hipLaunchKernelGGL((k_attn_prefill_half<QG, KG>), grid, block, 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, f.q, f.k, f.v);
+  if (out_form == FORM_HALF)
+    hipLaunchKernelGGL((k_attn_prefill_half<QG, KG, FORM_HALF>), grid, block, 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, f.q, f.k, f.v);
+  else
+    hipLaunchKernelGGL((k_attn_prefill_half<QG, KG, FORM_CUT>), grid, block, 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, f.q, f.k, f.v);
   return hipGetLastError();
 }
 }  // namespace
@@ -290,14 +296,14 @@ int attn_half_shape(int T, int H, int nseq, int num_cus) {
 }
 
 hipError_t launch_attn_prefill_half(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, void* out,
-                                    hipStream_t s, int nseq, size_t kv_stride, const HalfScales& f, int shape) {
-  if (nseq < 1 || nseq > 65535 || (reinterpret_cast<uintptr_t>(out) & 15)) return hipErrorInvalidValue;
+                                    hipStream_t s, int nseq, size_t kv_stride, const HalfScales& f, int shape, int out_form) {
+  if ((out_form != FORM_HALF && out_form != FORM_CUT) || nseq < 1 || nseq > 65535 || (reinterpret_cast<uintptr_t>(out) & 15)) return hipErrorInvalidValue;
   switch (shape) {
-    case 41: return start<4, 1>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, f);
-    case 22: return start<2, 2>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, f);
-    case 24: return start<2, 4>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, f);
-    case 18: return start<1, 8>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, f);
-    case 14: return start<1, 4>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, f);
+    case 41: return start<4, 1>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, f, out_form);
+    case 22: return start<2, 2>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, f, out_form);
+    case 24: return start<2, 4>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, f, out_form);
+    case 18: return start<1, 8>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, f, out_form);
+    case 14: return start<1, 4>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, f, out_form);
     default: return hipErrorInvalidValue;
   }
 }

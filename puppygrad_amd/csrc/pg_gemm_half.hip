@@ -54,6 +54,19 @@ __device__ __forceinline__ void vm_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// GELU of sum + bias, four columns of a row, with what f32 rounds away on the way.
+__device__ __forceinline__ void store_gelu(void* to, int mp, size_t m, size_t n, f4 sum, f4 bias, float scale) {
+  const f4 c = bias + sum, b = c - sum, c_rest = (bias - b) + (sum - (c - b));
+  f4 y, rest;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float r;
+    y[e] = gelu_tanh(c[e], c_rest[e], r);
+    rest[e] = r;
+  }
+  store_half4(to, mp, m, n, y, rest, scale);
+}
+
 // WM x WN wavefronts, each on MB x NB blocks of 32 x 32.  The operands are turned round: lane (l, half) of the first holds
 // columns 8 half .. 8 half + 7 of row l of W, of the second those of input row l, so that the result's lane is a row
 // of C and its values four by four neighbouring columns.  PW: parts of a weight (2: f32 rows).  K runs in stages of KT
@@ -250,19 +263,19 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
           *reinterpret_cast<f4*>(a.ws + ((size_t)blockIdx.y * a.M + m) * a.N + n) = c;
           continue;
         }
+        if constexpr (EPI == GEMM_GELU) {
+          store_gelu(a.C, mp, (size_t)m, (size_t)n, c, bias, a.c_scale);
+          continue;
+        }
         c += bias;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (EPI == GEMM_GELU) c[e] = gelu_tanh(c[e]);
         if (EPI == GEMM_RESID) c += *reinterpret_cast<const f4*>(a.resid + (size_t)m * a.ldc + n);
-        if constexpr (EPI == GEMM_GELU) store_half4(a.C, mp, (size_t)m, (size_t)n, c, a.c_scale);
-        else *reinterpret_cast<f4*>(a.C + (size_t)m * a.ldc + n) = c;
+        *reinterpret_cast<f4*>(a.C + (size_t)m * a.ldc + n) = c;
       }
     }
 }
 
 // ---- some tens to some hundreds of rows --------------------------------------------------------
-// A block owns 16 MT input rows (blockIdx.z) and up to 16 NG rows of W (a.rows_per_block of them, a multiple of eight); its
+// A block owns 16 MT input rows and up to 16 NG rows of W (a.rows_per_block of them, a multiple of eight); its
 // eight wavefronts take the steps of 32 columns in turn, operands from L2 straight to registers, and the eight partial tiles
 // are added through LDS.  gridDim.y > 1: K is cut over blocks as well, raw tiles go to a.ws[part][M][N].  As k_gemm_cut_rows
 // (pg_gemm_rows.hip), with 4 bytes per input value for 6, and rows of W that need no turn through LDS and no cut.
@@ -273,10 +286,11 @@ __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
   __shared__ __attribute__((aligned(16))) float slab[8][16 * MT * CSTR];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int i16 = lane & 15, kq = lane >> 4;
+  const int part = (int)blockIdx.y, parts = (int)gridDim.y;
   const int n0 = (int)blockIdx.x * a.rows_per_block, n1 = min(n0 + a.rows_per_block, a.N);
   const int m0 = (int)blockIdx.z * 16 * MT;
   const int mp = cut_rows(a.M);
-  const int piece = (int)blockIdx.y * 8 + wave, pieces = (int)gridDim.y * 8;
+  const int piece = part * 8 + wave, pieces = parts * 8;
   const int steps_all = a.K / 32;
   const int steps = piece < steps_all ? (steps_all - piece + pieces - 1) / pieces : 0;
 
@@ -304,7 +318,7 @@ __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
     const bool live = idx < ITEMS && m < a.M && n < n1;
     ebias[q] = eres[q] = emul[q] = f4{0.f, 0.f, 0.f, 0.f};
     if (live) emul[q] = *reinterpret_cast<const f4*>(a.w_half_mul + n) * a.a_unscale;
-    if (gridDim.y > 1) continue;
+    if (parts > 1) continue;
     if (live && a.bias) ebias[q] = *reinterpret_cast<const f4*>(a.bias + n);
     if (live && EPI == GEMM_RESID) eres[q] = *reinterpret_cast<const f4*>(a.resid + (size_t)m * a.ldc + n);
   }
@@ -384,36 +398,62 @@ __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
     const int idx = tid + 512 * q, mr = row_of(idx), nl = col_of(idx);
     const int m = m0 + mr, n = n0 + nl;
     if (idx >= ITEMS || m >= a.M || n >= n1) continue;
-    f4 part[8];
+    f4 w8[8];
 #pragma unroll
-    for (int w = 0; w < 8; ++w) part[w] = *reinterpret_cast<const f4*>(slab[w] + mr * CSTR + nl);
-    const f4 sum = (((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]))) * emul[q];
-    if (gridDim.y > 1) {
-      *reinterpret_cast<f4*>(a.ws + ((size_t)blockIdx.y * a.M + m) * a.N + n) = sum;
+    for (int w = 0; w < 8; ++w) w8[w] = *reinterpret_cast<const f4*>(slab[w] + mr * CSTR + nl);
+    const f4 sum = (((w8[0] + w8[1]) + (w8[2] + w8[3])) + ((w8[4] + w8[5]) + (w8[6] + w8[7]))) * emul[q];
+    if (parts > 1) {
+      *reinterpret_cast<f4*>(a.ws + ((size_t)part * a.M + m) * a.N + n) = sum;
+      continue;
+    }
+    if (EPI == GEMM_GELU) {
+      store_gelu(a.C, mp, (size_t)m, (size_t)n, sum, ebias[q], a.c_scale);
       continue;
     }
     f4 c = ebias[q] + sum;
-    if (EPI == GEMM_GELU) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) c[e] = gelu_tanh(c[e]);
-      store_half4(a.C, mp, (size_t)m, (size_t)n, c, a.c_scale);
-      continue;
-    }
     if (EPI == GEMM_RESID) c += eres[q];
     *reinterpret_cast<f4*>(a.C + (size_t)m * a.ldc + n) = c;
   }
 }
 
 // ---- norms -------------------------------------------------------------------------------------
+// A norm's values are worked out past f32 where they are cut: half form drops a bit of a f32 value in four, 4.4 10^-8, as much as
+// the roundings of (x - mean) / sigma g + b in f32 cost; so cut, they are as far off as f32 values were.
+struct Norm {
+  double mean, inv;
+  __device__ __forceinline__ Norm(float sum, float squares, int n, float eps)
+      : mean((double)sum / n) {
+    const double v = (double)squares / n + (double)eps;
+    const double y = (double)(1.0f / sqrtf((float)v));
+    inv = y * (1.5 - 0.5 * v * y * y);  // (one Newton step of the root)
+  }
+  // four columns of a row, part by part `stride` bytes apart: half form (PX 2), times scale, or cut form (3)
+  template <int PX>
+  __device__ __forceinline__ void store(char* at, size_t stride, f4 c, f4 g, f4 b, float scale) const {
+    double o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = ((double)c[e] - mean) * inv * (double)g[e] + (double)b[e];
+    unsigned ab[3], cd[3];
+    if constexpr (PX == 2) {
+      halves2(o[0] * (double)scale, o[1] * (double)scale, ab[0], ab[1]);
+      halves2(o[2] * (double)scale, o[3] * (double)scale, cd[0], cd[1]);
+    } else {
+      cut_safe2((float)o[0], (float)o[1], ab);
+      cut_safe2((float)o[2], (float)o[3], cd);
+    }
+#pragma unroll
+    for (int p = 0; p < PX; ++p) *reinterpret_cast<u2v*>(at + p * stride) = u2v{ab[p], cd[p]};
+  }
+};
 // Rows of N values to LayerNorm in half form (layer_norm_in_place, cpu.rs:119-143: mean, biased variance in a second pass,
 // eps inside the root), a wavefront a row, four rows a block: the 16-byte pieces of four rows lie next to each other in half
 // form, and the block writes them so, through LDS.  PARTS: the row is first put together from the parts of a cut K, bias and
 // residual, and written to a.C; otherwise it is read from there.  NQ: 256 NQ >= N.
 // Pairs of blocks whose rows share cache lines are on one XCD (block % 8).
-template <int NQ, bool PARTS>
+template <int NQ, bool PARTS, int PX>
 __global__ __launch_bounds__(256) void k_norm_rows_half(GemmArgs a, int parts) {
   extern __shared__ __attribute__((aligned(16))) char staged[];
-  constexpr int OSTR = 2 * 4 * 16 + 16;  // an octet of columns: two parts, four rows; padded
+  constexpr int OSTR = PX * 4 * 16 + 16;  // an octet of columns: its parts, four rows; padded
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int b = (int)blockIdx.x / 16 * 16 + (int)blockIdx.x % 8 * 2 + (int)blockIdx.x % 16 / 8;
   const int m0 = 4 * b, m = min(m0 + wave, a.M - 1), n4 = a.N / 4;
@@ -447,47 +487,116 @@ __global__ __launch_bounds__(256) void k_norm_rows_half(GemmArgs a, int parts) {
     if (PARTS && live && m0 + wave < a.M) *reinterpret_cast<f4*>(a.C + (size_t)m * a.ldc + col(q)) = c[q];
     if (live) sum += (c[q].x + c[q].y) + (c[q].z + c[q].w);
   }
-  const float mean = wave_sum(sum) / (float)a.N;
+  sum = wave_sum(sum);
+  const float mean = sum / (float)a.N;
   float var = 0.0f;
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
     const f4 d = c[q] - mean;
     if (lane + 64 * q < n4) var += (d.x * d.x + d.y * d.y) + (d.z * d.z + d.w * d.w);
   }
-  const float inv = 1.0f / sqrtf(wave_sum(var) / (float)a.N + a.ln_eps);
+  const Norm norm(sum, wave_sum(var), a.N, a.ln_eps);
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
     const int i = lane + 64 * q;
     if (i >= n4) continue;
-    const f4 o = (c[q] - mean) * inv * g[q] + sh[q];
-    unsigned h0, l0, h1, l1;
-    halves2(o.x, o.y, a.ln_scale, h0, l0);
-    halves2(o.z, o.w, a.ln_scale, h1, l1);
     char* at = staged + (i >> 1) * OSTR + wave * 16 + (i & 1) * 8;
-    *reinterpret_cast<u2v*>(at) = u2v{h0, h1};
-    *reinterpret_cast<u2v*>(at + 64) = u2v{l0, l1};
+    norm.store<PX>(at, 64, c[q], g[q], sh[q], a.ln_scale);
   }
   __syncthreads();
   const int mp = cut_rows(a.M);
-  for (int i = threadIdx.x; i < a.N; i += 256) {  // (octet, part, row)
+  for (int i = threadIdx.x; i < a.N / 2 * PX; i += 256) {  // (octet, part, row)
     const int row = i & 3;
     if (m0 + row >= a.M) continue;
     *reinterpret_cast<u4v*>(reinterpret_cast<char*>(a.ln_out) + ((size_t)(i >> 2) * mp + m0 + row) * 16) =
-        *reinterpret_cast<const u4v*>(staged + (i >> 3) * OSTR + (i & 7) * 16);
+        *reinterpret_cast<const u4v*>(staged + i / (4 * PX) * OSTR + i % (4 * PX) * 16);
   }
 }
 
-template <bool PARTS>
-hipError_t launch_norm_rows(const GemmArgs& a, int parts, hipStream_t s) {
-  if (a.N % 8 != 0 || a.N > 4096 || a.ldc != a.N || a.ln_scale == 0.0f) return hipErrorInvalidValue;
+// The same, a block a row, for few rows: everything a thread reads is requested before the first use.  Eight rows share cache
+// lines: their blocks are on one XCD (block % 8), whose L2 then writes whole lines back.  NQ: 1024 NQ >= N.
+template <int NQ, bool PARTS, int PX>
+__global__ __launch_bounds__(256) void k_norm_row_half(GemmArgs a, int parts) {
+  __shared__ float red[2][4];
+  const int m = (int)blockIdx.x / 64 * 64 + (int)blockIdx.x % 8 * 8 + (int)blockIdx.x % 64 / 8;
+  if (m >= a.M) return;
+  const int n4 = a.N / 4;
+  auto col = [&](int q) { return 4 * (size_t)min((int)threadIdx.x + 256 * q, n4 - 1); };
+  auto bsum = [&](float v, float (&r)[4]) {
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) r[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return (r[0] + r[1]) + (r[2] + r[3]);
+  };
+  f4 c[NQ], v[NQ][PARTS ? 8 : 1], bias[NQ], g[NQ], sh[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    if constexpr (PARTS) {
+#pragma unroll
+      for (int p = 0; p < 8; ++p) v[q][p] = *reinterpret_cast<const f4*>(a.ws + ((size_t)min(p, parts - 1) * a.M + m) * a.N + col(q));
+      bias[q] = a.bias ? *reinterpret_cast<const f4*>(a.bias + col(q)) : f4{0.f, 0.f, 0.f, 0.f};
+    }
+    c[q] = *reinterpret_cast<const f4*>((PARTS ? a.resid : a.C) + (size_t)m * a.ldc + col(q));
+    g[q] = *reinterpret_cast<const f4*>(a.ln_g + col(q));
+    sh[q] = *reinterpret_cast<const f4*>(a.ln_b + col(q));
+  }
+  float sum = 0.0f;
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const bool live = (int)threadIdx.x + 256 * q < n4;
+    if constexpr (PARTS) {
+      f4 t = v[q][0];
+#pragma unroll
+      for (int p = 1; p < 8; ++p)
+        if (p < parts) t += v[q][p];
+      c[q] += bias[q] + t;
+      if (live) *reinterpret_cast<f4*>(a.C + (size_t)m * a.ldc + col(q)) = c[q];
+    }
+    if (live) sum += (c[q].x + c[q].y) + (c[q].z + c[q].w);
+  }
+  sum = bsum(sum, red[0]);
+  const float mean = sum / (float)a.N;
+  float var = 0.0f;
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const f4 d = c[q] - mean;
+    if ((int)threadIdx.x + 256 * q < n4) var += (d.x * d.x + d.y * d.y) + (d.z * d.z + d.w * d.w);
+  }
+  const Norm norm(sum, bsum(var, red[1]), a.N, a.ln_eps);
+  const size_t mp = cut_rows(a.M);
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    if ((int)threadIdx.x + 256 * q >= n4) continue;
+    const size_t k = col(q);
+    char* at = reinterpret_cast<char*>(a.ln_out) + (k >> 3) * PX * mp * 16 + (size_t)m * 16 + (k & 4) * 2;
+    norm.store<PX>(at, mp * 16, c[q], g[q], sh[q], a.ln_scale);
+  }
+}
+
+constexpr int kNormRowMax = 256;  // rows up to which a block takes one
+template <bool PARTS, int PX>
+hipError_t launch_norm(const GemmArgs& a, int parts, hipStream_t s) {
+  if (a.N % 8 != 0 || a.N > 4096 || a.ldc != a.N) return hipErrorInvalidValue;
+  if (a.M <= kNormRowMax) {
+    const dim3 rows((unsigned)((a.M + 63) / 64 * 64));
+    if (a.N <= 1024) hipLaunchKernelGGL((k_norm_row_half<1, PARTS, PX>), rows, dim3(256), 0, s, a, parts);
+    else if (a.N <= 2048) hipLaunchKernelGGL((k_norm_row_half<2, PARTS, PX>), rows, dim3(256), 0, s, a, parts);
+    else hipLaunchKernelGGL((k_norm_row_half<4, PARTS, PX>), rows, dim3(256), 0, s, a, parts);
+    return hipGetLastError();
+  }
   const dim3 grid((unsigned)((a.M + 63) / 64 * 16));
-  const size_t lds = (size_t)a.N / 8 * (2 * 4 * 16 + 16);
-  if (a.N <= 768) hipLaunchKernelGGL((k_norm_rows_half<3, PARTS>), grid, dim3(256), lds, s, a, parts);
-  else if (a.N <= 1280) hipLaunchKernelGGL((k_norm_rows_half<5, PARTS>), grid, dim3(256), lds, s, a, parts);
-  else if (a.N <= 1792) hipLaunchKernelGGL((k_norm_rows_half<7, PARTS>), grid, dim3(256), lds, s, a, parts);
-  else hipLaunchKernelGGL((k_norm_rows_half<16, PARTS>), grid, dim3(256), lds, s, a, parts);
+  const size_t lds = (size_t)a.N / 8 * (PX * 4 * 16 + 16);
+  if (a.N <= 768) hipLaunchKernelGGL((k_norm_rows_half<3, PARTS, PX>), grid, dim3(256), lds, s, a, parts);
+  else if (a.N <= 1280) hipLaunchKernelGGL((k_norm_rows_half<5, PARTS, PX>), grid, dim3(256), lds, s, a, parts);
+  else if (a.N <= 1792) hipLaunchKernelGGL((k_norm_rows_half<7, PARTS, PX>), grid, dim3(256), lds, s, a, parts);
+  else hipLaunchKernelGGL((k_norm_rows_half<16, PARTS, PX>), grid, dim3(256), lds, s, a, parts);
   return hipGetLastError();
 }
+template <bool PARTS>
+hipError_t launch_norm_rows(const GemmArgs& a, int parts, hipStream_t s) {
+  return a.ln_scale > 0.0f ? launch_norm<PARTS, 2>(a, parts, s) : launch_norm<PARTS, 3>(a, parts, s);
+}
+
 // ---- weights -----------------------------------------------------------------------------------
 // Rows of W as stored (WT as elsewhere: f32, bf16, int8 with their scales) to half form: part p of element (n, k) is the
 // (k % 8)-th f16 of the 16 bytes at ((k / 8 * PW + p) * N + n) * 16, times mul[n]^-1; a f32 or bf16 row is scaled by the power of
@@ -632,13 +741,14 @@ hipError_t launch_tile(const GemmArgs& a, int epi, const HalfPlan& p, hipStream_
 
 template <int EPI, int PW>
 hipError_t launch_rows_form(const GemmArgs& a, const HalfPlan& p, hipStream_t s) {
-  const dim3 grid((unsigned)((a.N + a.rows_per_block - 1) / a.rows_per_block), (unsigned)p.parts,
-                  (unsigned)((a.M + 16 * p.mt - 1) / (16 * p.mt)));
+  const unsigned n_blocks = (unsigned)((a.N + a.rows_per_block - 1) / a.rows_per_block), m_blocks = (unsigned)((a.M + 16 * p.mt - 1) / (16 * p.mt));
+  if (m_blocks > 65535u) return hipErrorInvalidValue;
+  const dim3 grid(n_blocks, (unsigned)p.parts, m_blocks);
   const int ng = (p.rows + 15) / 16;
 #define PG_CASE(MT, NG) \
   if (p.mt == MT && ng == NG) { hipLaunchKernelGGL((k_gemm_half_rows<EPI, PW, MT, NG>), grid, dim3(512), 0, s, a); return hipGetLastError(); }
-  PG_CASE(2, 1) PG_CASE(3, 1) PG_CASE(4, 1)
-  PG_CASE(2, 2) PG_CASE(3, 2) PG_CASE(4, 2)
+  PG_CASE(1, 1) PG_CASE(2, 1) PG_CASE(3, 1) PG_CASE(4, 1)
+  PG_CASE(1, 2) PG_CASE(2, 2) PG_CASE(3, 2) PG_CASE(4, 2)
   PG_CASE(3, 3) PG_CASE(4, 3)
   PG_CASE(3, 4) PG_CASE(4, 4)
 #undef PG_CASE
@@ -657,9 +767,11 @@ hipError_t launch_rows(const GemmArgs& a, int epi, const HalfPlan& p, hipStream_
 
 // Time of a product in microseconds.  Tiles: a start, the stages of 32 columns at the pace of the CU with the most items (a stage
 // alone, each further item, a partly filled round).  Blocks of rows: rounds of the blocks over the CUs, of a block's steps over
-// its wavefronts.  And what is left to do behind it: the launch that adds the parts, with or without a norm, per part and
-// value, or a norm by itself.  Constants of the least regret over the four projections of widths 512 to 1600 at 17 to 8192 rows,
-// W from HBM (29000 plans): the plan of least predicted time is 1.2 % slower than the best measured one in the mean.
+// its wavefronts, and what it costs that blocks of the same rows of W lie on several XCDs (a number of them that eight does not
+// divide: 512 x 1280 x 1280 f32 rows, 48 rows of W 19.3 us, 40 rows 14.7).  And what is left to do behind it: the launch that adds
+// the parts, with or without a norm, per part and value, or a norm by itself.  Constants of the least regret over the four
+// projections of widths 512 to 1600 at 2 to 8192 rows, W from HBM (35000 plans): the plan of least predicted time is 2 % (f32 rows
+// 1.5 %) slower than the best measured one in the mean.
 struct TilePace {
   float start, stage, more, part;
 };
@@ -667,16 +779,16 @@ struct Finish {
   float reduce_norm, part, values_norm, reduce, values, norm, norm_values;
 };
 struct RowsPace {
-  float start, turn, step, mt, ng, both, fill_mt, fill_ng;
+  float start, turn, step, mt, ng, both, fill_mt, fill_ng, uneven;
 };
 // [one f16 number a weight][HalfTile]
 constexpr TilePace kTilePace[2][4] = {
-    {{3.796f, 0.532f, 0.032f, 0.251f}, {5.756f, 0.612f, 0.372f, 0.096f}, {5.263f, 0.48f, 0.654f, 1.153f}, {}},
-    {{5.567f, 0.356f, 0.007f, 0.175f}, {7.833f, 0.372f, 0.202f, 0.157f}, {6.345f, 0.331f, 0.72f, -0.094f}, {8.862f, 0.706f, 0.349f, 0.166f}}};
-constexpr Finish kFinish[2] = {{2.922f, 1.748f, -0.459f, 3.138f, -0.459f, 1.276f, 1.735f},
-                               {5.609f, 1.263f, 0.344f, 3.75f, -0.147f, 5.585f, 1.314f}};
-constexpr RowsPace kRowsPace[2] = {{1.161f, 0.813f, -0.651f, 0.288f, 0.59f, -0.099f, -0.01f, 0.189f},
-                                   {1.271f, 1.95f, -0.585f, 0.182f, 0.245f, -0.007f, -0.006f, 0.098f}};
+    {{5.981f, 0.546f, 0.074f, 0.197f}, {9.04f, 0.604f, 0.329f, 0.111f}, {7.24f, 0.503f, 11.3f, 2.426f}, {}},
+    {{5.243f, 0.389f, 0.027f, 0.13f}, {6.453f, 0.422f, 0.178f, 0.125f}, {5.701f, 0.36f, 1.06f, -0.021f}, {10.216f, 0.619f, 0.316f, 0.158f}}};
+constexpr Finish kFinish[2] = {{2.903f, 2.218f, 0.056f, 5.858f, -3.213f, 2.241f, 2.427f},
+                               {4.686f, 1.352f, 0.859f, 18.205f, -0.462f, 3.567f, 1.958f}};
+constexpr RowsPace kRowsPace[2] = {{6.051f, 0.928f, -0.147f, 0.191f, 0.302f, 0.003f, -0.07f, 0.019f, 0.077f},
+                                   {1.852f, 0.411f, -0.082f, 0.117f, 0.048f, 0.024f, 0.068f, 0.085f, 0.067f}};
 
 }  // namespace
 
@@ -687,7 +799,7 @@ bool gemm_half_takes(const GemmArgs& a, int epi) {
                        reinterpret_cast<uintptr_t>(a.ln_g) | reinterpret_cast<uintptr_t>(a.ln_b);
   return a.w_half && a.w_half_mul && (a.w_half_parts == 1 || a.w_half_parts == 2) && !(at & 15) && a.M >= 1 && a.M < (1 << 23) &&
          a.K >= 64 && a.K % 32 == 0 && a.N >= 64 && a.N % 8 == 0 && a.N < (1 << 24) && a.ldc % 4 == 0 && a.a_unscale > 0.0f &&
-         (epi == GEMM_GELU) == (a.c_scale > 0.0f) && (!a.ln_out || a.ln_scale > 0.0f) &&
+         (epi == GEMM_GELU) == (a.c_scale > 0.0f) &&
          (epi == GEMM_BIAS || epi == GEMM_GELU || epi == GEMM_RESID) && (epi != GEMM_GELU || a.ldc == a.N);
 }
 
@@ -717,18 +829,19 @@ HalfPlan gemm_half_plan(const GemmArgs& a, int epi, int num_cus) {
       take({t, parts, 0, 0}, p.start + (float)((steps + parts - 1) / parts) * (p.stage + (on_cu - 1.0f) * p.more + round * p.part) + finish(parts));
     }
   }
-  const int groups = (a.M + 63) / 64, mt = std::max(2, ((a.M + groups - 1) / groups + 15) / 16);
+  const int groups = (a.M + 63) / 64, mt = ((a.M + groups - 1) / groups + 15) / 16;
   const int m_blocks = (a.M + 16 * mt - 1) / (16 * mt);
   const RowsPace& p = kRowsPace[one];
-  for (int parts = 1; m_blocks <= 65535 && parts <= std::max(1, most); ++parts)
-    for (int rows = 8; rows <= (mt == 2 ? 32 : 64); rows += 8) {
+  for (int parts = 1; parts <= std::max(1, most); ++parts)
+    for (int rows = 8; rows <= (mt <= 2 ? 32 : 64); rows += 8) {
       const int ng = (rows + 15) / 16;
-      const long blocks = (long)((a.N + rows - 1) / rows) * m_blocks * parts;
+      const int n_blocks = (a.N + rows - 1) / rows;
+      const long blocks = (long)n_blocks * m_blocks * parts;
       const float turns = (float)((blocks + cus - 1) / cus), fill = (float)blocks / (float)cus;
       const float rounds = (float)(((steps + parts - 1) / parts + 7) / 8);
       take({HALF_ROWS, parts, mt, rows},
            p.start + turns * (p.turn + rounds * (p.step + p.mt * mt + p.ng * ng + p.both * mt * ng)) +
-               fill * rounds * (p.fill_mt * mt + p.fill_ng * ng) + finish(parts));
+               fill * rounds * (p.fill_mt * mt + p.fill_ng * ng + (n_blocks % 8 != 0 && m_blocks > 1 ? p.uneven : 0.0f)) + finish(parts));
     }
   return best;
 }
@@ -738,7 +851,7 @@ hipError_t launch_gemm_half_plan(const GemmArgs& a0, int epi, const HalfPlan& p,
   if (!gemm_half_takes(a, epi) || p.parts < 1 || p.parts > 8) return hipErrorInvalidValue;
   if (p.parts > 1 && (epi == GEMM_GELU || !a.ws || a.K / 32 < p.parts || (size_t)p.parts * a.M * a.N > a.ws_floats)) return hipErrorInvalidValue;
   if (p.tile != HALF_ROWS) return launch_tile(a, epi, p, s);
-  if (p.rows < 8 || p.rows % 8 != 0 || (a.M + 16 * p.mt - 1) / (16 * p.mt) > 65535) return hipErrorInvalidValue;
+  if (p.rows < 8 || p.rows % 8 != 0 || p.mt < 1) return hipErrorInvalidValue;
   a.rows_per_block = p.rows;
   return a.w_half_parts == 2 ? launch_rows<2>(a, epi, p, s) : launch_rows<1>(a, epi, p, s);
 }
@@ -750,18 +863,26 @@ hipError_t launch_gemm_half(const GemmArgs& a, int epi, int num_cus, hipStream_t
   return e != hipSuccess ? e : finish_gemm_half(a, epi, p, s);
 }
 hipError_t finish_gemm_half(const GemmArgs& a, int epi, const HalfPlan& p, hipStream_t s) {
-  if (p.parts == 1) return a.ln_out ? launch_norm_rows<false>(a, 0, s) : hipSuccess;
-  if (a.ln_out && epi == GEMM_RESID) return launch_norm_rows<true>(a, p.parts, s);
-  bool ln_done = false;
-  return a.ln_out ? hipErrorInvalidValue : launch_splitk_reduce(a, epi, p.parts, s, &ln_done);
+  if (p.parts == 1 && !a.ln_out) return hipSuccess;
+  if (!a.ln_out || a.ln_scale == 0.0f) {  // (a norm of f32 rows: the logits' input)
+    if (p.parts == 1) return launch_layer_norm_rows(a.C, a.ln_out, a.M, a.N, a.ln_g, a.ln_b, a.ln_eps, s, a.ln_packed ? FORM_PACKED32 : FORM_ROWS);
+    bool ln_done = false;
+    const hipError_t e = launch_splitk_reduce(a, epi, p.parts, s, &ln_done);
+    return e != hipSuccess || !a.ln_out || ln_done ? e : hipErrorInvalidValue;
+  }
+  if (p.parts == 1) return launch_norm_rows<false>(a, 0, s);
+  return epi == GEMM_RESID ? launch_norm_rows<true>(a, p.parts, s) : hipErrorInvalidValue;
 }
 
-hipError_t launch_norm_rows_half(const float* src, void* dst, int rows, int cols, const float* g, const float* b, float eps,
-                                 float scale, hipStream_t s) {
+hipError_t launch_norm_rows_half(float* src, void* dst, int rows, int cols, const float* g, const float* b, float eps, float scale,
+                                 hipStream_t s, int parts, const float* ws, const float* bias, const float* resid) {
   GemmArgs a{};
-  a.C = const_cast<float*>(src); a.ln_out = static_cast<float*>(dst); a.M = rows; a.N = a.ldc = cols;
+  a.C = src; a.ln_out = static_cast<float*>(dst); a.M = rows; a.N = a.ldc = cols;
   a.ln_g = g; a.ln_b = b; a.ln_eps = eps; a.ln_scale = scale;
-  return launch_norm_rows<false>(a, 0, s);
+  if (parts < 0 || parts > 8 || rows < 1) return hipErrorInvalidValue;
+  if (parts == 0) return launch_norm_rows<false>(a, 0, s);
+  a.ws = const_cast<float*>(ws); a.bias = bias; a.resid = resid;
+  return launch_norm_rows<true>(a, parts, s);
 }
 
 hipError_t launch_half_rows(const void* W, int w_bytes, const float* scales, size_t rows, int cols, void* to, float* mul,

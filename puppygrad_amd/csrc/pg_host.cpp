@@ -497,12 +497,19 @@ bool takes_cut_form(const pg_model* m, size_t rows) {
          pgk::gemm_takes_cut((int)rows, (int)g.C, (int)g.I, m->w_bf16, m->w_i8, m->cut_form_min_rows, m->num_cus);
 }
 
-// Whether so many rows of activations are kept in half form: from the rows on that the cut form starts at.  f32 rows: 65 to 128
-// stay on the f32 cores as they do there, and a set bound (gemm_b9_min_rows) holds for this form too.
+// Whether so many rows of activations, of prompts or of a batched step, are kept in half form.
+//  - bf16 and int8 rows: from 17 input rows on.  Prompts of the large model, ms, 20 rows 1.69 / 1.56 (bf16), 1.64 / 1.45 (int8), 64 rows
+//    2.17 / 1.94, 300 rows 4.33 / 3.50; eight steps of 32 sequences, XL 27.2 / 27.2 (bf16), 28.8 / 27.3 (int8), of 40 32.3 / 29.1.
+//    Fewer rows are bound by their launches and W's bytes: eight steps of 8, XL bf16, 20.0 / 20.7.
+//  - f32 rows: up to 32 (prompts of 9 rows, XL, 2.54 / 2.47, 32 rows 3.18 / 2.81; the f32 cores' sums are the less precise ones, logits
+//    1.3 to 1.5 times as far off), and past the rows of the cut form (takes_cut_form), whose three parts are the more precise ones there
+//    (33 to 1024 rows, this form 1.01 to 1.15 times as far off): two f16 numbers drop a bit of a f32 weight in four.  A set bound
+//    (gemm_b9_min_rows) holds here too, and 65 to 128 rows stay on the f32 cores as they do there.
 bool takes_half_form(const pg_model* m, size_t rows) {
   if (m->half.empty()) return false;
-  if (m->w_bf16 || m->w_i8) return rows >= (size_t)pgk::kCutFormMinRows;
-  return rows >= (size_t)m->cut_form_min_rows && (rows <= 64 || rows > 128);
+  if (m->w_bf16 || m->w_i8) return rows >= 17;
+  if (rows <= 32) return m->opts.gemm_b9_min_rows ? rows >= m->opts.gemm_b9_min_rows : true;
+  return rows >= (size_t)m->gemm_b9_min_rows && rows > 128 && !takes_cut_form(m, rows);
 }
 
 // The block matrices in half form.  Nothing of it is needed to serve a call: where it cannot be had the model goes without.
@@ -598,8 +605,8 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
   // split-K partial tiles of the projections back to n_embd columns (up to 8 parts)
   const size_t ws_floats = 8 * n * g.C;
   // the projections' inputs (XN, ATT, HB) in half form or in cut form
-  const bool cut = !c->drawn && takes_cut_form(m, n);
-  const bool half = !cut && !c->drawn && takes_half_form(m, n);
+  const bool half = !c->drawn && takes_half_form(m, n);
+  const bool cut = !half && !c->drawn && takes_cut_form(m, n);
   const int form_of = cut ? pgk::FORM_CUT : pgk::FORM_ROWS;
   {
     auto form = [&](size_t cols) { return cut ? std::max(n * cols, pgk::cut_floats(n, cols)) : half ? pgk::half_floats(n, cols) : n * cols; };
@@ -764,13 +771,20 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
   // that the 32-row kernel reads with contiguous loads; their producers write them that way.
   // c->cut_form: there is room for them in cut form, which this model's rows take (the cache may have been made for
   // another model of these sizes); not the logits' input.
-  const int pk = c->pack32 ? 1 : 0, cut = c->cut_form && takes_cut_form(m, c->B) ? 1 : 0;
-  const int form = cut ? pgk::FORM_CUT : pk ? pgk::FORM_PACKED32 : pgk::FORM_ROWS;
+  // Half form, which every cache has room for, goes before both (takes_half_form).
+  const bool half = takes_half_form(m, c->B);
+  const int pk = c->pack32 && !half ? 1 : 0, cut = !half && c->cut_form && takes_cut_form(m, c->B) ? 1 : 0;
+  const int form = half ? pgk::FORM_HALF : cut ? pgk::FORM_CUT : pk ? pgk::FORM_PACKED32 : pgk::FORM_ROWS;
   auto gemm = [&](const float* A, int lda, const float* W, const float* bias, float* Cout,
                   int ldc, int N, int K, int epi, const float* ln_g = nullptr,
-                  const float* ln_b = nullptr, int a_cut = 0, int ln_cut = 0) -> hipError_t {
+                  const float* ln_b = nullptr, int a_cut = 0, int ln_cut = 0, const void* w_half = nullptr,
+                  const float* w_half_mul = nullptr, float a_scale = 0.0f, float c_scale = 0.0f, float ln_scale = 0.0f) -> hipError_t {
     pgk::GemmArgs a{};
     a.A = A; a.w_bf16 = m->w_bf16; a.W = W; a.bias = bias; a.resid = Cout; a.C = Cout;
+    if (w_half) {
+      a.w_half = w_half; a.w_half_mul = w_half_mul; a.w_half_parts = m->w_bf16 || m->w_i8 ? 1 : 2;
+      a.a_unscale = 1.0f / a_scale; a.c_scale = c_scale; a.ln_scale = ln_scale;
+    }
     a.M = B; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc;
     if (m->w_i8) a.w_scale = i8_scales_of(W, (size_t)N, (size_t)K);
     a.ws = c->gemm_ws; a.ws_floats = c->gemm_ws_floats;
@@ -782,14 +796,20 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
     return pgk::launch_gemm(a, epi, m->num_cus, s);
   };
   PG_HIP(pgk::launch_embed_batch(c->x, m->wte, m->wpe, d_ids, B, (int)pos, C, s, m->w_bf16));
-  PG_HIP(pgk::launch_layer_norm_rows(c->x, c->xn_b, B, C, m->layers[0].ln_1_g, m->layers[0].ln_1_b,
-                                     g.eps, s, form));
+  if (half)
+    PG_HIP(pgk::launch_norm_rows_half(c->x, c->xn_b, B, C, m->layers[0].ln_1_g, m->layers[0].ln_1_b, g.eps, m->half[0].norm_1, s));
+  else
+    PG_HIP(pgk::launch_layer_norm_rows(c->x, c->xn_b, B, C, m->layers[0].ln_1_g, m->layers[0].ln_1_b,
+                                       g.eps, s, form));
   for (size_t l = 0; l < g.L; ++l) {
     const pgk::LayerW& w = m->layers[l];
     // the LayerNorm after this layer: the next layer's ln_1, or ln_f
     const float* next_g = l + 1 < g.L ? m->layers[l + 1].ln_1_g : m->ln_f_g;
     const float* next_b = l + 1 < g.L ? m->layers[l + 1].ln_1_b : m->ln_f_b;
-    PG_HIP(gemm(c->xn_b, C, w.c_attn_w, w.c_attn_b, c->qkv_b, 3 * C, 3 * C, C, pgk::GEMM_BIAS, nullptr, nullptr, cut));
+    const pg_model::HalfLayer hw = half ? m->half[l] : pg_model::HalfLayer{};
+    const float next_norm = half && l + 1 < g.L ? m->half[l + 1].norm_1 : 0.0f;  // (the logits' input is plain rows)
+    PG_HIP(gemm(c->xn_b, C, w.c_attn_w, w.c_attn_b, c->qkv_b, 3 * C, 3 * C, C, pgk::GEMM_BIAS, nullptr, nullptr, cut, 0,
+                hw.c_attn, hw.c_attn_mul, hw.norm_1));
     // K/V append (rust.rs:1677-1683): by the attention launch itself for head_dim 64
     const bool fused_append = hd == pgk::kHeadDim;
     if (!fused_append)
@@ -797,14 +817,16 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
                                    c->v_panel(l, 0), bs.kv, s));
     PG_HIP(pgk::launch_attn_decode(c->qkv_b, c->k_panel(l, 0), c->v_panel(l, 0), (int)pos, P, H,
                                    hd, nsplit, c->part_acc, c->part_m, c->part_l, s, B, bs,
-                                   fused_append ? C : 0, one_split ? c->att_b : nullptr, form));
+                                   fused_append ? C : 0, one_split ? c->att_b : nullptr, form, hw.attn.v));
     if (!one_split)
       PG_HIP(pgk::launch_attn_finish(c->part_acc, c->part_m, c->part_l, H, hd, nsplit, c->att_b, s,
-                                     B, bs, form));
-    PG_HIP(gemm(c->att_b, C, w.c_proj_w, w.c_proj_b, c->x, C, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b, cut, cut));
-    PG_HIP(gemm(c->xn_b, C, w.c_fc_w, w.c_fc_b, c->hbuf, I, I, C, pgk::GEMM_GELU, nullptr, nullptr, cut));
+                                     B, bs, form, hw.attn.v));
+    PG_HIP(gemm(c->att_b, C, w.c_proj_w, w.c_proj_b, c->x, C, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b, cut, cut,
+                hw.c_proj, hw.c_proj_mul, hw.attn.v, 0.0f, hw.norm_2));
+    PG_HIP(gemm(c->xn_b, C, w.c_fc_w, w.c_fc_b, c->hbuf, I, I, C, pgk::GEMM_GELU, nullptr, nullptr, cut, 0,
+                hw.c_fc, hw.c_fc_mul, hw.norm_2, hw.hidden));
     PG_HIP(gemm(c->hbuf, I, w.c_proj_mlp_w, w.c_proj_mlp_b, c->x, C, C, I, pgk::GEMM_RESID, next_g, next_b, cut,
-                cut && l + 1 < g.L));
+                cut && l + 1 < g.L, hw.c_proj_mlp, hw.c_proj_mlp_mul, hw.hidden, 0.0f, next_norm));
   }
   PG_HIP(gemm(c->xn_b, C, m->lm_w, nullptr, c->logits_buf, (int)g.V, (int)g.V, C, pgk::GEMM_BIAS));
   return PG_OK;
@@ -1358,7 +1380,7 @@ pg_status pg_kv_cache_create(const pg_model* m, uint32_t batch, pg_kv_cache** ou
   raw->pack32 = !raw->cut_form && B > 1 && B <= 32 && g.C % 16 == 0 && g.I % 16 == 0 && !m->w_i8 &&
                 pgk::gemm_takes_rows32((int)B, (int)g.C, (int)g.C, m->w_bf16) &&
                 pgk::gemm_takes_rows32((int)B, (int)g.I, (int)g.I, m->w_bf16);
-  const size_t act_rows = raw->pack32 ? 32 : B;
+  const size_t act_rows = raw->pack32 ? 32 : B > 1 ? round_up(B, 16) : B;  // (half form: rows in sixteens)
   auto act_floats = [&](size_t cols) {
     return raw->cut_form ? std::max(act_rows * cols, pgk::cut_floats(B, cols)) : act_rows * cols;
   };

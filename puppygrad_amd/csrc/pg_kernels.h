@@ -111,7 +111,7 @@ hipError_t launch_attn_decode(const float* q, const float* kcache, const float* 
                               int P, int H, int head_dim, int nsplit, float* part_acc,
                               float* part_m, float* part_l, hipStream_t s, int batch = 1,
                               BatchStrides bs = BatchStrides{}, int append_C = 0,
-                              float* direct_out = nullptr, int out_form = 0);
+                              float* direct_out = nullptr, int out_form = 0, float out_scale = 1.0f);
 // blocks_per_cu: (head, split) blocks per CU to aim for (tunable, 4 by default).
 int choose_nsplit(int n_keys, int H, int num_cus, int blocks_per_cu = 4);
 
@@ -194,7 +194,7 @@ hipError_t launch_transpose(const float* src, float* dst, int in_f, int out_f, h
 // Attention output from a single split's (acc, m, l): out = acc / l per head.
 hipError_t launch_attn_finish(const float* part_acc, const float* part_m, const float* part_l,
                               int H, int head_dim, int nsplit, float* out, hipStream_t s,
-                              int batch = 1, BatchStrides bs = BatchStrides{}, int out_form = 0);
+                              int batch = 1, BatchStrides bs = BatchStrides{}, int out_form = 0, float out_scale = 1.0f);
 hipError_t launch_fill_zero(float* p, size_t n, hipStream_t s);
 // out[2 o] = sum_i W[o,i] g[i], out[2 o + 1] = (bias ? bias[o] : 0) + sum_i W[o,i] b[i] for the
 // rows of W[rows][cols] as stored (w_bytes 4: f32, 2: bf16, 1: int8 with scales[o]); sums in f64.
@@ -265,7 +265,7 @@ struct GemmArgs {
   int a_cut = 0, c_cut = 0, ln_cut = 0;
   // a_unscale > 0: A is in half form (FORM_HALF), its values 1 / a_unscale times what they stand for, and W's half form is
   // w_half (launch_half_rows), of w_half_parts f16 numbers a weight.  GEMM_GELU then writes C in half form, times c_scale,
-  // and ln_out is in half form, times ln_scale; no other form goes with it.  Powers of two.
+  // and ln_out is in half form, times ln_scale (0: as it would be otherwise); no other form goes with it.  Powers of two.
   const void* w_half = nullptr;
   const float* w_half_mul = nullptr;
   int w_half_parts = 0;
@@ -297,9 +297,11 @@ __host__ __device__ inline size_t packed32_index(size_t b, size_t k) {
 // (store_half4 in pg_half.h; 4 * K * cut_rows(M) bytes).
 enum ActForm : int { FORM_ROWS = 0, FORM_PACKED32 = 1, FORM_CUT = 2, FORM_HALF = 3 };
 inline size_t half_floats(size_t M, size_t K) { return (M + 15) / 16 * 16 * K; }
-// LayerNorm of rows to half form, times scale; cols a multiple of 8 up to 4096.
-hipError_t launch_norm_rows_half(const float* src, void* dst, int rows, int cols, const float* g, const float* b, float eps,
-                                 float scale, hipStream_t s);
+// LayerNorm of rows to half form, times scale, or (scale 0) to cut form; cols a multiple of 8 up to 4096.  With parts > 0 a row is
+// first put together, resid + (bias + the parts at ws [parts][rows][cols]), and written to src.
+hipError_t launch_norm_rows_half(float* src, void* dst, int rows, int cols, const float* g, const float* b, float eps,
+                                 float scale, hipStream_t s, int parts = 0, const float* ws = nullptr, const float* bias = nullptr,
+                                 const float* resid = nullptr);
 // W[rows][cols] as stored (w_bytes 4: f32, 2: bf16, 1: int8 with scales[row]) in half form: two f16 numbers a weight (f32
 // rows) or one, cols a multiple of 32, and what a sum over them is to be multiplied with, mul[rows].  *refused is set (never
 // cleared) where the rows do not allow it (k_half_rows).
@@ -343,7 +345,7 @@ hipError_t launch_attn_prefill(const float* qkv, int T, int C, int H, int head_d
 int attn_cut_shape(int T, int H, int nseq, int num_cus);
 hipError_t launch_attn_prefill_cut(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, float* out,
                                    hipStream_t s, int nseq, size_t kv_stride, int out_form, int shape);
-// The same on the f16 matrix cores (pg_attn_half.hip): out in half form times scales.v; the scales are powers of two with which no
+// The same on the f16 matrix cores (pg_attn_half.hip): out in half form times scales.v, or in cut form; the scales are powers of two with which no
 // query, key or value is past 2^15.  Shapes (groups of 32 queries, groups of
 // keys) 41, 22, 24, 18, 14; attn_half_shape: the one to take.
 struct HalfScales {
@@ -351,7 +353,8 @@ struct HalfScales {
 };
 int attn_half_shape(int T, int H, int nseq, int num_cus);
 hipError_t launch_attn_prefill_half(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, void* out,
-                                    hipStream_t s, int nseq, size_t kv_stride, const HalfScales& scales, int shape);
+                                    hipStream_t s, int nseq, size_t kv_stride, const HalfScales& scales, int shape,
+                                    int out_form = FORM_HALF);
 // rows rows; row t is position t % period of its sequence (wpe may be null)
 hipError_t launch_embed_rows(float* x, const float* wte, const float* wpe, const uint32_t* ids,
                              int rows, int C, hipStream_t s, int w_bf16 = 0, int period = 0);

@@ -7,6 +7,7 @@
 // Shapes the launchers assume are checked on the host before any launch
 // (pg_host.cpp); kernels themselves guard only the ragged tails.
 #include "pg_cut.h"
+#include "pg_half.h"
 #include "pg_kernels.h"
 #include "pg_math.h"
 #include "pg_wave.h"
@@ -610,15 +611,15 @@ __device__ __forceinline__ float4 nt_load4(const float4* p) {
 // softmax_in_place, cpu.rs:152-165, rescaled when the max moves); the four are merged
 // through LDS at the end, and the per-split (acc, m, l) by the consumer.
 // The launcher picks IT so that one chunk covers the split where the split count allows.
-// CUT: direct_out is in cut form.
-template <int IT, bool CUT>
+// FORM: how direct_out lies, FORM_CUT, FORM_HALF (times out_scale) or as out_form says.
+template <int IT, int FORM>
 __global__ __launch_bounds__(kBlock) void k_attn_decode64(const float* __restrict__ q,
                                                           const float* kcache, const float* vcache,
                                                           int pos, int P, int nsplit,
                                                           float* part_acc, float* part_m,
                                                           float* part_l, BatchStrides bs,
                                                           int append_C, float* direct_out,
-                                                          int out_form) {
+                                                          int out_form, float out_scale) {
   // direct_out (only with nsplit == 1): the block's result is the head's attention output
   // and is written there (row blockIdx.z, in whichever ActForm), with no partials and no
   // merge launch.
@@ -733,7 +734,8 @@ __global__ __launch_bounds__(kBlock) void k_attn_decode64(const float* __restric
     }
     if (direct_out) {
       const size_t b = blockIdx.z, i = (size_t)h * 64 + tid;
-      if constexpr (CUT) store_cut1(direct_out, cut_rows((int)gridDim.z), b, i, t / l);
+      if constexpr (FORM == FORM_CUT) store_cut1(direct_out, cut_rows((int)gridDim.z), b, i, t / l);
+      else if constexpr (FORM == FORM_HALF) store_half1(direct_out, cut_rows((int)gridDim.z), b, i, t / l, out_scale);
       else direct_out[out_form == FORM_PACKED32 ? packed32_index(b, i) : b * bs.out + i] = t / l;
       return;
     }
@@ -793,10 +795,10 @@ __global__ __launch_bounds__(kBlock) void k_attn_decode_any(const float* q, cons
   }
 }
 
-template <bool CUT>
+template <int FORM>
 __global__ void k_attn_finish(const float* part_acc, const float* part_m, const float* part_l,
                               int C, int hd, int nsplit, float* out, BatchStrides bs,
-                              int out_form) {
+                              int out_form, float out_scale) {
   const size_t b = blockIdx.y;
   part_acc += b * bs.part * hd;
   part_m += b * bs.part;
@@ -804,7 +806,8 @@ __global__ void k_attn_finish(const float* part_acc, const float* part_m, const 
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= C) return;
   const float v = attn_combine_elem(part_acc, part_m, part_l, nsplit, hd, i);
-  if constexpr (CUT) store_cut1(out, cut_rows((int)gridDim.y), b, (size_t)i, v);
+  if constexpr (FORM == FORM_CUT) store_cut1(out, cut_rows((int)gridDim.y), b, (size_t)i, v);
+  else if constexpr (FORM == FORM_HALF) store_half1(out, cut_rows((int)gridDim.y), b, (size_t)i, v, out_scale);
   else out[out_form == FORM_PACKED32 ? packed32_index(b, (size_t)i) : b * bs.out + i] = v;
 }
 
@@ -1488,23 +1491,28 @@ int choose_nsplit(int n_keys, int H, int num_cus, int blocks_per_cu) {
 hipError_t launch_attn_decode(const float* q, const float* kcache, const float* vcache, int pos,
                               int P, int H, int head_dim, int nsplit, float* part_acc,
                               float* part_m, float* part_l, hipStream_t s, int batch,
-                              BatchStrides bs, int append_C, float* direct_out, int out_form) {
+                              BatchStrides bs, int append_C, float* direct_out, int out_form, float out_scale) {
   if (direct_out && (head_dim != kHeadDim || nsplit != 1 || (out_form == FORM_PACKED32 && batch > 32)))
     return hipErrorInvalidValue;
   if (head_dim == kHeadDim) {
     const int per = (pos + 1 + nsplit - 1) / nsplit;
     const dim3 grid(nsplit, H, batch);
     // steps of 16 keys a block needs for its split: the chunk is sized to it
-#define PG_ATTN(IT, CUT)                                                                                          \
-  hipLaunchKernelGGL((k_attn_decode64<IT, CUT>), grid, dim3(kBlock), 0, s, q, kcache, vcache, pos, P, nsplit, part_acc, \
-                     part_m, part_l, bs, append_C, direct_out, out_form)
-    const bool cut = direct_out && out_form == FORM_CUT;
-    if (per <= 32 && cut) PG_ATTN(2, true);
-    else if (per <= 32) PG_ATTN(2, false);
-    else if (per <= 64 && cut) PG_ATTN(4, true);
-    else if (per <= 64) PG_ATTN(4, false);
-    else if (cut) PG_ATTN(8, true);
-    else PG_ATTN(8, false);
+#define PG_ATTN(IT, FORM)                                                                                         \
+  hipLaunchKernelGGL((k_attn_decode64<IT, FORM>), grid, dim3(kBlock), 0, s, q, kcache, vcache, pos, P, nsplit, part_acc, \
+                     part_m, part_l, bs, append_C, direct_out, out_form, out_scale)
+#define PG_ATTN_IT(FORM)          \
+  if (per <= 32) PG_ATTN(2, FORM); \
+  else if (per <= 64) PG_ATTN(4, FORM); \
+  else PG_ATTN(8, FORM)
+    if (direct_out && out_form == FORM_CUT) {
+      PG_ATTN_IT(FORM_CUT);
+    } else if (direct_out && out_form == FORM_HALF) {
+      PG_ATTN_IT(FORM_HALF);
+    } else {
+      PG_ATTN_IT(FORM_ROWS);
+    }
+#undef PG_ATTN_IT
 #undef PG_ATTN
   } else {
     hipLaunchKernelGGL(k_attn_decode_any, dim3(1, H, batch), dim3(kBlock),
@@ -1516,14 +1524,16 @@ hipError_t launch_attn_decode(const float* q, const float* kcache, const float* 
 
 hipError_t launch_attn_finish(const float* part_acc, const float* part_m, const float* part_l,
                               int H, int head_dim, int nsplit, float* out, hipStream_t s,
-                              int batch, BatchStrides bs, int out_form) {
+                              int batch, BatchStrides bs, int out_form, float out_scale) {
   int C = H * head_dim;
   if (out_form == FORM_PACKED32 && batch > 32) return hipErrorInvalidValue;
   const dim3 grid((C + 255) / 256, batch);
-  if (out_form == FORM_CUT)
-    hipLaunchKernelGGL(k_attn_finish<true>, grid, dim3(256), 0, s, part_acc, part_m, part_l, C, head_dim, nsplit, out, bs, out_form);
-  else
-    hipLaunchKernelGGL(k_attn_finish<false>, grid, dim3(256), 0, s, part_acc, part_m, part_l, C, head_dim, nsplit, out, bs, out_form);
+#define PG_FINISH(FORM) \
+  hipLaunchKernelGGL(k_attn_finish<FORM>, grid, dim3(256), 0, s, part_acc, part_m, part_l, C, head_dim, nsplit, out, bs, out_form, out_scale)
+  if (out_form == FORM_CUT) PG_FINISH(FORM_CUT);
+  else if (out_form == FORM_HALF) PG_FINISH(FORM_HALF);
+  else PG_FINISH(FORM_ROWS);
+#undef PG_FINISH
   return hipGetLastError();
 }
 

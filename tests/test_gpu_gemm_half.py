@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 STORE = {"f32": _lib.PG_STORE_F32, "bf16": _lib.PG_STORE_BF16, "int8": _lib.PG_STORE_INT8}
 TILE_64x128, TILE_128x128, TILE_128x128_8, TILE_128x256, ROWS = range(5)
 FORMS = [(s, t, 0, 0) for s in STORE for t in (TILE_64x128, TILE_128x128, TILE_128x128_8, TILE_128x256) if s != "f32" or t != TILE_128x256]
-FORMS += [(s, ROWS, mt, rows) for s in STORE for mt in (2, 3, 4) for rows in (8, 16, 24, 32, 40, 48, 56, 64) if mt > 2 or rows <= 32]
+FORMS += [(s, ROWS, mt, rows) for s in STORE for mt in (1, 2, 3, 4) for rows in (8, 16, 24, 32, 40, 48, 56, 64) if mt > 2 or rows <= 32]
 
 
 def up(n):
@@ -133,7 +133,8 @@ def logits(model, ids):
 
 
 # the first rows that take the form, tiles that end in the middle, one prompt and several
-@pytest.mark.parametrize("storage,width,batch,n", [("f32", 768, 1, 1026), ("f32", 1280, 1, 257), ("bf16", 1024, 1, 330), ("int8", 1600, 1, 460),
+@pytest.mark.parametrize("storage,width,batch,n", [("f32", 768, 1, 5), ("f32", 1280, 1, 32), ("bf16", 1600, 1, 17), ("int8", 1024, 2, 33), ("bf16", 768, 1, 270),
+                                                   ("int8", 1280, 1, 190), ("f32", 768, 1, 1026), ("f32", 1280, 1, 257), ("bf16", 1024, 1, 330), ("int8", 1600, 1, 460),
                                                    ("f32", 1600, 3, 131), ("bf16", 768, 5, 207), ("int8", 768, 2, 700), ("f32", 512, 9, 130)])
 def test_prompts(storage, width, batch, n):
     cfg = Gpt2Config(vocab_size=300, n_positions=1100, n_embd=width, n_layer=2, n_head=width // 64)
@@ -151,6 +152,36 @@ def test_prompts(storage, width, batch, n):
         want = model.forward_one(int(ids[b, n - 1]), other).to_host()
         # (the same values, sums of at most 6400 terms in other orders)
         assert np.linalg.norm(got[b] - want) <= 1e-5 * np.linalg.norm(want)
+
+
+# steps whose rows take the form: the smallest, one more than a block's rows, K cut and not, several blocks of rows
+@pytest.mark.parametrize("storage,width,batch", [("f32", 768, 2), ("f32", 1600, 17), ("bf16", 1024, 17), ("int8", 1280, 33), ("bf16", 768, 70), ("int8", 512, 130)])
+@pytest.mark.parametrize("n", [3, 40, 300])
+def test_batched_steps(storage, width, batch, n):
+    cfg = Gpt2Config(vocab_size=300, n_positions=310, n_embd=width, n_layer=2, n_head=width // 64)
+    model = Gpt2Model.new(cfg, synth.random_weights(cfg, 0x5EED0B01, perturb=True), Gpt2HipConfig(weight_storage=STORE[storage]))
+    ids = synth.token_ids(batch * (n + 2), 0x70C00B01 + n, 300).reshape(batch, n + 2)
+    cache = model.new_kv_cache(batch)
+    model.prefill_batch(np.ascontiguousarray(ids[:, :n]), cache)
+    model.forward_one_batch(ids[:, n], cache)
+    got = model.forward_one_batch(ids[:, n + 1], cache).to_host()
+    for b in (0, batch - 1):
+        single = model.new_kv_cache()
+        model.prefill([int(t) for t in ids[b, :n]], single)
+        model.forward_one(int(ids[b, n]), single)
+        want = model.forward_one(int(ids[b, n + 1]), single).to_host()
+        # (the same values, sums of at most 6400 terms in other orders)
+        assert np.linalg.norm(got[b] - want) <= 1e-5 * np.linalg.norm(want)
+
+
+def test_a_set_bound_holds_for_few_rows():
+    cfg = Gpt2Config(vocab_size=97, n_positions=64, n_embd=768, n_layer=1, n_head=12)
+    w = synth.random_weights(cfg, 0x5EED0B04, perturb=True)
+    ids = [int(t) for t in synth.token_ids(20, 0x70C00B04, 97)]
+    never, at, past, alone = (logits(Gpt2Model.new(cfg, w, Gpt2HipConfig(gemm_b9_min_rows=b)), ids) for b in (0xffffffff, 20, 21, 0))
+    np.testing.assert_array_equal(past, never)
+    np.testing.assert_array_equal(at, alone)
+    assert (at != never).any()
 
 
 def test_scales_hold_for_models_of_any_size_of_values():
