@@ -688,9 +688,10 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
     PG_HIP(gemm(XN.p, C, w.c_attn_w, w.c_attn_b, QKV.p, 3 * C, 3 * C, C, pgk::GEMM_BIAS, nullptr, nullptr, cut, 0,
                 hw.c_attn, hw.c_attn_mul, hw.norm_1));
     PG_MARK(kQkv);
-    if (half)
+    if (half || (cut && !m->half.empty()))
       PG_HIP(pgk::launch_attn_prefill_half(QKV.p, Ts, C, H, P, c->k_panel(l, b), c->v_panel(l, b), ATT.p, s, (int)nb,
-                                           g.H * g.P * g.hd(), hw.attn, pgk::attn_half_shape(Ts, H, (int)nb, m->num_cus)));
+                                           g.H * g.P * g.hd(), m->half[l].attn, pgk::attn_half_shape(Ts, H, (int)nb, m->num_cus),
+                                           half ? pgk::FORM_HALF : pgk::FORM_CUT));
     else
       PG_HIP(pgk::launch_attn_prefill(QKV.p, Ts, C, H, hd, P, c->k_panel(l, b), c->v_panel(l, b),
                                       ATT.p, SCR.p, m->num_cus, s, (int)nb, g.H * g.P * g.hd(), form_of, c->drawn));

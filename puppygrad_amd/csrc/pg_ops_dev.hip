@@ -471,10 +471,10 @@ pg_status pg_testing_half_product_dev(int32_t device, void* stream, const float*
   return PG_OK;
 }
 
-// The same by pg_attn_half.hip: out in half form times sv (shape 0: as the planner has it).
+// The same by pg_attn_half.hip: out in half form times sv, or (cut) in cut form; shape 0: as the planner has it.
 pg_status pg_testing_attention_half_dev(int32_t device, void* stream, const float* qkv, uint64_t rows, uint64_t heads,
-                                        uint64_t sequences, int32_t shape, float sq, float sk, float sv, float* keys, float* values,
-                                        void* out) {
+                                        uint64_t sequences, int32_t shape, float sq, float sk, float sv, int32_t cut, float* keys,
+                                        float* values, void* out) {
   if (!qkv || !keys || !values || !out) return pgh::fail(PG_INVALID_INPUT, "null argument");
   if (rows == 0 || rows > 4096 || heads == 0 || heads > 64 || sequences == 0 || sequences > 1024)
     return pgh::fail(PG_INVALID_INPUT, "attention: sizes");
@@ -484,7 +484,8 @@ pg_status pg_testing_attention_half_dev(int32_t device, void* stream, const floa
   int cus = 0;
   PG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
   PG_HIP(pgk::launch_attn_prefill_half(qkv, T, 64 * H, H, T, keys, values, out, static_cast<hipStream_t>(stream), (int)sequences,
-                                       (size_t)H * T * 64, {sq, sk, sv}, shape ? shape : pgk::attn_half_shape(T, H, (int)sequences, cus)));
+                                       (size_t)H * T * 64, {sq, sk, sv}, shape ? shape : pgk::attn_half_shape(T, H, (int)sequences, cus),
+                                       cut ? pgk::FORM_CUT : pgk::FORM_HALF));
   return PG_OK;
 }
 

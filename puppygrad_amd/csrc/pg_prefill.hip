@@ -363,14 +363,10 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(GemmArgs a, int parts) {
 // EARLY: everything a thread reads is requested before the first use (a few rows: the launch
 // is a chain of memory round trips and this takes two out of it); otherwise column block by
 // column block, with few registers, for the many rows of a long prompt.
-// CUT: a.ln_out is in cut form.
-template <int EPI, bool EARLY, bool CUT = false>
+template <int EPI, bool EARLY>
 __global__ __launch_bounds__(256) void k_splitk_reduce_ln(GemmArgs a, int parts) {
   __shared__ float red[4];
-  // Eight rows of a matrix in cut form share cache lines: their blocks are on one XCD (block % 8), whose L2 then writes
-  // whole lines back.
-  const size_t m = CUT ? blockIdx.x / 64 * 64 + blockIdx.x % 8 * 8 + blockIdx.x % 64 / 8 : blockIdx.x;
-  if (CUT && m >= (size_t)a.M) return;
+  const size_t m = blockIdx.x;
   const int n4 = a.N / 4;
   const size_t stride = (size_t)a.M * a.N;
   auto bsum = [&](float v) {
@@ -458,8 +454,7 @@ __global__ __launch_bounds__(256) void k_splitk_reduce_ln(GemmArgs a, int parts)
       o.y = (c[q].y - mean) * inv * g.y + b.y;
       o.z = (c[q].z - mean) * inv * g.z + b.z;
       o.w = (c[q].w - mean) * inv * g.w + b.w;
-      if constexpr (CUT) store_cut4(a.ln_out, cut_rows(a.M), m, n, o);
-      else *reinterpret_cast<f4*>(a.ln_out + (a.ln_packed ? packed32_index(m, n) : m * a.N + n)) = o;
+      *reinterpret_cast<f4*>(a.ln_out + (a.ln_packed ? packed32_index(m, n) : m * a.N + n)) = o;
     }
   }
 }
@@ -1245,15 +1240,13 @@ __global__ void k_embed_rows(float* x, const float* wte, const float* wpe, const
 
 // dst[r] = LayerNorm(src[r])  (layer_norm_in_place, cpu.rs:119-143), one block per row
 // (dst_packed: dst is a packed activation matrix, see packed32_index)
-template <bool CUT>
 __global__ __launch_bounds__(256) void k_layer_norm_rows(const float* src, float* dst, int cols,
                                                          const float* g, const float* b,
                                                          float eps, int dst_form) {
   __shared__ float red[4];
   const float* row = src + (size_t)blockIdx.x * cols;
   auto put = [&](int i, float v) {
-    if (CUT) store_cut1(dst, cut_rows((int)gridDim.x), blockIdx.x, (size_t)i, v);
-    else dst[dst_form == FORM_PACKED32 ? packed32_index(blockIdx.x, (size_t)i) : (size_t)blockIdx.x * cols + i] = v;
+    dst[dst_form == FORM_PACKED32 ? packed32_index(blockIdx.x, (size_t)i) : (size_t)blockIdx.x * cols + i] = v;
   };
   auto bsum = [&](float v) {
     v = wave_sum(v);
@@ -1341,12 +1334,9 @@ hipError_t launch_splitk_reduce(const GemmArgs& a, int epi, int parts, hipStream
   if (a.ln_out && a.N % 4 == 0 && a.N <= 4096 && a.ldc == a.N) {
     const bool early = a.M <= 64;
     if (a.ln_cut) {
-      const dim3 rows((a.M + 63) / 64 * 64);
       if (epi != GEMM_RESID) return hipErrorInvalidValue;
-      if (early) hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_RESID, true, true>), rows, dim3(256), 0, s, a, parts);
-      else hipLaunchKernelGGL((k_splitk_reduce_ln<GEMM_RESID, false, true>), rows, dim3(256), 0, s, a, parts);
       *ln_done = true;
-      return hipGetLastError();
+      return launch_norm_rows_half(a.C, a.ln_out, a.M, a.N, a.ln_g, a.ln_b, a.ln_eps, 0.0f, s, parts, a.ws, a.bias, a.resid);
     }
     const dim3 rows(a.M);
     if (epi == GEMM_BIAS && early)
@@ -1830,10 +1820,8 @@ hipError_t launch_embed_rows(float* x, const float* wte, const float* wpe, const
 hipError_t launch_layer_norm_rows(const float* src, float* dst, int rows, int cols, const float* g,
                                   const float* b, float eps, hipStream_t s, int dst_form) {
   if ((dst_form == FORM_PACKED32 && rows > 32) || (dst_form == FORM_CUT && cols % 8 != 0)) return hipErrorInvalidValue;
-  if (dst_form == FORM_CUT)
-    hipLaunchKernelGGL(k_layer_norm_rows<true>, dim3(rows), dim3(256), 0, s, src, dst, cols, g, b, eps, dst_form);
-  else
-    hipLaunchKernelGGL(k_layer_norm_rows<false>, dim3(rows), dim3(256), 0, s, src, dst, cols, g, b, eps, dst_form);
+  if (dst_form == FORM_CUT) return launch_norm_rows_half(const_cast<float*>(src), dst, rows, cols, g, b, eps, 0.0f, s);
+  hipLaunchKernelGGL(k_layer_norm_rows, dim3(rows), dim3(256), 0, s, src, dst, cols, g, b, eps, dst_form);
   return hipGetLastError();
 }
 

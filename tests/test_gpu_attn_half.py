@@ -10,33 +10,38 @@ from puppygrad_amd import _lib
 pytestmark = pytest.mark.gpu
 
 
-def attention_half_dev(qkv, heads, shape, sq, sk, sv):
+def attention_half_dev(qkv, heads, shape, sq, sk, sv, cut=False):
     f = _lib.load().pg_testing_attention_half_dev
     u, v, i, s = C.c_uint64, C.c_void_p, C.c_int32, C.c_float
-    f.argtypes, f.restype = [i, v, v, u, u, u, i, s, s, s, v, v, v], C.c_int
+    f.argtypes, f.restype = [i, v, v, u, u, u, i, s, s, s, i, v, v, v], C.c_int
     n, t, _ = qkv.shape
     m, k = n * t, 64 * heads
     mp = (m + 15) // 16 * 16
-    held = [DeviceArray(qkv)] + [DeviceArray(np.full(size, np.nan, np.float32)) for size in (m * k, m * k, mp * k)]
-    status = f(0, None, held[0].ptr, t, heads, n, shape, sq, sk, sv, held[1].ptr, held[2].ptr, held[3].ptr)
+    held = [DeviceArray(qkv)] + [DeviceArray(np.full(size, np.nan, np.float32)) for size in (m * k, m * k, mp * k * 3 // 2)]
+    status = f(0, None, held[0].ptr, t, heads, n, shape, sq, sk, sv, cut, held[1].ptr, held[2].ptr, held[3].ptr)
     keys, values, out = (d.download() for d in held[1:])
     for d in held:
         d.free()
     assert status == 0, _lib.load().pg_last_error_message().decode()
-    out = out.view(np.float16).reshape(k // 8, 2, mp, 8)[:, :, :m].astype(np.float64).sum(1).transpose(1, 0, 2).reshape(n, t, k) / sv
+    if cut:
+        parts = (out.view(np.uint16).astype(np.uint32) << 16).view(np.float32).reshape(k // 8, 3, mp, 8)
+    else:
+        parts = out.view(np.float16)[:2 * mp * k].reshape(k // 8, 2, mp, 8) / np.float32(sv)
+    out = parts[:, :, :m].astype(np.float64).sum(1).transpose(1, 0, 2).reshape(n, t, k)
     return out, keys.reshape(n, heads, t, 64), values.reshape(n, heads, t, 64)
 
 
 # one tile, its edges, tiles that some key groups or query groups have none of
 @pytest.mark.parametrize("t", [1, 31, 32, 33, 64, 65, 127, 130, 200, 290])
 @pytest.mark.parametrize("shape", [41, 22, 24, 18, 14, 0])
-def test_shapes_at_their_edges(shape, t):
+@pytest.mark.parametrize("cut", [False, True])
+def test_shapes_at_their_edges(shape, t, cut):
     rng = np.random.default_rng([t, shape])
     heads, n = 2, 2
     qkv = rng.standard_normal((n, t, 3, heads, 64)).astype(np.float32)
     qkv[:, :, 0] *= 3.0
     qkv[1, :, 1:] *= 10.0 ** rng.uniform(-2, 1, (t, 1, 1, 1))  # keys and values of unequal size
-    out, keys, values = attention_half_dev(qkv.reshape(n, t, -1), heads, shape, 512.0, 256.0, 64.0)
+    out, keys, values = attention_half_dev(qkv.reshape(n, t, -1), heads, shape, 512.0, 256.0, 64.0, cut)
     np.testing.assert_array_equal(keys, qkv[:, :, 1].transpose(0, 2, 1, 3))
     np.testing.assert_array_equal(values, qkv[:, :, 2].transpose(0, 2, 1, 3))
     q, k, v = (qkv[:, :, j].transpose(0, 2, 1, 3).astype(np.float64) for j in range(3))
