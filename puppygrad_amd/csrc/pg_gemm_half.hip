@@ -25,6 +25,12 @@
 // but a chain's end.  1000 x 4800 x 1600 f32 rows 102 us and a reduction of 11 -> 52, 1000 x 6400 x 1600 113 -> 58, 8192 x
 // 4800 x 1600 606 -> 337; bf16 16384 x 4800 x 1600 610 -> 436, 16384 x 1600 x 6400 880 -> 606 (1125 TFLOP/s of matrix
 // instructions; a plain library product reaches 1354).
+//
+// The same kernels serve rows in cut form (bf16, three parts) with W in cut form beside its stored rows, six products: what
+// pg_gemm_rows.hip and pg_gemm_cut.hip do with W as stored, without the cut of W in every block.  For f32 models narrow enough
+// that W's six bytes a weight do not outweigh it (make_half_form): 1024 rows, 768 wide, the four products 28.4, 16.0, 40.0,
+// 34.6 -> 26.7, 15.7, 29.7, 34.6 us with the plans fitted to half form, 24.9, 15.7, 29.9, 32.5 the best ones; logits 0.86 to 0.95
+// of what they were off by (129 to 1024 tokens: chains as in half form).
 #include "pg_gemm_dev.h"
 #include "pg_half.h"
 #include "pg_wave.h"
@@ -54,7 +60,16 @@ __device__ __forceinline__ void vm_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// GELU of sum + bias, four columns of a row, with what f32 rounds away on the way.
+// The products of parts (input, weight) that stand for one in f32, small ones first: half form with one or two parts a weight, cut form.
+template <int PX, int PW>
+struct Products {
+  static constexpr int n = PX == 3 ? 6 : PW + 1;
+  static constexpr int x[6] = {PX - 1, 0, PX == 3 ? 1 : 0, 1, 0, 0};
+  static constexpr int w[6] = {0, PX == 3 ? 2 : PW - 1, PX == 3 ? 1 : 0, 0, PW > 1 ? 1 : 0, 0};
+};
+
+// GELU of sum + bias, four columns of a row, in half form with what f32 rounds away on the way, or in cut form.
+template <int PX>
 __device__ __forceinline__ void store_gelu(void* to, int mp, size_t m, size_t n, f4 sum, f4 bias, float scale) {
   const f4 c = bias + sum, b = c - sum, c_rest = (bias - b) + (sum - (c - b));
   f4 y, rest;
@@ -64,25 +79,27 @@ __device__ __forceinline__ void store_gelu(void* to, int mp, size_t m, size_t n,
     y[e] = gelu_tanh(c[e], c_rest[e], r);
     rest[e] = r;
   }
-  store_half4(to, mp, m, n, y, rest, scale);
+  if constexpr (PX == 3) store_cut4(to, mp, m, n, y);
+  else store_half4(to, mp, m, n, y, rest, scale);
 }
 
 // WM x WN wavefronts, each on MB x NB blocks of 32 x 32.  The operands are turned round: lane (l, half) of the first holds
 // columns 8 half .. 8 half + 7 of row l of W, of the second those of input row l, so that the result's lane is a row
-// of C and its values four by four neighbouring columns.  PW: parts of a weight (2: f32 rows).  K runs in stages of KT
+// of C and its values four by four neighbouring columns.  PX, PW: parts of an input value (3: cut form, on the bf16 cores; W
+// then has three parts too) and of a weight (2: f32 rows in half form).  K runs in stages of KT
 // columns in NA buffers, a stage in steps of 16 whose operands are read during the step before.  One barrier per stage, in front of the step that reads the next stage: by then the wavefront has
 // waited for its own share of that stage, and has read the stage before it to the end, whose buffer is free for the stage that
 // is asked for next.  CH: stages in a chain of matrix instructions (0: one chain).  TWO: the small products of a chain have a
 // sum of their own.  SPLIT: the stages are cut into gridDim.y parts, raw partial tiles go to a.ws[part][M][N].  OCC:
 // wavefronts per SIMD that the registers are kept for.
-template <int WM, int WN, int MB, int NB, int PW, int EPI, int SPLIT, int OCC, int NA, int KT, int CH, bool TWO>
+template <int WM, int WN, int MB, int NB, int PX, int PW, int EPI, int SPLIT, int OCC, int NA, int KT, int CH, bool TWO>
 __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
   constexpr int NW = WM * WN, BM = 32 * MB * WM, BN = 32 * NB * WN, NO = KT / 8, NS = KT / 16;
-  constexpr int IA = NO * 2 * BM / 64 / NW, IB = NO * PW * BN / 64 / NW;
+  constexpr int IA = NO * PX * BM / 64 / NW, IB = NO * PW * BN / 64 / NW;
   constexpr int UN = CH ? CH : NA;
   static_assert(UN % NA == 0 && (NS == 2 || UN % 2 == 0) && UN <= 8 && (CH != 0 || !TWO));
-  static_assert(NO * 2 * BM % (64 * NW) == 0 && NO * PW * BN % (64 * NW) == 0 && BM % 64 == 0 && BN % 64 == 0);
-  __shared__ u4v As[NA][NO * 2 * BM];
+  static_assert(NO * PX * BM % (64 * NW) == 0 && NO * PW * BN % (64 * NW) == 0 && BM % 64 == 0 && BN % 64 == 0);
+  __shared__ u4v As[NA][NO * PX * BM];
   __shared__ u4v Bs[NA][NO * PW * BN];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -118,14 +135,14 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
     const int at = (wave * IB + i) * 64, plane = at / BN, row = at % BN + lane;
     boff[i] = ((unsigned)plane * (unsigned)a.N + (unsigned)min(n0 + row, a.N - 1)) * 16u;
   }
-  const size_t astage = (size_t)NO * 2 * mp * 16, bstage = (size_t)NO * PW * a.N * 16;
+  const size_t astage = (size_t)NO * PX * mp * 16, bstage = (size_t)NO * PW * a.N * 16;
   const char* Ab = reinterpret_cast<const char*>(a.A) + kt0 * astage;
   const char* Wb = static_cast<const char*>(a.w_half) + kt0 * bstage;
   const unsigned as_lds = (unsigned)(size_t)(lds_ptr)(void*)&As[0][0], bs_lds = (unsigned)(size_t)(lds_ptr)(void*)&Bs[0][0];
   auto dma = [&](int t, int buf) __attribute__((always_inline)) {
     const size_t k = (size_t)min(t, T - 1);
 #pragma unroll
-    for (int i = 0; i < IA; ++i) lds_dma16(Ab + k * astage, aoff[i], as_lds + (unsigned)(buf * NO * 2 * BM * 16 + (wave * IA + i) * 1024));
+    for (int i = 0; i < IA; ++i) lds_dma16(Ab + k * astage, aoff[i], as_lds + (unsigned)(buf * NO * PX * BM * 16 + (wave * IA + i) * 1024));
 #pragma unroll
     for (int i = 0; i < IB; ++i) lds_dma16(Wb + k * bstage, boff[i], bs_lds + (unsigned)(buf * NO * PW * BN * 16 + (wave * IB + i) * 1024));
   };
@@ -140,21 +157,21 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
         acc[i][j][v] = 0.0f;
         if constexpr (CH != 0) tot[i][j][v] = 0.0f;
       }
-  struct Ops { u4v x[MB][2], w[NB][PW]; };
+  struct Ops { u4v x[MB][PX], w[NB][PW]; };
   auto read = [&](int buf, int s, Ops& o) __attribute__((always_inline)) {
 #pragma unroll
-    for (int p = 1; p >= 0; --p) {  // in the order in which the products need them
+    for (int p = PX - 1; p >= 0; --p) {  // in the order in which the products need them
 #pragma unroll
-      for (int i = 0; i < MB; ++i) o.x[i][p] = As[buf][((2 * s + half) * 2 + p) * BM + (wm * MB + i) * 32 + l32];
-      const int q = 1 - p;
+      for (int i = 0; i < MB; ++i) o.x[i][p] = As[buf][((2 * s + half) * PX + p) * BM + (wm * MB + i) * 32 + l32];
+      const int q = PX - 1 - p;
       if (q < PW) {
 #pragma unroll
         for (int j = 0; j < NB; ++j) o.w[j][q] = Bs[buf][((2 * s + half) * PW + q) * BN + (wn * NB + j) * 32 + l32];
       }
     }
   };
-  // products of parts (input, weight), small ones first
-  constexpr int NP = PW + 1;
+  using P = Products<PX, PW>;
+  constexpr int NP = P::n;
   auto step = [&](auto first, const Ops& cur, Ops& nxt, int buf, int s) __attribute__((always_inline)) {
     constexpr bool fresh = CH != 0 && decltype(first)::value;
     read(buf, s, nxt);
@@ -164,18 +181,21 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
       for (int j = 0; j < NB; ++j)
 #pragma unroll
         for (int i = 0; i < MB; ++i) {
-          const int px = p == 0 ? 1 : 0, pw = p == 1 && PW == 2 ? 1 : 0;
           f16v& sum = TWO && p < NP - 1 ? low[TWO ? i : 0][TWO ? j : 0] : acc[i][j];
           if (fresh && (p == 0 || (TWO && p == NP - 1))) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) sum[v] = 0.0f;
           }
-          sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, cur.w[j][pw]), __builtin_bit_cast(h8v, cur.x[i][px]), sum, 0, 0, 0);
+          const u4v &w = cur.w[j][P::w[p]], &x = cur.x[i][P::x[p]];
+          if constexpr (PX == 3)
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x), sum, 0, 0, 0);
+          else
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, w), __builtin_bit_cast(h8v, x), sum, 0, 0, 0);
         }
     }
   };
   auto interleave = [&] __attribute__((always_inline)) {
-    constexpr int NM = NP * MB * NB, NR = 2 * MB + PW * NB, PER = (NR + NM - 1) / NM;
+    constexpr int NM = NP * MB * NB, NR = PX * MB + PW * NB, PER = (NR + NM - 1) / NM;
 #pragma unroll
     for (int g = 0; g < NM; ++g) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -248,7 +268,8 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
     for (int g = 0; g < 4; ++g) {
       const int n = n0 + (wn * NB + j) * 32 + 8 * g + 4 * half;
       if (n >= a.N) continue;
-      const f4 mul = *reinterpret_cast<const f4*>(a.w_half_mul + n) * a.a_unscale;
+      f4 mul = f4{1.f, 1.f, 1.f, 1.f};
+      if constexpr (PX == 2) mul = *reinterpret_cast<const f4*>(a.w_half_mul + n) * a.a_unscale;
       f4 bias = f4{0.f, 0.f, 0.f, 0.f};
       if (!SPLIT && a.bias) bias = *reinterpret_cast<const f4*>(a.bias + n);
 #pragma unroll
@@ -264,7 +285,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
           continue;
         }
         if constexpr (EPI == GEMM_GELU) {
-          store_gelu(a.C, mp, (size_t)m, (size_t)n, c, bias, a.c_scale);
+          store_gelu<PX>(a.C, mp, (size_t)m, (size_t)n, c, bias, a.c_scale);
           continue;
         }
         c += bias;
@@ -278,11 +299,12 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
 // A block owns 16 MT input rows and up to 16 NG rows of W (a.rows_per_block of them, a multiple of eight); its
 // eight wavefronts take the steps of 32 columns in turn, operands from L2 straight to registers, and the eight partial tiles
 // are added through LDS.  gridDim.y > 1: K is cut over blocks as well, raw tiles go to a.ws[part][M][N].  As k_gemm_cut_rows
-// (pg_gemm_rows.hip), with 4 bytes per input value for 6, and rows of W that need no turn through LDS and no cut.
-template <int EPI, int PW, int MT, int NG>
+// (pg_gemm_rows.hip), with rows of W that need no turn through LDS and no cut, and in half form 4 bytes per input value for 6.
+// PX = PW = 3: both operands in cut form, on the bf16 cores: 1024 x 2304 x 768, us, 28.4 there, 24.9 here (48 rows of W a block).
+template <int EPI, int PX, int PW, int MT, int NG>
 __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
   constexpr int CSTR = 16 * NG + 4;  // row stride of the partial tile, floats
-  constexpr int PD = MT * NG * 8 + 8 * (NG * PW + MT * 2) <= 184 ? 2 : 1;  // steps requested ahead
+  constexpr int PD = MT * NG * 8 + 8 * (NG * PW + MT * PX) <= (PX == 3 ? 140 : 184) ? 2 : 1;  // steps requested ahead
   __shared__ __attribute__((aligned(16))) float slab[8][16 * MT * CSTR];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int i16 = lane & 15, kq = lane >> 4;
@@ -301,8 +323,8 @@ __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
   const char* xp[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
-    xp[mt] = reinterpret_cast<const char*>(a.A) + ((size_t)kq * 2 * mp + min(m0 + 16 * mt + i16, a.M - 1)) * 16;
-  const size_t wpart = (size_t)a.N * 16, wstep = wpart * 4 * PW, xpart = (size_t)mp * 16, xstep = xpart * 8;
+    xp[mt] = reinterpret_cast<const char*>(a.A) + ((size_t)kq * PX * mp + min(m0 + 16 * mt + i16, a.M - 1)) * 16;
+  const size_t wpart = (size_t)a.N * 16, wstep = wpart * 4 * PW, xpart = (size_t)mp * 16, xstep = xpart * 4 * PX;
 
   // The write-out takes four columns of a row at a time, neighbouring lanes neighbouring columns, or, into a matrix
   // in half form, neighbouring rows, which lie next to each other there.  What it adds is requested first.
@@ -317,7 +339,7 @@ __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
     const int idx = tid + 512 * q, m = m0 + row_of(idx), n = n0 + col_of(idx);
     const bool live = idx < ITEMS && m < a.M && n < n1;
     ebias[q] = eres[q] = emul[q] = f4{0.f, 0.f, 0.f, 0.f};
-    if (live) emul[q] = *reinterpret_cast<const f4*>(a.w_half_mul + n) * a.a_unscale;
+    if (PX == 2 && live) emul[q] = *reinterpret_cast<const f4*>(a.w_half_mul + n) * a.a_unscale;
     if (parts > 1) continue;
     if (live && a.bias) ebias[q] = *reinterpret_cast<const f4*>(a.bias + n);
     if (live && EPI == GEMM_RESID) eres[q] = *reinterpret_cast<const f4*>(a.resid + (size_t)m * a.ldc + n);
@@ -329,8 +351,8 @@ __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
 #pragma unroll
     for (int g = 0; g < NG; ++g) tot[mt][g] = f4{0.f, 0.f, 0.f, 0.f};
 
-  u4v rw[PD][NG][PW], rx[PD][MT][2];
-  auto load_step = [&](int s, u4v (&w)[NG][PW], u4v (&x)[MT][2]) {
+  u4v rw[PD][NG][PW], rx[PD][MT][PX];
+  auto load_step = [&](int s, u4v (&w)[NG][PW], u4v (&x)[MT][PX]) {
     const size_t col = (size_t)piece + (size_t)pieces * min(s, steps - 1);
 #pragma unroll
     for (int g = 0; g < NG; ++g)
@@ -339,24 +361,24 @@ __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int p = 0; p < 2; ++p) x[mt][p] = *reinterpret_cast<const u4v*>(xp[mt] + col * xstep + p * xpart);
+      for (int p = 0; p < PX; ++p) x[mt][p] = *reinterpret_cast<const u4v*>(xp[mt] + col * xstep + p * xpart);
   };
-  auto mul_step = [&](const u4v (&w)[NG][PW], const u4v (&x)[MT][2]) {
+  auto mul_step = [&](const u4v (&w)[NG][PW], const u4v (&x)[MT][PX]) {
     // a chain of matrix instructions is a step, the small products one of their own; each product over a row of tiles before
     // the next
     auto one = [](const u4v& x, const u4v& w, const f4& c) {
-      return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8v, x), __builtin_bit_cast(h8v, w), c, 0, 0, 0);
+      if constexpr (PX == 3) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x), __builtin_bit_cast(bf16x8, w), c, 0, 0, 0);
+      else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8v, x), __builtin_bit_cast(h8v, w), c, 0, 0, 0);
     };
+    using P = Products<PX, PW>;
     const f4 zero{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       f4 c[NG], big[NG];
 #pragma unroll
-      for (int g = 0; g < NG; ++g) c[g] = one(x[mt][1], w[g][0], zero);
-      if constexpr (PW == 2) {
+      for (int p = 0; p < P::n - 1; ++p)
 #pragma unroll
-        for (int g = 0; g < NG; ++g) c[g] = one(x[mt][0], w[g][PW - 1], c[g]);
-      }
+        for (int g = 0; g < NG; ++g) c[g] = one(x[mt][P::x[p]], w[g][P::w[p]], p ? c[g] : zero);
 #pragma unroll
       for (int g = 0; g < NG; ++g) big[g] = one(x[mt][0], w[g][0], zero);
 #pragma unroll
@@ -401,13 +423,13 @@ __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
     f4 w8[8];
 #pragma unroll
     for (int w = 0; w < 8; ++w) w8[w] = *reinterpret_cast<const f4*>(slab[w] + mr * CSTR + nl);
-    const f4 sum = (((w8[0] + w8[1]) + (w8[2] + w8[3])) + ((w8[4] + w8[5]) + (w8[6] + w8[7]))) * emul[q];
+    const f4 sum = (((w8[0] + w8[1]) + (w8[2] + w8[3])) + ((w8[4] + w8[5]) + (w8[6] + w8[7]))) * (PX == 2 ? emul[q] : f4{1.f, 1.f, 1.f, 1.f});
     if (parts > 1) {
       *reinterpret_cast<f4*>(a.ws + ((size_t)part * a.M + m) * a.N + n) = sum;
       continue;
     }
     if (EPI == GEMM_GELU) {
-      store_gelu(a.C, mp, (size_t)m, (size_t)n, sum, ebias[q], a.c_scale);
+      store_gelu<PX>(a.C, mp, (size_t)m, (size_t)n, sum, ebias[q], a.c_scale);
       continue;
     }
     f4 c = ebias[q] + sum;
@@ -668,6 +690,19 @@ __global__ __launch_bounds__(256) void k_half_rows(const void* W, const float* s
   if (bad) atomicOr(refused, 1u);
 }
 
+// f32 rows to cut form, three bf16 numbers a weight, in the order of k_half_rows.
+__global__ __launch_bounds__(256) void k_cut_weights(const float* W, void* to, int N, int K) {
+  const int n = (int)blockIdx.x * 64 + (threadIdx.x & 63);
+  if (n >= N) return;
+  for (int k = 8 * (threadIdx.x >> 6); k < K; k += 32) {
+    const f4* w = reinterpret_cast<const f4*>(W + (size_t)n * K + k);
+    const Cut c = cut8(w[0], w[1]);
+    u4v* at = static_cast<u4v*>(to) + (size_t)(k / 8) * 3 * N + n;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) at[(size_t)p * N] = c.p[p];
+  }
+}
+
 // The largest that an output of a projection behind a LayerNorm can be: the norm's values before scale and shift are at most
 // sqrt(C) long together, so |W_o . (g z + b) + bias_o| <= sqrt(C) |W_o g| + |W_o . b + bias_o|, the second as fold has it
 // (launch_ln_fold).  The maximum over the rows goes to *most, bits of a float that is not negative.
@@ -699,7 +734,7 @@ __global__ __launch_bounds__(256) void k_half_bound_norm(const float* g, const f
 }
 
 // ---- launchers ---------------------------------------------------------------------------------
-template <int WM, int WN, int MB, int NB, int PW, int OCC, int NA, int KT, int CH, bool TWO>
+template <int WM, int WN, int MB, int NB, int PX, int PW, int OCC, int NA, int KT, int CH, bool TWO>
 struct Shape {
   static constexpr int bm = 32 * MB * WM, bn = 32 * NB * WN;
   template <int EPI, int SPLIT>
@@ -708,7 +743,7 @@ struct Shape {
     const int tiles_m = (a.M + bm - 1) / bm, tiles_n = (a.N + bn - 1) / bn, tiles = tiles_m * tiles_n;
     a.band_rows = choose_band(tiles_m, std::max(1, (tiles + 7) / 8), bm, bn);
     const dim3 grid((unsigned)((tiles + 7) / 8 * 8), (unsigned)parts);  // whole rounds over the 8 XCDs
-    hipLaunchKernelGGL((k_gemm_half<WM, WN, MB, NB, PW, EPI, SPLIT, OCC, NA, KT, CH, TWO>), grid, dim3(64 * WM * WN), 0, s, a);
+    hipLaunchKernelGGL((k_gemm_half<WM, WN, MB, NB, PX, PW, EPI, SPLIT, OCC, NA, KT, CH, TWO>), grid, dim3(64 * WM * WN), 0, s, a);
     return hipGetLastError();
   }
   static hipError_t launch(const GemmArgs& a, int epi, int parts, hipStream_t s) {
@@ -722,45 +757,52 @@ struct Shape {
   }
 };
 hipError_t launch_tile(const GemmArgs& a, int epi, const HalfPlan& p, hipStream_t s) {
+  if (a.w_half_parts == 3) {
+    switch (p.tile) {
+      case HALF_64x128: return Shape<2, 2, 1, 2, 3, 3, 2, 2, 32, 4, true>::launch(a, epi, p.parts, s);
+      case HALF_128x128_8: return Shape<4, 2, 1, 2, 3, 3, 2, 3, 32, 3, true>::launch(a, epi, p.parts, s);
+      default: return hipErrorInvalidValue;
+    }
+  }
   if (a.w_half_parts == 2) {
     switch (p.tile) {
-      case HALF_64x128: return Shape<2, 2, 1, 2, 2, 3, 2, 32, 4, true>::launch(a, epi, p.parts, s);
-      case HALF_128x128: return Shape<2, 2, 2, 2, 2, 2, 4, 16, 4, false>::launch(a, epi, p.parts, s);
-      case HALF_128x128_8: return Shape<4, 2, 1, 2, 2, 2, 4, 32, 4, true>::launch(a, epi, p.parts, s);
+      case HALF_64x128: return Shape<2, 2, 1, 2, 2, 2, 3, 2, 32, 4, true>::launch(a, epi, p.parts, s);
+      case HALF_128x128: return Shape<2, 2, 2, 2, 2, 2, 2, 4, 16, 4, false>::launch(a, epi, p.parts, s);
+      case HALF_128x128_8: return Shape<4, 2, 1, 2, 2, 2, 2, 4, 32, 4, true>::launch(a, epi, p.parts, s);
       default: return hipErrorInvalidValue;
     }
   }
   switch (p.tile) {
-    case HALF_64x128: return Shape<2, 2, 1, 2, 1, 3, 2, 32, 4, true>::launch(a, epi, p.parts, s);
-    case HALF_128x128: return Shape<2, 2, 2, 2, 1, 2, 4, 16, 4, false>::launch(a, epi, p.parts, s);
-    case HALF_128x128_8: return Shape<4, 2, 1, 2, 1, 2, 4, 32, 4, true>::launch(a, epi, p.parts, s);
-    case HALF_128x256: return Shape<2, 2, 2, 4, 1, 2, 4, 16, 0, false>::launch(a, epi, p.parts, s);
+    case HALF_64x128: return Shape<2, 2, 1, 2, 2, 1, 3, 2, 32, 4, true>::launch(a, epi, p.parts, s);
+    case HALF_128x128: return Shape<2, 2, 2, 2, 2, 1, 2, 4, 16, 4, false>::launch(a, epi, p.parts, s);
+    case HALF_128x128_8: return Shape<4, 2, 1, 2, 2, 1, 2, 4, 32, 4, true>::launch(a, epi, p.parts, s);
+    case HALF_128x256: return Shape<2, 2, 2, 4, 2, 1, 2, 4, 16, 0, false>::launch(a, epi, p.parts, s);
     default: return hipErrorInvalidValue;
   }
 }
 
-template <int EPI, int PW>
+template <int EPI, int PX, int PW>
 hipError_t launch_rows_form(const GemmArgs& a, const HalfPlan& p, hipStream_t s) {
   const unsigned n_blocks = (unsigned)((a.N + a.rows_per_block - 1) / a.rows_per_block), m_blocks = (unsigned)((a.M + 16 * p.mt - 1) / (16 * p.mt));
   if (m_blocks > 65535u) return hipErrorInvalidValue;
   const dim3 grid(n_blocks, (unsigned)p.parts, m_blocks);
   const int ng = (p.rows + 15) / 16;
 #define PG_CASE(MT, NG) \
-  if (p.mt == MT && ng == NG) { hipLaunchKernelGGL((k_gemm_half_rows<EPI, PW, MT, NG>), grid, dim3(512), 0, s, a); return hipGetLastError(); }
+  if (p.mt == MT && ng == NG) { hipLaunchKernelGGL((k_gemm_half_rows<EPI, PX, PW, MT, NG>), grid, dim3(512), 0, s, a); return hipGetLastError(); }
   PG_CASE(1, 1) PG_CASE(2, 1) PG_CASE(3, 1) PG_CASE(4, 1)
   PG_CASE(1, 2) PG_CASE(2, 2) PG_CASE(3, 2) PG_CASE(4, 2)
   PG_CASE(3, 3) PG_CASE(4, 3)
-  PG_CASE(3, 4) PG_CASE(4, 4)
+  if constexpr (PX == 2) { PG_CASE(3, 4) PG_CASE(4, 4) }
 #undef PG_CASE
   return hipErrorInvalidValue;
 }
-template <int PW>
+template <int PX, int PW>
 hipError_t launch_rows(const GemmArgs& a, int epi, const HalfPlan& p, hipStream_t s) {
-  if (p.parts > 1) return launch_rows_form<GEMM_BIAS, PW>(a, p, s);
+  if (p.parts > 1) return launch_rows_form<GEMM_BIAS, PX, PW>(a, p, s);
   switch (epi) {
-    case GEMM_BIAS: return launch_rows_form<GEMM_BIAS, PW>(a, p, s);
-    case GEMM_GELU: return launch_rows_form<GEMM_GELU, PW>(a, p, s);
-    case GEMM_RESID: return launch_rows_form<GEMM_RESID, PW>(a, p, s);
+    case GEMM_BIAS: return launch_rows_form<GEMM_BIAS, PX, PW>(a, p, s);
+    case GEMM_GELU: return launch_rows_form<GEMM_GELU, PX, PW>(a, p, s);
+    case GEMM_RESID: return launch_rows_form<GEMM_RESID, PX, PW>(a, p, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -770,8 +812,8 @@ hipError_t launch_rows(const GemmArgs& a, int epi, const HalfPlan& p, hipStream_
 // its wavefronts, and what it costs that blocks of the same rows of W lie on several XCDs (a number of them that eight does not
 // divide: 512 x 1280 x 1280 f32 rows, 48 rows of W 19.3 us, 40 rows 14.7).  And what is left to do behind it: the launch that adds
 // the parts, with or without a norm, per part and value, or a norm by itself.  Constants of the least regret over the four
-// projections of widths 512 to 1600 at 2 to 8192 rows, W from HBM (35000 plans): the plan of least predicted time is 2 % (f32 rows
-// 1.5 %) slower than the best measured one in the mean.
+// projections of widths 512 to 1600 at 2 to 8192 rows, W from HBM (35000 plans; cut form widths 512 and 768, 33 to 1024 rows): the
+// plan of least predicted time is 2 % (f32 rows 1.5 %, cut form 0.6 %) slower than the best measured one in the mean.
 struct TilePace {
   float start, stage, more, part;
 };
@@ -781,14 +823,17 @@ struct Finish {
 struct RowsPace {
   float start, turn, step, mt, ng, both, fill_mt, fill_ng, uneven;
 };
-// [one f16 number a weight][HalfTile]
-constexpr TilePace kTilePace[2][4] = {
+// [half form of f32 rows, of bf16 and int8 rows, cut form][HalfTile]
+constexpr TilePace kTilePace[3][4] = {
     {{5.981f, 0.546f, 0.074f, 0.197f}, {9.04f, 0.604f, 0.329f, 0.111f}, {7.24f, 0.503f, 11.3f, 2.426f}, {}},
-    {{5.243f, 0.389f, 0.027f, 0.13f}, {6.453f, 0.422f, 0.178f, 0.125f}, {5.701f, 0.36f, 1.06f, -0.021f}, {10.216f, 0.619f, 0.316f, 0.158f}}};
-constexpr Finish kFinish[2] = {{2.903f, 2.218f, 0.056f, 5.858f, -3.213f, 2.241f, 2.427f},
-                               {4.686f, 1.352f, 0.859f, 18.205f, -0.462f, 3.567f, 1.958f}};
-constexpr RowsPace kRowsPace[2] = {{6.051f, 0.928f, -0.147f, 0.191f, 0.302f, 0.003f, -0.07f, 0.019f, 0.077f},
-                                   {1.852f, 0.411f, -0.082f, 0.117f, 0.048f, 0.024f, 0.068f, 0.085f, 0.067f}};
+    {{5.243f, 0.389f, 0.027f, 0.13f}, {6.453f, 0.422f, 0.178f, 0.125f}, {5.701f, 0.36f, 1.06f, -0.021f}, {10.216f, 0.619f, 0.316f, 0.158f}},
+    {{3.39f, 0.667f, 0.426f, -0.051f}, {}, {3.014f, 0.924f, 0.685f, 0.149f}, {}}};
+constexpr Finish kFinish[3] = {{2.903f, 2.218f, 0.056f, 5.858f, -3.213f, 2.241f, 2.427f},
+                               {4.686f, 1.352f, 0.859f, 18.205f, -0.462f, 3.567f, 1.958f},
+                               {3.025f, 1.971f, 0.603f, 0.682f, 0.016f, 1.99f, 5.505f}};
+constexpr RowsPace kRowsPace[3] = {{6.051f, 0.928f, -0.147f, 0.191f, 0.302f, 0.003f, -0.07f, 0.019f, 0.077f},
+                                   {1.852f, 0.411f, -0.082f, 0.117f, 0.048f, 0.024f, 0.068f, 0.085f, 0.067f},
+                                   {3.29f, 1.262f, 0.536f, 0.049f, -0.171f, 0.155f, -0.052f, -0.005f, 0.369f}};
 
 }  // namespace
 
@@ -797,18 +842,18 @@ bool gemm_half_takes(const GemmArgs& a, int epi) {
                        reinterpret_cast<uintptr_t>(a.w_half_mul) | reinterpret_cast<uintptr_t>(a.bias) |
                        reinterpret_cast<uintptr_t>(a.resid) | reinterpret_cast<uintptr_t>(a.ws) | reinterpret_cast<uintptr_t>(a.ln_out) |
                        reinterpret_cast<uintptr_t>(a.ln_g) | reinterpret_cast<uintptr_t>(a.ln_b);
-  return a.w_half && a.w_half_mul && (a.w_half_parts == 1 || a.w_half_parts == 2) && !(at & 15) && a.M >= 1 && a.M < (1 << 23) &&
+  return a.w_half && (a.w_half_parts == 3 || (a.w_half_mul && (a.w_half_parts == 1 || a.w_half_parts == 2))) && !(at & 15) && a.M >= 1 && a.M < (1 << 23) &&
          a.K >= 64 && a.K % 32 == 0 && a.N >= 64 && a.N % 8 == 0 && a.N < (1 << 24) && a.ldc % 4 == 0 && a.a_unscale > 0.0f &&
          (epi == GEMM_GELU) == (a.c_scale > 0.0f) &&
          (epi == GEMM_BIAS || epi == GEMM_GELU || epi == GEMM_RESID) && (epi != GEMM_GELU || a.ldc == a.N);
 }
 
 HalfPlan gemm_half_plan(const GemmArgs& a, int epi, int num_cus) {
-  const bool one = a.w_half_parts == 1;
+  const int kind = a.w_half_parts == 1 ? 1 : a.w_half_parts == 2 ? 0 : 2;
   const int steps = a.K / 32, cus = num_cus;
   const float mn = (float)a.M * (float)a.N * 1e-6f;
   const int most = epi != GEMM_GELU && a.ws ? (int)std::min<size_t>(std::min(8, a.K / 256), a.ws_floats / ((size_t)a.M * a.N)) : 1;
-  const Finish& f = kFinish[one];
+  const Finish& f = kFinish[kind];
   auto finish = [&](int parts) {
     if (parts == 1) return a.ln_out ? f.norm + f.norm_values * mn : 0.0f;
     return (a.ln_out ? f.reduce_norm : f.reduce) + (f.part * (float)parts + (a.ln_out ? f.values_norm : f.values)) * mn;
@@ -819,21 +864,21 @@ HalfPlan gemm_half_plan(const GemmArgs& a, int epi, int num_cus) {
     if (us < best_us) best = p, best_us = us;
   };
   for (int t : {HALF_64x128, HALF_128x128, HALF_128x128_8, HALF_128x256}) {
-    if (t == HALF_128x256 && !one) continue;
+    if ((t == HALF_128x256 && kind != 1) || (t == HALF_128x128 && kind == 2)) continue;
     const int bm = t == HALF_64x128 ? 64 : 128, bn = t == HALF_128x256 ? 256 : 128;
     const long tiles = (long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
     for (int parts = 1; parts <= std::max(1, most); ++parts) {
       const long items = (tiles + 7) / 8 * 8 * parts;  // (as many to each XCD as the fullest one has)
       const float on_cu = (float)((items + cus - 1) / cus), round = std::max(0.0f, (float)items / (float)cus - 1.0f);
-      const TilePace& p = kTilePace[one][t];
+      const TilePace& p = kTilePace[kind][t];
       take({t, parts, 0, 0}, p.start + (float)((steps + parts - 1) / parts) * (p.stage + (on_cu - 1.0f) * p.more + round * p.part) + finish(parts));
     }
   }
   const int groups = (a.M + 63) / 64, mt = ((a.M + groups - 1) / groups + 15) / 16;
   const int m_blocks = (a.M + 16 * mt - 1) / (16 * mt);
-  const RowsPace& p = kRowsPace[one];
+  const RowsPace& p = kRowsPace[kind];
   for (int parts = 1; parts <= std::max(1, most); ++parts)
-    for (int rows = 8; rows <= (mt <= 2 ? 32 : 64); rows += 8) {
+    for (int rows = 8; rows <= (mt <= 2 ? 32 : kind == 2 ? 48 : 64); rows += 8) {
       const int ng = (rows + 15) / 16;
       const int n_blocks = (a.N + rows - 1) / rows;
       const long blocks = (long)n_blocks * m_blocks * parts;
@@ -853,7 +898,7 @@ hipError_t launch_gemm_half_plan(const GemmArgs& a0, int epi, const HalfPlan& p,
   if (p.tile != HALF_ROWS) return launch_tile(a, epi, p, s);
   if (p.rows < 8 || p.rows % 8 != 0 || p.mt < 1) return hipErrorInvalidValue;
   a.rows_per_block = p.rows;
-  return a.w_half_parts == 2 ? launch_rows<2>(a, epi, p, s) : launch_rows<1>(a, epi, p, s);
+  return a.w_half_parts == 3 ? launch_rows<3, 3>(a, epi, p, s) : a.w_half_parts == 2 ? launch_rows<2, 2>(a, epi, p, s) : launch_rows<2, 1>(a, epi, p, s);
 }
 
 hipError_t launch_gemm_half(const GemmArgs& a, int epi, int num_cus, hipStream_t s) {
@@ -864,7 +909,7 @@ hipError_t launch_gemm_half(const GemmArgs& a, int epi, int num_cus, hipStream_t
 }
 hipError_t finish_gemm_half(const GemmArgs& a, int epi, const HalfPlan& p, hipStream_t s) {
   if (p.parts == 1 && !a.ln_out) return hipSuccess;
-  if (!a.ln_out || a.ln_scale == 0.0f) {  // (a norm of f32 rows: the logits' input)
+  if (!a.ln_out || (a.ln_scale == 0.0f && !a.ln_cut)) {  // (a norm of f32 rows: the logits' input)
     if (p.parts == 1) return launch_layer_norm_rows(a.C, a.ln_out, a.M, a.N, a.ln_g, a.ln_b, a.ln_eps, s, a.ln_packed ? FORM_PACKED32 : FORM_ROWS);
     bool ln_done = false;
     const hipError_t e = launch_splitk_reduce(a, epi, p.parts, s, &ln_done);
@@ -892,6 +937,11 @@ hipError_t launch_half_rows(const void* W, int w_bytes, const float* scales, siz
   if (w_bytes == 4) hipLaunchKernelGGL(k_half_rows<0>, grid, dim3(256), 0, s, W, scales, to, mul, refused, (int)rows, cols);
   else if (w_bytes == 2) hipLaunchKernelGGL(k_half_rows<1>, grid, dim3(256), 0, s, W, scales, to, mul, refused, (int)rows, cols);
   else hipLaunchKernelGGL(k_half_rows<2>, grid, dim3(256), 0, s, W, scales, to, mul, refused, (int)rows, cols);
+  return hipGetLastError();
+}
+hipError_t launch_cut_weights(const float* W, size_t rows, int cols, void* to, hipStream_t s) {
+  if (cols % 32 != 0 || rows > (1u << 24)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_cut_weights, dim3((unsigned)((rows + 63) / 64)), dim3(256), 0, s, W, to, (int)rows, cols);
   return hipGetLastError();
 }
 hipError_t launch_half_bound(const void* W, int w_bytes, const float* scales, const float* g, const float* fold, size_t rows, int cols,

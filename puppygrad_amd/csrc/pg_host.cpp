@@ -521,7 +521,12 @@ pg_status make_half_form(pg_model* m) {
   const size_t C = g.C, I = g.I;
   const size_t rows[4] = {3 * C, C, I, C}, cols[4] = {C, C, C, I};
   size_t layer = 0;
-  for (int i = 0; i < 4; ++i) layer += up(rows[i] * cols[i] * 2 * pw) + up(rows[i] * 4);
+  // Small f32 models have their matrices in cut form too, for the rows that takes_cut_form has: reading W cut takes its cutting
+  // out of every block, at six bytes a weight instead of four.  The four products of a layer, us, W as stored / cut: width 768,
+  // 176 rows 49.7 / 41.0, 512 rows 76.3 / 71.2, 1024 rows 119 / 107; width 512, 512 rows 49.0 / 46.1; but width 1024, 192 rows
+  // 63.9 / 66.0, 320 rows 90.1 / 91.0, and 1280, 192 rows 81.9 / 85.6: there W's bytes are what counts.
+  const bool cut = wb == 4 && C <= 768;
+  for (int i = 0; i < 4; ++i) layer += up(rows[i] * cols[i] * 2 * pw) + up(rows[i] * 4) + (cut ? up(rows[i] * cols[i] * 6) : 0);
   constexpr int kBounds = 6;  // of a layer: both norms, hidden, queries, keys, values
   const size_t words = up((g.L * kBounds + 1) * 4);
   if (hipMalloc(&m->half_arena, g.L * layer + words) != hipSuccess) {
@@ -538,7 +543,7 @@ pg_status make_half_form(pg_model* m) {
     const pgk::LayerW& w = m->layers[l];
     const float* mats[4] = {w.c_attn_w, w.c_proj_w, w.c_fc_w, w.c_proj_mlp_w};
     const float* scales[4] = {w.c_attn_s, w.c_proj_s, w.c_fc_s, w.c_proj_mlp_s};
-    void* to[4];
+    void *to[4], *cut_to[4] = {};
     float* mul[4];
     for (int i = 0; i < 4; ++i) {
       to[i] = at;
@@ -546,8 +551,12 @@ pg_status make_half_form(pg_model* m) {
       mul[i] = reinterpret_cast<float*>(at);
       at += up(rows[i] * 4);
       PG_HIP(pgk::launch_half_rows(mats[i], wb, scales[i], rows[i], (int)cols[i], to[i], mul[i], refused, nullptr));
+      if (!cut) continue;
+      cut_to[i] = at;
+      at += up(rows[i] * cols[i] * 6);
+      PG_HIP(pgk::launch_cut_weights(mats[i], rows[i], (int)cols[i], cut_to[i], nullptr));
     }
-    m->half[l] = pg_model::HalfLayer{to[0], to[1], to[2], to[3], mul[0], mul[1], mul[2], mul[3], 0, 0, 0, {}};
+    m->half[l] = pg_model::HalfLayer{to[0], to[1], to[2], to[3], mul[0], mul[1], mul[2], mul[3], 0, 0, 0, {}, cut_to[0], cut_to[1], cut_to[2], cut_to[3]};
     unsigned* b = bounds + l * kBounds;
     PG_HIP(pgk::launch_half_bound_norm(w.ln_1_g, w.ln_1_b, (int)C, b, nullptr));
     PG_HIP(pgk::launch_half_bound_norm(w.ln_2_g, w.ln_2_b, (int)C, b + 1, nullptr));
@@ -607,6 +616,7 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
   // the projections' inputs (XN, ATT, HB) in half form or in cut form
   const bool half = !c->drawn && takes_half_form(m, n);
   const bool cut = !half && !c->drawn && takes_cut_form(m, n);
+  const bool cut_w = cut && T > 128 && !m->half.empty() && m->half[0].c_attn_cut;  // (64 rows and fewer: no faster)
   const int form_of = cut ? pgk::FORM_CUT : pgk::FORM_ROWS;
   {
     auto form = [&](size_t cols) { return cut ? std::max(n * cols, pgk::cut_floats(n, cols)) : half ? pgk::half_floats(n, cols) : n * cols; };
@@ -664,6 +674,7 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
     if (w_half) {
       a.w_half = w_half; a.w_half_mul = w_half_mul; a.w_half_parts = m->w_bf16 || m->w_i8 ? 1 : 2;
       a.a_unscale = 1.0f / a_scale; a.c_scale = c_scale; a.ln_scale = ln_g ? ln_scale : 0.0f;
+      if (cut) a.w_half_parts = 3, a.a_cut = a.c_cut = 0;  // (W is in cut form)
     }
     a.M = T; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc;
     if (m->w_i8) a.w_scale = i8_scales_of(W, (size_t)N, (size_t)K);
@@ -680,7 +691,11 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
   PG_MARK(kLayerNorm);
   for (size_t l = 0; l < g.L; ++l) {
     const pgk::LayerW& w = m->layers[l];
-    const pg_model::HalfLayer hw = half ? m->half[l] : pg_model::HalfLayer{};
+    pg_model::HalfLayer hw = half || cut_w ? m->half[l] : pg_model::HalfLayer{};
+    if (cut_w) {
+      hw.c_attn = hw.c_attn_cut, hw.c_proj = hw.c_proj_cut, hw.c_fc = hw.c_fc_cut, hw.c_proj_mlp = hw.c_proj_mlp_cut;
+      hw.norm_1 = hw.norm_2 = hw.hidden = hw.attn.v = 1.0f;  // (cut form is not scaled)
+    }
     // the LayerNorm after this layer: the next layer's ln_1; ln_f is applied where it is needed
     const float* next_g = l + 1 < g.L ? m->layers[l + 1].ln_1_g : nullptr;
     const float* next_b = l + 1 < g.L ? m->layers[l + 1].ln_1_b : nullptr;
@@ -697,7 +712,7 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
                                       ATT.p, SCR.p, m->num_cus, s, (int)nb, g.H * g.P * g.hd(), form_of, c->drawn));
     PG_MARK(kAttention);
     PG_HIP(gemm(ATT.p, C, w.c_proj_w, w.c_proj_b, X.p, C, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b, cut, 0,
-                hw.c_proj, hw.c_proj_mul, hw.attn.v, 0.0f, hw.norm_2));
+                hw.c_proj, hw.c_proj_mul, hw.attn.v, 0.0f, half ? hw.norm_2 : 0.0f));
     PG_MARK(kAttnProj);
     PG_HIP(gemm(XN.p, C, w.c_fc_w, w.c_fc_b, HB.p, I, I, C, pgk::GEMM_GELU, nullptr, nullptr, cut, cut,
                 hw.c_fc, hw.c_fc_mul, hw.norm_2, hw.hidden));

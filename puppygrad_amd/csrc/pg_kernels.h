@@ -266,6 +266,7 @@ struct GemmArgs {
   // a_unscale > 0: A is in half form (FORM_HALF), its values 1 / a_unscale times what they stand for, and W's half form is
   // w_half (launch_half_rows), of w_half_parts f16 numbers a weight.  GEMM_GELU then writes C in half form, times c_scale,
   // and ln_out is in half form, times ln_scale (0: as it would be otherwise); no other form goes with it.  Powers of two.
+  // w_half_parts 3 (f32 rows): A, C of GEMM_GELU and, with ln_cut, ln_out are in cut form, W in launch_cut_weights'; the scales are 1.
   const void* w_half = nullptr;
   const float* w_half_mul = nullptr;
   int w_half_parts = 0;
@@ -306,6 +307,8 @@ hipError_t launch_norm_rows_half(float* src, void* dst, int rows, int cols, cons
 // rows) or one, cols a multiple of 32, and what a sum over them is to be multiplied with, mul[rows].  *refused is set (never
 // cleared) where the rows do not allow it (k_half_rows).
 constexpr int kHalfMostExp = 60;
+// f32 rows in cut form, three bf16 numbers a weight, for inputs in cut form.
+hipError_t launch_cut_weights(const float* W, size_t rows, int cols, void* to, hipStream_t s);
 hipError_t launch_half_rows(const void* W, int w_bytes, const float* scales, size_t rows, int cols, void* to, float* mul,
                             unsigned* refused, hipStream_t s);
 // *most = max(*most, the largest magnitude that an output of these rows behind a LayerNorm with scale g can have; fold as

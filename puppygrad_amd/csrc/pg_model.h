@@ -135,6 +135,7 @@ struct pg_model {
     const float *c_attn_mul, *c_proj_mul, *c_fc_mul, *c_proj_mlp_mul;
     float norm_1, norm_2, hidden;
     pgk::HalfScales attn;  // queries, keys, values (and what attention makes of them)
+    const void *c_attn_cut, *c_proj_cut, *c_fc_cut, *c_proj_mlp_cut;  // the same matrices in cut form, or null
   };
   char* half_arena = nullptr;
   std::vector<HalfLayer> half;

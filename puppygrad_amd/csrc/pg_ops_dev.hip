@@ -438,8 +438,8 @@ pg_status pg_testing_cut_product_dev(int32_t device, void* stream, const float* 
 
 // x, times scale, in half form through pg_gemm_half.hip: the given tile (pgk::HalfTile), or blocks of 16 mt input rows and `block_rows`
 // rows of W, K in `parts` parts (more than one: the raw parts [parts][rows][out_f] to out, without bias); gelu: with GELU, out
-// in half form times 1.  work: 4 * in_f * (rows rounded up to 16) bytes, as many as W's half form takes, 4 * out_f and 4, each
-// rounded up to 256; its last word says whether W was refused.
+// in half form times 1.  scale 0 (f32 rows): all of it in cut form instead.  work: 4 (6) * in_f * (rows rounded up to 16) bytes, as
+// many as W's half form takes (cut form 6 * in_f * out_f), 4 * out_f and 4, each rounded up to 256; its last word says whether W was refused.
 pg_status pg_testing_half_product_dev(int32_t device, void* stream, const float* x, uint64_t rows, uint64_t in_f,
                                       uint64_t out_f, const void* weight, int32_t storage, const float* scales,
                                       const float* bias, float* out, float scale, int32_t tile, int32_t parts, int32_t mt,
@@ -453,17 +453,25 @@ pg_status pg_testing_half_product_dev(int32_t device, void* stream, const float*
   if ((s = select_device(device))) return s;
   hipStream_t st = static_cast<hipStream_t>(stream);
   auto up = [](size_t n) { return (n + 255) / 256 * 256; };
-  const int pw = storage == PG_STORE_F32 ? 2 : 1;
-  char* w_half = work + up(in_f * pgk::cut_rows((int)rows) * 4);
+  const bool cut = scale == 0.0f;
+  if (cut && storage != PG_STORE_F32) return pgh::fail(PG_INVALID_INPUT, "cut form: f32 rows");
+  const int pw = cut ? 3 : storage == PG_STORE_F32 ? 2 : 1;
+  char* w_half = work + up(in_f * pgk::cut_rows((int)rows) * (cut ? 6 : 4));
   float* mul = reinterpret_cast<float*>(w_half + up(in_f * out_f * 2 * pw));
   unsigned* refused = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(mul) + up(out_f * 4));
   PG_HIP(pgk::launch_fill_zero(reinterpret_cast<float*>(refused), 1, st));
-  PG_HIP(pgk::launch_half_rows(weight, storage == PG_STORE_F32 ? 4 : storage == PG_STORE_BF16 ? 2 : 1, scales, out_f, (int)in_f,
-                               w_half, mul, refused, st));
-  hipLaunchKernelGGL(k_to_half, dim3((unsigned)((rows * in_f / 4 + 255) / 256)), dim3(256), 0, st, x, work, (int)rows, (int)in_f, scale);
+  const dim3 x_blocks((unsigned)((rows * in_f / 4 + 255) / 256));
+  if (cut) {
+    PG_HIP(pgk::launch_cut_weights(static_cast<const float*>(weight), out_f, (int)in_f, w_half, st));
+    hipLaunchKernelGGL(k_to_cut, x_blocks, dim3(256), 0, st, x, work, (int)rows, (int)in_f);
+  } else {
+    PG_HIP(pgk::launch_half_rows(weight, storage == PG_STORE_F32 ? 4 : storage == PG_STORE_BF16 ? 2 : 1, scales, out_f, (int)in_f,
+                                 w_half, mul, refused, st));
+    hipLaunchKernelGGL(k_to_half, x_blocks, dim3(256), 0, st, x, work, (int)rows, (int)in_f, scale);
+  }
   PG_HIP(hipGetLastError());
   pgk::GemmArgs a{};
-  a.A = reinterpret_cast<const float*>(work); a.w_half = w_half; a.w_half_mul = mul; a.w_half_parts = pw; a.a_unscale = 1.0f / scale;
+  a.A = reinterpret_cast<const float*>(work); a.w_half = w_half; a.w_half_mul = mul; a.w_half_parts = pw; a.a_unscale = cut ? 1.0f : 1.0f / scale;
   a.bias = bias; a.C = out; a.M = (int)rows; a.N = (int)out_f; a.K = (int)in_f; a.ldc = (int)out_f;
   a.ws = out; a.ws_floats = (size_t)parts * rows * out_f;
   if (gelu) a.c_scale = 1.0f;

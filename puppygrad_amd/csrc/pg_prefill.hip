@@ -1668,7 +1668,7 @@ hipError_t launch_gemm(const GemmArgs& a, int epi, int num_cus, hipStream_t s) {
   if (a.post_x && (epi != GEMM_BIAS || a.ln_out || a.ldc != a.N)) return hipErrorInvalidValue;
   if (a.raw_parts && (epi != GEMM_BIAS || a.bias || a.ln_out || a.post_x)) return hipErrorInvalidValue;
   if (a.a_unscale != 0.0f)
-    return a.post_x || a.raw_parts || a.rms_cols || a.a_cut || a.c_cut || a.ln_cut || a.a_packed || a.c_packed || (a.ln_packed && a.ln_scale != 0.0f)
+    return a.post_x || a.raw_parts || a.rms_cols || a.a_cut || a.c_cut || (a.ln_cut && a.w_half_parts != 3) || a.a_packed || a.c_packed || (a.ln_packed && a.ln_scale != 0.0f)
                ? hipErrorInvalidValue
                : launch_gemm_half(a, epi, num_cus, s);
   bool ln_done = false;

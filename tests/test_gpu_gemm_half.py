@@ -13,6 +13,8 @@ pytestmark = pytest.mark.gpu
 STORE = {"f32": _lib.PG_STORE_F32, "bf16": _lib.PG_STORE_BF16, "int8": _lib.PG_STORE_INT8}
 TILE_64x128, TILE_128x128, TILE_128x128_8, TILE_128x256, ROWS = range(5)
 FORMS = [(s, t, 0, 0) for s in STORE for t in (TILE_64x128, TILE_128x128, TILE_128x128_8, TILE_128x256) if s != "f32" or t != TILE_128x256]
+FORMS += [("cut", t, 0, 0) for t in (TILE_64x128, TILE_128x128_8)]  # f32 rows, both operands in cut form
+FORMS += [("cut", ROWS, mt, rows) for mt in (1, 2, 3, 4) for rows in (8, 16, 24, 32, 40, 48) if mt > 2 or rows <= 32]
 FORMS += [(s, ROWS, mt, rows) for s in STORE for mt in (1, 2, 3, 4) for rows in (8, 16, 24, 32, 40, 48, 56, 64) if mt > 2 or rows <= 32]
 
 
@@ -28,9 +30,10 @@ def half_product_dev(x, w, bias, scales, scale, tile, parts, mt, rows, gelu=Fals
     (m, k), n = x.shape, w.shape[0]
     storage = {np.dtype(np.float32): "f32", np.dtype(np.uint16): "bf16", np.dtype(np.int8): "int8"}[w.dtype]
     mp = (m + 15) // 16 * 16
-    size = up(4 * k * mp) + up(k * n * (4 if storage == "f32" else 2)) + up(4 * n) + 256
+    cut = scale == 0
+    size = up((6 if cut else 4) * k * mp) + up(k * n * (6 if cut else 4 if storage == "f32" else 2)) + up(4 * n) + 256
     # (room for padded rows: NaN, which no result may show)
-    held = [DeviceArray(x), DeviceArray(w, dtype=w.dtype), DeviceArray(np.full(parts * max(m, mp) * n, np.nan, np.float32)), DeviceArray(bias),
+    held = [DeviceArray(x), DeviceArray(w, dtype=w.dtype), DeviceArray(np.full(parts * max(m, mp) * n * (3 if cut and gelu else 2) // 2, np.nan, np.float32)), DeviceArray(bias),
             DeviceArray(np.full(size // 4, np.nan, np.float32))]
     if scales is not None:
         held.append(DeviceArray(scales))
@@ -41,6 +44,9 @@ def half_product_dev(x, w, bias, scales, scale, tile, parts, mt, rows, gelu=Fals
         d.free()
     assert status == 0, _lib.load().pg_last_error_message().decode()
     refused = work.view(np.uint32)[(size - 256) // 4] != 0
+    if gelu and cut:  # back from cut form
+        bf16 = got.view(np.uint16).reshape(-1)[:3 * n * mp].reshape(n // 8, 3, mp, 8)[:, :, :m].astype(np.uint32) << 16
+        return bf16.view(np.float32).astype(np.float64).sum(1).transpose(1, 0, 2).reshape(m, n), refused
     if gelu:  # back from half form
         parts_of = got.view(np.float16).reshape(-1)[:2 * n * mp].reshape(n // 8, 2, mp, 8)[:, :, :m].astype(np.float64)
         return parts_of.sum(1).transpose(1, 0, 2).reshape(m, n), refused
@@ -53,7 +59,7 @@ def operands(m, k, n, storage):
     x = (rng.standard_normal((m, k)) * 10.0 ** rng.uniform(-3, 1, (m, k))).astype(np.float32)
     w = (rng.standard_normal((n, k)) * 10.0 ** rng.uniform(-3, 1, (n, 1))).astype(np.float32)
     b = rng.standard_normal(n).astype(np.float32)
-    if storage == "f32":
+    if storage in ("f32", "cut"):
         return x, w, None, w.astype(np.float64), b
     if storage == "bf16":
         w = synth.round_bf16(w.reshape(-1)).reshape(w.shape)
@@ -64,9 +70,11 @@ def operands(m, k, n, storage):
 
 def bound_of(x, w, b, scale):
     """f32 sums of K products in any order, their operands off by 2^-23 (of x besides 2^-25 of the scaled unit) and lo lo left
-    out, 2^-22; the bias and an int8 row's scale each rounded once."""
+    out, 2^-22; the bias and an int8 row's scale each rounded once.  Cut form (scale 0): the operands are whole, three of nine
+    products are left out, 2^-24 and less together."""
     want = x @ w.T + b
-    return want, (x.shape[1] + 20) * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T) + 2.0 ** -25 / scale * np.abs(w).sum(1) + 2.0 ** -23 * np.abs(want)
+    unit = 2.0 ** -25 / scale if scale else 0.0
+    return want, (x.shape[1] + 20) * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T) + unit * np.abs(w).sum(1) + 2.0 ** -23 * np.abs(want)
 
 
 # a row, an octet of columns more than a tile, two stages of K; a tile's rows and one more or less on both sides; chains of uneven
@@ -76,8 +84,9 @@ def bound_of(x, w, b, scale):
 @pytest.mark.parametrize("storage,tile,mt,rows", FORMS)
 def test_forms_at_their_edges(storage, tile, mt, rows, m, k, n, parts):
     x, w, scales, values, b = operands(m, k, n, storage)
-    got, refused = half_product_dev(x, w, b, scales, 256.0, tile, parts, mt, rows)
-    want, bound = bound_of(x.astype(np.float64), values, b, 256.0)
+    scale = 0.0 if storage == "cut" else 256.0
+    got, refused = half_product_dev(x, w, b, scales, scale, tile, parts, mt, rows)
+    want, bound = bound_of(x.astype(np.float64), values, b, scale)
     assert not refused and (np.abs(got - want) <= bound).all(), f"{(np.abs(got - want) / bound).max():.2f} of the bound"
 
 
@@ -101,11 +110,25 @@ def test_every_product_of_the_parts_counts(storage, tile, mt, rows):
     assert (np.abs(got - want) <= 64 * 2.0 ** -24 * want).all(), (np.abs(got - want) / want).max() * 2.0 ** 24
 
 
-@pytest.mark.parametrize("tile,mt,rows", [(TILE_64x128, 0, 0), (TILE_128x256, 0, 0), (ROWS, 4, 40)])
-def test_gelu_in_half_form(tile, mt, rows):
-    x, w, scales, values, b = operands(77, 96, 136, "bf16")
-    got, _ = half_product_dev(x, w, b, scales, 64.0, tile, 1, mt, rows, gelu=True)
-    want, bound = bound_of(x.astype(np.float64), values, b, 64.0)
+@pytest.mark.parametrize("tile,mt,rows", [(TILE_64x128, 0, 0), (TILE_128x128_8, 0, 0), (ROWS, 1, 16), (ROWS, 3, 24), (ROWS, 4, 48)])
+def test_every_product_of_the_cut_parts_counts(tile, mt, rows):
+    """Operands 1 + 2^-9 + 2^-18 and a little: left out, one of the six products is 2^-18 of the sum at least."""
+    rng = np.random.default_rng(6)
+    x, w = ((1.0 + 2.0 ** -9 + 2.0 ** -18 + rng.integers(0, 4, (n, 64)) * 2.0 ** -22).astype(np.float32) for n in (70, 136))
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    got, _ = half_product_dev(x, w, np.zeros(len(w), np.float32), None, 0.0, tile, 1, mt, rows)
+    # (the first parts' products are 1, their sums whole numbers; the small ones' sum, 2^-8 of them, is off by 2^-18 of itself at most;
+    # the last additions round three times; three products of 2^-27 are left out)
+    assert (np.abs(got - want) <= 5 * 2.0 ** -24 * want).all(), (np.abs(got - want) / want).max() * 2.0 ** 24
+
+
+@pytest.mark.parametrize("storage,tile,mt,rows", [("bf16", TILE_64x128, 0, 0), ("bf16", TILE_128x256, 0, 0), ("bf16", ROWS, 4, 40),
+                                                  ("cut", TILE_64x128, 0, 0), ("cut", TILE_128x128_8, 0, 0), ("cut", ROWS, 4, 48)])
+def test_gelu_in_half_and_cut_form(storage, tile, mt, rows):
+    x, w, scales, values, b = operands(77, 96, 136, storage)
+    scale = 0.0 if storage == "cut" else 64.0
+    got, _ = half_product_dev(x, w, b, scales, scale, tile, 1, mt, rows, gelu=True)
+    want, bound = bound_of(x.astype(np.float64), values, b, scale)
     gelu = 0.5 * want * (1.0 + np.tanh(np.sqrt(2.0 / np.pi) * (want + 0.044715 * want ** 3)))
     # (its slope is at most 1.13; f32 arithmetic of a few steps; 2^-25 of half form's unit)
     assert (np.abs(got - gelu) <= 1.13 * bound + 2.0 ** -20 * np.abs(want) + 2.0 ** -24).all()
@@ -134,7 +157,7 @@ def logits(model, ids):
 
 # the first rows that take the form, tiles that end in the middle, one prompt and several
 @pytest.mark.parametrize("storage,width,batch,n", [("f32", 768, 1, 5), ("f32", 1280, 1, 32), ("bf16", 1600, 1, 17), ("int8", 1024, 2, 33), ("bf16", 768, 1, 270),
-                                                   ("int8", 1280, 1, 190), ("f32", 768, 1, 1026), ("f32", 1280, 1, 257), ("bf16", 1024, 1, 330), ("int8", 1600, 1, 460),
+                                                   ("int8", 1280, 1, 190), ("f32", 768, 1, 1026), ("f32", 768, 1, 129), ("f32", 512, 3, 300), ("f32", 768, 4, 256), ("f32", 1280, 1, 257), ("bf16", 1024, 1, 330), ("int8", 1600, 1, 460),
                                                    ("f32", 1600, 3, 131), ("bf16", 768, 5, 207), ("int8", 768, 2, 700), ("f32", 512, 9, 130)])
 def test_prompts(storage, width, batch, n):
     cfg = Gpt2Config(vocab_size=300, n_positions=1100, n_embd=width, n_layer=2, n_head=width // 64)
