@@ -447,7 +447,8 @@ struct Norm {
       : mean((double)sum / n) {
     const double v = (double)squares / n + (double)eps;
     const double y = (double)(1.0f / sqrtf((float)v));
-    inv = y * (1.5 - 0.5 * v * y * y);  // (one Newton step of the root)
+    // (one Newton step of the root; squares that are past f32 leave 0, as they do in f32)
+    inv = v < (double)INFINITY ? y * (1.5 - 0.5 * v * y * y) : y;
   }
   // four columns of a row, part by part `stride` bytes apart: half form (PX 2), times scale, or cut form (3)
   template <int PX>

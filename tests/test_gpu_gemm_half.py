@@ -228,6 +228,19 @@ def test_scales_hold_for_models_of_any_size_of_values():
         assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want), (gain, weight)
 
 
+@pytest.mark.parametrize("n", [20, 300])  # a block a row, a wavefront a row
+def test_rows_whose_squares_are_past_f32(n):
+    """Their norm is its shift, in half form as in f32 rows."""
+    cfg = Gpt2Config(vocab_size=97, n_positions=400, n_embd=1600, n_layer=2, n_head=25)
+    w = synth.random_weights(cfg, 0x5EED0B05, perturb=True)
+    w.wte = w.wte * np.float32(1e22)
+    w.wpe = w.wpe * np.float32(1e22)
+    ids = [int(t) for t in synth.token_ids(n, 0x70C00B05, 97)]
+    here, there = (Gpt2Model.new(cfg, w, Gpt2HipConfig(gemm_b9_min_rows=b)) for b in (0, 0xffffffff))
+    got, want = logits(here, ids) / np.float32(1e22), logits(there, ids) / np.float32(1e22)
+    assert np.isfinite(want).all() and np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
+
+
 def test_weights_without_half_form_are_served_as_before():
     cfg = Gpt2Config(vocab_size=97, n_positions=400, n_embd=512, n_layer=1, n_head=8)
     ids = [int(t) for t in synth.token_ids(400, 0x70C00B03, 97)]
