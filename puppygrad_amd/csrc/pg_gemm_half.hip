@@ -623,8 +623,9 @@ hipError_t launch_norm_rows(const GemmArgs& a, int parts, hipStream_t s) {
 // ---- weights -----------------------------------------------------------------------------------
 // Rows of W as stored (WT as elsewhere: f32, bf16, int8 with their scales) to half form: part p of element (n, k) is the
 // (k % 8)-th f16 of the 16 bytes at ((k / 8 * PW + p) * N + n) * 16, times mul[n]^-1; a f32 or bf16 row is scaled by the power of
-// two that puts its largest value between 2^14 and 2^15.  *refused is set where a bf16 weight is not a f16 number so (a row
-// that spans more than 2^32), a value is not finite, or a row is so small or large that its power of two would matter.
+// two that puts its largest value between 2^14 and 2^15.  A bf16 weight is then a f16 number as it is down to 2^-32 of the row's
+// largest and right to 2^-40 of that below, as a f32 weight's lo part is (of normally distributed weights one in 10^9 is as small:
+// a large model has some).  *refused is set where a value is not finite or a row so small or large that its power of two would matter.
 template <int WT>
 __global__ __launch_bounds__(256) void k_half_rows(const void* W, const float* scales, void* to, float* mul, unsigned* refused,
                                                    int N, int K) {
@@ -679,8 +680,6 @@ __global__ __launch_bounds__(256) void k_half_rows(const void* W, const float* s
       unsigned hi, lo;
       halves2(x[2 * e], x[2 * e + 1], scale, hi, lo);
       h[e] = hi, l[e] = lo;
-      const h2v f = __builtin_bit_cast(h2v, hi);
-      if (PW == 1) bad |= (float)f.x != x[2 * e] * scale || (float)f.y != x[2 * e + 1] * scale;
     }
     if (n < N) {
       u4v* at = static_cast<u4v*>(to) + (size_t)(k / 8) * PW * N + n;

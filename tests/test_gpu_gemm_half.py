@@ -136,19 +136,23 @@ def test_gelu_in_half_and_cut_form(storage, tile, mt, rows):
 
 @pytest.mark.parametrize("storage", ["f32", "bf16"])
 def test_weights_that_half_form_refuses(storage):
-    """Values that are not finite; a row too small or too large to be scaled; bf16: a row that spans more than f16 numbers do."""
+    """Values that are not finite; a row too small or too large to be scaled.  Not: a row that spans more than f16 numbers do, whose
+    small weights are right to 2^-40 of its largest."""
     x, _, _, _, b = operands(40, 64, 64, "f32")
     rng = np.random.default_rng(3)
     for value, least, refused in ((1.0, 2.0 ** -20, False), (np.inf, 1.0, True), (np.nan, 1.0, True), (2.0 ** 80, 1.0, True),
-                                  (2.0 ** -80, None, True), (1.0, 2.0 ** -45, storage == "bf16"), (0.0, 0.0, False)):
+                                  (2.0 ** -80, None, True), (1.0, 2.0 ** -45, False), (1.0, 2.0 ** -36, False), (0.0, 0.0, False)):
         w = synth.round_bf16(rng.standard_normal(64 * 64).astype(np.float32)).reshape(64, 64)
         if least is None or value == 0.0:
             w[5] = 0.0
         else:
             w[5, 9] = np.float32(1.0078125 * least)
         w[5, 7] = value
-        _, got = half_product_dev(x, as_bf16(w) if storage == "bf16" else w, b, None, 256.0, TILE_64x128, 1, 0, 0)
+        product, got = half_product_dev(x, as_bf16(w) if storage == "bf16" else w, b, None, 256.0, TILE_64x128, 1, 0, 0)
         assert got == refused, (value, least)
+        if not refused:
+            want, bound = bound_of(x.astype(np.float64), w.astype(np.float64), b, 256.0)
+            assert (np.abs(product - want) <= bound + 2.0 ** -40 * np.abs(w).max(1) * np.abs(x).sum(1, keepdims=True)).all(), (value, least)
 
 
 def logits(model, ids):
@@ -205,6 +209,17 @@ def test_a_set_bound_holds_for_few_rows():
     np.testing.assert_array_equal(past, never)
     np.testing.assert_array_equal(at, alone)
     assert (at != never).any()
+
+
+def test_a_bf16_weight_far_below_its_row_does_not_cost_a_model_its_form():
+    cfg = Gpt2Config(vocab_size=97, n_positions=64, n_embd=768, n_layer=1, n_head=12)
+    w = synth.random_weights(cfg, 0x5EED0B06, perturb=True)
+    ids = [int(t) for t in synth.token_ids(40, 0x70C00B06, 97)]
+    bf16 = Gpt2HipConfig(weight_storage=STORE["bf16"])
+    w.blocks[0].c_fc_w.reshape(-1)[5] = 0.0
+    want = logits(Gpt2Model.new(cfg, w, bf16), ids)
+    w.blocks[0].c_fc_w.reshape(-1)[5] = 1.0078125 * 2.0 ** -60
+    np.testing.assert_array_equal(logits(Gpt2Model.new(cfg, w, bf16), ids), want)  # (0 in that form; elsewhere other kernels' sums)
 
 
 def test_scales_hold_for_models_of_any_size_of_values():
