@@ -347,7 +347,7 @@ def measure_short_prefill(model, cfg, ids, T, steps, warmup):
     return {"workload": f"GPT-2 124M fp32 B=1 prefill of a {T}-token prompt into an empty KV cache (first-token latency)",
             "value": round(T / sec, 1), "unit": "tokens/s", "steps": steps, "ms_per_step": round(sec * 1e3, 4),
             "roofline": hbm_roofline(wbytes / sec / 1e9,
-                                     "whole prefill (k_gemm_rows32, k_attn_prefill64, k_splitk_reduce_ln, lm_head)",
+                                     "whole prefill (k_gemm_half_rows, k_attn_prefill_half, k_norm_row_half, lm_head)",
                                      traffic=TRAFFIC_124M_PREFILL_32 if T == 32 else None,
                                      traffic_source=TRAFFIC_SOURCE_124M_PREFILL if T == 32 else None,
                                      algorithmic_bytes_per_step=int(wbytes))}
@@ -380,7 +380,7 @@ def measure_prefill(model, cfg, ids, T, steps, warmup):
                          "unit": "TFLOP/s", "frac": round(whole / FP32_MFMA_PEAK_TFLOPS, 4),
                          "traffic": TRAFFIC_124M_PREFILL_1024 if T == 1024 else None,
                          "traffic_source": TRAFFIC_SOURCE_124M_PREFILL if T == 1024 else None,
-                         "kernel": "whole prefill (k_gemm_cut, k_gemm, k_attn_prefill64, LayerNorm, split-K reduces, lm_head)",
+                         "kernel": "whole prefill (k_gemm_half, k_gemm_half_rows, k_attn_prefill_half, LayerNorm, split-K reduces, lm_head)",
                          "algorithmic_flops_per_step": int(flops)},
             "gemm_part": {"ms": round(gemm_s * 1e3, 4), "achieved": round(gemm, 2), "unit": "TFLOP/s",
                           "frac": round(gemm / FP32_MFMA_PEAK_TFLOPS, 4), "flops": int(gemm_flops),
@@ -429,14 +429,14 @@ def prefill_flops(cfg, B, T):
 
 
 def bf16_prefill_roofline(flops, gemm_flops, sec, traffic=None, traffic_source=None):
-    """bf16 rows: the projections run on the bf16 matrix cores, every f32 input cut into three
-    bf16 parts (exact products, f32 sums): three matrix instructions' worth of work per
-    algorithmic product, so a third of the bf16 peak is this form's ceiling."""
+    """bf16 rows: the projections run on the f16 matrix cores (the bf16 ones' rate), every f32 input
+    scaled and kept as two f16 parts (exact products, f32 sums): two matrix instructions' worth of
+    work per algorithmic product, so half of the peak is this form's ceiling."""
     achieved = flops / sec / 1e12
     r = {"bound": "mfma", "achieved": round(achieved, 2), "peak": BF16_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
-         "frac": round(achieved / BF16_MFMA_PEAK_TFLOPS, 4), "traffic": traffic, "passes": 3,
-         "executed": round((2 * gemm_flops + flops) / sec / 1e12, 2),
-         "kernel": "whole prefill (k_gemm_cut and k_attn_prefill_cut on the bf16 matrix cores, lm_head in f32)",
+         "frac": round(achieved / BF16_MFMA_PEAK_TFLOPS, 4), "traffic": traffic, "passes": 2,
+         "executed": round((gemm_flops + flops) / sec / 1e12, 2),
+         "kernel": "whole prefill (k_gemm_half and k_attn_prefill_half on the f16 matrix cores, lm_head in f32)",
          "algorithmic_flops_per_step": int(flops), "gemm_flops_per_step": int(gemm_flops)}
     if traffic_source:
         r["traffic_source"] = traffic_source
@@ -507,8 +507,8 @@ def bench_prefill(args, cfg, model, ids, n_prefill) -> int:
                    "backend": model.describe()},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 2), "peak": FP32_MFMA_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(achieved / FP32_MFMA_PEAK_TFLOPS, 4), "traffic": None,
-                     "kernel": "whole prefill (k_gemm, or k_gemm_cut where it is faster; "
-                               "k_attn_prefill64, LayerNorm, split-K reduces, lm_head)",
+                     "kernel": "whole prefill (k_gemm_half, k_gemm_half_rows or k_gemm by its rows; "
+                               "k_attn_prefill_half, LayerNorm, split-K reduces, lm_head)",
                      "algorithmic_flops_per_step": int(flops), "gemm_flops_per_step": int(gemm_flops)},
     }
     if args.bf16:
@@ -521,7 +521,7 @@ def bench_prefill(args, cfg, model, ids, n_prefill) -> int:
     wbytes = weight_bytes(cfg, bf16=args.bf16)
     if wbytes / (HBM_PEAK_GBS * 1e9) > flops / (FP32_MFMA_PEAK_TFLOPS * 1e12):
         gbs = wbytes / sec / 1e9
-        result["roofline"] = hbm_roofline(gbs, "whole prefill (k_gemm_rows32, k_attn_prefill64, reduce + LayerNorm, lm_head)",
+        result["roofline"] = hbm_roofline(gbs, "whole prefill (k_gemm_half_rows, k_attn_prefill_half, reduce + LayerNorm, lm_head)",
                                           algorithmic_bytes_per_step=int(wbytes))
     print(json.dumps(result), flush=True)
     return 0
@@ -695,8 +695,8 @@ TRAFFIC_SOURCE = "profiles/k_decode_persistent_1600_xl_decode_traffic.txt"
 TRAFFIC_RATIO_124M = 0.983
 TRAFFIC_SOURCE_124M = "profiles/k_decode_persistent_768_124m_decode.txt"
 # HBM bytes of one 124M prefill (FETCH_SIZE + WRITE_SIZE of all its launches, scaled)
-TRAFFIC_124M_PREFILL_1024 = 3175900000
-TRAFFIC_124M_PREFILL_32 = 630900000
+TRAFFIC_124M_PREFILL_1024 = 4435300000
+TRAFFIC_124M_PREFILL_32 = 610200000
 TRAFFIC_SOURCE_124M_PREFILL = "profiles/prefill_124m_traffic.txt"
 TRAFFIC_RATIO_355M_B16 = 1.093
 TRAFFIC_RATIO_XL_BF16_B32 = 1.073  # same file, section (c)
@@ -704,8 +704,8 @@ TRAFFIC_SOURCE_355M_B16 = "profiles/batched_decode_355m_b16_xl_bf16_b32.txt"
 # Bytes through the L2s to and from the fabric per XL bf16 prefill of 32 x 512 tokens (FETCH_SIZE
 # scaled by 1.9994 + WRITE_SIZE over all launches of a step; most of the reads are operand
 # re-reads that the Infinity Cache serves).
-TRAFFIC_XL_BF16_PREFILL_B32_512 = 372600000000
-TRAFFIC_SOURCE_XL_BF16_PREFILL = "profiles/k_gemm_cut_xl_bf16_prefill_b32_512.txt"
+TRAFFIC_XL_BF16_PREFILL_B32_512 = 329700000000
+TRAFFIC_SOURCE_XL_BF16_PREFILL = "profiles/k_gemm_half_prompts.txt"
 
 
 def measured_traffic(args, n_prefill, persistent, bytes_per_launch):

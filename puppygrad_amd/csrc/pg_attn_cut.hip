@@ -1,4 +1,4 @@
-// Causal attention of prompts on the bf16 matrix cores.
+// Causal attention of prompts on the bf16 matrix cores, for models without half form (pg_attn_half.hip has the others').
 #include "pg_gemm_dev.h"
 
 namespace pgk {

@@ -1,5 +1,7 @@
 // Products of many rows on the bf16 matrix cores, with f32 inputs, f32 sums and W stored as f32, bf16 or
 // int8 rows (transposed_dense_projection_into, src/models/cpu.rs:58-75; QuantizedRows, cpu.rs:26-56).
+// Stack models' products and those of sampled streams, whose results do not change; the projections of GPT-2 models whose weights
+// have a half form go through pg_gemm_half.hip otherwise.
 //
 // Every f32 operand is cut into three bf16 numbers whose sum is the value: hi = bf16(x), mid =
 // bf16(x - hi), lo = bf16(x - hi - mid), rounded to nearest, every difference exact; lo holds all that is

@@ -1,4 +1,6 @@
-// Products of some tens to some hundreds of rows with activations in cut form (FORM_CUT; pg_cut.h).
+// Products of some tens to some hundreds of rows with activations in cut form (FORM_CUT; pg_cut.h): f32 rows, 33 to 64 of them, from 129
+// on those of models wider than 768 (narrower ones keep W in cut form too, pg_gemm_half.hip), and all of a model's whose weights have
+// no half form (takes_half_form).
 #include "pg_gemm_dev.h"
 
 namespace pgk {
@@ -238,8 +240,8 @@ constexpr RowsPace kRowsPace[3] = {{11.237f, -0.786f, 0.179f, 0.891f, -0.013f, 0
 
 }  // namespace
 
-// The rows up to which a model's four projections take this form, from whole prompts timed both ways (ms, other kernels
-// first).  A step in this form's time is a round of blocks (64 rows by 48 rows of W, 64 for int8 rows) over the CUs, so the
+// The rows up to which a model's four projections take cut form, from whole prompts timed both ways (ms, the tiles of pg_gemm_cut.hip
+// first, these kernels second; where half form is had it goes before both for bf16 and int8 rows, and past these rows for f32 ones).  A step in this form's time is a round of blocks (64 rows by 48 rows of W, 64 for int8 rows) over the CUs, so the
 // line is a number of rounds of the widest product, past which the tiles of pg_gemm_cut.hip, which read an input row once
 // for 128 columns, are the faster ones:
 //  - f32 and bf16 rows, two rounds.  f32 at width 1600: 192 rows 7.52 / 6.58, 193 rows 7.79 / 8.15; 1280: 256 rows 4.83 /
