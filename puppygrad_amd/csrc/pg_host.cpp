@@ -499,7 +499,7 @@ bool takes_cut_form(const pg_model* m, size_t rows) {
 
 // Whether so many rows of activations, of prompts or of a batched step, are kept in half form.
 //  - bf16 and int8 rows: from 17 input rows on.  Prompts of the large model, ms, 20 rows 1.69 / 1.56 (bf16), 1.64 / 1.45 (int8), 64 rows
-//    2.17 / 1.94, 300 rows 4.33 / 3.50; eight steps of 32 sequences, XL 27.2 / 27.2 (bf16), 28.8 / 27.3 (int8), of 40 32.3 / 29.1.
+//    2.17 / 1.94, 300 rows 4.33 / 3.50; eight steps of 32 sequences, XL int8 28.8 / 27.3, of 40 (bf16) 32.3 / 29.1.
 //    Fewer rows are bound by their launches and W's bytes: eight steps of 8, XL bf16, 20.0 / 20.7.
 //  - f32 rows: up to 32 (prompts of 9 rows, XL, 2.54 / 2.47, 32 rows 3.18 / 2.81; the f32 cores' sums are the less precise ones, logits
 //    1.3 to 1.5 times as far off), and past the rows of the cut form (takes_cut_form), whose three parts are the more precise ones there
@@ -787,8 +787,10 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
   // that the 32-row kernel reads with contiguous loads; their producers write them that way.
   // c->cut_form: there is room for them in cut form, which this model's rows take (the cache may have been made for
   // another model of these sizes); not the logits' input.
-  // Half form, which every cache has room for, goes before both (takes_half_form).
-  const bool half = takes_half_form(m, c->B);
+  // Half form, which every cache has room for, goes before both (takes_half_form), but for up to 32 sequences and bf16 rows, whose
+  // packed rows are a little faster (XL, eight steps behind 300 tokens, ms, packed / half form: 17 sequences (100) 20.9 / 21.3, 24 27.9 /
+  // 28.2, 32 30.9 / 31.3; int8 rows, unpacked, of 32 28.8 / 27.3).
+  const bool half = takes_half_form(m, c->B) && !(m->w_bf16 && c->pack32);
   const int pk = c->pack32 && !half ? 1 : 0, cut = !half && c->cut_form && takes_cut_form(m, c->B) ? 1 : 0;
   const int form = half ? pgk::FORM_HALF : cut ? pgk::FORM_CUT : pk ? pgk::FORM_PACKED32 : pgk::FORM_ROWS;
   auto gemm = [&](const float* A, int lda, const float* W, const float* bias, float* Cout,
