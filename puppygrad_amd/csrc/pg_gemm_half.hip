@@ -599,7 +599,7 @@ __global__ __launch_bounds__(256) void k_norm_row_half(GemmArgs a, int parts) {
 constexpr int kNormRowMax = 256;  // rows up to which a block takes one
 template <bool PARTS, int PX>
 hipError_t launch_norm(const GemmArgs& a, int parts, hipStream_t s) {
-  if (a.N % 8 != 0 || a.N > 4096 || a.ldc != a.N) return hipErrorInvalidValue;
+  if (a.N % 8 != 0 || a.N > kNormWidest || a.ldc != a.N) return hipErrorInvalidValue;
   if (a.M <= kNormRowMax) {
     const dim3 rows((unsigned)((a.M + 63) / 64 * 64));
     if (a.N <= 1024) hipLaunchKernelGGL((k_norm_row_half<1, PARTS, PX>), rows, dim3(256), 0, s, a, parts);

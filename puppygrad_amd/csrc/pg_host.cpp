@@ -515,7 +515,7 @@ bool takes_half_form(const pg_model* m, size_t rows) {
 // The block matrices in half form.  Nothing of it is needed to serve a call: where it cannot be had the model goes without.
 pg_status make_half_form(pg_model* m) {
   const Cfg& g = m->cfg;
-  if (g.hd() != pgk::kHeadDim || g.C < 256 || g.C % 32 != 0 || g.C > 4096 || g.I < 256 || g.I % 32 != 0) return PG_OK;
+  if (g.hd() != pgk::kHeadDim || g.C < 256 || g.C % 32 != 0 || g.C > (size_t)pgk::kNormWidest || g.I < 256 || g.I % 32 != 0) return PG_OK;
   const int wb = m->w_i8 ? 1 : m->w_bf16 ? 2 : 4, pw = wb == 4 ? 2 : 1;
   auto up = [](size_t n) { return (n + 255) / 256 * 256; };
   const size_t C = g.C, I = g.I;

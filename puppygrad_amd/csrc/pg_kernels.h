@@ -298,8 +298,9 @@ __host__ __device__ inline size_t packed32_index(size_t b, size_t k) {
 // (store_half4 in pg_half.h; 4 * K * cut_rows(M) bytes).
 enum ActForm : int { FORM_ROWS = 0, FORM_PACKED32 = 1, FORM_CUT = 2, FORM_HALF = 3 };
 inline size_t half_floats(size_t M, size_t K) { return (M + 15) / 16 * 16 * K; }
-// LayerNorm of rows to half form, times scale, or (scale 0) to cut form; cols a multiple of 8 up to 4096.  With parts > 0 a row is
+// LayerNorm of rows to half form, times scale, or (scale 0) to cut form; cols a multiple of 8 up to kNormWidest.  With parts > 0 a row is
 // first put together, resid + (bias + the parts at ws [parts][rows][cols]), and written to src.
+constexpr int kNormWidest = 4096;
 hipError_t launch_norm_rows_half(float* src, void* dst, int rows, int cols, const float* g, const float* b, float eps,
                                  float scale, hipStream_t s, int parts = 0, const float* ws = nullptr, const float* bias = nullptr,
                                  const float* resid = nullptr);

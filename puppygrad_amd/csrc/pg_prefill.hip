@@ -1239,14 +1239,16 @@ __global__ void k_embed_rows(float* x, const float* wte, const float* wpe, const
 }
 
 // dst[r] = LayerNorm(src[r])  (layer_norm_in_place, cpu.rs:119-143), one block per row
-// (dst_packed: dst is a packed activation matrix, see packed32_index)
+// (dst_packed: dst is a packed activation matrix, see packed32_index; CUT: it is in cut form, of rows of any width)
+template <bool CUT>
 __global__ __launch_bounds__(256) void k_layer_norm_rows(const float* src, float* dst, int cols,
                                                          const float* g, const float* b,
                                                          float eps, int dst_form) {
   __shared__ float red[4];
   const float* row = src + (size_t)blockIdx.x * cols;
   auto put = [&](int i, float v) {
-    dst[dst_form == FORM_PACKED32 ? packed32_index(blockIdx.x, (size_t)i) : (size_t)blockIdx.x * cols + i] = v;
+    if constexpr (CUT) store_cut1(dst, cut_rows((int)gridDim.x), blockIdx.x, (size_t)i, v);
+    else dst[dst_form == FORM_PACKED32 ? packed32_index(blockIdx.x, (size_t)i) : (size_t)blockIdx.x * cols + i] = v;
   };
   auto bsum = [&](float v) {
     v = wave_sum(v);
@@ -1820,8 +1822,11 @@ hipError_t launch_embed_rows(float* x, const float* wte, const float* wpe, const
 hipError_t launch_layer_norm_rows(const float* src, float* dst, int rows, int cols, const float* g,
                                   const float* b, float eps, hipStream_t s, int dst_form) {
   if ((dst_form == FORM_PACKED32 && rows > 32) || (dst_form == FORM_CUT && cols % 8 != 0)) return hipErrorInvalidValue;
-  if (dst_form == FORM_CUT) return launch_norm_rows_half(const_cast<float*>(src), dst, rows, cols, g, b, eps, 0.0f, s);
-  hipLaunchKernelGGL(k_layer_norm_rows, dim3(rows), dim3(256), 0, s, src, dst, cols, g, b, eps, dst_form);
+  if (dst_form == FORM_CUT && cols <= kNormWidest) return launch_norm_rows_half(const_cast<float*>(src), dst, rows, cols, g, b, eps, 0.0f, s);
+  if (dst_form == FORM_CUT)
+    hipLaunchKernelGGL(k_layer_norm_rows<true>, dim3(rows), dim3(256), 0, s, src, dst, cols, g, b, eps, dst_form);
+  else
+    hipLaunchKernelGGL(k_layer_norm_rows<false>, dim3(rows), dim3(256), 0, s, src, dst, cols, g, b, eps, dst_form);
   return hipGetLastError();
 }
 

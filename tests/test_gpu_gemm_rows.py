@@ -219,3 +219,29 @@ def test_a_cache_of_another_model_leaves_the_step_to_its_own(maker, user, batch)
         np.testing.assert_array_equal(steps[1], steps[0])
     else:  # (a cache of the model's own is packed: the same kernel, sums of at most 3072 terms in other orders)
         assert np.linalg.norm(steps[1] - steps[0]) <= 1e-5 * np.linalg.norm(steps[0])
+
+
+@pytest.mark.parametrize("storage,rows", [("f32", 40), ("bf16", 64), ("int8", 100)])
+def test_models_wider_than_the_norms_that_keep_a_row_in_registers(storage, rows):
+    """n_embd past 4096 has no half form and takes cut form: a prompt of so many rows, and a step of so many sequences."""
+    cfg = Gpt2Config(vocab_size=97, n_positions=128, n_embd=4160, n_layer=1, n_head=65, n_inner=512)
+    store = {"f32": _lib.PG_STORE_F32, "bf16": _lib.PG_STORE_BF16, "int8": _lib.PG_STORE_INT8}[storage]
+    assert takes(rows, 4160, store, 512)
+    model = Gpt2Model.new(cfg, synth.random_weights(cfg, 0x5EED0A03, perturb=True), Gpt2HipConfig(weight_storage=store))
+    ids = synth.token_ids(rows + 1, 0x70C00A03, cfg.vocab_size)
+    cache = model.new_kv_cache()
+    got = model.prefill([int(t) for t in ids[:rows]], cache).to_host()
+    single = model.new_kv_cache()
+    for at, t in enumerate(ids[:rows]):
+        last = model.prefill([int(t)], single) if at == 0 else model.forward_one(int(t), single)
+    want = last.to_host()
+    # (the same values, sums of at most 4160 terms in other orders)
+    assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
+    batch = model.new_kv_cache(rows)
+    model.prefill_batch(np.ascontiguousarray(ids[:rows, None]), batch)
+    step = model.forward_one_batch(np.full(rows, ids[rows], ids.dtype), batch).to_host()
+    for b in (0, rows - 1):
+        single = model.new_kv_cache()
+        model.prefill([int(ids[b])], single)
+        want = model.forward_one(int(ids[rows]), single).to_host()
+        assert np.linalg.norm(step[b] - want) <= 1e-5 * np.linalg.norm(want)
