@@ -612,7 +612,14 @@ hipError_t launch_norm(const GemmArgs& a, int parts, hipStream_t s) {
   if (a.N <= 768) hipLaunchKernelGGL((k_norm_rows_half<3, PARTS, PX>), grid, dim3(256), lds, s, a, parts);
   else if (a.N <= 1280) hipLaunchKernelGGL((k_norm_rows_half<5, PARTS, PX>), grid, dim3(256), lds, s, a, parts);
   else if (a.N <= 1792) hipLaunchKernelGGL((k_norm_rows_half<7, PARTS, PX>), grid, dim3(256), lds, s, a, parts);
-  else hipLaunchKernelGGL((k_norm_rows_half<16, PARTS, PX>), grid, dim3(256), lds, s, a, parts);
+  else {
+    if (lds > 48 * 1024) {  // (from 2731 columns on in half form, 1891 in cut form)
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_norm_rows_half<16, PARTS, PX>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((k_norm_rows_half<16, PARTS, PX>), grid, dim3(256), lds, s, a, parts);
+  }
   return hipGetLastError();
 }
 template <bool PARTS>

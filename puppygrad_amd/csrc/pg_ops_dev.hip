@@ -479,6 +479,19 @@ pg_status pg_testing_half_product_dev(int32_t device, void* stream, const float*
   return PG_OK;
 }
 
+// LayerNorm of rows as launch_norm_rows_half has it: to half form times scale, or (scale 0) to cut form.
+pg_status pg_testing_norm_half_dev(int32_t device, void* stream, float* x, uint64_t rows, uint64_t cols, const float* g, const float* b,
+                                   float eps, float scale, int32_t parts, const float* ws, const float* bias, const float* resid,
+                                   void* out) {
+  if (!x || !g || !b || !out || (parts > 0 && (!ws || !resid))) return pgh::fail(PG_INVALID_INPUT, "null argument");
+  if (rows == 0 || rows > (1u << 20) || cols < 8 || cols % 8 != 0 || cols > (uint64_t)pgk::kNormWidest || parts < 0 || parts > 8)
+    return pgh::fail(PG_INVALID_INPUT, "norm: sizes");
+  pg_status s;
+  if ((s = select_device(device))) return s;
+  PG_HIP(pgk::launch_norm_rows_half(x, out, (int)rows, (int)cols, g, b, eps, scale, static_cast<hipStream_t>(stream), parts, ws, bias, resid));
+  return PG_OK;
+}
+
 // The same by pg_attn_half.hip: out in half form times sv, or (cut) in cut form; shape 0: as the planner has it.
 pg_status pg_testing_attention_half_dev(int32_t device, void* stream, const float* qkv, uint64_t rows, uint64_t heads,
                                         uint64_t sequences, int32_t shape, float sq, float sk, float sv, int32_t cut, float* keys,

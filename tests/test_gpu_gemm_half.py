@@ -155,6 +155,52 @@ def test_weights_that_half_form_refuses(storage):
             assert (np.abs(product - want) <= bound + 2.0 ** -40 * np.abs(w).max(1) * np.abs(x).sum(1, keepdims=True)).all(), (value, least)
 
 
+def norm_half_dev(x, g, b, scale, parts=None, bias=None):
+    """LayerNorm of x, or of x + bias + parts [p][rows][cols], back from half form (times scale) or cut form (scale 0), and the row itself."""
+    f = _lib.load().pg_testing_norm_half_dev
+    u, v, i, s = C.c_uint64, C.c_void_p, C.c_int32, C.c_float
+    f.argtypes, f.restype = [i, v, v, u, u, v, v, s, s, i, v, v, v, v], C.c_int
+    (m, k), n = x.shape, 0 if parts is None else len(parts)
+    mp, planes = (m + 15) // 16 * 16, 2 if scale else 3
+    held = [DeviceArray(x if n == 0 else np.full_like(x, np.nan)), DeviceArray(g), DeviceArray(b), DeviceArray(np.full(planes * mp * k // 2, np.nan))]
+    held += [DeviceArray(a) for a in (parts, bias, x)] if n else []
+    status = f(0, None, held[0].ptr, m, k, held[1].ptr, held[2].ptr, 1e-5, scale, n, *((d.ptr for d in held[4:]) if n else (None,) * 3), held[3].ptr)
+    row, out = held[0].download(), held[3].download()
+    for d in held:
+        d.free()
+    assert status == 0, _lib.load().pg_last_error_message().decode()
+    if scale:
+        values = out.view(np.float16).reshape(k // 8, 2, mp, 8)[:, :, :m].astype(np.float64) / scale
+    else:
+        values = (out.view(np.uint16).reshape(k // 8, 3, mp, 8)[:, :, :m].astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    return values.sum(1).transpose(1, 0, 2).reshape(m, k), row
+
+
+# a block a row and a wavefront a row, at every number of values a lane holds: the last width of each, an odd octet, the widest
+@pytest.mark.parametrize("cols", [8, 768, 776, 1280, 1792, 1800, 2048, 2560, 2736, 3648, 4096])
+@pytest.mark.parametrize("rows", [1, 67, 300])
+@pytest.mark.parametrize("parts", [0, 3])
+@pytest.mark.parametrize("scale", [256.0, 0.0])
+def test_norms_of_every_width(cols, rows, parts, scale):
+    rng = np.random.default_rng([cols, rows, parts])
+    x, (g, b, bias) = rng.standard_normal((rows, cols)).astype(np.float32) + np.float32(0.5), rng.standard_normal((3, cols)).astype(np.float32)
+    ws = rng.standard_normal((parts, rows, cols)).astype(np.float32) if parts else None
+    got, row = norm_half_dev(x, g, b, scale, ws, bias)
+    want = x if not parts else x.astype(np.float64) + bias + ws.sum(0, dtype=np.float64)
+    # (four roundings of values under 32)
+    np.testing.assert_allclose(row, want, rtol=0, atol=4 * 2.0 ** -20 if parts else 0)
+    r = row.astype(np.float64)
+    d = r - r.mean(1, keepdims=True)
+    inv = 1.0 / np.sqrt((d * d).mean(1, keepdims=True) + 1e-5)
+    # (f32 sums over a lane's values and 64 lanes: of the mean, 72 + cols / 64 roundings of the values' mean size; of the squares as
+    # many of themselves, half of which the root passes on; the cut: half form's 2^-23 and 2^-25 of its unit)
+    n = (72 + cols / 64) * 2.0 ** -24
+    bound = np.abs(g) * inv * n * np.abs(r).mean(1, keepdims=True) + (n + 2.0 ** -23) * np.abs(d * inv * g) + 2.0 ** -23 * np.abs(d * inv * g + b)
+    bound += 2.0 ** -25 / scale if scale else 0.0
+    off = np.abs(got - (d * inv * g + b))
+    assert (off <= bound).all(), f"{(off / bound).max():.2f} of the bound"
+
+
 def logits(model, ids):
     return model.prefill(ids, model.new_kv_cache()).to_host()
 
