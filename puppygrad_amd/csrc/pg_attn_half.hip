@@ -13,20 +13,20 @@ __device__ __forceinline__ float other_half(float x) {
 __device__ __forceinline__ f16v mfma16(const u4v& a, const u4v& b, const f16v& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, a), __builtin_bit_cast(h8v, b), c, 0, 0, 0);
 }
-__device__ __forceinline__ void halves8(f4 a, f4 b, float mul, u4v (&part)[2]) {
+__device__ __forceinline__ void halves8(f4 a, f4 b, u4v (&part)[2]) {
   const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     unsigned h, l;
-    halves2(x[2 * e], x[2 * e + 1], mul, h, l);
+    halves2(x[2 * e], x[2 * e + 1], 1.0f, h, l);
     part[0][e] = h, part[1][e] = l;
   }
 }
 
 // causal_self_attention (src/models/gpt2/rust.rs:1580-1659) for head_dim 64 over qkv[T][3C], as k_attn_prefill_cut
 // (pg_attn_cut.hip) with two f16 numbers a value for three bf16 numbers: three products of the parts for six, half of the
-// cutting.  Q, K and V are scaled by powers of two, sq, sk and sv, with which none can be past 2^15 (half_bounds); the weights,
-// whose largest is 1, by 2^7.  FORM: out is in half form times sv, or in cut form, as the projection behind it wants it.  Scores, maxima, weights
+// cutting.  Every dim of Q, K and V of a head is kept times a power of two (HalfScales) with which none of its values can be past
+// 2^15; the weights, whose largest is 1, times 2^7.  FORM: out is in half form times V's, or in cut form, as the projection behind it wants it.  Scores, maxima, weights
 // and sums are f32.  A tile's products are chains of their own that are added to the output: over 1000 keys one chain of f32
 // roundings is off by more than all else in here.
 // A block holds QG x 32 queries: the QG wavefronts of a key group share a tile of 32 keys that they have cut once, in operand
@@ -42,7 +42,7 @@ template <int QG, int KG, int FORM>
 __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const float* __restrict__ qkv, int T, int C, int P,
                                                                       float* __restrict__ kcache,
                                                                       float* __restrict__ vcache,
-                                                                      void* __restrict__ out, size_t kv_stride, float sq, float sk, float sv) {
+                                                                      void* __restrict__ out, size_t kv_stride, HalfScales scales) {
   constexpr int NW = QG * KG;
   constexpr int KSTR = 32 * 16 + 16;            // bytes of an octet of dims of 32 keys, padded
   constexpr int KPART = 8 * KSTR, VPART = 4 * 64 * 16;
@@ -51,6 +51,7 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const flo
   constexpr int LDS = KG * TILE > NW * MERGE ? KG * TILE : NW * MERGE;
   __shared__ __attribute__((aligned(16))) char lds[LDS];
   __shared__ float Ms[NW][32], Ls[NW][32];
+  __shared__ __attribute__((aligned(16))) float Ks[2][64];  // K's and V's powers: read for every tile, there are no registers for them
   qkv += (size_t)blockIdx.z * T * 3 * C;
   kcache += (size_t)blockIdx.z * kv_stride;
   vcache += (size_t)blockIdx.z * kv_stride;
@@ -66,7 +67,8 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const flo
   const float* qbase = qkv + h * 64;
   const float* kbase = qkv + C + h * 64;
   const float* vbase = qkv + 2 * C + h * 64;
-  const float kC = 0.125f * 1.44269504088896341f / (sq * sk);  // (powers of two)
+  const float* sq = scales.q + h * 64;
+  const float kC = 0.125f * 1.44269504088896341f / scales.score[h];  // (a power of two)
   constexpr float kLag = 8.0f;  // a weight is at most 2^15, half form's most
   char* kt = lds + kg * TILE;
   char* vt = kt + 2 * KPART;
@@ -77,9 +79,11 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const flo
     const float* q = qbase + (size_t)min(qi, T - 1) * C3 + 8 * half;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      halves8(*reinterpret_cast<const f4*>(q + 16 * s), *reinterpret_cast<const f4*>(q + 16 * s + 4), sq, qp[s]);
+      const f4* p = reinterpret_cast<const f4*>(sq + 8 * half + 16 * s);
+      halves8(*reinterpret_cast<const f4*>(q + 16 * s) * p[0], *reinterpret_cast<const f4*>(q + 16 * s + 4) * p[1], qp[s]);
     }
   }
+  Ks[0][lane] = scales.k[h * 64 + lane], Ks[1][lane] = scales.v[h * 64 + lane];  // (every wavefront the same)
   f16v o0, o1;  // O^T rows 0..31 and 32..63
 #pragma unroll
   for (int v = 0; v < 16; ++v) o0[v] = o1[v] = 0.0f;
@@ -120,11 +124,14 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const flo
     meet();  // the last tile has been read
     if (tile <= last) {
       const bool append = tile >= qb * QG;  // the block's own positions go to the cache
+      asm volatile("" ::: "memory");        // (Ks is read here)
+      const f4 sk0 = *reinterpret_cast<const f4*>(Ks[0] + 8 * (lane & 7)), sk1 = *reinterpret_cast<const f4*>(Ks[0] + 8 * (lane & 7) + 4);
+      const float sv = Ks[1][lane];
 #pragma unroll
       for (int i = 0; i < KI; ++i) {
         const int id = lane + 64 * (qg * KI + i), key = id >> 3, o = id & 7;
         u4v c[2];
-        halves8(kr[i][0], kr[i][1], sk, c);
+        halves8(kr[i][0] * sk0, kr[i][1] * sk1, c);
 #pragma unroll
         for (int p = 0; p < 2; ++p) *reinterpret_cast<u4v*>(kt + p * KPART + o * KSTR + key * 16) = c[p];
         if (append && tile * 32 + key < T) {
@@ -137,7 +144,7 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const flo
       for (int i = 0; i < VI; ++i) {
         const int u = qg * VI + i;
         u4v c[2];
-        halves8(f4{vr[i][0], vr[i][1], vr[i][2], vr[i][3]}, f4{vr[i][4], vr[i][5], vr[i][6], vr[i][7]}, sv, c);
+        halves8(f4{vr[i][0], vr[i][1], vr[i][2], vr[i][3]} * sv, f4{vr[i][4], vr[i][5], vr[i][6], vr[i][7]} * sv, c);
 #pragma unroll
         for (int p = 0; p < 2; ++p) *reinterpret_cast<u4v*>(vt + p * VPART + (u * 64 + lane) * 16) = c[p];
         if (append) {
@@ -202,7 +209,7 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const flo
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       u4v pp[2], va[2], vb[2];
-      halves8(f4{sb[8 * s], sb[8 * s + 1], sb[8 * s + 2], sb[8 * s + 3]}, f4{sb[8 * s + 4], sb[8 * s + 5], sb[8 * s + 6], sb[8 * s + 7]}, 1.0f, pp);
+      halves8(f4{sb[8 * s], sb[8 * s + 1], sb[8 * s + 2], sb[8 * s + 3]}, f4{sb[8 * s + 4], sb[8 * s + 5], sb[8 * s + 6], sb[8 * s + 7]}, pp);
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
         const char* at = vt + p * VPART + ((2 * s + half) * 64 + l32) * 16;
@@ -260,9 +267,9 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const flo
       r[e] = sum * inv;
       rest[e] = fmaf(sum, inv, -r[e]) + r[e] * inv_rest;  // (what f32 rounds away: half form keeps some of it)
     }
-    // (times sv, as the values were)
-    if constexpr (FORM == FORM_HALF) store_half4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r, rest, 1.0f);
-    else store_cut4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r * (1.0f / sv));
+    // (times V's powers, as the values were)
+    if constexpr (FORM == FORM_HALF) store_half4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r, rest, f4{1.f, 1.f, 1.f, 1.f});
+    else store_cut4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r / *reinterpret_cast<const f4*>(scales.v + h * 64 + d));
   }
 }
 
@@ -271,9 +278,9 @@ hipError_t start(const float* qkv, int T, int C, int H, int P, float* kcache, fl
                  size_t kv_stride, const HalfScales& f, int out_form) {
   const dim3 grid(H, (T + 32 * QG - 1) / (32 * QG), nseq), block(64 * QG * KG);
   if (out_form == FORM_HALF)
-    hipLaunchKernelGGL((k_attn_prefill_half<QG, KG, FORM_HALF>), grid, block, 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, f.q, f.k, f.v);
+    hipLaunchKernelGGL((k_attn_prefill_half<QG, KG, FORM_HALF>), grid, block, 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, f);
   else
-    hipLaunchKernelGGL((k_attn_prefill_half<QG, KG, FORM_CUT>), grid, block, 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, f.q, f.k, f.v);
+    hipLaunchKernelGGL((k_attn_prefill_half<QG, KG, FORM_CUT>), grid, block, 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, f);
   return hipGetLastError();
 }
 }  // namespace

@@ -16,9 +16,11 @@
 // 64 a wavefront: 1.4, 2.1); bf16 rows 2.1 -> 1.1, 4.5 -> 1.5; 128 x 256 tiles, one chain, 16384 x 1600 x 1600 4.3 -> 3.6.
 // Logits of prompts of 450 to 1000 tokens, all sizes: 0.65 to 0.85 of what they were off by.
 //
-// The range of f16: values are scaled so that they cannot be past 2^15 whatever the inputs are (half_bounds: what a
-// LayerNorm, a projection of one, an average of such or a GELU of such can reach at most), and below 2^-2 a value is right
-// to 2^-25, 2^-40 of that bound.  f16 subnormals count in these instructions.
+// The range of f16: every column of the inputs has a power of two of its own, with which none of its values can be past 2^15
+// whatever the model is given (k_half_bound: what a LayerNorm, a projection of one, an average of such or a GELU of such can
+// reach at most), and W's half form has its inverse in that column.  Below 2^-2 a value is right to 2^-25, 2^-40 of its own column's
+// bound, and so is a weight with its column's power to 2^-40 of the largest in its row: of a product that counts, whatever the
+// sizes of the gains and of the columns of W are to each other.  f16 subnormals count in these instructions.
 //
 // How operands travel: a producer cuts a value once, in its epilogue; here all are operands as they lie, whole KB by
 // global_load_lds without registers, LDS reads free of conflicts without a permutation, no vector instruction in the loop
@@ -70,7 +72,7 @@ struct Products {
 
 // GELU of sum + bias, four columns of a row, in half form with what f32 rounds away on the way, or in cut form.
 template <int PX>
-__device__ __forceinline__ void store_gelu(void* to, int mp, size_t m, size_t n, f4 sum, f4 bias, float scale) {
+__device__ __forceinline__ void store_gelu(void* to, int mp, size_t m, size_t n, f4 sum, f4 bias, f4 scale) {
   const f4 c = bias + sum, b = c - sum, c_rest = (bias - b) + (sum - (c - b));
   f4 y, rest;
 #pragma unroll
@@ -272,6 +274,8 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
       if constexpr (PX == 2) mul = *reinterpret_cast<const f4*>(a.w_half_mul + n) * a.a_unscale;
       f4 bias = f4{0.f, 0.f, 0.f, 0.f};
       if (!SPLIT && a.bias) bias = *reinterpret_cast<const f4*>(a.bias + n);
+      f4 scale = f4{1.f, 1.f, 1.f, 1.f};
+      if constexpr (EPI == GEMM_GELU && PX == 2) scale = *reinterpret_cast<const f4*>(a.c_scale + n);
 #pragma unroll
       for (int i = 0; i < MB; ++i) {
         const int m = m0 + (wm * MB + i) * 32 + l32;
@@ -285,7 +289,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
           continue;
         }
         if constexpr (EPI == GEMM_GELU) {
-          store_gelu<PX>(a.C, mp, (size_t)m, (size_t)n, c, bias, a.c_scale);
+          store_gelu<PX>(a.C, mp, (size_t)m, (size_t)n, c, bias, scale);
           continue;
         }
         c += bias;
@@ -343,6 +347,7 @@ __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
     if (parts > 1) continue;
     if (live && a.bias) ebias[q] = *reinterpret_cast<const f4*>(a.bias + n);
     if (live && EPI == GEMM_RESID) eres[q] = *reinterpret_cast<const f4*>(a.resid + (size_t)m * a.ldc + n);
+    if (live && EPI == GEMM_GELU && PX == 2) eres[q] = *reinterpret_cast<const f4*>(a.c_scale + n);
   }
 
   f4 tot[MT][NG];
@@ -429,7 +434,7 @@ __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
       continue;
     }
     if (EPI == GEMM_GELU) {
-      store_gelu<PX>(a.C, mp, (size_t)m, (size_t)n, sum, ebias[q], a.c_scale);
+      store_gelu<PX>(a.C, mp, (size_t)m, (size_t)n, sum, ebias[q], eres[q]);
       continue;
     }
     f4 c = ebias[q] + sum;
@@ -629,13 +634,14 @@ hipError_t launch_norm_rows(const GemmArgs& a, int parts, hipStream_t s) {
 
 // ---- weights -----------------------------------------------------------------------------------
 // Rows of W as stored (WT as elsewhere: f32, bf16, int8 with their scales) to half form: part p of element (n, k) is the
-// (k % 8)-th f16 of the 16 bytes at ((k / 8 * PW + p) * N + n) * 16, times mul[n]^-1; a f32 or bf16 row is scaled by the power of
-// two that puts its largest value between 2^14 and 2^15.  A bf16 weight is then a f16 number as it is down to 2^-32 of the row's
-// largest and right to 2^-40 of that below, as a f32 weight's lo part is (of normally distributed weights one in 10^9 is as small:
-// a large model has some).  *refused is set where a value is not finite or a row so small or large that its power of two would matter.
+// (k % 8)-th f16 of the 16 bytes at ((k / 8 * PW + p) * N + n) * 16, times mul[n]^-1: divided by the power of two that column k of the
+// inputs is kept times (powers; null: 1), and its row scaled by the one that puts the largest between 2^14 and 2^15.  A bf16 weight is
+// then a f16 number as it is down to 2^-32 of the row's largest and right to 2^-40 of that below, as a f32 weight's lo part is (of
+// normally distributed weights one in 10^9 is as small: a large model has some).  *refused is set where a value is not finite or a row
+// so small or large that its power of two, or an int8 row's scale beside it, would matter.
 template <int WT>
-__global__ __launch_bounds__(256) void k_half_rows(const void* W, const float* scales, void* to, float* mul, unsigned* refused,
-                                                   int N, int K) {
+__global__ __launch_bounds__(256) void k_half_rows(const void* W, const float* scales, const float* powers, void* to, float* mul,
+                                                   unsigned* refused, int N, int K) {
   constexpr int PW = WT == 0 ? 2 : 1;
   __shared__ float biggest[4][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -655,30 +661,34 @@ __global__ __launch_bounds__(256) void k_half_rows(const void* W, const float* s
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] = (float)((int)(w[e / 4] << (24 - 8 * (e % 4))) >> 24);
     }
-  };
-  float x[8], scale = 1.0f;
-  bool bad = false;
-  if constexpr (WT != 2) {
-    float most = 0.0f;
-    for (int k = 8 * wave; k < K; k += 32) {
-      get(k, x);
+    if (powers)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        bad |= !(fabsf(x[e]) < INFINITY);
-        most = fmaxf(most, fabsf(x[e]));
-      }
+      for (int e = 0; e < 8; ++e) x[e] *= 1.0f / powers[k + e];
+  };
+  float x[8], most = 0.0f, row_scale = 1.0f;
+  bool bad = false;
+  for (int k = 8 * wave; k < K; k += 32) {
+    get(k, x);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      bad |= !(fabsf(x[e]) < INFINITY);
+      most = fmaxf(most, fabsf(x[e]));
     }
-    biggest[wave][lane] = most;
-    __syncthreads();
-    most = fmaxf(fmaxf(biggest[0][lane], biggest[1][lane]), fmaxf(biggest[2][lane], biggest[3][lane]));
-    int e = 15;
-    if (most > 0.0f && most < INFINITY) frexpf(most, &e);
-    bad |= most > 0.0f && abs(15 - e) > kHalfMostExp;
-    scale = bad ? 1.0f : ldexpf(1.0f, 15 - e);
-  } else {
-    bad = !(fabsf(scales[row]) < INFINITY);
   }
-  if (wave == 0 && n < N) mul[n] = WT == 2 ? scales[row] : 1.0f / scale;
+  biggest[wave][lane] = most;
+  __syncthreads();
+  most = fmaxf(fmaxf(biggest[0][lane], biggest[1][lane]), fmaxf(biggest[2][lane], biggest[3][lane]));
+  int top = 15;
+  if (most > 0.0f && most < INFINITY) frexpf(most, &top);
+  if constexpr (WT == 2) {
+    row_scale = scales[row];
+    int e = 0;
+    if (most > 0.0f && row_scale != 0.0f) frexpf(row_scale, &e);
+    bad |= !(fabsf(row_scale) < INFINITY) || abs(e) > kHalfMostExp;
+  }
+  bad |= most > 0.0f && abs(15 - top) > kHalfMostExp;
+  const float scale = bad ? 1.0f : ldexpf(1.0f, 15 - top);
+  if (wave == 0 && n < N) mul[n] = row_scale / scale;
   for (int k = 8 * wave; k < K; k += 32) {
     get(k, x);
     u4v h, l;
@@ -712,10 +722,10 @@ __global__ __launch_bounds__(256) void k_cut_weights(const float* W, void* to, i
 
 // The largest that an output of a projection behind a LayerNorm can be: the norm's values before scale and shift are at most
 // sqrt(C) long together, so |W_o . (g z + b) + bias_o| <= sqrt(C) |W_o g| + |W_o . b + bias_o|, the second as fold has it
-// (launch_ln_fold).  The maximum over the rows goes to *most, bits of a float that is not negative.
+// (launch_ln_fold).
 template <int WT>
 __global__ __launch_bounds__(256) void k_half_bound(const void* W, const float* scales, const float* g, const float* fold,
-                                                    unsigned* most, int N, int K) {
+                                                    float* bounds, int N, int K) {
   const int lane = threadIdx.x & 63, row = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= N) return;
   float ss = 0.0f;
@@ -727,17 +737,52 @@ __global__ __launch_bounds__(256) void k_half_bound(const void* W, const float* 
     ss = fmaf(w * g[k], w * g[k], ss);
   }
   ss = wave_sum(ss);
-  if (lane == 0) {
-    const float b = sqrtf(ss * (float)K) + fabsf(fold[2 * row + 1]);
-    atomicMax(most, b < INFINITY ? __float_as_uint(b) : 0x7f800000u);  // (NaN too)
-  }
+  if (lane == 0) bounds[row] = sqrtf(ss * (float)K) + fabsf(fold[2 * row + 1]);
 }
-// The same of the norm's own values: sqrt(C) |g_c| + |b_c|.
-__global__ __launch_bounds__(256) void k_half_bound_norm(const float* g, const float* b, unsigned* most, int C) {
+// The exponent of the power of two that puts values up to `bound` at 2^15 at most; refused where it is out of bounds itself.
+__device__ __forceinline__ int half_power(float bound, bool& refused) {
+  int e = 15;  // (a bound of 0: a column of zeros)
+  if (bound > 0.0f && bound < INFINITY) frexpf(bound, &e);
+  refused |= !(bound < INFINITY) || abs(15 - e) > kHalfMostExp;  // (NaN too)
+  return 15 - e;
+}
+__global__ __launch_bounds__(256) void k_half_powers(float* at, unsigned* refused, int n) {
+  const int i = (int)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  bool bad = false;
+  at[i] = ldexpf(1.0f, half_power(at[i], bad));
+  if (bad) atomicOr(refused, 1u);
+}
+// The norm's own values, sqrt(C) |g_c| + |b_c| at most: their powers, and gains and shifts times them.
+__global__ __launch_bounds__(256) void k_half_norm_powers(const float* g, const float* b, float* powers, float* g_out, float* b_out,
+                                                          unsigned* refused, int C) {
   const int i = (int)blockIdx.x * 256 + threadIdx.x;
   if (i >= C) return;
-  const float v = fabsf(g[i]) * sqrtf((float)C) + fabsf(b[i]);
-  atomicMax(most, v < INFINITY ? __float_as_uint(v) : 0x7f800000u);
+  bool bad = false;
+  const float p = ldexpf(1.0f, half_power(fabsf(g[i]) * sqrtf((float)C) + fabsf(b[i]), bad));
+  powers[i] = p, g_out[i] = g[i] * p, b_out[i] = b[i] * p;
+  if (bad) atomicOr(refused, 1u);
+}
+// Queries and keys, whose products over a head's 64 dims are added: the product of their powers is the same for all of a head's dims,
+// score[h].  Queries take the whole range, keys of dim d as much of it as the largest product of d is of the head's largest.  A
+// wavefront a head; q and k hold the bounds and get the powers.
+__global__ __launch_bounds__(64) void k_half_score_powers(float* q, float* k, float* score, unsigned* refused) {
+  const int h = (int)blockIdx.x, i = h * 64 + (int)threadIdx.x;
+  const float bq = q[i], bk = k[i];
+  bool bad = false;
+  const int pq = half_power(bq, bad), pk = half_power(bk, bad);
+  const bool counts = bq > 0.0f && bk > 0.0f;  // (otherwise the product is 0 whatever the powers are)
+  __shared__ int least[64];
+  least[threadIdx.x] = counts ? pq + pk : 1 << 20;
+  __syncthreads();
+  int both = 1 << 20;
+  for (int j = 0; j < 64; ++j) both = min(both, least[j]);
+  if (both == 1 << 20) both = 0;
+  const int pk_of = counts ? both - pq : pk;
+  bad |= abs(pk_of) > 2 * kHalfMostExp;
+  q[i] = ldexpf(1.0f, pq), k[i] = ldexpf(1.0f, bad ? 0 : pk_of);
+  if (threadIdx.x == 0) score[h] = ldexpf(1.0f, both);
+  if (bad) atomicOr(refused, 1u);
 }
 
 // ---- launchers ---------------------------------------------------------------------------------
@@ -851,7 +896,7 @@ bool gemm_half_takes(const GemmArgs& a, int epi) {
                        reinterpret_cast<uintptr_t>(a.ln_g) | reinterpret_cast<uintptr_t>(a.ln_b);
   return a.w_half && (a.w_half_parts == 3 || (a.w_half_mul && (a.w_half_parts == 1 || a.w_half_parts == 2))) && !(at & 15) && a.M >= 1 && a.M < (1 << 23) &&
          a.K >= 64 && a.K % 32 == 0 && a.N >= 64 && a.N % 8 == 0 && a.N < (1 << 24) && a.ldc % 4 == 0 && a.a_unscale > 0.0f &&
-         (epi == GEMM_GELU) == (a.c_scale > 0.0f) &&
+         (a.c_scale != nullptr) == (epi == GEMM_GELU && a.w_half_parts != 3) && !(reinterpret_cast<uintptr_t>(a.c_scale) & 15) &&
          (epi == GEMM_BIAS || epi == GEMM_GELU || epi == GEMM_RESID) && (epi != GEMM_GELU || a.ldc == a.N);
 }
 
@@ -937,13 +982,13 @@ hipError_t launch_norm_rows_half(float* src, void* dst, int rows, int cols, cons
   return launch_norm_rows<true>(a, parts, s);
 }
 
-hipError_t launch_half_rows(const void* W, int w_bytes, const float* scales, size_t rows, int cols, void* to, float* mul,
-                            unsigned* refused, hipStream_t s) {
+hipError_t launch_half_rows(const void* W, int w_bytes, const float* scales, const float* powers, size_t rows, int cols, void* to,
+                            float* mul, unsigned* refused, hipStream_t s) {
   const dim3 grid((unsigned)((rows + 63) / 64));
   if (cols % 32 != 0 || rows > (1u << 24)) return hipErrorInvalidValue;
-  if (w_bytes == 4) hipLaunchKernelGGL(k_half_rows<0>, grid, dim3(256), 0, s, W, scales, to, mul, refused, (int)rows, cols);
-  else if (w_bytes == 2) hipLaunchKernelGGL(k_half_rows<1>, grid, dim3(256), 0, s, W, scales, to, mul, refused, (int)rows, cols);
-  else hipLaunchKernelGGL(k_half_rows<2>, grid, dim3(256), 0, s, W, scales, to, mul, refused, (int)rows, cols);
+  if (w_bytes == 4) hipLaunchKernelGGL(k_half_rows<0>, grid, dim3(256), 0, s, W, scales, powers, to, mul, refused, (int)rows, cols);
+  else if (w_bytes == 2) hipLaunchKernelGGL(k_half_rows<1>, grid, dim3(256), 0, s, W, scales, powers, to, mul, refused, (int)rows, cols);
+  else hipLaunchKernelGGL(k_half_rows<2>, grid, dim3(256), 0, s, W, scales, powers, to, mul, refused, (int)rows, cols);
   return hipGetLastError();
 }
 hipError_t launch_cut_weights(const float* W, size_t rows, int cols, void* to, hipStream_t s) {
@@ -952,15 +997,24 @@ hipError_t launch_cut_weights(const float* W, size_t rows, int cols, void* to, h
   return hipGetLastError();
 }
 hipError_t launch_half_bound(const void* W, int w_bytes, const float* scales, const float* g, const float* fold, size_t rows, int cols,
-                             unsigned* most, hipStream_t s) {
+                             float* bounds, hipStream_t s) {
   const dim3 grid((unsigned)((rows + 3) / 4));
-  if (w_bytes == 4) hipLaunchKernelGGL(k_half_bound<0>, grid, dim3(256), 0, s, W, scales, g, fold, most, (int)rows, cols);
-  else if (w_bytes == 2) hipLaunchKernelGGL(k_half_bound<1>, grid, dim3(256), 0, s, W, scales, g, fold, most, (int)rows, cols);
-  else hipLaunchKernelGGL(k_half_bound<2>, grid, dim3(256), 0, s, W, scales, g, fold, most, (int)rows, cols);
+  if (w_bytes == 4) hipLaunchKernelGGL(k_half_bound<0>, grid, dim3(256), 0, s, W, scales, g, fold, bounds, (int)rows, cols);
+  else if (w_bytes == 2) hipLaunchKernelGGL(k_half_bound<1>, grid, dim3(256), 0, s, W, scales, g, fold, bounds, (int)rows, cols);
+  else hipLaunchKernelGGL(k_half_bound<2>, grid, dim3(256), 0, s, W, scales, g, fold, bounds, (int)rows, cols);
   return hipGetLastError();
 }
-hipError_t launch_half_bound_norm(const float* g, const float* b, int cols, unsigned* most, hipStream_t s) {
-  hipLaunchKernelGGL(k_half_bound_norm, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, s, g, b, most, cols);
+hipError_t launch_half_norm_powers(const float* g, const float* b, int cols, float* powers, float* g_out, float* b_out, unsigned* refused,
+                                   hipStream_t s) {
+  hipLaunchKernelGGL(k_half_norm_powers, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, s, g, b, powers, g_out, b_out, refused, cols);
+  return hipGetLastError();
+}
+hipError_t launch_half_powers(float* at, int n, unsigned* refused, hipStream_t s) {
+  hipLaunchKernelGGL(k_half_powers, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, at, refused, n);
+  return hipGetLastError();
+}
+hipError_t launch_half_score_powers(float* q, float* k, int heads, float* score, unsigned* refused, hipStream_t s) {
+  hipLaunchKernelGGL(k_half_score_powers, dim3((unsigned)heads), dim3(64), 0, s, q, k, score, refused);
   return hipGetLastError();
 }
 

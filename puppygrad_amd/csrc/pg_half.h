@@ -25,7 +25,7 @@ __device__ __forceinline__ void halves2(double a, double b, unsigned& hi, unsign
   const h2v l = __builtin_convertvector(f2{(float)(a - (double)(float)h.x), (float)(b - (double)(float)h.y)}, h2v);
   hi = __builtin_bit_cast(unsigned, h), lo = __builtin_bit_cast(unsigned, l);
 }
-// An activation matrix in half form: as in cut form (pg_cut.h) with two parts for three and a power of two in front:
+// An activation matrix in half form: as in cut form (pg_cut.h) with two parts for three and a power of two in front of every column:
 // part p of element (m, k) is the (k % 8)-th f16 of the 16 bytes at ((k / 8 * 2 + p) * cut_rows(M) + m) * 16.
 // Columns k .. k + 3 (k a multiple of 4) of row m of a matrix with room for mp rows.
 __device__ __forceinline__ void store_half4(void* to, int mp, size_t m, size_t k, f4 v, float mul) {
@@ -36,14 +36,14 @@ __device__ __forceinline__ void store_half4(void* to, int mp, size_t m, size_t k
   *reinterpret_cast<u2v*>(at) = u2v{h0, h1};
   *reinterpret_cast<u2v*>(at + (size_t)mp * 16) = u2v{l0, l1};
 }
-// The same of values with what f32 rounded away.
-__device__ __forceinline__ void store_half4(void* to, int mp, size_t m, size_t k, f4 v, f4 rest, float mul) {
+// The same of values with what f32 rounded away, times a power of two a column.
+__device__ __forceinline__ void store_half4(void* to, int mp, size_t m, size_t k, f4 v, f4 rest, f4 mul) {
   unsigned h[2], l[2];
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
-    const float a = v[2 * e] * mul, b = v[2 * e + 1] * mul;
+    const float a = v[2 * e] * mul[2 * e], b = v[2 * e + 1] * mul[2 * e + 1];
     const h2v hi = __builtin_convertvector(f2{a, b}, h2v);
-    const h2v lo = __builtin_convertvector(f2{fmaf(rest[2 * e], mul, a - (float)hi.x), fmaf(rest[2 * e + 1], mul, b - (float)hi.y)}, h2v);
+    const h2v lo = __builtin_convertvector(f2{fmaf(rest[2 * e], mul[2 * e], a - (float)hi.x), fmaf(rest[2 * e + 1], mul[2 * e + 1], b - (float)hi.y)}, h2v);
     h[e] = __builtin_bit_cast(unsigned, hi), l[e] = __builtin_bit_cast(unsigned, lo);
   }
   char* at = static_cast<char*>(to) + (k >> 3) * 2 * mp * 16 + m * 16 + (k & 4) * 2;

@@ -527,20 +527,36 @@ pg_status make_half_form(pg_model* m) {
   // 63.9 / 66.0, 320 rows 90.1 / 91.0, and 1280, 192 rows 81.9 / 85.6: there W's bytes are what counts.
   const bool cut = wb == 4 && C <= 768;
   for (int i = 0; i < 4; ++i) layer += up(rows[i] * cols[i] * 2 * pw) + up(rows[i] * 4) + (cut ? up(rows[i] * cols[i] * 6) : 0);
-  constexpr int kBounds = 6;  // of a layer: both norms, hidden, queries, keys, values
-  const size_t words = up((g.L * kBounds + 1) * 4);
-  if (hipMalloc(&m->half_arena, g.L * layer + words) != hipSuccess) {
+  layer += 9 * up(C * 4) + up(I * 4) + up(g.H * 4);  // the columns' powers; gains and shifts times them
+  if (hipMalloc(&m->half_arena, g.L * layer + up(4)) != hipSuccess) {
     (void)hipGetLastError();
     m->half_arena = nullptr;
     return PG_OK;
   }
-  unsigned* bounds = reinterpret_cast<unsigned*>(m->half_arena);
-  unsigned* refused = bounds + g.L * kBounds;
-  PG_HIP(pgk::launch_fill_zero(reinterpret_cast<float*>(bounds), g.L * kBounds + 1, nullptr));
+  unsigned* refused = reinterpret_cast<unsigned*>(m->half_arena);
+  PG_HIP(pgk::launch_fill_zero(reinterpret_cast<float*>(refused), 1, nullptr));
   m->half.resize(g.L);
-  char* at = m->half_arena + words;
+  char* at = m->half_arena + up(4);
+  auto floats = [&](size_t n) {
+    float* p = reinterpret_cast<float*>(at);
+    at += up(n * 4);
+    return p;
+  };
   for (size_t l = 0; l < g.L; ++l) {
     const pgk::LayerW& w = m->layers[l];
+    // the inputs of the four matrices, column by column
+    float *norm_1 = floats(C), *norm_1_g = floats(C), *norm_1_b = floats(C), *norm_2 = floats(C), *norm_2_g = floats(C), *norm_2_b = floats(C);
+    float *qkv[3] = {floats(C), floats(C), floats(C)}, *hidden = floats(I), *score = floats(g.H);
+    PG_HIP(pgk::launch_half_norm_powers(w.ln_1_g, w.ln_1_b, (int)C, norm_1, norm_1_g, norm_1_b, refused, nullptr));
+    PG_HIP(pgk::launch_half_norm_powers(w.ln_2_g, w.ln_2_b, (int)C, norm_2, norm_2_g, norm_2_b, refused, nullptr));
+    PG_HIP(pgk::launch_half_bound(w.c_fc_w, wb, w.c_fc_s, w.ln_2_g, w.c_fc_f, I, (int)C, hidden, nullptr));  // (|gelu(x)| <= |x|)
+    PG_HIP(pgk::launch_half_powers(hidden, (int)I, refused, nullptr));
+    for (size_t part = 0; part < 3; ++part)  // (an average of values is no larger than they are)
+      PG_HIP(pgk::launch_half_bound(reinterpret_cast<const char*>(w.c_attn_w) + part * C * C * wb, wb, w.c_attn_s ? w.c_attn_s + part * C : nullptr,
+                                    w.ln_1_g, w.c_attn_f + 2 * part * C, C, (int)C, qkv[part], nullptr));
+    PG_HIP(pgk::launch_half_score_powers(qkv[0], qkv[1], (int)g.H, score, refused, nullptr));
+    PG_HIP(pgk::launch_half_powers(qkv[2], (int)C, refused, nullptr));
+    const float* powers[4] = {norm_1, qkv[2], norm_2, hidden};
     const float* mats[4] = {w.c_attn_w, w.c_proj_w, w.c_fc_w, w.c_proj_mlp_w};
     const float* scales[4] = {w.c_attn_s, w.c_proj_s, w.c_fc_s, w.c_proj_mlp_s};
     void *to[4], *cut_to[4] = {};
@@ -548,42 +564,19 @@ pg_status make_half_form(pg_model* m) {
     for (int i = 0; i < 4; ++i) {
       to[i] = at;
       at += up(rows[i] * cols[i] * 2 * pw);
-      mul[i] = reinterpret_cast<float*>(at);
-      at += up(rows[i] * 4);
-      PG_HIP(pgk::launch_half_rows(mats[i], wb, scales[i], rows[i], (int)cols[i], to[i], mul[i], refused, nullptr));
+      mul[i] = floats(rows[i]);
+      PG_HIP(pgk::launch_half_rows(mats[i], wb, scales[i], powers[i], rows[i], (int)cols[i], to[i], mul[i], refused, nullptr));
       if (!cut) continue;
       cut_to[i] = at;
       at += up(rows[i] * cols[i] * 6);
       PG_HIP(pgk::launch_cut_weights(mats[i], rows[i], (int)cols[i], cut_to[i], nullptr));
     }
-    m->half[l] = pg_model::HalfLayer{to[0], to[1], to[2], to[3], mul[0], mul[1], mul[2], mul[3], 0, 0, 0, {}, cut_to[0], cut_to[1], cut_to[2], cut_to[3]};
-    unsigned* b = bounds + l * kBounds;
-    PG_HIP(pgk::launch_half_bound_norm(w.ln_1_g, w.ln_1_b, (int)C, b, nullptr));
-    PG_HIP(pgk::launch_half_bound_norm(w.ln_2_g, w.ln_2_b, (int)C, b + 1, nullptr));
-    PG_HIP(pgk::launch_half_bound(w.c_fc_w, wb, w.c_fc_s, w.ln_2_g, w.c_fc_f, I, (int)C, b + 2, nullptr));  // (|gelu(x)| <= |x|)
-    for (size_t part = 0; part < 3; ++part)  // (an average of values is no larger than they are)
-      PG_HIP(pgk::launch_half_bound(reinterpret_cast<const char*>(w.c_attn_w) + part * C * C * wb, wb, w.c_attn_s ? w.c_attn_s + part * C : nullptr,
-                                    w.ln_1_g, w.c_attn_f + 2 * part * C, C, (int)C, b + 3 + part, nullptr));
+    m->half[l] = pg_model::HalfLayer{to[0], to[1], to[2], to[3], mul[0], mul[1], mul[2], mul[3], norm_1_g, norm_1_b, norm_2_g, norm_2_b, hidden,
+                                     {qkv[0], qkv[1], qkv[2], score}, cut_to[0], cut_to[1], cut_to[2], cut_to[3]};
   }
-  std::vector<unsigned> got(g.L * kBounds + 1);
-  PG_HIP(hipMemcpy(got.data(), bounds, got.size() * 4, hipMemcpyDeviceToHost));
-  bool ok = got.back() == 0;
-  auto scale = [&](unsigned bits) {
-    float bound;
-    memcpy(&bound, &bits, 4);
-    int e = 0;
-    if (!std::isfinite(bound)) ok = false;
-    else if (bound > 0.0f) frexpf(bound, &e);
-    if (std::abs(15 - e) > pgk::kHalfMostExp) ok = false;
-    return ldexpf(1.0f, ok ? 15 - e : 0);
-  };
-  for (size_t l = 0; l < g.L; ++l) {
-    pg_model::HalfLayer& w = m->half[l];
-    const unsigned* b = got.data() + l * kBounds;
-    w.norm_1 = scale(b[0]), w.norm_2 = scale(b[1]), w.hidden = scale(b[2]);
-    w.attn = {scale(b[3]), scale(b[4]), scale(b[5])};
-  }
-  if (!ok) {
+  unsigned got = 0;
+  PG_HIP(hipMemcpy(&got, refused, 4, hipMemcpyDeviceToHost));
+  if (got) {
     m->half.clear();
     (void)hipFree(m->half_arena);
     m->half_arena = nullptr;
@@ -667,13 +660,13 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
   auto gemm = [&](const float* A, int lda, const float* W, const float* bias, float* Cout,
                   int ldc, int N, int K, int epi, const float* ln_g = nullptr,
                   const float* ln_b = nullptr, int a_cut = 0, int c_cut = 0, const void* w_half = nullptr,
-                  const float* w_half_mul = nullptr, float a_scale = 0.0f, float c_scale = 0.0f, float ln_scale = 0.0f) -> hipError_t {
+                  const float* w_half_mul = nullptr, const float* c_scale = nullptr, bool ln_half = false) -> hipError_t {
     pgk::GemmArgs a{};
     a.A = A; a.w_bf16 = m->w_bf16; a.W = W; a.bias = bias; a.resid = Cout; a.C = Cout;
     a.a_cut = a.ln_cut = a_cut; a.c_cut = c_cut;
     if (w_half) {
       a.w_half = w_half; a.w_half_mul = w_half_mul; a.w_half_parts = m->w_bf16 || m->w_i8 ? 1 : 2;
-      a.a_unscale = 1.0f / a_scale; a.c_scale = c_scale; a.ln_scale = ln_g ? ln_scale : 0.0f;
+      a.a_unscale = 1.0f; a.c_scale = c_scale; a.ln_scale = ln_half ? 1.0f : 0.0f;  // (the powers are in W and in the norms)
       if (cut) a.w_half_parts = 3, a.a_cut = a.c_cut = 0;  // (W is in cut form)
     }
     a.M = T; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc;
@@ -685,7 +678,7 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
     return pgk::launch_gemm(a, epi, m->num_cus, s);
   };
   if (half)
-    PG_HIP(pgk::launch_norm_rows_half(X.p, XN.p, T, C, m->layers[0].ln_1_g, m->layers[0].ln_1_b, g.eps, m->half[0].norm_1, s));
+    PG_HIP(pgk::launch_norm_rows_half(X.p, XN.p, T, C, m->half[0].norm_1_g, m->half[0].norm_1_b, g.eps, 1.0f, s));
   else
     PG_HIP(pgk::launch_layer_norm_rows(X.p, XN.p, T, C, m->layers[0].ln_1_g, m->layers[0].ln_1_b, g.eps, s, form_of));
   PG_MARK(kLayerNorm);
@@ -694,14 +687,16 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
     pg_model::HalfLayer hw = half || cut_w ? m->half[l] : pg_model::HalfLayer{};
     if (cut_w) {
       hw.c_attn = hw.c_attn_cut, hw.c_proj = hw.c_proj_cut, hw.c_fc = hw.c_fc_cut, hw.c_proj_mlp = hw.c_proj_mlp_cut;
-      hw.norm_1 = hw.norm_2 = hw.hidden = hw.attn.v = 1.0f;  // (cut form is not scaled)
+      hw.hidden = nullptr;  // (cut form is not scaled)
     }
     // the LayerNorm after this layer: the next layer's ln_1; ln_f is applied where it is needed
-    const float* next_g = l + 1 < g.L ? m->layers[l + 1].ln_1_g : nullptr;
-    const float* next_b = l + 1 < g.L ? m->layers[l + 1].ln_1_b : nullptr;
-    const float next_norm = half && l + 1 < g.L ? m->half[l + 1].norm_1 : 0.0f;
+    const bool next = l + 1 < g.L;
+    const float* next_g = !next ? nullptr : half ? m->half[l + 1].norm_1_g : m->layers[l + 1].ln_1_g;
+    const float* next_b = !next ? nullptr : half ? m->half[l + 1].norm_1_b : m->layers[l + 1].ln_1_b;
+    const float* ln_2_g = half ? hw.norm_2_g : w.ln_2_g;
+    const float* ln_2_b = half ? hw.norm_2_b : w.ln_2_b;
     PG_HIP(gemm(XN.p, C, w.c_attn_w, w.c_attn_b, QKV.p, 3 * C, 3 * C, C, pgk::GEMM_BIAS, nullptr, nullptr, cut, 0,
-                hw.c_attn, hw.c_attn_mul, hw.norm_1));
+                hw.c_attn, hw.c_attn_mul));
     PG_MARK(kQkv);
     if (half || (cut && !m->half.empty()))
       PG_HIP(pgk::launch_attn_prefill_half(QKV.p, Ts, C, H, P, c->k_panel(l, b), c->v_panel(l, b), ATT.p, s, (int)nb,
@@ -711,14 +706,14 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
       PG_HIP(pgk::launch_attn_prefill(QKV.p, Ts, C, H, hd, P, c->k_panel(l, b), c->v_panel(l, b),
                                       ATT.p, SCR.p, m->num_cus, s, (int)nb, g.H * g.P * g.hd(), form_of, c->drawn));
     PG_MARK(kAttention);
-    PG_HIP(gemm(ATT.p, C, w.c_proj_w, w.c_proj_b, X.p, C, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b, cut, 0,
-                hw.c_proj, hw.c_proj_mul, hw.attn.v, 0.0f, half ? hw.norm_2 : 0.0f));
+    PG_HIP(gemm(ATT.p, C, w.c_proj_w, w.c_proj_b, X.p, C, C, C, pgk::GEMM_RESID, ln_2_g, ln_2_b, cut, 0,
+                hw.c_proj, hw.c_proj_mul, nullptr, half));
     PG_MARK(kAttnProj);
     PG_HIP(gemm(XN.p, C, w.c_fc_w, w.c_fc_b, HB.p, I, I, C, pgk::GEMM_GELU, nullptr, nullptr, cut, cut,
-                hw.c_fc, hw.c_fc_mul, hw.norm_2, hw.hidden));
+                hw.c_fc, hw.c_fc_mul, hw.hidden));
     PG_MARK(kMlpFc);
     PG_HIP(gemm(HB.p, I, w.c_proj_mlp_w, w.c_proj_mlp_b, X.p, C, C, I, pgk::GEMM_RESID, next_g, next_b, cut, 0,
-                hw.c_proj_mlp, hw.c_proj_mlp_mul, hw.hidden, 0.0f, next_norm));
+                hw.c_proj_mlp, hw.c_proj_mlp_mul, nullptr, half && next));
     PG_MARK(kMlpProj);
   }
   if (all_logits_dst) {
@@ -796,12 +791,12 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
   auto gemm = [&](const float* A, int lda, const float* W, const float* bias, float* Cout,
                   int ldc, int N, int K, int epi, const float* ln_g = nullptr,
                   const float* ln_b = nullptr, int a_cut = 0, int ln_cut = 0, const void* w_half = nullptr,
-                  const float* w_half_mul = nullptr, float a_scale = 0.0f, float c_scale = 0.0f, float ln_scale = 0.0f) -> hipError_t {
+                  const float* w_half_mul = nullptr, const float* c_scale = nullptr, bool ln_half = false) -> hipError_t {
     pgk::GemmArgs a{};
     a.A = A; a.w_bf16 = m->w_bf16; a.W = W; a.bias = bias; a.resid = Cout; a.C = Cout;
     if (w_half) {
       a.w_half = w_half; a.w_half_mul = w_half_mul; a.w_half_parts = m->w_bf16 || m->w_i8 ? 1 : 2;
-      a.a_unscale = 1.0f / a_scale; a.c_scale = c_scale; a.ln_scale = ln_scale;
+      a.a_unscale = 1.0f; a.c_scale = c_scale; a.ln_scale = ln_half ? 1.0f : 0.0f;  // (the powers are in W and in the norms)
     }
     a.M = B; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc;
     if (m->w_i8) a.w_scale = i8_scales_of(W, (size_t)N, (size_t)K);
@@ -815,19 +810,19 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
   };
   PG_HIP(pgk::launch_embed_batch(c->x, m->wte, m->wpe, d_ids, B, (int)pos, C, s, m->w_bf16));
   if (half)
-    PG_HIP(pgk::launch_norm_rows_half(c->x, c->xn_b, B, C, m->layers[0].ln_1_g, m->layers[0].ln_1_b, g.eps, m->half[0].norm_1, s));
+    PG_HIP(pgk::launch_norm_rows_half(c->x, c->xn_b, B, C, m->half[0].norm_1_g, m->half[0].norm_1_b, g.eps, 1.0f, s));
   else
     PG_HIP(pgk::launch_layer_norm_rows(c->x, c->xn_b, B, C, m->layers[0].ln_1_g, m->layers[0].ln_1_b,
                                        g.eps, s, form));
   for (size_t l = 0; l < g.L; ++l) {
     const pgk::LayerW& w = m->layers[l];
     // the LayerNorm after this layer: the next layer's ln_1, or ln_f
-    const float* next_g = l + 1 < g.L ? m->layers[l + 1].ln_1_g : m->ln_f_g;
-    const float* next_b = l + 1 < g.L ? m->layers[l + 1].ln_1_b : m->ln_f_b;
+    const bool next_half = half && l + 1 < g.L;  // (the logits' input is plain rows)
+    const float* next_g = next_half ? m->half[l + 1].norm_1_g : l + 1 < g.L ? m->layers[l + 1].ln_1_g : m->ln_f_g;
+    const float* next_b = next_half ? m->half[l + 1].norm_1_b : l + 1 < g.L ? m->layers[l + 1].ln_1_b : m->ln_f_b;
     const pg_model::HalfLayer hw = half ? m->half[l] : pg_model::HalfLayer{};
-    const float next_norm = half && l + 1 < g.L ? m->half[l + 1].norm_1 : 0.0f;  // (the logits' input is plain rows)
     PG_HIP(gemm(c->xn_b, C, w.c_attn_w, w.c_attn_b, c->qkv_b, 3 * C, 3 * C, C, pgk::GEMM_BIAS, nullptr, nullptr, cut, 0,
-                hw.c_attn, hw.c_attn_mul, hw.norm_1));
+                hw.c_attn, hw.c_attn_mul));
     // K/V append (rust.rs:1677-1683): by the attention launch itself for head_dim 64
     const bool fused_append = hd == pgk::kHeadDim;
     if (!fused_append)
@@ -839,12 +834,12 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
     if (!one_split)
       PG_HIP(pgk::launch_attn_finish(c->part_acc, c->part_m, c->part_l, H, hd, nsplit, c->att_b, s,
                                      B, bs, form, hw.attn.v));
-    PG_HIP(gemm(c->att_b, C, w.c_proj_w, w.c_proj_b, c->x, C, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b, cut, cut,
-                hw.c_proj, hw.c_proj_mul, hw.attn.v, 0.0f, hw.norm_2));
+    PG_HIP(gemm(c->att_b, C, w.c_proj_w, w.c_proj_b, c->x, C, C, C, pgk::GEMM_RESID, half ? hw.norm_2_g : w.ln_2_g,
+                half ? hw.norm_2_b : w.ln_2_b, cut, cut, hw.c_proj, hw.c_proj_mul, nullptr, half));
     PG_HIP(gemm(c->xn_b, C, w.c_fc_w, w.c_fc_b, c->hbuf, I, I, C, pgk::GEMM_GELU, nullptr, nullptr, cut, 0,
-                hw.c_fc, hw.c_fc_mul, hw.norm_2, hw.hidden));
+                hw.c_fc, hw.c_fc_mul, hw.hidden));
     PG_HIP(gemm(c->hbuf, I, w.c_proj_mlp_w, w.c_proj_mlp_b, c->x, C, C, I, pgk::GEMM_RESID, next_g, next_b, cut,
-                cut && l + 1 < g.L, hw.c_proj_mlp, hw.c_proj_mlp_mul, hw.hidden, 0.0f, next_norm));
+                cut && l + 1 < g.L, hw.c_proj_mlp, hw.c_proj_mlp_mul, nullptr, next_half));
   }
   PG_HIP(gemm(c->xn_b, C, m->lm_w, nullptr, c->logits_buf, (int)g.V, (int)g.V, C, pgk::GEMM_BIAS));
   return PG_OK;

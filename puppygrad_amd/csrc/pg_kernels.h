@@ -111,7 +111,7 @@ hipError_t launch_attn_decode(const float* q, const float* kcache, const float* 
                               int P, int H, int head_dim, int nsplit, float* part_acc,
                               float* part_m, float* part_l, hipStream_t s, int batch = 1,
                               BatchStrides bs = BatchStrides{}, int append_C = 0,
-                              float* direct_out = nullptr, int out_form = 0, float out_scale = 1.0f);
+                              float* direct_out = nullptr, int out_form = 0, const float* out_scale = nullptr);
 // blocks_per_cu: (head, split) blocks per CU to aim for (tunable, 4 by default).
 int choose_nsplit(int n_keys, int H, int num_cus, int blocks_per_cu = 4);
 
@@ -194,7 +194,7 @@ hipError_t launch_transpose(const float* src, float* dst, int in_f, int out_f, h
 // Attention output from a single split's (acc, m, l): out = acc / l per head.
 hipError_t launch_attn_finish(const float* part_acc, const float* part_m, const float* part_l,
                               int H, int head_dim, int nsplit, float* out, hipStream_t s,
-                              int batch = 1, BatchStrides bs = BatchStrides{}, int out_form = 0, float out_scale = 1.0f);
+                              int batch = 1, BatchStrides bs = BatchStrides{}, int out_form = 0, const float* out_scale = nullptr);
 hipError_t launch_fill_zero(float* p, size_t n, hipStream_t s);
 // out[2 o] = sum_i W[o,i] g[i], out[2 o + 1] = (bias ? bias[o] : 0) + sum_i W[o,i] b[i] for the
 // rows of W[rows][cols] as stored (w_bytes 4: f32, 2: bf16, 1: int8 with scales[o]); sums in f64.
@@ -264,13 +264,14 @@ struct GemmArgs {
   // name; a_cut decides the kernel, the other two may go with it only.
   int a_cut = 0, c_cut = 0, ln_cut = 0;
   // a_unscale > 0: A is in half form (FORM_HALF), its values 1 / a_unscale times what they stand for, and W's half form is
-  // w_half (launch_half_rows), of w_half_parts f16 numbers a weight.  GEMM_GELU then writes C in half form, times c_scale,
-  // and ln_out is in half form, times ln_scale (0: as it would be otherwise); no other form goes with it.  Powers of two.
-  // w_half_parts 3 (f32 rows): A, C of GEMM_GELU and, with ln_cut, ln_out are in cut form, W in launch_cut_weights'; the scales are 1.
+  // w_half (launch_half_rows), of w_half_parts f16 numbers a weight.  GEMM_GELU then writes C in half form, column n times
+  // c_scale[n], and ln_out is in half form, times ln_scale (0: as it would be otherwise); no other form goes with it.  Powers of two.
+  // w_half_parts 3 (f32 rows): A, C of GEMM_GELU and, with ln_cut, ln_out are in cut form, W in launch_cut_weights'; a_unscale is 1, c_scale null.
   const void* w_half = nullptr;
   const float* w_half_mul = nullptr;
   int w_half_parts = 0;
-  float a_unscale = 0.0f, c_scale = 0.0f, ln_scale = 0.0f;
+  const float* c_scale = nullptr;
+  float a_unscale = 0.0f, ln_scale = 0.0f;
   // Tunable: a GEMM whose M x N leaves CUs idle is cut along K into about this many work items
   // per CU (gemm_split_parts).
   int split_items_per_cu = 3;
@@ -304,19 +305,24 @@ constexpr int kNormWidest = 4096;
 hipError_t launch_norm_rows_half(float* src, void* dst, int rows, int cols, const float* g, const float* b, float eps,
                                  float scale, hipStream_t s, int parts = 0, const float* ws = nullptr, const float* bias = nullptr,
                                  const float* resid = nullptr);
-// W[rows][cols] as stored (w_bytes 4: f32, 2: bf16, 1: int8 with scales[row]) in half form: two f16 numbers a weight (f32
-// rows) or one, cols a multiple of 32, and what a sum over them is to be multiplied with, mul[rows].  *refused is set (never
-// cleared) where the rows do not allow it (k_half_rows).
+// W[rows][cols] as stored (w_bytes 4: f32, 2: bf16, 1: int8 with scales[row]) in half form, for inputs whose column k is kept times
+// powers[k] (null: as they are): two f16 numbers a weight (f32 rows) or one, cols a multiple of 32, and what a sum over them is to
+// be multiplied with, mul[rows].  *refused is set (never cleared), here and below, where the values do not allow it (k_half_rows).
 constexpr int kHalfMostExp = 60;
 // f32 rows in cut form, three bf16 numbers a weight, for inputs in cut form.
 hipError_t launch_cut_weights(const float* W, size_t rows, int cols, void* to, hipStream_t s);
-hipError_t launch_half_rows(const void* W, int w_bytes, const float* scales, size_t rows, int cols, void* to, float* mul,
-                            unsigned* refused, hipStream_t s);
-// *most = max(*most, the largest magnitude that an output of these rows behind a LayerNorm with scale g can have; fold as
-// launch_ln_fold leaves it), and that of the norm's own values.  Bits of floats; infinite where there is no bound.
+hipError_t launch_half_rows(const void* W, int w_bytes, const float* scales, const float* powers, size_t rows, int cols, void* to,
+                            float* mul, unsigned* refused, hipStream_t s);
+// bounds[row]: the largest magnitude that an output of this row behind a LayerNorm with gains g can have; fold as launch_ln_fold
+// leaves it.  launch_half_powers: to the powers of two that put them at 2^15 at most.
 hipError_t launch_half_bound(const void* W, int w_bytes, const float* scales, const float* g, const float* fold, size_t rows, int cols,
-                             unsigned* most, hipStream_t s);
-hipError_t launch_half_bound_norm(const float* g, const float* b, int cols, unsigned* most, hipStream_t s);
+                             float* bounds, hipStream_t s);
+hipError_t launch_half_powers(float* at, int n, unsigned* refused, hipStream_t s);
+// The same of a LayerNorm's own values, and its gains and shifts times the powers.
+hipError_t launch_half_norm_powers(const float* g, const float* b, int cols, float* powers, float* g_out, float* b_out, unsigned* refused,
+                                   hipStream_t s);
+// The same of heads of 64 queries' and keys' dims, whose powers' product is score[head] (HalfScales).
+hipError_t launch_half_score_powers(float* q, float* k, int heads, float* score, unsigned* refused, hipStream_t s);
 // Rows that an activation matrix of M rows in cut form has room for; it takes 6 * K * cut_rows(M) bytes.
 __host__ __device__ inline int cut_rows(int M) { return (M + 15) / 16 * 16; }
 inline size_t cut_floats(size_t M, size_t K) { return (M + 15) / 16 * 16 * K * 3 / 2; }
@@ -349,11 +355,11 @@ hipError_t launch_attn_prefill(const float* qkv, int T, int C, int H, int head_d
 int attn_cut_shape(int T, int H, int nseq, int num_cus);
 hipError_t launch_attn_prefill_cut(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, float* out,
                                    hipStream_t s, int nseq, size_t kv_stride, int out_form, int shape);
-// The same on the f16 matrix cores (pg_attn_half.hip): out in half form times scales.v, or in cut form; the scales are powers of two with which no
-// query, key or value is past 2^15.  Shapes (groups of 32 queries, groups of
-// keys) 41, 22, 24, 18, 14; attn_half_shape: the one to take.
+// The same on the f16 matrix cores (pg_attn_half.hip): out in half form times scales.v, or in cut form; the scales are powers of two,
+// one for each of the C columns, with which no query, key or value is past 2^15, q[c] k[c] = score[head] wherever neither is always
+// 0.  Shapes (groups of 32 queries, groups of keys) 41, 22, 24, 18, 14; attn_half_shape: the one to take.
 struct HalfScales {
-  float q, k, v;
+  const float *q, *k, *v, *score;
 };
 int attn_half_shape(int T, int H, int nseq, int num_cus);
 hipError_t launch_attn_prefill_half(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, void* out,

@@ -611,7 +611,7 @@ __device__ __forceinline__ float4 nt_load4(const float4* p) {
 // softmax_in_place, cpu.rs:152-165, rescaled when the max moves); the four are merged
 // through LDS at the end, and the per-split (acc, m, l) by the consumer.
 // The launcher picks IT so that one chunk covers the split where the split count allows.
-// FORM: how direct_out lies, FORM_CUT, FORM_HALF (times out_scale) or as out_form says.
+// FORM: how direct_out lies, FORM_CUT, FORM_HALF (column i times out_scale[i]) or as out_form says.
 template <int IT, int FORM>
 __global__ __launch_bounds__(kBlock) void k_attn_decode64(const float* __restrict__ q,
                                                           const float* kcache, const float* vcache,
@@ -619,7 +619,7 @@ __global__ __launch_bounds__(kBlock) void k_attn_decode64(const float* __restric
                                                           float* part_acc, float* part_m,
                                                           float* part_l, BatchStrides bs,
                                                           int append_C, float* direct_out,
-                                                          int out_form, float out_scale) {
+                                                          int out_form, const float* out_scale) {
   // direct_out (only with nsplit == 1): the block's result is the head's attention output
   // and is written there (row blockIdx.z, in whichever ActForm), with no partials and no
   // merge launch.
@@ -735,7 +735,7 @@ __global__ __launch_bounds__(kBlock) void k_attn_decode64(const float* __restric
     if (direct_out) {
       const size_t b = blockIdx.z, i = (size_t)h * 64 + tid;
       if constexpr (FORM == FORM_CUT) store_cut1(direct_out, cut_rows((int)gridDim.z), b, i, t / l);
-      else if constexpr (FORM == FORM_HALF) store_half1(direct_out, cut_rows((int)gridDim.z), b, i, t / l, out_scale);
+      else if constexpr (FORM == FORM_HALF) store_half1(direct_out, cut_rows((int)gridDim.z), b, i, t / l, out_scale[i]);
       else direct_out[out_form == FORM_PACKED32 ? packed32_index(b, i) : b * bs.out + i] = t / l;
       return;
     }
@@ -798,7 +798,7 @@ __global__ __launch_bounds__(kBlock) void k_attn_decode_any(const float* q, cons
 template <int FORM>
 __global__ void k_attn_finish(const float* part_acc, const float* part_m, const float* part_l,
                               int C, int hd, int nsplit, float* out, BatchStrides bs,
-                              int out_form, float out_scale) {
+                              int out_form, const float* out_scale) {
   const size_t b = blockIdx.y;
   part_acc += b * bs.part * hd;
   part_m += b * bs.part;
@@ -807,7 +807,7 @@ __global__ void k_attn_finish(const float* part_acc, const float* part_m, const 
   if (i >= C) return;
   const float v = attn_combine_elem(part_acc, part_m, part_l, nsplit, hd, i);
   if constexpr (FORM == FORM_CUT) store_cut1(out, cut_rows((int)gridDim.y), b, (size_t)i, v);
-  else if constexpr (FORM == FORM_HALF) store_half1(out, cut_rows((int)gridDim.y), b, (size_t)i, v, out_scale);
+  else if constexpr (FORM == FORM_HALF) store_half1(out, cut_rows((int)gridDim.y), b, (size_t)i, v, out_scale[i]);
   else out[out_form == FORM_PACKED32 ? packed32_index(b, (size_t)i) : b * bs.out + i] = v;
 }
 
@@ -1491,7 +1491,7 @@ int choose_nsplit(int n_keys, int H, int num_cus, int blocks_per_cu) {
 hipError_t launch_attn_decode(const float* q, const float* kcache, const float* vcache, int pos,
                               int P, int H, int head_dim, int nsplit, float* part_acc,
                               float* part_m, float* part_l, hipStream_t s, int batch,
-                              BatchStrides bs, int append_C, float* direct_out, int out_form, float out_scale) {
+                              BatchStrides bs, int append_C, float* direct_out, int out_form, const float* out_scale) {
   if (direct_out && (head_dim != kHeadDim || nsplit != 1 || (out_form == FORM_PACKED32 && batch > 32)))
     return hipErrorInvalidValue;
   if (head_dim == kHeadDim) {
@@ -1524,7 +1524,7 @@ hipError_t launch_attn_decode(const float* q, const float* kcache, const float* 
 
 hipError_t launch_attn_finish(const float* part_acc, const float* part_m, const float* part_l,
                               int H, int head_dim, int nsplit, float* out, hipStream_t s,
-                              int batch, BatchStrides bs, int out_form, float out_scale) {
+                              int batch, BatchStrides bs, int out_form, const float* out_scale) {
   int C = H * head_dim;
   if (out_form == FORM_PACKED32 && batch > 32) return hipErrorInvalidValue;
   const dim3 grid((C + 255) / 256, batch);

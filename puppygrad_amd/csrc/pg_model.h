@@ -127,13 +127,13 @@ struct pg_model {
   float* lm_w = nullptr;
   float* lm_s = nullptr;
   float* lm_f = nullptr;  // [2 V]: LN_f folded into the lm_head rows (pgk::launch_ln_fold)
-  // The block matrices in half form beside their rows (pgk::launch_half_rows), and what a layer's activations are multiplied
-  // with where they are kept so: powers of two that put the largest value that each can have (pgk::launch_half_bound) at
-  // 2^15 at most.  Empty where the weights do not allow it or there was no memory for them.
+  // The block matrices in half form beside their rows (pgk::launch_half_rows), and what the columns of a layer's activations are
+  // multiplied with where they are kept so: powers of two that put the largest value that each can have (pgk::launch_half_bound)
+  // at 2^15 at most; norms have them in their gains and shifts.  Empty where the weights do not allow it or there was no memory for them.
   struct HalfLayer {
     const void *c_attn, *c_proj, *c_fc, *c_proj_mlp;
     const float *c_attn_mul, *c_proj_mul, *c_fc_mul, *c_proj_mlp_mul;
-    float norm_1, norm_2, hidden;
+    const float *norm_1_g, *norm_1_b, *norm_2_g, *norm_2_b, *hidden;
     pgk::HalfScales attn;  // queries, keys, values (and what attention makes of them)
     const void *c_attn_cut, *c_proj_cut, *c_fc_cut, *c_proj_mlp_cut;  // the same matrices in cut form, or null
   };

@@ -9,8 +9,10 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <initializer_list>
 #include <mutex>
 #include <string>
+#include <vector>
 
 #include "pg_gemm_dev.h"
 #include "pg_half.h"
@@ -173,6 +175,19 @@ __global__ __launch_bounds__(kBlk) void k_attention_rows(const float* __restrict
     for (int gg = 0; gg < groups; ++gg) t += part[gg * hd + tid];
     out[(size_t)query * state + (size_t)head * hd + tid] = t;
   }
+}
+
+// (for the tests: each of `values` n times, on the device)
+struct Constants {
+  float* p = nullptr;
+  ~Constants() { (void)hipFree(p); }
+};
+pg_status constants(std::initializer_list<float> values, size_t n, Constants* to) {
+  std::vector<float> all;
+  for (float v : values) all.insert(all.end(), n, v);
+  PG_HIP(hipMalloc(&to->p, all.size() * sizeof(float)));
+  PG_HIP(hipMemcpy(to->p, all.data(), all.size() * sizeof(float), hipMemcpyHostToDevice));
+  return PG_OK;
 }
 
 // (for the tests: x[M][K] in cut form, K a multiple of 8)
@@ -465,8 +480,8 @@ pg_status pg_testing_half_product_dev(int32_t device, void* stream, const float*
     PG_HIP(pgk::launch_cut_weights(static_cast<const float*>(weight), out_f, (int)in_f, w_half, st));
     hipLaunchKernelGGL(k_to_cut, x_blocks, dim3(256), 0, st, x, work, (int)rows, (int)in_f);
   } else {
-    PG_HIP(pgk::launch_half_rows(weight, storage == PG_STORE_F32 ? 4 : storage == PG_STORE_BF16 ? 2 : 1, scales, out_f, (int)in_f,
-                                 w_half, mul, refused, st));
+    PG_HIP(pgk::launch_half_rows(weight, storage == PG_STORE_F32 ? 4 : storage == PG_STORE_BF16 ? 2 : 1, scales, nullptr, out_f,
+                                 (int)in_f, w_half, mul, refused, st));
     hipLaunchKernelGGL(k_to_half, x_blocks, dim3(256), 0, st, x, work, (int)rows, (int)in_f, scale);
   }
   PG_HIP(hipGetLastError());
@@ -474,8 +489,13 @@ pg_status pg_testing_half_product_dev(int32_t device, void* stream, const float*
   a.A = reinterpret_cast<const float*>(work); a.w_half = w_half; a.w_half_mul = mul; a.w_half_parts = pw; a.a_unscale = cut ? 1.0f : 1.0f / scale;
   a.bias = bias; a.C = out; a.M = (int)rows; a.N = (int)out_f; a.K = (int)in_f; a.ldc = (int)out_f;
   a.ws = out; a.ws_floats = (size_t)parts * rows * out_f;
-  if (gelu) a.c_scale = 1.0f;
+  Constants ones;
+  if (gelu && !cut) {
+    if ((s = constants({1.0f}, out_f, &ones))) return s;
+    a.c_scale = ones.p;
+  }
   PG_HIP(pgk::launch_gemm_half_plan(a, gelu ? pgk::GEMM_GELU : pgk::GEMM_BIAS, {tile, parts, mt, block_rows}, st));
+  if (ones.p) PG_HIP(hipStreamSynchronize(st));
   return PG_OK;
 }
 
@@ -492,7 +512,8 @@ pg_status pg_testing_norm_half_dev(int32_t device, void* stream, float* x, uint6
   return PG_OK;
 }
 
-// The same by pg_attn_half.hip: out in half form times sv, or (cut) in cut form; shape 0: as the planner has it.
+// The same by pg_attn_half.hip, all queries, keys and values times sq, sk and sv: out in half form times sv, or (cut) in cut form; shape 0:
+// as the planner has it.
 pg_status pg_testing_attention_half_dev(int32_t device, void* stream, const float* qkv, uint64_t rows, uint64_t heads,
                                         uint64_t sequences, int32_t shape, float sq, float sk, float sv, int32_t cut, float* keys,
                                         float* values, void* out) {
@@ -504,9 +525,13 @@ pg_status pg_testing_attention_half_dev(int32_t device, void* stream, const floa
   const int T = (int)rows, H = (int)heads;
   int cus = 0;
   PG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+  Constants scales;
+  const size_t C = 64 * heads;
+  if ((s = constants({sq, sk, sv, sq * sk}, C, &scales))) return s;
   PG_HIP(pgk::launch_attn_prefill_half(qkv, T, 64 * H, H, T, keys, values, out, static_cast<hipStream_t>(stream), (int)sequences,
-                                       (size_t)H * T * 64, {sq, sk, sv}, shape ? shape : pgk::attn_half_shape(T, H, (int)sequences, cus),
-                                       cut ? pgk::FORM_CUT : pgk::FORM_HALF));
+                                       (size_t)H * T * 64, {scales.p, scales.p + C, scales.p + 2 * C, scales.p + 3 * C},
+                                       shape ? shape : pgk::attn_half_shape(T, H, (int)sequences, cus), cut ? pgk::FORM_CUT : pgk::FORM_HALF));
+  PG_HIP(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
   return PG_OK;
 }
 

@@ -1734,7 +1734,7 @@ bool gemm_takes_rows32(int M, int K, int lda, int w_bf16) {
 
 namespace {
 hipError_t launch_gemm_form(const GemmArgs& a, int epi, int num_cus, hipStream_t s, bool* ln_done) {
-  if (a.c_scale != 0.0f || a.ln_scale != 0.0f) return hipErrorInvalidValue;
+  if (a.c_scale || a.ln_scale != 0.0f) return hipErrorInvalidValue;
   if (a.a_cut) {
     CutRowsPlan plan;
     if (!gemm_cut_rows_plan(a, num_cus, &plan)) return hipErrorInvalidValue;

@@ -289,6 +289,70 @@ def test_scales_hold_for_models_of_any_size_of_values():
         assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want), (gain, weight)
 
 
+def uneven_weights(cfg, seed):
+    """Norms, values, hidden units and dims of queries and keys whose columns are of sizes up to 10^8 apart, and what reads them of the inverse."""
+    w = synth.random_weights(cfg, seed, perturb=True)
+    rng, c, n = np.random.default_rng(seed), cfg.n_embd, cfg.n_inner
+
+    def times(blk, name, by, rows, cols, at=slice(None)):  # by a column, or by a row (of the [in, out] matrix)
+        a = np.array(getattr(blk, name), np.float32).reshape(rows, cols)
+        a[:, at] *= by.astype(np.float32)
+        setattr(blk, name, a.reshape(np.shape(getattr(blk, name))))
+
+    for blk in w.blocks:
+        for norm, matrix, out in (("ln_1", "c_attn_w", 3 * c), ("ln_2", "c_fc_w", n)):
+            by = 10.0 ** rng.uniform(-4, 4, c)
+            times(blk, norm + "_g", by, 1, c)
+            times(blk, norm + "_b", by, 1, c)
+            times(blk, matrix, 1.0 / by[:, None], c, out)
+        score, value, inner = 10.0 ** rng.uniform(-4, 4, c), 10.0 ** rng.uniform(-4, 4, c), 10.0 ** rng.uniform(-3, 3, n)
+        for at, by in ((slice(0, c), score), (slice(c, 2 * c), 1.0 / score), (slice(2 * c, None), value)):
+            times(blk, "c_attn_w", by, c, 3 * c, at)
+            times(blk, "c_attn_b", by, 1, 3 * c, at)
+        times(blk, "c_proj_w", 1.0 / value[:, None], c, c)
+        times(blk, "c_fc_w", inner, c, n)
+        times(blk, "c_fc_b", inner, 1, n)
+        times(blk, "c_proj_mlp_w", 1.0 / inner[:, None], n, c)
+    return w
+
+
+# (f32, 300 rows: cut form, with attention in half form)
+@pytest.mark.parametrize("storage,batch,n", [("f32", 1, 20), ("f32", 1, 300), ("f32", 4, 300), ("bf16", 1, 40), ("bf16", 1, 300), ("int8", 1, 40), ("int8", 2, 170)])
+def test_columns_of_unequal_size(storage, batch, n):
+    """Every column counts as it does in f32, however far below the largest it is."""
+    cfg = Gpt2Config(vocab_size=97, n_positions=320, n_embd=512, n_layer=2, n_head=8)
+    model = Gpt2Model.new(cfg, uneven_weights(cfg, 0x5EED0B07), Gpt2HipConfig(weight_storage=STORE[storage]))
+    ids = synth.token_ids(batch * (n + 1), 0x70C00B07, 97).reshape(batch, n + 1)
+    cache = model.new_kv_cache(batch)
+    got = [model.prefill_batch(np.ascontiguousarray(ids[:, :n]), cache).to_host().reshape(batch, -1)]
+    if batch > 1:
+        got.append(model.forward_one_batch(ids[:, n], cache).to_host())
+    for b in (0, batch - 1):  # the one-sequence kernels
+        single = model.new_kv_cache()
+        want = [model.prefill([int(ids[b, 0])], single)]
+        for t in ids[b, 1:]:
+            want.append(model.forward_one(int(t), single))
+            want[-1] = want[-1].to_host()
+        for logit, ref in zip(got, want[n - 1:]):
+            # (the same values, sums of at most 2048 terms in other orders)
+            assert np.linalg.norm(logit[b] - ref) <= 1e-5 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("storage,batch", [("f32", 8), ("bf16", 40), ("int8", 24)])
+def test_steps_of_columns_of_unequal_size(storage, batch):
+    cfg = Gpt2Config(vocab_size=97, n_positions=32, n_embd=512, n_layer=2, n_head=8)
+    model = Gpt2Model.new(cfg, uneven_weights(cfg, 0x5EED0B08), Gpt2HipConfig(weight_storage=STORE[storage]))
+    ids = synth.token_ids(batch * 3, 0x70C00B08, 97).reshape(batch, 3)
+    cache = model.new_kv_cache(batch)
+    model.prefill_batch(np.ascontiguousarray(ids[:, :2]), cache)
+    got = model.forward_one_batch(ids[:, 2], cache).to_host()
+    for b in (0, batch - 1):
+        single = model.new_kv_cache()
+        model.prefill([int(t) for t in ids[b, :2]], single)
+        want = model.forward_one(int(ids[b, 2]), single).to_host()
+        assert np.linalg.norm(got[b] - want) <= 1e-5 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("n", [20, 300])  # a block a row, a wavefront a row
 def test_rows_whose_squares_are_past_f32(n):
     """Their norm is its shift, in half form as in f32 rows."""
