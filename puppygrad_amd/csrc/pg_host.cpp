@@ -140,8 +140,8 @@ pg_status validate_input(const Cfg& c, const uint32_t* ids, size_t n) {
   return PG_OK;
 }
 
-// Gpt2KvCache::check_compatible (src/models/gpt2/rust.rs:206-234).
-pg_status check_compatible(const pg_model* m, const pg_kv_cache* c) {
+// Gpt2KvCache::check_compatible (src/models/gpt2/rust.rs:206-234), for a call in which the model writes to the cache.
+pg_status check_compatible(const pg_model* m, pg_kv_cache* c) {
   if (m->stack || c->stack) {  // the layers of a stack model differ in kind and size
     if (c->stack_model != m) return fail(PG_INVALID_INPUT, "cache was made for another model");
     return PG_OK;
@@ -161,6 +161,7 @@ pg_status check_compatible(const pg_model* m, const pg_kv_cache* c) {
   if (c->device != m->device)
     return fail(PG_INVALID_INPUT, "cache lives on device " + std::to_string(c->device) +
                                       " but the model is on device " + std::to_string(m->device));
+  c->values_of = c->values_of == 0 || c->values_of == m->serial ? m->serial : pg_kv_cache::kSeveral;
   return PG_OK;
 }
 
@@ -785,7 +786,8 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
   // Half form, which every cache has room for, goes before both (takes_half_form), but for up to 32 sequences and bf16 rows, whose
   // packed rows are a little faster (XL, eight steps behind 300 tokens, ms, packed / half form: 17 sequences (100) 20.9 / 21.3, 24 27.9 /
   // 28.2, 32 30.9 / 31.3; int8 rows, unpacked, of 32 28.8 / 27.3).
-  const bool half = takes_half_form(m, c->B) && !(m->w_bf16 && c->pack32);
+  // Not where the cache holds another model's values: this model's bounds on its own (make_half_form) say nothing of their averages.
+  const bool half = takes_half_form(m, c->B) && !(m->w_bf16 && c->pack32) && c->values_of == m->serial;
   const int pk = c->pack32 && !half ? 1 : 0, cut = !half && c->cut_form && takes_cut_form(m, c->B) ? 1 : 0;
   const int form = half ? pgk::FORM_HALF : cut ? pgk::FORM_CUT : pk ? pgk::FORM_PACKED32 : pgk::FORM_ROWS;
   auto gemm = [&](const float* A, int lda, const float* W, const float* bias, float* Cout,
@@ -1118,6 +1120,8 @@ pg_status pg_gpt2_create(const pg_gpt2_config* config, const pg_gpt2_weights_vie
   if ((s = select_device(opts.device))) return s;
 
   auto m = std::make_unique<pg_model>();
+  static std::atomic<uint64_t> models{0};
+  m->serial = ++models;
   m->cfg = g;
   m->device = opts.device;
   m->opts = opts;

@@ -97,6 +97,7 @@ struct ProfileMarks {
 
 struct pg_model {
   pgh::Cfg cfg;
+  uint64_t serial = 0;  // GPT-2 models: a number of its own, from 1 on
   int device = 0;
   int num_cus = 0;
   pg_hip_options opts{};
@@ -157,6 +158,10 @@ struct pg_kv_cache {
   uint32_t B = 1;
   size_t seq_len = 0;
   float* kv = nullptr;  // [L][2][B][H][P][hd]
+  // The model whose keys and values these are (pg_model::serial), 0: none's yet.  Once another model has written here, kSeveral for
+  // good: positions that one has left may come to light again (pg_kv_cache_set_seq_len).
+  static constexpr uint64_t kSeveral = ~0ull;
+  uint64_t values_of = 0;
   // per-sequence activation scratch, [B][...]
   float* seq_scratch = nullptr;  // activations of the full-sequence (GEMM) forward, grown on demand
   size_t seq_scratch_floats = 0;

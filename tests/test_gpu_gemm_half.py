@@ -353,6 +353,28 @@ def test_steps_of_columns_of_unequal_size(storage, batch):
         assert np.linalg.norm(got[b] - want) <= 1e-5 * np.linalg.norm(want)
 
 
+@pytest.mark.parametrize("storage,batch", [("f32", 8), ("bf16", 40), ("int8", 24)])
+@pytest.mark.parametrize("behind", [5, 60])  # (one share of the keys and several)
+def test_a_step_behind_another_models_values(storage, batch, behind):
+    """The cache holds values 10^4 times the largest that the stepping model can have itself."""
+    cfg = Gpt2Config(vocab_size=97, n_positions=80, n_embd=512, n_layer=2, n_head=8)
+    small, large = (synth.random_weights(cfg, 0x5EED0B09, perturb=True) for _ in range(2))
+    for blk in large.blocks:
+        blk.c_attn_b = np.array(blk.c_attn_b, np.float32)
+        blk.c_attn_b[1024:] += np.float32(1e5)
+    maker, model = (Gpt2Model.new(cfg, w, Gpt2HipConfig(weight_storage=STORE[storage])) for w in (large, small))
+    ids = synth.token_ids(batch * (behind + 1), 0x70C00B09, 97).reshape(batch, behind + 1)
+    cache = model.new_kv_cache(batch)
+    maker.prefill_batch(np.ascontiguousarray(ids[:, :behind]), cache)
+    got = model.forward_one_batch(ids[:, behind], cache).to_host()
+    for b in (0, batch - 1):
+        single = model.new_kv_cache()
+        maker.prefill([int(t) for t in ids[b, :behind]], single)
+        want = model.forward_one(int(ids[b, behind]), single).to_host()
+        # (the same values, sums of at most 2048 terms in other orders)
+        assert np.isfinite(want).all() and np.linalg.norm(got[b] - want) <= 1e-5 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("n", [20, 300])  # a block a row, a wavefront a row
 def test_rows_whose_squares_are_past_f32(n):
     """Their norm is its shift, in half form as in f32 rows."""
