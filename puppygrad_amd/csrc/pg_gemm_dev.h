@@ -35,8 +35,8 @@ hipError_t launch_gemm_cut_grouped(const GemmArgs& a, int epi, int tile_rows, hi
 
 // A product with activations and W in half form (pg_gemm_half.hip): the tile, or blocks of 16 mt input rows and `rows` rows of W
 // (HALF_ROWS), and parts of K (1: whole tiles; otherwise raw partial tiles to GemmArgs::ws).
-// (HALF_128x128_8: by eight wavefronts)
-enum HalfTile : int { HALF_64x128 = 0, HALF_128x128 = 1, HALF_128x128_8 = 2, HALF_128x256 = 3, HALF_ROWS = 4 };
+// (_8: by eight wavefronts; HALF_128x256: one chain of matrix instructions, its sums are the less precise ones)
+enum HalfTile : int { HALF_64x128 = 0, HALF_128x128 = 1, HALF_128x128_8 = 2, HALF_128x256 = 3, HALF_ROWS = 4, HALF_128x256_8 = 5 };
 struct HalfPlan {
   int tile, parts, mt, rows;
 };

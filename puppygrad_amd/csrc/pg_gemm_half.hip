@@ -11,7 +11,7 @@
 // (bf16 and int8 rows 4 10^-8), below what its roundings cost: with one f32 sum over K = 1600 2.7 10^-7.  Those are made
 // fewer for it: a chain of matrix instructions ends after CH stages, 64 to 128 columns, and is added to a total, and wherever
 // there are registers for it the small products are a chain of their own (in one with the others they are cut downward, and
-// the error has a mean: a model's logits were off by up to 1.4 times as much).  Error against f64 (values N(0, 1) by N(0, 0.02), of
+// the error has a mean: a model's logits were off by up to 1.4 times as much), or every second chain has the other sign.  Error against f64 (values N(0, 1) by N(0, 0.02), of
 // the result's norm, 512 rows), one part of K, before -> now: 1280 x 1280 f32 rows 2.1 10^-7 -> 1.3, K = 5120 4.5 -> 1.6 (64 x
 // 64 a wavefront: 1.4, 2.1); bf16 rows 2.1 -> 1.1, 4.5 -> 1.5; 128 x 256 tiles, one chain, 16384 x 1600 x 1600 4.3 -> 3.6.
 // Logits of prompts of 450 to 1000 tokens, all sizes: 0.65 to 0.85 of what they were off by.
@@ -92,13 +92,16 @@ __device__ __forceinline__ void store_gelu(void* to, int mp, size_t m, size_t n,
 // columns in NA buffers, a stage in steps of 16 whose operands are read during the step before.  One barrier per stage, in front of the step that reads the next stage: by then the wavefront has
 // waited for its own share of that stage, and has read the stage before it to the end, whose buffer is free for the stage that
 // is asked for next.  CH: stages in a chain of matrix instructions (0: one chain).  TWO: the small products of a chain have a
-// sum of their own.  SPLIT: the stages are cut into gridDim.y parts, raw partial tiles go to a.ws[part][M][N].  OCC:
+// sum of their own.  TURN: where there are no registers for that, every second chain has W's sign turned, and its sum is taken away
+// instead of added: the instructions cut what they add downward, most of all what is small next to the sum, and so the errors of two
+// chains cancel, which are of one sign otherwise (bf16 rows, K = 1024, a mean of -0.19 of 2^-23 of the outputs' size -> -0.01).  SPLIT: the stages are cut into gridDim.y parts, raw partial tiles go to a.ws[part][M][N].  OCC:
 // wavefronts per SIMD that the registers are kept for.
-template <int WM, int WN, int MB, int NB, int PX, int PW, int EPI, int SPLIT, int OCC, int NA, int KT, int CH, bool TWO>
+template <int WM, int WN, int MB, int NB, int PX, int PW, int EPI, int SPLIT, int OCC, int NA, int KT, int CH, bool TWO, bool TURN>
 __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
   constexpr int NW = WM * WN, BM = 32 * MB * WM, BN = 32 * NB * WN, NO = KT / 8, NS = KT / 16;
   constexpr int IA = NO * PX * BM / 64 / NW, IB = NO * PW * BN / 64 / NW;
   constexpr int UN = CH ? CH : NA;
+  static_assert(!TURN || (!TWO && CH != 0));
   static_assert(UN % NA == 0 && (NS == 2 || UN % 2 == 0) && UN <= 8 && (CH != 0 || !TWO));
   static_assert(NO * PX * BM % (64 * NW) == 0 && NO * PW * BN % (64 * NW) == 0 && BM % 64 == 0 && BN % 64 == 0);
   __shared__ u4v As[NA][NO * PX * BM];
@@ -174,9 +177,16 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
   };
   using P = Products<PX, PW>;
   constexpr int NP = P::n;
-  auto step = [&](auto first, const Ops& cur, Ops& nxt, int buf, int s) __attribute__((always_inline)) {
+  unsigned turned = 0;  // sign bits of two f16 numbers
+  auto step = [&](auto first, Ops& cur, Ops& nxt, int buf, int s) __attribute__((always_inline)) {
     constexpr bool fresh = CH != 0 && decltype(first)::value;
     read(buf, s, nxt);
+    if constexpr (TURN) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int p = 0; p < PW; ++p) cur.w[j][p] ^= turned;
+    }
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
 #pragma unroll
@@ -257,9 +267,15 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
 #pragma unroll
           for (int i = 0; i < MB; ++i) {
             if constexpr (TWO) acc[i][j] += low[TWO ? i : 0][TWO ? j : 0];
-            tot[CH ? i : 0][CH ? j : 0] += acc[i][j];
+            if constexpr (TURN) {
+#pragma unroll
+              for (int v = 0; v < 16; ++v) tot[CH ? i : 0][CH ? j : 0][v] = fmaf(acc[i][j][v], turned ? -1.0f : 1.0f, tot[CH ? i : 0][CH ? j : 0][v]);
+            } else {
+              tot[CH ? i : 0][CH ? j : 0] += acc[i][j];
+            }
           }
       }
+      if (TURN) turned ^= 0x80008000u;
     }
     vm_wait<0>();
   }
@@ -786,7 +802,7 @@ __global__ __launch_bounds__(64) void k_half_score_powers(float* q, float* k, fl
 }
 
 // ---- launchers ---------------------------------------------------------------------------------
-template <int WM, int WN, int MB, int NB, int PX, int PW, int OCC, int NA, int KT, int CH, bool TWO>
+template <int WM, int WN, int MB, int NB, int PX, int PW, int OCC, int NA, int KT, int CH, bool TWO, bool TURN = false>
 struct Shape {
   static constexpr int bm = 32 * MB * WM, bn = 32 * NB * WN;
   template <int EPI, int SPLIT>
@@ -795,7 +811,7 @@ struct Shape {
     const int tiles_m = (a.M + bm - 1) / bm, tiles_n = (a.N + bn - 1) / bn, tiles = tiles_m * tiles_n;
     a.band_rows = choose_band(tiles_m, std::max(1, (tiles + 7) / 8), bm, bn);
     const dim3 grid((unsigned)((tiles + 7) / 8 * 8), (unsigned)parts);  // whole rounds over the 8 XCDs
-    hipLaunchKernelGGL((k_gemm_half<WM, WN, MB, NB, PX, PW, EPI, SPLIT, OCC, NA, KT, CH, TWO>), grid, dim3(64 * WM * WN), 0, s, a);
+    hipLaunchKernelGGL((k_gemm_half<WM, WN, MB, NB, PX, PW, EPI, SPLIT, OCC, NA, KT, CH, TWO, TURN>), grid, dim3(64 * WM * WN), 0, s, a);
     return hipGetLastError();
   }
   static hipError_t launch(const GemmArgs& a, int epi, int parts, hipStream_t s) {
@@ -826,9 +842,10 @@ hipError_t launch_tile(const GemmArgs& a, int epi, const HalfPlan& p, hipStream_
   }
   switch (p.tile) {
     case HALF_64x128: return Shape<2, 2, 1, 2, 2, 1, 3, 2, 32, 4, true>::launch(a, epi, p.parts, s);
-    case HALF_128x128: return Shape<2, 2, 2, 2, 2, 1, 2, 4, 16, 4, false>::launch(a, epi, p.parts, s);
+    case HALF_128x128: return Shape<2, 2, 2, 2, 2, 1, 2, 3, 32, 3, false, true>::launch(a, epi, p.parts, s);
     case HALF_128x128_8: return Shape<4, 2, 1, 2, 2, 1, 2, 4, 32, 4, true>::launch(a, epi, p.parts, s);
     case HALF_128x256: return Shape<2, 2, 2, 4, 2, 1, 2, 4, 16, 0, false>::launch(a, epi, p.parts, s);
+    case HALF_128x256_8: return Shape<2, 4, 2, 2, 2, 1, 2, 4, 32, 4, true>::launch(a, epi, p.parts, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -876,10 +893,20 @@ struct RowsPace {
   float start, turn, step, mt, ng, both, fill_mt, fill_ng, uneven;
 };
 // [half form of f32 rows, of bf16 and int8 rows, cut form][HalfTile]
-constexpr TilePace kTilePace[3][4] = {
-    {{5.981f, 0.546f, 0.074f, 0.197f}, {9.04f, 0.604f, 0.329f, 0.111f}, {7.24f, 0.503f, 11.3f, 2.426f}, {}},
-    {{5.243f, 0.389f, 0.027f, 0.13f}, {6.453f, 0.422f, 0.178f, 0.125f}, {5.701f, 0.36f, 1.06f, -0.021f}, {10.216f, 0.619f, 0.316f, 0.158f}},
-    {{3.39f, 0.667f, 0.426f, -0.051f}, {}, {3.014f, 0.924f, 0.685f, 0.149f}, {}}};
+constexpr TilePace kTilePace[3][3] = {
+    {{5.981f, 0.546f, 0.074f, 0.197f}, {9.04f, 0.604f, 0.329f, 0.111f}, {7.24f, 0.503f, 11.3f, 2.426f}},
+    {{5.243f, 0.389f, 0.027f, 0.13f}, {6.453f, 0.422f, 0.178f, 0.125f}, {5.701f, 0.36f, 1.06f, -0.021f}},
+    {{3.39f, 0.667f, 0.426f, -0.051f}, {}, {3.014f, 0.924f, 0.685f, 0.149f}}};
+// Products of half form with a tile of 128 x 128 for every CU or more: K is not cut, and the tiles' times are fitted by themselves
+// (224 products of widths 768 to 1600, 130 to 16384 rows; 5 to 10 % off, the choice 1 to 1.5 % slower than the best tile in the mean).
+// HALF_128x256 is for bf16 rows and K up to 2048 only.  Its one chain errs by 3.6 10^-7 at K = 1600 and 7.3 10^-7 at 6400, the chains
+// of the eight wavefronts by 1.2 and 1.6 10^-7, at 1.12 to 1.24 of its time (16384 x 4800 x 1600 490 us for 412, x 1600 x 6400 644
+// for 588).  With it the logits of int8 models' prompts of 2000 rows were off by 1.2 times as much as three bf16 parts are, those
+// of bf16 models with it at K = 4096 too, without at 0.8.
+constexpr TilePace kFullPace[2][6] = {
+    {{6.49f, 0.469f, 0.075f, 0.323f}, {8.01f, 0.54f, 0.459f, 0.258f}, {8.36f, 0.462f, 0.668f, 0.168f}, {}, {}, {}},
+    {{6.31f, 0.402f, -0.014f, 0.292f}, {7.97f, 0.416f, 0.242f, 0.292f}, {8.27f, 0.324f, 0.473f, 0.148f}, {11.59f, 0.577f, 0.623f, 0.275f}, {},
+     {10.65f, 0.544f, 0.85f, 0.311f}}};
 constexpr Finish kFinish[3] = {{2.903f, 2.218f, 0.056f, 5.858f, -3.213f, 2.241f, 2.427f},
                                {4.686f, 1.352f, 0.859f, 18.205f, -0.462f, 3.567f, 1.958f},
                                {3.025f, 1.971f, 0.603f, 0.682f, 0.016f, 1.99f, 5.505f}};
@@ -915,9 +942,21 @@ HalfPlan gemm_half_plan(const GemmArgs& a, int epi, int num_cus) {
   auto take = [&](const HalfPlan& p, float us) {
     if (us < best_us) best = p, best_us = us;
   };
-  for (int t : {HALF_64x128, HALF_128x128, HALF_128x128_8, HALF_128x256}) {
-    if ((t == HALF_128x256 && kind != 1) || (t == HALF_128x128 && kind == 2)) continue;
-    const int bm = t == HALF_64x128 ? 64 : 128, bn = t == HALF_128x256 ? 256 : 128;
+  if (kind != 2 && (long)((a.M + 127) / 128) * ((a.N + 127) / 128) >= cus) {
+    for (int t : {HALF_64x128, HALF_128x128, HALF_128x128_8, HALF_128x256, HALF_128x256_8}) {
+      if (t >= HALF_128x256 && kind != 1) continue;
+      if (t == HALF_128x256 && (a.w_scale || a.K > 2048)) continue;
+      const int bm = t == HALF_64x128 ? 64 : 128, bn = t >= HALF_128x256 ? 256 : 128;
+      const long items = ((long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) + 7) / 8 * 8;
+      const float on_cu = (float)((items + cus - 1) / cus), round = std::max(0.0f, (float)items / (float)cus - 1.0f);
+      const TilePace& p = kFullPace[kind][t];
+      take({t, 1, 0, 0}, p.start + (float)steps * (p.stage + (on_cu - 1.0f) * p.more + round * p.part));
+    }
+    return best;
+  }
+  for (int t : {HALF_64x128, HALF_128x128, HALF_128x128_8}) {
+    if (t == HALF_128x128 && kind == 2) continue;
+    const int bm = t == HALF_64x128 ? 64 : 128, bn = 128;
     const long tiles = (long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
     for (int parts = 1; parts <= std::max(1, most); ++parts) {
       const long items = (tiles + 7) / 8 * 8 * parts;  // (as many to each XCD as the fullest one has)
