@@ -70,6 +70,16 @@ struct Products {
   static constexpr int w[6] = {0, PX == 3 ? 2 : PW - 1, PX == 3 ? 1 : 0, 0, PW > 1 ? 1 : 0, 0};
 };
 
+// Planes of W in an octet of columns, and which of them is the second part for the m-th block of input rows (k_half_rows).
+template <int PW>
+__device__ __forceinline__ int planes_of(const GemmArgs& a) {
+  return PW == 2 ? a.w_half_planes : PW;
+}
+template <int PW>
+__device__ __forceinline__ int second_plane(const GemmArgs& a, int m) {
+  return PW == 2 ? 1 + (m & (a.w_half_planes - 2)) : 1;
+}
+
 // GELU of sum + bias, four columns of a row, in half form with what f32 rounds away on the way, or in cut form.
 template <int PX>
 __device__ __forceinline__ void store_gelu(void* to, int mp, size_t m, size_t n, f4 sum, f4 bias, f4 scale) {
@@ -129,6 +139,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
   const int kt1 = SPLIT ? (int)(((long)(blockIdx.y + 1) * T_all) / gridDim.y) : T_all;
   const int T = kt1 - kt0;
 
+  const int wplanes = planes_of<PW>(a), second = second_plane<PW>(a, tm);
   unsigned aoff[IA], boff[IB];
 #pragma unroll
   for (int i = 0; i < IA; ++i) {
@@ -137,10 +148,11 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
   }
 #pragma unroll
   for (int i = 0; i < IB; ++i) {
-    const int at = (wave * IB + i) * 64, plane = at / BN, row = at % BN + lane;
+    const int at = (wave * IB + i) * 64, part = at / BN % PW, row = at % BN + lane;
+    const int plane = at / BN / PW * wplanes + (part == 1 ? second : part);
     boff[i] = ((unsigned)plane * (unsigned)a.N + (unsigned)min(n0 + row, a.N - 1)) * 16u;
   }
-  const size_t astage = (size_t)NO * PX * mp * 16, bstage = (size_t)NO * PW * a.N * 16;
+  const size_t astage = (size_t)NO * PX * mp * 16, bstage = (size_t)NO * wplanes * a.N * 16;
   const char* Ab = reinterpret_cast<const char*>(a.A) + kt0 * astage;
   const char* Wb = static_cast<const char*>(a.w_half) + kt0 * bstage;
   const unsigned as_lds = (unsigned)(size_t)(lds_ptr)(void*)&As[0][0], bs_lds = (unsigned)(size_t)(lds_ptr)(void*)&Bs[0][0];
@@ -336,15 +348,16 @@ __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
   const int steps_all = a.K / 32;
   const int steps = piece < steps_all ? (steps_all - piece + pieces - 1) / pieces : 0;
 
+  const int wplanes = planes_of<PW>(a), second = second_plane<PW>(a, (int)blockIdx.z);
   const char* wp[NG];
 #pragma unroll
   for (int g = 0; g < NG; ++g)
-    wp[g] = static_cast<const char*>(a.w_half) + ((size_t)kq * PW * a.N + min(n0 + 16 * g + i16, n1 - 1)) * 16;
+    wp[g] = static_cast<const char*>(a.w_half) + ((size_t)kq * wplanes * a.N + min(n0 + 16 * g + i16, n1 - 1)) * 16;
   const char* xp[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
     xp[mt] = reinterpret_cast<const char*>(a.A) + ((size_t)kq * PX * mp + min(m0 + 16 * mt + i16, a.M - 1)) * 16;
-  const size_t wpart = (size_t)a.N * 16, wstep = wpart * 4 * PW, xpart = (size_t)mp * 16, xstep = xpart * 4 * PX;
+  const size_t wpart = (size_t)a.N * 16, wstep = wpart * 4 * wplanes, xpart = (size_t)mp * 16, xstep = xpart * 4 * PX;
 
   // The write-out takes four columns of a row at a time, neighbouring lanes neighbouring columns, or, into a matrix
   // in half form, neighbouring rows, which lie next to each other there.  What it adds is requested first.
@@ -378,7 +391,7 @@ __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
 #pragma unroll
     for (int g = 0; g < NG; ++g)
 #pragma unroll
-      for (int p = 0; p < PW; ++p) w[g][p] = *reinterpret_cast<const u4v*>(wp[g] + col * wstep + p * wpart);
+      for (int p = 0; p < PW; ++p) w[g][p] = *reinterpret_cast<const u4v*>(wp[g] + col * wstep + (p == 1 ? second : p) * wpart);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -655,10 +668,13 @@ hipError_t launch_norm_rows(const GemmArgs& a, int parts, hipStream_t s) {
 // then a f16 number as it is down to 2^-32 of the row's largest and right to 2^-40 of that below, as a f32 weight's lo part is (of
 // normally distributed weights one in 10^9 is as small: a large model has some).  *refused is set where a value is not finite or a row
 // so small or large that its power of two, or an int8 row's scale beside it, would matter.
+// A f32 weight in four lies half-way between two values of its second part.  Over the positions of a prompt that is the same error
+// every time, and attention adds them up: behind prompts of 300 to 900 tokens the next token's logits were off by 1.02 to 1.04 times
+// as much as with W whole, though each position's were off by less.  planes 3: the other of the two values is there as well, and
+// every second block of input rows takes it.
 template <int WT>
 __global__ __launch_bounds__(256) void k_half_rows(const void* W, const float* scales, const float* powers, void* to, float* mul,
-                                                   unsigned* refused, int N, int K) {
-  constexpr int PW = WT == 0 ? 2 : 1;
+                                                   unsigned* refused, int N, int K, int planes) {
   __shared__ float biggest[4][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int n = (int)blockIdx.x * 64 + lane, row = min(n, N - 1);
@@ -707,17 +723,24 @@ __global__ __launch_bounds__(256) void k_half_rows(const void* W, const float* s
   if (wave == 0 && n < N) mul[n] = row_scale / scale;
   for (int k = 8 * wave; k < K; k += 32) {
     get(k, x);
-    u4v h, l;
+    u4v h, l, other;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       unsigned hi, lo;
       halves2(x[2 * e], x[2 * e + 1], scale, hi, lo);
       h[e] = hi, l[e] = lo;
+      if (WT == 0) {  // 2 (x - hi) - lo
+        const h2v hv = __builtin_bit_cast(h2v, hi), lv = __builtin_bit_cast(h2v, lo);
+        const float a = x[2 * e] * scale - (float)hv.x, b = x[2 * e + 1] * scale - (float)hv.y;
+        const f2 o{fmaf(2.0f, a, -(float)lv.x), fmaf(2.0f, b, -(float)lv.y)};
+        other[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(o, h2v));
+      }
     }
     if (n < N) {
-      u4v* at = static_cast<u4v*>(to) + (size_t)(k / 8) * PW * N + n;
+      u4v* at = static_cast<u4v*>(to) + (size_t)(k / 8) * planes * N + n;
       at[0] = h;
-      if (PW == 2) at[N] = l;
+      if (planes > 1) at[N] = l;
+      if (planes > 2) at[2 * (size_t)N] = other;
     }
   }
   if (bad) atomicOr(refused, 1u);
@@ -921,7 +944,7 @@ bool gemm_half_takes(const GemmArgs& a, int epi) {
                        reinterpret_cast<uintptr_t>(a.w_half_mul) | reinterpret_cast<uintptr_t>(a.bias) |
                        reinterpret_cast<uintptr_t>(a.resid) | reinterpret_cast<uintptr_t>(a.ws) | reinterpret_cast<uintptr_t>(a.ln_out) |
                        reinterpret_cast<uintptr_t>(a.ln_g) | reinterpret_cast<uintptr_t>(a.ln_b);
-  return a.w_half && (a.w_half_parts == 3 || (a.w_half_mul && (a.w_half_parts == 1 || a.w_half_parts == 2))) && !(at & 15) && a.M >= 1 && a.M < (1 << 23) &&
+  return a.w_half && (a.w_half_parts == 3 || (a.w_half_mul && (a.w_half_parts == 1 || (a.w_half_parts == 2 && (a.w_half_planes == 2 || a.w_half_planes == 3))))) && !(at & 15) && a.M >= 1 && a.M < (1 << 23) &&
          a.K >= 64 && a.K % 32 == 0 && a.N >= 64 && a.N % 8 == 0 && a.N < (1 << 24) && a.ldc % 4 == 0 && a.a_unscale > 0.0f &&
          (a.c_scale != nullptr) == (epi == GEMM_GELU && a.w_half_parts != 3) && !(reinterpret_cast<uintptr_t>(a.c_scale) & 15) &&
          (epi == GEMM_BIAS || epi == GEMM_GELU || epi == GEMM_RESID) && (epi != GEMM_GELU || a.ldc == a.N);
@@ -1022,12 +1045,12 @@ hipError_t launch_norm_rows_half(float* src, void* dst, int rows, int cols, cons
 }
 
 hipError_t launch_half_rows(const void* W, int w_bytes, const float* scales, const float* powers, size_t rows, int cols, void* to,
-                            float* mul, unsigned* refused, hipStream_t s) {
+                            float* mul, unsigned* refused, hipStream_t s, int planes) {
   const dim3 grid((unsigned)((rows + 63) / 64));
-  if (cols % 32 != 0 || rows > (1u << 24)) return hipErrorInvalidValue;
-  if (w_bytes == 4) hipLaunchKernelGGL(k_half_rows<0>, grid, dim3(256), 0, s, W, scales, powers, to, mul, refused, (int)rows, cols);
-  else if (w_bytes == 2) hipLaunchKernelGGL(k_half_rows<1>, grid, dim3(256), 0, s, W, scales, powers, to, mul, refused, (int)rows, cols);
-  else hipLaunchKernelGGL(k_half_rows<2>, grid, dim3(256), 0, s, W, scales, powers, to, mul, refused, (int)rows, cols);
+  if (cols % 32 != 0 || rows > (1u << 24) || (w_bytes == 4 ? planes != 2 && planes != 3 : planes != 1)) return hipErrorInvalidValue;
+  if (w_bytes == 4) hipLaunchKernelGGL(k_half_rows<0>, grid, dim3(256), 0, s, W, scales, powers, to, mul, refused, (int)rows, cols, planes);
+  else if (w_bytes == 2) hipLaunchKernelGGL(k_half_rows<1>, grid, dim3(256), 0, s, W, scales, powers, to, mul, refused, (int)rows, cols, planes);
+  else hipLaunchKernelGGL(k_half_rows<2>, grid, dim3(256), 0, s, W, scales, powers, to, mul, refused, (int)rows, cols, planes);
   return hipGetLastError();
 }
 hipError_t launch_cut_weights(const float* W, size_t rows, int cols, void* to, hipStream_t s) {

@@ -517,7 +517,7 @@ bool takes_half_form(const pg_model* m, size_t rows) {
 pg_status make_half_form(pg_model* m) {
   const Cfg& g = m->cfg;
   if (g.hd() != pgk::kHeadDim || g.C < 256 || g.C % 32 != 0 || g.C > (size_t)pgk::kNormWidest || g.I < 256 || g.I % 32 != 0) return PG_OK;
-  const int wb = m->w_i8 ? 1 : m->w_bf16 ? 2 : 4, pw = wb == 4 ? 2 : 1;
+  const int wb = m->w_i8 ? 1 : m->w_bf16 ? 2 : 4, pw = wb == 4 ? pgk::kHalfPlanes : 1;
   auto up = [](size_t n) { return (n + 255) / 256 * 256; };
   const size_t C = g.C, I = g.I;
   const size_t rows[4] = {3 * C, C, I, C}, cols[4] = {C, C, C, I};
@@ -566,7 +566,7 @@ pg_status make_half_form(pg_model* m) {
       to[i] = at;
       at += up(rows[i] * cols[i] * 2 * pw);
       mul[i] = floats(rows[i]);
-      PG_HIP(pgk::launch_half_rows(mats[i], wb, scales[i], powers[i], rows[i], (int)cols[i], to[i], mul[i], refused, nullptr));
+      PG_HIP(pgk::launch_half_rows(mats[i], wb, scales[i], powers[i], rows[i], (int)cols[i], to[i], mul[i], refused, nullptr, pw));
       if (!cut) continue;
       cut_to[i] = at;
       at += up(rows[i] * cols[i] * 6);
@@ -666,7 +666,7 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
     a.A = A; a.w_bf16 = m->w_bf16; a.W = W; a.bias = bias; a.resid = Cout; a.C = Cout;
     a.a_cut = a.ln_cut = a_cut; a.c_cut = c_cut;
     if (w_half) {
-      a.w_half = w_half; a.w_half_mul = w_half_mul; a.w_half_parts = m->w_bf16 || m->w_i8 ? 1 : 2;
+      a.w_half = w_half; a.w_half_mul = w_half_mul; a.w_half_parts = m->w_bf16 || m->w_i8 ? 1 : 2, a.w_half_planes = pgk::kHalfPlanes;
       a.a_unscale = 1.0f; a.c_scale = c_scale; a.ln_scale = ln_half ? 1.0f : 0.0f;  // (the powers are in W and in the norms)
       if (cut) a.w_half_parts = 3, a.a_cut = a.c_cut = 0;  // (W is in cut form)
     }
@@ -797,7 +797,7 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
     pgk::GemmArgs a{};
     a.A = A; a.w_bf16 = m->w_bf16; a.W = W; a.bias = bias; a.resid = Cout; a.C = Cout;
     if (w_half) {
-      a.w_half = w_half; a.w_half_mul = w_half_mul; a.w_half_parts = m->w_bf16 || m->w_i8 ? 1 : 2;
+      a.w_half = w_half; a.w_half_mul = w_half_mul; a.w_half_parts = m->w_bf16 || m->w_i8 ? 1 : 2, a.w_half_planes = pgk::kHalfPlanes;
       a.a_unscale = 1.0f; a.c_scale = c_scale; a.ln_scale = ln_half ? 1.0f : 0.0f;  // (the powers are in W and in the norms)
     }
     a.M = B; a.N = N; a.K = K; a.lda = lda; a.ldc = ldc;

@@ -269,7 +269,7 @@ struct GemmArgs {
   // w_half_parts 3 (f32 rows): A, C of GEMM_GELU and, with ln_cut, ln_out are in cut form, W in launch_cut_weights'; a_unscale is 1, c_scale null.
   const void* w_half = nullptr;
   const float* w_half_mul = nullptr;
-  int w_half_parts = 0;
+  int w_half_parts = 0, w_half_planes = 0;  // (planes: of f32 rows, 2 or 3)
   const float* c_scale = nullptr;
   float a_unscale = 0.0f, ln_scale = 0.0f;
   // Tunable: a GEMM whose M x N leaves CUs idle is cut along K into about this many work items
@@ -307,12 +307,13 @@ hipError_t launch_norm_rows_half(float* src, void* dst, int rows, int cols, cons
                                  const float* resid = nullptr);
 // W[rows][cols] as stored (w_bytes 4: f32, 2: bf16, 1: int8 with scales[row]) in half form, for inputs whose column k is kept times
 // powers[k] (null: as they are): two f16 numbers a weight (f32 rows) or one, cols a multiple of 32, and what a sum over them is to
-// be multiplied with, mul[rows].  *refused is set (never cleared), here and below, where the values do not allow it (k_half_rows).
+// be multiplied with, mul[rows]; planes 3 (f32 rows): a second value of the second part too.  *refused is set (never cleared), here and below, where the values do not allow it (k_half_rows).
 constexpr int kHalfMostExp = 60;
+constexpr int kHalfPlanes = 3;  // of a model's f32 rows
 // f32 rows in cut form, three bf16 numbers a weight, for inputs in cut form.
 hipError_t launch_cut_weights(const float* W, size_t rows, int cols, void* to, hipStream_t s);
 hipError_t launch_half_rows(const void* W, int w_bytes, const float* scales, const float* powers, size_t rows, int cols, void* to,
-                            float* mul, unsigned* refused, hipStream_t s);
+                            float* mul, unsigned* refused, hipStream_t s, int planes);
 // bounds[row]: the largest magnitude that an output of this row behind a LayerNorm with gains g can have; fold as launch_ln_fold
 // leaves it.  launch_half_powers: to the powers of two that put them at 2^15 at most.
 hipError_t launch_half_bound(const void* W, int w_bytes, const float* scales, const float* g, const float* fold, size_t rows, int cols,

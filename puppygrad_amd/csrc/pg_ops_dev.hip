@@ -481,12 +481,12 @@ pg_status pg_testing_half_product_dev(int32_t device, void* stream, const float*
     hipLaunchKernelGGL(k_to_cut, x_blocks, dim3(256), 0, st, x, work, (int)rows, (int)in_f);
   } else {
     PG_HIP(pgk::launch_half_rows(weight, storage == PG_STORE_F32 ? 4 : storage == PG_STORE_BF16 ? 2 : 1, scales, nullptr, out_f,
-                                 (int)in_f, w_half, mul, refused, st));
+                                 (int)in_f, w_half, mul, refused, st, pw));
     hipLaunchKernelGGL(k_to_half, x_blocks, dim3(256), 0, st, x, work, (int)rows, (int)in_f, scale);
   }
   PG_HIP(hipGetLastError());
   pgk::GemmArgs a{};
-  a.A = reinterpret_cast<const float*>(work); a.w_half = w_half; a.w_half_mul = mul; a.w_half_parts = pw; a.a_unscale = cut ? 1.0f : 1.0f / scale;
+  a.A = reinterpret_cast<const float*>(work); a.w_half = w_half; a.w_half_mul = mul; a.w_half_parts = a.w_half_planes = pw; a.a_unscale = cut ? 1.0f : 1.0f / scale;
   a.bias = bias; a.C = out; a.M = (int)rows; a.N = (int)out_f; a.K = (int)in_f; a.ldc = (int)out_f;
   a.ws = out; a.ws_floats = (size_t)parts * rows * out_f;
   Constants ones;

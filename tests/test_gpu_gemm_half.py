@@ -371,6 +371,30 @@ def test_steps_of_columns_of_unequal_size(storage, batch):
         assert np.linalg.norm(got[b] - want) <= 1e-5 * np.linalg.norm(want)
 
 
+def test_weights_of_24_bits_do_not_shift_the_keys():
+    """Two f16 numbers drop a bit of a f32 weight in four.  Norms that are mostly their shifts make that the same error at every position;
+    over the positions it is gone."""
+    cfg = Gpt2Config(vocab_size=97, n_positions=512, n_embd=1280, n_layer=1, n_head=20)
+    w = synth.random_weights(cfg, 0x5EED0B0A, perturb=True)
+    blk, rng = w.blocks[0], np.random.default_rng(10)
+    blk.ln_1_g = np.full(1280, 0.05, np.float32)
+    blk.ln_1_b = rng.uniform(0.5, 1.0, 1280).astype(np.float32)
+    ids = synth.token_ids(512, 0x70C00B0A, 97)
+    model = Gpt2Model.new(cfg, w)
+    cache = model.new_kv_cache()
+    model.prefill([int(t) for t in ids], cache)
+    got = cache.read_layer(0, 0).astype(np.float64).reshape(20, 512, 64)
+    x = (np.float32(w.wte).reshape(97, 1280)[ids] + np.float32(w.wpe).reshape(-1, 1280)[:512]).astype(np.float64)
+    d = x - x.mean(1, keepdims=True)
+    y = d / np.sqrt((d * d).mean(1, keepdims=True) + cfg.layer_norm_epsilon) * 0.05 + blk.ln_1_b.astype(np.float64)
+    at = slice(1280, 2560)
+    want = y @ np.asarray(blk.c_attn_w, np.float64).reshape(1280, 3840)[:, at] + np.asarray(blk.c_attn_b, np.float64)[at]
+    off = got.transpose(1, 0, 2).reshape(512, 1280) - want
+    # (a quarter of the weights off by 2^-23 to 2^-24 of themselves is 0.7 of 2^-24 of the keys at every position; the sums' own roundings,
+    # which are much the same at every position here, leave 0.36)
+    assert np.sqrt((off.mean(0) ** 2).mean() / (want ** 2).mean()) <= 0.5 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("storage,batch", [("f32", 8), ("bf16", 40), ("int8", 24)])
 @pytest.mark.parametrize("behind", [5, 60])  # (one share of the keys and several)
 def test_a_step_behind_another_models_values(storage, batch, behind):
