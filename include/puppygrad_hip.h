@@ -113,7 +113,14 @@ typedef struct pg_hip_options {
   uint32_t seq_gemm_min_tokens;     /* prompts of at least this many tokens take the GEMM
                                        prefill, shorter ones run token by token through the
                                        decode path (default 4; at most 65536) */
-  uint32_t reserved;                /* must be 0 */
+  union {
+    uint32_t weight_copies;         /* GPT-2: 0: the block matrices are kept a second time, in the parts that prompts and
+                                       batched steps multiply with (f32 rows 6 bytes a weight beside 4, up to a width of
+                                       768 12, bf16 2 beside 2, int8 2 beside 1), where that takes at most a quarter of
+                                       the memory that is free when the model is made; 1: never.  Stack models make
+                                       none */
+    uint32_t reserved;              /* (its name before) */
+  };
 } pg_hip_options;
 
 /* A model of any registered architecture (pg_model_create_from_dir); GPT-2 models are one of

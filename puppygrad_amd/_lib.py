@@ -45,7 +45,7 @@ class pg_hip_options(C.Structure):
                 ("decode_path", C.c_uint32), ("prefill_path", C.c_uint32),
                 ("attn_item_keys", C.c_uint32), ("attn_blocks_per_cu", C.c_uint32),
                 ("gemm_split_items_per_cu", C.c_uint32), ("gemm_b9_min_rows", C.c_uint32),
-                ("seq_gemm_min_tokens", C.c_uint32), ("reserved", C.c_uint32)]
+                ("seq_gemm_min_tokens", C.c_uint32), ("weight_copies", C.c_uint32)]
 
 
 class pg_model_info(C.Structure):

@@ -516,6 +516,7 @@ bool takes_half_form(const pg_model* m, size_t rows) {
 // The block matrices in half form.  Nothing of it is needed to serve a call: where it cannot be had the model goes without.
 pg_status make_half_form(pg_model* m) {
   const Cfg& g = m->cfg;
+  if (m->opts.weight_copies == 1 || (!m->w_bf16 && !m->w_i8 && m->gemm_b9_min_rows == 0x7fffffff)) return PG_OK;  // (no rows would take it)
   if (g.hd() != pgk::kHeadDim || g.C < 256 || g.C % 32 != 0 || g.C > (size_t)pgk::kNormWidest || g.I < 256 || g.I % 32 != 0) return PG_OK;
   const int wb = m->w_i8 ? 1 : m->w_bf16 ? 2 : 4, pw = wb == 4 ? pgk::kHalfPlanes : 1;
   auto up = [](size_t n) { return (n + 255) / 256 * 256; };
@@ -529,6 +530,10 @@ pg_status make_half_form(pg_model* m) {
   const bool cut = wb == 4 && C <= 768;
   for (int i = 0; i < 4; ++i) layer += up(rows[i] * cols[i] * 2 * pw) + up(rows[i] * 4) + (cut ? up(rows[i] * cols[i] * 6) : 0);
   layer += 9 * up(C * 4) + up(I * 4) + up(g.H * 4);  // the columns' powers; gains and shifts times them
+  // Caches and the scratch memory of prompts are allocated later, and a model that fitted without the copies has to serve its calls.
+  size_t available = 0, total = 0;
+  PG_HIP(hipMemGetInfo(&available, &total));
+  if (g.L * layer > available / 4) return PG_OK;
   if (hipMalloc(&m->half_arena, g.L * layer + up(4)) != hipSuccess) {
     (void)hipGetLastError();
     m->half_arena = nullptr;
@@ -1116,7 +1121,7 @@ pg_status pg_gpt2_create(const pg_gpt2_config* config, const pg_gpt2_weights_vie
     return fail(PG_INVALID_CONFIG, "hip backend gemm_split_items_per_cu must be at most 16");
   if (opts.seq_gemm_min_tokens > 65536)
     return fail(PG_INVALID_CONFIG, "hip backend seq_gemm_min_tokens must be at most 65536");
-  if (opts.reserved != 0) return fail(PG_INVALID_CONFIG, "hip backend options: reserved must be 0");
+  if (opts.weight_copies > 1) return fail(PG_INVALID_CONFIG, "hip backend weight_copies must be 0 or 1");
   if ((s = select_device(opts.device))) return s;
 
   auto m = std::make_unique<pg_model>();

@@ -788,7 +788,7 @@ pg_status stack_create(const std::string& config_path, const Json& config, const
     return fail(PG_INVALID_CONFIG, "hip backend weight_storage of a " + m->architecture + " model must be f32 or bf16");
   if (opts.decode_path > PG_DECODE_KERNELS)
     return fail(PG_INVALID_CONFIG, "hip backend decode_path of a " + m->architecture + " model must be auto or kernels");
-  if (opts.reserved != 0) return fail(PG_INVALID_CONFIG, "hip backend options: reserved must be 0");
+  if (opts.weight_copies > 1) return fail(PG_INVALID_CONFIG, "hip backend weight_copies must be 0 or 1");
   if ((s = select_device(opts.device))) return s;
 
   auto model = std::make_unique<pg_model>();

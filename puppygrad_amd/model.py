@@ -117,12 +117,13 @@ class Gpt2HipConfig:
     gemm_split_items_per_cu: int = 0
     gemm_b9_min_rows: int = 0
     seq_gemm_min_tokens: int = 0
+    weight_copies: int = 0  # 1: GPT-2 block matrices are not kept a second time for prompts and batched steps
 
     def to_c(self) -> _lib.pg_hip_options:
         return _lib.pg_hip_options(self.device, self.weight_storage, self.decode_path,
                                    self.prefill_path, self.attn_item_keys, self.attn_blocks_per_cu,
                                    self.gemm_split_items_per_cu, self.gemm_b9_min_rows,
-                                   self.seq_gemm_min_tokens, 0)
+                                   self.seq_gemm_min_tokens, self.weight_copies)
 
 
 @dataclass

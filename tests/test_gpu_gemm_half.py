@@ -265,6 +265,34 @@ def test_batched_steps(storage, width, batch, n):
         assert np.linalg.norm(got[b] - want) <= 1e-5 * np.linalg.norm(want)
 
 
+def test_copies_of_the_weights_can_be_declined():
+    """A model without them takes their memory less and serves the same calls; none are made where no rows could take them."""
+    import torch
+
+    cfg = Gpt2Config(vocab_size=97, n_positions=512, n_embd=1280, n_layer=2, n_head=20)
+    w = synth.random_weights(cfg, 0x5EED0B0B, perturb=True)
+    ids = [int(t) for t in synth.token_ids(300, 0x70C00B0B, 97)]
+    weights = cfg.n_layer * 12 * cfg.n_embd ** 2
+
+    def taken(**kw):
+        before = torch.cuda.mem_get_info()[0]
+        model = Gpt2Model.new(cfg, w, Gpt2HipConfig(**kw))
+        return model, before - torch.cuda.mem_get_info()[0]
+
+    logits(Gpt2Model.new(cfg, w), ids)  # (what the process allocates once)
+    for storage, bytes_each in (("f32", 6), ("bf16", 2), ("int8", 2)):
+        with_them, more = taken(weight_storage=STORE[storage])
+        without, less = taken(weight_storage=STORE[storage], weight_copies=1)
+        # (allocations in pages of 2 MB)
+        assert abs(more - less - bytes_each * weights) <= 8 << 20, (more, less)
+        got, want = logits(without, ids), logits(with_them, ids)
+        assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
+    _, never = taken(gemm_b9_min_rows=0xffffffff)
+    assert never <= 4 * (weights + 700 * cfg.n_embd) + (8 << 20)
+    with pytest.raises(Exception, match="weight_copies must be 0 or 1"):
+        Gpt2Model.new(cfg, w, Gpt2HipConfig(weight_copies=2))
+
+
 def test_a_set_bound_holds_for_few_rows():
     cfg = Gpt2Config(vocab_size=97, n_positions=64, n_embd=768, n_layer=1, n_head=12)
     w = synth.random_weights(cfg, 0x5EED0B04, perturb=True)
