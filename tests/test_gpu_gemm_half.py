@@ -267,17 +267,20 @@ def test_batched_steps(storage, width, batch, n):
 
 def test_copies_of_the_weights_can_be_declined():
     """A model without them takes their memory less and serves the same calls; none are made where no rows could take them."""
-    import torch
-
     cfg = Gpt2Config(vocab_size=97, n_positions=512, n_embd=1280, n_layer=2, n_head=20)
     w = synth.random_weights(cfg, 0x5EED0B0B, perturb=True)
     ids = [int(t) for t in synth.token_ids(300, 0x70C00B0B, 97)]
     weights = cfg.n_layer * 12 * cfg.n_embd ** 2
 
+    def free():
+        at = (C.c_size_t * 2)()
+        assert _lib.load().hipMemGetInfo(C.byref(at, 0), C.byref(at, C.sizeof(C.c_size_t))) == 0
+        return at[0]
+
     def taken(**kw):
-        before = torch.cuda.mem_get_info()[0]
+        before = free()
         model = Gpt2Model.new(cfg, w, Gpt2HipConfig(**kw))
-        return model, before - torch.cuda.mem_get_info()[0]
+        return model, before - free()
 
     logits(Gpt2Model.new(cfg, w), ids)  # (what the process allocates once)
     for storage, bytes_each in (("f32", 6), ("bf16", 2), ("int8", 2)):
