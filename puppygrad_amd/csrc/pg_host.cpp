@@ -788,11 +788,17 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
   // that the 32-row kernel reads with contiguous loads; their producers write them that way.
   // c->cut_form: there is room for them in cut form, which this model's rows take (the cache may have been made for
   // another model of these sizes); not the logits' input.
-  // Half form, which every cache has room for, goes before both (takes_half_form), but for up to 32 sequences and bf16 rows, whose
-  // packed rows are a little faster (XL, eight steps behind 300 tokens, ms, packed / half form: 17 sequences (100) 20.9 / 21.3, 24 27.9 /
-  // 28.2, 32 30.9 / 31.3; int8 rows, unpacked, of 32 28.8 / 27.3).
+  // Half form, which every cache has room for, goes before both (takes_half_form), but where packed rows are the faster ones (eight
+  // steps, ms, packed / half form):
+  //  - bf16 rows, up to 32 sequences: XL behind 300 tokens, 17 sequences (100) 20.9 / 21.3, 24 27.9 / 28.2, 32 30.9 / 31.3 (int8 rows,
+  //    unpacked, of 32 28.8 / 27.3);
+  //  - f32 rows, up to 16 sequences: one step behind 120 tokens, width 768, 5 0.457 / 0.49, 1024, 16 0.96 / 0.98, 1280, 2 1.647 / 1.656, 5
+  //    1.677 / 1.669, 9 1.737 / 1.764, 16 1.743 / 1.738, 1600, 2 2.540 / 2.565, 9 2.662 / 2.721, 14 2.552 / 2.581, 16 2.689 / 2.678.  From 17 on
+  //    the f32 cores take a second block of rows: eight steps, 17 sequences, 768 3.84 / 3.65, 1024 7.63 / 6.97, 1280 13.5 / 12.7, 1600
+  //    20.7 / 19.5, of 32 3.74 / 3.58, 8.00 / 7.56, 14.5 / 14.0, 22.1 / 21.3.
   // Not where the cache holds another model's values: this model's bounds on its own (make_half_form) say nothing of their averages.
-  const bool half = takes_half_form(m, c->B) && !(m->w_bf16 && c->pack32) && c->values_of == m->serial;
+  const bool packed = c->pack32 && (m->w_bf16 || (!m->w_i8 && c->B <= 16));
+  const bool half = takes_half_form(m, c->B) && !packed && c->values_of == m->serial;
   const int pk = c->pack32 && !half ? 1 : 0, cut = !half && c->cut_form && takes_cut_form(m, c->B) ? 1 : 0;
   const int form = half ? pgk::FORM_HALF : cut ? pgk::FORM_CUT : pk ? pgk::FORM_PACKED32 : pgk::FORM_ROWS;
   auto gemm = [&](const float* A, int lda, const float* W, const float* bias, float* Cout,

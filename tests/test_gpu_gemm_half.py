@@ -245,8 +245,10 @@ def test_prompts(storage, width, batch, n):
         assert np.linalg.norm(got[b] - want) <= 1e-5 * np.linalg.norm(want)
 
 
-# steps whose rows take the form: the smallest, one more than a block's rows, K cut and not, several blocks of rows
-@pytest.mark.parametrize("storage,width,batch", [("f32", 768, 2), ("f32", 1600, 17), ("bf16", 1024, 17), ("int8", 1280, 33), ("bf16", 768, 70), ("int8", 512, 130)])
+# steps whose rows take the form: the smallest, one more than a block's rows, K cut and not, several blocks of rows; and on the other
+# side of the line (f32 up to 16 sequences, bf16 up to 32: packed rows)
+@pytest.mark.parametrize("storage,width,batch", [("f32", 768, 17), ("f32", 1600, 17), ("bf16", 1024, 33), ("int8", 768, 17), ("int8", 1280, 33), ("bf16", 768, 70),
+                                                 ("int8", 512, 130), ("f32", 768, 2), ("f32", 1600, 16), ("bf16", 1024, 32)])
 @pytest.mark.parametrize("n", [3, 40, 300])
 def test_batched_steps(storage, width, batch, n):
     cfg = Gpt2Config(vocab_size=300, n_positions=310, n_embd=width, n_layer=2, n_head=width // 64)
