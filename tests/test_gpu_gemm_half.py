@@ -463,10 +463,35 @@ def test_rows_whose_squares_are_past_f32(n):
     assert np.isfinite(want).all() and np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
 
 
-def test_weights_without_half_form_are_served_as_before():
+@pytest.mark.parametrize("storage", STORE)
+@pytest.mark.parametrize("how", ["small row", "large row", "infinite bound"])
+def test_weights_without_half_form_are_served_as_before(storage, how):
+    """A row that cannot be scaled, of a hidden unit whose share is kept; a bound that is not finite, of one that no token reaches."""
     cfg = Gpt2Config(vocab_size=97, n_positions=400, n_embd=512, n_layer=1, n_head=8)
     ids = [int(t) for t in synth.token_ids(400, 0x70C00B03, 97)]
     w = synth.random_weights(cfg, 0x5EED0B03, perturb=True)
-    w.blocks[0].c_fc_b[3] = np.inf
-    got = logits(Gpt2Model.new(cfg, w, Gpt2HipConfig(weight_storage=STORE["bf16"])), ids)
-    assert got.shape == (97,)
+    blk = w.blocks[0]
+    if how == "infinite bound":
+        blk.c_fc_b[3] = -np.inf
+    else:
+        by = np.float32(2.0 ** -80 if how == "small row" else 2.0 ** 80)
+        blk.c_fc_w = np.array(blk.c_fc_w, np.float32).reshape(512, 2048)
+        blk.c_fc_w[:, 3] *= by
+        blk.c_fc_w = blk.c_fc_w.reshape(-1)
+        blk.c_proj_mlp_w = np.array(blk.c_proj_mlp_w, np.float32).reshape(2048, 512)
+        blk.c_proj_mlp_w[3] *= 1.0 / by if how == "large row" else 1.0
+        blk.c_proj_mlp_w = blk.c_proj_mlp_w.reshape(-1)
+    refused, without = (Gpt2Model.new(cfg, w, Gpt2HipConfig(weight_storage=STORE[storage], weight_copies=c)) for c in (0, 1))
+    for n in (20, 50, 100, 400):
+        got = logits(refused, ids[:n])
+        np.testing.assert_array_equal(got, logits(without, ids[:n]))
+        single = without.new_kv_cache()
+        without.prefill(ids[:3], single)
+        for t in ids[3:n - 1]:
+            without.forward_one(t, single)
+        want = without.forward_one(ids[n - 1], single).to_host()
+        if np.isfinite(want).all():
+            # (the same values, sums of at most 2048 terms in other orders)
+            assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
+        else:
+            assert how == "infinite bound" and not np.isfinite(got).any()

@@ -140,11 +140,12 @@ def test_infinite_weights_and_weights_past_bf16():
                                              ("int8", 1280, 300), ("f32", 768, 455), ("f32", 768, 456), ("f32", 768, 1024), ("f32", 768, 1025),
                                              ("f32", 1280, 256), ("f32", 1600, 192), ("bf16", 768, 512), ("bf16", 768, 513), ("bf16", 1600, 192),
                                              ("int8", 768, 1024), ("int8", 768, 1025), ("int8", 1600, 448)])
-def test_prompts(storage, width, n):
+@pytest.mark.parametrize("copies", [False, True])  # (with the weights kept a second time most of these rows are kept in other forms)
+def test_prompts(storage, width, n, copies):
     cfg = Gpt2Config(vocab_size=300, n_positions=1100 if n > 512 else 512, n_embd=width, n_layer=2, n_head=width // 64)
     store = {"f32": _lib.PG_STORE_F32, "bf16": _lib.PG_STORE_BF16, "int8": _lib.PG_STORE_INT8}[storage]
     assert takes(n, width, store) == (n <= LAST[store][width])
-    model = Gpt2Model.new(cfg, synth.random_weights(cfg, 0x5EED0A00, perturb=True), Gpt2HipConfig(weight_storage=store))
+    model = Gpt2Model.new(cfg, synth.random_weights(cfg, 0x5EED0A00, perturb=True), Gpt2HipConfig(weight_storage=store, weight_copies=0 if copies else 1))
     ids = [int(t) for t in synth.token_ids(n, 0x70C00A00 + n, cfg.vocab_size)]
     cache, other = model.new_kv_cache(), model.new_kv_cache()
     got = model.prefill(ids, cache).to_host()
@@ -181,10 +182,11 @@ def test_a_set_bound_of_the_bf16_cores_holds_for_the_cut_form():
 
 @pytest.mark.parametrize("storage,batch,n", [("f32", 33, 3), ("f32", 48, 20), ("bf16", 40, 7), ("int8", 17, 5), ("int8", 31, 9), ("int8", 65, 4),
                                              ("f32", 128, 3), ("f32", 129, 3), ("f32", 130, 2)])
-def test_batched_steps(storage, batch, n):
+@pytest.mark.parametrize("copies", [False, True])
+def test_batched_steps(storage, batch, n, copies):
     cfg = Gpt2Config(vocab_size=300, n_positions=600, n_embd=768, n_layer=2, n_head=12)
     store = {"f32": _lib.PG_STORE_F32, "bf16": _lib.PG_STORE_BF16, "int8": _lib.PG_STORE_INT8}[storage]
-    model = Gpt2Model.new(cfg, synth.random_weights(cfg, 0x5EED0A01, perturb=True), Gpt2HipConfig(weight_storage=store))
+    model = Gpt2Model.new(cfg, synth.random_weights(cfg, 0x5EED0A01, perturb=True), Gpt2HipConfig(weight_storage=store, weight_copies=0 if copies else 1))
     ids = synth.token_ids(batch * (n + 2), 0x70C00A01 + n, cfg.vocab_size).reshape(batch, n + 2)
     cache = model.new_kv_cache(batch)
     model.prefill_batch(np.ascontiguousarray(ids[:, :n]), cache)
