@@ -140,6 +140,41 @@ pg_status validate_input(const Cfg& c, const uint32_t* ids, size_t n) {
   return PG_OK;
 }
 
+// n_inner and vocab_size are no sizes of a cache (check_compatible), so its working memory has to follow the model's: a model of a
+// wider MLP or of more logits than the maker's wrote past it.
+size_t activation_floats(const pg_kv_cache* c, size_t cols) {
+  return c->cut_form ? std::max(c->act_rows * cols, pgk::cut_floats(c->B, cols)) : c->act_rows * cols;
+}
+pg_status make_room(const pg_model* m, pg_kv_cache* c) {
+  if (c->cfg.V == m->cfg.V && c->inner_room >= m->cfg.I) return PG_OK;
+  pg_status s;
+  if ((s = select_device(c->device))) return s;
+  PG_HIP(hipStreamSynchronize(c->stream));
+  auto grow = [](float** p, size_t floats) -> pg_status {
+    float* more = nullptr;
+    PG_HIP(hipMalloc(&more, floats * sizeof(float)));
+    (void)hipFree(*p);
+    *p = more;
+    return PG_OK;
+  };
+  if (c->inner_room < m->cfg.I) {
+    if ((s = grow(&c->hbuf, activation_floats(c, m->cfg.I)))) return s;
+    c->inner_room = m->cfg.I;
+  }
+  if (c->cfg.V != m->cfg.V) {
+    c->logits_valid = c->next_valid = false;  // (logits of another vocabulary)
+    if (c->want_buf) (void)hipFree(c->want_buf);
+    c->want_buf = nullptr;
+    c->want_cap = 0;
+    if (c->logits_room < m->cfg.V) {
+      if ((s = grow(&c->logits_buf, c->B * m->cfg.V))) return s;
+      c->logits_room = m->cfg.V;
+    }
+    c->cfg.V = m->cfg.V;
+  }
+  return PG_OK;
+}
+
 // Gpt2KvCache::check_compatible (src/models/gpt2/rust.rs:206-234), for a call in which the model writes to the cache.
 pg_status check_compatible(const pg_model* m, pg_kv_cache* c) {
   if (m->stack || c->stack) {  // the layers of a stack model differ in kind and size
@@ -161,6 +196,8 @@ pg_status check_compatible(const pg_model* m, pg_kv_cache* c) {
   if (c->device != m->device)
     return fail(PG_INVALID_INPUT, "cache lives on device " + std::to_string(c->device) +
                                       " but the model is on device " + std::to_string(m->device));
+  pg_status s;
+  if ((s = make_room(m, c))) return s;
   c->values_of = c->values_of == 0 || c->values_of == m->serial ? m->serial : pg_kv_cache::kSeveral;
   return PG_OK;
 }
@@ -1408,11 +1445,10 @@ pg_status pg_kv_cache_create(const pg_model* m, uint32_t batch, pg_kv_cache** ou
   raw->pack32 = !raw->cut_form && B > 1 && B <= 32 && g.C % 16 == 0 && g.I % 16 == 0 && !m->w_i8 &&
                 pgk::gemm_takes_rows32((int)B, (int)g.C, (int)g.C, m->w_bf16) &&
                 pgk::gemm_takes_rows32((int)B, (int)g.I, (int)g.I, m->w_bf16);
-  const size_t act_rows = raw->pack32 ? 32 : B > 1 ? round_up(B, 16) : B;  // (half form: rows in sixteens)
-  auto act_floats = [&](size_t cols) {
-    return raw->cut_form ? std::max(act_rows * cols, pgk::cut_floats(B, cols)) : act_rows * cols;
-  };
-  PG_HIP(hipMalloc(&raw->hbuf, act_floats(g.I) * sizeof(float)));
+  raw->act_rows = raw->pack32 ? 32 : B > 1 ? round_up(B, 16) : B;  // (half form: rows in sixteens)
+  raw->inner_room = g.I;
+  raw->logits_room = g.V;
+  PG_HIP(hipMalloc(&raw->hbuf, activation_floats(raw, g.I) * sizeof(float)));
   if (B > 1) {
     raw->gemm_ws_floats = 8 * B * std::max<size_t>(3 * g.C, g.I);
     PG_HIP(hipMalloc(&raw->gemm_ws, raw->gemm_ws_floats * sizeof(float)));
@@ -1422,18 +1458,17 @@ pg_status pg_kv_cache_create(const pg_model* m, uint32_t batch, pg_kv_cache** ou
   PG_HIP(hipMalloc(&raw->part_l, parts * sizeof(float)));
   PG_HIP(hipMalloc(&raw->logits_buf, B * g.V * sizeof(float)));
   PG_HIP(hipMalloc(&raw->qkv_b, B * 3 * g.C * sizeof(float)));
-  PG_HIP(hipMalloc(&raw->xn_b, act_floats(g.C) * sizeof(float)));
-  PG_HIP(hipMalloc(&raw->att_b, act_floats(g.C) * sizeof(float)));
+  PG_HIP(hipMalloc(&raw->xn_b, activation_floats(raw, g.C) * sizeof(float)));
+  PG_HIP(hipMalloc(&raw->att_b, activation_floats(raw, g.C) * sizeof(float)));
   PG_HIP(hipMalloc(&raw->d_tok, B * sizeof(uint32_t)));
   PG_HIP(hipMalloc(&raw->d_out_ids, g.P * B * sizeof(uint32_t)));
   PG_HIP(hipHostMalloc(&raw->h_ids, g.P * B * sizeof(uint32_t), hipHostMallocDefault));
   raw->ids_cap = g.P * B;
   if (m->persistent && batch == 1) {
     // (every vector starts on a 64-byte line: the scalar probes read whole lines; n_embd is a
-    // multiple of 64 here)
+    // multiple of 64 here; room for the splits of the smallest items, which another model may be set to)
     const size_t n_best = 2 * (size_t)m->persistent_grid;
-    const size_t set_words =
-        pgk::persistent_exchange_set_words((int)g.C, g.H * (size_t)m->attn_splits * 66);
+    const size_t set_words = pgk::persistent_exchange_set_words((int)g.C, g.H * std::max<size_t>(m->attn_splits, (g.P + 127) / 128) * 66);
     const size_t x_words = 2 * set_words;
     PG_HIP(exchange_acquire(raw->device, n_best * sizeof(unsigned long long) + x_words * sizeof(unsigned),
                             reinterpret_cast<void**>(&raw->best_t), &raw->tagged_bytes));

@@ -175,6 +175,8 @@ struct pg_kv_cache {
   // apart, and logits moved by their last bits (another kernel's order of additions: 5 10^-7) changed two in five streams
   // of 80 ids from some id on.  Decode steps have one kernel either way.
   bool drawn = false;
+  size_t act_rows = 1;    // rows that xn_b, att_b and hbuf have room for
+  size_t logits_room = 0, inner_room = 0;  // vocabulary and inner width that logits_buf and hbuf have room for
   bool cut_form = false;  // batched step: xn_b, att_b and hbuf have room for the cut form (pgk::FORM_CUT)
   bool pack32 = false;  // batched step: xn_b, att_b and hbuf are packed (pgk::packed32_index)
   // device-side candidate selection for sampling, allocated at first use: kept candidates

@@ -247,3 +247,25 @@ def test_models_wider_than_the_norms_that_keep_a_row_in_registers(storage, rows)
         model.prefill([int(ids[b])], single)
         want = model.forward_one(int(ids[rows]), single).to_host()
         assert np.linalg.norm(step[b] - want) <= 1e-5 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("batch", [1, 3, 40])
+@pytest.mark.parametrize("width,inner,vocab", [(768, 3072, 1031), (256, 1024, 300), (768, 256, 97)])
+def test_a_cache_follows_the_sizes_of_the_model_that_uses_it(batch, width, inner, vocab):
+    """n_inner and vocab_size are no sizes of a cache: one made by a model of others, smaller or larger, serves as the model's own does."""
+    sizes = dict(n_positions=300, n_embd=width, n_layer=2, n_head=width // 64)
+    cfg, other = Gpt2Config(vocab_size=vocab, n_inner=inner, **sizes), Gpt2Config(vocab_size=260, n_inner=512, **sizes)
+    model = Gpt2Model.new(cfg, synth.random_weights(cfg, 0x5EED0A05, perturb=True))
+    maker = Gpt2Model.new(other, synth.random_weights(other, 0x5EED0A06, perturb=True), Gpt2HipConfig(attn_item_keys=256))
+    ids = synth.token_ids(batch * 10, 0x70C00A05, 90).reshape(batch, 10)
+    got = []
+    for cache in (model.new_kv_cache(batch), maker.new_kv_cache(batch)):
+        if got:
+            maker.prefill_batch(np.ascontiguousarray(ids), cache)
+        steps = [model.prefill_batch(np.ascontiguousarray(ids[:, :9]), cache).to_host(), model.forward_one_batch(ids[:, 9], cache).to_host()]
+        steps.append(model.decode_greedy_batch(cache, 5)[0])
+        got.append(steps)
+    for a, b in zip(*got):
+        assert a.shape == b.shape
+        # (steps in other forms: sums of at most 3072 terms in other orders)
+        assert np.linalg.norm(a.astype(np.float64) - b) <= 1e-5 * np.linalg.norm(a)
