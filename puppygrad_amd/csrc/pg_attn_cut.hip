@@ -1,14 +1,10 @@
 // Causal attention of prompts on the bf16 matrix cores, for models without half form (pg_attn_half.hip has the others').
 #include "pg_gemm_dev.h"
+#include "pg_wave.h"
 
 namespace pgk {
 namespace {
 
-// The value the lane 32 away holds.
-__device__ __forceinline__ float other_half(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return (threadIdx.x & 32) ? __uint_as_float(r[0]) : __uint_as_float(r[1]);
-}
 __device__ __forceinline__ f16v mfma16(const u4v& a, const u4v& b, const f16v& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }

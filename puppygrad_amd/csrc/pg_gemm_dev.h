@@ -52,6 +52,38 @@ hipError_t launch_splitk_reduce(const GemmArgs& a, int epi, int parts, hipStream
 namespace {
 
 typedef float f16v __attribute__((ext_vector_type(16)));
+
+typedef __attribute__((address_space(3))) char* lds_ptr;
+
+// 16 bytes per lane from base + byte_off (per lane) to lds + 16 lane (LDS address, wavefront-uniform).
+// Inline assembly, so that the compiler's count of loads in flight does not know it: it would wait for all
+// of them at every LDS read.  vm_wait is the wait that belongs to it; a wait that the compiler places for a
+// load of its own is at worst too long (loads return in order).
+__device__ __forceinline__ void lds_dma16(const void* base, unsigned byte_off, unsigned lds) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, %2"
+      :
+      : "s"(lds), "v"(byte_off), "s"(base)
+      : "memory", "m0");
+}
+// The same from an address per lane.
+__device__ __forceinline__ void lds_dma16_at(const void* from, unsigned lds) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off"
+      :
+      : "s"(lds), "v"(from)
+      : "memory", "m0");
+}
+// At most N loads of the wavefront in flight.
+template <int N>
+__device__ __forceinline__ void vm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
 typedef unsigned u4v __attribute__((ext_vector_type(4)));
 // Eight columns of a row as three MFMA operands.
 struct Cut {

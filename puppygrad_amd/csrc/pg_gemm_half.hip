@@ -43,25 +43,6 @@ namespace pgk {
 
 namespace {
 
-typedef __attribute__((address_space(3))) char* lds_ptr;
-
-// 16 bytes per lane from base + byte_off (per lane) to lds + 16 lane (LDS address, wavefront-uniform); vm_wait is the
-// wait that belongs to it (inline assembly, which the compiler's own count of loads does not know).
-__device__ __forceinline__ void lds_dma16(const void* base, unsigned byte_off, unsigned lds) {
-  asm volatile(
-      "s_mov_b32 m0, %0\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %2"
-      :
-      : "s"(lds), "v"(byte_off), "s"(base)
-      : "memory", "m0");
-}
-// At most N loads of the wavefront in flight.
-template <int N>
-__device__ __forceinline__ void vm_wait() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 // The products of parts (input, weight) that stand for one in f32, small ones first: half form with one or two parts a weight, cut form.
 template <int PX, int PW>
 struct Products {

@@ -962,14 +962,6 @@ __global__ __launch_bounds__(256) void k_tail_reduce(GemmArgs a) {
 // Grid: x = head, y = block of queries, longest rows first (blocks are handed out x
 // fastest: every head's long blocks start before any short one).
 // ---------------------------------------------------------------------------
-// The value the lane 32 away holds (v_permlane32_swap: one VALU instruction, no LDS trip).
-__device__ __forceinline__ float other_half(float x) {
-  typedef unsigned u2x __attribute__((ext_vector_type(2)));
-  const u2x r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  // r.x holds lanes 0..31 of x in both halves, r.y lanes 32..63
-  return (threadIdx.x & 32) ? __uint_as_float(r.x) : __uint_as_float(r.y);
-}
-
 // NWV: wavefronts per block.  CUT: out is in cut form.
 template <int NWV, bool CUT>
 __global__ __launch_bounds__(64 * NWV) void k_attn_prefill64(const float* __restrict__ qkv, int T,

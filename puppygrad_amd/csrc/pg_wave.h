@@ -103,5 +103,13 @@ __device__ __forceinline__ void wave_best(float& v, unsigned& i, Take take) {
   }
 }
 
+// The value the lane 32 away holds (v_permlane32_swap: one VALU instruction, no LDS trip).
+__device__ __forceinline__ float other_half(float x) {
+  typedef unsigned u2x __attribute__((ext_vector_type(2)));
+  const u2x r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  // r.x holds lanes 0..31 of x in both halves, r.y lanes 32..63
+  return (threadIdx.x & 32) ? __uint_as_float(r.x) : __uint_as_float(r.y);
+}
+
 }  // namespace
 }  // namespace pgk
