@@ -47,7 +47,7 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const flo
   constexpr int LDS = KG * TILE > NW * MERGE ? KG * TILE : NW * MERGE;
   __shared__ __attribute__((aligned(16))) char lds[LDS];
   __shared__ float Ms[NW][32], Ls[NW][32];
-  __shared__ __attribute__((aligned(16))) float Ks[2][64];  // K's and V's powers: read for every tile, there are no registers for them
+  __shared__ __attribute__((aligned(16))) float Ks[2][QG == 1 ? 64 : 1];  // K's and V's powers where there are no registers for them
   qkv += (size_t)blockIdx.z * T * 3 * C;
   kcache += (size_t)blockIdx.z * kv_stride;
   vcache += (size_t)blockIdx.z * kv_stride;
@@ -64,22 +64,29 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const flo
   const float* kbase = qkv + C + h * 64;
   const float* vbase = qkv + 2 * C + h * 64;
   const float* sq = scales.q + h * 64;
-  const float kC = 0.125f * 1.44269504088896341f / scales.score[h];  // (a power of two)
+  // (a power of two; uniform, and no register to spare)
+  const float kC = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(0.125f * 1.44269504088896341f / scales.score[h])));
   constexpr float kLag = 8.0f;  // a weight is at most 2^15, half form's most
   char* kt = lds + kg * TILE;
   char* vt = kt + 2 * KPART;
 
-  // Q^T operands: step s holds dims 16 s + 8 half .. + 7 of query l32
-  u4v qp[4][2];
-  {
-    const float* q = qbase + (size_t)min(qi, T - 1) * C3 + 8 * half;
+  // Everything the first tile needs is requested before any of it is waited for.  Q^T operands: step s holds dims 16 s + 8 half .. + 7
+  // of query l32.
+  f4 q_raw[8], q_pow[8];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const f4* p = reinterpret_cast<const f4*>(sq + 8 * half + 16 * s);
-      halves8(*reinterpret_cast<const f4*>(q + 16 * s) * p[0], *reinterpret_cast<const f4*>(q + 16 * s + 4) * p[1], qp[s]);
-    }
+  for (int s = 0; s < 8; ++s) {
+    const int at = 8 * half + 16 * (s >> 1) + 4 * (s & 1);
+    q_raw[s] = *reinterpret_cast<const f4*>(qbase + (size_t)min(qi, T - 1) * C3 + at);
+    q_pow[s] = *reinterpret_cast<const f4*>(sq + at);
   }
-  Ks[0][lane] = scales.k[h * 64 + lane], Ks[1][lane] = scales.v[h * 64 + lane];  // (every wavefront the same)
+  f4 sk0, sk1;
+  float sv = scales.v[h * 64 + lane];
+  if constexpr (QG == 1) {
+    sk0.x = scales.k[h * 64 + lane];
+  } else {
+    const f4* k = reinterpret_cast<const f4*>(scales.k + h * 64 + 8 * (lane & 7));
+    sk0 = k[0], sk1 = k[1];
+  }
   f16v o0, o1;  // O^T rows 0..31 and 32..63
 #pragma unroll
   for (int v = 0; v < 16; ++v) o0[v] = o1[v] = 0.0f;
@@ -115,14 +122,20 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const flo
     else __syncthreads();
   };
   if (kg <= last) fetch(kg);
+  u4v qp[4][2];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) halves8(q_raw[2 * s] * q_pow[2 * s], q_raw[2 * s + 1] * q_pow[2 * s + 1], qp[s]);
+  if constexpr (QG == 1) Ks[0][lane] = sk0.x, Ks[1][lane] = sv;  // (every wavefront the same)
   for (int turn = 0; turn < turns; ++turn) {
     const int tile = kg + KG * turn;
     meet();  // the last tile has been read
     if (tile <= last) {
       const bool append = tile >= qb * QG;  // the block's own positions go to the cache
-      asm volatile("" ::: "memory");        // (Ks is read here)
-      const f4 sk0 = *reinterpret_cast<const f4*>(Ks[0] + 8 * (lane & 7)), sk1 = *reinterpret_cast<const f4*>(Ks[0] + 8 * (lane & 7) + 4);
-      const float sv = Ks[1][lane];
+      if constexpr (QG == 1) {
+        asm volatile("" ::: "memory");  // (not before the loop)
+        sk0 = *reinterpret_cast<const f4*>(Ks[0] + 8 * (lane & 7)), sk1 = *reinterpret_cast<const f4*>(Ks[0] + 8 * (lane & 7) + 4);
+        sv = Ks[1][lane];
+      }
 #pragma unroll
       for (int i = 0; i < KI; ++i) {
         const int id = lane + 64 * (qg * KI + i), key = id >> 3, o = id & 7;
@@ -265,7 +278,10 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const flo
     }
     // (times V's powers, as the values were)
     if constexpr (FORM == FORM_HALF) store_half4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r, rest, f4{1.f, 1.f, 1.f, 1.f});
-    else store_cut4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r / *reinterpret_cast<const f4*>(scales.v + h * 64 + d));
+    else {
+      const u4v p = *reinterpret_cast<const u4v*>(scales.v + h * 64 + d);  // (one over a power of two)
+      store_cut4(out, cut_rows((int)gridDim.z * T), row, (size_t)h * 64 + d, r * __builtin_bit_cast(f4, (254u << 23) - p));
+    }
   }
 }
 
