@@ -539,8 +539,9 @@ bool takes_cut_form(const pg_model* m, size_t rows) {
 //  - bf16 and int8 rows: from 17 input rows on.  Prompts of the large model, ms, 20 rows 1.69 / 1.56 (bf16), 1.64 / 1.45 (int8), 64 rows
 //    2.17 / 1.94, 300 rows 4.33 / 3.50; eight steps of 32 sequences, XL int8 28.8 / 27.3, of 40 (bf16) 32.3 / 29.1.
 //    Fewer rows are bound by their launches and W's bytes: eight steps of 8, XL bf16, 20.0 / 20.7.
-//  - f32 rows: up to 32 (prompts of 9 rows, XL, 2.54 / 2.47, 32 rows 3.18 / 2.81; the f32 cores' sums are the less precise ones, logits
-//    1.3 to 1.5 times as far off), and past the rows of the cut form (takes_cut_form), whose three parts are the more precise ones there
+//  - f32 rows: up to 32 (prompts, XL, 9 rows 2.50 / 2.53, 20 2.90 / 2.70, 32 3.13 / 2.83; medium, 6 0.97 / 0.93, 20 1.12 / 1.00; small, 9 0.45 /
+//    0.46, 20 0.51 / 0.48; the f32 cores' sums are the less precise ones, logits 1.3 to 1.5 times as far off; steps:
+//    enqueue_forward_batch), and past the rows of the cut form (takes_cut_form), whose three parts are the more precise ones there
 //    (33 to 1024 rows, this form 1.01 to 1.15 times as far off): two f16 numbers drop a bit of a f32 weight in four.  A set bound
 //    (gemm_b9_min_rows) holds here too, and 65 to 128 rows stay on the f32 cores as they do there.
 bool takes_half_form(const pg_model* m, size_t rows) {
