@@ -97,6 +97,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
   static_assert(NO * PX * BM % (64 * NW) == 0 && NO * PW * BN % (64 * NW) == 0 && BM % 64 == 0 && BN % 64 == 0);
   __shared__ u4v As[NA][NO * PX * BM];
   __shared__ u4v Bs[NA][NO * PW * BN];
+  __shared__ f4 Es[3][64];  // of the tile's columns: factors of the sums, bias, GELU's powers
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -170,15 +171,14 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
   };
   using P = Products<PX, PW>;
   constexpr int NP = P::n;
-  unsigned turned = 0;  // sign bits of two f16 numbers
-  auto step = [&](auto first, Ops& cur, Ops& nxt, int buf, int s) __attribute__((always_inline)) {
+  auto step = [&](auto turned, auto first, Ops& cur, Ops& nxt, int buf, int s) __attribute__((always_inline)) {
     constexpr bool fresh = CH != 0 && decltype(first)::value;
     read(buf, s, nxt);
-    if constexpr (TURN) {
+    if constexpr (decltype(turned)::value) {  // (the sign bits of two f16 numbers)
 #pragma unroll
       for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int p = 0; p < PW; ++p) cur.w[j][p] ^= turned;
+        for (int p = 0; p < PW; ++p) cur.w[j][p] ^= 0x80008000u;
     }
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
@@ -211,17 +211,24 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
 
   if (T > 0) {
     Ops pa, pb;
+    // What the write-out needs of the columns is asked for first of all: by then it is there, and takes no registers.
+    if (wave == 0) {
+      const unsigned off = (unsigned)min(n0 + 4 * lane, a.N - 4) * 4u, es = (unsigned)(size_t)(lds_ptr)(void*)&Es[0][0];
+      if constexpr (PX == 2) lds_dma16(a.w_half_mul, off, es);
+      if (!SPLIT && a.bias) lds_dma16(a.bias, off, es + 1024);
+      if constexpr (EPI == GEMM_GELU && PX == 2) lds_dma16(a.c_scale, off, es + 2048);
+    }
 #pragma unroll
     for (int t = 0; t < NA; ++t) dma(t, t);
     vm_wait<(NA - 1) * (IA + IB)>();
     asm volatile("s_barrier" ::: "memory");
     read(0, 0, pa);
-    auto stage = [&](auto u, int t, Ops& p0, Ops& p1) __attribute__((always_inline)) {
+    auto stage = [&](auto turned, auto u, int t, Ops& p0, Ops& p1) __attribute__((always_inline)) {
       constexpr int U = decltype(u)::value, ab = U % NA, nb = (U + 1) % NA;
       const std::integral_constant<bool, U == 0> head;
       const std::false_type rest;
       if constexpr (NS == 2) {
-        step(head, p0, p1, ab, 1);
+        step(turned, head, p0, p1, ab, 1);
         interleave();
       }
       vm_wait<(NA - 2) * (IA + IB)>();
@@ -231,19 +238,19 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
       dma(t + NA, ab);
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (NS == 2) {
-        step(rest, p1, p0, nb, 0);
+        step(turned, rest, p1, p0, nb, 0);
         interleave();
       } else {
-        step(head, p0, p1, nb, 0);
+        step(turned, head, p0, p1, nb, 0);
         interleave();
       }
     };
-    for (int t = 0; t < T; t += UN) {
+    auto chain = [&](auto turned, int t) __attribute__((always_inline)) {
       auto at = [&](auto u) __attribute__((always_inline)) {
         constexpr int U = decltype(u)::value;
         if (t + U < T) {
-          if constexpr (NS == 2 || U % 2 == 0) stage(u, t + U, pa, pb);
-          else stage(u, t + U, pb, pa);
+          if constexpr (NS == 2 || U % 2 == 0) stage(turned, u, t + U, pa, pb);
+          else stage(turned, u, t + U, pb, pa);
         }
       };
       at(std::integral_constant<int, 0>());
@@ -260,15 +267,17 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
 #pragma unroll
           for (int i = 0; i < MB; ++i) {
             if constexpr (TWO) acc[i][j] += low[TWO ? i : 0][TWO ? j : 0];
-            if constexpr (TURN) {
-#pragma unroll
-              for (int v = 0; v < 16; ++v) tot[CH ? i : 0][CH ? j : 0][v] = fmaf(acc[i][j][v], turned ? -1.0f : 1.0f, tot[CH ? i : 0][CH ? j : 0][v]);
-            } else {
-              tot[CH ? i : 0][CH ? j : 0] += acc[i][j];
-            }
+            if constexpr (decltype(turned)::value) tot[CH ? i : 0][CH ? j : 0] -= acc[i][j];
+            else tot[CH ? i : 0][CH ? j : 0] += acc[i][j];
           }
       }
-      if (TURN) turned ^= 0x80008000u;
+    };
+    for (int t = 0; t < T; t += UN) {
+      chain(std::false_type(), t);
+      if constexpr (TURN) {
+        t += UN;
+        if (t < T) chain(std::true_type(), t);
+      }
     }
     vm_wait<0>();
   }
@@ -279,12 +288,13 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
     for (int g = 0; g < 4; ++g) {
       const int n = n0 + (wn * NB + j) * 32 + 8 * g + 4 * half;
       if (n >= a.N) continue;
+      const int e4 = (n - n0) / 4;
       f4 mul = f4{1.f, 1.f, 1.f, 1.f};
-      if constexpr (PX == 2) mul = *reinterpret_cast<const f4*>(a.w_half_mul + n) * a.a_unscale;
+      if constexpr (PX == 2) mul = Es[0][e4] * a.a_unscale;
       f4 bias = f4{0.f, 0.f, 0.f, 0.f};
-      if (!SPLIT && a.bias) bias = *reinterpret_cast<const f4*>(a.bias + n);
+      if (!SPLIT && a.bias) bias = Es[1][e4];
       f4 scale = f4{1.f, 1.f, 1.f, 1.f};
-      if constexpr (EPI == GEMM_GELU && PX == 2) scale = *reinterpret_cast<const f4*>(a.c_scale + n);
+      if constexpr (EPI == GEMM_GELU && PX == 2) scale = Es[2][e4];
 #pragma unroll
       for (int i = 0; i < MB; ++i) {
         const int m = m0 + (wm * MB + i) * 32 + l32;
@@ -357,7 +367,6 @@ __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
     if (parts > 1) continue;
     if (live && a.bias) ebias[q] = *reinterpret_cast<const f4*>(a.bias + n);
     if (live && EPI == GEMM_RESID) eres[q] = *reinterpret_cast<const f4*>(a.resid + (size_t)m * a.ldc + n);
-    if (live && EPI == GEMM_GELU && PX == 2) eres[q] = *reinterpret_cast<const f4*>(a.c_scale + n);
   }
 
   f4 tot[MT][NG];
@@ -419,6 +428,14 @@ __global__ __launch_bounds__(512) void k_gemm_half_rows(GemmArgs a) {
 #pragma unroll
     for (int i = 0; i < PD; ++i)
       if (s + PD + i < steps) mul_step(rw[i], rx[i]);
+  }
+  // (GELU's column powers: over the loop there are no registers for them)
+  if constexpr (EPI == GEMM_GELU && PX == 2) {
+#pragma unroll
+    for (int q = 0; q < IPT; ++q) {
+      const int idx = tid + 512 * q, n = n0 + col_of(idx);
+      if (idx < ITEMS && n < n1) eres[q] = *reinterpret_cast<const f4*>(a.c_scale + n);
+    }
   }
   // tot[mt][g][r] is row 16 mt + 4 kq + r, column 16 g + i16
   float* mine = slab[wave];
@@ -839,7 +856,7 @@ hipError_t launch_tile(const GemmArgs& a, int epi, const HalfPlan& p, hipStream_
   if (a.w_half_parts == 2) {
     switch (p.tile) {
       case HALF_64x128: return Shape<2, 2, 1, 2, 2, 2, 3, 2, 32, 4, true>::launch(a, epi, p.parts, s);
-      case HALF_128x128: return Shape<2, 2, 2, 2, 2, 2, 2, 4, 16, 4, false>::launch(a, epi, p.parts, s);
+      case HALF_128x128: return Shape<2, 2, 2, 2, 2, 2, 2, 2, 32, 4, false, true>::launch(a, epi, p.parts, s);
       case HALF_128x128_8: return Shape<4, 2, 1, 2, 2, 2, 2, 4, 32, 4, true>::launch(a, epi, p.parts, s);
       default: return hipErrorInvalidValue;
     }
@@ -901,16 +918,19 @@ constexpr TilePace kTilePace[3][3] = {
     {{5.981f, 0.546f, 0.074f, 0.197f}, {9.04f, 0.604f, 0.329f, 0.111f}, {7.24f, 0.503f, 11.3f, 2.426f}},
     {{5.243f, 0.389f, 0.027f, 0.13f}, {6.453f, 0.422f, 0.178f, 0.125f}, {5.701f, 0.36f, 1.06f, -0.021f}},
     {{3.39f, 0.667f, 0.426f, -0.051f}, {}, {3.014f, 0.924f, 0.685f, 0.149f}}};
-// Products of half form with a tile of 128 x 128 for every CU or more: K is not cut, and the tiles' times are fitted by themselves
-// (224 products of widths 768 to 1600, 130 to 16384 rows; 5 to 10 % off, the choice 1 to 1.5 % slower than the best tile in the mean).
-// HALF_128x256 is for bf16 rows and K up to 2048 only.  Its one chain errs by 3.6 10^-7 at K = 1600 and 7.3 10^-7 at 6400, the chains
+// Products of half form with a tile of 128 x 128 for every CU or more: tiles only, and their times are fitted by themselves
+// (160 products of widths 768 to 1600, 700 to 16384 rows; 4 to 10 % off, the choice 0.4 to 1.5 % slower than the best tile in the mean).
+// HALF_128x256 is for bf16 rows and parts of K up to 2048 only.  Its one chain errs by 3.6 10^-7 at K = 1600 and 7.3 10^-7 at 6400, the chains
 // of the eight wavefronts by 1.2 and 1.6 10^-7, at 1.12 to 1.24 of its time (16384 x 4800 x 1600 490 us for 412, x 1600 x 6400 644
 // for 588).  With it the logits of int8 models' prompts of 2000 rows were off by 1.2 times as much as three bf16 parts are, those
 // of bf16 models with it at K = 4096 too, without at 0.8.
-constexpr TilePace kFullPace[2][6] = {
-    {{6.49f, 0.469f, 0.075f, 0.323f}, {8.01f, 0.54f, 0.459f, 0.258f}, {8.36f, 0.462f, 0.668f, 0.168f}, {}, {}, {}},
-    {{6.31f, 0.402f, -0.014f, 0.292f}, {7.97f, 0.416f, 0.242f, 0.292f}, {8.27f, 0.324f, 0.473f, 0.148f}, {11.59f, 0.577f, 0.623f, 0.275f}, {},
-     {10.65f, 0.544f, 0.85f, 0.311f}}};
+struct FullPace {
+  float start, stage, more, part, gelu;  // (gelu: of an item's write-out)
+};
+constexpr FullPace kFullPace[2][6] = {
+    {{5.17f, 0.463f, 0.077f, 0.314f, 0.83f}, {7.13f, 0.602f, 0.388f, 0.319f, 2.21f}, {7.37f, 0.495f, 0.619f, 0.191f, 3.58f}, {}, {}, {}},
+    {{5.01f, 0.39f, 0.01f, 0.259f, 1.06f}, {7.24f, 0.412f, 0.252f, 0.267f, 2.23f}, {7.15f, 0.348f, 0.426f, 0.184f, 3.41f},
+     {9.13f, 0.629f, 0.61f, 0.247f, 5.74f}, {}, {9.64f, 0.592f, 0.836f, 0.234f, 5.8f}}};
 constexpr Finish kFinish[3] = {{2.903f, 2.218f, 0.056f, 5.858f, -3.213f, 2.241f, 2.427f},
                                {4.686f, 1.352f, 0.859f, 18.205f, -0.462f, 3.567f, 1.958f},
                                {3.025f, 1.971f, 0.603f, 0.682f, 0.016f, 1.99f, 5.505f}};
@@ -946,15 +966,23 @@ HalfPlan gemm_half_plan(const GemmArgs& a, int epi, int num_cus) {
   auto take = [&](const HalfPlan& p, float us) {
     if (us < best_us) best = p, best_us = us;
   };
+  // (many values: their bytes; 4000 x 1280 values in a norm by itself 10.8 us, with two parts 18.7, three 20.9)
+  auto full_finish = [&](int parts) {
+    if (parts == 1) return a.ln_out ? 2.0f + 1.65f * mn : 0.0f;
+    return 1.0f + ((a.ln_out ? 2.3f : 1.3f) + 0.55f * (float)parts) * mn;
+  };
   if (kind != 2 && (long)((a.M + 127) / 128) * ((a.N + 127) / 128) >= cus) {
     for (int t : {HALF_64x128, HALF_128x128, HALF_128x128_8, HALF_128x256, HALF_128x256_8}) {
       if (t >= HALF_128x256 && kind != 1) continue;
-      if (t == HALF_128x256 && (a.w_scale || a.K > 2048)) continue;
       const int bm = t == HALF_64x128 ? 64 : 128, bn = t >= HALF_128x256 ? 256 : 128;
-      const long items = ((long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) + 7) / 8 * 8;
-      const float on_cu = (float)((items + cus - 1) / cus), round = std::max(0.0f, (float)items / (float)cus - 1.0f);
-      const TilePace& p = kFullPace[kind][t];
-      take({t, 1, 0, 0}, p.start + (float)steps * (p.stage + (on_cu - 1.0f) * p.more + round * p.part));
+      for (int parts = 1; parts <= std::max(1, most); ++parts) {
+        if (t == HALF_128x256 && (a.w_scale || a.K > 2048 * parts)) continue;
+        const long items = ((long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) + 7) / 8 * 8 * parts;
+        const float on_cu = (float)((items + cus - 1) / cus), round = std::max(0.0f, (float)items / (float)cus - 1.0f);
+        const FullPace& p = kFullPace[kind][t];
+        take({t, parts, 0, 0}, p.start + (float)((steps + parts - 1) / parts) * (p.stage + (on_cu - 1.0f) * p.more + round * p.part) +
+                                (epi == GEMM_GELU ? on_cu * p.gelu : 0.0f) + full_finish(parts));
+      }
     }
     return best;
   }
