@@ -704,7 +704,7 @@ TRAFFIC_SOURCE_355M_B16 = "profiles/batched_decode_355m_b16_xl_bf16_b32.txt"
 # Bytes through the L2s to and from the fabric per XL bf16 prefill of 32 x 512 tokens (FETCH_SIZE
 # scaled by 1.9994 + WRITE_SIZE over all launches of a step; most of the reads are operand
 # re-reads that the Infinity Cache serves).
-TRAFFIC_XL_BF16_PREFILL_B32_512 = 333500000000
+TRAFFIC_XL_BF16_PREFILL_B32_512 = 328400000000
 TRAFFIC_SOURCE_XL_BF16_PREFILL = "profiles/k_gemm_half_prompts.txt"
 
 
