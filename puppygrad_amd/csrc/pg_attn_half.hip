@@ -32,7 +32,8 @@ __device__ __forceinline__ void halves8(f4 a, f4 b, u4v (&part)[2]) {
 //   online softmax per query            a lane holds 16 keys of one query
 //   O^T (dims x queries) += V^T . P^T   a lane's own weights are the operand; V's keys are in LDS in that order
 // It appends K and V to the cache panels.  512 tokens x 32, 25 heads 231 us (k_attn_prefill_cut) -> 177; 1000 tokens 42 -> 33.5; 1024
-// tokens, 12 heads 29.5 (k_attn_prefill64) -> 27 (with one power of two for all of Q, of K and of V 32 and 25).  Error against f64 1.4 to 1.8 10^-7, as on the f32 cores (1.2 to 1.9).
+// tokens, 12 heads 29.5 (k_attn_prefill64) -> 27 (with one power of two for all of Q, of K and of V 32 and 25).  Error against f64,
+// values N(0, 1), 1.4 to 1.85 10^-7: 0.95 to 1.1 of the f32 cores' (queries three times as large 0.83 to 0.93), 1.5 of k_attn_prefill_cut's (1.2).
 // What bounds it: per tile and wavefront 768 clocks of matrix instructions and about 1100 of vector ones.  Grid: x = head, y = block of queries, longest rows first, z = sequence.
 template <int QG, int KG, int FORM>
 __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const float* __restrict__ qkv, int T, int C, int P,
