@@ -90,7 +90,8 @@ __device__ __forceinline__ void store_gelu(void* to, int mp, size_t m, size_t n,
 template <int WM, int WN, int MB, int NB, int PX, int PW, int EPI, int SPLIT, int OCC, int NA, int KT, int CH, bool TWO, bool TURN>
 __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
   constexpr int NW = WM * WN, BM = 32 * MB * WM, BN = 32 * NB * WN, NO = KT / 8, NS = KT / 16;
-  constexpr int IA = NO * PX * BM / 64 / NW, IB = NO * PW * BN / 64 / NW;
+  constexpr int IA = NO * PX * BM / 64 / NW, IB = NO * PW * BN / 64 / NW, IC = IA + IB;
+  constexpr int H = NS == 2 && NA > 2 ? (IC + 1) / 2 : IC;  // requests of a stage behind the barrier; the rest in the step before the next
   constexpr int UN = CH ? CH : NA;
   static_assert(!TURN || (!TWO && CH != 0));
   static_assert(UN % NA == 0 && (NS == 2 || UN % 2 == 0) && UN <= 8 && (CH != 0 || !TWO));
@@ -138,12 +139,15 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
   const char* Ab = reinterpret_cast<const char*>(a.A) + kt0 * astage;
   const char* Wb = static_cast<const char*>(a.w_half) + kt0 * bstage;
   const unsigned as_lds = (unsigned)(size_t)(lds_ptr)(void*)&As[0][0], bs_lds = (unsigned)(size_t)(lds_ptr)(void*)&Bs[0][0];
-  auto dma = [&](int t, int buf) __attribute__((always_inline)) {
+  // The i-th of a wavefront's requests for stage t, of which `an` and `bn` are the operands.
+  auto request = [&](const char* an, const char* bn, int buf, int i) __attribute__((always_inline)) {
+    if (i < IA) lds_dma16(an, aoff[i < IA ? i : 0], as_lds + (unsigned)(buf * NO * PX * BM * 16 + (wave * IA + i) * 1024));
+    else lds_dma16(bn, boff[i < IA ? 0 : i - IA], bs_lds + (unsigned)(buf * NO * PW * BN * 16 + (wave * IB + i - IA) * 1024));
+  };
+  auto requests = [&](int t, int buf, int n) __attribute__((always_inline)) {
     const size_t k = (size_t)min(t, T - 1);
 #pragma unroll
-    for (int i = 0; i < IA; ++i) lds_dma16(Ab + k * astage, aoff[i], as_lds + (unsigned)(buf * NO * PX * BM * 16 + (wave * IA + i) * 1024));
-#pragma unroll
-    for (int i = 0; i < IB; ++i) lds_dma16(Wb + k * bstage, boff[i], bs_lds + (unsigned)(buf * NO * PW * BN * 16 + (wave * IB + i) * 1024));
+    for (int i = 0; i < n; ++i) request(Ab + k * astage, Wb + k * bstage, buf, i);
   };
 
   f16v acc[MB][NB], tot[CH ? MB : 1][CH ? NB : 1], low[TWO ? MB : 1][TWO ? NB : 1];
@@ -157,56 +161,66 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
         if constexpr (CH != 0) tot[i][j][v] = 0.0f;
       }
   struct Ops { u4v x[MB][PX], w[NB][PW]; };
-  auto read = [&](int buf, int s, Ops& o) __attribute__((always_inline)) {
+  constexpr int NR = PX * MB + PW * NB;
+  auto read = [&](int buf, int s, Ops& o, int r) __attribute__((always_inline)) {  // the r-th, in the order in which the products need them
+    int at = 0;
 #pragma unroll
-    for (int p = PX - 1; p >= 0; --p) {  // in the order in which the products need them
+    for (int p = PX - 1; p >= 0; --p) {
 #pragma unroll
-      for (int i = 0; i < MB; ++i) o.x[i][p] = As[buf][((2 * s + half) * PX + p) * BM + (wm * MB + i) * 32 + l32];
+      for (int i = 0; i < MB; ++i)
+        if (at++ == r) o.x[i][p] = As[buf][((2 * s + half) * PX + p) * BM + (wm * MB + i) * 32 + l32];
       const int q = PX - 1 - p;
       if (q < PW) {
 #pragma unroll
-        for (int j = 0; j < NB; ++j) o.w[j][q] = Bs[buf][((2 * s + half) * PW + q) * BN + (wn * NB + j) * 32 + l32];
+        for (int j = 0; j < NB; ++j)
+          if (at++ == r) o.w[j][q] = Bs[buf][((2 * s + half) * PW + q) * BN + (wn * NB + j) * 32 + l32];
       }
     }
   };
   using P = Products<PX, PW>;
-  constexpr int NP = P::n;
-  auto step = [&](auto turned, auto first, Ops& cur, Ops& nxt, int buf, int s) __attribute__((always_inline)) {
+  constexpr int NP = P::n, NM = NP * MB * NB;
+  auto multiply = [&](auto first, const Ops& cur, int f) __attribute__((always_inline)) {  // the f-th of a step
     constexpr bool fresh = CH != 0 && decltype(first)::value;
-    read(buf, s, nxt);
+    const int p = f / (MB * NB), j = f / MB % NB, i = f % MB;
+    f16v& sum = TWO && p < NP - 1 ? low[TWO ? i : 0][TWO ? j : 0] : acc[i][j];
+    if (fresh && (p == 0 || (TWO && p == NP - 1))) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) sum[v] = 0.0f;
+    }
+    const u4v &w = cur.w[j][P::w[p]], &x = cur.x[i][P::x[p]];
+    if constexpr (PX == 3)
+      sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x), sum, 0, 0, 0);
+    else
+      sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, w), __builtin_bit_cast(h8v, x), sum, 0, 0, 0);
+  };
+  // A step: its matrix instructions, the reads of the next step's operands (step s of buffer buf) and requests FROM .. UPTO - 1 of a
+  // wavefront for stage t, to buffer `to`, spread over one another: all
+  // requests of a stage in one go behind the barrier keep every wavefront of a CU from its matrix instructions until the path to LDS
+  // has taken them (32 KB a stage; single products 0 to 7 % longer; a prompt of 1000 against f32 rows 1600 wide, 48 layers, 13.28 ms
+  // so and 13.03 spread, 32 prompts of 512 against bf16 rows 105.8 and 104.4).  With two buffers all of them stay behind the barrier:
+  // later ones are late (1000 x 6400 x 1600 70.8 and 73.7 us).
+  auto step = [&](auto turned, auto first, Ops& cur, Ops& nxt, int buf, int s, int t, int to, auto from, auto upto) __attribute__((always_inline)) {
+    constexpr int FROM = decltype(from)::value, N = decltype(upto)::value - FROM, G = N > 0 ? N : NM;
     if constexpr (decltype(turned)::value) {  // (the sign bits of two f16 numbers)
 #pragma unroll
       for (int j = 0; j < NB; ++j)
 #pragma unroll
         for (int p = 0; p < PW; ++p) cur.w[j][p] ^= 0x80008000u;
     }
+    const size_t k = (size_t)min(t, T - 1);
+    const char *an = Ab + k * astage, *bn = Wb + k * bstage;
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
+    for (int g = 0; g < G; ++g) {
 #pragma unroll
-      for (int j = 0; j < NB; ++j)
+      for (int r = g * NR / G; r < (g + 1) * NR / G; ++r) read(buf, s, nxt, r);
 #pragma unroll
-        for (int i = 0; i < MB; ++i) {
-          f16v& sum = TWO && p < NP - 1 ? low[TWO ? i : 0][TWO ? j : 0] : acc[i][j];
-          if (fresh && (p == 0 || (TWO && p == NP - 1))) {
-#pragma unroll
-            for (int v = 0; v < 16; ++v) sum[v] = 0.0f;
-          }
-          const u4v &w = cur.w[j][P::w[p]], &x = cur.x[i][P::x[p]];
-          if constexpr (PX == 3)
-            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x), sum, 0, 0, 0);
-          else
-            sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, w), __builtin_bit_cast(h8v, x), sum, 0, 0, 0);
-        }
+      for (int f = g * NM / G; f < (g + 1) * NM / G; ++f) multiply(first, cur, f);
+      __builtin_amdgcn_sched_barrier(0);
+      if (N > 0) {
+        request(an, bn, to, FROM + g);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
-  };
-  auto interleave = [&] __attribute__((always_inline)) {
-    constexpr int NM = NP * MB * NB, NR = PX * MB + PW * NB, PER = (NR + NM - 1) / NM;
-#pragma unroll
-    for (int g = 0; g < NM; ++g) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if (g * PER < NR) __builtin_amdgcn_sched_group_barrier(0x100, PER, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
   };
 
   if (T > 0) {
@@ -219,31 +233,26 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void k_gemm_half(GemmArgs a) {
       if constexpr (EPI == GEMM_GELU && PX == 2) lds_dma16(a.c_scale, off, es + 2048);
     }
 #pragma unroll
-    for (int t = 0; t < NA; ++t) dma(t, t);
-    vm_wait<(NA - 1) * (IA + IB)>();
+    for (int t = 0; t < NA - 1; ++t) requests(t, t, IC);
+    requests(NA - 1, NA - 1, H);
+    vm_wait<(NA - 2) * IC + H>();
     asm volatile("s_barrier" ::: "memory");
-    read(0, 0, pa);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) read(0, 0, pa, r);
     auto stage = [&](auto turned, auto u, int t, Ops& p0, Ops& p1) __attribute__((always_inline)) {
       constexpr int U = decltype(u)::value, ab = U % NA, nb = (U + 1) % NA;
       const std::integral_constant<bool, U == 0> head;
       const std::false_type rest;
-      if constexpr (NS == 2) {
-        step(turned, head, p0, p1, ab, 1);
-        interleave();
-      }
-      vm_wait<(NA - 2) * (IA + IB)>();
+      const std::integral_constant<int, 0> none;
+      const std::integral_constant<int, H> some;
+      const std::integral_constant<int, IC> all;
+      if constexpr (NS == 2) step(turned, head, p0, p1, ab, 1, t - 1 + NA, (U + NA - 1) % NA, some, all);
+      vm_wait<(NA - 2) * IC>();
       __builtin_amdgcn_sched_barrier(0);
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
-      dma(t + NA, ab);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (NS == 2) {
-        step(turned, rest, p1, p0, nb, 0);
-        interleave();
-      } else {
-        step(turned, head, p0, p1, nb, 0);
-        interleave();
-      }
+      if constexpr (NS == 2) step(turned, rest, p1, p0, nb, 0, t + NA, ab, none, some);
+      else step(turned, head, p0, p1, nb, 0, t + NA, ab, none, all);
     };
     auto chain = [&](auto turned, int t) __attribute__((always_inline)) {
       auto at = [&](auto u) __attribute__((always_inline)) {
