@@ -842,7 +842,9 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
   auto gemm = [&](const float* A, int lda, const float* W, const float* bias, float* Cout,
                   int ldc, int N, int K, int epi, const float* ln_g = nullptr,
                   const float* ln_b = nullptr, int a_cut = 0, int ln_cut = 0, const void* w_half = nullptr,
-                  const float* w_half_mul = nullptr, const float* c_scale = nullptr, bool ln_half = false) -> hipError_t {
+                  const float* w_half_mul = nullptr, const float* c_scale = nullptr, bool ln_half = false,
+                  const float* next_W = nullptr, int next_N = 0) -> hipError_t {
+    pgk::Ahead ahead;
     pgk::GemmArgs a{};
     a.A = A; a.w_bf16 = m->w_bf16; a.W = W; a.bias = bias; a.resid = Cout; a.C = Cout;
     if (w_half) {
@@ -886,11 +888,12 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
       PG_HIP(pgk::launch_attn_finish(c->part_acc, c->part_m, c->part_l, H, hd, nsplit, c->att_b, s,
                                      B, bs, form, hw.attn.v));
     PG_HIP(gemm(c->att_b, C, w.c_proj_w, w.c_proj_b, c->x, C, C, C, pgk::GEMM_RESID, half ? hw.norm_2_g : w.ln_2_g,
-                half ? hw.norm_2_b : w.ln_2_b, cut, cut, hw.c_proj, hw.c_proj_mul, nullptr, half));
+                half ? hw.norm_2_b : w.ln_2_b, cut, cut, hw.c_proj, hw.c_proj_mul, nullptr, half, w.c_fc_w, I));
     PG_HIP(gemm(c->xn_b, C, w.c_fc_w, w.c_fc_b, c->hbuf, I, I, C, pgk::GEMM_GELU, nullptr, nullptr, cut, 0,
                 hw.c_fc, hw.c_fc_mul, hw.hidden));
     PG_HIP(gemm(c->hbuf, I, w.c_proj_mlp_w, w.c_proj_mlp_b, c->x, C, C, I, pgk::GEMM_RESID, next_g, next_b, cut,
-                cut && l + 1 < g.L, hw.c_proj_mlp, hw.c_proj_mlp_mul, nullptr, next_half));
+                cut && l + 1 < g.L, hw.c_proj_mlp, hw.c_proj_mlp_mul, nullptr, next_half,
+                l + 1 < g.L ? m->layers[l + 1].c_attn_w : nullptr, 3 * C));
   }
   PG_HIP(gemm(c->xn_b, C, m->lm_w, nullptr, c->logits_buf, (int)g.V, (int)g.V, C, pgk::GEMM_BIAS));
   return PG_OK;
@@ -933,6 +936,13 @@ pg_status stack_advance(const pg_model* m, pg_kv_cache* c, const uint32_t* ids, 
   if ((s = ensure_ids(c, c->B * std::min<size_t>(n, std::max<size_t>(32, 8192 / c->B))))) return s;
   if ((s = pgh::stack_rows(m, c, ids, n, c->seq_len, rows, dst, marks))) return s;
   PG_HIP(hipStreamSynchronize(c->stream));
+    if (next_W && !half && !cut) {
+      pgk::GemmArgs n = a;
+      n.W = next_W; n.N = next_N; n.K = C; n.lda = C;
+      if (m->w_i8) n.w_scale = i8_scales_of(next_W, (size_t)next_N, (size_t)C);
+      ahead = pgk::gemm_rows32_ahead(n, m->num_cus);
+      a.ahead = &ahead;
+    }
   c->seq_len += n;
   return PG_OK;
 }

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "pg_ahead.h"
+
 namespace pgk {
 
 constexpr int kHeadDim = 64;       // every GPT-2 size has head_dim 64; other sizes use the generic path
@@ -91,6 +93,8 @@ struct GemvPair {
 constexpr int kPairMaxSplits = 8;
 constexpr int kPairMaxK = 16320;
 hipError_t launch_gemv_pair(const GemvPair& a, hipStream_t s);
+// What a launch before launch_gemv_pair(a) can read ahead for it.
+Ahead gemv_pair_ahead(const GemvPair& a);
 
 // x = wte[tok] + wpe[pos]; tok comes from tok_ptr[0] when tok_ptr != nullptr.
 hipError_t launch_embed(float* x, const float* wte, const float* wpe, const uint32_t* tok_ptr,
@@ -289,6 +293,7 @@ struct GemmArgs {
 };
 // Element (row b < 32, column k) of a packed activation matrix: the float4 of columns
 // 4j..4j+3 of all 32 rows lie next to each other, so that 32 lanes which each read four
+  const Ahead* ahead = nullptr;  // (host) what the launch that ends the product can read ahead for the next one
 // columns of "their" row read one contiguous 512 bytes.  A packed matrix of K columns takes
 // 32 K floats whatever its row count.
 __host__ __device__ inline size_t packed32_index(size_t b, size_t k) {
@@ -338,6 +343,8 @@ bool gemm_tail_plan(GemmArgs& a, int num_cus, int bm = 64, int bn = 64);
 hipError_t launch_gemm(const GemmArgs& a, int epilogue, int num_cus, hipStream_t s);
 // Many small products in one launch: rows are sorted by the matrix they meet.  Row m of the product
 // takes row group_rows[m] of A (any row where that is -1), and the rows of tile m / tile_rows meet
+// What a launch before launch_gemm(a) can read ahead for it, where the 32-row kernel takes it whole.
+Ahead gemm_rows32_ahead(const GemmArgs& a, int num_cus);
 // matrix group_tile[m / tile_rows] of W [groups][N][K] (-1: the tile is left out).  a.M counts the rows
 // with their padding, a multiple of tile_rows (16, 32, 64 or, bf16 rows only, 128).  C has a row per m.
 // group_rows null: row m itself.  GEMM_BIAS (without bias) or GEMM_SILU_PAIR.

@@ -11,6 +11,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "pg_ahead.h"
+
 namespace pgk {
 
 constexpr int kMixMaxDim = 256;   // key and value sizes per head
@@ -126,6 +128,7 @@ struct MixDecode {
   GatedMlp mlp;
   int attn_splits;
   float* part;
+  Ahead ahead;  // of a step of one sequence
 };
 // Key splits of a layer's attention (rec: the recurrence beside it, or null).
 int mix_decode_splits(const ChunkAttn& a, const Recurrence* rec);

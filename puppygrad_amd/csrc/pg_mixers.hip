@@ -512,7 +512,7 @@ __device__ void recurrence_role(const MixDecode& m, int b, int h, float* lds) {
 }
 
 template <int NT, int RPT, int NV>
-__global__ __launch_bounds__(NT) void k_mix_decode(MixDecode m, int attn_items, int rec_items) {
+__global__ __launch_bounds__(NT) void k_mix_decode(MixDecode m, int attn_items, int rec_items, int mlp_items) {
   __shared__ __attribute__((aligned(16))) float lds[kDecodeLds<NT>];
   const int b = blockIdx.y;
   int item = blockIdx.x;
@@ -526,6 +526,10 @@ __global__ __launch_bounds__(NT) void k_mix_decode(MixDecode m, int attn_items, 
     return;
   }
   item -= attn_items;
+  if (item >= mlp_items) {
+    read_ahead(m.ahead, item - mlp_items, blockIdx.x, NT);
+    return;
+  }
   const int j = item * NT + threadIdx.x;
   if (j >= m.mlp.ff_pad) return;
   const float* y = m.y + (size_t)b * m.ld_y;
@@ -1697,15 +1701,15 @@ hipError_t launch_mix_decode(const MixDecode& a, hipStream_t s) {
   const int rec_items = a.has_rec ? a.rec.heads : 0;
   const int rows = a.has_rec ? rows_per_thread(a.rec.dim, a.rec.vdim) : 1, nt = decode_threads(rows);
   const int mlp_items = a.has_mlp ? (a.mlp.ff_pad + nt - 1) / nt : 0;
-  const dim3 grid((unsigned)(attn_items + rec_items + mlp_items), (unsigned)a.nseq);
+  const dim3 grid((unsigned)(attn_items + rec_items + mlp_items + (a.nseq == 1 ? a.ahead.blocks : 0)), (unsigned)a.nseq);
   if (grid.x == 0) return hipSuccess;
   const int nv = !a.has_attn || a.attn.dim_pad <= 64 ? 1 : a.attn.dim_pad <= 128 ? 2 : 4;
   switch (rows) {
 #define PG_RPT(R, NT, N)                                                                                             \
   case R:                                                                                                            \
-    if (nv == 1) hipLaunchKernelGGL((k_mix_decode<NT, N, 1>), grid, dim3(NT), 0, s, a, attn_items, rec_items);        \
-    else if (nv == 2) hipLaunchKernelGGL((k_mix_decode<NT, N, 2>), grid, dim3(NT), 0, s, a, attn_items, rec_items);   \
-    else hipLaunchKernelGGL((k_mix_decode<NT, N, 4>), grid, dim3(NT), 0, s, a, attn_items, rec_items);                \
+    if (nv == 1) hipLaunchKernelGGL((k_mix_decode<NT, N, 1>), grid, dim3(NT), 0, s, a, attn_items, rec_items, mlp_items);        \
+    else if (nv == 2) hipLaunchKernelGGL((k_mix_decode<NT, N, 2>), grid, dim3(NT), 0, s, a, attn_items, rec_items, mlp_items);   \
+    else hipLaunchKernelGGL((k_mix_decode<NT, N, 4>), grid, dim3(NT), 0, s, a, attn_items, rec_items, mlp_items);                \
     break;
     PG_RPT(1, 256, 1) PG_RPT(2, 256, 2) PG_RPT(4, 256, 4) PG_RPT(8, 256, 8) PG_RPT(16, 256, 16)
     PG_RPT(32, 512, 16) PG_RPT(64, 512, 32) PG_RPT(128, 1024, 32) PG_RPT(256, 1024, 64)

@@ -1195,6 +1195,16 @@ pg_status step_launches(const pg_model* model, pg_kv_cache* c, ProfileMarks* mar
     d.attn = b.attn; d.rec = b.rec; d.mlp = l.mlp;
     d.attn_splits = l.has_attn ? pgk::mix_decode_splits(l.attn, l.has_rec ? &l.rec : nullptr) : 1;
     d.part = st.part;
+    pgk::GemvPair p{};
+    p.w_bf16 = model->w_bf16;
+    p.num_cus = model->num_cus;
+    p.W1 = l.out_w; p.x1 = st.mix; p.s1 = l.ls1; p.K1 = l.mix_pad;
+    p.resid = st.x; p.y = st.x; p.nout = Cp;
+    const bool both = l.has_mlp && l.mix_pad + l.mlp.ff_pad <= pgk::kPairMaxK;
+    if (both) {
+      p.W2 = l.down_w; p.x2 = st.act; p.s2 = l.ls2; p.K2 = l.mlp.ff_pad;
+    }
+    if (B == 1) d.ahead = pgk::gemv_pair_ahead(p);
     PG_HIP(pgk::launch_mix_decode(d, s));
     // the attention's key splits are added by the projection of the one-sequence step, where
     // they are few
@@ -1203,18 +1213,9 @@ pg_status step_launches(const pg_model* model, pg_kv_cache* c, ProfileMarks* mar
     PG_MARK(kAttention);
     const bool more = i + 1 < m.layers.size();
     if (B == 1) {
-      pgk::GemvPair p{};
-      p.w_bf16 = model->w_bf16;
-      p.num_cus = model->num_cus;
-      p.W1 = l.out_w; p.x1 = st.mix; p.s1 = l.ls1; p.K1 = l.mix_pad;
-      p.resid = st.x; p.y = st.x; p.nout = Cp;
       if (sum_in_pair) {
         p.part = st.part; p.part_splits = d.attn_splits; p.part_n = l.attn.heads * l.attn.dim;
         p.part_col = l.attn.out_col;
-      }
-      const bool both = l.has_mlp && l.mix_pad + l.mlp.ff_pad <= pgk::kPairMaxK;
-      if (both) {
-        p.W2 = l.down_w; p.x2 = st.act; p.s2 = l.ls2; p.K2 = l.mlp.ff_pad;
       }
       PG_HIP(pgk::launch_gemv_pair(p, s));
       if (l.has_mlp && !both) {  // (too wide for one launch)
