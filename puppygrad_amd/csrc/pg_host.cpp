@@ -859,6 +859,13 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
     if (ln_g) { a.ln_out = c->xn_b; a.ln_g = ln_g; a.ln_b = ln_b; a.ln_eps = g.eps; a.ln_packed = pk; }
     a.split_items_per_cu = m->gemm_split_items;
     a.b9_min_rows = m->gemm_b9_min_rows;
+    if (next_W && !half && !cut) {
+      pgk::GemmArgs n = a;
+      n.W = next_W; n.N = next_N; n.K = C; n.lda = C;
+      if (m->w_i8) n.w_scale = i8_scales_of(next_W, (size_t)next_N, (size_t)C);
+      ahead = pgk::gemm_rows32_ahead(n, m->num_cus);
+      a.ahead = &ahead;
+    }
     return pgk::launch_gemm(a, epi, m->num_cus, s);
   };
   PG_HIP(pgk::launch_embed_batch(c->x, m->wte, m->wpe, d_ids, B, (int)pos, C, s, m->w_bf16));
@@ -936,13 +943,6 @@ pg_status stack_advance(const pg_model* m, pg_kv_cache* c, const uint32_t* ids, 
   if ((s = ensure_ids(c, c->B * std::min<size_t>(n, std::max<size_t>(32, 8192 / c->B))))) return s;
   if ((s = pgh::stack_rows(m, c, ids, n, c->seq_len, rows, dst, marks))) return s;
   PG_HIP(hipStreamSynchronize(c->stream));
-    if (next_W && !half && !cut) {
-      pgk::GemmArgs n = a;
-      n.W = next_W; n.N = next_N; n.K = C; n.lda = C;
-      if (m->w_i8) n.w_scale = i8_scales_of(next_W, (size_t)next_N, (size_t)C);
-      ahead = pgk::gemm_rows32_ahead(n, m->num_cus);
-      a.ahead = &ahead;
-    }
   c->seq_len += n;
   return PG_OK;
 }

@@ -290,10 +290,10 @@ struct GemmArgs {
   int plan_band = 0;  // band height of the tile numbering (0: chosen by the launcher)
   int plan_bk16 = 0;  // 1: k-tiles of 16 columns also where K would allow 32
   const int *group_tile = nullptr, *group_rows = nullptr;  // launch_gemm_grouped
+  const Ahead* ahead = nullptr;  // (host) what the launch that ends the product can read ahead for the next one
 };
 // Element (row b < 32, column k) of a packed activation matrix: the float4 of columns
 // 4j..4j+3 of all 32 rows lie next to each other, so that 32 lanes which each read four
-  const Ahead* ahead = nullptr;  // (host) what the launch that ends the product can read ahead for the next one
 // columns of "their" row read one contiguous 512 bytes.  A packed matrix of K columns takes
 // 32 K floats whatever its row count.
 __host__ __device__ inline size_t packed32_index(size_t b, size_t k) {
@@ -340,11 +340,11 @@ bool gemm_takes_rows32(int M, int K, int lda, int w_bf16);
 bool gemm_supported(const GemmArgs& a);
 int gemm_split_parts(const GemmArgs& a, int num_cus, int bm = 64, int bn = 64);
 bool gemm_tail_plan(GemmArgs& a, int num_cus, int bm = 64, int bn = 64);
+// What a launch before launch_gemm(a) can read ahead for it, where the 32-row kernel takes it whole.
+Ahead gemm_rows32_ahead(const GemmArgs& a, int num_cus);
 hipError_t launch_gemm(const GemmArgs& a, int epilogue, int num_cus, hipStream_t s);
 // Many small products in one launch: rows are sorted by the matrix they meet.  Row m of the product
 // takes row group_rows[m] of A (any row where that is -1), and the rows of tile m / tile_rows meet
-// What a launch before launch_gemm(a) can read ahead for it, where the 32-row kernel takes it whole.
-Ahead gemm_rows32_ahead(const GemmArgs& a, int num_cus);
 // matrix group_tile[m / tile_rows] of W [groups][N][K] (-1: the tile is left out).  a.M counts the rows
 // with their padding, a multiple of tile_rows (16, 32, 64 or, bf16 rows only, 128).  C has a row per m.
 // group_rows null: row m itself.  GEMM_BIAS (without bias) or GEMM_SILU_PAIR.

@@ -1453,15 +1453,6 @@ hipError_t launch_gemv(const GemvArgs& a, int prologue, int epilogue, hipStream_
   return hipErrorInvalidValue;
 }
 
-hipError_t launch_gemv_pair(const GemvPair& a, hipStream_t s) {
-  if (a.K1 % 32 != 0 || a.K2 % 32 != 0 || a.K1 + a.K2 > kPairMaxK || (a.W2 == nullptr) != (a.K2 == 0))
-    return hipErrorInvalidValue;
-  const size_t lds = (size_t)(a.K1 + a.K2) * sizeof(float);
-  const int waves = pair_waves(a);
-  const dim3 grid((a.nout + waves - 1) / waves);
-  if (a.w_bf16)
-    hipLaunchKernelGGL((k_gemv_pair<1, WM_BF16X8>), grid, dim3(64 * waves), lds, s, a);
-  else
 namespace {
 int pair_waves(const GemvPair& a) { return std::min(kPairMaxThreads / 64, std::max(kWaves, (a.nout + a.num_cus - 1) / a.num_cus)); }
 }  // namespace
@@ -1478,6 +1469,15 @@ Ahead gemv_pair_ahead(const GemvPair& a) {
   return r;
 }
 
+hipError_t launch_gemv_pair(const GemvPair& a, hipStream_t s) {
+  if (a.K1 % 32 != 0 || a.K2 % 32 != 0 || a.K1 + a.K2 > kPairMaxK || (a.W2 == nullptr) != (a.K2 == 0))
+    return hipErrorInvalidValue;
+  const size_t lds = (size_t)(a.K1 + a.K2) * sizeof(float);
+  const int waves = pair_waves(a);
+  const dim3 grid((a.nout + waves - 1) / waves);
+  if (a.w_bf16)
+    hipLaunchKernelGGL((k_gemv_pair<1, WM_BF16X8>), grid, dim3(64 * waves), lds, s, a);
+  else
     hipLaunchKernelGGL((k_gemv_pair<1, WM_F32X4>), grid, dim3(64 * waves), lds, s, a);
   return hipGetLastError();
 }
