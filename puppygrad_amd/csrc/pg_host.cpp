@@ -202,30 +202,72 @@ pg_status check_compatible(const pg_model* m, pg_kv_cache* c) {
   return PG_OK;
 }
 
-// One cached decoder step for sequence b (forward_one_profiled_with_scratch,
-// src/models/gpt2/rust.rs:943-1006, block at 1136-1250) as a chain of fused
-// launches on the cache's stream.  The token comes from tok_ptr (device) when
-// it is non-null.  With want_logits false the final LayerNorm and lm_head are
-// skipped (prefill discards those logits, rust.rs:922-926).
 #define PG_MARK(b) \
   do {             \
     if (marks) PG_HIP(marks->mark(s, ProfileMarks::b)); \
   } while (0)
 
-pg_status enqueue_forward_one(const pg_model* m, pg_kv_cache* c, size_t b,
-                              const uint32_t* tok_ptr, uint32_t tok, size_t pos,
-                              bool want_logits, ProfileMarks* marks = nullptr) {
+// What follows c_attn in layer l for the row of sequence b at position pos: attention of q, c_proj and the MLP, x += both.  The
+// cache holds keys and values up to pos; hb: the hidden row.
+pg_status enqueue_row_behind_qkv(const pg_model* m, pg_kv_cache* c, size_t b, size_t l, float* x, float* q, float* hb, size_t pos,
+                                 ProfileMarks* marks) {
   const Cfg& g = m->cfg;
   const int C = (int)g.C, I = (int)g.I, H = (int)g.H, hd = (int)g.hd(), P = (int)g.P;
   hipStream_t s = c->stream;
-  float* x = c->x + b * g.C;
-  float* q = c->q + b * g.C;
-  float* hb = c->hbuf + b * g.I;
+  const pgk::LayerW& w = m->layers[l];
   const size_t part_stride = (size_t)H * pgk::kMaxSplits;
   float* pa = c->part_acc + b * part_stride * hd;
   float* pm = c->part_m + b * part_stride;
   float* pl = c->part_l + b * part_stride;
   const int nsplit = hd == pgk::kHeadDim ? pgk::choose_nsplit((int)pos + 1, H, m->num_cus, m->attn_blocks_per_cu) : 1;
+  // attention over keys [0, pos]
+  PG_HIP(pgk::launch_attn_decode(q, c->k_panel(l, b), c->v_panel(l, b), (int)pos, P, H, hd,
+                                 nsplit, pa, pm, pl, s));
+  if (!(nsplit > 2 && hd == pgk::kHeadDim)) PG_MARK(kAttention);
+  // merge splits + c_proj + residual.  Every block of the projection repeats the merge in
+  // its prologue, which is cheap for a few splits; beyond that the merge gets a launch of
+  // its own (into q, which the attention has finished reading).
+  pgk::GemvArgs a{};
+  a.w_bf16 = m->w_bf16; a.W = w.c_proj_w; a.w_scale = w.c_proj_s; a.bias = w.c_proj_b; a.y = x; a.resid = x; a.K = C; a.nout = C;
+  if (nsplit > 2 && hd == pgk::kHeadDim) {
+    PG_HIP(pgk::launch_attn_finish(pa, pm, pl, H, hd, nsplit, q, s));
+    PG_MARK(kAttention);
+    a.x = q;
+    PG_HIP(pgk::launch_gemv(a, pgk::PRO_NONE, pgk::EPI_RESID, s));
+  } else {
+    a.part_acc = pa; a.part_m = pm; a.part_l = pl; a.nsplit = nsplit; a.head_dim = hd;
+    PG_HIP(pgk::launch_gemv(a, pgk::PRO_ATTN_COMBINE, pgk::EPI_RESID, s));
+  }
+  PG_MARK(kAttnProj);
+  // LN2 + c_fc + GELU
+  a = pgk::GemvArgs{};
+  a.w_bf16 = m->w_bf16; a.W = w.c_fc_w; a.w_scale = w.c_fc_s; a.bias = w.c_fc_b; a.x = x; a.y = hb; a.K = C; a.nout = I;
+  a.ln_g = w.ln_2_g; a.ln_b = w.ln_2_b; a.eps = g.eps;
+  PG_HIP(pgk::launch_gemv(a, pgk::PRO_LN, pgk::EPI_GELU, s));
+  PG_MARK(kMlpFc);
+  // mlp c_proj + residual
+  a = pgk::GemvArgs{};
+  a.w_bf16 = m->w_bf16; a.W = w.c_proj_mlp_w; a.w_scale = w.c_proj_mlp_s; a.bias = w.c_proj_mlp_b; a.x = hb; a.y = x; a.resid = x; a.K = I;
+  a.nout = C;
+  PG_HIP(pgk::launch_gemv(a, pgk::PRO_NONE, pgk::EPI_RESID, s));
+  PG_MARK(kMlpProj);
+  return PG_OK;
+}
+
+// One cached decoder step for sequence b (forward_one_profiled_with_scratch,
+// src/models/gpt2/rust.rs:943-1006, block at 1136-1250) as a chain of fused
+// launches on the cache's stream.  The token comes from tok_ptr (device) when
+// it is non-null.  With want_logits false the final LayerNorm and lm_head are
+// skipped (prefill discards those logits, rust.rs:922-926).
+pg_status enqueue_forward_one(const pg_model* m, pg_kv_cache* c, size_t b,
+                              const uint32_t* tok_ptr, uint32_t tok, size_t pos,
+                              bool want_logits, ProfileMarks* marks = nullptr) {
+  const Cfg& g = m->cfg;
+  const int C = (int)g.C, hd = (int)g.hd(), P = (int)g.P;
+  hipStream_t s = c->stream;
+  float* x = c->x + b * g.C;
+  float* q = c->q + b * g.C;
+  float* hb = c->hbuf + b * g.I;
 
   PG_HIP(pgk::launch_embed(x, m->wte, m->wpe, tok_ptr, tok, (int)pos, C, s, m->w_bf16));
   PG_MARK(kNone);  // the embedding is in no bucket (rust.rs:966-974)
@@ -239,37 +281,7 @@ pg_status enqueue_forward_one(const pg_model* m, pg_kv_cache* c, size_t b,
     a.pos = (int)pos; a.P = P; a.C = C; a.head_dim = hd;
     PG_HIP(pgk::launch_gemv(a, pgk::PRO_LN, pgk::EPI_QKV, s));
     PG_MARK(kQkv);
-    // attention over keys [0, pos]
-    PG_HIP(pgk::launch_attn_decode(q, c->k_panel(l, b), c->v_panel(l, b), (int)pos, P, H, hd,
-                                   nsplit, pa, pm, pl, s));
-    if (!(nsplit > 2 && hd == pgk::kHeadDim)) PG_MARK(kAttention);
-    // merge splits + c_proj + residual.  Every block of the projection repeats the merge in
-    // its prologue, which is cheap for a few splits; beyond that the merge gets a launch of
-    // its own (into q, which the attention has finished reading).
-    a = pgk::GemvArgs{};
-    a.w_bf16 = m->w_bf16; a.W = w.c_proj_w; a.w_scale = w.c_proj_s; a.bias = w.c_proj_b; a.y = x; a.resid = x; a.K = C; a.nout = C;
-    if (nsplit > 2 && hd == pgk::kHeadDim) {
-      PG_HIP(pgk::launch_attn_finish(pa, pm, pl, H, hd, nsplit, q, s));
-      PG_MARK(kAttention);
-      a.x = q;
-      PG_HIP(pgk::launch_gemv(a, pgk::PRO_NONE, pgk::EPI_RESID, s));
-    } else {
-      a.part_acc = pa; a.part_m = pm; a.part_l = pl; a.nsplit = nsplit; a.head_dim = hd;
-      PG_HIP(pgk::launch_gemv(a, pgk::PRO_ATTN_COMBINE, pgk::EPI_RESID, s));
-    }
-    PG_MARK(kAttnProj);
-    // LN2 + c_fc + GELU
-    a = pgk::GemvArgs{};
-    a.w_bf16 = m->w_bf16; a.W = w.c_fc_w; a.w_scale = w.c_fc_s; a.bias = w.c_fc_b; a.x = x; a.y = hb; a.K = C; a.nout = I;
-    a.ln_g = w.ln_2_g; a.ln_b = w.ln_2_b; a.eps = g.eps;
-    PG_HIP(pgk::launch_gemv(a, pgk::PRO_LN, pgk::EPI_GELU, s));
-    PG_MARK(kMlpFc);
-    // mlp c_proj + residual
-    a = pgk::GemvArgs{};
-    a.w_bf16 = m->w_bf16; a.W = w.c_proj_mlp_w; a.w_scale = w.c_proj_mlp_s; a.bias = w.c_proj_mlp_b; a.x = hb; a.y = x; a.resid = x; a.K = I;
-    a.nout = C;
-    PG_HIP(pgk::launch_gemv(a, pgk::PRO_NONE, pgk::EPI_RESID, s));
-    PG_MARK(kMlpProj);
+    if (pg_status e = enqueue_row_behind_qkv(m, c, b, l, x, q, hb, pos, marks)) return e;
   }
   if (want_logits) {
     pgk::GemvArgs a{};
@@ -280,6 +292,65 @@ pg_status enqueue_forward_one(const pg_model* m, pg_kv_cache* c, size_t b,
   }
   return PG_OK;
 }
+// Key splits of an attention launch of B sequences, one row each, over `keys` keys.
+// With at least one (sequence, head) pair per CU a block takes all keys of its pair and writes
+// the attention output itself: no partials and no merge launch (355M B = 16: -3.5 % per step
+// at 128..192 keys, -6 % at 300, -5 % at 600).  Beyond 256 keys only where the pairs fill whole
+// rounds of CUs: with 800 pairs on 256 CUs the longer serial chunks of the last, short round
+// cost more than the merge launch (XL B = 32 at 528 keys: +1.6 %).
+int batch_splits(const pg_model* m, int B, size_t keys, bool* one_split) {
+  const Cfg& g = m->cfg;
+  const int pairs = (int)g.H * B, rounds = (pairs + m->num_cus - 1) / m->num_cus;
+  const bool whole_rounds = (long)rounds * m->num_cus * 10 <= (long)pairs * 11;
+  *one_split = g.hd() == pgk::kHeadDim && pairs >= m->num_cus && (keys <= 256 || whole_rounds);
+  return *one_split || g.hd() != pgk::kHeadDim ? 1 : pgk::choose_nsplit((int)keys, pairs, m->num_cus, m->attn_blocks_per_cu);
+}
+
+// enqueue_row_behind_qkv for the last rows of sequences b .. b + nb - 1, n_seq rows each, in the last layer, and the norm of the logits'
+// input, [nb][C] to xn.  x: [nb * n_seq][C] as it was in front of the layer; qkv, att, hidden: overwritten.
+pg_status enqueue_rows_behind_qkv(const pg_model* m, pg_kv_cache* c, size_t b, size_t nb, size_t n_seq, const float* x, float* qkv,
+                                  float* att, float* hidden, float* xn, float* ws, size_t ws_floats, ProfileMarks* marks) {
+  const Cfg& g = m->cfg;
+  const int B = (int)nb, C = (int)g.C, I = (int)g.I, H = (int)g.H, hd = (int)g.hd();
+  hipStream_t s = c->stream;
+  const size_t l = g.L - 1, part = (size_t)H * pgk::kMaxSplits;
+  const pgk::LayerW& w = m->layers[l];
+  bool one_split;
+  const int nsplit = batch_splits(m, B, n_seq, &one_split);
+  pgk::BatchStrides bs;
+  bs.q = n_seq * 3 * g.C;
+  bs.kv = g.H * g.P * g.hd();
+  bs.part = part;
+  bs.out = g.C;
+  float *pa = c->part_acc + b * part * hd, *pm = c->part_m + b * part, *pl = c->part_l + b * part;
+  PG_HIP(pgk::launch_attn_decode(qkv + (n_seq - 1) * 3 * g.C, c->k_panel(l, b), c->v_panel(l, b), (int)n_seq - 1, (int)g.P, H, hd, nsplit,
+                                 pa, pm, pl, s, B, bs, 0, one_split ? att : nullptr));
+  if (!one_split) PG_HIP(pgk::launch_attn_finish(pa, pm, pl, H, hd, nsplit, att, s, B, bs));
+  PG_MARK(kAttention);
+  float* rows = qkv;  // (its queries have been read)
+  PG_HIP(hipMemcpy2DAsync(rows, g.C * sizeof(float), x + (n_seq - 1) * g.C, n_seq * g.C * sizeof(float), g.C * sizeof(float), nb,
+                          hipMemcpyDeviceToDevice, s));
+  auto gemm = [&](const float* A, const float* W, const float* bias, float* Cout, int N, int K, int epi, const float* ln_g,
+                  const float* ln_b) -> hipError_t {
+    pgk::GemmArgs a{};
+    a.A = A; a.w_bf16 = m->w_bf16; a.W = W; a.bias = bias; a.resid = Cout; a.C = Cout;
+    a.M = B; a.N = N; a.K = K; a.lda = K; a.ldc = N;
+    if (m->w_i8) a.w_scale = i8_scales_of(W, (size_t)N, (size_t)K);
+    a.ws = ws; a.ws_floats = ws_floats;
+    if (ln_g) { a.ln_out = xn; a.ln_g = ln_g; a.ln_b = ln_b; a.ln_eps = g.eps; }
+    a.split_items_per_cu = m->gemm_split_items;
+    a.b9_min_rows = m->gemm_b9_min_rows;
+    return pgk::launch_gemm(a, epi, m->num_cus, s);
+  };
+  PG_HIP(gemm(att, w.c_proj_w, w.c_proj_b, rows, C, C, pgk::GEMM_RESID, w.ln_2_g, w.ln_2_b));
+  PG_MARK(kAttnProj);
+  PG_HIP(gemm(xn, w.c_fc_w, w.c_fc_b, hidden, I, C, pgk::GEMM_GELU, nullptr, nullptr));
+  PG_MARK(kMlpFc);
+  PG_HIP(gemm(hidden, w.c_proj_mlp_w, w.c_proj_mlp_b, rows, C, I, pgk::GEMM_RESID, m->ln_f_g, m->ln_f_b));
+  PG_MARK(kMlpProj);
+  return PG_OK;
+}
+
 #undef PG_MARK
 
 // The tagged activation words live in uncached device memory: a word written by one
@@ -628,6 +699,12 @@ pg_status make_half_form(pg_model* m) {
   return PG_OK;
 }
 
+// From how many rows on a prompt's last layer goes on with the last row of every sequence alone: attention of one query, c_proj and the
+// MLP of a row read W as long as those of some tens of rows do.  us, whole and so: width 768, f32 rows, 37 rows 600 and 606, 200 835 and 829,
+// 1024 1833 and 1770; 1024, 24 rows 1061 and 1074, 32 x 8 2521 and 2460, 16 x 64 3458 and 3373; 1600, bf16 rows, 64 rows 2964 and
+// 2987, 32 x 512 105.0 ms and 103.3.  More sequences than a 32-row product takes would need tiles again.
+constexpr size_t kLastRowsMin = 128, kLastRowsTokens = 8, kLastRowsMost = 32;
+
 // Full-sequence forward of the nb sequences b .. b + nb - 1 over ids[nb][n] (each one
 // Gpt2Model::forward, src/models/gpt2/rust.rs:831-882, block_forward at 1053-1134) with MFMA
 // GEMMs over all nb * n rows at once and tiled causal attention per sequence; K and V of every
@@ -655,6 +732,9 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
   const bool cut = !half && !c->drawn && takes_cut_form(m, n);
   const bool cut_w = cut && T > 128 && !m->half.empty() && m->half[0].c_attn_cut;  // (64 rows and fewer: no faster)
   const int form_of = cut ? pgk::FORM_CUT : pgk::FORM_ROWS;
+  // Behind the last layer's keys and values only the last row of every sequence is read.  (Drawn streams keep the order of their sums.)
+  const bool last_rows = !all_logits_dst && !c->drawn && hd == pgk::kHeadDim && n >= kLastRowsMin && n_seq >= kLastRowsTokens &&
+                         nb <= kLastRowsMost;
   {
     auto form = [&](size_t cols) { return cut ? std::max(n * cols, pgk::cut_floats(n, cols)) : half ? pgk::half_floats(n, cols) : n * cols; };
     auto up = [](size_t v) { return (v + 63) / 64 * 64; };  // 256-byte boundaries
@@ -742,6 +822,13 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
     PG_HIP(gemm(XN.p, C, w.c_attn_w, w.c_attn_b, QKV.p, 3 * C, 3 * C, C, pgk::GEMM_BIAS, nullptr, nullptr, cut, 0,
                 hw.c_attn, hw.c_attn_mul));
     PG_MARK(kQkv);
+    if (last_rows && !next) {
+      PG_HIP(pgk::launch_keep_rows(QKV.p, Ts, C, P, c->k_panel(l, b), c->v_panel(l, b), s, (int)nb, g.H * g.P * g.hd()));
+      st = nb == 1 ? enqueue_row_behind_qkv(m, c, b, l, X.p + (n - 1) * g.C, QKV.p + (n - 1) * 3 * g.C, HB.p, n - 1, marks)
+                   : enqueue_rows_behind_qkv(m, c, b, nb, n_seq, X.p, QKV.p, ATT.p, HB.p, XN.p, WS.p, ws_floats, marks);
+      if (st) return st;
+      break;
+    }
     if (half || (cut && !m->half.empty()))
       PG_HIP(pgk::launch_attn_prefill_half(QKV.p, Ts, C, H, P, c->k_panel(l, b), c->v_panel(l, b), ATT.p, s, (int)nb,
                                            g.H * g.P * g.hd(), m->half[l].attn, pgk::attn_half_shape(Ts, H, (int)nb, m->num_cus),
@@ -774,10 +861,12 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
     PG_HIP(pgk::launch_gemv(a, pgk::PRO_LN, pgk::EPI_BIAS, s));
   } else {
     // the nb last rows, gathered and normalised, against wte in one projection
-    PG_HIP(hipMemcpy2DAsync(ATT.p, g.C * sizeof(float), X.p + (n_seq - 1) * g.C,
-                            n_seq * g.C * sizeof(float), g.C * sizeof(float), nb,
-                            hipMemcpyDeviceToDevice, s));
-    PG_HIP(pgk::launch_layer_norm_rows(ATT.p, XN.p, (int)nb, C, m->ln_f_g, m->ln_f_b, g.eps, s));
+    if (!last_rows) {
+      PG_HIP(hipMemcpy2DAsync(ATT.p, g.C * sizeof(float), X.p + (n_seq - 1) * g.C,
+                              n_seq * g.C * sizeof(float), g.C * sizeof(float), nb,
+                              hipMemcpyDeviceToDevice, s));
+      PG_HIP(pgk::launch_layer_norm_rows(ATT.p, XN.p, (int)nb, C, m->ln_f_g, m->ln_f_b, g.eps, s));
+    }
     pgk::GemmArgs a{};
     a.A = XN.p; a.w_bf16 = m->w_bf16; a.W = m->lm_w; a.bias = nullptr; a.resid = nullptr;
     a.C = c->logits_buf + b * g.V;
@@ -804,17 +893,8 @@ pg_status enqueue_forward_batch(const pg_model* m, pg_kv_cache* c, const uint32_
   const int B = (int)c->B, C = (int)g.C, I = (int)g.I, H = (int)g.H, hd = (int)g.hd(),
             P = (int)g.P;
   hipStream_t s = c->stream;
-  // With at least one (sequence, head) pair per CU a block takes all keys of its pair and writes
-  // the attention output itself: no partials and no merge launch (355M B = 16: -3.5 % per step
-  // at 128..192 keys, -6 % at 300, -5 % at 600).  Beyond 256 keys only where the pairs fill whole
-  // rounds of CUs: with 800 pairs on 256 CUs the longer serial chunks of the last, short round
-  // cost more than the merge launch (XL B = 32 at 528 keys: +1.6 %).
-  const int pairs = H * B, rounds = (pairs + m->num_cus - 1) / m->num_cus;
-  const bool whole_rounds = (long)rounds * m->num_cus * 10 <= (long)pairs * 11;
-  const bool one_split =
-      hd == pgk::kHeadDim && pairs >= m->num_cus && (pos + 1 <= 256 || whole_rounds);
-  const int nsplit = hd != pgk::kHeadDim ? 1 : one_split
-                         ? 1 : pgk::choose_nsplit((int)pos + 1, H * B, m->num_cus, m->attn_blocks_per_cu);
+  bool one_split;
+  const int nsplit = batch_splits(m, B, pos + 1, &one_split);
   pgk::BatchStrides bs;
   bs.q = 3 * g.C;
   bs.kv = g.H * g.P * g.hd();

@@ -187,6 +187,9 @@ hipError_t launch_embed_batch(float* x, const float* wte, const float* wpe, cons
 hipError_t launch_kv_append(const float* qkv, int batch, int C, int head_dim, int P, int pos,
                             float* kcache, float* vcache, size_t kv_stride, hipStream_t s);
 
+// Keys and values of T rows of each of nseq sequences (qkv [nseq][T][3C], 64 values a head) to positions 0 .. T - 1 of their panels.
+hipError_t launch_keep_rows(const float* qkv, int T, int C, int P, float* kcache, float* vcache, hipStream_t s, int nseq, size_t kv_stride);
+
 // Stand-alone forms of the cpu.rs ops (rows handled one block each).
 hipError_t launch_layer_norm(float* x, int rows, int cols, const float* g, const float* b,
                              float eps, hipStream_t s);

@@ -1253,6 +1253,15 @@ __global__ void k_kv_append(const float* qkv, int C, int hd, int P, int pos, flo
   vcache[dst] = qkv[(size_t)b * 3 * C + 2 * C + c];
 }
 
+__global__ __launch_bounds__(256) void k_keep_rows(const float* qkv, int C, int P, float* kcache, float* vcache, size_t kv_stride) {
+  const int t = blockIdx.x, c = 4 * ((int)blockIdx.y * 256 + (int)threadIdx.x);
+  if (c >= C) return;
+  const float* row = qkv + ((size_t)blockIdx.z * gridDim.x + t) * 3 * C + c;
+  const size_t dst = blockIdx.z * kv_stride + ((size_t)(c / 64) * P + t) * 64 + c % 64;
+  *reinterpret_cast<float4*>(kcache + dst) = *reinterpret_cast<const float4*>(row + C);
+  *reinterpret_cast<float4*>(vcache + dst) = *reinterpret_cast<const float4*>(row + 2 * C);
+}
+
 // ---- stand-alone cpu.rs ops -------------------------------------------------
 
 __global__ __launch_bounds__(kBlock) void k_layer_norm(float* x, int cols, const float* g,
@@ -1564,6 +1573,11 @@ hipError_t launch_kv_append(const float* qkv, int batch, int C, int head_dim, in
                             float* kcache, float* vcache, size_t kv_stride, hipStream_t s) {
   hipLaunchKernelGGL(k_kv_append, dim3((C + 255) / 256, batch), dim3(256), 0, s, qkv, C, head_dim,
                      P, pos, kcache, vcache, kv_stride);
+  return hipGetLastError();
+}
+
+hipError_t launch_keep_rows(const float* qkv, int T, int C, int P, float* kcache, float* vcache, hipStream_t s, int nseq, size_t kv_stride) {
+  hipLaunchKernelGGL(k_keep_rows, dim3(T, (C / 4 + 255) / 256, nseq), dim3(256), 0, s, qkv, C, P, kcache, vcache, kv_stride);
   return hipGetLastError();
 }
 

@@ -1,0 +1,33 @@
+"""Prompts whose last layer goes on with the rows that logits are wanted of: both sides of where that begins, what the cache
+holds afterwards, and the steps that follow."""
+import numpy as np
+import pytest
+
+import oracle
+from helpers import assert_logits_close
+from puppygrad_amd import Gpt2Config, Gpt2HipConfig, Gpt2Model, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("storage", [0, 1, 2], ids=["f32", "bf16", "int8"])
+@pytest.mark.parametrize("B,n", [(1, 127), (1, 128), (1, 300), (2, 63), (2, 64), (3, 70), (8, 33), (15, 8), (16, 8),
+                                  (32, 7), (32, 9), (33, 9)])
+def test_prompts(B, n, storage):
+    cfg = Gpt2Config(vocab_size=131, n_positions=304, n_embd=128, n_layer=2, n_head=2)
+    w = synth.random_weights(cfg, 0x5EED0D00, perturb=True)
+    ids = synth.token_ids(B * n, 0x70C00D00 + n, cfg.vocab_size).reshape(B, n)
+    model = Gpt2Model.new(cfg, w, Gpt2HipConfig(weight_storage=storage))
+    ref = oracle.Model(cfg, synth.bf16_rounded(w) if storage == 1 else w, oracle.rust_config(8, quantized_weights=int(storage == 2)))
+    cache = model.new_kv_cache(B)
+    got = model.prefill_batch(ids, cache).to_host() if B > 1 else model.prefill(ids[0], cache).to_host()[None]
+    some = sorted({0, B // 2, B - 1})
+    rcs = {b: ref.new_kv_cache() for b in some}
+    for b in some:
+        assert_logits_close(got[b], ref.prefill(ids[b], rcs[b]))
+        for kv in (0, 1):
+            np.testing.assert_allclose(cache.read_layer(1, kv, b)[:, :n], rcs[b].read_layer(1, kv)[:, :n], atol=2e-5, rtol=1e-4)
+    nxt = ids[:, 0]
+    got = model.forward_one_batch(nxt, cache).to_host() if B > 1 else model.forward_one(int(nxt[0]), cache).to_host()[None]
+    for b in some:
+        assert_logits_close(got[b], ref.forward_one(int(nxt[b]), rcs[b]))
