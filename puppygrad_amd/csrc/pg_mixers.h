@@ -179,6 +179,9 @@ hipError_t launch_add_norm_rows(float* dst, const float* src, int rows, int cols
 hipError_t launch_group_rms_rows(const float* src, int ld_src, float* dst, int ld_dst, int rows, int cols, int groups,
                                  const float* gain, float eps, const int* rows_at, hipStream_t s);
 
+// dst[r] = src[rows_at[r]], rows of ld floats (a multiple of 4).
+hipError_t launch_take_rows(const float* src, float* dst, int rows, int ld, const int* rows_at, hipStream_t s);
+
 // ---- latent attention (pg_latent.hip) ----
 // Keys and values of all heads come from one latent row c[kv_rank] per position and a rotated
 // part r[rot_dim] shared by the heads: the score of query head h is (q_h . (W_uk_h c) + q'_h . r) *

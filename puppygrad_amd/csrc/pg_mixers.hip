@@ -1642,6 +1642,12 @@ __global__ __launch_bounds__(256) void k_group_rms_rows(const float* src, int ld
   for (int i = cols + tid; i < ld_dst; i += 256) y[i] = 0.0f;
 }
 
+__global__ __launch_bounds__(256) void k_take_rows(const float* src, float* dst, int ld, const int* rows_at) {
+  const int i = 4 * ((int)blockIdx.y * 256 + (int)threadIdx.x);
+  if (i < ld)
+    *reinterpret_cast<float4*>(dst + (size_t)blockIdx.x * ld + i) = *reinterpret_cast<const float4*>(src + (size_t)rows_at[blockIdx.x] * ld + i);
+}
+
 __global__ __launch_bounds__(256) void k_begin_step(float* x, const void* table, int table_bf16, const uint32_t* ids,
                                                     int width, StepWords* words) {
   const int b = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;
@@ -1903,6 +1909,11 @@ hipError_t launch_group_rms_rows(const float* src, int ld_src, float* dst, int l
   return hipGetLastError();
 }
 
+hipError_t launch_take_rows(const float* src, float* dst, int rows, int ld, const int* rows_at, hipStream_t s) {
+  if (ld % 4 != 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_take_rows, dim3(rows, (ld / 4 + 255) / 256), dim3(256), 0, s, src, dst, ld, rows_at);
+  return hipGetLastError();
+}
 hipError_t launch_begin_step(float* x, const void* table, int table_bf16, const uint32_t* ids, int nseq, int width,
                              StepWords* words, hipStream_t s) {
   hipLaunchKernelGGL(k_begin_step, dim3((width + 255) / 256, nseq), dim3(256), 0, s, x, table, table_bf16, ids, width,

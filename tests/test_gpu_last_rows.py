@@ -5,7 +5,10 @@ import pytest
 
 import oracle
 from helpers import assert_logits_close
+from oracle import movudra
 from puppygrad_amd import Gpt2Config, Gpt2HipConfig, Gpt2Model, synth
+from stack_helpers import Pair, check
+from test_gpu_movudra import MIXED, config, delta, latent, mamba, moe, weights
 
 pytestmark = pytest.mark.gpu
 
@@ -31,3 +34,34 @@ def test_prompts(B, n, storage):
     got = model.forward_one_batch(nxt, cache).to_host() if B > 1 else model.forward_one(int(nxt[0]), cache).to_host()[None]
     for b in some:
         assert_logits_close(got[b], ref.forward_one(int(nxt[b]), rcs[b]))
+
+
+# (a last layer with experts, with a dense feed-forward and with none)
+LAST = [config([delta(), mamba(mlp=moe(5, 3, 20))]), MIXED, config([mamba(), latent()])]
+
+
+@pytest.fixture(scope="module", params=range(len(LAST)), ids=["experts", "dense", "none"])
+def pair(request, tmp_path_factory):
+    return Pair(movudra, tmp_path_factory.mktemp("last"), LAST[request.param], weights(LAST[request.param], 17))
+
+
+# (5e-5: what models of six layers are held to, whichever rows are wanted)
+@pytest.mark.parametrize("n,wanted", [(40, []), (3, [2]), (4, [3]), (4, [0]), (7, [2, 5]), (8, [2, 5]), (131, range(99, 131)),
+                                      (127, range(95, 127)), (140, range(0, 132, 4))])
+def test_wanted_rows(pair, n, wanted):
+    ids, wanted = pair.ids(n + 2, seed=n), list(wanted)
+    want = pair.ref.run(ids)
+    cache = pair.dev.new_kv_cache()
+    got = pair.dev.extend(ids[:n], cache, wanted)
+    if wanted:
+        check(got.to_host().reshape(len(wanted), -1), want[wanted], 5e-5)
+    check(pair.dev.extend(ids[n:], cache, [0, 1]).to_host(), want[n:], 5e-5)
+
+
+@pytest.mark.parametrize("B,n", [(2, 3), (2, 4), (5, 21), (32, 5), (33, 5)])
+def test_batches(pair, B, n):
+    ids = np.array([pair.ids(n, seed=100 + b) for b in range(B)], np.uint32)
+    cache = pair.dev.new_kv_cache(B)
+    got = pair.dev.prefill_batch(ids, cache).to_host()
+    for b in sorted({0, B // 2, B - 1}):
+        check(got[b], pair.ref.run([int(t) for t in ids[b]])[-1:], 5e-5)
