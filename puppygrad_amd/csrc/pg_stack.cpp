@@ -1164,6 +1164,27 @@ pg_status post_norm_step(const pg_model* model, pg_kv_cache* c, ProfileMarks* ma
   return PG_OK;
 }
 
+// A row of a layer of parallel sublayers back to the residual: x += ls1 (W_out mix) + ls2 (W_down act), where the two fit one launch,
+// else without the second.
+pgk::GemvPair pair_of(const pg_model* model, const StackLayer& l, float* x, const float* mix, const float* act) {
+  pgk::GemvPair p{};
+  p.w_bf16 = model->w_bf16;
+  p.num_cus = model->num_cus;
+  p.W1 = l.out_w; p.x1 = mix; p.s1 = l.ls1; p.K1 = l.mix_pad;
+  p.resid = x; p.y = x; p.nout = model->stack->width_pad;
+  if (l.has_mlp && l.mix_pad + l.mlp.ff_pad <= pgk::kPairMaxK) {
+    p.W2 = l.down_w; p.x2 = act; p.s2 = l.ls2; p.K2 = l.mlp.ff_pad;
+  }
+  return p;
+}
+hipError_t launch_pair(pgk::GemvPair p, const StackLayer& l, const float* act, hipStream_t s) {
+  const hipError_t e = pgk::launch_gemv_pair(p, s);
+  if (e != hipSuccess || !l.has_mlp || p.W2) return e;
+  p.W1 = l.down_w; p.x1 = act; p.s1 = l.ls2; p.K1 = l.mlp.ff_pad;  // (too wide for one launch)
+  p.part_splits = 0;
+  return pgk::launch_gemv_pair(p, s);
+}
+
 pg_status step_launches(const pg_model* model, pg_kv_cache* c, ProfileMarks* marks) {
   const StackModel& m = *model->stack;
   if (m.post_norm) return post_norm_step(model, c, marks);
@@ -1195,15 +1216,7 @@ pg_status step_launches(const pg_model* model, pg_kv_cache* c, ProfileMarks* mar
     d.attn = b.attn; d.rec = b.rec; d.mlp = l.mlp;
     d.attn_splits = l.has_attn ? pgk::mix_decode_splits(l.attn, l.has_rec ? &l.rec : nullptr) : 1;
     d.part = st.part;
-    pgk::GemvPair p{};
-    p.w_bf16 = model->w_bf16;
-    p.num_cus = model->num_cus;
-    p.W1 = l.out_w; p.x1 = st.mix; p.s1 = l.ls1; p.K1 = l.mix_pad;
-    p.resid = st.x; p.y = st.x; p.nout = Cp;
-    const bool both = l.has_mlp && l.mix_pad + l.mlp.ff_pad <= pgk::kPairMaxK;
-    if (both) {
-      p.W2 = l.down_w; p.x2 = st.act; p.s2 = l.ls2; p.K2 = l.mlp.ff_pad;
-    }
+    pgk::GemvPair p = pair_of(model, l, st.x, st.mix, st.act);
     if (B == 1) d.ahead = pgk::gemv_pair_ahead(p);
     PG_HIP(pgk::launch_mix_decode(d, s));
     // the attention's key splits are added by the projection of the one-sequence step, where
@@ -1217,12 +1230,7 @@ pg_status step_launches(const pg_model* model, pg_kv_cache* c, ProfileMarks* mar
         p.part = st.part; p.part_splits = d.attn_splits; p.part_n = l.attn.heads * l.attn.dim;
         p.part_col = l.attn.out_col;
       }
-      PG_HIP(pgk::launch_gemv_pair(p, s));
-      if (l.has_mlp && !both) {  // (too wide for one launch)
-        p.W1 = l.down_w; p.x1 = st.act; p.s1 = l.ls2; p.K1 = l.mlp.ff_pad;
-        p.part_splits = 0;
-        PG_HIP(pgk::launch_gemv_pair(p, s));
-      }
+      PG_HIP(launch_pair(p, l, st.act, s));
       PG_MARK(kMlpProj);
     } else {
       float* next_h = more ? st.h : nullptr;
@@ -1325,6 +1333,15 @@ pg_status wanted_rows(const pg_model* model, StackCache& st, Gemm gemm, const fl
   gemm.rows = (int)want.size();
   return head_rows(model, gemm, x, h, st.rows_at, dst);
 }
+// Whether the last layer, behind whose mixers only the rows whose logits are wanted are read, goes on with those alone: `cols` values of
+// each of them lie where the projections, max_in a row, did.  Several are gathered first, which pays from `each` rows to a wanted one
+// on.  Prompts and 2 tokens, ms, all rows and so: Movudra at 1600, 32 x 100 11.18 and 10.76, 1000 4.32 and 4.16, 16 1.80 and 1.78, at 1280
+// 20 x 8 3.49 and 3.47; parallel sublayers at 1600, 32 x 100 9.99 and 9.80, 1000 3.57 and 3.51, at 768 8 x 20 1.544 and 1.558, 4 x
+// 100 1.586 and 1.634 (2048 rows are needed there).  Up to 32 rows one product reads W once; drawn streams keep the order of their sums.
+bool few_rows(const pg_kv_cache* c, const std::vector<int>& want, size_t rows, size_t cols, int max_in, size_t each) {
+  return !c->drawn && want.size() <= 32 && (want.size() > 1 ? each : 4) * want.size() <= rows && want.size() * cols <= rows * (size_t)max_in;
+}
+
 
 // rows_segment for post-norm layers.
 pg_status post_norm_rows(const pg_model* model, pg_kv_cache* c, const uint32_t* d_ids, size_t n, size_t pos0,
@@ -1333,12 +1350,8 @@ pg_status post_norm_rows(const pg_model* model, pg_kv_cache* c, const uint32_t* 
   StackCache& st = *c->stack;
   hipStream_t s = c->stream;
   const size_t B = c->B, rows = B * n, Cp = (size_t)m.width_pad;
-  // Behind the last layer's mixer only the rows whose logits are wanted are read.  (Prompts at width 1600 and 2 tokens, ms, all rows
-  // and so: 32 x 100 11.18 and 10.76, 1000 4.32 and 4.16, 16 1.80 and 1.78; 20 x 8 at 1280 3.49 and 3.47.  Up to 32 rows one product reads
-  // W once; drawn streams keep the order of their sums.)
   const int W = (int)want.size();
-  const bool few = !c->drawn && W <= 32 && 4 * want.size() <= rows &&
-                   (size_t)W * (Cp + m.layers.back().mix_pad) <= rows * (size_t)m.max_in;
+  const bool few = few_rows(c, want, rows, Cp + m.layers.back().mix_pad, m.max_in, 4);
   size_t work_floats = 0, lat_floats = 0, kv_floats = 0, act_floats = 0;
   MoeSizes ms;
   for (const StackLayer& l : m.layers) {
@@ -1453,6 +1466,10 @@ pg_status rows_segment(const pg_model* model, pg_kv_cache* c, const uint32_t* d_
   StackCache& st = *c->stack;
   hipStream_t s = c->stream;
   const size_t B = c->B, rows = B * n, Cp = (size_t)m.width_pad;
+  const StackLayer& last = m.layers.back();
+  const int W = (int)want.size();
+  const bool few = few_rows(c, want, rows, Cp + last.mix_pad + (last.has_mlp ? last.mlp.ff_pad : 0), m.max_in,
+                            std::max<size_t>(32, 2048 / std::max(W, 1)));
   const size_t ws_floats = 8 * rows * Cp;
   float *x, *h, *y, *mix, *act, *krot, *conv, *decay, *work, *ws, *ws_side;
   size_t work_floats = 0;
@@ -1479,7 +1496,7 @@ pg_status rows_segment(const pg_model* model, pg_kv_cache* c, const uint32_t* d_
     r.out = mix; r.ld_out = l.mix_pad; r.out_cols = l.mix_cols;
     r.act = act; r.k_rot = krot; r.conv_out = conv; r.decay = decay;
     r.work = work; r.work_floats = work_floats;
-    const bool more = i + 1 < m.layers.size();
+    const bool more = i + 1 < m.layers.size(), whole = more || !few;
     float* next_h = more ? h : nullptr;
     const float* next_g = more ? m.layers[i + 1].norm : nullptr;
     // The recurrence is a chain over the tokens that leaves most of the chip idle: with enough
@@ -1502,7 +1519,7 @@ pg_status rows_segment(const pg_model* model, pg_kv_cache* c, const uint32_t* d_
     if (l.has_mlp) {
       PG_HIP(pgk::launch_gated_mlp_rows(r, l.mlp, side));
       PG_MARK(kMlpFc);
-      PG_HIP(side_gemm(act, l.down_w, x, (int)Cp, l.mlp.ff_pad, l.ls2, nullptr, nullptr));
+      if (whole) PG_HIP(side_gemm(act, l.down_w, x, (int)Cp, l.mlp.ff_pad, l.ls2, nullptr, nullptr));
       PG_MARK(kMlpProj);
     }
     if (l.has_rec) {
@@ -1515,10 +1532,34 @@ pg_status rows_segment(const pg_model* model, pg_kv_cache* c, const uint32_t* d_
       PG_HIP(hipStreamWaitEvent(s, st.joined, 0));
     }
     PG_MARK(kAttention);
+    if (!whole) break;
     PG_HIP(gemm(mix, l.out_w, x, (int)Cp, l.mix_pad, l.ls1, next_g, next_h));
     PG_MARK(kAttnProj);
   }
-  if (pg_status e = wanted_rows(model, st, gemm, x, h, want, dst)) return e;
+  if (few && W == 1) {
+    x += (size_t)want[0] * Cp, mix += (size_t)want[0] * last.mix_pad;
+    if (last.has_mlp) act += (size_t)want[0] * last.mlp.ff_pad;
+    PG_HIP(launch_pair(pair_of(model, last, x, mix, act), last, act, s));
+    PG_MARK(kAttnProj);
+    if (pg_status e = head_one(model, x, dst, s)) return e;
+  } else if (few && W > 0) {
+    if (pg_status e = send_rows_at(st, want, s)) return e;
+    float *some_x = y, *some_mix = some_x + (size_t)W * Cp, *some_act = some_mix + (size_t)W * last.mix_pad;  // (y has been read)
+    Gemm some = gemm;
+    some.rows = W;
+    PG_HIP(pgk::launch_take_rows(x, some_x, W, (int)Cp, st.rows_at, s));
+    PG_HIP(pgk::launch_take_rows(mix, some_mix, W, last.mix_pad, st.rows_at, s));
+    PG_HIP(some(some_mix, last.out_w, some_x, (int)Cp, last.mix_pad, last.ls1, nullptr, nullptr));
+    PG_MARK(kAttnProj);
+    if (last.has_mlp) {
+      PG_HIP(pgk::launch_take_rows(act, some_act, W, last.mlp.ff_pad, st.rows_at, s));
+      PG_HIP(some(some_act, last.down_w, some_x, (int)Cp, last.mlp.ff_pad, last.ls2, nullptr, nullptr));
+      PG_MARK(kMlpProj);
+    }
+    if (pg_status e = head_rows(model, some, some_x, h, nullptr, dst)) return e;
+  } else if (pg_status e = wanted_rows(model, st, gemm, x, h, want, dst)) {
+    return e;
+  }
   PG_MARK(kLogits);
   return PG_OK;
 }

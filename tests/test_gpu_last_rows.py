@@ -4,8 +4,9 @@ import numpy as np
 import pytest
 
 import oracle
+import test_gpu_tarepel as other
 from helpers import assert_logits_close
-from oracle import movudra
+from oracle import movudra, tarepel
 from puppygrad_amd import Gpt2Config, Gpt2HipConfig, Gpt2Model, synth
 from stack_helpers import Pair, check
 from test_gpu_movudra import MIXED, config, delta, latent, mamba, moe, weights
@@ -36,18 +37,24 @@ def test_prompts(B, n, storage):
         assert_logits_close(got[b], ref.forward_one(int(nxt[b]), rcs[b]))
 
 
-# (a last layer with experts, with a dense feed-forward and with none)
-LAST = [config([delta(), mamba(mlp=moe(5, 3, 20))]), MIXED, config([mamba(), latent()])]
+# (a last layer with experts, with a dense feed-forward and with none; one of parallel sublayers, of two kinds, without its MLP, and
+# with one too wide for a launch together with the mixers)
+LAST = {"experts": config([delta(), mamba(mlp=moe(5, 3, 20))]), "dense": MIXED, "none": config([mamba(), latent()]),
+        "parallel": other.config([other.gla(), other.parallel()]), "gla": other.config([other.parallel(), other.gla()]),
+        "no-mlp": other.config([other.gla(), other.parallel(ff=None)]), "wide": other.config([other.parallel(ff=16300)])}
 
 
-@pytest.fixture(scope="module", params=range(len(LAST)), ids=["experts", "dense", "none"])
+@pytest.fixture(scope="module", params=LAST)
 def pair(request, tmp_path_factory):
-    return Pair(movudra, tmp_path_factory.mktemp("last"), LAST[request.param], weights(LAST[request.param], 17))
+    cfg = LAST[request.param]
+    orc, make = (movudra, weights) if cfg["architecture"] == "Movudra" else (tarepel, other.weights)
+    return Pair(orc, tmp_path_factory.mktemp("last"), cfg, make(cfg, 17))
 
 
 # (5e-5: what models of six layers are held to, whichever rows are wanted)
 @pytest.mark.parametrize("n,wanted", [(40, []), (3, [2]), (4, [3]), (4, [0]), (7, [2, 5]), (8, [2, 5]), (131, range(99, 131)),
-                                      (127, range(95, 127)), (140, range(0, 132, 4))])
+                                      (127, range(95, 127)), (140, range(0, 132, 4)),
+                                      (2047, [1, 2046]), (2048, [1, 2046])])
 def test_wanted_rows(pair, n, wanted):
     ids, wanted = pair.ids(n + 2, seed=n), list(wanted)
     want = pair.ref.run(ids)
@@ -58,7 +65,7 @@ def test_wanted_rows(pair, n, wanted):
     check(pair.dev.extend(ids[n:], cache, [0, 1]).to_host(), want[n:], 5e-5)
 
 
-@pytest.mark.parametrize("B,n", [(2, 3), (2, 4), (5, 21), (32, 5), (33, 5)])
+@pytest.mark.parametrize("B,n", [(2, 3), (2, 4), (5, 21), (32, 5), (33, 5), (32, 63), (32, 64)])
 def test_batches(pair, B, n):
     ids = np.array([pair.ids(n, seed=100 + b) for b in range(B)], np.uint32)
     cache = pair.dev.new_kv_cache(B)
