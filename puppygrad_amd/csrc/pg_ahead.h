@@ -12,6 +12,9 @@
 
 namespace pgk {
 
+// No weights to read ahead (a branch for them in the launches that have none cost 0.2 to 0.7 us each).
+struct Nothing {};
+
 constexpr unsigned kDies = 8;  // block i of a launch runs on die i % kDies, and each die has a cache (4 MB) of its own
 constexpr unsigned kAheadLine = 128;
 
@@ -22,6 +25,7 @@ struct Ahead {
   const void* at[2] = {nullptr, nullptr};
   unsigned slabs[2] = {0, 0}, slab_bytes[2] = {0, 0}, group_bytes[2] = {0, 0}, lines[2] = {1, 1}, words[2] = {1, 1};
   int blocks = 0;
+  size_t total() const { return (size_t)slabs[0] * slab_bytes[0] + (size_t)slabs[1] * slab_bytes[1]; }
   void matrix(int k, const void* from, size_t n_slabs, size_t slab, size_t group) {
     at[k] = from;
     slabs[k] = (unsigned)n_slabs, slab_bytes[k] = (unsigned)slab, group_bytes[k] = (unsigned)group;

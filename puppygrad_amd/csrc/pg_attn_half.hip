@@ -35,11 +35,11 @@ __device__ __forceinline__ void halves8(f4 a, f4 b, u4v (&part)[2]) {
 // tokens, 12 heads 29.5 (k_attn_prefill64) -> 27 (with one power of two for all of Q, of K and of V 32 and 25).  Error against f64,
 // values N(0, 1), 1.4 to 1.85 10^-7: 0.95 to 1.1 of the f32 cores' (queries three times as large 0.83 to 0.93), 1.5 of k_attn_prefill_cut's (1.2).
 // What bounds it: per tile and wavefront 768 clocks of matrix instructions and about 1100 of vector ones.  Grid: x = head, y = block of queries, longest rows first, z = sequence.
-template <int QG, int KG, int FORM>
+template <int QG, int KG, int FORM, typename Next = Nothing>
 __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const float* __restrict__ qkv, int T, int C, int P,
                                                                       float* __restrict__ kcache,
                                                                       float* __restrict__ vcache,
-                                                                      void* __restrict__ out, size_t kv_stride, HalfScales scales) {
+                                                                      void* __restrict__ out, size_t kv_stride, HalfScales scales, Next next) {
   constexpr int NW = QG * KG;
   constexpr int KSTR = 32 * 16 + 16;            // bytes of an octet of dims of 32 keys, padded
   constexpr int KPART = 8 * KSTR, VPART = 4 * 64 * 16;
@@ -49,6 +49,14 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void k_attn_prefill_half(const flo
   __shared__ __attribute__((aligned(16))) char lds[LDS];
   __shared__ float Ms[NW][32], Ls[NW][32];
   __shared__ __attribute__((aligned(16))) float Ks[2][QG == 1 ? 64 : 1];  // K's and V's powers where there are no registers for them
+  if constexpr (std::is_same_v<Next, Ahead>) {  // one sequence: the rows of blocks behind those of queries (attention of 37 tokens by
+    // 20 heads is 20 blocks and 6.7 us; c_fc behind it, 13 MB from HBM, 9.7)
+    const int first = (T + 32 * QG - 1) / (32 * QG) * (int)gridDim.x, id = (int)(blockIdx.x + gridDim.x * blockIdx.y);
+    if (id >= first) {
+      if (id - first < next.blocks) read_ahead(next, id - first, (unsigned)id, 64 * NW);
+      return;
+    }
+  }
   qkv += (size_t)blockIdx.z * T * 3 * C;
   kcache += (size_t)blockIdx.z * kv_stride;
   vcache += (size_t)blockIdx.z * kv_stride;
@@ -291,9 +299,9 @@ hipError_t start(const float* qkv, int T, int C, int H, int P, float* kcache, fl
                  size_t kv_stride, const HalfScales& f, int out_form) {
   const dim3 grid(H, (T + 32 * QG - 1) / (32 * QG), nseq), block(64 * QG * KG);
   if (out_form == FORM_HALF)
-    hipLaunchKernelGGL((k_attn_prefill_half<QG, KG, FORM_HALF>), grid, block, 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, f);
+    hipLaunchKernelGGL((k_attn_prefill_half<QG, KG, FORM_HALF>), grid, block, 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, f, Nothing{});
   else
-    hipLaunchKernelGGL((k_attn_prefill_half<QG, KG, FORM_CUT>), grid, block, 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, f);
+    hipLaunchKernelGGL((k_attn_prefill_half<QG, KG, FORM_CUT>), grid, block, 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, f, Nothing{});
   return hipGetLastError();
 }
 }  // namespace
@@ -316,8 +324,13 @@ int attn_half_shape(int T, int H, int nseq, int num_cus) {
 }
 
 hipError_t launch_attn_prefill_half(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, void* out,
-                                    hipStream_t s, int nseq, size_t kv_stride, const HalfScales& f, int shape, int out_form) {
+                                    hipStream_t s, int nseq, size_t kv_stride, const HalfScales& f, int shape, int out_form, const Ahead* next) {
   if ((out_form != FORM_HALF && out_form != FORM_CUT) || nseq < 1 || nseq > 65535 || (reinterpret_cast<uintptr_t>(out) & 15)) return hipErrorInvalidValue;
+  if (next && next->blocks > 0 && nseq == 1 && shape == 22 && out_form == FORM_HALF) {
+    const dim3 grid(H, (T + 63) / 64 + (next->blocks + H - 1) / H);
+    hipLaunchKernelGGL((k_attn_prefill_half<2, 2, FORM_HALF, Ahead>), grid, dim3(256), 0, s, qkv, T, C, P, kcache, vcache, out, kv_stride, f, *next);
+    return hipGetLastError();
+  }
   switch (shape) {
     case 41: return start<4, 1>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, f, out_form);
     case 22: return start<2, 2>(qkv, T, C, H, P, kcache, vcache, out, s, nseq, kv_stride, f, out_form);

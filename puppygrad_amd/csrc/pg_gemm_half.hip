@@ -579,9 +579,15 @@ __global__ __launch_bounds__(256) void k_norm_rows_half(GemmArgs a, int parts) {
 
 // The same, a block a row, for few rows: everything a thread reads is requested before the first use.  Eight rows share cache
 // lines: their blocks are on one XCD (block % 8), whose L2 then writes whole lines back.  NQ: 1024 NQ >= N.
-template <int NQ, bool PARTS, int PX>
-__global__ __launch_bounds__(256) void k_norm_row_half(GemmArgs a, int parts) {
+template <int NQ, bool PARTS, int PX, typename Next = Nothing>
+__global__ __launch_bounds__(256) void k_norm_row_half(GemmArgs a, int parts, Next next) {
   __shared__ float red[2][4];
+  if constexpr (std::is_same_v<Next, Ahead>) {
+    if ((int)blockIdx.x >= (a.M + 63) / 64 * 64) {
+      read_ahead(next, (int)blockIdx.x - (a.M + 63) / 64 * 64, blockIdx.x, 256);
+      return;
+    }
+  }
   const int m = (int)blockIdx.x / 64 * 64 + (int)blockIdx.x % 8 * 8 + (int)blockIdx.x % 64 / 8;
   if (m >= a.M) return;
   const int n4 = a.N / 4;
@@ -643,9 +649,15 @@ hipError_t launch_norm(const GemmArgs& a, int parts, hipStream_t s) {
   if (a.N % 8 != 0 || a.N > kNormWidest || a.ldc != a.N) return hipErrorInvalidValue;
   if (a.M <= kNormRowMax) {
     const dim3 rows((unsigned)((a.M + 63) / 64 * 64));
-    if (a.N <= 1024) hipLaunchKernelGGL((k_norm_row_half<1, PARTS, PX>), rows, dim3(256), 0, s, a, parts);
-    else if (a.N <= 2048) hipLaunchKernelGGL((k_norm_row_half<2, PARTS, PX>), rows, dim3(256), 0, s, a, parts);
-    else hipLaunchKernelGGL((k_norm_row_half<4, PARTS, PX>), rows, dim3(256), 0, s, a, parts);
+    if constexpr (PARTS && PX == 2) {
+      if (a.ahead && a.ahead->blocks > 0 && a.N > 1024 && a.N <= 2048) {  // (narrower models have too few bytes to read ahead here)
+        hipLaunchKernelGGL((k_norm_row_half<2, PARTS, PX, Ahead>), dim3(rows.x + a.ahead->blocks), dim3(256), 0, s, a, parts, *a.ahead);
+        return hipGetLastError();
+      }
+    }
+    if (a.N <= 1024) hipLaunchKernelGGL((k_norm_row_half<1, PARTS, PX>), rows, dim3(256), 0, s, a, parts, Nothing{});
+    else if (a.N <= 2048) hipLaunchKernelGGL((k_norm_row_half<2, PARTS, PX>), rows, dim3(256), 0, s, a, parts, Nothing{});
+    else hipLaunchKernelGGL((k_norm_row_half<4, PARTS, PX>), rows, dim3(256), 0, s, a, parts, Nothing{});
     return hipGetLastError();
   }
   const dim3 grid((unsigned)((a.M + 63) / 64 * 16));
@@ -1031,6 +1043,12 @@ hipError_t launch_gemm_half_plan(const GemmArgs& a0, int epi, const HalfPlan& p,
   if (p.rows < 8 || p.rows % 8 != 0 || p.mt < 1) return hipErrorInvalidValue;
   a.rows_per_block = p.rows;
   return a.w_half_parts == 3 ? launch_rows<3, 3>(a, epi, p, s) : a.w_half_parts == 2 ? launch_rows<2, 2>(a, epi, p, s) : launch_rows<2, 1>(a, epi, p, s);
+}
+
+void gemm_half_ahead(const GemmArgs& a, int epi, int num_cus, int k, Ahead* to) {
+  if (!a.w_half || a.w_half_parts != 1) return;
+  const HalfPlan p = gemm_half_plan(a, epi, num_cus);
+  if (p.tile == HALF_ROWS && a.M <= 16 * p.mt) to->matrix(k, a.w_half, a.K / 8, (size_t)a.N * 16, (size_t)p.rows * 16);
 }
 
 hipError_t launch_gemm_half(const GemmArgs& a, int epi, int num_cus, hipStream_t s) {

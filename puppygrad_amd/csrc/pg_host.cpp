@@ -705,6 +705,13 @@ pg_status make_half_form(pg_model* m) {
 // 2987, 32 x 512 105.0 ms and 103.3.  More sequences than a 32-row product takes would need tiles again.
 constexpr size_t kLastRowsMin = 128, kLastRowsTokens = 8, kLastRowsMost = 32;
 
+// Prompts whose attention and norms leave most CUs idle, and the bytes that those then read ahead of the products behind them: bf16 and int8
+// rows, one f16 number a value.  A prompt whole, us, without and with: width 1280 (16 MB for attention, 10 for the norm), 37 tokens 1790
+// and 1685; 1600 (26 and 15 MB), 64 tokens 2964 and 2774, 10 tokens 2117 and 2128; 1024 (10 and 6 MB, of which the norm reads none), 50
+// tokens 1112 and 1070, 20 tokens 939 and 928.  192 spare blocks are as good, 64 gain half; more than 26 MB do not fit the caches.
+constexpr int kAheadTokens = 64, kAheadBlocks = 128;
+constexpr size_t kAheadBytes = 8000000, kAheadMostBytes = 26000000;
+
 // Full-sequence forward of the nb sequences b .. b + nb - 1 over ids[nb][n] (each one
 // Gpt2Model::forward, src/models/gpt2/rust.rs:831-882, block_forward at 1053-1134) with MFMA
 // GEMMs over all nb * n rows at once and tiled causal attention per sequence; K and V of every
@@ -784,8 +791,10 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
   auto gemm = [&](const float* A, int lda, const float* W, const float* bias, float* Cout,
                   int ldc, int N, int K, int epi, const float* ln_g = nullptr,
                   const float* ln_b = nullptr, int a_cut = 0, int c_cut = 0, const void* w_half = nullptr,
-                  const float* w_half_mul = nullptr, const float* c_scale = nullptr, bool ln_half = false) -> hipError_t {
+                  const float* w_half_mul = nullptr, const float* c_scale = nullptr, bool ln_half = false,
+                  const pgk::Ahead* ahead = nullptr) -> hipError_t {
     pgk::GemmArgs a{};
+    a.ahead = ahead;
     a.A = A; a.w_bf16 = m->w_bf16; a.W = W; a.bias = bias; a.resid = Cout; a.C = Cout;
     a.a_cut = a.ln_cut = a_cut; a.c_cut = c_cut;
     if (w_half) {
@@ -800,6 +809,17 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
     a.split_items_per_cu = m->gemm_split_items;
     a.b9_min_rows = m->gemm_b9_min_rows;
     return pgk::launch_gemm(a, epi, m->num_cus, s);
+  };
+  // Weights that a launch of few blocks reads ahead: c_proj's and c_fc's for attention, the next c_attn's for the sums of mlp c_proj.
+  auto ahead_of = [&](const void* w_half, int N, int K, int epi, int k, pgk::Ahead* to) {
+    if (!half || nb != 1 || Ts > kAheadTokens) return;
+    pgk::GemmArgs a{};
+    a.w_half = w_half; a.w_half_parts = m->w_bf16 || m->w_i8 ? 1 : 2; a.w_half_planes = pgk::kHalfPlanes;
+    a.M = T; a.N = N; a.K = K;
+    a.ws = WS.p; a.ws_floats = ws_floats;
+    if (epi == pgk::GEMM_RESID) a.ln_out = XN.p;
+    pgk::gemm_half_ahead(a, epi, m->num_cus, k, to);
+    to->blocks = to->total() >= kAheadBytes && to->total() <= kAheadMostBytes ? kAheadBlocks : 0;
   };
   if (half)
     PG_HIP(pgk::launch_norm_rows_half(X.p, XN.p, T, C, m->half[0].norm_1_g, m->half[0].norm_1_b, g.eps, 1.0f, s));
@@ -829,10 +849,13 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
       if (st) return st;
       break;
     }
+    pgk::Ahead mlp_ahead;
+    ahead_of(hw.c_proj, C, C, pgk::GEMM_RESID, 0, &mlp_ahead);
+    ahead_of(hw.c_fc, I, C, pgk::GEMM_GELU, 1, &mlp_ahead);
     if (half || (cut && !m->half.empty()))
       PG_HIP(pgk::launch_attn_prefill_half(QKV.p, Ts, C, H, P, c->k_panel(l, b), c->v_panel(l, b), ATT.p, s, (int)nb,
                                            g.H * g.P * g.hd(), m->half[l].attn, pgk::attn_half_shape(Ts, H, (int)nb, m->num_cus),
-                                           half ? pgk::FORM_HALF : pgk::FORM_CUT));
+                                           half ? pgk::FORM_HALF : pgk::FORM_CUT, &mlp_ahead));
     else
       PG_HIP(pgk::launch_attn_prefill(QKV.p, Ts, C, H, hd, P, c->k_panel(l, b), c->v_panel(l, b),
                                       ATT.p, SCR.p, m->num_cus, s, (int)nb, g.H * g.P * g.hd(), form_of, c->drawn));
@@ -843,8 +866,10 @@ pg_status run_sequence_gemm(const pg_model* m, pg_kv_cache* c, size_t b, size_t 
     PG_HIP(gemm(XN.p, C, w.c_fc_w, w.c_fc_b, HB.p, I, I, C, pgk::GEMM_GELU, nullptr, nullptr, cut, cut,
                 hw.c_fc, hw.c_fc_mul, hw.hidden));
     PG_MARK(kMlpFc);
+    pgk::Ahead attn_ahead;
+    if (next) ahead_of(m->half.empty() ? nullptr : m->half[l + 1].c_attn, 3 * C, C, pgk::GEMM_BIAS, 0, &attn_ahead);
     PG_HIP(gemm(HB.p, I, w.c_proj_mlp_w, w.c_proj_mlp_b, X.p, C, C, I, pgk::GEMM_RESID, next_g, next_b, cut, 0,
-                hw.c_proj_mlp, hw.c_proj_mlp_mul, nullptr, half && next));
+                hw.c_proj_mlp, hw.c_proj_mlp_mul, nullptr, half && next, &attn_ahead));
     PG_MARK(kMlpProj);
   }
   if (all_logits_dst) {

@@ -343,6 +343,9 @@ bool gemm_takes_rows32(int M, int K, int lda, int w_bf16);
 bool gemm_supported(const GemmArgs& a);
 int gemm_split_parts(const GemmArgs& a, int num_cus, int bm = 64, int bn = 64);
 bool gemm_tail_plan(GemmArgs& a, int num_cus, int bm = 64, int bn = 64);
+// Likewise, as matrix k of *to, where the product takes W in half form, one f16 number a value, as blocks of rows that all see every row
+// of the input (with K cut over blocks a part's may be on another die).
+void gemm_half_ahead(const GemmArgs& a, int epi, int num_cus, int k, Ahead* to);
 // What a launch before launch_gemm(a) can read ahead for it, where the 32-row kernel takes it whole.
 Ahead gemm_rows32_ahead(const GemmArgs& a, int num_cus);
 hipError_t launch_gemm(const GemmArgs& a, int epilogue, int num_cus, hipStream_t s);
@@ -375,7 +378,7 @@ struct HalfScales {
 int attn_half_shape(int T, int H, int nseq, int num_cus);
 hipError_t launch_attn_prefill_half(const float* qkv, int T, int C, int H, int P, float* kcache, float* vcache, void* out,
                                     hipStream_t s, int nseq, size_t kv_stride, const HalfScales& scales, int shape,
-                                    int out_form = FORM_HALF);
+                                    int out_form = FORM_HALF, const Ahead* next = nullptr);
 // rows rows; row t is position t % period of its sequence (wpe may be null)
 hipError_t launch_embed_rows(float* x, const float* wte, const float* wpe, const uint32_t* ids,
                              int rows, int C, hipStream_t s, int w_bf16 = 0, int period = 0);

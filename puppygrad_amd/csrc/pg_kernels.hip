@@ -1474,7 +1474,7 @@ Ahead gemv_pair_ahead(const GemvPair& a) {
   }
   // (beside about 60 blocks of mixers, of 512 threads; a request of 32 tokens behind 1000, ms: no spare block 10.55, 32 10.42, 48 10.20,
   // 64 10.19, 80 10.25, 112 10.46, 128 10.33, 256 10.42)
-  r.blocks = ahead_pays((size_t)r.slab_bytes[0] + r.slab_bytes[1]) ? 64 : 0;
+  r.blocks = ahead_pays(r.total()) ? 64 : 0;
   return r;
 }
 

@@ -356,9 +356,6 @@ __global__ __launch_bounds__(256) void k_splitk_reduce(GemmArgs a, int parts) {
   }
 }
 
-// No weights to read ahead (a branch for them in the launches that have none cost 0.2 to 0.7 us each).
-struct Nothing {};
-
 // k_splitk_reduce for one whole row per block, followed by the LayerNorm of that row
 // (layer_norm_in_place, cpu.rs:119-143: mean, biased variance in a second pass, eps inside
 // the root) into a.ln_out: the projection back to n_embd and the LayerNorm that reads its

@@ -74,6 +74,19 @@ def test_batched_steps_that_read_ahead(C, storage, B):
         assert_logits_close(got[b], want)
 
 
+# (1280: attention reads 16 MB ahead, the norm 10; 1600: 26 and 15; 1024: 10 and none)
+@pytest.mark.gpu
+@pytest.mark.parametrize("C,storage,n", [(1024, 1, 50), (1280, 1, 5), (1280, 2, 37), (1280, 1, 64), (1280, 1, 65), (1600, 2, 17), (1600, 1, 64)])
+def test_prompts_that_read_ahead(C, storage, n):
+    cfg = Gpt2Config(vocab_size=97, n_positions=72, n_embd=C, n_layer=3, n_head=C // 64)
+    w = synth.random_weights(cfg, 0x5EED0C02 + C, perturb=True)
+    ids = synth.token_ids(n, 0x70C00C02 + n, cfg.vocab_size)
+    model = Gpt2Model.new(cfg, w, Gpt2HipConfig(weight_storage=storage))
+    ref = oracle.Model(cfg, synth.bf16_rounded(w) if storage == 1 else w, oracle.rust_config(8, quantized_weights=int(storage == 2)))
+    cache, rc = model.new_kv_cache(), ref.new_kv_cache()
+    assert_logits_close(model.prefill(ids, cache).to_host(), ref.prefill(ids, rc))
+
+
 @pytest.mark.gpu
 def test_stack_step_that_reads_ahead(tmp_path):
     cfg = synth.tarepel_config(1600, 3, vocab=61)
