@@ -357,10 +357,8 @@ def measure_prefill(model, cfg, ids, T, steps, warmup):
     """One prefill of T tokens into an empty cache through the full-sequence path, MFMA-bound:
     wall time over `steps` runs for the whole prefill, and one profiled run (HIP events between
     the launches) for the share of the four projections."""
-    C_, I, L, V = cfg.n_embd, cfg.n_inner, cfg.n_layer, cfg.vocab_size
-    gemm_flops = 2.0 * T * L * (3 * C_ * C_ + C_ * C_ + 2 * C_ * I)
-    attn_flops = 4.0 * C_ * (T * (T + 1) / 2) * L
-    flops = gemm_flops + attn_flops + 2.0 * V * C_
+    flops, gemm_flops = prefill_flops(cfg, 1, T)
+    attn_flops = flops - gemm_flops - 2.0 * cfg.vocab_size * cfg.n_embd
     cache = model.new_kv_cache()
     for _ in range(max(1, warmup)):
         model.prefill(ids, cache).argmax()
@@ -421,10 +419,12 @@ BF16_MFMA_PEAK_TFLOPS = 2500.0  # MI355X published dense bf16 matrix rate
 
 
 def prefill_flops(cfg, B, T):
-    """(all, projections only) algorithmic flops of B prompts of T tokens."""
+    """(all, projections only) algorithmic flops of B prompts of T tokens.  Behind the last layer's keys and
+    values, prompts of 128 rows or more go on with the last row of each sequence."""
     C_, I, L, V = cfg.n_embd, cfg.n_inner, cfg.n_layer, cfg.vocab_size
-    gemm_flops = 2.0 * B * T * L * (3 * C_ * C_ + C_ * C_ + 2 * C_ * I)
-    attn_flops = 4.0 * B * C_ * (T * (T + 1) / 2) * L
+    cut = B * T >= 128 and T >= 8 and B <= 32
+    gemm_flops = 2.0 * B * (T * L * 3 * C_ * C_ + (T * (L - cut) + cut) * (C_ * C_ + 2 * C_ * I))
+    attn_flops = 4.0 * B * C_ * ((T * (T + 1) / 2) * (L - cut) + T * cut)
     return gemm_flops + attn_flops + 2.0 * B * V * C_, gemm_flops
 
 
@@ -468,8 +468,8 @@ def bench_prefill(args, cfg, model, ids, n_prefill) -> int:
     """Secondary workload (prompt processing, e.g. GPT-2 124M with 1024 tokens): a step is one
     prefill of n_prefill tokens into an empty cache through the GEMM path; with --batch B > 1
     (given explicitly) B prompts of that length at once (pg_gpt2_prefill_batch).  Algorithmic
-    flops: the four projections of every layer over all tokens, causal attention
-    (QK^T and PV over the lower triangle), and the lm_head row of the last token."""
+    flops: the four projections of every layer, causal attention (QK^T and PV over the lower triangle;
+    what the last layer does behind its keys and values: prefill_flops), and the lm_head row of the last token."""
     from puppygrad_amd import synth
     T = n_prefill
     B = args.batch if args.batch_given else 1
@@ -576,7 +576,7 @@ def bench_stack(args) -> int:
                 logits = model.prefill(ids, cache)
             logits.argmax()
             sec = (time.time() - t0) / n
-            flops = 2.0 * params * T
+            flops = 2.0 * params * T  # (as if the last layer's way back to the residual ran for every token)
             out["prefill"] = {"tokens_per_s": round(T / sec, 1), "ms": round(sec * 1e3, 3),
                               "product_tflops": round(flops / sec / 1e12, 1),
                               "frac_bf16_mfma": round(flops / sec / 1e12 / BF16_MFMA_PEAK_TFLOPS, 4)}
