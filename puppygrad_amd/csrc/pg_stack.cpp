@@ -1540,7 +1540,8 @@ pg_status rows_segment(const pg_model* model, pg_kv_cache* c, const uint32_t* d_
     x += (size_t)want[0] * Cp, mix += (size_t)want[0] * last.mix_pad;
     if (last.has_mlp) act += (size_t)want[0] * last.mlp.ff_pad;
     PG_HIP(launch_pair(pair_of(model, last, x, mix, act), last, act, s));
-    PG_MARK(kAttnProj);
+    if (last.has_mlp) PG_MARK(kMlpProj);  // (both products, as in a step)
+    else PG_MARK(kAttnProj);
     if (pg_status e = head_one(model, x, dst, s)) return e;
   } else if (few && W > 0) {
     if (pg_status e = send_rows_at(st, want, s)) return e;

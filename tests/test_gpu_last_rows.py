@@ -72,3 +72,12 @@ def test_batches(pair, B, n):
     got = pair.dev.prefill_batch(ids, cache).to_host()
     for b in sorted({0, B // 2, B - 1}):
         check(got[b], pair.ref.run([int(t) for t in ids[b]])[-1:], 5e-5)
+
+
+@pytest.mark.parametrize("ff", [40, None])
+def test_the_last_row_is_booked_as_a_step_books_it(tmp_path, ff):
+    """Both products back to the residual are one launch: the MLP's, where there is one."""
+    cfg = other.config([other.parallel(ff=ff)])
+    dev = Pair(tarepel, tmp_path, cfg, other.weights(cfg, 19)).dev
+    prof = dev.prefill_profiled([3, 1, 4, 1, 5], dev.new_kv_cache())[1]
+    assert (prof.attention_projection == 0) == (ff is not None) and (prof.mlp_projection > 0) == (ff is not None)
