@@ -706,9 +706,12 @@ pg_status make_half_form(pg_model* m) {
 constexpr size_t kLastRowsMin = 128, kLastRowsTokens = 8, kLastRowsMost = 32;
 
 // Prompts whose attention and norms leave most CUs idle, and the bytes that those then read ahead of the products behind them: bf16 and int8
-// rows, one f16 number a value.  A prompt whole, us, without and with: width 1280 (16 MB for attention, 10 for the norm), 37 tokens 1790
-// and 1685; 1600 (26 and 15 MB), 64 tokens 2964 and 2774, 10 tokens 2117 and 2128; 1024 (10 and 6 MB, of which the norm reads none), 50
-// tokens 1112 and 1070, 20 tokens 939 and 928.  192 spare blocks are as good, 64 gain half; more than 26 MB do not fit the caches.
+// rows, one f16 number a value (half form: from 17 rows on).  A prompt whole, us, without and with: width 1280 (16 MB for attention, 10 for the
+// norm), 37 tokens 1807 and 1720; 1600 (26 and 15 MB), 64 tokens 2968 and 2710, 20 tokens 2374 and 2233; 1024 (10 and 6 MB, of which the norm
+// reads none), 50 tokens 1112 and 1070.  192 spare blocks are as good, 64 gain half.  Below the lower line: width 768 (5.9 MB for attention) 37
+// tokens 468 and 476, 64 509 and 530, 832 (6.9 MB) 475 and 480, 896 (8.0 MB) 491 and 491.  Past the upper one, which is as far as the four
+// sizes of GPT-2 go, it still gains, less and less: 50 tokens, 12 layers, 27.7 MB (1664) 786 and 757, 32 (1792) 832 and 813, 37 tokens of 32 MB 755 and
+// 763, of 36.9 (1920) 793 and 794.  More than 64 rows are two blocks of input rows or tiles, with which a row of W has several readers.
 constexpr int kAheadTokens = 64, kAheadBlocks = 128;
 constexpr size_t kAheadBytes = 8000000, kAheadMostBytes = 26000000;
 

@@ -343,11 +343,14 @@ bool gemm_takes_rows32(int M, int K, int lda, int w_bf16);
 bool gemm_supported(const GemmArgs& a);
 int gemm_split_parts(const GemmArgs& a, int num_cus, int bm = 64, int bn = 64);
 bool gemm_tail_plan(GemmArgs& a, int num_cus, int bm = 64, int bn = 64);
-// Likewise, as matrix k of *to, where the product takes W in half form, one f16 number a value, as blocks of rows that all see every row
-// of the input (with K cut over blocks a part's may be on another die).
-void gemm_half_ahead(const GemmArgs& a, int epi, int num_cus, int k, Ahead* to);
 // What a launch before launch_gemm(a) can read ahead for it, where the 32-row kernel takes it whole.
 Ahead gemm_rows32_ahead(const GemmArgs& a, int num_cus);
+// Likewise, as matrix k of *to, where the product takes W in half form, one f16 number a value, as blocks of rows that all see every row
+// of the input.  With K cut over blocks that are no multiple of eight to a part, the words of all parts but the first come to another die's
+// cache than their block's, and the product finds them in the memory-side cache: c_proj of width 1600, 64 rows (50 blocks, four
+// parts), not read ahead 6.3 us, so 5.2; with each part on its own die 5.0, but every launch that reads ahead was 0.1 us longer for it
+// (prompts 0.2 to 1.8 % slower), and without such a product's words they were 2 to 4 % slower.
+void gemm_half_ahead(const GemmArgs& a, int epi, int num_cus, int k, Ahead* to);
 hipError_t launch_gemm(const GemmArgs& a, int epilogue, int num_cus, hipStream_t s);
 // Many small products in one launch: rows are sorted by the matrix they meet.  Row m of the product
 // takes row group_rows[m] of A (any row where that is -1), and the rows of tile m / tile_rows meet

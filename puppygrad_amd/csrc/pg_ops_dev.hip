@@ -545,6 +545,23 @@ int32_t pg_testing_attn_shape(int32_t rows, int32_t heads, int32_t sequences, in
   return pgk::attn_cut_shape(rows, heads, sequences, num_cus);
 }
 
+// The plan of a product of `rows` input rows with bf16 or int8 rows in half form, behind attention or a norm, and what is read ahead for
+// it: tile, parts, mt, rows of W a block; slabs, bytes of a slab and of a group.
+void pg_testing_half_ahead(int32_t rows, int32_t in_f, int32_t out_f, int32_t resid, int32_t num_cus, uint32_t* out) {
+  pgk::GemmArgs a{};
+  float any = 0.0f;  // (neither read nor written)
+  a.w_half = &any; a.w_half_parts = 1; a.w_half_planes = pgk::kHalfPlanes;
+  a.M = rows; a.N = out_f; a.K = in_f;
+  a.ws = &any; a.ws_floats = (size_t)8 * rows * std::min(in_f, out_f);
+  if (resid) a.ln_out = &any;
+  const int epi = resid ? pgk::GEMM_RESID : pgk::GEMM_BIAS;
+  const pgk::HalfPlan p = pgk::gemm_half_plan(a, epi, num_cus);
+  pgk::Ahead h;
+  pgk::gemm_half_ahead(a, epi, num_cus, 0, &h);
+  const uint32_t v[7] = {(uint32_t)p.tile, (uint32_t)p.parts, (uint32_t)p.mt, (uint32_t)p.rows, h.slabs[0], h.slab_bytes[0], h.group_bytes[0]};
+  std::copy(v, v + 7, out);
+}
+
 // Attention of `sequences` prompts of `rows` tokens each, head size 64, keys and values to panels [sequences][heads][rows][64]:
 // in blocks of the given shape of pg_attn_cut.hip (0: as the planner has it).
 pg_status pg_testing_attention_rows_dev(int32_t device, void* stream, const float* qkv, uint64_t rows, uint64_t heads,

@@ -1,4 +1,5 @@
 """Weights read ahead by a launch's spare blocks (pg_ahead.h): which words, and the steps that do it."""
+import ctypes
 import subprocess
 from pathlib import Path
 
@@ -8,22 +9,26 @@ import pytest
 import oracle
 from helpers import assert_logits_close
 from oracle import tarepel
-from puppygrad_amd import Gpt2Config, Gpt2HipConfig, Gpt2Model, synth
+from puppygrad_amd import Gpt2Config, Gpt2HipConfig, Gpt2Model, _lib, synth
 from stack_helpers import Pair, check, rounded
 
 CSRC = Path(__file__).resolve().parents[1] / "puppygrad_amd" / "csrc"
 DIES, LINE = 8, 128
+ROWS = 4  # HALF_ROWS
 PROGRAM = """
 #include <cstdio>
 #include <cstdlib>
 #include "pg_ahead.h"
+// every word that the spare blocks, the first of them block `first` of its launch, read: die and place
 int main(int, char** v) {
   pgk::Ahead a;
   a.matrix(1, nullptr, atoi(v[1]), atoi(v[2]), atoi(v[3]));
-  for (unsigned die = 0; die < pgk::kDies; ++die)
-    for (unsigned w = 0; w < a.words[1]; ++w) {
-      unsigned at;
-      if (pgk::ahead_word(a, 1, die, w, &at)) printf("%u %u\\n", die, at);
+  a.blocks = atoi(v[4]);
+  const int first = atoi(v[5]), threads = atoi(v[6]);
+  for (int block = 0; block < a.blocks; ++block)
+    for (int tid = 0; tid < threads; ++tid) {
+      auto load = [&](unsigned at) { return printf("%d %u\\n", (first + block) % 8, at), at; };
+      pgk::ahead_words(a, 1, block, first + block, tid, threads, load, [](const unsigned (&)[pgk::kAheadAtOnce]) {});
     }
 }
 """
@@ -33,23 +38,37 @@ int main(int, char** v) {
 def words_of(tmp_path_factory):
     tmp = tmp_path_factory.mktemp("ahead")
     (tmp / "words.cpp").write_text(PROGRAM)
-    subprocess.run(["g++", "-std=c++17", f"-I{CSRC}", str(tmp / "words.cpp"), "-o", str(tmp / "words")], check=True)
-    return lambda *args: np.loadtxt(subprocess.run([str(tmp / "words"), *map(str, args)], check=True, capture_output=True,
-                                                   text=True).stdout.splitlines(), dtype=np.int64).reshape(-1, 2)
+    subprocess.run(["g++", "-O2", "-std=c++17", f"-I{CSRC}", str(tmp / "words.cpp"), "-o", str(tmp / "words")], check=True)
+    return lambda *args: np.array(subprocess.run([str(tmp / "words"), *map(str, args)], check=True, capture_output=True).stdout.split(),
+                                  np.int64).reshape(-1, 2)
 
 
-@pytest.mark.parametrize("row,rows,group", [(4096, 3072, 12), (3200, 4800, 19), (3200, 6400, 25), (7296, 1600, 7), (4, 3, 1),
-                                            (128, 8, 1), (132, 9, 2), (5120, 15, 4), (64, 1000, 3), (3200, 8, 8)])
-def test_every_line_of_a_group_is_read_by_its_own_die(words_of, row, rows, group):
-    got = words_of(1, row * rows, row * group)
-    assert (got[:, 1] % 4 == 0).all() and (got[:, 1] + 4 <= row * rows).all()
-    assert len(np.unique(got[:, 1])) == len(got)
-    size = row * group
-    for g in range(0, -(-rows // group)):
-        first, last = g * size, min((g + 1) * size, row * rows)
-        mine = got[got[:, 1] // size == g]
-        assert (mine[:, 0] == g % DIES).all()
-        np.testing.assert_array_equal(np.sort(mine[:, 1]), np.arange(first, last, LINE))
+# rows one after the other, and slabs; spare blocks behind any number of others
+@pytest.mark.parametrize("slabs,slab,group", [
+    (1, 4096 * 3072, 4096 * 12), (1, 3200 * 4800, 3200 * 19), (1, 3200 * 6400, 3200 * 25), (1, 7296 * 1600, 7296 * 7), (1, 12, 4),
+    (1, 128 * 8, 128), (1, 132 * 9, 132 * 2), (1, 64 * 1000, 64 * 3), (160, 1280 * 16, 40 * 16), (160, 5120 * 16, 24 * 16),
+    (200, 1600 * 16, 32 * 16), (67, 72 * 16, 8 * 16), (3, 30000 * 16, 8 * 16)])
+@pytest.mark.parametrize("blocks,first,threads", [(8, 0, 64), (64, 57, 512), (128, 20, 256)])
+def test_every_line_of_a_group_is_read_once_by_its_own_die(words_of, slabs, slab, group, blocks, first, threads):
+    got = words_of(slabs, slab, group, blocks, first, threads)
+    want = {s * slab + at: g % DIES for s in range(slabs) for g in range(-(-slab // group))
+            for at in range(g * group, min((g + 1) * group, slab), LINE)}
+    assert len(got) == len(want) and {int(at): int(die) for die, at in got} == want
+
+
+@pytest.mark.parametrize("width", [1088, 1216, 1280, 1408, 1600])
+@pytest.mark.parametrize("rows", [17, 37, 50, 64, 65])
+def test_groups_of_short_prompts_products_are_their_blocks(width, rows):
+    f = _lib.load().pg_testing_half_ahead
+    f.argtypes, f.restype = [ctypes.c_int32] * 5 + [ctypes.POINTER(ctypes.c_uint32)], None
+    for in_f, out_f, resid in ((width, width, 1), (width, 4 * width, 0), (width, 3 * width, 0)):
+        out = (ctypes.c_uint32 * 7)()
+        f(rows, in_f, out_f, resid, 256, out)
+        tile, _, mt, block_rows, slabs, slab, group = out
+        if tile == ROWS and rows <= 16 * mt:
+            assert (slabs, slab, group) == (in_f // 8, out_f * 16, block_rows * 16)
+        else:
+            assert slabs == 0
 
 
 # (1408: f32 rows of c_attn 23.8 MB, c_fc beyond what is read ahead; 1600: bf16 rows 15.4 and 20.5 MB)
@@ -74,9 +93,9 @@ def test_batched_steps_that_read_ahead(C, storage, B):
         assert_logits_close(got[b], want)
 
 
-# (1280: attention reads 16 MB ahead, the norm 10; 1600: 26 and 15; 1024: 10 and none)
+# (1280: attention reads 16 MB ahead, the norm 10; 1600: 26 and 15; 1024: 10 and none; 16 and 65 tokens: on the far sides of the lines)
 @pytest.mark.gpu
-@pytest.mark.parametrize("C,storage,n", [(1024, 1, 50), (1280, 1, 5), (1280, 2, 37), (1280, 1, 64), (1280, 1, 65), (1600, 2, 17), (1600, 1, 64)])
+@pytest.mark.parametrize("C,storage,n", [(1024, 1, 50), (1280, 1, 16), (1280, 1, 17), (1280, 2, 37), (1280, 1, 64), (1280, 1, 65), (1600, 2, 17), (1600, 1, 64)])
 def test_prompts_that_read_ahead(C, storage, n):
     cfg = Gpt2Config(vocab_size=97, n_positions=72, n_embd=C, n_layer=3, n_head=C // 64)
     w = synth.random_weights(cfg, 0x5EED0C02 + C, perturb=True)
