@@ -1333,15 +1333,16 @@ pg_status wanted_rows(const pg_model* model, StackCache& st, Gemm gemm, const fl
   gemm.rows = (int)want.size();
   return head_rows(model, gemm, x, h, st.rows_at, dst);
 }
-// Whether the last layer, behind whose mixers only the rows whose logits are wanted are read, goes on with those alone: `cols` values of
-// each of them lie where the projections, max_in a row, did.  Several are gathered first, which pays from `each` rows to a wanted one
-// on.  Prompts and 2 tokens, ms, all rows and so: Movudra at 1600, 32 x 100 11.18 and 10.76, 1000 4.32 and 4.16, 16 1.80 and 1.78, at 1280
-// 20 x 8 3.49 and 3.47; parallel sublayers at 1600, 32 x 100 9.99 and 9.80, 1000 3.57 and 3.51, at 768 8 x 20 1.544 and 1.558, 4 x
-// 100 1.586 and 1.634 (2048 rows are needed there).  Up to 32 rows one product reads W once; drawn streams keep the order of their sums.
-bool few_rows(const pg_kv_cache* c, const std::vector<int>& want, size_t rows, size_t cols, int max_in, size_t each) {
-  return !c->drawn && want.size() <= 32 && (want.size() > 1 ? each : 4) * want.size() <= rows && want.size() * cols <= rows * (size_t)max_in;
+// From how many rows on the last layer, behind whose mixers only the rows whose logits are wanted are read, goes on with those alone.
+// Several are gathered first.  Prompts and 2 tokens, ms, all rows and so: Movudra at 1600, 32 x 100 11.18 and 10.76, 1000 4.32 and 4.16, 16 1.80
+// and 1.78, at 1280 20 x 8 3.49 and 3.47; parallel sublayers at 1600, 32 x 100 9.99 and 9.80, 1000 3.57 and 3.51, at 768 8 x 20 1.544 and
+// 1.558, 4 x 100 1.586 and 1.634.
+size_t few_rows_from(bool post_norm, size_t wanted) { return wanted > 1 && !post_norm ? 2048 : 4 * wanted; }
+// Whether it does: `cols` values of each wanted row lie where the projections did.  Up to 32 rows one product reads W once; drawn streams
+// keep the order of their sums.
+bool few_rows(const StackModel& m, const pg_kv_cache* c, const std::vector<int>& want, size_t rows, size_t cols) {
+  return !c->drawn && want.size() <= 32 && rows >= few_rows_from(m.post_norm, want.size()) && want.size() * cols <= rows * (size_t)m.max_in;
 }
-
 
 // rows_segment for post-norm layers.
 pg_status post_norm_rows(const pg_model* model, pg_kv_cache* c, const uint32_t* d_ids, size_t n, size_t pos0,
@@ -1351,7 +1352,7 @@ pg_status post_norm_rows(const pg_model* model, pg_kv_cache* c, const uint32_t* 
   hipStream_t s = c->stream;
   const size_t B = c->B, rows = B * n, Cp = (size_t)m.width_pad;
   const int W = (int)want.size();
-  const bool few = few_rows(c, want, rows, Cp + m.layers.back().mix_pad, m.max_in, 4);
+  const bool few = few_rows(m, c, want, rows, Cp + m.layers.back().mix_pad);
   size_t work_floats = 0, lat_floats = 0, kv_floats = 0, act_floats = 0;
   MoeSizes ms;
   for (const StackLayer& l : m.layers) {
@@ -1468,8 +1469,7 @@ pg_status rows_segment(const pg_model* model, pg_kv_cache* c, const uint32_t* d_
   const size_t B = c->B, rows = B * n, Cp = (size_t)m.width_pad;
   const StackLayer& last = m.layers.back();
   const int W = (int)want.size();
-  const bool few = few_rows(c, want, rows, Cp + last.mix_pad + (last.has_mlp ? last.mlp.ff_pad : 0), m.max_in,
-                            std::max<size_t>(32, 2048 / std::max(W, 1)));
+  const bool few = few_rows(m, c, want, rows, Cp + last.mix_pad + (last.has_mlp ? last.mlp.ff_pad : 0));
   const size_t ws_floats = 8 * rows * Cp;
   float *x, *h, *y, *mix, *act, *krot, *conv, *decay, *work, *ws, *ws_side;
   size_t work_floats = 0;
@@ -1516,7 +1516,7 @@ pg_status rows_segment(const pg_model* model, pg_kv_cache* c, const uint32_t* d_
       PG_HIP(pgk::launch_commit_rows(r, &b.attn, nullptr, side));
     }
     PG_MARK(kAttention);
-    if (l.has_mlp) {
+    if (l.has_mlp && (whole || W > 0)) {
       PG_HIP(pgk::launch_gated_mlp_rows(r, l.mlp, side));
       PG_MARK(kMlpFc);
       if (whole) PG_HIP(side_gemm(act, l.down_w, x, (int)Cp, l.mlp.ff_pad, l.ls2, nullptr, nullptr));
@@ -1610,3 +1610,6 @@ pg_status stack_rows(const pg_model* model, pg_kv_cache* c, const uint32_t* ids,
 }
 
 }  // namespace pgh
+
+// few_rows_from
+extern "C" uint64_t pg_testing_few_rows_from(int32_t post_norm, uint64_t wanted) { return pgh::few_rows_from(post_norm != 0, wanted); }

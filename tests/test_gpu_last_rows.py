@@ -54,7 +54,7 @@ def pair(request, tmp_path_factory):
 # (5e-5: what models of six layers are held to, whichever rows are wanted)
 @pytest.mark.parametrize("n,wanted", [(40, []), (3, [2]), (4, [3]), (4, [0]), (7, [2, 5]), (8, [2, 5]), (131, range(99, 131)),
                                       (127, range(95, 127)), (140, range(0, 132, 4)),
-                                      (2047, [1, 2046]), (2048, [1, 2046])])
+                                      (2047, [1, 2046]), (2047, [1, 7, 2046]), (2048, [1, 2046]), (2048, [1, 7, 2046])])
 def test_wanted_rows(pair, n, wanted):
     ids, wanted = pair.ids(n + 2, seed=n), list(wanted)
     want = pair.ref.run(ids)
