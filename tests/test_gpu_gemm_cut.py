@@ -61,7 +61,8 @@ def test_int8_rows(rows, k, n):
 # a short prompt (64-row tiles, cut K), a ragged one, and batches with 128-row and 128 x 256 tiles
 @pytest.mark.parametrize("batch,n", [(1, 65), (1, 333), (5, 200), (16, 512)])
 def test_bf16_rows_give_what_f32_rows_of_the_same_values_give(batch, n):
-    cfg = Gpt2Config(vocab_size=300, n_positions=512, n_embd=768, n_layer=1, n_head=12)
+    # (two layers: behind the last one's keys and values a prompt goes on with its last row)
+    cfg = Gpt2Config(vocab_size=300, n_positions=512, n_embd=768, n_layer=2, n_head=12)
     w = synth.bf16_rounded(synth.random_weights(cfg, 0x5EED0900, perturb=True))
     ids = synth.token_ids(batch * n, 0x70C00900 + n, cfg.vocab_size).reshape(batch, n)
     got = []

@@ -337,6 +337,13 @@ def test_scales_hold_for_models_of_any_size_of_values():
         there = Gpt2Model.new(cfg, w, Gpt2HipConfig(gemm_b9_min_rows=0xffffffff))
         got, want = logits(here, ids), logits(there, ids)
         assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want), (gain, weight)
+        # Of a prompt's rows all but the last leave the last layer behind its keys and values; here all of them go through it.  Queries and keys
+        # are right to 3 2^-24, a score of size s to 6 2^-24 of it, and a weight to twice that where two keys share it; a score's standard
+        # deviation is a query's times a key's, and the largest about four of them.
+        size = 4 * (weight * 0.02) ** 2 * 512
+        got, want = here.forward(ids).logits, there.forward(ids).logits
+        off = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+        assert (off <= 1e-5 + size * 12 * 2.0 ** -24).all() and np.median(off) <= 1e-5, (gain, weight, off.max())
 
 
 def uneven_weights(cfg, seed):
@@ -494,3 +501,8 @@ def test_weights_without_half_form_are_served_as_before(storage, how):
             assert np.linalg.norm(got - want) <= 1e-5 * np.linalg.norm(want)
         else:
             assert how == "infinite bound" and not np.isfinite(got).any()
+        # (the last layer's products of all rows: a prompt of 128 goes on with its last one there)
+        every = refused.forward(ids[:n]).logits
+        np.testing.assert_array_equal(every, without.forward(ids[:n]).logits)
+        if np.isfinite(want).all():
+            assert np.linalg.norm(every[-1] - want) <= 1e-5 * np.linalg.norm(want)

@@ -74,8 +74,9 @@ def test_per_operation_and_batched_paths_with_other_split_plans(blocks, items):
     model, ref = Gpt2Model.new(cfg, w, hip), oracle.Model(cfg, w)
     assert f"attn_blocks_per_cu={blocks}" in model.describe()
     decode_against_oracle(model, ref, ids)
-    # 124M's layer shapes at 512 tokens: the projections back to n_embd are cut along K
-    cfg = Gpt2Config(vocab_size=97, n_positions=512, n_embd=768, n_layer=1, n_head=12)
+    # 124M's layer shapes at 512 tokens: the projections back to n_embd are cut along K (in all layers but the last, where a prompt
+    # goes on with its last row)
+    cfg = Gpt2Config(vocab_size=97, n_positions=512, n_embd=768, n_layer=2, n_head=12)
     w = synth.random_weights(cfg, 0x5EED0214, perturb=True)
     ids = list(synth.token_ids(512, 0x70C00214, 97))
     per_op = Gpt2Model.new(cfg, w, Gpt2HipConfig(decode_path=1, attn_blocks_per_cu=blocks,
@@ -103,7 +104,7 @@ def test_planner_tunables_move_the_prompt_to_other_kernels_with_the_same_logits(
     """seq_gemm_min_tokens decides from which prompt length the GEMM prefill runs,
     gemm_b9_min_rows from which row count f32 products take the bf16 matrix cores: every
     setting gives the oracle's logits (there the products are right to 2^-24)."""
-    cfg = Gpt2Config(vocab_size=97, n_positions=512, n_embd=768, n_layer=1, n_head=12)
+    cfg = Gpt2Config(vocab_size=97, n_positions=512, n_embd=768, n_layer=2, n_head=12)
     w = synth.random_weights(cfg, 0x5EED0650, perturb=True)
     ref = oracle.Model(cfg, w, oracle.rust_config(8))
     ids = [int(t) for t in synth.token_ids(512, 0x70C00650, 97)]
@@ -133,13 +134,13 @@ def test_min_rows_of_the_bf16_cores_is_a_bound_beside_the_planners_rule():
     few_tiles = logits(w, cfg, ids, 0xffffffff)
     for rows in (0, 65, 128, 1024):
         np.testing.assert_array_equal(logits(w, cfg, ids, rows), few_tiles)
-    cfg = Gpt2Config(vocab_size=97, n_positions=512, n_embd=768, n_layer=1, n_head=12)
+    cfg = Gpt2Config(vocab_size=97, n_positions=512, n_embd=768, n_layer=2, n_head=12)
     w, ids = synth.random_weights(cfg, 0x5EED0650, perturb=True), ids[:512]
     np.testing.assert_array_equal(logits(w, cfg, ids, 0), logits(w, cfg, ids, 65))
     np.testing.assert_array_equal(logits(w, cfg, ids, 513), logits(w, cfg, ids, 0xffffffff))
     assert (logits(w, cfg, ids, 0) != logits(w, cfg, ids, 513)).any()
     # two rows of tiles that leave half of the CUs without one stay on the f32 cores, three do not
-    cfg = Gpt2Config(vocab_size=97, n_positions=256, n_embd=1280, n_layer=1, n_head=20)
+    cfg = Gpt2Config(vocab_size=97, n_positions=256, n_embd=1280, n_layer=2, n_head=20)
     w = synth.random_weights(cfg, 0x5EED0652, perturb=True)
     for rows in (66, 128):
         np.testing.assert_array_equal(logits(w, cfg, ids[:rows], 0), logits(w, cfg, ids[:rows], 0xffffffff))
