@@ -695,16 +695,16 @@ TRAFFIC_SOURCE = "profiles/k_decode_persistent_1600_xl_decode_traffic.txt"
 TRAFFIC_RATIO_124M = 0.983
 TRAFFIC_SOURCE_124M = "profiles/k_decode_persistent_768_124m_decode.txt"
 # HBM bytes of one 124M prefill (FETCH_SIZE + WRITE_SIZE of all its launches, scaled)
-TRAFFIC_124M_PREFILL_1024 = 4435300000
+TRAFFIC_124M_PREFILL_1024 = 4151600000
 TRAFFIC_124M_PREFILL_32 = 610200000
 TRAFFIC_SOURCE_124M_PREFILL = "profiles/prefill_124m_traffic.txt"
-TRAFFIC_RATIO_355M_B16 = 1.093
-TRAFFIC_RATIO_XL_BF16_B32 = 1.073  # same file, section (c)
+TRAFFIC_RATIO_355M_B16 = 1.091  # section (d); what is read ahead is counted once
+TRAFFIC_RATIO_XL_BF16_B32 = 1.063  # same file and section
 TRAFFIC_SOURCE_355M_B16 = "profiles/batched_decode_355m_b16_xl_bf16_b32.txt"
 # Bytes through the L2s to and from the fabric per XL bf16 prefill of 32 x 512 tokens (FETCH_SIZE
 # scaled by 1.9994 + WRITE_SIZE over all launches of a step; most of the reads are operand
 # re-reads that the Infinity Cache serves).
-TRAFFIC_XL_BF16_PREFILL_B32_512 = 328400000000
+TRAFFIC_XL_BF16_PREFILL_B32_512 = 326900000000
 TRAFFIC_SOURCE_XL_BF16_PREFILL = "profiles/k_gemm_half_prompts.txt"
 
 
